@@ -227,7 +227,8 @@ int sa_mask_pack_partial(const uint8_t *mask, const int64_t mask_strides[4], int
  *                    do not differ between batch elements
  *   packed           optional (NULL: lists only): as in sa_mask_pack_partial; plane (b, 0) is written for every
  *                    distinct b, packed_strides[1] must be 0 when H > 1, base and batch stride multiples of 4 bytes
- *   workspace        sa_mask_terms_workspace_bytes(distinct batch planes, ...) bytes of device memory
+ *   workspace        sa_mask_terms_workspace_bytes(distinct batch planes, ...) bytes of device memory (checked; the
+ *                    present kernel keeps its state on the chip and leaves it untouched)
  * BLOCK_K: a power of two >= 16.
  */
 size_t sa_mask_terms_workspace_bytes(int distinct_b, int Sq, int Sk, int BQ, int BK);

@@ -89,16 +89,16 @@ struct TermsParams {
     const int32_t *doc_q, *doc_k;  // [uB, Sq] and [uB, Sk] document numbers, or null
     int64_t dqs[2], dks[2];        // their strides in elements
     int uB;                        // distinct planes (the mask never depends on the head)
-    int Sq, Sk, BQ, BK, nQ, nK;
-    uint8_t *cls;                  // [uB, nQ, nK] class bytes (classification)
-    // packing: the PARTIAL lists of the distinct planes and the output in PackParams layout
-    const int32_t *part_ids, *part_lens;
-    int64_t pis[4], pls[3];
-    uint8_t *packed;
-    int64_t ob;  // bytes between packed planes along b
+    int Sq, Sk, BQ, BK, lbk, nQ, nK;
+    // the lists: oH planes along the head, and along the batch all oB planes from the one distinct plane (oB_all) or
+    // the distinct plane's own
+    int oB_all, oB, oH;
+    int32_t *full_ids, *full_lens, *part_ids, *part_lens;
+    int64_t fis[4], fls[3], pis[4], pls[3];
+    uint8_t *packed;  // PackParams layout, or null
+    int64_t ob;       // bytes between packed planes along b
 };
-hipError_t launch_classify_terms(const TermsParams &p, hipStream_t stream);
-hipError_t launch_pack_terms(const TermsParams &p, hipStream_t stream);
+hipError_t launch_mask_terms(const TermsParams &p, hipStream_t stream);
 
 // ---- block-sparse forward ------------------------------------------------------------------------
 struct FwdParams {

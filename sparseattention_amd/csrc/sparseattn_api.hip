@@ -659,6 +659,7 @@ int sa_mask_classify_terms(const int32_t *terms, int n_terms, const int32_t *doc
     const int nQ = Sq / BQ, nK = Sk / BK;
     if (nQ > 65535 || uB > 65535)
         return fail(SA_ERR_UNSUPPORTED, "sa_mask_classify_terms: more than 65535 Q tiles or distinct mask planes");
+    // (part of the contract; the kernel keeps the tiles' states in LDS and does not touch it)
     const size_t need = sa_mask_terms_workspace_bytes(uB, Sq, Sk, BQ, BK);
     if (!workspace || workspace_bytes < need)
         return fail(SA_ERR_WORKSPACE, "sa_mask_classify_terms: workspace of %zu bytes required, %zu given", need,
@@ -697,44 +698,27 @@ int sa_mask_classify_terms(const int32_t *terms, int n_terms, const int32_t *doc
     tp.BQ = BQ;
     tp.BK = BK;
     tp.nQ = nQ;
+    tp.lbk = lbk;
     tp.nK = nK;
-    tp.cls = static_cast<uint8_t *>(workspace);
-    hipError_t e = sa::launch_classify_terms(tp, static_cast<hipStream_t>(stream));
-    if (e != hipSuccess) return fail(SA_ERR_HIP, "sa_mask_classify_terms: classify launch failed: %s", hipGetErrorString(e));
-
-    sa::CompactParams kp{};
-    kp.cls = tp.cls;
-    kp.uH = 1;
-    kp.bcast_b = !per_batch;
-    kp.bcast_h = true;
-    kp.oB = (B > 1 && zb == 4) ? 1 : B;
-    kp.oH = (H > 1 && zh == 4) ? 1 : H;
-    kp.nQ = nQ;
-    kp.nK = nK;
-    kp.full_ids = full_ids;
-    kp.full_lens = full_lens;
-    kp.part_ids = part_ids;
-    kp.part_lens = part_lens;
-    for (int i = 0; i < 4; i++) {
-        kp.fis[i] = full_ids_strides[i];
-        kp.pis[i] = part_ids_strides[i];
-    }
-    for (int i = 0; i < 3; i++) {
-        kp.fls[i] = full_lens_strides[i];
-        kp.pls[i] = part_lens_strides[i];
-    }
-    e = sa::launch_compact(kp, static_cast<hipStream_t>(stream));
-    if (e != hipSuccess) return fail(SA_ERR_HIP, "sa_mask_classify_terms: compaction launch failed: %s", hipGetErrorString(e));
-    if (!packed) return SA_OK;
-
+    tp.oB_all = !per_batch;
+    tp.oB = (B > 1 && zb == 4) ? 1 : B;
+    tp.oH = (H > 1 && zh == 4) ? 1 : H;
+    tp.full_ids = full_ids;
+    tp.full_lens = full_lens;
     tp.part_ids = part_ids;
     tp.part_lens = part_lens;
-    for (int i = 0; i < 4; i++) tp.pis[i] = part_ids_strides[i];
-    for (int i = 0; i < 3; i++) tp.pls[i] = part_lens_strides[i];
+    for (int i = 0; i < 4; i++) {
+        tp.fis[i] = full_ids_strides[i];
+        tp.pis[i] = part_ids_strides[i];
+    }
+    for (int i = 0; i < 3; i++) {
+        tp.fls[i] = full_lens_strides[i];
+        tp.pls[i] = part_lens_strides[i];
+    }
     tp.packed = packed;
-    tp.ob = packed_strides[0];
-    e = sa::launch_pack_terms(tp, static_cast<hipStream_t>(stream));
-    if (e != hipSuccess) return fail(SA_ERR_HIP, "sa_mask_classify_terms: packing launch failed: %s", hipGetErrorString(e));
+    tp.ob = packed ? packed_strides[0] : 0;
+    const hipError_t e = sa::launch_mask_terms(tp, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(SA_ERR_HIP, "sa_mask_classify_terms: launch failed: %s", hipGetErrorString(e));
     return SA_OK;
 }
 

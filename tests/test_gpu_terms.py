@@ -180,3 +180,23 @@ def test_seeded_random_terms(gpu, seed):
     same_metadata(md, want, BQ, BK)
     m_or = oracle.mask_from_terms([t.encode() for t in terms], B, Sq, Sk, dq.cpu().numpy(), dk.cpu().numpy())
     assert np.array_equal(m_or, mask.expand(B, 1, Sq, Sk)[:, 0].cpu().numpy())
+
+
+@pytest.mark.parametrize("Sq,Sk,BQ,BK", [(96, 196608, 48, 16), (96, 196608, 48, 64), (32, 262144, 16, 131072),
+                                         (65, 2112, 1, 16), (130, 1088, 65, 64), (200, 640, 200, 128)])
+def test_long_rows_wide_tiles_and_odd_row_counts(gpu, Sq, Sk, BQ, BK):
+    """More tiles per Q tile than one pass over them holds, a tile wider than that, row counts that are no multiple of a
+    wave, documents in no order: lists and packed tiles as from the materialised mask."""
+    B, H = 2, 2
+    g = torch.Generator().manual_seed(Sk + BQ)
+    dk = torch.randint(0, 3, (B, Sk // 16), generator=g, dtype=torch.int32).repeat_interleave(16, 1)
+    dk[:, : Sk // 2] = torch.div(torch.arange(Sk // 2), 300, rounding_mode="floor").to(torch.int32)
+    dk = dk.to(gpu)
+    dq = dk[:, Sk - Sq:].contiguous()
+    terms = [MaskTerm(ahead=1, offset=Sk - Sq, same_doc=True), MaskTerm(back=Sk // 3, ahead=9, offset=Sk // 2),
+             block_term((1, Sq // 2), (Sk // 4, Sk // 4 + BK + 7))]
+    md = compute_mask_terms(terms, B, H, Sq, Sk, BQ, BK, dq, dk)
+    mask = materialize_mask_terms(terms, B, Sq, Sk, dq, dk, device=gpu).expand(B, H, Sq, Sk)
+    want = compute_mask_kernel(mask, BQ, BK, pack_partial=True)
+    assert int(want.masked_lens.sum()) > 0
+    same_metadata(md, want, BQ, BK)
