@@ -38,7 +38,7 @@
 extern "C" {
 #endif
 
-#define SA_ABI_VERSION 14
+#define SA_ABI_VERSION 15
 
 enum sa_status {
     SA_OK = 0,
@@ -343,6 +343,26 @@ int sa_sparse_attention_fwd_kernel(const void *q, const int64_t q_strides[4], co
                                    const int64_t packed_strides[2], float *lse, const int64_t lse_strides[3], int B,
                                    int H, int Sq, int Sk, int D, int BQ, int BK, int dtype, float sm_scale_log2,
                                    int kernel, void *stream);
+
+/*
+ * The same forward for launches with too few Q tiles to fill the device (a chunk of a prompt against a long cache): the
+ * list of a Q tile is shared by several workgroups and their partial results are added up by a second launch.
+ *   workspace   sa_fwd_split_workspace_bytes(...) bytes of device memory, 16-byte aligned; may be NULL when that is 0,
+ *               which says that the launch has no use for it (the call is then sa_sparse_attention_fwd_kernel with the
+ *               default kernel).  The bytes depend on the current device.
+ * Results agree with the default kernel within rounding (a row's keys are added up in other groups).
+ */
+size_t sa_fwd_split_workspace_bytes(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype);
+int sa_sparse_attention_fwd_split(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
+                                  const void *v, const int64_t v_strides[4], void *o, const int64_t o_strides[4],
+                                  const uint8_t *mask, const int64_t mask_strides[4], const int32_t *full_ids,
+                                  const int64_t full_ids_strides[4], const int32_t *full_lens,
+                                  const int64_t full_lens_strides[3], const int32_t *part_ids,
+                                  const int64_t part_ids_strides[4], const int32_t *part_lens,
+                                  const int64_t part_lens_strides[3], const uint8_t *packed,
+                                  const int64_t packed_strides[2], float *lse, const int64_t lse_strides[3], int B,
+                                  int H, int Sq, int Sk, int D, int BQ, int BK, int dtype, float sm_scale_log2,
+                                  void *workspace, size_t workspace_bytes, void *stream);
 
 /*
  * The forward for few query rows against a long K/V (decode): Sq <= 32 rows form the single Q tile of every (b, h),

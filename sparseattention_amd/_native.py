@@ -10,7 +10,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libsparseattn_hip.so")
 
-SA_ABI_VERSION = 14
+SA_ABI_VERSION = 15
 SA_OK = 0
 SA_ERR_INVALID_ARGUMENT = -1
 SA_ERR_UNSUPPORTED = -2
@@ -44,6 +44,8 @@ EXPORTS = (
     "sa_sparse_attention_fwd_ex",
     "sa_sparse_attention_fwd_lse",
     "sa_sparse_attention_fwd_kernel",
+    "sa_fwd_split_workspace_bytes",
+    "sa_sparse_attention_fwd_split",
     "sa_decode_num_splits",
     "sa_decode_workspace_bytes",
     "sa_sparse_attention_decode",
@@ -125,6 +127,13 @@ def load() -> ctypes.CDLL:
     lib.sa_sparse_attention_fwd_kernel.argtypes = (
         [_vp, _i64p] * 4 + [_vp, _i64p] + [_vp, _i64p] * 4 + [_vp, _i64p] + [_vp, _i64p] + [ctypes.c_int] * 8
         + [ctypes.c_float, ctypes.c_int, _vp]
+    )
+    lib.sa_fwd_split_workspace_bytes.restype = ctypes.c_size_t
+    lib.sa_fwd_split_workspace_bytes.argtypes = [ctypes.c_int] * 8
+    lib.sa_sparse_attention_fwd_split.restype = ctypes.c_int
+    lib.sa_sparse_attention_fwd_split.argtypes = (
+        [_vp, _i64p] * 4 + [_vp, _i64p] + [_vp, _i64p] * 4 + [_vp, _i64p] + [_vp, _i64p] + [ctypes.c_int] * 8
+        + [ctypes.c_float] + [_vp, ctypes.c_size_t] + [_vp]
     )
     lib.sa_sparse_attention_decode.argtypes = (
         [_vp, _i64p] * 4 + [_vp, _i64p] + [_vp, _i64p] * 4 + [ctypes.c_int] * 7 + [ctypes.c_float, ctypes.c_int]

@@ -24,11 +24,11 @@ UNITS = [("sparseattn_api.hip", "sparseattn_api.o", []), ("mask_classify.hip", "
          ("mask_terms.hip", "mask_terms.o", []),
          ("fwd_schedule.hip", "fwd_schedule.o", []), ("sparse_fwd.hip", "sparse_fwd.o", []),
          ("sparse_fwd_f32.hip", "sparse_fwd_f32.o", []), ("sparse_fwd_c32.hip", "sparse_fwd_c32.o", []),
-         ("sparse_fwd_f32_mfma.hip", "sparse_fwd_f32_mfma.o", []),
+         ("sparse_fwd_f32_mfma.hip", "sparse_fwd_f32_mfma.o", []), ("sparse_fwd_merge.hip", "sparse_fwd_merge.o", []),
          ("sparse_decode.hip", "sparse_decode.o", []), ("sparse_bwd.hip", "sparse_bwd.o", [])]
-UNITS += [("sparse_fwd_inst.hip", f"sparse_fwd_dt{dt}_pk{pk}_ps{ps}.o",
-           [f"-DSA_FWD_DT={dt}", f"-DSA_FWD_PK={pk}", f"-DSA_FWD_PS={ps}"])
-          for dt in (0, 1) for pk in (0, 1) for ps in (0, 1)]
+UNITS += [("sparse_fwd_inst.hip", f"sparse_fwd_dt{dt}_pk{pk}_how{how}.o",
+           [f"-DSA_FWD_DT={dt}", f"-DSA_FWD_PK={pk}", f"-DSA_FWD_HOW={how}"])
+          for dt in (0, 1) for pk in (0, 1) for how in (0, 1, 2)]
 
 # -packed-fp32-ops is switched off on purpose: the compiler must not form v_pk_*_f32 from float code.
 HIPCC_FLAGS = [

@@ -133,9 +133,24 @@ __device__ __forceinline__ void dma16(const void *base, uint32_t lane_offset, ui
 // memory round trip each; at the start of a Q tile that is most of the time before the first K/V request.
 template <int N>
 __device__ __forceinline__ void scalar_gather(const int32_t *const (&a)[N], int (&o)[N]) {
-    static_assert(N == 4 || N == 6 || N == 10, "counts + first slots of both lists for 1, 2 or 4 entries per chunk");
+    static_assert(N == 2 || N == 4 || N == 6 || N == 8 || N == 10,
+                  "counts, first slots of both lists for 1, 2 or 4 entries per chunk, or both");
     const uint64_t *const q = reinterpret_cast<const uint64_t *>(&a[0]);  // (pointers as 64-bit scalars)
-    if constexpr (N == 4) {
+    if constexpr (N == 2) {
+        asm volatile(
+            "s_load_dword %0, %2, 0x0\n\ts_load_dword %1, %3, 0x0\n\ts_waitcnt lgkmcnt(0)"
+            : "=&s"(o[0]), "=&s"(o[1])
+            : "s"(q[0]), "s"(q[1])
+            : "memory");
+    } else if constexpr (N == 8) {
+        asm volatile(
+            "s_load_dword %0, %8, 0x0\n\ts_load_dword %1, %9, 0x0\n\ts_load_dword %2, %10, 0x0\n\t"
+            "s_load_dword %3, %11, 0x0\n\ts_load_dword %4, %12, 0x0\n\ts_load_dword %5, %13, 0x0\n\t"
+            "s_load_dword %6, %14, 0x0\n\ts_load_dword %7, %15, 0x0\n\ts_waitcnt lgkmcnt(0)"
+            : "=&s"(o[0]), "=&s"(o[1]), "=&s"(o[2]), "=&s"(o[3]), "=&s"(o[4]), "=&s"(o[5]), "=&s"(o[6]), "=&s"(o[7])
+            : "s"(q[0]), "s"(q[1]), "s"(q[2]), "s"(q[3]), "s"(q[4]), "s"(q[5]), "s"(q[6]), "s"(q[7])
+            : "memory");
+    } else if constexpr (N == 4) {
         asm volatile(
             "s_load_dword %0, %4, 0x0\n\ts_load_dword %1, %5, 0x0\n\ts_load_dword %2, %6, 0x0\n\t"
             "s_load_dword %3, %7, 0x0\n\ts_waitcnt lgkmcnt(0)"

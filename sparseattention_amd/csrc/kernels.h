@@ -127,7 +127,32 @@ struct FwdParams {
     // (-inf for rows without one), or null.
     float *lse;
     int64_t lses[3];  // b, h, row strides in elements
+    // Lists shared by up to nsplit > 1 workgroups each (fwd_split_share), or nsplit <= 1: the workgroups' partial results,
+    //   ws    [B*H*nQ][nsplit][BQ/32][D/8][64 lanes][4] floats: unnormalised rows in the order the registers hold them
+    //   ws_ml [B*H*nQ][nsplit][BQ][2] floats: reference value (-inf: no attended key) and sum of every row
+    int nsplit, split_chunks;  // split_chunks: chunks of one part (the last ones may be shorter)
+    float *ws, *ws_ml;
 };
+
+// How many workgroups share a list of NE entries of 2^lbk keys, walked in chunks of 2^lck keys, and the first entry of
+// part s of them (s = share: the end of the list).  Entries of one chunk stay together.
+__host__ __device__ inline int fwd_split_share(int NE, int lbk, int lck, int split_chunks, int nsplit) {
+    const int le = lck > lbk ? lck - lbk : 0, lc = lbk > lck ? lbk - lck : 0;
+    const int groups = (NE + (1 << le) - 1) >> le;
+    const int parts = ((groups << lc) + split_chunks - 1) / split_chunks;
+    const int most = groups < nsplit ? groups : nsplit;
+    return parts < most ? (parts > 1 ? parts : 1) : (most > 1 ? most : 1);
+}
+__host__ __device__ inline int fwd_split_first(int NE, int lbk, int lck, int s, int share) {
+    const int le = lck > lbk ? lck - lbk : 0;
+    const unsigned groups = (unsigned)(NE + (1 << le) - 1) >> le;
+    const int e = (int)(groups * (unsigned)s / (unsigned)share) << le;
+    return e < NE ? e : NE;
+}
+// The rule for nsplit and split_chunks: sparse_fwd_merge.hip.
+void fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus, int *nsplit, int *split_chunks);
+// Adds up the parts of shared lists (dtype 2: float32 output).
+hipError_t launch_fwd_merge(const FwdParams &p, int dtype, int D, int BQ, hipStream_t stream);
 
 // dtype: 0 bf16, 1 fp16.  Returns hipErrorInvalidValue when no instantiation matches (D, BQ).
 hipError_t launch_fwd(const FwdParams &p, int dtype, int D, int BQ, hipStream_t stream);

@@ -4,26 +4,28 @@
 
 namespace sa {
 
-template <int DT, bool PK, bool PS>
+template <int DT, bool PK, int HOW>
 hipError_t launch_fwd_variant(const FwdParams &p, int D, int BQ, hipStream_t stream);
-#define SA_DECL(DT, PK, PS) \
-    extern template hipError_t launch_fwd_variant<DT, PK, PS>(const FwdParams &, int, int, hipStream_t);
-SA_DECL(0, false, false) SA_DECL(0, false, true) SA_DECL(0, true, false) SA_DECL(0, true, true)
-SA_DECL(1, false, false) SA_DECL(1, false, true) SA_DECL(1, true, false) SA_DECL(1, true, true)
+#define SA_DECL(DT, PK, HOW) \
+    extern template hipError_t launch_fwd_variant<DT, PK, HOW>(const FwdParams &, int, int, hipStream_t);
+SA_DECL(0, false, 0) SA_DECL(0, false, 1) SA_DECL(0, false, 2) SA_DECL(0, true, 0) SA_DECL(0, true, 1) SA_DECL(0, true, 2)
+SA_DECL(1, false, 0) SA_DECL(1, false, 1) SA_DECL(1, false, 2) SA_DECL(1, true, 0) SA_DECL(1, true, 1) SA_DECL(1, true, 2)
 #undef SA_DECL
 
 namespace {
-template <int DT>
-hipError_t by_flags(const FwdParams &p, int D, int BQ, hipStream_t stream) {
-    const bool pk = p.packed != nullptr, ps = p.sched != nullptr;
-    if (pk) return ps ? launch_fwd_variant<DT, true, true>(p, D, BQ, stream) : launch_fwd_variant<DT, true, false>(p, D, BQ, stream);
-    return ps ? launch_fwd_variant<DT, false, true>(p, D, BQ, stream) : launch_fwd_variant<DT, false, false>(p, D, BQ, stream);
+template <int DT, bool PK>
+hipError_t by_hand_out(const FwdParams &p, int D, int BQ, hipStream_t stream) {
+    if (p.sched != nullptr) return launch_fwd_variant<DT, PK, 1>(p, D, BQ, stream);
+    if (p.nsplit <= 1) return launch_fwd_variant<DT, PK, 0>(p, D, BQ, stream);
+    const hipError_t e = launch_fwd_variant<DT, PK, 2>(p, D, BQ, stream);
+    return e != hipSuccess ? e : launch_fwd_merge(p, DT, D, BQ, stream);
 }
 }  // namespace
 
 hipError_t launch_fwd(const FwdParams &p, int dtype, int D, int BQ, hipStream_t stream) {
-    if (dtype == 0) return by_flags<0>(p, D, BQ, stream);
-    if (dtype == 1) return by_flags<1>(p, D, BQ, stream);
+    const bool pk = p.packed != nullptr;
+    if (dtype == 0) return pk ? by_hand_out<0, true>(p, D, BQ, stream) : by_hand_out<0, false>(p, D, BQ, stream);
+    if (dtype == 1) return pk ? by_hand_out<1, true>(p, D, BQ, stream) : by_hand_out<1, false>(p, D, BQ, stream);
     return hipErrorInvalidValue;
 }
 

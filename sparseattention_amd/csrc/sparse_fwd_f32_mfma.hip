@@ -77,10 +77,14 @@ __global__ __launch_bounds__(NW * 64, NW >= 4 ? 2 : 1) void sparse_fwd_f32_mfma_
     // in turn; the remap gives every XCD whole planes (so that the Q tiles sharing a K/V plane meet in one L2 and every
     // XCD gets the same mix of long and short lists), planes two at a time with their Q tiles interleaved, last Q tile
     // first.
-    int b, h, qt;
+    int b, h, qt, s0 = 0;  // s0: this workgroup's part of a shared list
     {
-        const int total = gridDim.x, per = total >> 3;
+        const int total = p.nQ * p.B * p.H, per = total >> 3;
         int lin = blockIdx.x;
+        if (p.nsplit > 1) {  // the first parts of all tiles, then the second ones, ...
+            s0 = lin / total;
+            lin -= s0 * total;
+        }
         if (lin < (per << 3)) lin = (lin & 7) * per + (lin >> 3);
         int pair = lin / (2 * p.nQ);
         const int r = lin - pair * 2 * p.nQ;
@@ -99,10 +103,21 @@ __global__ __launch_bounds__(NW * 64, NW >= 4 ? 2 : 1) void sparse_fwd_f32_mfma_
 
     const float *const kbase = reinterpret_cast<const float *>(p.k) + b * p.ks[0] + h * p.ks[1];
     const float *const vbase = reinterpret_cast<const float *>(p.v) + b * p.vs[0] + h * p.vs[1];
-    const int32_t *const fid = p.full_ids + b * p.fis[0] + h * p.fis[1] + qt * p.fis[2];
-    const int32_t *const pid = p.part_ids + b * p.pis[0] + h * p.pis[1] + qt * p.pis[2];
-    const int F = min(min(max(p.full_lens[b * p.fls[0] + h * p.fls[1] + qt * p.fls[2]], 0), p.nK), kF32ListCap);
-    const int NE = F + min(min(max(p.part_lens[b * p.pls[0] + h * p.pls[1] + qt * p.pls[2]], 0), p.nK - F), kF32ListCap - F);
+    const int32_t *fid = p.full_ids + b * p.fis[0] + h * p.fis[1] + qt * p.fis[2];
+    const int32_t *pid = p.part_ids + b * p.pis[0] + h * p.pis[1] + qt * p.pis[2];
+    int F = min(min(max(p.full_lens[b * p.fls[0] + h * p.fls[1] + qt * p.fls[2]], 0), p.nK), kF32ListCap);
+    int NE = F + min(min(max(p.part_lens[b * p.pls[0] + h * p.pls[1] + qt * p.pls[2]], 0), p.nK - F), kF32ListCap - F);
+    int share = 1, p_lo = 0;
+    if (p.nsplit > 1) {
+        share = fwd_split_share(NE, p.lbk, 5, p.split_chunks, p.nsplit);
+        if (s0 >= share) return;
+        const int e_lo = fwd_split_first(NE, p.lbk, 5, s0, share), e_hi = fwd_split_first(NE, p.lbk, 5, s0 + 1, share);
+        fid += (int64_t)min(e_lo, F) * p.fis[3];
+        p_lo = max(e_lo - F, 0);
+        pid += (int64_t)p_lo * p.pis[3];
+        F = min(max(F - e_lo, 0), e_hi - e_lo);
+        NE = e_hi - e_lo;
+    }
     const int T = MODE == 2 ? (NE << (p.lbk - 5)) : ((NE + EPC - 1) / EPC);
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const SA_LDS uint8_t *)smem);
 
@@ -126,7 +141,7 @@ __global__ __launch_bounds__(NW * 64, NW >= 4 ? 2 : 1) void sparse_fwd_f32_mfma_
     const int ld_r = lane / PPR, ld_slot = lane % PPR;
     const int64_t ld_kbase = ((int64_t)ld_r * p.ks[2]) * 4, ld_vbase = ((int64_t)ld_r * p.vs[2]) * 4;
     const int64_t tile_bytes = (int64_t)(NW * 4) * p.BK;
-    const uint8_t *const pbase = PK ? p.packed + b * p.pks[0] + h * p.pks[1] + (int64_t)qt * p.nK * tile_bytes : nullptr;
+    const uint8_t *const pbase = PK ? p.packed + b * p.pks[0] + h * p.pks[1] + ((int64_t)qt * p.nK + p_lo) * tile_bytes : nullptr;
     const uint8_t *const mrow0 = PK ? nullptr : p.mask + b * p.ms[0] + h * p.ms[1] + (int64_t)(qt * (NW * 32)) * p.ms[2];
 
     struct Plan {
@@ -320,6 +335,17 @@ __global__ __launch_bounds__(NW * 64, NW >= 4 ? 2 : 1) void sparse_fwd_f32_mfma_
         const uint32_t lu = __float_as_uint(l_i);
         const auto sw = __builtin_amdgcn_permlane32_swap(lu, lu, false, false);
         const float l_tot = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+        if (share > 1) {
+            const int64_t part_id = ((int64_t)(b * p.H + h) * p.nQ + qt) * p.nsplit + s0;
+            float *const wo = p.ws + (part_id * NW + wave_u) * (32 * D) + 4 * lane;
+#pragma unroll
+            for (int db = 0; db < D / 32; db++)
+#pragma unroll
+                for (int g = 0; g < 4; g++)
+                    *(f32x4 *)(wo + 256 * (4 * db + g)) = f32x4{acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]};
+            if (hh == 0) *(f32x2 *)(p.ws_ml + 2 * (part_id * (NW * 32) + wave * 32 + l32)) = f32x2{m_i, l_tot};
+            return;
+        }
         const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
         if (p.lse != nullptr && hh == 0)
             p.lse[b * p.lses[0] + h * p.lses[1] + (int64_t)qrow * p.lses[2]] =
@@ -342,7 +368,8 @@ hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     auto kern = sparse_fwd_f32_mfma_kernel<D, NW, MODE, PK>;
     static unsigned long long attr_done = 0;
     if (const hipError_t e0 = allow_dynamic_smem(kern, smem, attr_done); e0 != hipSuccess) return e0;
-    hipLaunchKernelGGL(kern, dim3((unsigned)p.nQ * (unsigned)(p.B * p.H)), dim3(NW * 64), smem, stream, p);
+    hipLaunchKernelGGL(kern, dim3((unsigned)p.nQ * (unsigned)(p.B * p.H) * (unsigned)(p.nsplit > 1 ? p.nsplit : 1)),
+                       dim3(NW * 64), smem, stream, p);
     return hipGetLastError();
 }
 
@@ -383,8 +410,9 @@ bool fwd_f32_mfma_has(const FwdParams &p, int D, int BQ) {
 
 hipError_t launch_fwd_f32_mfma(const FwdParams &p, int D, int BQ, hipStream_t stream) {
     if (!fwd_f32_mfma_has(p, D, BQ)) return hipErrorInvalidValue;
-    if (p.packed != nullptr) return D == 64 ? launch_bq<64, true>(p, BQ, stream) : launch_bq<128, true>(p, BQ, stream);
-    return D == 64 ? launch_bq<64, false>(p, BQ, stream) : launch_bq<128, false>(p, BQ, stream);
+    const hipError_t e = p.packed != nullptr ? (D == 64 ? launch_bq<64, true>(p, BQ, stream) : launch_bq<128, true>(p, BQ, stream))
+                                             : (D == 64 ? launch_bq<64, false>(p, BQ, stream) : launch_bq<128, false>(p, BQ, stream));
+    return e != hipSuccess || p.nsplit <= 1 ? e : launch_fwd_merge(p, 2, D, BQ, stream);
 }
 
 }  // namespace sa

@@ -66,9 +66,14 @@ __device__ __forceinline__ void wait_vm_at_most(int n, int step) {
 // chunk of one tile is computed, the first chunk of the next is fetched and its queries are loaded, and the
 // lists of the tiles after that are on their way, so that the latencies a fresh workgroup would pay one after
 // the other (arguments, counts, lists, first K/V chunk) are paid once per workgroup instead of once per tile.
-template <int DT, int D, int NW, int MODE, int NS, bool PP, bool PK, bool PS>
+// SP: the list of a Q tile is shared by up to p.nsplit workgroups (fwd_split_share), for launches with too few Q tiles to
+// fill the device: a chunk of a prompt against a long cache.  Every workgroup walks a range of its own and leaves
+// unnormalised rows with their reference values and sums in p.ws, which fwd_merge_kernel adds up; a tile whose list is
+// too short to be shared is written as by the plain kernel.
+template <int DT, int D, int NW, int MODE, int NS, bool PP, bool PK, bool PS, bool SP>
 __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse_fwd_kernel(const FwdParams p) {
     static_assert(!PS || (!PP && NS == 2), "persistent workgroups use the two-stage loop");
+    static_assert(!SP || (!PS && !PP && D <= 128), "shared lists use the plain loop");
     using E = Elem<DT>;
     constexpr int ROWB = D * 2;                   // bytes per K/V row in LDS
     constexpr int KBUF = 64 * ROWB, VBUF = 64 * ROWB;
@@ -171,6 +176,7 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
     // {(b << 16) | h, qt, F, P} per Q tile.
     const int4 *const sched_row = reinterpret_cast<const int4 *>(p.sched) + (int64_t)blockIdx.x * (p.sched_R + 1);
     int n_items = 1;
+    int share = 1, share_part = 0;  // workgroups that share this Q tile's list, and which of their parts this one is
     if constexpr (PS) {
         n_items = __builtin_amdgcn_readfirstlane(sched_row[0].x);
         if (n_items <= 0) return;
@@ -179,8 +185,13 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
         set_item(bh0 >> 16, bh0 & 0xffff, __builtin_amdgcn_readfirstlane(e0.y), __builtin_amdgcn_readfirstlane(e0.z),
                  __builtin_amdgcn_readfirstlane(e0.w));
     } else {
-        const int total = gridDim.x, per = total >> 3;
-        int lin = blockIdx.x;
+        // (shared lists: the first parts of all tiles, then the second ones, ...; parts that turn out empty come last)
+        const int total = SP ? p.nQ * p.B * p.H : gridDim.x, per = total >> 3;
+        int lin = blockIdx.x, s0 = 0;
+        if constexpr (SP) {
+            s0 = lin / total;
+            lin -= s0 * total;
+        }
         if (lin < (per << 3)) lin = (lin & 7) * per + (lin >> 3);
         int pair = lin / (2 * p.nQ);
         const int r = lin - pair * 2 * p.nQ;
@@ -202,7 +213,39 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
         // past a count hold anything; early_entry() picks the ones that count.
         const int32_t *const fl0 = p.full_lens + (b0 * p.fls[0] + h0 * p.fls[1] + qt0 * p.fls[2]);
         const int32_t *const pl0 = p.part_lens + (b0 * p.pls[0] + h0 * p.pls[1] + qt0 * p.pls[2]);
-        if constexpr (kEarlyFirstChunk) {
+        if constexpr (SP) {
+            // (the counts say where this workgroup's part of the list begins, so they come by a round trip of their own)
+            load_q(b0, h0, qt0);
+            int cnt[2];
+            const int32_t *const cnt_addr[2] = {fl0, pl0};
+            scalar_gather(cnt_addr, cnt);
+            set_item(b0, h0, qt0, cnt[0], cnt[1]);
+            share = fwd_split_share(NE, p.lbk, 6, p.split_chunks, p.nsplit);
+            share_part = s0;
+            if (s0 >= share) return;
+            const int e_lo = fwd_split_first(NE, p.lbk, 6, s0, share), e_hi = fwd_split_first(NE, p.lbk, 6, s0 + 1, share);
+            const int f_lo = min(e_lo, F), p_lo = max(e_lo - F, 0);
+            fid += f_lo * p.fis[3];
+            pid += p_lo * p.pis[3];
+            prow += p_lo * tile_bytes;
+            const int f_left = p.nK - 1 - f_lo, p_left = p.nK - 1 - p_lo;  // slots behind the first one (>= -1: empty list)
+            F = min(max(F - e_lo, 0), e_hi - e_lo);
+            NE = e_hi - e_lo;
+            T = chunks_of(NE);
+            const int32_t *addr[2 * EPC];
+            int got[2 * EPC];
+            static_for<EPC>([&](auto i_c) {
+                constexpr int i = decltype(i_c)::value;
+                addr[i] = fid + (int64_t)min(i, f_left) * p.fis[3];
+                addr[EPC + i] = pid + (int64_t)min(i, p_left) * p.pis[3];
+            });
+            scalar_gather(addr, got);
+            static_for<EPC>([&](auto i_c) {
+                constexpr int i = decltype(i_c)::value;
+                early_f[i] = got[i];
+                early_p[i] = got[EPC + i];
+            });
+        } else if constexpr (kEarlyFirstChunk) {
             load_q(b0, h0, qt0);
             const int32_t *f0 = p.full_ids + b0 * p.fis[0] + h0 * p.fis[1] + qt0 * p.fis[2];
             const int32_t *p0 = p.part_ids + b0 * p.pis[0] + h0 * p.pis[1] + qt0 * p.pis[2];
@@ -1140,42 +1183,60 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
     }
 
     if constexpr (PP) __syncthreads();  // the late waves of the ping-pong schedule have read their last stage
+    if constexpr (SP) {
+        if (share > 1) {
+            // in the order the registers hold them: whole 1 KiB runs per store instruction (fwd_merge_kernel reads them so)
+            const int64_t part_id = ((int64_t)(b * p.H + h) * p.nQ + qt) * p.nsplit + share_part;
+            float *const wo = p.ws + (part_id * NW + wave_u) * (32 * D) + 4 * lane;
+#pragma unroll
+            for (int db = 0; db < D / 32; db++)
+#pragma unroll
+                for (int g = 0; g < 4; g++)
+                    *(f32x4 *)(wo + 256 * (4 * db + g)) = f32x4{acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]};
+            if (hh == 0)
+                *(f32x2 *)(p.ws_ml + 2 * (part_id * (NW * 32) + wave * 32 + l32)) =
+                    f32x2{raise_above == kMaxSlack ? m_ref : kNegInf, l32 < 16 ? acc_l[0] : acc_l[1]};
+            return;
+        }
+    }
     store_o_rows();
 }
 
-template <int DT, int D, int NW, int MODE, bool PK, bool PS>
+// HOW 0: one workgroup per Q tile, 1: persistent workgroups, 2: lists shared by workgroups (SP)
+template <int DT, int D, int NW, int MODE, bool PK, int HOW>
 hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     // Eight waves fill a CU's register file on their own, so that workgroup can have most of the LDS: 4 stages.
     constexpr int NS = NW == 8 ? 4 : 2;
     static_assert(kListCap == 2 * kPsListCap, "one long list or two short ones in the same LDS");
     constexpr int smem = 2 * NS * 64 * D * 2 + kListCap * 4;  // NS stages of 64 rows for K and for V + the list(s)
-    auto kern = sparse_fwd_kernel<DT, D, NW, MODE, NS, NW == 8, PK, PS>;
+    auto kern = sparse_fwd_kernel<DT, D, NW, MODE, NS, NW == 8, PK, HOW == 1, HOW == 2>;
     static unsigned long long attr_done = 0;  // devices on which this kernel may use `smem` bytes of LDS
     if (const hipError_t e0 = allow_dynamic_smem(kern, smem, attr_done); e0 != hipSuccess) return e0;
-    const unsigned grid = PS ? (unsigned)p.sched_G : (unsigned)p.nQ * (unsigned)p.B * (unsigned)p.H;
+    const unsigned grid = HOW == 1 ? (unsigned)p.sched_G
+                                   : (unsigned)p.nQ * (unsigned)p.B * (unsigned)p.H * (HOW == 2 ? (unsigned)p.nsplit : 1u);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(NW * 64), smem, stream, p);
     return hipGetLastError();
 }
 
-template <int DT, int D, int NW, bool PK, bool PS>
+template <int DT, int D, int NW, bool PK, int HOW>
 hipError_t launch_mode(const FwdParams &p, hipStream_t stream) {
-    if (p.BK == 16) return launch_one<DT, D, NW, 0, PK, PS>(p, stream);
-    if (p.BK == 32) return launch_one<DT, D, NW, 1, PK, PS>(p, stream);
-    return launch_one<DT, D, NW, 2, PK, PS>(p, stream);
+    if (p.BK == 16) return launch_one<DT, D, NW, 0, PK, HOW>(p, stream);
+    if (p.BK == 32) return launch_one<DT, D, NW, 1, PK, HOW>(p, stream);
+    return launch_one<DT, D, NW, 2, PK, HOW>(p, stream);
 }
 
-template <int DT, int D, bool PK, bool PS>
+template <int DT, int D, bool PK, int HOW>
 hipError_t launch_bq(const FwdParams &p, int BQ, hipStream_t stream) {
     switch (BQ) {
         case 32:
             if constexpr (D > 128) return hipErrorInvalidValue;  // a lone wave would spill its registers there
-            else return launch_mode<DT, D, 1, PK, PS>(p, stream);
-        case 64: return launch_mode<DT, D, 2, PK, PS>(p, stream);
-        case 128: return launch_mode<DT, D, 4, PK, PS>(p, stream);
+            else return launch_mode<DT, D, 1, PK, HOW>(p, stream);
+        case 64: return launch_mode<DT, D, 2, PK, HOW>(p, stream);
+        case 128: return launch_mode<DT, D, 4, PK, HOW>(p, stream);
         case 256:
-            // 8-wave workgroups are not persistent, and their four stages do not fit the LDS at D = 256
-            if constexpr (PS || D > 128) return hipErrorInvalidValue;
-            else return launch_mode<DT, D, 8, PK, false>(p, stream);
+            // 8-wave workgroups are neither persistent nor share lists, and their four stages do not fit the LDS at D = 256
+            if constexpr (HOW != 0 || D > 128) return hipErrorInvalidValue;
+            else return launch_mode<DT, D, 8, PK, 0>(p, stream);
         default: return hipErrorInvalidValue;
     }
 }
@@ -1184,17 +1245,17 @@ hipError_t launch_bq(const FwdParams &p, int BQ, hipStream_t stream) {
 
 // Every kernel for one element type, one source of the PARTIAL tiles' mask entries and one way of handing out
 // Q tiles.  Each combination is instantiated in a translation unit of its own (sparse_fwd_inst.hip compiled
-// with SA_FWD_DT / SA_FWD_PK / SA_FWD_PS).
-template <int DT, bool PK, bool PS>
+// with SA_FWD_DT / SA_FWD_PK / SA_FWD_HOW).
+template <int DT, bool PK, int HOW>
 hipError_t launch_fwd_variant(const FwdParams &p, int D, int BQ, hipStream_t stream) {
     switch (D) {
-        case 64: return launch_bq<DT, 64, PK, PS>(p, BQ, stream);
-        case 128: return launch_bq<DT, 128, PK, PS>(p, BQ, stream);
+        case 64: return launch_bq<DT, 64, PK, HOW>(p, BQ, stream);
+        case 128: return launch_bq<DT, 128, PK, HOW>(p, BQ, stream);
         case 256:
             // one workgroup per CU (its two stages of K and V take 128 KiB of LDS) with the whole register file:
-            // one wave per SIMD; no schedules
-            if constexpr (PS) return hipErrorInvalidValue;
-            else return launch_bq<DT, 256, PK, false>(p, BQ, stream);
+            // one wave per SIMD; no schedules, no shared lists
+            if constexpr (HOW != 0) return hipErrorInvalidValue;
+            else return launch_bq<DT, 256, PK, 0>(p, BQ, stream);
         default: return hipErrorInvalidValue;
     }
 }

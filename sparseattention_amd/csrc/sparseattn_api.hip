@@ -239,6 +239,20 @@ size_t schedule_shape(int B, int H, int Sq, int Sk, int BQ, int BK, int mode, in
     return (size_t)G * (size_t)(R + 1) * 16;
 }
 
+// Parts of a shared list and chunks per part on the current device (1: no sharing), and the bytes of the partial results.
+size_t split_shape(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype, int *nsplit, int *split_chunks) {
+    *nsplit = 1;
+    *split_chunks = 1 << 30;
+    if (B <= 0 || H <= 0 || Sq <= 0 || Sk <= 0 || BQ <= 0 || BK <= 0 || Sq % BQ || Sk % BK || log2_exact(BK) < 4) return 0;
+    const int64_t tiles = (int64_t)B * H * (Sq / BQ);
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+    if (tiles > 2 * cus) return 0;
+    sa::fwd_split_plan((int)tiles, Sk, BQ, D, dtype, cus, nsplit, split_chunks);
+    return *nsplit > 1 ? (size_t)tiles * (size_t)*nsplit * (size_t)BQ * (size_t)(D + 2) * 4 : 0;
+}
+
 int forward_impl(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4], const void *v,
                  const int64_t v_strides[4], void *o, const int64_t o_strides[4], const uint8_t *mask,
                  const int64_t mask_strides[4], const int32_t *full_ids, const int64_t full_ids_strides[4],
@@ -247,7 +261,7 @@ int forward_impl(const void *q, const int64_t q_strides[4], const void *k, const
                  const uint8_t *packed, const int64_t packed_strides[2], bool use_packed, const int32_t *schedule,
                  size_t schedule_bytes, int schedule_mode, float *lse, const int64_t lse_strides[3], int B, int H,
                  int Sq, int Sk, int D, int BQ, int BK, int dtype, float sm_scale_log2, void *stream,
-                 int kernel = SA_FWD_KERNEL_DEFAULT) {
+                 int kernel = SA_FWD_KERNEL_DEFAULT, void *workspace = nullptr, size_t workspace_bytes = 0) {
     g_error[0] = 0;
     const int rot_group = kernel >> 8;
     kernel &= 0xff;
@@ -366,6 +380,14 @@ int forward_impl(const void *q, const int64_t q_strides[4], const void *k, const
         fp.lse = lse;
         for (int i = 0; i < 3; i++) fp.lses[i] = lse_strides[i];
     }
+    fp.nsplit = 1;
+    if (workspace && kernel == SA_FWD_KERNEL_DEFAULT && !fp.sched) {
+        const size_t need = split_shape(B, H, Sq, Sk, D, BQ, BK, dtype, &fp.nsplit, &fp.split_chunks);
+        if (need != 0 && (workspace_bytes < need || !aligned(workspace, 16)))
+            return fail(SA_ERR_WORKSPACE, "sa_sparse_attention_fwd_split: a 16-byte aligned workspace of %zu bytes required, %zu given", need, workspace_bytes);
+        fp.ws = static_cast<float *>(workspace);
+        fp.ws_ml = fp.ws + (need / 4 / (size_t)(D + 2)) * (size_t)D;
+    }
     if (kernel == SA_FWD_KERNEL_SHORT_LISTS) {
         if (f32 || !sa::fwd_c32_has(fp, dtype, D, BQ))
             return fail(SA_ERR_UNSUPPORTED, "sa_sparse_attention_fwd_kernel: the short-list kernel needs bf16 or fp16, head dim 128, BLOCK_Q 128, packed PARTIAL tiles and no schedule");
@@ -480,6 +502,35 @@ int sa_sparse_attention_fwd_kernel(const void *q, const int64_t q_strides[4], co
                         full_ids_strides, full_lens, full_lens_strides, part_ids, part_ids_strides, part_lens,
                         part_lens_strides, packed, packed_strides, use_packed, nullptr, 0, 0, lse, lse_strides, B, H, Sq,
                         Sk, D, BQ, BK, dtype, sm_scale_log2, stream, kernel);
+}
+
+size_t sa_fwd_split_workspace_bytes(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype) {
+    int nsplit, split_chunks;
+    if ((D != 64 && D != 128) || dtype < SA_DTYPE_BF16 || dtype > SA_DTYPE_FP32) return 0;
+    return split_shape(B, H, Sq, Sk, D, BQ, BK, dtype, &nsplit, &split_chunks);
+}
+
+int sa_sparse_attention_fwd_split(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
+                                  const void *v, const int64_t v_strides[4], void *o, const int64_t o_strides[4],
+                                  const uint8_t *mask, const int64_t mask_strides[4], const int32_t *full_ids,
+                                  const int64_t full_ids_strides[4], const int32_t *full_lens,
+                                  const int64_t full_lens_strides[3], const int32_t *part_ids,
+                                  const int64_t part_ids_strides[4], const int32_t *part_lens,
+                                  const int64_t part_lens_strides[3], const uint8_t *packed,
+                                  const int64_t packed_strides[2], float *lse, const int64_t lse_strides[3], int B,
+                                  int H, int Sq, int Sk, int D, int BQ, int BK, int dtype, float sm_scale_log2,
+                                  void *workspace, size_t workspace_bytes, void *stream) {
+    const bool use_packed = packed != nullptr;
+    if (use_packed) {
+        g_error[0] = 0;
+        if (!packed_strides) return fail(SA_ERR_INVALID_ARGUMENT, "sa_sparse_attention_fwd_split: null pointer argument (packed_strides)");
+        if ((B > 1 && packed_strides[0] % 4) || (H > 1 && packed_strides[1] % 4) || !aligned(packed, 4))
+            return fail(SA_ERR_UNSUPPORTED, "sa_sparse_attention_fwd_split: packed needs a 4-byte aligned base and plane strides");
+    }
+    return forward_impl(q, q_strides, k, k_strides, v, v_strides, o, o_strides, mask, mask_strides, full_ids,
+                        full_ids_strides, full_lens, full_lens_strides, part_ids, part_ids_strides, part_lens,
+                        part_lens_strides, packed, packed_strides, use_packed, nullptr, 0, 0, lse, lse_strides, B, H, Sq,
+                        Sk, D, BQ, BK, dtype, sm_scale_log2, stream, SA_FWD_KERNEL_DEFAULT, workspace, workspace_bytes);
 }
 
 int sa_validate_metadata(const int32_t *full_ids, const int64_t full_ids_strides[4], const int32_t *full_lens,

@@ -154,7 +154,8 @@ def sparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: to
     ``mask`` may be None when ``mask_metadata`` carries ``packed_masks`` (the kernels then read no mask tensor), which
     is how masks given by a formula run (:func:`compute_mask_terms`).
     ``kernel`` (not in the reference, whose one kernel Triton autotunes at the first call, sparse_attn_kernel.py:66-72):
-    "default" = two workgroups per compute unit, 64 keys per step; "short" = the form for masks that leave a Q tile
+    "default" = two workgroups per compute unit, 64 keys per step (the list of a Q tile shared by several workgroups
+    where there are too few Q tiles to fill the device); "short" = the form for masks that leave a Q tile
     few KV tiles (three workgroups per compute unit, 32 keys per step; bf16/fp16, D = 128, BLOCK_Q = 128, packed
     PARTIAL tiles, ``mask_metadata.list_stats`` with no list above 256 entries); None / "auto" = "short" when the
     metadata carries ``list_stats`` (``compute_mask_kernel(..., list_stats=True)``) that say the lists are short,
@@ -271,6 +272,13 @@ def sparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: to
                 *common, *((packed.data_ptr(), S(packed.stride()[:2])) if packed is not None else (None, None)),
                 lse.data_ptr() if return_lse else None, S(lse.stride()) if return_lse else None, *tail[:-1],
                 _native.SA_FWD_KERNEL_ROTATED | (group << 8), tail[-1])
+        elif sched is None and (ws_bytes := lib.sa_fwd_split_workspace_bytes(*tail[:8])):
+            # too few Q tiles to fill the device: their lists are shared by several workgroups
+            ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=q.device)
+            rc = lib.sa_sparse_attention_fwd_split(
+                *common, *((packed.data_ptr(), S(packed.stride()[:2])) if packed is not None else (None, None)),
+                lse.data_ptr() if return_lse else None, S(lse.stride()) if return_lse else None, *tail[:-1],
+                ws.data_ptr(), ws_bytes, tail[-1])
         elif packed is not None or sched is not None or return_lse:
             pk = (packed.data_ptr(), S(packed.stride()[:2])) if packed is not None else (None, None)
             sc = ((sched.data_ptr(), sched.numel() * 4, int(getattr(mask_metadata, "schedule_mode", 0)))
