@@ -58,6 +58,7 @@ EXPORTS = (
 )
 
 _lib = None
+_host = None
 
 _i64p = ctypes.POINTER(ctypes.c_int64)
 _vp = ctypes.c_void_p
@@ -163,6 +164,21 @@ def load() -> ctypes.CDLL:
         raise RuntimeError(f"libsparseattn_hip ABI {lib.sa_abi_version()} != expected {SA_ABI_VERSION}")
     _lib = lib
     return lib
+
+
+def host():
+    """The extension module that checks, allocates and launches for the wrappers (csrc/host_ops.cpp).  Raises if it or the
+    HIP library under it has not been built."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise RuntimeError("sparseattention_amd._host is missing or does not load: build it with "
+                               "`python -m sparseattention_amd.build`") from e
+        _host = module
+    return _host
 
 
 def strides(values):

@@ -10,6 +10,7 @@ import re
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -17,6 +18,7 @@ _ROOT = os.path.dirname(_HERE)
 CSRC = os.path.join(_HERE, "csrc")
 INCLUDE = os.path.join(_ROOT, "include")
 LIB_PATH = os.path.join(_HERE, "libsparseattn_hip.so")
+HOST_PATH = os.path.join(_HERE, "_host" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
 
 # (source, object name, extra defines).  The forward kernels are one source compiled per element type and
 # mask source, so that the variants build in parallel.
@@ -109,6 +111,26 @@ def _run(cmd):
     return res
 
 
+def build_host(verbose: bool = False) -> str:
+    """Compile the host side of the wrappers (csrc/host_ops.cpp) against torch and the library built before it."""
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-DTORCH_API_INCLUDE_EXTENSION_H",
+           "-DTORCH_EXTENSION_NAME=_host", f"-I{INCLUDE}", *(f"-isystem{p}" for p in include_paths()),
+           f"-isystem{sysconfig.get_paths()['include']}", f"-isystem{rocm}/include",
+           os.path.join(CSRC, "host_ops.cpp"), "-o", HOST_PATH, f"-L{_HERE}", "-lsparseattn_hip", "-Wl,-rpath,$ORIGIN",
+           *(f"-L{p}" for p in library_paths()), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    if verbose:
+        print(" ".join(cmd))
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError("command failed: " + " ".join(cmd) + "\n" + r.stdout + r.stderr)
+    return HOST_PATH
+
+
 def build_library(verbose: bool = False, extra_flags=()) -> str:
     """Compile every kernel translation unit and link the shared library.  Always recompiles."""
     hipcc = _hipcc()
@@ -123,6 +145,7 @@ def build_library(verbose: bool = False, extra_flags=()) -> str:
     with ThreadPoolExecutor(max_workers=min(os.cpu_count() or 4, len(cmds), 8)) as ex:
         list(ex.map(_run, cmds))
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc", *objs, "-o", LIB_PATH])
+    build_host(verbose)
     return LIB_PATH
 
 

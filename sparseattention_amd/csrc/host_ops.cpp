@@ -1,0 +1,577 @@
+// The host side of one call: checks, output and workspace tensors, strides and the launch through the C ABI
+// (include/sparseattn.h), for the Python wrappers of sparse_attn_kernel.py and mask_utils.py.
+//
+// Why native: a small call's kernels take 10 to 40 us, and the same steps in Python with ctypes took 27 us for a forward
+// with metadata, 68 us with the mask classified on the way and 220 us for a training step, so the device waited for the
+// host.  Nothing is kept between calls; every workspace is a tensor of the caching allocator, ordered by the stream.
+//
+// Errors are the Python exceptions the wrappers document: ValueError, TypeError, AssertionError, RuntimeError, and
+// SparseAttnError for the library's own error codes.
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/core/DeviceGuard.h>
+#include <torch/extension.h>
+
+#include <cmath>
+#include <optional>
+#include <string>
+
+#include "sparseattn.h"
+
+namespace py = pybind11;
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+
+namespace {
+
+[[noreturn]] void value_error(const std::string &m) { throw py::value_error(m); }
+[[noreturn]] void type_error(const std::string &m) { throw py::type_error(m); }
+[[noreturn]] void assertion(const char *m) {
+    PyErr_SetString(PyExc_AssertionError, m);
+    throw py::error_already_set();
+}
+
+std::string str(at::IntArrayRef s) {
+    std::string out = "(";
+    for (size_t i = 0; i < s.size(); i++) out += (i ? ", " : "") + std::to_string(s[i]);
+    return out + (s.size() == 1 ? ",)" : ")");
+}
+std::string str(const Tensor &t) { return std::string(c10::toString(t.scalar_type())) + " " + str(t.sizes()) + " on " + t.device().str(); }
+
+void check_rc(int rc) {
+    if (rc == SA_OK) return;
+    if (rc == SA_ERR_INVALID_ARGUMENT) value_error(std::string("libsparseattn_hip: ") + sa_last_error());
+    // (the backward of the autograd function runs on a thread of its own, without the interpreter's lock)
+    py::gil_scoped_acquire gil;
+    const py::object cls = py::module_::import("sparseattention_amd._native").attr("SparseAttnError");
+    const py::object err = cls(rc, py::str(sa_last_error()));
+    PyErr_SetObject(cls.ptr(), err.ptr());
+    throw py::error_already_set();
+}
+
+void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream(); }
+
+const int64_t *st(const Tensor &t) { return t.strides().data(); }
+const int64_t *st(const OptTensor &t) { return t ? t->strides().data() : nullptr; }
+template <class T>
+T *ptr(const Tensor &t) { return static_cast<T *>(t.data_ptr()); }
+template <class T>
+T *ptr(const OptTensor &t) { return t ? static_cast<T *>(t->data_ptr()) : nullptr; }
+
+int dtype_code(at::ScalarType t) {
+    return t == at::kBFloat16 ? SA_DTYPE_BF16 : t == at::kHalf ? SA_DTYPE_FP16 : t == at::kFloat ? SA_DTYPE_FP32 : -1;
+}
+
+// Every tensor whose address goes to a kernel must live where `ref` lives.
+void same_device(const Tensor &ref, const char *name, const Tensor &t) {
+    if (t.device() != ref.device())
+        value_error(std::string(name) + " is on " + t.device().str() + ", expected " + ref.device().str() +
+                    " (every tensor argument must be on q's device)");
+}
+void same_device(const Tensor &ref, const char *name, const OptTensor &t) {
+    if (t) same_device(ref, name, *t);
+}
+
+// The kernels want a unit stride in D and 16-byte aligned rows; copied only when that does not hold.
+Tensor kernel_ready(const Tensor &t) {
+    const int64_t per16 = 16 / t.element_size();
+    bool ok = t.stride(-1) == 1 && (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
+    for (int64_t d = 0; d + 1 < t.dim(); d++) ok = ok && t.stride(d) % per16 == 0;
+    return ok ? t : t.contiguous();
+}
+int64_t kernel_head_dim(int64_t D, bool has256) { return D <= 64 ? 64 : D <= 128 ? 128 : has256 && D <= 256 ? 256 : D; }
+Tensor pad_head_dim(const Tensor &t, int64_t Dk) {
+    return t.size(-1) == Dk ? t : at::constant_pad_nd(t, {0, Dk - t.size(-1)});
+}
+Tensor cut_head_dim(const Tensor &t, int64_t D) { return t.size(-1) == D ? t : t.narrow(-1, 0, D).contiguous(); }
+
+bool pow2_from_16(int64_t n) { return n >= 16 && (n & (n - 1)) == 0; }
+double scale_log2(int64_t D) { return 1.0 / std::sqrt((double)D) * 1.0 / std::log(2.0); }  // exp2 replaces exp (sparse_attn_kernel.py:152)
+
+// ---- the tile lists of a mask -------------------------------------------------------------------------------------
+struct Lists {
+    Tensor fid, fl, pid, pl;
+    OptTensor packed;
+};
+
+// Attribute of a metadata object: a new reference, or an empty object where there is none or it is None.
+py::object attr(py::handle o, const char *name) {
+    PyObject *v = PyObject_GetAttrString(o.ptr(), name);
+    if (!v) {
+        if (!PyErr_ExceptionMatches(PyExc_AttributeError)) throw py::error_already_set();
+        PyErr_Clear();
+        return py::object();
+    }
+    if (v == Py_None) {
+        Py_DECREF(v);
+        return py::object();
+    }
+    return py::reinterpret_steal<py::object>(v);
+}
+Tensor tensor_attr(py::handle o, const char *name) {
+    const py::object v = attr(o, name);
+    if (!v || !THPVariable_Check(v.ptr())) type_error(std::string("mask_metadata.") + name + " is not a tensor");
+    return THPVariable_Unpack(v.ptr());
+}
+OptTensor opt_tensor_attr(py::handle o, const char *name) {
+    const py::object v = attr(o, name);
+    if (!v) return std::nullopt;
+    if (!THPVariable_Check(v.ptr())) type_error(std::string("mask_metadata.") + name + " is not a tensor");
+    return THPVariable_Unpack(v.ptr());
+}
+
+Lists lists_of(py::handle md) {
+    return {tensor_attr(md, "unmasked_kv_ids"), tensor_attr(md, "unmasked_lens"), tensor_attr(md, "masked_kv_ids"),
+            tensor_attr(md, "masked_lens"), opt_tensor_attr(md, "packed_masks")};
+}
+
+// Whether md._validated_for is mask_utils.validation_key(md, Sk, BK): the sizes, then address and version counter of the
+// four list tensors.
+bool validated(py::handle md, const Lists &l, int64_t Sk, int64_t BK) {
+    const py::object key = attr(md, "_validated_for");
+    if (!key || !PyTuple_Check(key.ptr()) || PyTuple_GET_SIZE(key.ptr()) != 6) return false;
+    auto is = [](PyObject *o, unsigned long long want) {
+        const unsigned long long got = PyLong_Check(o) ? PyLong_AsUnsignedLongLongMask(o) : ~want;
+        return got == want;
+    };
+    if (!is(PyTuple_GET_ITEM(key.ptr(), 0), (unsigned long long)Sk) || !is(PyTuple_GET_ITEM(key.ptr(), 1), (unsigned long long)BK)) return false;
+    const Tensor *t[4] = {&l.fid, &l.fl, &l.pid, &l.pl};
+    for (int i = 0; i < 4; i++) {
+        PyObject *e = PyTuple_GET_ITEM(key.ptr(), 2 + i);
+        if (!PyTuple_Check(e) || PyTuple_GET_SIZE(e) != 2 || !is(PyTuple_GET_ITEM(e, 0), (unsigned long long)(uintptr_t)t[i]->data_ptr()) ||
+            !is(PyTuple_GET_ITEM(e, 1), (unsigned long long)t[i]->_version()))
+            return false;
+    }
+    return true;
+}
+void checked_metadata(py::handle md, const Lists &l, int64_t Sk, int64_t BK) {
+    if (!validated(md, l, Sk, BK))
+        py::module_::import("sparseattention_amd.sparse_attn_kernel").attr("_checked_metadata")(md, Sk, BK);
+}
+
+void check_lists(const Lists &l, const Tensor &ref, int64_t B, int64_t H, int64_t nQ, int64_t nK, const char *what) {
+    const int64_t ids[4] = {B, H, nQ, nK};
+    const Tensor *t[4] = {&l.fid, &l.pid, &l.fl, &l.pl};
+    const char *name[4] = {"unmasked_kv_ids", "masked_kv_ids", "unmasked_lens", "masked_lens"};
+    for (int i = 0; i < 4; i++) {
+        const at::IntArrayRef want(ids, i < 2 ? 4 : 3);
+        if (t[i]->sizes() != want || t[i]->scalar_type() != at::kInt || t[i]->device() != ref.device())
+            value_error(std::string(what) + "." + name[i] + ": expected int32 " + str(want) + " on " + ref.device().str() + ", got " + str(*t[i]));
+    }
+}
+void check_packed(const Tensor &pk, const Tensor &ref, int64_t B, int64_t H, int64_t nQ, int64_t nK, int64_t tile_bytes, const char *what) {
+    const int64_t want[5] = {B, H, nQ, nK, tile_bytes};
+    if (pk.sizes() != at::IntArrayRef(want, 5) || pk.scalar_type() != at::kByte || pk.device() != ref.device() ||
+        pk.stride(2) != nK * tile_bytes || pk.stride(3) != tile_bytes || pk.stride(4) != 1)
+        value_error(std::string(what) + ".packed_masks: expected uint8 " + str(at::IntArrayRef(want, 5)) + " on " + ref.device().str() +
+                    " with contiguous tiles, got " + str(pk) + " strides " + str(pk.strides()));
+}
+
+// The tensors a classification fills: distinct planes only, seen through the whole [B,H] by stride 0.
+Lists empty_lists(int64_t uB, int64_t uH, int64_t B, int64_t H, int64_t nQ, int64_t nK, int64_t tile_bytes, bool pack, const at::Device &dev) {
+    const auto i32 = at::TensorOptions().dtype(at::kInt).device(dev);
+    // (one allocation for the four: offsets are multiples of four bytes, and the views keep it alive)
+    const int64_t planes = uB * uH, ids = planes * nQ * nK, lens = planes * nQ;
+    const Tensor all = at::empty({2 * ids + 2 * lens}, i32);
+    const int64_t sB = uB == 1 && B > 1 ? 0 : uH * nQ, sH = uH == 1 && H > 1 ? 0 : nQ;
+    auto ids_at = [&](int64_t o) { return all.as_strided({B, H, nQ, nK}, {sB * nK, sH * nK, nK, 1}, o); };
+    auto lens_at = [&](int64_t o) { return all.as_strided({B, H, nQ}, {sB, sH, 1}, o); };
+    Lists l{ids_at(0), lens_at(2 * ids), ids_at(ids), lens_at(2 * ids + lens), std::nullopt};
+    if (pack)
+        l.packed = at::empty({uB, uH, nQ, nK, tile_bytes}, at::TensorOptions().dtype(at::kByte).device(dev)).expand({B, H, nQ, nK, tile_bytes});
+    return l;
+}
+
+Lists classify_lists(const Tensor &mask, int64_t BQ, int64_t BK, std::optional<bool> pack_partial) {
+    if (mask.dim() != 4) value_error("mask must be [B,H,Sq,Sk] (got " + str(mask.sizes()) + "); use mask.expand(B,H,Sq,Sk)");
+    const int64_t B = mask.size(0), H = mask.size(1), Sq = mask.size(2), Sk = mask.size(3);
+    // the reference asserts these (mask_utils.py:18-20, :89-90)
+    if (mask.scalar_type() != at::kBool) assertion("mask must be a torch.bool tensor");
+    if (BQ <= 0 || Sq % BQ) assertion("Sq must be a multiple of BLOCK_Q");
+    if (BK <= 0 || Sk % BK) assertion("Sk must be a multiple of BLOCK_K");
+    if (!mask.is_cuda()) throw std::runtime_error("compute_mask_kernel needs the mask on a ROCm GPU; compute_mask_slow runs anywhere");
+    const bool pack = pack_partial.value_or(BK % 8 == 0);
+    if (pack && BK % 8) value_error("pack_partial needs BLOCK_K to be a multiple of 8 (got " + std::to_string(BK) + ")");
+    const int64_t uB = mask.stride(0) == 0 || B == 1 ? 1 : B, uH = mask.stride(1) == 0 || H == 1 ? 1 : H;
+    const int64_t nQ = Sq / BQ, nK = Sk / BK;
+    const c10::DeviceGuard guard(mask.device());
+    void *const stream = stream_of(mask);
+    Lists l = empty_lists(uB, uH, B, H, nQ, nK, BQ * BK / 8, pack, mask.device());
+    const size_t need = sa_mask_classify_workspace_bytes(st(mask), B, H, Sq, Sk, BQ, BK);
+    // (dropped at the end of this call: the allocator hands the block out again only behind these launches on the stream)
+    const Tensor ws = at::empty({(int64_t)std::max<size_t>(need, 1)}, at::TensorOptions().dtype(at::kByte).device(mask.device()));
+    check_rc(sa_mask_classify(ptr<uint8_t>(mask), st(mask), B, H, Sq, Sk, BQ, BK, ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl),
+                              ptr<int32_t>(l.pid), st(l.pid), ptr<int32_t>(l.pl), st(l.pl), ws.data_ptr(), ws.numel(), stream));
+    if (pack)
+        check_rc(sa_mask_pack_partial(ptr<uint8_t>(mask), st(mask), B, H, Sq, Sk, BQ, BK, ptr<int32_t>(l.pid), st(l.pid), ptr<int32_t>(l.pl),
+                                      st(l.pl), ptr<uint8_t>(*l.packed), st(*l.packed), stream));
+    return l;
+}
+
+py::tuple as_tuple(const Lists &l) { return py::make_tuple(l.fid, l.fl, l.pid, l.pl, l.packed ? py::cast(*l.packed) : py::none()); }
+
+// compute_mask_kernel: (unmasked_kv_ids, unmasked_lens, masked_kv_ids, masked_lens, packed_masks or None)
+py::tuple classify(const Tensor &mask, int64_t BQ, int64_t BK, std::optional<bool> pack_partial) {
+    return as_tuple(classify_lists(mask, BQ, BK, pack_partial));
+}
+
+// compute_mask_terms: the same from terms, eight int32 each (their and the documents' shapes are checked by the caller)
+py::tuple classify_terms(const std::vector<int32_t> &terms, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t BQ, int64_t BK,
+                         const OptTensor &doc_q, const OptTensor &doc_k, bool pack, const at::Device &dev) {
+    const int64_t nQ = Sq / BQ, nK = Sk / BK;
+    const bool per_batch = B > 1 && ((doc_q && doc_q->stride(0) != 0) || (doc_k && doc_k->stride(0) != 0));
+    const int64_t uB = per_batch ? B : 1;
+    const c10::DeviceGuard guard(dev);
+    Lists l = empty_lists(uB, 1, B, H, nQ, nK, BQ * BK / 8, pack, dev);
+    const size_t need = sa_mask_terms_workspace_bytes(uB, Sq, Sk, BQ, BK);
+    const Tensor ws = at::empty({(int64_t)std::max<size_t>(need, 1)}, at::TensorOptions().dtype(at::kByte).device(dev));
+    check_rc(sa_mask_classify_terms(terms.data(), (int)(terms.size() / 8), ptr<int32_t>(doc_q), st(doc_q), ptr<int32_t>(doc_k), st(doc_k), B, H, Sq, Sk,
+                                    BQ, BK, ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl), ptr<int32_t>(l.pid), st(l.pid),
+                                    ptr<int32_t>(l.pl), st(l.pl), ptr<uint8_t>(l.packed), st(l.packed), ws.data_ptr(), ws.numel(), stream_of(l.fid)));
+    return as_tuple(l);
+}
+
+// ---- decode -------------------------------------------------------------------------------------------------------
+struct Out {
+    Tensor o;
+    OptTensor lse;
+};
+py::object as_object(const Out &r) { return r.lse ? py::object(py::make_tuple(r.o, *r.lse)) : py::cast(r.o); }
+
+void check_qkv(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &mask, const char *what) {
+    if (q.dim() != 4 || k.dim() != 4 || v.dim() != 4) value_error("q, k, v must be [B,H,S,D]");
+    const int64_t want[4] = {q.size(0), q.size(1), k.size(2), q.size(3)};
+    if (k.sizes() != at::IntArrayRef(want, 4) || v.sizes() != k.sizes())
+        value_error("k/v shapes " + str(k.sizes()) + "/" + str(v.sizes()) + " do not match q " + str(q.sizes()));
+    if (!q.is_cuda()) throw std::runtime_error(std::string(what) + " needs q, k, v on a ROCm GPU; there is no CPU path");
+    same_device(q, "k", k);
+    same_device(q, "v", v);
+    same_device(q, "mask", mask);
+}
+
+Out decode_impl(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &mask_in, int64_t BK, py::handle md, int64_t num_splits, bool return_lse) {
+    const int64_t B = q.size(0), H = q.size(1), Sq = q.size(2), D = q.size(3), Sk = k.size(2);
+    const int dt = dtype_code(q.scalar_type());
+    if ((dt != SA_DTYPE_BF16 && dt != SA_DTYPE_FP16) || k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type())
+        type_error(std::string("q, k, v must share dtype bfloat16 or float16 (got ") + c10::toString(q.scalar_type()) + ", " +
+                   c10::toString(k.scalar_type()) + ", " + c10::toString(v.scalar_type()) + ")");
+    OptTensor mask = mask_in;
+    if (mask) mask = mask->expand({B, H, Sq, Sk});
+    Lists l;
+    if (md.is_none()) {
+        if (!mask) value_error("sparse_attention_decode needs the mask or mask_metadata with packed_masks");
+        l = classify_lists(*mask, Sq, BK, std::nullopt);
+    } else {
+        l = lists_of(md);
+        if (BK <= 0) value_error("BLOCK_K must be positive");
+        check_lists(l, q, B, H, 1, Sk / BK, "mask_metadata");
+        checked_metadata(md, l, Sk, BK);
+        if (l.packed) check_packed(*l.packed, q, B, H, 1, Sk / BK, Sq * BK / 8, "mask_metadata");
+    }
+    if (l.packed && BK == 16 && Sq % 2) l.packed.reset();  // (halfword rows: the kernels want an even number of them)
+    if (!l.packed) {
+        if (!mask)
+            value_error("sparse_attention_decode without a mask tensor needs mask_metadata with packed_masks (and an even number of query rows at BLOCK_K = 16)");
+        if (mask->scalar_type() != at::kBool) assertion("mask must be a torch.bool tensor");
+    }
+    const int64_t Dk = kernel_head_dim(D, false);
+    const c10::DeviceGuard guard(q.device());
+    const Tensor qc = kernel_ready(pad_head_dim(q, Dk)), kc = kernel_ready(pad_head_dim(k, Dk)), vc = kernel_ready(pad_head_dim(v, Dk));
+    const Tensor o = at::empty_like(qc);
+    const auto f32 = at::TensorOptions().dtype(at::kFloat).device(q.device());
+    if (num_splits == 0) num_splits = sa_decode_num_splits(B, H, Sq, Sk, BK);
+    const size_t ws_bytes = sa_decode_workspace_bytes(B, H, Sq, Dk, num_splits);
+    Tensor ws;
+    if (ws_bytes) ws = at::empty({(int64_t)(ws_bytes / 4)}, f32);
+    OptTensor lse;
+    if (return_lse) lse = at::empty({B, H, Sq}, f32);
+    check_rc(sa_sparse_attention_decode_ex(qc.data_ptr(), st(qc), kc.data_ptr(), st(kc), vc.data_ptr(), st(vc), o.data_ptr(), st(o), ptr<uint8_t>(mask),
+                                           st(mask), ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl), ptr<int32_t>(l.pid), st(l.pid),
+                                           ptr<int32_t>(l.pl), st(l.pl), ptr<uint8_t>(l.packed), st(l.packed), B, H, Sq, Sk, Dk, BK, dt,
+                                           (float)scale_log2(D), num_splits, ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, ptr<float>(lse), st(lse),
+                                           stream_of(q)));
+    return {cut_head_dim(o, D), lse};
+}
+
+py::object decode(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &mask, int64_t BK, py::object md, int64_t num_splits, bool return_lse) {
+    check_qkv(q, k, v, mask, "sparse_attention_decode");
+    return as_object(decode_impl(q, k, v, mask, BK, md, num_splits, return_lse));
+}
+
+// ---- forward ------------------------------------------------------------------------------------------------------
+// Whether the kernels tile by the caller's own sizes (kernel_tiles of sparse_attn_kernel.py returns them unchanged).
+bool tiles_as_asked(int64_t Sq, int64_t Sk, int64_t D, int64_t BQ, int64_t BK, bool f32) {
+    if (BQ < 1 || BK < 1 || Sq % BQ || Sk % BK) return false;
+    if (f32 && BQ <= (D <= 128 ? 256 : 128)) return true;  // the float32 kernels tile by any sizes up to that
+    if (!pow2_from_16(BK)) return false;
+    if (Sq < 32) return D <= 128 && BQ == Sq;
+    return BQ == 128 || BQ == 64 || (D <= 128 && (BQ == 32 || BQ == 256));
+}
+
+// Below this many listed keys per Q tile (mean over the Q tiles) the forward runs its short-list kernel when the
+// metadata says so (MaskMetadata.list_stats) and the kernel has the sizes.  Measured on MI355X (B8 H32 S4096 D128,
+// tiles 128x32, default / short-list kernel): 448 keys per Q tile 0.343 / 0.340 ms, 1222 keys 0.709 / 0.719 ms,
+// 2100 keys and more +5 ... +8 %: the third workgroup per compute unit pays for itself on the shortest lists only.
+constexpr double kShortListKeys = 512;
+
+// The forward where the kernels tile by the caller's sizes, or nothing (then the wrapper makes other tiles of the mask).
+std::optional<Out> forward_impl(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &mask_in, int64_t BQ, int64_t BK, py::handle md,
+                                bool return_lse, const std::string &kernel) {
+    check_qkv(q, k, v, mask_in, "sparse_attention");
+    const int64_t B = q.size(0), H = q.size(1), Sq = q.size(2), D = q.size(3), Sk = k.size(2);
+    const int dt = dtype_code(q.scalar_type());
+    if (dt < 0 || k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type())
+        type_error(std::string("q, k, v must share dtype bfloat16, float16 or float32 (got ") + c10::toString(q.scalar_type()) + ", " +
+                   c10::toString(k.scalar_type()) + ", " + c10::toString(v.scalar_type()) + ")");
+    const bool f32 = dt == SA_DTYPE_FP32, has_md = !md.is_none();
+    if (!mask_in && !(has_md && attr(md, "packed_masks")))
+        value_error("sparse_attention without a mask tensor needs mask_metadata with packed_masks");
+    OptTensor mask = mask_in;
+    if (mask) mask = mask->expand({B, H, Sq, Sk});
+    if (!tiles_as_asked(Sq, Sk, D, BQ, BK, f32)) return std::nullopt;
+    // one Q tile of fewer rows than the forward kernels tile by: the split-KV kernels (they use no schedule)
+    if (Sq == BQ && Sq < 32 && BK >= 16 && !f32) return decode_impl(q, k, v, mask, BK, md, 0, return_lse);
+
+    const int64_t nQ = Sq / BQ, nK = Sk / BK;
+    Lists l;
+    OptTensor sched;
+    int sched_mode = 0;
+    double mean_list = 0;
+    int64_t longest_list = 0, rotation = 0;
+    bool stats = false;
+    if (!has_md) {
+        l = classify_lists(*mask, BQ, BK, std::nullopt);
+    } else {
+        l = lists_of(md);
+        check_lists(l, q, B, H, nQ, nK, "mask_metadata");
+        checked_metadata(md, l, Sk, BK);
+        if (l.packed) check_packed(*l.packed, q, B, H, nQ, nK, BQ * BK / 8, "mask_metadata");
+        sched = opt_tensor_attr(md, "schedule");
+        if (sched) {
+            if (sched->scalar_type() != at::kInt || sched->device() != q.device() || !sched->is_contiguous())
+                value_error("mask_metadata.schedule: expected a contiguous int32 tensor on q's device");
+            if (const py::object m = attr(md, "schedule_mode")) sched_mode = m.cast<int>();
+        }
+        if (const py::object s = attr(md, "list_stats")) {
+            stats = true;
+            mean_list = s[py::int_(0)].cast<double>();
+            longest_list = s[py::int_(1)].cast<int64_t>();
+        }
+        if (const py::object r = attr(md, "list_rotation")) rotation = r.cast<int64_t>();
+    }
+    if (mask && mask->scalar_type() != at::kBool) assertion("mask must be a torch.bool tensor");
+
+    const int64_t Dk = kernel_head_dim(D, true);
+    // which of the forward kernels: 0 default, otherwise the code of the C ABI
+    if (kernel != "auto" && kernel != "default" && kernel != "short" && kernel != "rotated")
+        value_error("kernel must be 'auto', 'default', 'rotated' or 'short' (got '" + kernel + "')");
+    if (kernel == "rotated" && (sched || f32)) value_error("kernel='rotated' needs bf16/fp16 and mask_metadata without a schedule");
+    int code = SA_FWD_KERNEL_DEFAULT;
+    const bool short_has = !f32 && Dk == 128 && BQ == 128 && pow2_from_16(BK) && l.packed && !sched;
+    const bool short_fits = stats && longest_list <= SA_FWD_SHORT_LISTS_MAX_ENTRIES;
+    if (kernel == "short") {
+        if (!(short_has && short_fits))
+            value_error("kernel='short' needs bf16/fp16, head dim 128, BLOCK_Q 128, mask_metadata with packed_masks, no schedule, and list_stats whose longest list has at most " +
+                        std::to_string(SA_FWD_SHORT_LISTS_MAX_ENTRIES) + " entries");
+        code = SA_FWD_KERNEL_SHORT_LISTS;
+    } else if (kernel == "auto" && short_has && short_fits && mean_list * (double)BK < kShortListKeys) {
+        code = SA_FWD_KERNEL_SHORT_LISTS;
+    } else if (!sched && !f32 && (kernel == "rotated" || (kernel == "auto" && rotation > 0))) {
+        // the default kernel with the FULL entries of Q tile qt walked from a start that depends on qt
+        code = SA_FWD_KERNEL_ROTATED | ((int)(rotation ? rotation : 16) << 8);
+    }
+
+    const c10::DeviceGuard guard(q.device());
+    const Tensor qc = kernel_ready(pad_head_dim(q, Dk)), kc = kernel_ready(pad_head_dim(k, Dk)), vc = kernel_ready(pad_head_dim(v, Dk));
+    const Tensor o = at::empty_like(qc);
+    const auto opt_f32 = at::TensorOptions().dtype(at::kFloat).device(q.device());
+    OptTensor lse;
+    if (return_lse) lse = at::empty({B, H, Sq}, opt_f32);
+    const float scale = (float)scale_log2(D);
+    void *const stream = stream_of(q);
+    if (sched) {
+        check_rc(sa_sparse_attention_fwd_lse(qc.data_ptr(), st(qc), kc.data_ptr(), st(kc), vc.data_ptr(), st(vc), o.data_ptr(), st(o), ptr<uint8_t>(mask),
+                                             st(mask), ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl), ptr<int32_t>(l.pid), st(l.pid),
+                                             ptr<int32_t>(l.pl), st(l.pl), ptr<uint8_t>(l.packed), st(l.packed), ptr<int32_t>(*sched),
+                                             sched->numel() * 4, sched_mode, ptr<float>(lse), st(lse), B, H, Sq, Sk, Dk, BQ, BK, dt, scale, stream));
+    } else if (code != SA_FWD_KERNEL_DEFAULT) {
+        check_rc(sa_sparse_attention_fwd_kernel(qc.data_ptr(), st(qc), kc.data_ptr(), st(kc), vc.data_ptr(), st(vc), o.data_ptr(), st(o),
+                                                ptr<uint8_t>(mask), st(mask), ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl),
+                                                ptr<int32_t>(l.pid), st(l.pid), ptr<int32_t>(l.pl), st(l.pl), ptr<uint8_t>(l.packed), st(l.packed),
+                                                ptr<float>(lse), st(lse), B, H, Sq, Sk, Dk, BQ, BK, dt, scale, code, stream));
+    } else {
+        // (too few Q tiles to fill the device: their lists are shared by several workgroups, which need a workspace)
+        const size_t ws_bytes = sa_fwd_split_workspace_bytes(B, H, Sq, Sk, Dk, BQ, BK, dt);
+        Tensor ws;
+        if (ws_bytes) ws = at::empty({(int64_t)(ws_bytes / 4)}, opt_f32);
+        check_rc(sa_sparse_attention_fwd_split(qc.data_ptr(), st(qc), kc.data_ptr(), st(kc), vc.data_ptr(), st(vc), o.data_ptr(), st(o),
+                                               ptr<uint8_t>(mask), st(mask), ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl),
+                                               ptr<int32_t>(l.pid), st(l.pid), ptr<int32_t>(l.pl), st(l.pl), ptr<uint8_t>(l.packed), st(l.packed),
+                                               ptr<float>(lse), st(lse), B, H, Sq, Sk, Dk, BQ, BK, dt, scale, ws_bytes ? ws.data_ptr() : nullptr,
+                                               ws_bytes, stream));
+    }
+    return Out{cut_head_dim(o, D), lse};
+}
+
+py::object forward(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &mask, int64_t BQ, int64_t BK, py::object md, bool return_lse,
+                   const std::string &kernel) {
+    const auto r = forward_impl(q, k, v, mask, BQ, BK, md, return_lse, kernel);
+    return r ? as_object(*r) : py::none();
+}
+
+// ---- backward -----------------------------------------------------------------------------------------------------
+// What the backward walks: the lists of the mask per 128 queries (KV tiles of 64) and of the transposed mask per 128 keys.
+struct BackwardLists {
+    Lists by_query, by_key;
+    OptTensor transposed_mask;
+};
+
+BackwardLists backward_lists_of(py::handle bmd, const Tensor &q, int64_t Sk) {
+    const int64_t B = q.size(0), H = q.size(1), Sq = q.size(2);
+    const py::object mq = attr(bmd, "by_query"), mk = attr(bmd, "by_key");
+    if (!mq || !mk) type_error("bwd_metadata has no by_query / by_key lists");
+    BackwardLists l{lists_of(mq), lists_of(mk), opt_tensor_attr(bmd, "transposed_mask")};
+    check_lists(l.by_query, q, B, H, Sq / 128, Sk / 64, "bwd_metadata");
+    checked_metadata(mq, l.by_query, Sk, 64);
+    check_lists(l.by_key, q, B, H, Sk / 128, Sq / 64, "bwd_metadata");
+    checked_metadata(mk, l.by_key, Sq, 64);
+    if (l.by_query.packed) check_packed(*l.by_query.packed, q, B, H, Sq / 128, Sk / 64, 1024, "bwd_metadata");
+    if (l.by_key.packed) check_packed(*l.by_key.packed, q, B, H, Sk / 128, Sq / 64, 1024, "bwd_metadata");
+    if (const OptTensor &mt = l.transposed_mask) {
+        const int64_t want[4] = {B, H, Sk, Sq};
+        if (mt->sizes() != at::IntArrayRef(want, 4) || mt->scalar_type() != at::kBool || mt->device() != q.device())
+            value_error("bwd_metadata.transposed_mask: expected bool " + str(at::IntArrayRef(want, 4)) + " on " + q.device().str());
+    }
+    return l;
+}
+
+// The lists made from the mask itself (compute_backward_metadata with packed tiles; Sq and Sk multiples of 128).
+BackwardLists backward_lists_from(const Tensor &mask) {
+    const int64_t B = mask.size(0), H = mask.size(1);
+    const Tensor distinct = mask.narrow(0, 0, mask.stride(0) == 0 ? 1 : B).narrow(1, 0, mask.stride(1) == 0 ? 1 : H);
+    const Tensor transposed = distinct.transpose(-1, -2).contiguous().expand({B, H, mask.size(3), mask.size(2)});
+    return {classify_lists(mask, 128, 64, true), classify_lists(transposed, 128, 64, true), std::nullopt};
+}
+
+std::tuple<Tensor, Tensor, Tensor> backward_impl(const Tensor &do_, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &o, const Tensor &lse,
+                                                 const OptTensor &mask, const BackwardLists &l) {
+    const int64_t B = q.size(0), H = q.size(1), Sq = q.size(2), D = q.size(3), Sk = k.size(2);
+    if (!mask && !(l.by_query.packed && l.by_key.packed))
+        value_error("sparse_attention_backward without a mask needs packed_masks in both lists of bwd_metadata");
+    const int64_t Dk = kernel_head_dim(D, false);
+    const c10::DeviceGuard guard(q.device());
+    const Tensor qc = kernel_ready(pad_head_dim(q, Dk)), kc = kernel_ready(pad_head_dim(k, Dk)), vc = kernel_ready(pad_head_dim(v, Dk));
+    const Tensor oc = kernel_ready(pad_head_dim(o, Dk)), doc = kernel_ready(pad_head_dim(do_, Dk));
+    const Tensor dq = at::empty_like(qc), dk = at::empty_like(kc), dv = at::empty_like(vc);
+    const size_t ws_bytes = sa_bwd_workspace_bytes(B, H, Sq);
+    const Tensor ws = at::empty({(int64_t)(ws_bytes / 4)}, at::TensorOptions().dtype(at::kFloat).device(q.device()));
+    const Lists &a = l.by_query, &b = l.by_key;
+    check_rc(sa_sparse_attention_bwd(qc.data_ptr(), st(qc), kc.data_ptr(), st(kc), vc.data_ptr(), st(vc), oc.data_ptr(), st(oc), doc.data_ptr(), st(doc),
+                                     ptr<float>(lse), st(lse), dq.data_ptr(), st(dq), dk.data_ptr(), st(dk), dv.data_ptr(), st(dv), ptr<uint8_t>(mask),
+                                     st(mask), ptr<uint8_t>(l.transposed_mask), st(l.transposed_mask), ptr<uint8_t>(a.packed), st(a.packed),
+                                     ptr<uint8_t>(b.packed), st(b.packed), ptr<int32_t>(a.fid), st(a.fid), ptr<int32_t>(a.fl), st(a.fl),
+                                     ptr<int32_t>(a.pid), st(a.pid), ptr<int32_t>(a.pl), st(a.pl), ptr<int32_t>(b.fid), st(b.fid), ptr<int32_t>(b.fl),
+                                     st(b.fl), ptr<int32_t>(b.pid), st(b.pid), ptr<int32_t>(b.pl), st(b.pl), ws.data_ptr(), ws_bytes, B, H, Sq, Sk, Dk,
+                                     dtype_code(q.scalar_type()), (float)scale_log2(D), stream_of(q)));
+    return {cut_head_dim(dq, D), cut_head_dim(dk, D), cut_head_dim(dv, D)};
+}
+
+void check_backward(const Tensor &do_, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &o, const Tensor &lse, const OptTensor &mask) {
+    if (q.dim() != 4 || k.dim() != 4) value_error("q, k, v must be [B,H,S,D]");
+    if (!q.is_cuda()) throw std::runtime_error("sparse_attention_backward needs its tensors on a ROCm GPU; there is no CPU path");
+    same_device(q, "k", k);
+    same_device(q, "v", v);
+    same_device(q, "o", o);
+    same_device(q, "do", do_);
+    same_device(q, "lse", lse);
+    same_device(q, "mask", mask);
+    const int dt = dtype_code(q.scalar_type());
+    if (dt != SA_DTYPE_BF16 && dt != SA_DTYPE_FP16) type_error("q, k, v, o, do must share dtype bfloat16 or float16");
+    for (const Tensor *t : {&k, &v, &o, &do_})
+        if (t->scalar_type() != q.scalar_type()) type_error("q, k, v, o, do must share dtype bfloat16 or float16");
+    const int64_t kw[4] = {q.size(0), q.size(1), k.size(2), q.size(3)}, lw[3] = {q.size(0), q.size(1), q.size(2)};
+    if (k.sizes() != at::IntArrayRef(kw, 4) || v.sizes() != k.sizes() || o.sizes() != q.sizes() || do_.sizes() != q.sizes())
+        value_error("shapes: q/o/do must be " + str(q.sizes()) + " and k/v " + str(at::IntArrayRef(kw, 4)) + " (got q " + str(q.sizes()) + ", k " +
+                    str(k.sizes()) + ", v " + str(v.sizes()) + ", o " + str(o.sizes()) + ", do " + str(do_.sizes()) + ")");
+    if (lse.scalar_type() != at::kFloat || lse.sizes() != at::IntArrayRef(lw, 3))
+        value_error("lse: expected float32 " + str(at::IntArrayRef(lw, 3)) + ", got " + str(lse));
+    if (mask && mask->scalar_type() != at::kBool) assertion("mask must be a torch.bool tensor");
+}
+
+// (dq, dk, dv), or None where Sq or Sk is no multiple of the kernels' 128 rows (then the wrapper pads)
+py::object backward(const Tensor &do_, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &o, const Tensor &lse, const OptTensor &mask_in,
+                    py::object bmd) {
+    check_backward(do_, q, k, v, o, lse, mask_in);
+    const int64_t Sq = q.size(2), Sk = k.size(2);
+    OptTensor mask = mask_in;
+    if (mask) mask = mask->expand({q.size(0), q.size(1), Sq, Sk});
+    if (Sq % 128 || Sk % 128) return py::none();
+    if (bmd.is_none() && !mask) value_error("sparse_attention_backward needs the mask or a BackwardMetadata with packed tiles");
+    const auto g = backward_impl(do_, q, k, v, o, lse, mask, bmd.is_none() ? backward_lists_from(*mask) : backward_lists_of(bmd, q, Sk));
+    return py::make_tuple(std::get<0>(g), std::get<1>(g), std::get<2>(g));
+}
+
+// ---- autograd -----------------------------------------------------------------------------------------------------
+// Everything the backward needs is taken out of the Python objects in the forward: autograd runs backwards on a thread of
+// its own, without the interpreter's lock.
+struct AttentionFunction : public torch::autograd::Function<AttentionFunction> {
+    static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &mask, const Out &r,
+                          const std::optional<BackwardLists> &lists) {
+        std::vector<at::Tensor> keep = {q, k, v, r.o, *r.lse, mask.value_or(Tensor())};
+        // (the lists are no outputs or inputs of the function: kept as they are, in the order backward() takes them)
+        std::vector<at::Tensor> l;
+        if (lists) {
+            for (const Lists *p : {&lists->by_query, &lists->by_key})
+                for (const Tensor &t : {p->fid, p->fl, p->pid, p->pl, p->packed.value_or(Tensor())}) l.push_back(t);
+            l.push_back(lists->transposed_mask.value_or(Tensor()));
+        }
+        for (const Tensor &t : l) keep.push_back(t);
+        ctx->save_for_backward(keep);
+        return r.o;
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        const auto s = ctx->get_saved_variables();
+        const Tensor &q = s[0], &k = s[1];
+        OptTensor mask;
+        if (s[5].defined()) mask = s[5];
+        auto opt = [](const Tensor &t) -> OptTensor { return t.defined() ? OptTensor(t) : std::nullopt; };
+        BackwardLists l;
+        if (s.size() > 6) {
+            l = {{s[6], s[7], s[8], s[9], opt(s[10])}, {s[11], s[12], s[13], s[14], opt(s[15])}, opt(s[16])};
+        } else {
+            l = backward_lists_from(*mask);
+        }
+        check_backward(grads[0], q, k, s[2], s[3], s[4], mask);
+        const auto g = backward_impl(grads[0], q, k, s[2], s[3], s[4], mask, l);
+        return {std::get<0>(g), std::get<1>(g), std::get<2>(g), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+// sparse_attention_trainable, or None where the wrapper has to pad or to make other tiles
+py::object trainable(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &mask_in, int64_t BQ, int64_t BK, py::object md, py::object bmd) {
+    if (q.dim() != 4 || k.dim() != 4 || q.size(2) % 128 || k.size(2) % 128 || q.scalar_type() == at::kFloat || (bmd.is_none() && !mask_in))
+        return py::none();
+    std::optional<Out> r;
+    {
+        const at::NoGradGuard no_grad;
+        r = forward_impl(q, k, v, mask_in, BQ, BK, md, true, "auto");
+    }
+    if (!r) return py::none();
+    const int64_t Sq = q.size(2), Sk = k.size(2);
+    OptTensor mask = mask_in;
+    if (mask) mask = mask->expand({q.size(0), q.size(1), Sq, Sk});
+    std::optional<BackwardLists> lists;
+    if (!bmd.is_none()) lists = backward_lists_of(bmd, q, Sk);
+    return py::cast(AttentionFunction::apply(q, k, v, mask, *r, lists));
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_host, m) {
+    m.doc() = "Checks, allocations and launches of the wrappers in sparse_attn_kernel.py and mask_utils.py.";
+    m.def("forward", &forward);
+    m.def("decode", &decode);
+    m.def("classify", &classify);
+    m.def("classify_terms", &classify_terms);
+    m.def("backward", &backward);
+    m.def("trainable", &trainable);
+}

@@ -5,7 +5,6 @@ Mirrors the interface of the reference's ``sparseattention/mask_utils.py``:
 """
 from __future__ import annotations
 
-import ctypes
 from dataclasses import dataclass, field
 from typing import Optional, Sequence, Tuple
 
@@ -137,9 +136,7 @@ def compute_mask_slow(mask: torch.Tensor, BLOCK_Q: int, BLOCK_K: int) -> MaskMet
 
 
 def _make_schedule(lib, fl, pl, B, H, Sq, Sk, BLOCK_Q, BLOCK_K, schedule, dev):
-    """(schedule tensor, mode) for ``compute_mask_kernel(..., schedule=...)``; (None, 0) without one."""
-    if not schedule:
-        return None, 0
+    """(schedule tensor, mode) for ``compute_mask_kernel(..., schedule=...)``."""
     modes = {"persistent": _native.SA_SCHEDULE_PERSISTENT, "pairs": _native.SA_SCHEDULE_PAIRS,
              True: _native.SA_SCHEDULE_PAIRS}
     if schedule not in modes:
@@ -188,50 +185,12 @@ def compute_mask_kernel(mask: torch.Tensor, BLOCK_Q: int, BLOCK_K: int, pack_par
     ``MaskMetadata.list_stats``), which lets :func:`sparse_attention` choose the kernel form for short lists.  This is
     the one option that synchronises the host with the device; preprocessing is paid once per mask (README.md:46).
     """
-    B, H, Sq, Sk = _check_mask(mask, BLOCK_Q, BLOCK_K)
-    if not mask.is_cuda:
-        raise RuntimeError("compute_mask_kernel needs the mask on a ROCm GPU; compute_mask_slow runs anywhere")
-    lib = _native.load()
-    nQ, nK = Sq // BLOCK_Q, Sk // BLOCK_K
-    uB = 1 if (mask.stride(0) == 0 or B == 1) else B
-    uH = 1 if (mask.stride(1) == 0 or H == 1) else H
-    dev = mask.device
-    with torch.cuda.device(dev):
-        fid = torch.empty(uB, uH, nQ, nK, dtype=torch.int32, device=dev)
-        pid = torch.empty(uB, uH, nQ, nK, dtype=torch.int32, device=dev)
-        fl = torch.empty(uB, uH, nQ, dtype=torch.int32, device=dev)
-        pl = torch.empty(uB, uH, nQ, dtype=torch.int32, device=dev)
-        fid, pid = fid.expand(B, H, nQ, nK), pid.expand(B, H, nQ, nK)
-        fl, pl = fl.expand(B, H, nQ), pl.expand(B, H, nQ)
-        ms = _native.strides(mask.stride())
-        need = lib.sa_mask_classify_workspace_bytes(ms, B, H, Sq, Sk, BLOCK_Q, BLOCK_K)
-        workspace = torch.empty(max(int(need), 1), dtype=torch.uint8, device=dev)
-        rc = lib.sa_mask_classify(
-            mask.data_ptr(), ms, B, H, Sq, Sk, BLOCK_Q, BLOCK_K,
-            fid.data_ptr(), _native.strides(fid.stride()), fl.data_ptr(), _native.strides(fl.stride()),
-            pid.data_ptr(), _native.strides(pid.stride()), pl.data_ptr(), _native.strides(pl.stride()),
-            workspace.data_ptr(), workspace.numel(), torch.cuda.current_stream(dev).cuda_stream,
-        )
-        _native.check(rc)
-        # the kernels run on the current stream; the caching allocator may hand this block out again
-        # only to work queued after them on the same stream, so dropping the reference here is safe
-        del workspace
-        packed = None
-        if pack_partial is None:
-            pack_partial = BLOCK_K % 8 == 0
-        if pack_partial:
-            if BLOCK_K % 8:
-                raise ValueError(f"pack_partial needs BLOCK_K to be a multiple of 8 (got {BLOCK_K})")
-            packed = torch.empty(uB, uH, nQ, nK, BLOCK_Q * BLOCK_K // 8, dtype=torch.uint8, device=dev)
-            rc = lib.sa_mask_pack_partial(
-                mask.data_ptr(), ms, B, H, Sq, Sk, BLOCK_Q, BLOCK_K,
-                pid.data_ptr(), _native.strides(pid.stride()), pl.data_ptr(), _native.strides(pl.stride()),
-                packed.data_ptr(), _native.strides(packed.stride()[:2]),
-                torch.cuda.current_stream(dev).cuda_stream,
-            )
-            _native.check(rc)
-            packed = packed.expand(B, H, nQ, nK, BLOCK_Q * BLOCK_K // 8)
-        sched, mode = _make_schedule(lib, fl, pl, B, H, Sq, Sk, BLOCK_Q, BLOCK_K, schedule, dev)
+    fid, fl, pid, pl, packed = _native.host().classify(mask, BLOCK_Q, BLOCK_K, pack_partial)
+    B, H, Sq, Sk = mask.shape
+    sched, mode = None, 0
+    if schedule:
+        with torch.cuda.device(mask.device):
+            sched, mode = _make_schedule(_native.load(), fl, pl, B, H, Sq, Sk, BLOCK_Q, BLOCK_K, schedule, mask.device)
     md = MaskMetadata(fid, fl, pid, pl, packed, sched, mode)
     md._validated_for = validation_key(md, Sk, BLOCK_K)  # lists made by the kernels above fit by construction
     return with_list_stats(md) if list_stats else md
@@ -449,36 +408,12 @@ def compute_mask_terms(terms: Sequence[MaskTerm], B: int, H: int, Sq: int, Sk: i
     if dev.type != "cuda" or any(d is not None and d.device != dev for d in (doc_q, doc_k)):
         raise RuntimeError("compute_mask_terms runs on a ROCm GPU (documents on the same device); "
                            "materialize_mask_terms + compute_mask_slow run anywhere")
-    lib = _native.load()
-    nQ, nK = Sq // BLOCK_Q, Sk // BLOCK_K
-    per_batch = B > 1 and any(d is not None and d.stride(0) != 0 for d in (doc_q, doc_k))
-    uB = B if per_batch else 1
     flat = [w for t in terms for w in t.encode()]
-    c_terms = (ctypes.c_int32 * len(flat))(*flat)
-    S = _native.strides
-    with torch.cuda.device(dev):
-        fid = torch.empty(uB, 1, nQ, nK, dtype=torch.int32, device=dev).expand(B, H, nQ, nK)
-        pid = torch.empty(uB, 1, nQ, nK, dtype=torch.int32, device=dev).expand(B, H, nQ, nK)
-        fl = torch.empty(uB, 1, nQ, dtype=torch.int32, device=dev).expand(B, H, nQ)
-        pl = torch.empty(uB, 1, nQ, dtype=torch.int32, device=dev).expand(B, H, nQ)
-        packed = None
-        if pack_partial:
-            packed = torch.empty(uB, 1, nQ, nK, BLOCK_Q * BLOCK_K // 8, dtype=torch.uint8, device=dev)
-            packed = packed.expand(B, H, nQ, nK, BLOCK_Q * BLOCK_K // 8)
-        need = int(lib.sa_mask_terms_workspace_bytes(uB, Sq, Sk, BLOCK_Q, BLOCK_K))
-        workspace = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
-        rc = lib.sa_mask_classify_terms(
-            c_terms, len(terms),
-            doc_q.data_ptr() if doc_q is not None else None, S(doc_q.stride()) if doc_q is not None else None,
-            doc_k.data_ptr() if doc_k is not None else None, S(doc_k.stride()) if doc_k is not None else None,
-            B, H, Sq, Sk, BLOCK_Q, BLOCK_K,
-            fid.data_ptr(), S(fid.stride()), fl.data_ptr(), S(fl.stride()),
-            pid.data_ptr(), S(pid.stride()), pl.data_ptr(), S(pl.stride()),
-            packed.data_ptr() if packed is not None else None, S(packed.stride()[:2]) if packed is not None else None,
-            workspace.data_ptr(), workspace.numel(), torch.cuda.current_stream(dev).cuda_stream)
-        _native.check(rc)
-        del workspace
-        sched, mode = _make_schedule(lib, fl, pl, B, H, Sq, Sk, BLOCK_Q, BLOCK_K, schedule, dev)
+    fid, fl, pid, pl, packed = _native.host().classify_terms(flat, B, H, Sq, Sk, BLOCK_Q, BLOCK_K, doc_q, doc_k, bool(pack_partial), dev)
+    sched, mode = None, 0
+    if schedule:
+        with torch.cuda.device(dev):
+            sched, mode = _make_schedule(_native.load(), fl, pl, B, H, Sq, Sk, BLOCK_Q, BLOCK_K, schedule, fl.device)
     md = MaskMetadata(fid, fl, pid, pl, packed, sched, mode)
     md._validated_for = validation_key(md, Sk, BLOCK_K)  # lists made by the kernels above fit by construction
     return md

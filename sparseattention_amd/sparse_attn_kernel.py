@@ -1,7 +1,8 @@
-"""Block-sparse attention forward (replaces the reference's ``sparseattention/sparse_attn_kernel.py``)."""
-from __future__ import annotations
+"""Block-sparse attention forward (replaces the reference's ``sparseattention/sparse_attn_kernel.py``).
 
-import math
+The steps of a call - checks, outputs, strides, launch - are native (csrc/host_ops.cpp); here is what a caller sees and
+what sizes without a kernel need around it."""
+from __future__ import annotations
 
 import torch
 
@@ -9,16 +10,6 @@ from . import _native
 from .mask_utils import MaskMetadata, Tiling, compute_mask_kernel, compute_mask_terms, validation_key
 
 _DTYPES = {torch.bfloat16: _native.SA_DTYPE_BF16, torch.float16: _native.SA_DTYPE_FP16}
-# the forward also takes float32 (kernels that compute in float32 throughout: on the fp32 matrix instruction at head
-# dims 64 and 128 with Q tiles of 64 or 128 rows, on the vector units otherwise)
-_FWD_DTYPES = {**_DTYPES, torch.float32: _native.SA_DTYPE_FP32}
-
-
-def _kernel_ready(t: torch.Tensor) -> torch.Tensor:
-    """The kernels want a unit stride in D, 16-byte aligned rows; copy only when that does not hold."""
-    per16 = 16 // t.element_size()
-    ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % per16 == 0 for s in t.stride()[:-1])
-    return t if ok else t.contiguous()
 
 
 def _kernel_head_dim(D: int, sizes) -> int:
@@ -26,10 +17,6 @@ def _kernel_head_dim(D: int, sizes) -> int:
     padded with zero columns, which change neither the scores nor the first D columns of the result; the softmax scale
     stays that of D).  A D beyond all of them is passed on, for the library to refuse."""
     return next((s for s in sizes if D <= s), D)
-
-
-def _pad_head_dim(t: torch.Tensor, Dk: int) -> torch.Tensor:
-    return t if t.shape[-1] == Dk else torch.nn.functional.pad(t, (0, Dk - t.shape[-1]))
 
 
 def _pad_mask(mask: torch.Tensor, q_multiple: int, k_multiple: int) -> torch.Tensor:
@@ -112,33 +99,6 @@ def kernel_tiles(Sq: int, Sk: int, D: int, BLOCK_Q: int, BLOCK_K: int):
     return next(((bq, bk) for bk in (32, 64, 16) if Sk % bk == 0), None)
 
 
-# Below this many listed keys per Q tile (mean over the Q tiles) the forward runs its short-list kernel when the
-# metadata says so (MaskMetadata.list_stats) and the kernel has the sizes.  Measured on MI355X (B8 H32 S4096 D128,
-# tiles 128x32, default / short-list kernel): 448 keys per Q tile 0.343 / 0.340 ms, 1222 keys 0.709 / 0.719 ms,
-# 2100 keys and more +5 ... +8 %: the third workgroup per compute unit pays for itself on the shortest lists only.
-SHORT_LIST_KEYS = 512
-
-
-def _short_list_kernel(mask_metadata, dtype, D, BLOCK_Q, BLOCK_K, kernel) -> bool:
-    """Whether this call runs the kernel for short lists (three workgroups per compute unit, 32 keys per step)."""
-    if kernel not in (None, "auto", "default", "short", "rotated"):
-        raise ValueError(f"kernel must be 'auto', 'default', 'rotated' or 'short' (got {kernel!r})")
-    if kernel in ("default", "rotated"):
-        return False
-    has = (dtype in _DTYPES and D == 128 and BLOCK_Q == 128 and BLOCK_K >= 16 and BLOCK_K & (BLOCK_K - 1) == 0
-           and getattr(mask_metadata, "packed_masks", None) is not None
-           and getattr(mask_metadata, "schedule", None) is None)
-    stats = getattr(mask_metadata, "list_stats", None)
-    fits = stats is not None and stats[1] <= _native.SA_FWD_SHORT_LISTS_MAX_ENTRIES
-    if kernel == "short":
-        if not (has and fits):
-            raise ValueError("kernel='short' needs bf16/fp16, head dim 128, BLOCK_Q 128, mask_metadata with packed_masks, "
-                             "no schedule, and list_stats whose longest list has at most "
-                             f"{_native.SA_FWD_SHORT_LISTS_MAX_ENTRIES} entries")
-        return True
-    return has and fits and stats[0] * BLOCK_K < SHORT_LIST_KEYS
-
-
 def sparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: torch.Tensor | None, BLOCK_Q, BLOCK_K,
                      mask_metadata: MaskMetadata | None = None, *, return_lse: bool = False, kernel: str | None = None):
     """softmax(q kᵀ / sqrt(D) + (mask ? 0 : -inf)) v, skipping KV tiles the mask empties.
@@ -162,27 +122,17 @@ def sparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: to
     else "default".  "rotated" = the default kernel with the FULL entries of Q tile qt walked from a start that depends
     on qt (for sliding windows; "auto" takes it when ``mask_metadata.list_rotation`` says so).  All agree within rounding.
     """
-    if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
-        raise ValueError("q, k, v must be [B,H,S,D]")
+    BLOCK_Q, BLOCK_K = int(BLOCK_Q), int(BLOCK_K)
+    kernel = "auto" if kernel is None else kernel
+    out = _native.host().forward(q, k, v, mask, BLOCK_Q, BLOCK_K, mask_metadata, return_lse, kernel)
+    if out is not None:
+        return out
+    # Sizes the kernels do not tile by (everything else about the arguments has been checked).
     B, H, Sq, D = q.shape
     Sk = k.shape[-2]
-    if k.shape != (B, H, Sk, D) or v.shape != (B, H, Sk, D):
-        raise ValueError(f"k/v shapes {tuple(k.shape)}/{tuple(v.shape)} do not match q {tuple(q.shape)}")
-    if not q.is_cuda:
-        raise RuntimeError("sparse_attention needs q, k, v on a ROCm GPU; there is no CPU path")
-    _same_device(q, k=k, v=v, mask=mask)
-    if q.dtype not in _FWD_DTYPES or k.dtype != q.dtype or v.dtype != q.dtype:
-        raise TypeError(f"q, k, v must share dtype bfloat16, float16 or float32 (got {q.dtype}, {k.dtype}, {v.dtype})")
-    f32 = q.dtype == torch.float32
-    if mask is None and getattr(mask_metadata, "packed_masks", None) is None:
-        raise ValueError("sparse_attention without a mask tensor needs mask_metadata with packed_masks")
     if mask is not None:
         mask = mask.expand(B, H, Sq, Sk)
-    BLOCK_Q, BLOCK_K = int(BLOCK_Q), int(BLOCK_K)
-    if f32 and 1 <= BLOCK_Q <= (256 if D <= 128 else 128) and BLOCK_K >= 1 and Sq % BLOCK_Q == 0 and Sk % BLOCK_K == 0:
-        tiles = (BLOCK_Q, BLOCK_K)  # the float32 kernel tiles by any sizes up to 256 query rows (128 at head dims above 128)
-    else:
-        tiles = kernel_tiles(Sq, Sk, D, BLOCK_Q, BLOCK_K)
+    tiles = kernel_tiles(Sq, Sk, D, BLOCK_Q, BLOCK_K)
     row_multiple = 32 if D <= 128 else 64  # the smallest Q tile the kernels have
     if tiles is None and mask is not None and Sq % row_multiple and Sq % BLOCK_Q == 0 and Sk % BLOCK_K == 0:
         # A row count that no Q tile of the kernels divides (48, 80, ...; fewer than 32 rows at a head dim the few-rows
@@ -195,104 +145,21 @@ def sparse_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, mask: to
                                    *padded_tiles, return_lse=return_lse)
             return (out[0][:, :, :Sq].contiguous(), out[1][:, :, :Sq].contiguous()) if return_lse \
                 else out[:, :, :Sq].contiguous()
-    if tiles != (BLOCK_Q, BLOCK_K):
-        # Tile sizes the kernels do not tile by.  They only say how the mask is cut up, not what is computed, so the
-        # mask is classified again at sizes the kernels have; the lists are kept on the caller's metadata.
-        # what the reference asserts (mask_utils.py:89-90)
-        assert Sq % BLOCK_Q == 0 and Sk % BLOCK_K == 0, \
-            f"Sq={Sq} / Sk={Sk} must be multiples of BLOCK_Q={BLOCK_Q} / BLOCK_K={BLOCK_K}"
-        if tiles is None or mask is None:
-            raise ValueError(f"sparse_attention: no kernel tiles for BLOCK_Q={BLOCK_Q}, BLOCK_K={BLOCK_K} at Sq={Sq}, "
-                             f"Sk={Sk}, D={D}" + ("" if tiles is None else " without a mask tensor to classify again"))
-        again = getattr(mask_metadata, "_retiled", None)
-        if again is None or again[0] != (tiles, mask.data_ptr(), tuple(mask.stride()), mask._version):
-            again = ((tiles, mask.data_ptr(), tuple(mask.stride()), mask._version),
-                     compute_mask_kernel(mask, *tiles, pack_partial=None if Sq >= 32 else False))
-            if mask_metadata is not None:
-                mask_metadata._retiled = again
-        BLOCK_Q, BLOCK_K = tiles
-        mask_metadata = again[1]
-
-    if Sq == BLOCK_Q and Sq < 32 and BLOCK_K >= 16 and not f32:
-        # one Q tile of fewer rows than the forward kernels tile by: the split-KV kernels (they use no schedule, and take
-        # the packed tiles where the metadata carries them, so `mask` may be None there as it may for the forward)
-        return sparse_attention_decode(q, k, v, mask, BLOCK_K, mask_metadata, return_lse=return_lse)
-    sm_scale = D ** (-0.5) * 1 / math.log(2)  # exp2 replaces exp (sparse_attn_kernel.py:152)
-
-    if mask_metadata is None:
-        mask_metadata = compute_mask_kernel(mask, BLOCK_Q, BLOCK_K)
-    fid, fl = mask_metadata.unmasked_kv_ids, mask_metadata.unmasked_lens
-    pid, pl = mask_metadata.masked_kv_ids, mask_metadata.masked_lens
-    nQ, nK = Sq // BLOCK_Q, Sk // BLOCK_K
-    for name, t, shape in (("unmasked_kv_ids", fid, (B, H, nQ, nK)), ("masked_kv_ids", pid, (B, H, nQ, nK)),
-                           ("unmasked_lens", fl, (B, H, nQ)), ("masked_lens", pl, (B, H, nQ))):
-        if tuple(t.shape) != shape or t.dtype != torch.int32 or t.device != q.device:
-            raise ValueError(f"mask_metadata.{name}: expected int32 {shape} on {q.device}, got {t.dtype} {tuple(t.shape)} on {t.device}")
-    _checked_metadata(mask_metadata, Sk, BLOCK_K)
-    if mask is not None:
-        assert mask.dtype == torch.bool, "mask must be a torch.bool tensor"
-    packed = getattr(mask_metadata, "packed_masks", None)
-    if packed is not None:
-        shape = (B, H, nQ, nK, BLOCK_Q * BLOCK_K // 8)
-        if (tuple(packed.shape) != shape or packed.dtype != torch.uint8 or packed.device != q.device
-                or packed.stride()[2:] != (nK * shape[4], shape[4], 1)):
-            raise ValueError(f"mask_metadata.packed_masks: expected uint8 {shape} on {q.device} with contiguous "
-                             f"tiles, got {packed.dtype} {tuple(packed.shape)} strides {packed.stride()}")
-
-    sched = getattr(mask_metadata, "schedule", None)
-    if sched is not None and (sched.dtype != torch.int32 or sched.device != q.device or not sched.is_contiguous()):
-        raise ValueError("mask_metadata.schedule: expected a contiguous int32 tensor on q's device")
-
-    Dk = _kernel_head_dim(D, (64, 128, 256))
-    qc, kc, vc = (_kernel_ready(_pad_head_dim(t, Dk)) for t in (q, k, v))
-    o = torch.empty_like(qc)
-    lib = _native.load()
-    S = _native.strides
-    with torch.cuda.device(q.device):
-        common = (qc.data_ptr(), S(qc.stride()), kc.data_ptr(), S(kc.stride()), vc.data_ptr(), S(vc.stride()),
-                  o.data_ptr(), S(o.stride()),
-                  mask.data_ptr() if mask is not None else None, S(mask.stride()) if mask is not None else None,
-                  fid.data_ptr(), S(fid.stride()), fl.data_ptr(), S(fl.stride()),
-                  pid.data_ptr(), S(pid.stride()), pl.data_ptr(), S(pl.stride()))
-        tail = (B, H, Sq, Sk, Dk, int(BLOCK_Q), int(BLOCK_K), _FWD_DTYPES[q.dtype], sm_scale,
-                torch.cuda.current_stream(q.device).cuda_stream)
-        sched = getattr(mask_metadata, "schedule", None)
-        if kernel == "rotated" and (sched is not None or q.dtype not in _DTYPES):
-            raise ValueError("kernel='rotated' needs bf16/fp16 and mask_metadata without a schedule")
-        lse = torch.empty(B, H, Sq, dtype=torch.float32, device=q.device) if return_lse else None
-        if _short_list_kernel(mask_metadata, q.dtype, Dk, int(BLOCK_Q), int(BLOCK_K), kernel):
-            rc = lib.sa_sparse_attention_fwd_kernel(
-                *common, packed.data_ptr(), S(packed.stride()[:2]), lse.data_ptr() if return_lse else None,
-                S(lse.stride()) if return_lse else None, *tail[:-1], _native.SA_FWD_KERNEL_SHORT_LISTS, tail[-1])
-        elif (sched is None and q.dtype in _DTYPES
-              and (kernel == "rotated" or (kernel in (None, "auto") and getattr(mask_metadata, "list_rotation", 0) > 0))):
-            # the default kernel with the FULL entries of Q tile qt walked from a start that depends on qt
-            group = int(getattr(mask_metadata, "list_rotation", 0)) or 16
-            rc = lib.sa_sparse_attention_fwd_kernel(
-                *common, *((packed.data_ptr(), S(packed.stride()[:2])) if packed is not None else (None, None)),
-                lse.data_ptr() if return_lse else None, S(lse.stride()) if return_lse else None, *tail[:-1],
-                _native.SA_FWD_KERNEL_ROTATED | (group << 8), tail[-1])
-        elif sched is None and (ws_bytes := lib.sa_fwd_split_workspace_bytes(*tail[:8])):
-            # too few Q tiles to fill the device: their lists are shared by several workgroups
-            ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=q.device)
-            rc = lib.sa_sparse_attention_fwd_split(
-                *common, *((packed.data_ptr(), S(packed.stride()[:2])) if packed is not None else (None, None)),
-                lse.data_ptr() if return_lse else None, S(lse.stride()) if return_lse else None, *tail[:-1],
-                ws.data_ptr(), ws_bytes, tail[-1])
-        elif packed is not None or sched is not None or return_lse:
-            pk = (packed.data_ptr(), S(packed.stride()[:2])) if packed is not None else (None, None)
-            sc = ((sched.data_ptr(), sched.numel() * 4, int(getattr(mask_metadata, "schedule_mode", 0)))
-                  if sched is not None else (None, 0, 0))
-            if return_lse:
-                rc = lib.sa_sparse_attention_fwd_lse(*common, *pk, *sc, lse.data_ptr(), S(lse.stride()), *tail)
-            else:
-                rc = lib.sa_sparse_attention_fwd_ex(*common, *pk, *sc, *tail)
-        else:
-            rc = lib.sa_sparse_attention_fwd(*common, *tail)
-    _native.check(rc)
-    if Dk != D:
-        o = o[..., :D].contiguous()
-    return (o, lse) if return_lse else o
+    # The sizes only say how the mask is cut up, not what is computed, so the mask is classified again at sizes the
+    # kernels have; the lists are kept on the caller's metadata.
+    # what the reference asserts (mask_utils.py:89-90)
+    assert Sq % BLOCK_Q == 0 and Sk % BLOCK_K == 0, \
+        f"Sq={Sq} / Sk={Sk} must be multiples of BLOCK_Q={BLOCK_Q} / BLOCK_K={BLOCK_K}"
+    if tiles is None or mask is None:
+        raise ValueError(f"sparse_attention: no kernel tiles for BLOCK_Q={BLOCK_Q}, BLOCK_K={BLOCK_K} at Sq={Sq}, "
+                         f"Sk={Sk}, D={D}" + ("" if tiles is None else " without a mask tensor to classify again"))
+    again = getattr(mask_metadata, "_retiled", None)
+    if again is None or again[0] != (tiles, mask.data_ptr(), tuple(mask.stride()), mask._version):
+        again = ((tiles, mask.data_ptr(), tuple(mask.stride()), mask._version),
+                 compute_mask_kernel(mask, *tiles, pack_partial=None if Sq >= 32 else False))
+        if mask_metadata is not None:
+            mask_metadata._retiled = again
+    return _native.host().forward(q, k, v, mask, *tiles, again[1], return_lse, kernel)
 
 
 def sparse_attention_tiled(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tiling: Tiling, *, return_lse: bool = False):
@@ -330,72 +197,7 @@ def sparse_attention_decode(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, m
     ``packed_masks`` (the default there) the kernels read those bits and ``mask`` may be None (at BLOCK_K = 16 with an odd
     number of query rows the bool mask is read instead).  ``return_lse``: as in :func:`sparse_attention`.
     """
-    if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
-        raise ValueError("q, k, v must be [B,H,S,D]")
-    B, H, Sq, D = q.shape
-    Sk = k.shape[-2]
-    if k.shape != (B, H, Sk, D) or v.shape != (B, H, Sk, D):
-        raise ValueError(f"k/v shapes {tuple(k.shape)}/{tuple(v.shape)} do not match q {tuple(q.shape)}")
-    if not q.is_cuda:
-        raise RuntimeError("sparse_attention_decode needs q, k, v on a ROCm GPU; there is no CPU path")
-    _same_device(q, k=k, v=v, mask=mask)
-    if q.dtype not in _DTYPES or k.dtype != q.dtype or v.dtype != q.dtype:
-        raise TypeError(f"q, k, v must share dtype bfloat16 or float16 (got {q.dtype}, {k.dtype}, {v.dtype})")
-    sm_scale = D ** (-0.5) * 1 / math.log(2)
-    if mask is not None:
-        mask = mask.expand(B, H, Sq, Sk)
-    if mask_metadata is None:
-        if mask is None:
-            raise ValueError("sparse_attention_decode needs the mask or mask_metadata with packed_masks")
-        mask_metadata = compute_mask_kernel(mask, Sq, BLOCK_K)
-    fid, fl = mask_metadata.unmasked_kv_ids, mask_metadata.unmasked_lens
-    pid, pl = mask_metadata.masked_kv_ids, mask_metadata.masked_lens
-    nK = Sk // BLOCK_K
-    for name, t, shape in (("unmasked_kv_ids", fid, (B, H, 1, nK)), ("masked_kv_ids", pid, (B, H, 1, nK)),
-                           ("unmasked_lens", fl, (B, H, 1)), ("masked_lens", pl, (B, H, 1))):
-        if tuple(t.shape) != shape or t.dtype != torch.int32 or t.device != q.device:
-            raise ValueError(f"mask_metadata.{name}: expected int32 {shape} on {q.device}, got {t.dtype} {tuple(t.shape)} on {t.device}")
-    _checked_metadata(mask_metadata, Sk, BLOCK_K)
-    packed = getattr(mask_metadata, "packed_masks", None)
-    if packed is not None:
-        shape = (B, H, 1, nK, Sq * int(BLOCK_K) // 8)
-        if (tuple(packed.shape) != shape or packed.dtype != torch.uint8 or packed.device != q.device
-                or packed.stride()[2:] != (nK * shape[4], shape[4], 1)):
-            raise ValueError(f"mask_metadata.packed_masks: expected uint8 {shape} on {q.device} with contiguous tiles, got "
-                             f"{packed.dtype} {tuple(packed.shape)} strides {packed.stride()}")
-        if int(BLOCK_K) == 16 and Sq % 2:  # (halfword rows: the kernels want an even number of them)
-            packed = None
-    if packed is None:
-        if mask is None:
-            raise ValueError("sparse_attention_decode without a mask tensor needs mask_metadata with packed_masks "
-                             "(and an even number of query rows at BLOCK_K = 16)")
-        assert mask.dtype == torch.bool, "mask must be a torch.bool tensor"
-    Dk = _kernel_head_dim(D, (64, 128))
-    qc, kc, vc = (_kernel_ready(_pad_head_dim(t, Dk)) for t in (q, k, v))
-    o = torch.empty_like(qc)
-    lib = _native.load()
-    S = _native.strides
-    with torch.cuda.device(q.device):
-        if num_splits == 0:
-            num_splits = lib.sa_decode_num_splits(B, H, Sq, Sk, int(BLOCK_K))
-        ws_bytes = lib.sa_decode_workspace_bytes(B, H, Sq, Dk, int(num_splits))
-        ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=q.device) if ws_bytes else None
-        lse = torch.empty(B, H, Sq, dtype=torch.float32, device=q.device) if return_lse else None
-        rc = lib.sa_sparse_attention_decode_ex(
-            qc.data_ptr(), S(qc.stride()), kc.data_ptr(), S(kc.stride()), vc.data_ptr(), S(vc.stride()),
-            o.data_ptr(), S(o.stride()), mask.data_ptr() if mask is not None else None,
-            S(mask.stride()) if mask is not None else None,
-            fid.data_ptr(), S(fid.stride()), fl.data_ptr(), S(fl.stride()),
-            pid.data_ptr(), S(pid.stride()), pl.data_ptr(), S(pl.stride()),
-            packed.data_ptr() if packed is not None else None, S(packed.stride()[:2]) if packed is not None else None,
-            B, H, Sq, Sk, Dk, int(BLOCK_K), _DTYPES[q.dtype], sm_scale, int(num_splits),
-            ws.data_ptr() if ws is not None else None, ws_bytes,
-            lse.data_ptr() if lse is not None else None, S(lse.stride()) if lse is not None else None,
-            torch.cuda.current_stream(q.device).cuda_stream)
-    _native.check(rc)
-    if Dk != D:
-        o = o[..., :D].contiguous()
-    return (o, lse) if return_lse else o
+    return _native.host().decode(q, k, v, mask, int(BLOCK_K), mask_metadata, int(num_splits), return_lse)
 
 
 class BackwardMetadata:
@@ -454,74 +256,19 @@ def sparse_attention_backward(do: torch.Tensor, q: torch.Tensor, k: torch.Tensor
     (128 x 64 both ways), whatever BLOCK_Q / BLOCK_K the forward used.  ``mask`` may be None when ``bwd_metadata``
     carries the packed PARTIAL tiles of both tilings.
     """
-    B, H, Sq, D = q.shape
+    grads = _native.host().backward(do, q, k, v, o, lse, mask, bwd_metadata)
+    if grads is not None:
+        return grads
+    # The kernels tile by 128 rows both ways: zero rows (lse = -inf: rows that attended to nothing) and mask rows and
+    # columns that attend to nothing are added, and the gradients of the added rows dropped.
+    B, H, Sq, _ = q.shape
     Sk = k.shape[-2]
-    if not q.is_cuda:
-        raise RuntimeError("sparse_attention_backward needs its tensors on a ROCm GPU; there is no CPU path")
-    _same_device(q, k=k, v=v, o=o, do=do, lse=lse, mask=mask)
-    if q.dtype not in _DTYPES or any(t.dtype != q.dtype for t in (k, v, o, do)):
-        raise TypeError("q, k, v, o, do must share dtype bfloat16 or float16")
-    if k.shape != (B, H, Sk, D) or v.shape != k.shape or o.shape != q.shape or do.shape != q.shape:
-        raise ValueError(f"shapes: q/o/do must be {(B, H, Sq, D)} and k/v {(B, H, Sk, D)} (got q {tuple(q.shape)}, "
-                         f"k {tuple(k.shape)}, v {tuple(v.shape)}, o {tuple(o.shape)}, do {tuple(do.shape)})")
-    if lse.dtype != torch.float32 or tuple(lse.shape) != (B, H, Sq):
-        raise ValueError(f"lse: expected float32 {(B, H, Sq)}, got {lse.dtype} {tuple(lse.shape)}")
-    if mask is not None:
-        mask = mask.expand(B, H, Sq, Sk)
-        assert mask.dtype == torch.bool, "mask must be a torch.bool tensor"
-    if Sq % 128 or Sk % 128:
-        # the kernels tile by 128 rows both ways: zero rows (lse = -inf: rows that attended to nothing) and mask rows
-        # and columns that attend to nothing are added, and the gradients of the added rows dropped
-        rows = lambda t, n: torch.nn.functional.pad(t, (0, 0, 0, -n % 128))  # noqa: E731
-        dq, dk, dv = sparse_attention_backward(
-            rows(do, Sq), rows(q, Sq), rows(k, Sk), rows(v, Sk), rows(o, Sq),
-            torch.nn.functional.pad(lse, (0, -Sq % 128), value=float("-inf")),
-            None if mask is None else _pad_mask(mask, 128, 128), bwd_metadata)
-        return dq[:, :, :Sq].contiguous(), dk[:, :, :Sk].contiguous(), dv[:, :, :Sk].contiguous()
-    if bwd_metadata is None:
-        if mask is None:
-            raise ValueError("sparse_attention_backward needs the mask or a BackwardMetadata with packed tiles")
-        bwd_metadata = compute_backward_metadata(mask)
-    sm_scale = D ** (-0.5) * 1 / math.log(2)
-    Dk = _kernel_head_dim(D, (64, 128))
-    qc, kc, vc, oc, doc = (_kernel_ready(_pad_head_dim(t, Dk)) for t in (q, k, v, o, do))
-    dq, dk, dv = torch.empty_like(qc), torch.empty_like(kc), torch.empty_like(vc)
-    lib = _native.load()
-    S = _native.strides
-    lists, packs = [], []
-    for md, shape in ((bwd_metadata.by_query, (B, H, Sq // 128, Sk // 64)), (bwd_metadata.by_key, (B, H, Sk // 128, Sq // 64))):
-        for t, shp in ((md.unmasked_kv_ids, shape), (md.unmasked_lens, shape[:3]), (md.masked_kv_ids, shape),
-                       (md.masked_lens, shape[:3])):
-            if tuple(t.shape) != shp or t.dtype != torch.int32 or t.device != q.device:
-                raise ValueError(f"bwd_metadata: expected int32 {shp} on {q.device}, got {t.dtype} {tuple(t.shape)}")
-            lists += [t.data_ptr(), S(t.stride())]
-        _checked_metadata(md, 64 * shape[3], 64)
-        pk = getattr(md, "packed_masks", None)
-        if pk is not None and (tuple(pk.shape) != shape + (1024,) or pk.dtype != torch.uint8 or pk.device != q.device
-                               or pk.stride()[2:] != (shape[3] * 1024, 1024, 1)):
-            raise ValueError(f"bwd_metadata packed_masks: expected uint8 {shape + (1024,)} on {q.device} with "
-                             f"contiguous tiles, got {pk.dtype} {tuple(pk.shape)} strides {pk.stride()}")
-        packs += [pk.data_ptr(), S(pk.stride()[:2])] if pk is not None else [None, None]
-    if mask is None and None in packs:
-        raise ValueError("sparse_attention_backward without a mask needs packed_masks in both lists of bwd_metadata")
-    mt = getattr(bwd_metadata, "transposed_mask", None)
-    if mt is not None and (tuple(mt.shape) != (B, H, Sk, Sq) or mt.dtype != torch.bool or mt.device != q.device):
-        raise ValueError(f"bwd_metadata.transposed_mask: expected bool {(B, H, Sk, Sq)} on {q.device}")
-    with torch.cuda.device(q.device):
-        ws_bytes = lib.sa_bwd_workspace_bytes(B, H, Sq)
-        ws = torch.empty(ws_bytes // 4, dtype=torch.float32, device=q.device)
-        rc = lib.sa_sparse_attention_bwd(
-            qc.data_ptr(), S(qc.stride()), kc.data_ptr(), S(kc.stride()), vc.data_ptr(), S(vc.stride()),
-            oc.data_ptr(), S(oc.stride()), doc.data_ptr(), S(doc.stride()), lse.data_ptr(), S(lse.stride()),
-            dq.data_ptr(), S(dq.stride()), dk.data_ptr(), S(dk.stride()), dv.data_ptr(), S(dv.stride()),
-            mask.data_ptr() if mask is not None else None, S(mask.stride()) if mask is not None else None,
-            mt.data_ptr() if mt is not None else None, S(mt.stride()) if mt is not None else None,
-            *packs, *lists, ws.data_ptr(), ws_bytes,
-            B, H, Sq, Sk, Dk, _DTYPES[q.dtype], sm_scale, torch.cuda.current_stream(q.device).cuda_stream)
-    _native.check(rc)
-    if Dk != D:
-        dq, dk, dv = (t[..., :D].contiguous() for t in (dq, dk, dv))
-    return dq, dk, dv
+    rows = lambda t, n: torch.nn.functional.pad(t, (0, 0, 0, -n % 128))  # noqa: E731
+    dq, dk, dv = sparse_attention_backward(
+        rows(do, Sq), rows(q, Sq), rows(k, Sk), rows(v, Sk), rows(o, Sq),
+        torch.nn.functional.pad(lse, (0, -Sq % 128), value=float("-inf")),
+        None if mask is None else _pad_mask(mask.expand(B, H, Sq, Sk), 128, 128), bwd_metadata)
+    return dq[:, :, :Sq].contiguous(), dk[:, :, :Sk].contiguous(), dv[:, :, :Sk].contiguous()
 
 
 class _SparseAttentionFunction(torch.autograd.Function):
@@ -543,7 +290,10 @@ def sparse_attention_trainable(q, k, v, mask, BLOCK_Q, BLOCK_K, mask_metadata: M
                                bwd_metadata: BackwardMetadata | None = None) -> torch.Tensor:
     """:func:`sparse_attention` as a differentiable torch function (gradients for q, k, v through
     :func:`sparse_attention_backward`)."""
-    return _SparseAttentionFunction.apply(q, k, v, mask, BLOCK_Q, BLOCK_K, mask_metadata, bwd_metadata)
+    out = _native.host().trainable(q, k, v, mask, int(BLOCK_Q), int(BLOCK_K), mask_metadata, bwd_metadata)
+    if out is None:  # sizes that the wrappers pad or tile anew
+        out = _SparseAttentionFunction.apply(q, k, v, mask, BLOCK_Q, BLOCK_K, mask_metadata, bwd_metadata)
+    return out
 
 
 def merge_attention_parts(o_parts: torch.Tensor, lse_parts: torch.Tensor, return_lse: bool = False):
