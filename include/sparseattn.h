@@ -38,7 +38,7 @@
 extern "C" {
 #endif
 
-#define SA_ABI_VERSION 15
+#define SA_ABI_VERSION 16
 
 enum sa_status {
     SA_OK = 0,
@@ -363,6 +363,23 @@ int sa_sparse_attention_fwd_split(const void *q, const int64_t q_strides[4], con
                                   const int64_t packed_strides[2], float *lse, const int64_t lse_strides[3], int B,
                                   int H, int Sq, int Sk, int D, int BQ, int BK, int dtype, float sm_scale_log2,
                                   void *workspace, size_t workspace_bytes, void *stream);
+
+/*
+ * The same forward for tensors smaller than the tile grid of their mask, and for head dims between the kernels': the lists
+ * and the packed PARTIAL tiles are those of a padded mask of grid_Sq x grid_Sk entries (multiples of BQ and BK) in which
+ * the tensors' Sq queries and Sk keys start at q_offset and k_offset; what lies outside attends to nothing and is attended
+ * by nothing.  q, k, v and o have Sq or Sk rows of D elements and are neither padded nor copied.
+ * bf16 or fp16, D a multiple of 8 up to 128, BQ 32, 64 or 128, packed tiles.  lse [B,H,Sq] or NULL.
+ */
+int sa_sparse_attention_fwd_ragged(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
+                                   const void *v, const int64_t v_strides[4], void *o, const int64_t o_strides[4],
+                                   const int32_t *full_ids, const int64_t full_ids_strides[4], const int32_t *full_lens,
+                                   const int64_t full_lens_strides[3], const int32_t *part_ids,
+                                   const int64_t part_ids_strides[4], const int32_t *part_lens,
+                                   const int64_t part_lens_strides[3], const uint8_t *packed,
+                                   const int64_t packed_strides[2], float *lse, const int64_t lse_strides[3], int B,
+                                   int H, int Sq, int Sk, int D, int BQ, int BK, int q_offset, int k_offset, int grid_Sq,
+                                   int grid_Sk, int dtype, float sm_scale_log2, void *stream);
 
 /*
  * The forward for few query rows against a long K/V (decode): Sq <= 32 rows form the single Q tile of every (b, h),

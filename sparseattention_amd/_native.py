@@ -10,7 +10,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libsparseattn_hip.so")
 
-SA_ABI_VERSION = 15
+SA_ABI_VERSION = 16
 SA_OK = 0
 SA_ERR_INVALID_ARGUMENT = -1
 SA_ERR_UNSUPPORTED = -2
@@ -46,6 +46,7 @@ EXPORTS = (
     "sa_sparse_attention_fwd_kernel",
     "sa_fwd_split_workspace_bytes",
     "sa_sparse_attention_fwd_split",
+    "sa_sparse_attention_fwd_ragged",
     "sa_decode_num_splits",
     "sa_decode_workspace_bytes",
     "sa_sparse_attention_decode",
@@ -135,6 +136,10 @@ def load() -> ctypes.CDLL:
     lib.sa_sparse_attention_fwd_split.argtypes = (
         [_vp, _i64p] * 4 + [_vp, _i64p] + [_vp, _i64p] * 4 + [_vp, _i64p] + [_vp, _i64p] + [ctypes.c_int] * 8
         + [ctypes.c_float] + [_vp, ctypes.c_size_t] + [_vp]
+    )
+    lib.sa_sparse_attention_fwd_ragged.restype = ctypes.c_int
+    lib.sa_sparse_attention_fwd_ragged.argtypes = (
+        [_vp, _i64p] * 4 + [_vp, _i64p] * 4 + [_vp, _i64p] * 2 + [ctypes.c_int] * 12 + [ctypes.c_float, _vp]
     )
     lib.sa_sparse_attention_decode.argtypes = (
         [_vp, _i64p] * 4 + [_vp, _i64p] + [_vp, _i64p] * 4 + [ctypes.c_int] * 7 + [ctypes.c_float, ctypes.c_int]

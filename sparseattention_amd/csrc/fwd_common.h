@@ -128,6 +128,21 @@ __device__ __forceinline__ void dma16(const void *base, uint32_t lane_offset, ui
     }
 }
 
+// The same with an address per lane.
+__device__ __forceinline__ void dma16_lane(const void *lane_addr, uint32_t lds_addr) {
+    lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
+    asm volatile(
+        "s_mov_b32 m0, %1\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %0, off"
+        :
+        : "v"(lane_addr), "s"(lds_addr)
+        : "memory");
+}
+
+// What a lane whose 16 bytes do not exist fetches.
+__device__ const uint32_t kZeros[4] __attribute__((aligned(16))) = {0u, 0u, 0u, 0u};
+
 // N dwords from N wave-uniform addresses by scalar loads that are issued back to back and share ONE wait.  Left to
 // the compiler, loads whose addresses it forms one after the other are waited for one after the other as well, a
 // memory round trip each; at the start of a Q tile that is most of the time before the first K/V request.

@@ -313,6 +313,26 @@ bool tiles_as_asked(int64_t Sq, int64_t Sk, int64_t D, int64_t BQ, int64_t BK, b
 // 2100 keys and more +5 ... +8 %: the third workgroup per compute unit pays for itself on the shortest lists only.
 constexpr double kShortListKeys = 512;
 
+// Whether tensors of these sizes run on a larger tile grid as they are (sa_sparse_attention_fwd_ragged): nothing is padded.
+bool ragged_has(const Tensor &q, int64_t BQ, int64_t BK, const Lists &l) {
+    const int dt = dtype_code(q.scalar_type());
+    return (dt == SA_DTYPE_BF16 || dt == SA_DTYPE_FP16) && q.size(3) % 8 == 0 && q.size(3) <= 128 && (BQ == 32 || BQ == 64 || BQ == 128) &&
+           pow2_from_16(BK) && l.packed.has_value();
+}
+Out ragged_forward(const Tensor &q, const Tensor &k, const Tensor &v, const Lists &l, int64_t BQ, int64_t BK, int64_t q0, int64_t k0, int64_t Pq,
+                   int64_t Pk, bool return_lse) {
+    const int64_t B = q.size(0), H = q.size(1), Sq = q.size(2), D = q.size(3), Sk = k.size(2);
+    const c10::DeviceGuard guard(q.device());
+    const Tensor qc = kernel_ready(q), kc = kernel_ready(k), vc = kernel_ready(v), o = at::empty_like(qc);
+    OptTensor lse;
+    if (return_lse) lse = at::empty({B, H, Sq}, at::TensorOptions().dtype(at::kFloat).device(q.device()));
+    check_rc(sa_sparse_attention_fwd_ragged(qc.data_ptr(), st(qc), kc.data_ptr(), st(kc), vc.data_ptr(), st(vc), o.data_ptr(), st(o), ptr<int32_t>(l.fid),
+                                            st(l.fid), ptr<int32_t>(l.fl), st(l.fl), ptr<int32_t>(l.pid), st(l.pid), ptr<int32_t>(l.pl), st(l.pl),
+                                            ptr<uint8_t>(*l.packed), st(*l.packed), ptr<float>(lse), st(lse), B, H, Sq, Sk, D, BQ, BK, q0, k0, Pq, Pk,
+                                            dtype_code(q.scalar_type()), (float)scale_log2(D), stream_of(q)));
+    return {o, lse};
+}
+
 // The forward where the kernels tile by the caller's sizes, or nothing (then the wrapper makes other tiles of the mask).
 std::optional<Out> forward_impl(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &mask_in, int64_t BQ, int64_t BK, py::handle md,
                                 bool return_lse, const std::string &kernel) {
@@ -380,6 +400,9 @@ std::optional<Out> forward_impl(const Tensor &q, const Tensor &k, const Tensor &
         code = SA_FWD_KERNEL_ROTATED | ((int)(rotation ? rotation : 16) << 8);
     }
 
+    if (D != Dk && !sched && code == SA_FWD_KERNEL_DEFAULT && ragged_has(q, BQ, BK, l))
+        return ragged_forward(q, k, v, l, BQ, BK, 0, 0, Sq, Sk, return_lse);
+
     const c10::DeviceGuard guard(q.device());
     const Tensor qc = kernel_ready(pad_head_dim(q, Dk)), kc = kernel_ready(pad_head_dim(k, Dk)), vc = kernel_ready(pad_head_dim(v, Dk));
     const Tensor o = at::empty_like(qc);
@@ -416,6 +439,19 @@ py::object forward(const Tensor &q, const Tensor &k, const Tensor &v, const OptT
                    const std::string &kernel) {
     const auto r = forward_impl(q, k, v, mask, BQ, BK, md, return_lse, kernel);
     return r ? as_object(*r) : py::none();
+}
+
+// The forward on the tile grid of a padded mask (sparse_attention_tiled), or None where the wrapper has to pad the tensors.
+py::object forward_tiled(const Tensor &q, const Tensor &k, const Tensor &v, int64_t BQ, int64_t BK, int64_t q0, int64_t k0, int64_t Pq, int64_t Pk,
+                         py::object md, bool return_lse) {
+    check_qkv(q, k, v, std::nullopt, "sparse_attention");
+    if (k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type() || BQ < 1 || BK < 1 || Pq % BQ || Pk % BK) return py::none();
+    const Lists l = lists_of(md);
+    if (!ragged_has(q, BQ, BK, l) || attr(md, "schedule")) return py::none();
+    check_lists(l, q, q.size(0), q.size(1), Pq / BQ, Pk / BK, "tiling.metadata");
+    checked_metadata(md, l, Pk, BK);
+    check_packed(*l.packed, q, q.size(0), q.size(1), Pq / BQ, Pk / BK, BQ * BK / 8, "tiling.metadata");
+    return as_object(ragged_forward(q, k, v, l, BQ, BK, q0, k0, Pq, Pk, return_lse));
 }
 
 // ---- backward -----------------------------------------------------------------------------------------------------
@@ -569,6 +605,7 @@ py::object trainable(const Tensor &q, const Tensor &k, const Tensor &v, const Op
 PYBIND11_MODULE(_host, m) {
     m.doc() = "Checks, allocations and launches of the wrappers in sparse_attn_kernel.py and mask_utils.py.";
     m.def("forward", &forward);
+    m.def("forward_tiled", &forward_tiled);
     m.def("decode", &decode);
     m.def("classify", &classify);
     m.def("classify_terms", &classify_terms);

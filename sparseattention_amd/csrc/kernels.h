@@ -132,6 +132,10 @@ struct FwdParams {
     //   ws_ml [B*H*nQ][nsplit][BQ][2] floats: reference value (-inf: no attended key) and sum of every row
     int nsplit, split_chunks;  // split_chunks: chunks of one part (the last ones may be shorter)
     float *ws, *ws_ml;
+    // Ragged sizes: the tile grid (Sq, Sk, nQ, nK, lists, packed tiles) is that of a padded mask, the tensors have Sq_in
+    // and Sk_in rows, which stand q0 and k0 rows into the grid, of D_in elements (a multiple of 8, at most the kernel's D).
+    int ragged;
+    int q0, k0, Sq_in, Sk_in, D_in;
 };
 
 // How many workgroups share a list of NE entries of 2^lbk keys, walked in chunks of 2^lck keys, and the first entry of

@@ -41,17 +41,6 @@ __device__ __forceinline__ void f32_dma4(const void *lane_addr, uint32_t lds_add
         : "v"(lane_addr), "s"(lds_addr)
         : "memory");
 }
-__device__ __forceinline__ void f32_dma16(const void *lane_addr, uint32_t lds_addr) {
-    lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
-    asm volatile(
-        "s_mov_b32 m0, %1\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %0, off"
-        :
-        : "v"(lane_addr), "s"(lds_addr)
-        : "memory");
-}
-
 // MODE 0: BK = 16 (two list entries per chunk), MODE 1: BK = 32, MODE 2: BK >= 64 (BK/32 chunks per entry).
 // PK: mask entries of PARTIAL tiles from the bit-packed tiles; else from the bool mask (key stride 1, rows and base
 // 16-byte aligned: checked by the launcher).
@@ -180,8 +169,8 @@ __global__ __launch_bounds__(NW * 64, NW >= 4 ? 2 : 1) void sparse_fwd_f32_mfma_
                                  16 * (ld_slot ^ ((kswz | ld_r) & 15));
             const uint8_t *vs_ = reinterpret_cast<const uint8_t *>(vbase + (int64_t)col * p.vs[2]) + ld_vbase +
                                  16 * (ld_slot ^ (vswz ^ (8 * ((ld_r >> 2) & 1))));
-            f32_dma16(ks_, lds0 + buf * KBUF + row0 * ROWB);
-            f32_dma16(vs_, lds0 + OFF_V + buf * KBUF + row0 * ROWB);
+            dma16_lane(ks_, lds0 + buf * KBUF + row0 * ROWB);
+            dma16_lane(vs_, lds0 + OFF_V + buf * KBUF + row0 * ROWB);
         }
         // mask words of this wave's 32 rows
         const uint32_t mdst = lds0 + OFF_M + buf * MBUF + wave_u * 1024;
@@ -197,7 +186,7 @@ __global__ __launch_bounds__(NW * 64, NW >= 4 ? 2 : 1) void sparse_fwd_f32_mfma_
         } else {
             // 16 mask bytes per lane: keys 16 hh .. 16 hh + 15 of the chunk (BK = 16: entry hh)
             const int col = MODE == 0 ? (hh ? pl.col[EPC - 1] : pl.col[0]) : pl.col[0] + 16 * hh;
-            f32_dma16(mrow0 + (int64_t)(wave * 32 + l32) * p.ms[2] + col, mdst);
+            dma16_lane(mrow0 + (int64_t)(wave * 32 + l32) * p.ms[2] + col, mdst);
         }
     };
 

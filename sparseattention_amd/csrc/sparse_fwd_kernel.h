@@ -70,10 +70,17 @@ __device__ __forceinline__ void wait_vm_at_most(int n, int step) {
 // fill the device: a chunk of a prompt against a long cache.  Every workgroup walks a range of its own and leaves
 // unnormalised rows with their reference values and sums in p.ws, which fwd_merge_kernel adds up; a tile whose list is
 // too short to be shared is written as by the plain kernel.
-template <int DT, int D, int NW, int MODE, int NS, bool PP, bool PK, bool PS, bool SP>
+// RG: the tile grid is larger than the tensors (p.q0, p.k0: rows of it in front of the first query and key; p.Sq_in, p.Sk_in:
+// rows there are) and the head dim may be smaller than D (p.D_in, a multiple of 8).  Nothing is padded in memory: queries
+// and pieces of rows that do not exist enter as zeros (pieces from a zero in device memory, since a direct load brings
+// every lane 16 bytes), keys before the first and behind the last one as that one, which the mask of their tile leaves
+// out, and what has no place in the output is not stored.  The address of a direct load is formed per lane then, some six
+// instructions each.  B2 H16 S1499 D80 against padding q, k, v and cutting the result (14 launches): 82 -> 22 us.
+template <int DT, int D, int NW, int MODE, int NS, bool PP, bool PK, bool PS, bool SP, bool RG>
 __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse_fwd_kernel(const FwdParams p) {
     static_assert(!PS || (!PP && NS == 2), "persistent workgroups use the two-stage loop");
     static_assert(!SP || (!PS && !PP && D <= 128), "shared lists use the plain loop");
+    static_assert(!RG || (PK && !SP && !PS && !PP && D <= 128), "ragged sizes use the plain loop and packed tiles");
     using E = Elem<DT>;
     constexpr int ROWB = D * 2;                   // bytes per K/V row in LDS
     constexpr int KBUF = 64 * ROWB, VBUF = 64 * ROWB;
@@ -153,17 +160,24 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
         prow = m.prow;
         fid = p.full_ids + b * p.fis[0] + h * p.fis[1] + qt * p.fis[2];
         pid = p.part_ids + b * p.pis[0] + h * p.pis[1] + qt * p.pis[2];
-        const int qrow_ = qt * (NW * 32) + wave * 32 + l32;
+        const int qrow_ = qt * (NW * 32) + wave * 32 + l32 - (RG ? p.q0 : 0);
         orow_off = b * p.os[0] + h * p.os[1] + (int64_t)qrow_ * p.os[2] + 4 * hh;
         lse_off = b * p.lses[0] + h * p.lses[1] + (int64_t)qrow_ * p.lses[2];
     };
     // Q^T operand: lane (l32, hh) keeps d = 16c + 8hh .. +7 of its query row for every 16-wide step c.
     u32x4 qf[D / 16];
     auto load_q = [&](int b_, int h_, int qt_) {
-        const int qrow_ = qt_ * (NW * 32) + wave * 32 + l32;
+        const int qrow_ = qt_ * (NW * 32) + wave * 32 + l32 - (RG ? p.q0 : 0);
         const uint16_t *qp = p.q + b_ * p.qs[0] + h_ * p.qs[1] + (int64_t)qrow_ * p.qs[2] + 8 * hh;
 #pragma unroll
-        for (int c = 0; c < D / 16; c++) qf[c] = *(const u32x4 *)(qp + 16 * c);
+        for (int c = 0; c < D / 16; c++) {
+            if constexpr (RG) {
+                qf[c] = u32x4{0u, 0u, 0u, 0u};
+                if ((unsigned)qrow_ < (unsigned)p.Sq_in && 16 * c + 8 * hh < p.D_in) qf[c] = *(const u32x4 *)(qp + 16 * c);
+            } else {
+                qf[c] = *(const u32x4 *)(qp + 16 * c);
+            }
+        }
     };
     // The scale (softmax scale / ln 2) goes into Q once, so that the S MFMAs deliver exp2 arguments.
     auto scale_q = [&]() {
@@ -495,6 +509,7 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
     // therefore hands them out one at a time between the MFMA bundles of the chunk being computed.
     struct StagePlan {
         const uint16_t *kp[EPC], *vp[EPC];  // first row of every list entry of the chunk (scalar registers)
+        int col[RG ? EPC : 1];              // RG: its first key column instead
     };
     // first row of a list entry as an element offset: key column and row stride are both below 2^32 (the strides
     // are checked on the host), so one 32 x 32 -> 64 bit product does
@@ -503,12 +518,34 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
     auto plan_chunk = [&](const int(&col)[EPC], StagePlan &pl) {
 #pragma unroll
         for (int j = 0; j < EPC; j++) {
-            pl.kp[j] = kbase + row_off(col[j], ks2);
-            pl.vp[j] = vbase + row_off(col[j], vs2);
+            if constexpr (RG) {
+                pl.col[j] = col[j];
+            } else {
+                pl.kp[j] = kbase + row_off(col[j], ks2);
+                pl.vp[j] = vbase + row_off(col[j], vs2);
+            }
         }
     };
     auto stage_piece = [&](int buf, int piece, const StagePlan &pl) {
         const int i = piece >> 1;
+        if constexpr (RG) {
+            const bool is_k = (piece & 1) == 0;
+            const int r = RPI * (NW * i + wave_u) + ld_r0;  // this lane's row of the chunk
+            const int j0 = MODE == 2 ? 0 : ((RPI * (NW * i + wave_u)) >> LBKC);
+            int first = pl.col[0];
+#pragma unroll
+            for (int jj = 1; jj < EPC; jj++) {
+                int cand = pl.col[jj];
+                if constexpr (EPC > 2) asm volatile("" : "+s"(cand));  // (see below: no load at a variable index)
+                if (j0 == jj) first = cand;
+            }
+            const int row = min(max(first + (MODE == 2 ? r : (r & ((1 << LBKC) - 1))) - p.k0, 0), p.Sk_in - 1);
+            const int src = 8 * (ld_slot ^ (is_k ? k_swizzle<D>(r) : v_swizzle<D>(r)));  // element of the row
+            const uint16_t *a = (is_k ? kbase : vbase) + (int64_t)((uint64_t)(uint32_t)row * (is_k ? ks2 : vs2)) + src;
+            const uint16_t *lane_addr = src < p.D_in ? a : reinterpret_cast<const uint16_t *>(kZeros);
+            dma16_lane(lane_addr, lds0 + (is_k ? 0 : NS * KBUF) + buf * (is_k ? KBUF : VBUF) + RPI * (NW * i + wave_u) * ROWB);
+            return;
+        }
         // rows [rbase, rbase + RPI) lie inside one list entry; when the rows of all waves of load i do, the
         // entry is known at compile time
         constexpr bool kEntryByLoad = MODE == 2 || RPI * NW <= (1 << LBKC);
@@ -809,7 +846,8 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
     auto store_o_rows = [&]() {
         const float l_tot = l32 < 16 ? acc_l[0] : acc_l[1];
         const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-        if (p.lse != nullptr && hh == 0)
+        const int row0 = qt * (NW * 32) + wave * 32 - (RG ? p.q0 : 0);  // the wave's first row of the output
+        if (p.lse != nullptr && hh == 0 && (!RG || (unsigned)(row0 + l32) < (unsigned)p.Sq_in))
             p.lse[lse_off] = l_tot > 0.f ? (m_ref + __builtin_amdgcn_logf(l_tot)) * 0.69314718056f : kNegInf;
         constexpr int OROW = ROWB + 16;
         static_assert(NW * 32 * OROW <= 2 * NS * 64 * ROWB, "the rows of all waves fit the K/V stages");
@@ -823,11 +861,12 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
                 *(u32x2 *)(ob + l32 * OROW + 2 * (32 * db + 8 * g + 4 * hh)) = w;
             }
         // 64 lanes x 16 bytes = 1024 / ROWB rows per store
-        uint16_t *const o0 = p.o + b * p.os[0] + h * p.os[1] + (int64_t)(qt * (NW * 32) + wave * 32) * p.os[2];
+        uint16_t *const o0 = p.o + b * p.os[0] + h * p.os[1] + (int64_t)row0 * p.os[2];
 #pragma unroll
         for (int i = 0; i < 32 * PPR / 64; i++) {
             const int idx = 64 * i + lane, r = idx / PPR, pc = idx % PPR;
             const u32x4 x = *(const u32x4 *)(ob + r * OROW + 16 * pc);
+            if (RG && ((unsigned)(row0 + r) >= (unsigned)p.Sq_in || 8 * pc >= p.D_in)) continue;
             // (written once, whole rows: a streaming store leaves the lines of K and V in L2 alone)
             __builtin_nontemporal_store(x, (u32x4 *)(o0 + (int64_t)r * p.os[2] + 8 * pc));
         }
@@ -1161,7 +1200,8 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
                         if (b == 0) entries_use(t2, raw, col2, valid2, part2);
 #pragma unroll
                         for (int i = b * per; i < (b + 1) * per && i < 2 * EPC; i++) {
-                            if (i & 1) pl2.vp[i >> 1] = vbase + row_off(col2[i >> 1], vs2);
+                            if constexpr (RG) pl2.col[i >> 1] = col2[i >> 1];
+                            else if (i & 1) pl2.vp[i >> 1] = vbase + row_off(col2[i >> 1], vs2);
                             else pl2.kp[i >> 1] = kbase + row_off(col2[i >> 1], ks2);
                         }
                         if (b == nb - 1) entries_read(t3, raw);
@@ -1202,14 +1242,14 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
     store_o_rows();
 }
 
-// HOW 0: one workgroup per Q tile, 1: persistent workgroups, 2: lists shared by workgroups (SP)
+// HOW 0: one workgroup per Q tile, 1: persistent workgroups, 2: lists shared by workgroups (SP), 3: ragged sizes (RG)
 template <int DT, int D, int NW, int MODE, bool PK, int HOW>
 hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     // Eight waves fill a CU's register file on their own, so that workgroup can have most of the LDS: 4 stages.
     constexpr int NS = NW == 8 ? 4 : 2;
     static_assert(kListCap == 2 * kPsListCap, "one long list or two short ones in the same LDS");
     constexpr int smem = 2 * NS * 64 * D * 2 + kListCap * 4;  // NS stages of 64 rows for K and for V + the list(s)
-    auto kern = sparse_fwd_kernel<DT, D, NW, MODE, NS, NW == 8, PK, HOW == 1, HOW == 2>;
+    auto kern = sparse_fwd_kernel<DT, D, NW, MODE, NS, NW == 8, PK, HOW == 1, HOW == 2, HOW == 3>;
     static unsigned long long attr_done = 0;  // devices on which this kernel may use `smem` bytes of LDS
     if (const hipError_t e0 = allow_dynamic_smem(kern, smem, attr_done); e0 != hipSuccess) return e0;
     const unsigned grid = HOW == 1 ? (unsigned)p.sched_G
@@ -1234,7 +1274,7 @@ hipError_t launch_bq(const FwdParams &p, int BQ, hipStream_t stream) {
         case 64: return launch_mode<DT, D, 2, PK, HOW>(p, stream);
         case 128: return launch_mode<DT, D, 4, PK, HOW>(p, stream);
         case 256:
-            // 8-wave workgroups are neither persistent nor share lists, and their four stages do not fit the LDS at D = 256
+            // 8-wave workgroups have the plain form only, and their four stages do not fit the LDS at D = 256
             if constexpr (HOW != 0 || D > 128) return hipErrorInvalidValue;
             else return launch_mode<DT, D, 8, PK, 0>(p, stream);
         default: return hipErrorInvalidValue;
@@ -1253,7 +1293,7 @@ hipError_t launch_fwd_variant(const FwdParams &p, int D, int BQ, hipStream_t str
         case 128: return launch_bq<DT, 128, PK, HOW>(p, BQ, stream);
         case 256:
             // one workgroup per CU (its two stages of K and V take 128 KiB of LDS) with the whole register file:
-            // one wave per SIMD; no schedules, no shared lists
+            // one wave per SIMD; the plain form only
             if constexpr (HOW != 0) return hipErrorInvalidValue;
             else return launch_bq<DT, 256, PK, 0>(p, BQ, stream);
         default: return hipErrorInvalidValue;

@@ -253,6 +253,11 @@ size_t split_shape(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtyp
     return *nsplit > 1 ? (size_t)tiles * (size_t)*nsplit * (size_t)BQ * (size_t)(D + 2) * 4 : 0;
 }
 
+// Tensors that are smaller than the tile grid of their mask (FwdParams::ragged).
+struct Ragged {
+    int q0, k0, Sq, Sk, D;
+};
+
 int forward_impl(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4], const void *v,
                  const int64_t v_strides[4], void *o, const int64_t o_strides[4], const uint8_t *mask,
                  const int64_t mask_strides[4], const int32_t *full_ids, const int64_t full_ids_strides[4],
@@ -261,7 +266,8 @@ int forward_impl(const void *q, const int64_t q_strides[4], const void *k, const
                  const uint8_t *packed, const int64_t packed_strides[2], bool use_packed, const int32_t *schedule,
                  size_t schedule_bytes, int schedule_mode, float *lse, const int64_t lse_strides[3], int B, int H,
                  int Sq, int Sk, int D, int BQ, int BK, int dtype, float sm_scale_log2, void *stream,
-                 int kernel = SA_FWD_KERNEL_DEFAULT, void *workspace = nullptr, size_t workspace_bytes = 0) {
+                 int kernel = SA_FWD_KERNEL_DEFAULT, void *workspace = nullptr, size_t workspace_bytes = 0,
+                 const Ragged *ragged = nullptr) {
     g_error[0] = 0;
     const int rot_group = kernel >> 8;
     kernel &= 0xff;
@@ -379,6 +385,14 @@ int forward_impl(const void *q, const int64_t q_strides[4], const void *k, const
             return fail(SA_ERR_INVALID_ARGUMENT, "sa_sparse_attention_fwd_lse: lse must be 4-byte aligned and must not alias itself (zero stride)");
         fp.lse = lse;
         for (int i = 0; i < 3; i++) fp.lses[i] = lse_strides[i];
+    }
+    if (ragged) {
+        fp.ragged = 1;
+        fp.q0 = ragged->q0;
+        fp.k0 = ragged->k0;
+        fp.Sq_in = ragged->Sq;
+        fp.Sk_in = ragged->Sk;
+        fp.D_in = ragged->D;
     }
     fp.nsplit = 1;
     if (workspace && kernel == SA_FWD_KERNEL_DEFAULT && !fp.sched) {
@@ -531,6 +545,34 @@ int sa_sparse_attention_fwd_split(const void *q, const int64_t q_strides[4], con
                         full_ids_strides, full_lens, full_lens_strides, part_ids, part_ids_strides, part_lens,
                         part_lens_strides, packed, packed_strides, use_packed, nullptr, 0, 0, lse, lse_strides, B, H, Sq,
                         Sk, D, BQ, BK, dtype, sm_scale_log2, stream, SA_FWD_KERNEL_DEFAULT, workspace, workspace_bytes);
+}
+
+int sa_sparse_attention_fwd_ragged(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
+                                   const void *v, const int64_t v_strides[4], void *o, const int64_t o_strides[4],
+                                   const int32_t *full_ids, const int64_t full_ids_strides[4], const int32_t *full_lens,
+                                   const int64_t full_lens_strides[3], const int32_t *part_ids,
+                                   const int64_t part_ids_strides[4], const int32_t *part_lens,
+                                   const int64_t part_lens_strides[3], const uint8_t *packed,
+                                   const int64_t packed_strides[2], float *lse, const int64_t lse_strides[3], int B,
+                                   int H, int Sq, int Sk, int D, int BQ, int BK, int q_offset, int k_offset, int grid_Sq,
+                                   int grid_Sk, int dtype, float sm_scale_log2, void *stream) {
+    g_error[0] = 0;
+    if (!packed || !packed_strides) return fail(SA_ERR_INVALID_ARGUMENT, "sa_sparse_attention_fwd_ragged: null pointer argument (packed)");
+    if ((B > 1 && packed_strides[0] % 4) || (H > 1 && packed_strides[1] % 4) || !aligned(packed, 4))
+        return fail(SA_ERR_UNSUPPORTED, "sa_sparse_attention_fwd_ragged: packed needs a 4-byte aligned base and plane strides");
+    if (Sq <= 0 || Sk <= 0 || q_offset < 0 || k_offset < 0 || (int64_t)q_offset + Sq > grid_Sq || (int64_t)k_offset + Sk > grid_Sk)
+        return fail(SA_ERR_INVALID_ARGUMENT, "sa_sparse_attention_fwd_ragged: %d queries at %d and %d keys at %d do not fit a grid of %d x %d", Sq, q_offset, Sk, k_offset, grid_Sq, grid_Sk);
+    if (dtype != SA_DTYPE_BF16 && dtype != SA_DTYPE_FP16)
+        return fail(SA_ERR_UNSUPPORTED, "sa_sparse_attention_fwd_ragged: dtype code %d (supported: 0 = bf16, 1 = fp16)", dtype);
+    if (D <= 0 || D > 128 || D % 8)
+        return fail(SA_ERR_UNSUPPORTED, "sa_sparse_attention_fwd_ragged: head dim %d (supported: multiples of 8 up to 128)", D);
+    if (BQ != 32 && BQ != 64 && BQ != 128)
+        return fail(SA_ERR_UNSUPPORTED, "sa_sparse_attention_fwd_ragged: BLOCK_Q %d (supported: 32, 64, 128)", BQ);
+    const Ragged ragged{q_offset, k_offset, Sq, Sk, D};
+    return forward_impl(q, q_strides, k, k_strides, v, v_strides, o, o_strides, nullptr, nullptr, full_ids, full_ids_strides,
+                        full_lens, full_lens_strides, part_ids, part_ids_strides, part_lens, part_lens_strides, packed,
+                        packed_strides, true, nullptr, 0, 0, lse, lse_strides, B, H, grid_Sq, grid_Sk, D <= 64 ? 64 : 128, BQ,
+                        BK, dtype, sm_scale_log2, stream, SA_FWD_KERNEL_DEFAULT, nullptr, 0, &ragged);
 }
 
 int sa_validate_metadata(const int32_t *full_ids, const int64_t full_ids_strides[4], const int32_t *full_lens,

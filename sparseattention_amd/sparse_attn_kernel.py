@@ -166,12 +166,18 @@ def sparse_attention_tiled(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ti
     """:func:`sparse_attention` on the tile grid chosen by :func:`sparseattention_amd.select_tiling`: q, k, v get
     ``q_offset`` / ``k_offset`` zero rows in front (and zero rows at the end up to whole tiles), which the padded mask
     lets nothing attend to or from, and the rows of the result that belong to the caller's queries are returned.  With
-    both offsets 0 and sizes that are whole tiles this is sparse_attention itself; otherwise it costs a copy of q, k, v."""
+    both offsets 0 and sizes that are whole tiles this is sparse_attention itself.  In bf16 and fp16 with packed tiles,
+    BLOCK_Q up to 128 and head dims that are multiples of 8 up to 128 the kernel leaves the rows out that do not exist;
+    otherwise it costs a copy of q, k, v."""
     Sq, Sk = q.shape[-2], k.shape[-2]
     Pq, Pk = tiling.padded_mask.shape[-2:]
     qo, ko = tiling.q_offset, tiling.k_offset
     if not (qo + Sq <= Pq and ko + Sk <= Pk):
         raise ValueError(f"tiling for a mask of {Pq - qo}x{Pk - ko} or smaller, got Sq={Sq}, Sk={Sk}")
+    if (qo, Pq, ko, Pk) != (0, Sq, 0, Sk):
+        out = _native.host().forward_tiled(q, k, v, tiling.BLOCK_Q, tiling.BLOCK_K, qo, ko, Pq, Pk, tiling.metadata, return_lse)
+        if out is not None:
+            return out
     pad = torch.nn.functional.pad
     qp = q if (qo, Pq) == (0, Sq) else pad(q, (0, 0, qo, Pq - qo - Sq))
     kp = k if (ko, Pk) == (0, Sk) else pad(k, (0, 0, ko, Pk - ko - Sk))
