@@ -140,6 +140,18 @@ __device__ __forceinline__ void dma16_lane(const void *lane_addr, uint32_t lds_a
         : "memory");
 }
 
+// 4 bytes per lane: lane i of the wave writes LDS address lds_addr + 4*i.
+__device__ __forceinline__ void dma4_lane(const void *lane_addr, uint32_t lds_addr) {
+    lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
+    asm volatile(
+        "s_mov_b32 m0, %1\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dword %0, off"
+        :
+        : "v"(lane_addr), "s"(lds_addr)
+        : "memory");
+}
+
 // What a lane whose 16 bytes do not exist fetches.
 __device__ const uint32_t kZeros[4] __attribute__((aligned(16))) = {0u, 0u, 0u, 0u};
 

@@ -234,8 +234,15 @@ struct BwdParams {
     int first_tile_first;          // launch order of a plane's tiles: 0 last tile first (queries), 1 first tile first (keys)
     float scale;                   // softmax scale / ln 2 (folded into x)
     float out_scale;               // softmax scale for dQ and dK, 1 for dV
+    uint16_t *out2;                // dV, where one pass makes both
+    int64_t outs2[3];
 };
-hipError_t launch_bwd(const BwdParams &p, int dtype, int D, bool lane_stats, bool out_p, hipStream_t stream);
+// The passes of one launch: workgroup first[i] + t has tile t of pass i.
+struct BwdLaunch {
+    BwdParams pass[3];
+    int first[3], tiles[3];
+};
+hipError_t launch_bwd(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, int dtype, int D, hipStream_t stream);
 
 struct BwdPrepParams {
     const uint16_t *o, *d_o;

@@ -37,22 +37,39 @@ __device__ __forceinline__ int bwd_swizzle(int row) {
     else return (((row >> 1) & 1) << 2) | (((row >> 3) & 1) << 1) | ((row >> 2) & 1);
 }
 
-// LANE_STATS: queries are the resident side (dQ).  OUT_P: the output product takes P and Z (dV) instead of dS and Y.
-template <int DT, int D, bool LANE_STATS, bool OUT_P>
-__global__ __launch_bounds__(256, 2) void sparse_bwd_kernel(const BwdParams p) {
+// What a workgroup makes of its resident tile.
+constexpr int kDQ = 0;   // queries resident
+constexpr int kDK = 1;   // keys resident, as for the following
+constexpr int kDV = 2;
+constexpr int kDKV = 3;  // both from one walk: S and P once instead of twice (D = 64, where two accumulators leave room for
+                         // two waves per SIMD)
+
+// LDS, two stages of each: [Y][Z][stats: 64 L then 64 Delta floats][mask: 8 bytes per resident row][list]
+template <int D, bool PK>
+struct BwdLds {
+    static constexpr int NS = 2;
+    static constexpr int CBUF = 64 * D * 2;  // one streamed chunk of one tensor
+    static constexpr int Z0 = NS * CBUF, STAT0 = 2 * NS * CBUF, MASK0 = STAT0 + NS * 512, LIST0 = MASK0 + (PK ? NS * 1024 : 0);
+    static constexpr int bytes = LIST0 + kBwdListCap * 4;
+};
+
+// PK: the mask entries of PARTIAL tiles come bit-packed from p.packed, else from the bool mask.
+template <int DT, int D, int KIND, bool PK, int PASS>
+__device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, uint8_t *smem) {
     using E = Elem<DT>;
     static_assert(D == 128 || D == 64, "head dim");
     constexpr int ROWB = D * 2;
-    constexpr int CBUF = 64 * ROWB;  // one streamed chunk of one tensor
+    using Lds = BwdLds<D, PK>;
+    constexpr int NS = Lds::NS, CBUF = Lds::CBUF, Z0 = Lds::Z0, STAT0 = Lds::STAT0, MASK0 = Lds::MASK0;
     constexpr int NC = D / 16, NDB = D / 32;
     constexpr int PPR = ROWB / 16;   // 16-byte pieces per row
     constexpr int RPI = 64 / PPR;    // rows per wave-wide direct load (1 KiB)
     constexpr int NLD = 16 / RPI;    // direct loads per wave per chunk and tensor
-    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-    // [Y stage 0,1][Z stage 0,1][stats stage 0,1: 64 L then 64 Delta floats][list]
-    constexpr int STAT0 = 4 * CBUF;
-    constexpr int LIST0 = STAT0 + 2 * 512;
-    int *const ent = reinterpret_cast<int *>(smem + LIST0);
+    constexpr bool LANE_STATS = KIND == kDQ;                // queries are the resident side
+    constexpr bool OUT_P = KIND == kDV;                     // P and Z enter the output product, nothing else is needed
+    constexpr bool BOTH = KIND == kDKV;
+    constexpr int NMW = PK ? 1 : 8;                         // mask words per lane and chunk in registers (PK: in LDS)
+    int *const ent = reinterpret_cast<int *>(smem + Lds::LIST0);
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l32 = lane & 31, hh = lane >> 5;
@@ -60,8 +77,7 @@ __global__ __launch_bounds__(256, 2) void sparse_bwd_kernel(const BwdParams p) {
     // so each XCD gets a contiguous range of the plane-major order (the tiles that share K/V or Q/dO meet in one L2),
     // planes two at a time with their tiles interleaved, the tile that is heaviest under causal-like masks first
     // (the last queries, the first keys: p.first_tile_first).
-    const int total = gridDim.x, per = total >> 3;
-    int lin = blockIdx.x;
+    const int per = total >> 3;
     if (lin < (per << 3)) lin = (lin & 7) * per + (lin >> 3);
     int pair = lin / (2 * p.nR);
     const int pr = lin - pair * 2 * p.nR;
@@ -81,14 +97,9 @@ __global__ __launch_bounds__(256, 2) void sparse_bwd_kernel(const BwdParams p) {
     const uint16_t *zbase = p.z + b * p.zs[0] + h * p.zs[1];
     const int32_t *fid = p.full_ids + b * p.fis[0] + h * p.fis[1] + rt * p.fis[2];
     const int32_t *pid = p.part_ids + b * p.pis[0] + h * p.pis[1] + rt * p.pis[2];
-    // Counts and tile indices are clamped to the nS streamed tiles there are (the reference guards every K/V and mask
-    // load with kv_offset < SEQLEN_K, sparse_attn_kernel.py:35,39,60): stale or foreign metadata then gives wrong
-    // numbers, never an access outside the tensors or past the list's LDS copy (nS <= kBwdListCap, checked by the host).
-    const int F = min(max(p.full_lens[b * p.fls[0] + h * p.fls[1] + rt * p.fls[2]], 0), p.nS);
-    const int T = F + min(max(p.part_lens[b * p.pls[0] + h * p.pls[1] + rt * p.pls[2]], 0), p.nS - F);  // chunks = list entries
-    const uint8_t *mrow = p.mask + b * p.ms[0] + h * p.ms[1] + (int64_t)rrow * p.mrs;
-    // this lane's row in a packed tile: 8 bytes per row, 1024 per tile, nS tiles per resident tile
-    const uint8_t *prow = p.packed + b * p.pks[0] + h * p.pks[1] + (int64_t)rt * p.nS * 1024 + (wave * 32 + l32) * 8;
+    const uint8_t *mrow = PK ? nullptr : p.mask + b * p.ms[0] + h * p.ms[1] + (int64_t)rrow * p.mrs;
+    // packed tiles: 8 bytes per row, 1024 per tile, nS tiles per resident tile; a lane's four bytes of its wave's 32 rows
+    const uint8_t *prow = PK ? p.packed + b * p.pks[0] + h * p.pks[1] + (int64_t)rt * p.nS * 1024 + wave * 256 + 4 * lane : nullptr;
     const float *statL = p.stat_l + b * p.sts[0] + h * p.sts[1];
     const float *statD = p.stat_d + b * p.sts[0] + h * p.sts[1];
     // bytes from a query's L to its Delta (both live in one workspace, less than 4 GiB apart)
@@ -115,11 +126,23 @@ __global__ __launch_bounds__(256, 2) void sparse_bwd_kernel(const BwdParams p) {
         laneL = statL[(int64_t)rrow * p.sts[2]];
         laneD = statD[(int64_t)rrow * p.sts[2]];
     }
-    f32x16 acc[NDB];
+    // Counts and tile indices are clamped to the nS streamed tiles there are (the reference guards every K/V and mask
+    // load with kv_offset < SEQLEN_K, sparse_attn_kernel.py:35,39,60): stale or foreign metadata then gives wrong
+    // numbers, never an access outside the tensors or past the list's LDS copy (nS <= kBwdListCap, checked by the host).
+    int cnt[2];
+    const int32_t *const cnt_addr[2] = {p.full_lens + (b * p.fls[0] + h * p.fls[1] + rt * p.fls[2]),
+                                        p.part_lens + (b * p.pls[0] + h * p.pls[1] + rt * p.pls[2])};
+    scalar_gather(cnt_addr, cnt);
+    const int F = min(max(cnt[0], 0), p.nS);
+    const int T = F + min(max(cnt[1], 0), p.nS - F);  // chunks = list entries
+    f32x16 acc[NDB], acc2[BOTH ? NDB : 1];  // acc2: dV beside dK
 #pragma unroll
     for (int db = 0; db < NDB; db++)
 #pragma unroll
-        for (int i = 0; i < 16; i++) acc[db][i] = 0.f;
+        for (int i = 0; i < 16; i++) {
+            acc[db][i] = 0.f;
+            if constexpr (BOTH) acc2[db][i] = 0.f;
+        }
 
     // LDS offsets inside a chunk buffer: row-wise operand reads (row 32kb + l32, piece 2c + hh) and transposing
     // reads (rows 16kc + 4hh + j and + 8 of a 32-row block, 32-wide d block db), both through bwd_swizzle
@@ -162,13 +185,13 @@ __global__ __launch_bounds__(256, 2) void sparse_bwd_kernel(const BwdParams p) {
     __syncthreads();
 
     // everything chunk t needs from memory, into stage st
-    auto issue = [&](int t, int st, uint32_t(&mk)[8]) {
+    auto issue = [&](int t, int st, uint32_t(&mk)[NMW]) {
         const int col = __builtin_amdgcn_readfirstlane(ent[t]);
 #pragma unroll
         for (int i = 0; i < NLD; i++) {
             const uint32_t dst = 1024 * (4 * i + wave_u);  // RPI rows per load
             dma16(ybase + (int64_t)col * p.ys[2], ld_yoff[i], lds0 + st * CBUF + dst);
-            dma16(zbase + (int64_t)col * p.zs[2], ld_zoff[i], lds0 + (2 + st) * CBUF + dst);
+            dma16(zbase + (int64_t)col * p.zs[2], ld_zoff[i], lds0 + Z0 + st * CBUF + dst);
         }
         if constexpr (!LANE_STATS) {
             if (wave_u == 0 && lane < 32) {  // 64 L values, then 64 Delta values, 16 bytes per lane (row stride 1)
@@ -176,34 +199,32 @@ __global__ __launch_bounds__(256, 2) void sparse_bwd_kernel(const BwdParams p) {
                 dma16(statL + col, off, lds0 + STAT0 + st * 512);
             }
         }
-        if (t >= F && p.packed != nullptr) {  // the row's 64 bits of the tile in slot t - F
-            const u32x2 w = *(const u32x2 *)(prow + (int64_t)(t - F) * 1024);
-            mk[0] = w.x;
-            mk[1] = w.y;
+        if (t >= F) {
+            if constexpr (PK) {  // the rows' bits of the tile in slot t - F, every wave those of its own rows
+                dma4_lane(prow + (int64_t)(t - F) * 1024, lds0 + MASK0 + st * 1024 + wave_u * 256);
+            } else {
 #pragma unroll
-            for (int i = 2; i < 8; i++) mk[i] = 0u;
-        } else if (t >= F) {
+                for (int kb = 0; kb < 2; kb++)
 #pragma unroll
-            for (int kb = 0; kb < 2; kb++)
-#pragma unroll
-                for (int g = 0; g < 4; g++) {
-                    const int64_t cc = col + 32 * kb + 8 * g + 4 * hh;
-                    if (p.mask_vec4) {
-                        mk[4 * kb + g] = *(const uint32_t *)(mrow + cc);
-                    } else {
-                        const uint8_t *m0 = mrow + cc * p.mcs;
-                        mk[4 * kb + g] = (uint32_t)m0[0] | ((uint32_t)m0[p.mcs] << 8) | ((uint32_t)m0[2 * p.mcs] << 16) |
-                                         ((uint32_t)m0[3 * p.mcs] << 24);
+                    for (int g = 0; g < 4; g++) {
+                        const int64_t cc = col + 32 * kb + 8 * g + 4 * hh;
+                        if (p.mask_vec4) {
+                            mk[4 * kb + g] = *(const uint32_t *)(mrow + cc);
+                        } else {
+                            const uint8_t *m0 = mrow + cc * p.mcs;
+                            mk[4 * kb + g] = (uint32_t)m0[0] | ((uint32_t)m0[p.mcs] << 8) | ((uint32_t)m0[2 * p.mcs] << 16) |
+                                             ((uint32_t)m0[3 * p.mcs] << 24);
+                        }
                     }
-                }
+            }
         }
     };
 
-    auto compute = [&](int t, int st, const uint32_t(&mk)[8]) {
-        const uint8_t *yb = smem + st * CBUF, *zb = smem + (2 + st) * CBUF;
+    auto compute = [&](int t, int st, const uint32_t(&mk)[NMW]) {
+        const uint8_t *yb = smem + st * CBUF, *zb = smem + Z0 + st * CBUF;
         const float *sl = reinterpret_cast<const float *>(smem + STAT0 + st * 512);
-#pragma unroll
-        for (int kb = 0; kb < 2; kb++) {
+        static_for<2>([&](auto kb_c) {
+            constexpr int kb = decltype(kb_c)::value;
             f32x16 s, dp;
 #pragma unroll
             for (int i = 0; i < 16; i++) s[i] = 0.f;
@@ -218,8 +239,8 @@ __global__ __launch_bounds__(256, 2) void sparse_bwd_kernel(const BwdParams p) {
             if (t >= F) {
                 // w: bit 8g + jj says whether this lane's entry (streamed row 32kb + 8g + 4hh + jj) attends
                 uint32_t w;
-                if (p.packed != nullptr) {  // bit k of the packed word: streamed row 32kb + k
-                    w = mk[kb] >> (4 * hh);
+                if constexpr (PK) {  // bit k of the packed word: streamed row 32kb + k
+                    w = *(const uint32_t *)(smem + MASK0 + st * 1024 + wave * 256 + 8 * l32 + 4 * kb) >> (4 * hh);
                 } else {  // one byte per entry: the non-zero bytes of each dword become four bits
                     w = 0u;
 #pragma unroll
@@ -236,7 +257,7 @@ __global__ __launch_bounds__(256, 2) void sparse_bwd_kernel(const BwdParams p) {
                         if (((w >> (8 * g + jj)) & 1u) == 0u) s[4 * g + jj] = kNegInf;
             }
             // P^T = exp2(S^T - L) and, unless OUT_P, dS^T = P^T o (dP^T - Delta); rounded to the input type
-            uint32_t pw[8];
+            uint32_t pw[8], pp[BOTH ? 8 : 1];
 #pragma unroll
             for (int g = 0; g < 4; g++) {
                 f32x4 L4, D4;
@@ -247,18 +268,23 @@ __global__ __launch_bounds__(256, 2) void sparse_bwd_kernel(const BwdParams p) {
                     L4 = *(const f32x4 *)(sl + 32 * kb + 8 * g + 4 * hh);
                     D4 = *(const f32x4 *)(sl + 64 + 32 * kb + 8 * g + 4 * hh);
                 }
-                float w[4];
+                float w[4], pv[4];
 #pragma unroll
                 for (int jj = 0; jj < 4; jj++) {
                     const float pr = __builtin_amdgcn_exp2f(s[4 * g + jj] - L4[jj]);
+                    pv[jj] = pr;
                     w[jj] = OUT_P ? pr : pr * (dp[4 * g + jj] - D4[jj]);
                 }
                 pw[2 * g] = E::pack2(w[0], w[1]);
                 pw[2 * g + 1] = E::pack2(w[2], w[3]);
+                if constexpr (BOTH) {
+                    pp[2 * g] = E::pack2(pv[0], pv[1]);
+                    pp[2 * g + 1] = E::pack2(pv[2], pv[3]);
+                }
             }
             const uint8_t *tb = (OUT_P ? zb : yb) + 32 * kb * ROWB;
-#pragma unroll
-            for (int kc = 0; kc < 2; kc++) {
+            static_for<2>([&](auto kc_c) {
+                constexpr int kc = decltype(kc_c)::value;
                 const u32x4 pk4 = u32x4{pw[4 * kc], pw[4 * kc + 1], pw[4 * kc + 2], pw[4 * kc + 3]};
 #pragma unroll
                 for (int db = 0; db < NDB; db++) {
@@ -266,27 +292,49 @@ __global__ __launch_bounds__(256, 2) void sparse_bwd_kernel(const BwdParams p) {
                     const u32x2 hi = E::tr_read(tb + 16 * kc * ROWB + toff[1][db]);
                     acc[db] = E::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, pk4, acc[db]);
                 }
-            }
-        }
+                if constexpr (BOTH) {
+                    const uint8_t *vb = zb + 32 * kb * ROWB;
+                    const u32x4 pp4 = u32x4{pp[4 * kc], pp[4 * kc + 1], pp[4 * kc + 2], pp[4 * kc + 3]};
+#pragma unroll
+                    for (int db = 0; db < NDB; db++) {
+                        const u32x2 lo = E::tr_read(vb + 16 * kc * ROWB + toff[0][db]);
+                        const u32x2 hi = E::tr_read(vb + 16 * kc * ROWB + toff[1][db]);
+                        acc2[db] = E::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, pp4, acc2[db]);
+                    }
+                }
+            });
+        });
     };
 
     {
-        uint32_t mk[2][8];
+        uint32_t mk[NS][NMW];
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int j = 0; j < NS; j++)
 #pragma unroll
-            for (int i = 0; i < 8; i++) mk[j][i] = 0u;
+            for (int i = 0; i < NMW; i++) mk[j][i] = 0u;
+        // The resident operands were requested before the list and have landed with it.  "Used" here, they are no loads any
+        // more to the compiler, whose wait in front of their first use in the loop would take the direct loads of the
+        // chunks behind along, in every trip.
+#pragma unroll
+        for (int c = 0; c < NC; c++) asm volatile("" : "+v"(xf[c]));
+        if constexpr (!OUT_P) {
+#pragma unroll
+            for (int c = 0; c < NC; c++) asm volatile("" : "+v"(gf[c]));
+        }
+        if constexpr (LANE_STATS) asm volatile("" : "+v"(laneL), "+v"(laneD));
         if (T > 0) issue(0, 0, mk[0]);
-        for (int t0 = 0; t0 < T; t0 += 2) {
-            static_for<2>([&](auto jc) {
-                constexpr int j = decltype(jc)::value;
+        for (int t0 = 0; t0 < T; t0 += NS) {
+            static_for<NS>([&](auto jc) {
+                constexpr int j = decltype(jc)::value, jn = j ^ 1;
                 const int t = t0 + j;
                 if (t >= T) return;
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // own pieces of chunk t and its mask words
+                if constexpr (!PK) {
 #pragma unroll
-                for (int i = 0; i < 8; i++) asm volatile("" ::"v"(mk[j][i]));
+                    for (int i = 0; i < NMW; i++) asm volatile("" ::"v"(mk[j][i]));
+                }
                 __syncthreads();  // everyone's pieces; and everyone is done with the other stage
-                if (t + 1 < T) issue(t + 1, j ^ 1, mk[j ^ 1]);
+                if (t + 1 < T) issue(t + 1, jn, mk[jn]);
                 compute(t, j, mk[j]);
             });
         }
@@ -298,24 +346,62 @@ __global__ __launch_bounds__(256, 2) void sparse_bwd_kernel(const BwdParams p) {
     // period, and leave as whole rows, 16 bytes per lane.
     __syncthreads();  // every wave is done with the chunk buffers
     constexpr int OROW = ROWB + 16;
-    static_assert(4 * 32 * OROW <= 4 * CBUF, "the rows of the four waves fit the chunk buffers");
+    static_assert(4 * 32 * OROW <= 2 * NS * CBUF, "the rows of the four waves fit the chunk buffers");
     uint8_t *const ob = smem + wave * 32 * OROW;
-#pragma unroll
-    for (int db = 0; db < NDB; db++)
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-            const u32x2 w = {E::pack2(acc[db][4 * g] * p.out_scale, acc[db][4 * g + 1] * p.out_scale),
-                             E::pack2(acc[db][4 * g + 2] * p.out_scale, acc[db][4 * g + 3] * p.out_scale)};
-            *(u32x2 *)(ob + l32 * OROW + 2 * (32 * db + 8 * g + 4 * hh)) = w;
-        }
     constexpr int PPR_O = ROWB / 16;  // 16-byte pieces per row
-    uint16_t *const o0 = p.out + b * p.outs[0] + h * p.outs[1] + (int64_t)(rt * 128 + wave * 32) * p.outs[2];
+    // Where the rows go is read from the argument block only now (the pointer passes through an asm statement): held in
+    // scalar registers through the loop these strides had others spilled.
+    typedef const __attribute__((address_space(4))) BwdLaunch *ArgPtr;
+    ArgPtr args = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    auto store = [&](const f32x16(&a)[NDB], float scale, uint16_t *out, int64_t os0, int64_t os1, int64_t os2) {
 #pragma unroll
-    for (int i = 0; i < 32 * PPR_O / 64; i++) {
-        const int idx = 64 * i + lane, r = idx / PPR_O, pc = idx % PPR_O;
-        const u32x4 x = *(const u32x4 *)(ob + r * OROW + 16 * pc);
-        // (written once, whole rows: a streaming store leaves the streamed operands' lines in L2 alone)
-        __builtin_nontemporal_store(x, (u32x4 *)(o0 + (int64_t)r * p.outs[2] + 8 * pc));
+        for (int db = 0; db < NDB; db++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const u32x2 w = {E::pack2(a[db][4 * g] * scale, a[db][4 * g + 1] * scale),
+                                 E::pack2(a[db][4 * g + 2] * scale, a[db][4 * g + 3] * scale)};
+                *(u32x2 *)(ob + l32 * OROW + 2 * (32 * db + 8 * g + 4 * hh)) = w;
+            }
+        uint16_t *const o0 = out + b * os0 + h * os1 + (int64_t)(rt * 128 + wave * 32) * os2;
+#pragma unroll
+        for (int i = 0; i < 32 * PPR_O / 64; i++) {
+            const int idx = 64 * i + lane, r = idx / PPR_O, pc = idx % PPR_O;
+            const u32x4 x = *(const u32x4 *)(ob + r * OROW + 16 * pc);
+            // (written once, whole rows: a streaming store leaves the streamed operands' lines in L2 alone)
+            __builtin_nontemporal_store(x, (u32x4 *)(o0 + (int64_t)r * os2 + 8 * pc));
+        }
+    };
+    store(acc, args->pass[PASS].out_scale, args->pass[PASS].out, args->pass[PASS].outs[0], args->pass[PASS].outs[1], args->pass[PASS].outs[2]);
+    if constexpr (BOTH)  // (a wave's slice is its own: its reads above come first)
+        store(acc2, 1.f, args->pass[PASS].out2, args->pass[PASS].outs2[0], args->pass[PASS].outs2[1], args->pass[PASS].outs2[2]);
+}
+
+// D = 64 with packed tiles: three workgroups per compute unit (168 registers, 43 KB of LDS; a third stage of the chunks
+// beside two of them instead: 2 ... 14 % slower).  Both passes of B4 H12 S2048 documents: 125 us as three launches with dK
+// and dV apart, 80 us now; causal B8 H12 S4096 910 -> 753 us; D = 128 causal B4 H16 S2048 358 -> 315, B2 H8 S1024 97 -> 41 us.
+// All passes in one launch: a launch each would leave the device to the last tiles of every pass, and passes of fewer tiles
+// than workgroup slots would run one after the other (B2 H8 S1024: 128 tiles a pass on 512 slots).  The passes whose
+// tiles take longest come first; every pass starts at a multiple of eight workgroups, so that the plane-to-XCD mapping of
+// bwd_tile holds for each.
+template <int DT, int D, bool PK>
+__global__ __launch_bounds__(256, D == 64 && PK ? 3 : 2) void sparse_bwd_kernel(const BwdLaunch l) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    const int id = blockIdx.x;
+    if constexpr (D == 64) {
+        if (id < l.first[1]) {
+            if (id < l.tiles[0]) bwd_tile<DT, D, kDKV, PK, 0>(l.pass[0], id, l.tiles[0], smem);
+        } else {
+            bwd_tile<DT, D, kDQ, PK, 1>(l.pass[1], id - l.first[1], l.tiles[1], smem);
+        }
+    } else {
+        if (id < l.first[1]) {
+            if (id < l.tiles[0]) bwd_tile<DT, D, kDK, PK, 0>(l.pass[0], id, l.tiles[0], smem);
+        } else if (id < l.first[2]) {
+            if (id - l.first[1] < l.tiles[1]) bwd_tile<DT, D, kDQ, PK, 1>(l.pass[1], id - l.first[1], l.tiles[1], smem);
+        } else {
+            bwd_tile<DT, D, kDV, PK, 2>(l.pass[2], id - l.first[2], l.tiles[2], smem);
+        }
     }
 }
 
@@ -354,20 +440,28 @@ __global__ __launch_bounds__(256) void bwd_prepare_kernel(const BwdPrepParams p)
     }
 }
 
-template <int DT, int D, bool LANE_STATS, bool OUT_P>
-hipError_t launch_bwd_one(const BwdParams &p, hipStream_t stream) {
-    constexpr int smem = 4 * 64 * D * 2 + 2 * 512 + kBwdListCap * 4;
-    auto kern = sparse_bwd_kernel<DT, D, LANE_STATS, OUT_P>;
+template <int DT, int D, bool PK>
+hipError_t launch_bwd_one(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, hipStream_t stream) {
+    constexpr int smem = BwdLds<D, PK>::bytes;
+    auto kern = sparse_bwd_kernel<DT, D, PK>;
     static unsigned long long attr_done = 0;
     if (const hipError_t e0 = allow_dynamic_smem(kern, smem, attr_done); e0 != hipSuccess) return e0;
-    hipLaunchKernelGGL(kern, dim3((unsigned)p.nR * (unsigned)p.B * (unsigned)p.H), dim3(256), smem, stream, p);
+    BwdLaunch l{};
+    const BwdParams *order[3] = {&dk, &dq, &dv};
+    constexpr int n = D == 64 ? 2 : 3;
+    int next = 0;
+    for (int i = 0; i < n; i++) {
+        l.pass[i] = *order[i];
+        l.tiles[i] = order[i]->nR * order[i]->B * order[i]->H;
+        l.first[i] = next;
+        next += (l.tiles[i] + 7) & ~7;
+    }
+    if (D == 64) {
+        l.pass[0].out2 = dv.out;
+        for (int i = 0; i < 3; i++) l.pass[0].outs2[i] = dv.outs[i];
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)(l.first[n - 1] + l.tiles[n - 1])), dim3(256), smem, stream, l);
     return hipGetLastError();
-}
-
-template <int DT, int D>
-hipError_t launch_bwd_pass(const BwdParams &p, bool lane_stats, bool out_p, hipStream_t stream) {
-    if (lane_stats) return launch_bwd_one<DT, D, true, false>(p, stream);
-    return out_p ? launch_bwd_one<DT, D, false, true>(p, stream) : launch_bwd_one<DT, D, false, false>(p, stream);
 }
 
 template <int DT, int D>
@@ -380,11 +474,16 @@ hipError_t launch_prepare_one(const BwdPrepParams &p, hipStream_t stream) {
 
 }  // namespace
 
-hipError_t launch_bwd(const BwdParams &p, int dtype, int D, bool lane_stats, bool out_p, hipStream_t stream) {
-    if (dtype == 0 && D == 128) return launch_bwd_pass<0, 128>(p, lane_stats, out_p, stream);
-    if (dtype == 0 && D == 64) return launch_bwd_pass<0, 64>(p, lane_stats, out_p, stream);
-    if (dtype == 1 && D == 128) return launch_bwd_pass<1, 128>(p, lane_stats, out_p, stream);
-    if (dtype == 1 && D == 64) return launch_bwd_pass<1, 64>(p, lane_stats, out_p, stream);
+hipError_t launch_bwd(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, int dtype, int D, hipStream_t stream) {
+    const bool pk = dq.packed != nullptr && dk.packed != nullptr;  // (with only one of them the mask is there too)
+#define SA_BWD(DT, DD) \
+    if (dtype == DT && D == DD) \
+        return pk ? launch_bwd_one<DT, DD, true>(dq, dk, dv, stream) : launch_bwd_one<DT, DD, false>(dq, dk, dv, stream)
+    SA_BWD(0, 128);
+    SA_BWD(0, 64);
+    SA_BWD(1, 128);
+    SA_BWD(1, 64);
+#undef SA_BWD
     return hipErrorInvalidValue;
 }
 

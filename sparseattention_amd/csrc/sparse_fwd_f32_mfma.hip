@@ -31,16 +31,6 @@ namespace {
 
 constexpr int kF32ListCap = 1024;  // list entries kept in LDS (the launcher refuses longer rows of tiles)
 
-__device__ __forceinline__ void f32_dma4(const void *lane_addr, uint32_t lds_addr) {
-    lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
-    asm volatile(
-        "s_mov_b32 m0, %1\n\t"
-        "s_nop 0\n\t"
-        "global_load_lds_dword %0, off"
-        :
-        : "v"(lane_addr), "s"(lds_addr)
-        : "memory");
-}
 // MODE 0: BK = 16 (two list entries per chunk), MODE 1: BK = 32, MODE 2: BK >= 64 (BK/32 chunks per entry).
 // PK: mask entries of PARTIAL tiles from the bit-packed tiles; else from the bool mask (key stride 1, rows and base
 // 16-byte aligned: checked by the launcher).
@@ -182,7 +172,7 @@ __global__ __launch_bounds__(NW * 64, NW >= 4 ? 2 : 1) void sparse_fwd_f32_mfma_
             if constexpr (MODE == 0) src = pbase + (int64_t)(hh ? pl.slot[EPC - 1] : pl.slot[0]) * tile_bytes + (r & ~1) * 2;
             else if constexpr (MODE == 1) src = pbase + (int64_t)pl.slot[0] * tile_bytes + r * 4;
             else src = pbase + (int64_t)pl.slot[0] * tile_bytes + (int64_t)r * (p.BK >> 3) + 4 * (t & ((1 << (p.lbk - 5)) - 1));
-            f32_dma4(src, mdst);
+            dma4_lane(src, mdst);
         } else {
             // 16 mask bytes per lane: keys 16 hh .. 16 hh + 15 of the chunk (BK = 16: entry hh)
             const int col = MODE == 0 ? (hh ? pl.col[EPC - 1] : pl.col[0]) : pl.col[0] + 16 * hh;
@@ -203,7 +193,7 @@ __global__ __launch_bounds__(NW * 64, NW >= 4 ? 2 : 1) void sparse_fwd_f32_mfma_
         for (int base = 64 * wave_u; base < NE; base += 64 * NW) {
             const int e = min(base + lane, NE - 1);
             const int32_t *src = e < F ? fid + (int64_t)e * p.fis[3] : pid + (int64_t)(e - F) * p.pis[3];
-            f32_dma4(src, lds0 + OFF_L + 4 * base);
+            dma4_lane(src, lds0 + OFF_L + 4 * base);
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();

@@ -1022,8 +1022,8 @@ int sa_sparse_attention_bwd(const void *q, const int64_t q_strides[4], const voi
         return fail(SA_ERR_INVALID_ARGUMENT, "sa_sparse_attention_bwd: sm_scale_log2 must be positive and finite");
     if (Sq / 64 > 2048 || Sk / 64 > 2048)
         return fail(SA_ERR_UNSUPPORTED, "sa_sparse_attention_bwd: more than 2048 tiles of 64 rows along Sq or Sk");
-    if ((int64_t)B * H * ((Sq > Sk ? Sq : Sk) / 128) > 0x7fffffffLL)
-        return fail(SA_ERR_UNSUPPORTED, "sa_sparse_attention_bwd: more than 2^31-1 workgroups");
+    if ((int64_t)B * H * ((Sq > Sk ? Sq : Sk) / 128) > 0x7fffffffLL / 4)
+        return fail(SA_ERR_UNSUPPORTED, "sa_sparse_attention_bwd: more than 2^29 tiles of 128 rows");
     const int64_t *st[9] = {q_strides, k_strides, v_strides, o_strides, do_strides, dq_strides, dk_strides, dv_strides};
     const void *tp[8] = {q, k, v, o, d_o, dq, dk, dv};
     const char *name[8] = {"q", "k", "v", "o", "do", "dq", "dk", "dv"};
@@ -1120,8 +1120,7 @@ int sa_sparse_attention_bwd(const void *q, const int64_t q_strides[4], const voi
     bp.nR = Sq / 128;
     bp.first_tile_first = 0;
     bp.out_scale = sm_scale;
-    e = sa::launch_bwd(bp, dtype, D, true, false, hs);
-    if (e != hipSuccess) return fail(SA_ERR_HIP, "sa_sparse_attention_bwd: launch failed: %s", hipGetErrorString(e));
+    const sa::BwdParams dq_pass = bp;
 
     // dK and dV: keys resident, queries streamed; the mask is walked transposed, or read from the caller's
     // transposed copy [B,H,Sk,Sq], whose rows are contiguous in the streamed direction
@@ -1168,12 +1167,11 @@ int sa_sparse_attention_bwd(const void *q, const int64_t q_strides[4], const voi
     bp.out = static_cast<uint16_t *>(dk);
     set3(bp.outs, dk_strides);
     bp.out_scale = sm_scale;
-    e = sa::launch_bwd(bp, dtype, D, false, false, hs);
-    if (e != hipSuccess) return fail(SA_ERR_HIP, "sa_sparse_attention_bwd: launch failed: %s", hipGetErrorString(e));
+    const sa::BwdParams dk_pass = bp;
     bp.out = static_cast<uint16_t *>(dv);
     set3(bp.outs, dv_strides);
     bp.out_scale = 1.f;
-    e = sa::launch_bwd(bp, dtype, D, false, true, hs);
+    e = sa::launch_bwd(dq_pass, dk_pass, bp, dtype, D, hs);
     if (e != hipSuccess) return fail(SA_ERR_HIP, "sa_sparse_attention_bwd: launch failed: %s", hipGetErrorString(e));
     return SA_OK;
 }
