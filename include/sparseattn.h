@@ -457,11 +457,15 @@ int sa_merge_attention_parts(const void *o_parts, const int64_t o_parts_strides[
  *                   BK = 64 and the q_* lists; the transposed mask with BQ = 128, BK = 64 and the k_* lists), or
  *                   NULL.  A pass that has its packed buffer reads no mask; with both, `mask` and `mask_t` may be
  *                   NULL, so the bool tensors can be released after preprocessing.
- *   workspace       sa_bwd_workspace_bytes(B, H, Sq) bytes of device memory, 16-byte aligned
+ *   workspace       sa_bwd_workspace_bytes(B, H, Sq) bytes of device memory, 16-byte aligned.  With
+ *                   sa_bwd_workspace_bytes_ex(B, H, Sq, Sk, D) bytes (never less; at most 4 GiB more) and both packed
+ *                   buffers, dS is kept between the passes where that is faster: dQ is then made from it by one
+ *                   product instead of three.  Memory only: the sums are the same, of the same rounded dS.
  * D = 64 or 128, bf16 or fp16, Sq and Sk multiples of 128; tensors as for the forward (last dimension contiguous).
  * The tile sizes of the backward are its own: they need not be those the forward ran with.
  */
 size_t sa_bwd_workspace_bytes(int B, int H, int Sq);
+size_t sa_bwd_workspace_bytes_ex(int B, int H, int Sq, int Sk, int D);
 int sa_sparse_attention_bwd(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
                             const void *v, const int64_t v_strides[4], const void *o, const int64_t o_strides[4],
                             const void *d_o, const int64_t do_strides[4], const float *lse,

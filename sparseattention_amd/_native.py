@@ -53,6 +53,7 @@ EXPORTS = (
     "sa_sparse_attention_decode_ex",
     "sa_merge_attention_parts",
     "sa_bwd_workspace_bytes",
+    "sa_bwd_workspace_bytes_ex",
     "sa_sparse_attention_bwd",
     "sa_mask_terms_workspace_bytes",
     "sa_mask_classify_terms",
@@ -154,6 +155,8 @@ def load() -> ctypes.CDLL:
     lib.sa_merge_attention_parts.argtypes = [_vp, _i64p] * 4 + [ctypes.c_int] * 6 + [_vp]
     lib.sa_bwd_workspace_bytes.restype = ctypes.c_size_t
     lib.sa_bwd_workspace_bytes.argtypes = [ctypes.c_int] * 3
+    lib.sa_bwd_workspace_bytes_ex.restype = ctypes.c_size_t
+    lib.sa_bwd_workspace_bytes_ex.argtypes = [ctypes.c_int] * 5
     lib.sa_sparse_attention_bwd.restype = ctypes.c_int
     lib.sa_sparse_attention_bwd.argtypes = (
         [_vp, _i64p] * 13 + [_vp, _i64p] * 8 + [_vp, ctypes.c_size_t] + [ctypes.c_int] * 6 + [ctypes.c_float, _vp]

@@ -46,7 +46,8 @@ struct Elem<0> {  // bf16
     static __device__ __forceinline__ uint32_t scale2(uint32_t w, float s) {  // both halves times s, rounded again
         return pack2(__uint_as_float(w << 16) * s, __uint_as_float(w & 0xffff0000u) * s);
     }
-    static __device__ __forceinline__ u32x2 tr_read(const uint8_t *lds_ptr) {
+    template <class P>
+    static __device__ __forceinline__ u32x2 tr_read(P lds_ptr) {
         return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((SA_LDS bf16x4 *)lds_ptr));
     }
     static __device__ __forceinline__ u32x4 ones4() {  // eight 1.0 values, an all-ones MFMA operand
@@ -72,7 +73,8 @@ struct Elem<1> {  // fp16
         const f16x2 h = __builtin_bit_cast(f16x2, w);
         return pack2((float)h.x * s, (float)h.y * s);
     }
-    static __device__ __forceinline__ u32x2 tr_read(const uint8_t *lds_ptr) {
+    template <class P>
+    static __device__ __forceinline__ u32x2 tr_read(P lds_ptr) {
         // the transposing read only moves 16-bit lanes around, so the bf16 flavour serves fp16 too
         return __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4bf16((SA_LDS bf16x4 *)lds_ptr));
     }
@@ -141,6 +143,19 @@ __device__ __forceinline__ void dma16_lane(const void *lane_addr, uint32_t lds_a
 }
 
 // 4 bytes per lane: lane i of the wave writes LDS address lds_addr + 4*i.
+__device__ __forceinline__ void dma4(const void *base, uint32_t lane_offset, uint32_t lds_addr) {
+    const uint64_t b = (uint64_t)(uintptr_t)base;
+    const uint64_t ub = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b) |
+                        ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) << 32);
+    lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
+    asm volatile(
+        "s_mov_b32 m0, %2\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dword %0, %1"
+        :
+        : "v"(lane_offset), "s"(ub), "s"(lds_addr)
+        : "memory");
+}
 __device__ __forceinline__ void dma4_lane(const void *lane_addr, uint32_t lds_addr) {
     lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
     asm volatile(

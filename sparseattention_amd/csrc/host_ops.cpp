@@ -498,9 +498,16 @@ std::tuple<Tensor, Tensor, Tensor> backward_impl(const Tensor &do_, const Tensor
     const Tensor qc = kernel_ready(pad_head_dim(q, Dk)), kc = kernel_ready(pad_head_dim(k, Dk)), vc = kernel_ready(pad_head_dim(v, Dk));
     const Tensor oc = kernel_ready(pad_head_dim(o, Dk)), doc = kernel_ready(pad_head_dim(do_, Dk));
     const Tensor dq = at::empty_like(qc), dk = at::empty_like(kc), dv = at::empty_like(vc);
-    const size_t ws_bytes = sa_bwd_workspace_bytes(B, H, Sq);
-    const Tensor ws = at::empty({(int64_t)(ws_bytes / 4)}, at::TensorOptions().dtype(at::kFloat).device(q.device()));
     const Lists &a = l.by_query, &b = l.by_key;
+    const auto workspace = [&](size_t bytes) { return at::empty({(int64_t)bytes}, at::TensorOptions().dtype(at::kByte).device(q.device())); };
+    size_t ws_bytes = a.packed && b.packed ? sa_bwd_workspace_bytes_ex(B, H, Sq, Sk, Dk) : sa_bwd_workspace_bytes(B, H, Sq);
+    Tensor ws;
+    try {
+        ws = workspace(ws_bytes);
+    } catch (const c10::OutOfMemoryError &) {  // dS finds no place: the passes that make it anew
+        ws_bytes = sa_bwd_workspace_bytes(B, H, Sq);
+        ws = workspace(ws_bytes);
+    }
     check_rc(sa_sparse_attention_bwd(qc.data_ptr(), st(qc), kc.data_ptr(), st(kc), vc.data_ptr(), st(vc), oc.data_ptr(), st(oc), doc.data_ptr(), st(doc),
                                      ptr<float>(lse), st(lse), dq.data_ptr(), st(dq), dk.data_ptr(), st(dk), dv.data_ptr(), st(dv), ptr<uint8_t>(mask),
                                      st(mask), ptr<uint8_t>(l.transposed_mask), st(l.transposed_mask), ptr<uint8_t>(a.packed), st(a.packed),

@@ -228,7 +228,7 @@ struct BwdParams {
     int nS;            // streamed tiles per resident tile (slots in `packed`)
     const int32_t *full_ids, *full_lens, *part_ids, *part_lens;  // per resident tile, streamed tiles of 64
     int64_t fis[4], fls[3], pis[4], pls[3];
-    const float *stat_l, *stat_d;  // per query: lse / ln 2 (+inf for dead rows) and rowsum(dO o O)
+    const float *stat_l, *stat_d;  // per query: -lse / ln 2 (-inf for dead rows) and -rowsum(dO o O)
     int64_t sts[3];                // their b, h, row strides in elements (row stride 1 when queries are streamed)
     int B, H, nR;                  // nR: resident tiles
     int first_tile_first;          // launch order of a plane's tiles: 0 last tile first (queries), 1 first tile first (keys)
@@ -236,19 +236,27 @@ struct BwdParams {
     float out_scale;               // softmax scale for dQ and dK, 1 for dV
     uint16_t *out2;                // dV, where one pass makes both
     int64_t outs2[3];
+    int plane0, planes;            // the pass covers planes plane0 .. plane0 + planes - 1 of the B * H
+    uint8_t *ds;                   // workspace of dS of these planes (bwd_dq_tile), Sq * Sk elements each
 };
 // The passes of one launch: workgroup first[i] + t has tile t of pass i.
 struct BwdLaunch {
     BwdParams pass[3];
     int first[3], tiles[3];
 };
-hipError_t launch_bwd(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, int dtype, int D, hipStream_t stream);
+// group > 0 (D = 128 and both packed buffers): dS of that many planes at a time goes through `ds`, and dQ is made from it.
+hipError_t launch_bwd(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, int dtype, int D, uint8_t *ds, int group, hipStream_t stream);
+// The rule for group: sparse_bwd.hip.  bytes: what the workspace holds besides the statistics.
+int bwd_ds_group(int B, int H, int Sq, int Sk, int D, size_t bytes);
+// Bytes of dS that are worth their place, 0 where none are.
+size_t bwd_ds_bytes(int B, int H, int Sq, int Sk, int D);
 
 struct BwdPrepParams {
     const uint16_t *o, *d_o;
     const float *lse;
     int64_t os[3], dos[3], ls[3];
     float *stat_l, *stat_d;  // [B*H*Sq] each, contiguous
+    float l_mul;             // stat_l = lse * l_mul: -1 / ln 2, or -1 / (ln 2 scale) where the kernel scales S - L
     int B, H, Sq;
 };
 hipError_t launch_bwd_prepare(const BwdPrepParams &p, int dtype, int D, hipStream_t stream);

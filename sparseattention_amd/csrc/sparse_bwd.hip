@@ -16,7 +16,8 @@
 // are streamed.  Streamed chunks of 64 rows arrive by direct loads global -> LDS in two stages, one barrier per chunk.
 // A chunk buffer is read both ways - row-wise as MFMA A operand (ds_read_b128) and transposed (ds_read_b64_tr_b16) -
 // so the 16-byte pieces of a row are swizzled with a function of the row that keeps both patterns free of bank
-// conflicts (bwd_swizzle).
+// conflicts (bwd_swizzle).  Where there is enough work at D = 128 the pass over the keys makes dK, dV and dS at once and
+// dQ is made from the stored dS (bwd_ds_group, bwd_dq_tile).
 #include "fwd_common.h"
 
 namespace sa {
@@ -37,6 +38,17 @@ __device__ __forceinline__ int bwd_swizzle(int row) {
     else return (((row >> 1) & 1) << 2) | (((row >> 3) & 1) << 1) | ((row >> 2) & 1);
 }
 
+// LDS offset of a lane's transposing read of rows 4hh + j, j = 0..3, of d block 0; rows + 8 of them: ^ bwd_tr_rows8, d
+// block db: ^ 64 db, rows + 16: + 16 rows.
+template <int D>
+__device__ __forceinline__ int bwd_tr_base(int lane) {
+    const int hh = lane >> 5, j = (lane & 15) >> 2, x = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+    const int grp = D == 128 ? j : (j >> 1);  // the 64-byte-group part of bwd_swizzle(4hh + j); its piece part is hh
+    return (4 * hh + j) * D * 2 + 64 * grp + 16 * (x ^ hh) + 8 * (lane & 1);
+}
+template <int D>
+constexpr int bwd_tr_rows8 = 8 * D * 2 + 32;
+
 // What a workgroup makes of its resident tile.
 constexpr int kDQ = 0;   // queries resident
 constexpr int kDK = 1;   // keys resident, as for the following
@@ -53,8 +65,61 @@ struct BwdLds {
     static constexpr int bytes = LIST0 + kBwdListCap * 4;
 };
 
-// PK: the mask entries of PARTIAL tiles come bit-packed from p.packed, else from the bool mask.
-template <int DT, int D, int KIND, bool PK, int PASS>
+// Workgroup -> (plane of the pass, resident tile) as in sparse_fwd_kernel: consecutive workgroup ids go to the 8 XCDs in
+// turn, so each XCD gets a contiguous range of the plane-major order (the tiles that share K/V or Q/dO meet in one L2),
+// planes two at a time with their tiles interleaved, the tile that is heaviest under causal-like masks first
+// (the last queries, the first keys: p.first_tile_first).
+struct BwdPlace {
+    int plane, rt;
+};
+__device__ __forceinline__ BwdPlace bwd_place(const BwdParams &p, int lin, int total) {
+    const int per = total >> 3;
+    if (lin < (per << 3)) lin = (lin & 7) * per + (lin >> 3);
+    int pair = lin / (2 * p.nR);
+    const int pr = lin - pair * 2 * p.nR;
+    if ((p.planes & 15) == 0) {  // every eighth pair of planes to an XCD: masks that differ per batch element load them alike
+        const int ppx = p.planes >> 4;
+        const int x = pair / ppx;
+        pair = (pair - x * ppx) * 8 + x;
+    }
+    const bool paired = 2 * pair + 1 < p.planes;
+    const int order = paired ? (pr >> 1) : pr;
+    return {2 * pair + (paired ? (pr & 1) : 0), p.first_tile_first ? order : p.nR - 1 - order};
+}
+
+// out = acc * scale; acc holds the transposed tile: lane (row l32, hh), register 4g + jj of block db is
+// d = 32 db + 8g + 4hh + jj.  A lane's 8-byte pieces would make every store instruction touch 32 rows, so the wave's 32
+// rows go through a private slice `ob` of the (now idle) chunk buffers, rows 16 bytes apart from the banks' period, and
+// leave as whole rows, 16 bytes per lane.  o0: the wave's first row, rows os2 elements apart.
+template <int D>
+constexpr int bwd_out_row = D * 2 + 16;
+template <int DT, int D>
+__device__ __forceinline__ void bwd_store_rows(const f32x16 (&a)[D / 32], float scale, uint8_t *ob, uint16_t *o0, int64_t os2, int lane) {
+    using E = Elem<DT>;
+    constexpr int OROW = bwd_out_row<D>, PPR = D / 8;  // 16-byte pieces per row
+    const int l32 = lane & 31, hh = lane >> 5;
+#pragma unroll
+    for (int db = 0; db < D / 32; db++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const u32x2 w = {E::pack2(a[db][4 * g] * scale, a[db][4 * g + 1] * scale),
+                             E::pack2(a[db][4 * g + 2] * scale, a[db][4 * g + 3] * scale)};
+            *(u32x2 *)(ob + l32 * OROW + 2 * (32 * db + 8 * g + 4 * hh)) = w;
+        }
+#pragma unroll
+    for (int i = 0; i < 32 * PPR / 64; i++) {
+        const int idx = 64 * i + lane, r = idx / PPR, pc = idx % PPR;
+        const u32x4 x = *(const u32x4 *)(ob + r * OROW + 16 * pc);
+        // (written once, whole rows: a streaming store leaves the streamed operands' lines in L2 alone)
+        __builtin_nontemporal_store(x, (u32x4 *)(o0 + (int64_t)r * os2 + 8 * pc));
+    }
+}
+
+// PK: the mask entries of PARTIAL tiles come bit-packed from p.packed, else from the bool mask.  DS: dS, rounded as it
+// enters dK's product, is stored for bwd_dq_tile too (D = 128: both accumulators, K and V take 192 of 256 registers, so that
+// S, dP and the reads on their way share the rest: see `phase`).  K then stays unscaled and S - L is scaled in float32 (a rounded
+// scale K would give dQ another P than the rounded scale Q of the forward: 3 % more error, this is less than before).
+template <int DT, int D, int KIND, bool PK, int PASS, bool DS = false>
 __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, uint8_t *smem) {
     using E = Elem<DT>;
     static_assert(D == 128 || D == 64, "head dim");
@@ -73,23 +138,8 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l32 = lane & 31, hh = lane >> 5;
-    // Workgroup -> (plane, resident tile) as in sparse_fwd_kernel: consecutive workgroup ids go to the 8 XCDs in turn,
-    // so each XCD gets a contiguous range of the plane-major order (the tiles that share K/V or Q/dO meet in one L2),
-    // planes two at a time with their tiles interleaved, the tile that is heaviest under causal-like masks first
-    // (the last queries, the first keys: p.first_tile_first).
-    const int per = total >> 3;
-    if (lin < (per << 3)) lin = (lin & 7) * per + (lin >> 3);
-    int pair = lin / (2 * p.nR);
-    const int pr = lin - pair * 2 * p.nR;
-    if (((p.B * p.H) & 15) == 0) {  // every eighth pair of planes to an XCD: masks that differ per batch element load them alike
-        const int ppx = (p.B * p.H) >> 4;
-        const int x = pair / ppx;
-        pair = (pair - x * ppx) * 8 + x;
-    }
-    const bool paired = 2 * pair + 1 < p.B * p.H;
-    const int bh = 2 * pair + (paired ? (pr & 1) : 0);
-    const int order = paired ? (pr >> 1) : pr;
-    const int rt = p.first_tile_first ? order : p.nR - 1 - order;  // resident tile
+    const BwdPlace at = bwd_place(p, lin, total);
+    const int plane = at.plane, rt = at.rt, bh = p.plane0 + plane;
     const int b = bh / p.H, h = bh - b * p.H;
     const int rrow = rt * 128 + wave * 32 + l32;
 
@@ -99,7 +149,7 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
     const int32_t *pid = p.part_ids + b * p.pis[0] + h * p.pis[1] + rt * p.pis[2];
     const uint8_t *mrow = PK ? nullptr : p.mask + b * p.ms[0] + h * p.ms[1] + (int64_t)rrow * p.mrs;
     // packed tiles: 8 bytes per row, 1024 per tile, nS tiles per resident tile; a lane's four bytes of its wave's 32 rows
-    const uint8_t *prow = PK ? p.packed + b * p.pks[0] + h * p.pks[1] + (int64_t)rt * p.nS * 1024 + wave * 256 + 4 * lane : nullptr;
+    const uint8_t *prow = PK ? p.packed + b * p.pks[0] + h * p.pks[1] + (int64_t)rt * p.nS * 1024 : nullptr;
     const float *statL = p.stat_l + b * p.sts[0] + h * p.sts[1];
     const float *statD = p.stat_d + b * p.sts[0] + h * p.sts[1];
     // bytes from a query's L to its Delta (both live in one workspace, less than 4 GiB apart)
@@ -113,7 +163,8 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
         for (int c = 0; c < NC; c++) {
             xf[c] = *(const u32x4 *)(xp + 16 * c);
 #pragma unroll
-            for (int e = 0; e < 4; e++) xf[c][e] = E::scale2(xf[c][e], p.scale);
+            for (int e = 0; e < 4; e++)
+                if constexpr (!DS) xf[c][e] = E::scale2(xf[c][e], p.scale);
         }
         if constexpr (!OUT_P) {
             const uint16_t *gp = p.g + b * p.gs[0] + h * p.gs[1] + (int64_t)rrow * p.gs[2] + 8 * hh;
@@ -145,37 +196,18 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
         }
 
     // LDS offsets inside a chunk buffer: row-wise operand reads (row 32kb + l32, piece 2c + hh) and transposing
-    // reads (rows 16kc + 4hh + j and + 8 of a 32-row block, 32-wide d block db), both through bwd_swizzle
-    int noff[NC];
-#pragma unroll
-    for (int c = 0; c < NC; c++) noff[c] = l32 * ROWB + 16 * ((2 * c + hh) ^ bwd_swizzle<D>(l32));
-    int toff[2][NDB];
-    {
-        const int j = (lane & 15) >> 2;
-        const int x = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            const int row = 4 * hh + j + 8 * u;
-#pragma unroll
-            for (int db = 0; db < NDB; db++) {
-                // bwd_swizzle of row 16kc + 4hh + j + 8u, split into its 64-byte-group and its piece-in-group part
-                const int grp = D == 128 ? j : (j >> 1), pc = D == 128 ? ((hh + 2 * u) & 3) : ((u << 1) | hh);
-                toff[u][db] = row * ROWB + 64 * (db ^ grp) + 16 * (x ^ pc) + 8 * (lane & 1);
-            }
-        }
-    }
+    // reads (rows 16kc + 4hh + j and + 8 of a 32-row block, 32-wide d block db), both through bwd_swizzle.  The
+    // swizzle being an XOR, so are the steps from one piece, row group or d block to the next.
+    const int nbase = l32 * ROWB + 16 * (hh ^ bwd_swizzle<D>(l32));
+    const int tbase = bwd_tr_base<D>(lane);
     // direct loads: load i of this wave fills rows RPI (4i + wave) .. + RPI - 1 of the chunk; the lane writes LDS
     // piece lane % PPR of its row and therefore fetches the swizzled source piece
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const SA_LDS uint8_t *)smem);
-    uint32_t ld_yoff[NLD], ld_zoff[NLD];
-#pragma unroll
-    for (int i = 0; i < NLD; i++) {
-        const int r = RPI * (4 * i + wave_u) + lane / PPR;
-        const int piece = (lane % PPR) ^ bwd_swizzle<D>(r);
-        ld_yoff[i] = (uint32_t)((r * p.ys[2] + 8 * piece) * 2);
-        ld_zoff[i] = (uint32_t)((r * p.zs[2] + 8 * piece) * 2);
-    }
+    // (rows 4 RPI apart have the same swizzle, so the loads differ by a scalar)
+    const int ld_row = RPI * wave_u + lane / PPR, ld_piece = (lane % PPR) ^ bwd_swizzle<D>(ld_row);
+    const uint32_t ld_yoff = (uint32_t)((ld_row * p.ys[2] + 8 * ld_piece) * 2);
+    const uint32_t ld_zoff = (uint32_t)((ld_row * p.zs[2] + 8 * ld_piece) * 2);
 
     // the tile's list (FULL entries, then PARTIAL ones) as first streamed rows
     for (int e = tid; e < T; e += 256) {
@@ -184,24 +216,34 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
     }
     __syncthreads();
 
+    // where this wave's keys' dS of the 64 queries from ent[t] goes: two pieces of 2 KiB, 4 KiB apart
+    const int64_t ds_row = (int64_t)p.nR * 2 * 16384;  // all keys of 128 queries
+    uint8_t *const ds0 = DS ? p.ds + (int64_t)plane * (p.nS >> 1) * ds_row + (2 * rt + (wave_u >> 1)) * 16384 + (wave_u & 1) * 2048 : nullptr;
+    auto ds_out = [&](int t) {
+        const int row = __builtin_amdgcn_readfirstlane(ent[t]);
+        return ds0 + (row >> 7) * ds_row + ((row & 64) << 7);
+    };
+
     // everything chunk t needs from memory, into stage st
     auto issue = [&](int t, int st, uint32_t(&mk)[NMW]) {
+        int ln = lane;
+        if constexpr (DS) asm volatile("" : "+v"(ln));
         const int col = __builtin_amdgcn_readfirstlane(ent[t]);
 #pragma unroll
         for (int i = 0; i < NLD; i++) {
             const uint32_t dst = 1024 * (4 * i + wave_u);  // RPI rows per load
-            dma16(ybase + (int64_t)col * p.ys[2], ld_yoff[i], lds0 + st * CBUF + dst);
-            dma16(zbase + (int64_t)col * p.zs[2], ld_zoff[i], lds0 + Z0 + st * CBUF + dst);
+            dma16(ybase + (int64_t)(col + 4 * RPI * i) * p.ys[2], ld_yoff, lds0 + st * CBUF + dst);
+            dma16(zbase + (int64_t)(col + 4 * RPI * i) * p.zs[2], ld_zoff, lds0 + Z0 + st * CBUF + dst);
         }
         if constexpr (!LANE_STATS) {
-            if (wave_u == 0 && lane < 32) {  // 64 L values, then 64 Delta values, 16 bytes per lane (row stride 1)
-                const uint32_t off = (lane < 16 ? 0u : stat_gap) + 16u * (lane & 15);
+            if (wave_u == 0 && ln < 32) {  // 64 L values, then 64 Delta values, 16 bytes per lane (row stride 1)
+                const uint32_t off = (ln < 16 ? 0u : stat_gap) + 16u * (ln & 15);
                 dma16(statL + col, off, lds0 + STAT0 + st * 512);
             }
         }
         if (t >= F) {
             if constexpr (PK) {  // the rows' bits of the tile in slot t - F, every wave those of its own rows
-                dma4_lane(prow + (int64_t)(t - F) * 1024, lds0 + MASK0 + st * 1024 + wave_u * 256);
+                dma4(prow + (int64_t)(t - F) * 1024 + wave_u * 256, 4 * ln, lds0 + MASK0 + st * 1024 + wave_u * 256);
             } else {
 #pragma unroll
                 for (int kb = 0; kb < 2; kb++)
@@ -221,26 +263,63 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
     };
 
     auto compute = [&](int t, int st, const uint32_t(&mk)[NMW]) {
-        const uint8_t *yb = smem + st * CBUF, *zb = smem + Z0 + st * CBUF;
-        const float *sl = reinterpret_cast<const float *>(smem + STAT0 + st * 512);
+        // Two accumulators of D = 128 leave no register over: the offsets are made anew from their bases per phase (kept,
+        // they spill), and no phase's reads move into another.
+        uint32_t nb = lds0 + nbase, tb0 = lds0 + tbase, sb = lds0 + STAT0 + 16 * hh;
+        int ln = lane;
+        auto phase = [&] {
+            if constexpr (DS) {
+                __builtin_amdgcn_sched_barrier(0);
+                asm volatile("" : "+v"(nb), "+v"(tb0), "+v"(ln));
+                sb = lds0 + STAT0 + 16 * (ln >> 5);
+            }
+        };
+        constexpr int kAhead = 4;
+        auto paced = [] {  // operand reads this far ahead of the products
+            if constexpr (DS) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 4 + kAhead, 0);
+                static_for<NC - kAhead>([](auto) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                });
+                __builtin_amdgcn_sched_group_barrier(0x008, kAhead, 0);
+            }
+        };
+        phase();
+        constexpr auto lds = [](uint32_t a) { return (const SA_LDS uint8_t *)(uintptr_t)a; };
+        const uint32_t yb = st * CBUF, zb = Z0 + st * CBUF;
         static_for<2>([&](auto kb_c) {
             constexpr int kb = decltype(kb_c)::value;
+            // the products start from -L and -Delta where those come with the streamed rows, from zero where they are the lane's
             f32x16 s, dp;
+            auto start = [&](f32x16 &a, int which) {
 #pragma unroll
-            for (int i = 0; i < 16; i++) s[i] = 0.f;
+                for (int g = 0; g < 4; g++) {
+                    f32x4 x = {0.f, 0.f, 0.f, 0.f};
+                    if constexpr (!LANE_STATS) x = *(const SA_LDS f32x4 *)lds(sb + st * 512 + 256 * which + 128 * kb + 32 * g);
 #pragma unroll
-            for (int c = 0; c < NC; c++) s = E::mfma(*(const u32x4 *)(yb + 32 * kb * ROWB + noff[c]), xf[c], s);
+                    for (int jj = 0; jj < 4; jj++) a[4 * g + jj] = x[jj];
+                }
+            };
+            start(s, 0);
+#pragma unroll
+            for (int c = 0; c < NC; c++) s = E::mfma(*(const SA_LDS u32x4 *)lds((nb ^ (32 * c)) + yb + 32 * kb * ROWB), xf[c], s);
+            if constexpr (DS) asm volatile("" : "+v"(s));
+            paced();
+            phase();
             if constexpr (!OUT_P) {
+                start(dp, 1);
 #pragma unroll
-                for (int i = 0; i < 16; i++) dp[i] = 0.f;
-#pragma unroll
-                for (int c = 0; c < NC; c++) dp = E::mfma(*(const u32x4 *)(zb + 32 * kb * ROWB + noff[c]), gf[c], dp);
+                for (int c = 0; c < NC; c++) dp = E::mfma(*(const SA_LDS u32x4 *)lds((nb ^ (32 * c)) + zb + 32 * kb * ROWB), gf[c], dp);
             }
+            if constexpr (DS) asm volatile("" : "+v"(s), "+v"(dp));
+            paced();
+            phase();
             if (t >= F) {
                 // w: bit 8g + jj says whether this lane's entry (streamed row 32kb + 8g + 4hh + jj) attends
                 uint32_t w;
                 if constexpr (PK) {  // bit k of the packed word: streamed row 32kb + k
-                    w = *(const uint32_t *)(smem + MASK0 + st * 1024 + wave * 256 + 8 * l32 + 4 * kb) >> (4 * hh);
+                    w = *(const SA_LDS uint32_t *)lds(lds0 + MASK0 + st * 1024 + wave_u * 256 + 8 * (ln & 31) + 4 * kb) >> (4 * (ln >> 5));
                 } else {  // one byte per entry: the non-zero bytes of each dword become four bits
                     w = 0u;
 #pragma unroll
@@ -260,20 +339,12 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
             uint32_t pw[8], pp[BOTH ? 8 : 1];
 #pragma unroll
             for (int g = 0; g < 4; g++) {
-                f32x4 L4, D4;
-                if constexpr (LANE_STATS) {
-                    L4 = f32x4{laneL, laneL, laneL, laneL};
-                    D4 = f32x4{laneD, laneD, laneD, laneD};
-                } else {
-                    L4 = *(const f32x4 *)(sl + 32 * kb + 8 * g + 4 * hh);
-                    D4 = *(const f32x4 *)(sl + 64 + 32 * kb + 8 * g + 4 * hh);
-                }
                 float w[4], pv[4];
 #pragma unroll
                 for (int jj = 0; jj < 4; jj++) {
-                    const float pr = __builtin_amdgcn_exp2f(s[4 * g + jj] - L4[jj]);
+                    const float pr = __builtin_amdgcn_exp2f(LANE_STATS ? s[4 * g + jj] + laneL : DS ? s[4 * g + jj] * p.scale : s[4 * g + jj]);
                     pv[jj] = pr;
-                    w[jj] = OUT_P ? pr : pr * (dp[4 * g + jj] - D4[jj]);
+                    w[jj] = OUT_P ? pr : pr * (LANE_STATS ? dp[4 * g + jj] + laneD : dp[4 * g + jj]);
                 }
                 pw[2 * g] = E::pack2(w[0], w[1]);
                 pw[2 * g + 1] = E::pack2(w[2], w[3]);
@@ -282,26 +353,35 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
                     pp[2 * g + 1] = E::pack2(pv[2], pv[3]);
                 }
             }
-            const uint8_t *tb = (OUT_P ? zb : yb) + 32 * kb * ROWB;
+            if constexpr (DS) {  // (the order of the pieces: bwd_dq_tile)
+#pragma unroll
+                for (int c = 0; c < 2; c++)
+                    *(u32x4 *)(ds_out(t) + 4096 * kb + 1024 * c + (uint32_t)((32 * (ln & 31) + 16 * (ln >> 5)) ^ (128 * c))) =
+                        u32x4{pw[4 * c], pw[4 * c + 1], pw[4 * c + 2], pw[4 * c + 3]};
+            }
+            phase();
+            const uint32_t tb = (OUT_P ? zb : yb) + 32 * kb * ROWB;
             static_for<2>([&](auto kc_c) {
                 constexpr int kc = decltype(kc_c)::value;
                 const u32x4 pk4 = u32x4{pw[4 * kc], pw[4 * kc + 1], pw[4 * kc + 2], pw[4 * kc + 3]};
 #pragma unroll
                 for (int db = 0; db < NDB; db++) {
-                    const u32x2 lo = E::tr_read(tb + 16 * kc * ROWB + toff[0][db]);
-                    const u32x2 hi = E::tr_read(tb + 16 * kc * ROWB + toff[1][db]);
+                    const u32x2 lo = E::tr_read(lds((tb0 ^ (64 * db)) + tb + 16 * kc * ROWB));
+                    const u32x2 hi = E::tr_read(lds((tb0 ^ (64 * db) ^ bwd_tr_rows8<D>) + tb + 16 * kc * ROWB));
                     acc[db] = E::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, pk4, acc[db]);
                 }
+                phase();
                 if constexpr (BOTH) {
-                    const uint8_t *vb = zb + 32 * kb * ROWB;
+                    const uint32_t vb = zb + 32 * kb * ROWB;
                     const u32x4 pp4 = u32x4{pp[4 * kc], pp[4 * kc + 1], pp[4 * kc + 2], pp[4 * kc + 3]};
 #pragma unroll
                     for (int db = 0; db < NDB; db++) {
-                        const u32x2 lo = E::tr_read(vb + 16 * kc * ROWB + toff[0][db]);
-                        const u32x2 hi = E::tr_read(vb + 16 * kc * ROWB + toff[1][db]);
+                        const u32x2 lo = E::tr_read(lds((tb0 ^ (64 * db)) + vb + 16 * kc * ROWB));
+                        const u32x2 hi = E::tr_read(lds((tb0 ^ (64 * db) ^ bwd_tr_rows8<D>) + vb + 16 * kc * ROWB));
                         acc2[db] = E::mfma(u32x4{lo.x, lo.y, hi.x, hi.y}, pp4, acc2[db]);
                     }
                 }
+                phase();
             });
         });
     };
@@ -323,12 +403,15 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
         }
         if constexpr (LANE_STATS) asm volatile("" : "+v"(laneL), "+v"(laneD));
         if (T > 0) issue(0, 0, mk[0]);
+        if constexpr (DS) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         for (int t0 = 0; t0 < T; t0 += NS) {
             static_for<NS>([&](auto jc) {
                 constexpr int j = decltype(jc)::value, jn = j ^ 1;
                 const int t = t0 + j;
                 if (t >= T) return;
-                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // own pieces of chunk t and its mask words
+                // own pieces of chunk t and its mask words; four stores of dS came after their requests
+                if constexpr (DS) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+                else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 if constexpr (!PK) {
 #pragma unroll
                     for (int i = 0; i < NMW; i++) asm volatile("" ::"v"(mk[j][i]));
@@ -340,41 +423,139 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
         }
     }
 
-    // out = acc * out_scale; acc holds the transposed tile: lane (row l32, hh), register 4g + jj of block db is
-    // d = 32 db + 8g + 4hh + jj.  A lane's 8-byte pieces would make every store instruction touch 32 rows, so the
-    // wave's 32 rows go through a private slice of the (now idle) chunk buffers, rows 16 bytes apart from the banks'
-    // period, and leave as whole rows, 16 bytes per lane.
     __syncthreads();  // every wave is done with the chunk buffers
-    constexpr int OROW = ROWB + 16;
-    static_assert(4 * 32 * OROW <= 2 * NS * CBUF, "the rows of the four waves fit the chunk buffers");
-    uint8_t *const ob = smem + wave * 32 * OROW;
-    constexpr int PPR_O = ROWB / 16;  // 16-byte pieces per row
+    static_assert(4 * 32 * bwd_out_row<D> <= 2 * NS * CBUF, "the rows of the four waves fit the chunk buffers");
+    uint8_t *const ob = smem + wave_u * 32 * bwd_out_row<D>;
+    int ln = lane;
+    if constexpr (DS) asm volatile("" : "+v"(ln));
     // Where the rows go is read from the argument block only now (the pointer passes through an asm statement): held in
     // scalar registers through the loop these strides had others spilled.
     typedef const __attribute__((address_space(4))) BwdLaunch *ArgPtr;
     ArgPtr args = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(args));
     auto store = [&](const f32x16(&a)[NDB], float scale, uint16_t *out, int64_t os0, int64_t os1, int64_t os2) {
-#pragma unroll
-        for (int db = 0; db < NDB; db++)
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const u32x2 w = {E::pack2(a[db][4 * g] * scale, a[db][4 * g + 1] * scale),
-                                 E::pack2(a[db][4 * g + 2] * scale, a[db][4 * g + 3] * scale)};
-                *(u32x2 *)(ob + l32 * OROW + 2 * (32 * db + 8 * g + 4 * hh)) = w;
-            }
-        uint16_t *const o0 = out + b * os0 + h * os1 + (int64_t)(rt * 128 + wave * 32) * os2;
-#pragma unroll
-        for (int i = 0; i < 32 * PPR_O / 64; i++) {
-            const int idx = 64 * i + lane, r = idx / PPR_O, pc = idx % PPR_O;
-            const u32x4 x = *(const u32x4 *)(ob + r * OROW + 16 * pc);
-            // (written once, whole rows: a streaming store leaves the streamed operands' lines in L2 alone)
-            __builtin_nontemporal_store(x, (u32x4 *)(o0 + (int64_t)r * os2 + 8 * pc));
-        }
+        bwd_store_rows<DT, D>(a, scale, ob, out + b * os0 + h * os1 + (int64_t)(rt * 128 + wave_u * 32) * os2, os2, ln);
     };
     store(acc, args->pass[PASS].out_scale, args->pass[PASS].out, args->pass[PASS].outs[0], args->pass[PASS].outs[1], args->pass[PASS].outs[2]);
     if constexpr (BOTH)  // (a wave's slice is its own: its reads above come first)
         store(acc2, 1.f, args->pass[PASS].out2, args->pass[PASS].outs2[0], args->pass[PASS].outs2[1], args->pass[PASS].outs2[2]);
+}
+
+// dQ from the dS that the pass over the keys stored: dQ^T += K^T . dS^T, one product instead of three, bound by the reads
+// of dS (B8 H16 S4096 causal: 2.15 GB in 505 us, 4.3 TB/s; 312 us with the same dS from L2, so neither the products nor the
+// loads into LDS bound it; two stages and four workgroups per compute unit: 535 us).  128 queries per workgroup, 32 per wave; a chunk of 64 keys is 16 KiB of K, shared, and 4 KiB of dS per wave.
+// dS lies as [plane][128 queries][64 keys][32 queries][32 keys]: what a workgroup here reads is contiguous.  In the 2 KiB of
+// the last two,
+// key k's queries 8g + 4h .. + 3 are the 8 bytes at 1024 (g / 2) + ((32 k + 16 h) ^ 128 (g / 2)) + 8 (g & 1): the key
+// pass stores 1 KiB per instruction, and a transposing read (four keys, two groups of 16 queries) meets no bank twice.
+// A block that the key pass did not visit holds whatever the memory held: none of its entries attends, so it lies in
+// PARTIAL tiles only, where the entries that do not attend are set to zero here.
+template <int D>
+struct BwdDqLds {
+    static constexpr int NST = 4, SBUF = 32 * D * 2;  // stages, and bytes of K in one; of dS as many at D = 128
+    static constexpr int DS0 = NST * SBUF, MASK0 = DS0 + NST * 8192, LIST0 = MASK0 + 4096, bytes = LIST0 + kBwdListCap * 2;
+};
+template <int DT, int D>
+__device__ __forceinline__ void bwd_dq_tile(const BwdParams &p, int lin, int total, uint8_t *smem) {
+    using E = Elem<DT>;
+    using Lds = BwdDqLds<D>;
+    constexpr int ROWB = D * 2, NDB = D / 32, PPR = ROWB / 16, RPI = 64 / PPR, SLD = 8 / RPI;
+    constexpr int NST = Lds::NST, SBUF = Lds::SBUF, DS0 = Lds::DS0, MASK0 = Lds::MASK0;
+    uint16_t *const ent = reinterpret_cast<uint16_t *>(smem + Lds::LIST0);
+    const int tid = threadIdx.x, lane = tid & 63, wave_u = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, hh = lane >> 5;
+    const BwdPlace at = bwd_place(p, lin, total);
+    const int plane = at.plane, rt = at.rt, bh = p.plane0 + plane;
+    const int b = bh / p.H, h = bh - b * p.H;
+    const uint16_t *ybase = p.y + b * p.ys[0] + h * p.ys[1];
+    const int32_t *fid = p.full_ids + b * p.fis[0] + h * p.fis[1] + rt * p.fis[2];
+    const int32_t *pid = p.part_ids + b * p.pis[0] + h * p.pis[1] + rt * p.pis[2];
+    const uint8_t *prow = p.packed + b * p.pks[0] + h * p.pks[1] + (int64_t)rt * p.nS * 1024 + wave_u * 256;
+    const uint8_t *dsbase = p.ds + ((int64_t)plane * p.nR + rt) * p.nS * 16384 + wave_u * 4096;
+    int cnt[2];  // (clamped as in bwd_tile)
+    const int32_t *const cnt_addr[2] = {p.full_lens + (b * p.fls[0] + h * p.fls[1] + rt * p.fls[2]),
+                                        p.part_lens + (b * p.pls[0] + h * p.pls[1] + rt * p.pls[2])};
+    scalar_gather(cnt_addr, cnt);
+    const int F = min(max(cnt[0], 0), p.nS);
+    const int T = F + min(max(cnt[1], 0), p.nS - F);
+    f32x16 acc[NDB];
+#pragma unroll
+    for (int db = 0; db < NDB; db++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[db][i] = 0.f;
+    const int tbase = bwd_tr_base<D>(lane);
+    const int cq = (lane >> 4) & 1;
+    const int dbase = 1024 * cq + 128 * (hh ^ cq) + 32 * ((lane & 15) >> 2) + 16 * (lane & 1) + 8 * ((lane >> 1) & 1);
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const SA_LDS uint8_t *)smem);
+    const int ld_row = RPI * wave_u + lane / PPR, ld_piece = (lane % PPR) ^ bwd_swizzle<D>(ld_row);
+    const uint32_t ld_yoff = (uint32_t)((ld_row * p.ys[2] + 8 * ld_piece) * 2);
+    for (int e = tid; e < T; e += 256) {
+        const int idx = e < F ? fid[(int64_t)e * p.fis[3]] : pid[(int64_t)(e - F) * p.pis[3]];
+        ent[e] = (uint16_t)min(max(idx, 0), p.nS - 1);
+    }
+    __syncthreads();
+    // Steps of 32 keys, two per list entry.
+    const int64_t ytile = 64 * p.ys[2], yhalf = 32 * p.ys[2], yload = 4 * RPI * p.ys[2];
+    auto issue = [&](int u, int st) {
+        const int t = u >> 1, kt = __builtin_amdgcn_readfirstlane(ent[t]);
+        const uint8_t *dsp = dsbase + (int64_t)kt * 16384 + (u & 1) * 2048;
+        if (t >= F && (u & 1) == 0) dma4(prow + (int64_t)(t - F) * 1024, 4 * lane, lds0 + MASK0 + (t & 3) * 1024 + wave_u * 256);
+#pragma unroll
+        for (int i = 0; i < 2; i++) dma16<true>(dsp + 1024 * i, 16 * lane, lds0 + DS0 + st * 8192 + wave_u * 2048 + 1024 * i);
+        const uint16_t *yp = ybase + kt * ytile + ((u & 1) ? yhalf : 0);
+#pragma unroll
+        for (int i = 0; i < SLD; i++) dma16(yp + i * yload, ld_yoff, lds0 + st * SBUF + 1024 * (4 * i + wave_u));
+    };
+    auto compute = [&](int u, int st) {
+        const uint8_t *yb = smem + st * SBUF, *db_ = smem + DS0 + st * 8192 + wave_u * 2048 + dbase;
+        u32x4 x[2];  // dS^T of keys 16kc ..
+#pragma unroll
+        for (int kc = 0; kc < 2; kc++) {
+            const u32x2 lo = E::tr_read(db_ + 512 * kc), hi = E::tr_read(db_ + 512 * kc + 256);
+            x[kc] = u32x4{lo.x, lo.y, hi.x, hi.y};
+        }
+        const int t = u >> 1;
+        if (t >= F) {  // bit k of the packed word: key k of the step
+            const uint32_t w = *(const uint32_t *)(smem + MASK0 + (t & 3) * 1024 + wave_u * 256 + 8 * l32 + 4 * (u & 1)) >> (4 * hh);
+#pragma unroll
+            for (int kc = 0; kc < 2; kc++)
+#pragma unroll
+                for (int d = 0; d < 4; d++) {
+                    const uint32_t two = w >> (16 * kc + 8 * (d >> 1) + 2 * (d & 1));
+                    x[kc][d] &= ((two & 1u) ? 0xffffu : 0u) | ((two & 2u) ? 0xffff0000u : 0u);
+                }
+        }
+#pragma unroll
+        for (int kc = 0; kc < 2; kc++)
+#pragma unroll
+            for (int db = 0; db < NDB; db++) {
+                const uint8_t *tb = yb + 16 * kc * ROWB;
+                const u32x2 klo = E::tr_read(tb + (tbase ^ (64 * db)));
+                const u32x2 khi = E::tr_read(tb + (tbase ^ (64 * db) ^ bwd_tr_rows8<D>));
+                acc[db] = E::mfma(u32x4{klo.x, klo.y, khi.x, khi.y}, x[kc], acc[db]);
+            }
+    };
+    const int U = 2 * T;
+#pragma unroll
+    for (int u = 0; u < NST - 1; u++)
+        if (u < U) issue(u, u);
+    for (int u0 = 0; u0 < U; u0 += NST) {
+        static_for<NST>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            const int u = u0 + j;
+            if (u >= U) return;
+            // own pieces of step u: behind them are the loads of at most two steps, four or (with mask words) five each
+            if (u + 2 < U) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (2 + SLD)) : "memory");
+            else if (u + 1 < U) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 + SLD) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();  // everyone's pieces; and everyone is done with the stage of step u - 1
+            if (u + NST - 1 < U) issue(u + NST - 1, (j + NST - 1) % NST);
+            compute(u, j);
+        });
+    }
+    __syncthreads();
+    bwd_store_rows<DT, D>(acc, p.out_scale, smem + wave_u * 32 * bwd_out_row<D>,
+                          p.out + b * p.outs[0] + h * p.outs[1] + (int64_t)(rt * 128 + wave_u * 32) * p.outs[2], p.outs[2], lane);
 }
 
 // D = 64 with packed tiles: three workgroups per compute unit (168 registers, 43 KB of LDS; a third stage of the chunks
@@ -405,7 +586,21 @@ __global__ __launch_bounds__(256, D == 64 && PK ? 3 : 2) void sparse_bwd_kernel(
     }
 }
 
-// Per query row: Delta = sum_d dO o O, and L = lse / ln 2 (+inf for rows that attended to nothing, so that their
+// dK, dV and dS from one walk over the keys' lists.
+template <int DT>
+__global__ __launch_bounds__(256, 2) void sparse_bwd_keys_kernel(const BwdLaunch l) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    bwd_tile<DT, 128, kDKV, true, 0, true>(l.pass[0], blockIdx.x, l.tiles[0], smem);
+}
+
+// dQ from the stored dS.  LDS: [K, four stages][dS, four stages][mask words of four entries][list]
+template <int DT, int D>
+__global__ __launch_bounds__(256, 2) void sparse_bwd_queries_kernel(const BwdParams p, int tiles) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    bwd_dq_tile<DT, D>(p, blockIdx.x, tiles, smem);
+}
+
+// Per query row: -Delta = -sum_d dO o O, and -L = -lse / ln 2 (-inf for rows that attended to nothing, so that their
 // P = exp2(S - L) is 0).  D/8 lanes per row, 8 elements each.
 template <int DT, int D>
 __global__ __launch_bounds__(256) void bwd_prepare_kernel(const BwdPrepParams p) {
@@ -435,8 +630,8 @@ __global__ __launch_bounds__(256) void bwd_prepare_kernel(const BwdPrepParams p)
     for (int m = LPR / 2; m >= 1; m >>= 1) sum += __shfl_xor(sum, m, LPR);
     if (part == 0) {
         const float lse = p.lse[b * p.ls[0] + h * p.ls[1] + (int64_t)q * p.ls[2]];
-        p.stat_l[row] = lse == kNegInf ? __builtin_inff() : lse * 1.44269504089f;
-        p.stat_d[row] = sum;
+        p.stat_l[row] = lse == kNegInf ? kNegInf : lse * p.l_mul;
+        p.stat_d[row] = -sum;
     }
 }
 
@@ -464,6 +659,38 @@ hipError_t launch_bwd_one(const BwdParams &dq, const BwdParams &dk, const BwdPar
     return hipGetLastError();
 }
 
+// The planes in groups of `group`, whose dS takes its turn in the workspace.  (The key tiles of a group in one launch with the
+// query tiles of the group before, dealt out evenly: 2 ... 15 % slower than launches of their own, with 2 ... 8 groups.)
+template <int DT>
+hipError_t launch_bwd_ds(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, uint8_t *ds, int group, hipStream_t stream) {
+    constexpr int smem = BwdLds<128, true>::bytes;
+    auto kern = sparse_bwd_keys_kernel<DT>;
+    static unsigned long long attr_done = 0;
+    if (const hipError_t e0 = allow_dynamic_smem(kern, smem, attr_done); e0 != hipSuccess) return e0;
+    auto kern_q = sparse_bwd_queries_kernel<DT, 128>;
+    static unsigned long long attr_done_q = 0;
+    if (const hipError_t e0 = allow_dynamic_smem(kern_q, BwdDqLds<128>::bytes, attr_done_q); e0 != hipSuccess) return e0;
+    const int planes = dq.B * dq.H;
+    for (int p0 = 0; p0 < planes; p0 += group) {
+        BwdLaunch l{};
+        l.pass[0] = dk;
+        l.pass[0].out2 = dv.out;
+        for (int c = 0; c < 3; c++) l.pass[0].outs2[c] = dv.outs[c];
+        BwdParams q = dq;
+        for (BwdParams *p : {&l.pass[0], &q}) {
+            p->plane0 = p0;
+            p->planes = planes - p0 < group ? planes - p0 : group;
+            p->ds = ds;
+        }
+        l.tiles[0] = l.pass[0].planes * dk.nR;
+        hipLaunchKernelGGL(kern, dim3((unsigned)l.tiles[0]), dim3(256), smem, stream, l);
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+        hipLaunchKernelGGL(kern_q, dim3((unsigned)(q.planes * q.nR)), dim3(256), BwdDqLds<128>::bytes, stream, q, q.planes * q.nR);
+        if (const hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 template <int DT, int D>
 hipError_t launch_prepare_one(const BwdPrepParams &p, hipStream_t stream) {
     const int64_t rows = (int64_t)p.B * p.H * p.Sq;
@@ -474,7 +701,37 @@ hipError_t launch_prepare_one(const BwdPrepParams &p, hipStream_t stream) {
 
 }  // namespace
 
-hipError_t launch_bwd(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, int dtype, int D, hipStream_t stream) {
+// dS through memory: a pass over the keys (S, dP, dK, dV) and one over the queries (dQ), against one launch of three passes
+// and 8 products.  It needs the device filled twice over by the key tiles alone (two workgroups on each of 256 compute units):
+// causal, D = 128, backward with prepare in us, dS | three passes:
+//   256 key tiles  B1 H32 S1024  68 |  58   B1 H8  S4096  206 |  191   B2 H8 S2048 113 | 93
+//   512            B8 H32 S256   49 |  52   B2 H16 S2048  158 |  166   B1 H16 S4096 256 | 292   B1 H8 S8192 500 | 629
+//   1024           B8 H32 S512  113 | 127   B4 H16 S2048  263 |  313   B2 H16 S4096 443 | 546
+//   4096           B8 H16 S4096 1792 | 2195;  documents of 512 B4 H16 S8192 452 | 560;  random blocks B1 H16 S4096 132 | 162
+// D = 64 stays with its two passes: dS is as large there and its two products half as long.
+int bwd_ds_group(int B, int H, int Sq, int Sk, int D, size_t bytes) {
+    constexpr int64_t kLeastTiles = 512;  // key tiles of a group
+    if (D != 128) return 0;
+    const size_t plane = (size_t)Sq * Sk * 2;
+    const int64_t planes = (int64_t)B * H;
+    int64_t n = (int64_t)(bytes / plane);
+    if (n > planes) n = planes;
+    if (n * (Sk / 128) < kLeastTiles) return 0;
+    const int64_t groups = (planes + n - 1) / n;
+    n = (planes + groups - 1) / groups;  // groups of even size
+    return n * (Sk / 128) < kLeastTiles ? 0 : (int)n;
+}
+
+// At most 4 GiB, a seventieth of the device's memory.
+size_t bwd_ds_bytes(int B, int H, int Sq, int Sk, int D) {
+    return (size_t)Sq * Sk * 2 * bwd_ds_group(B, H, Sq, Sk, D, (size_t)4 << 30);
+}
+
+hipError_t launch_bwd(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, int dtype, int D, uint8_t *ds, int group, hipStream_t stream) {
+    if (group > 0) {
+        if (dtype == 0) return launch_bwd_ds<0>(dq, dk, dv, ds, group, stream);
+        return launch_bwd_ds<1>(dq, dk, dv, ds, group, stream);
+    }
     const bool pk = dq.packed != nullptr && dk.packed != nullptr;  // (with only one of them the mask is there too)
 #define SA_BWD(DT, DD) \
     if (dtype == DT && D == DD) \

@@ -985,6 +985,16 @@ size_t sa_bwd_workspace_bytes(int B, int H, int Sq) {
     return (size_t)B * H * Sq * 2 * sizeof(float);
 }
 
+// where dS starts in the workspace, behind `stats` bytes of statistics
+static size_t ds_offset(size_t stats) { return (stats + 1023) & ~(size_t)1023; }
+
+size_t sa_bwd_workspace_bytes_ex(int B, int H, int Sq, int Sk, int D) {
+    const size_t stats = sa_bwd_workspace_bytes(B, H, Sq);
+    if (stats == 0 || Sk <= 0) return 0;
+    const size_t ds = sa::bwd_ds_bytes(B, H, Sq, Sk, D);
+    return ds ? ds_offset(stats) + ds : stats;
+}
+
 int sa_sparse_attention_bwd(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
                             const void *v, const int64_t v_strides[4], const void *o, const int64_t o_strides[4],
                             const void *d_o, const int64_t do_strides[4], const float *lse,
@@ -1058,6 +1068,10 @@ int sa_sparse_attention_bwd(const void *q, const int64_t q_strides[4], const voi
     }
     pp.stat_l = stat_l;
     pp.stat_d = stat_d;
+    // what the workspace holds besides the statistics takes dS, where that pays
+    uint8_t *const ds = static_cast<uint8_t *>(workspace) + ds_offset(need);
+    const int group = q_packed && k_packed && workspace_bytes > ds_offset(need) ? sa::bwd_ds_group(B, H, Sq, Sk, D, workspace_bytes - ds_offset(need)) : 0;
+    pp.l_mul = group > 0 ? -1.44269504089f / sm_scale_log2 : -1.44269504089f;
     pp.B = B;
     pp.H = H;
     pp.Sq = Sq;
@@ -1086,6 +1100,7 @@ int sa_sparse_attention_bwd(const void *q, const int64_t q_strides[4], const voi
     bp.sts[2] = 1;
     bp.B = B;
     bp.H = H;
+    bp.planes = B * H;
     bp.scale = sm_scale_log2;
     const bool m4 = mask && aligned(mask, 4) && mask_strides[0] % 4 == 0 && mask_strides[1] % 4 == 0;
 
@@ -1171,7 +1186,7 @@ int sa_sparse_attention_bwd(const void *q, const int64_t q_strides[4], const voi
     bp.out = static_cast<uint16_t *>(dv);
     set3(bp.outs, dv_strides);
     bp.out_scale = 1.f;
-    e = sa::launch_bwd(dq_pass, dk_pass, bp, dtype, D, hs);
+    e = sa::launch_bwd(dq_pass, dk_pass, bp, dtype, D, ds, group, hs);
     if (e != hipSuccess) return fail(SA_ERR_HIP, "sa_sparse_attention_bwd: launch failed: %s", hipGetErrorString(e));
     return SA_OK;
 }

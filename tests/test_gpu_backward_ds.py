@@ -1,0 +1,62 @@
+"""The backward whose dQ comes from stored dS (D = 128, packed tiles, 512 key tiles and more): masks with blocks no pass visits,
+a query without a key and a key without a query, one group of planes and several."""
+import pytest
+import torch
+
+from sparseattention_amd import compute_backward_metadata, compute_mask_kernel, sparse_attention, sparse_attention_backward
+from sparseattention_amd import _native
+
+pytestmark = pytest.mark.gpu
+
+
+def _poison(nbytes, gpu):
+    """Leaves NaN patterns in the memory that the next workspace of this size is taken from."""
+    torch.full((nbytes,), 0xFF, dtype=torch.uint8, device=gpu)
+
+
+def _rel(a, b):
+    return float((a.double() - b.double()).norm() / b.double().norm())
+
+
+# Outputs of a correct backward are within 3.2e-3 (bf16) and 3.8e-4 (fp16) of float64 in the relative 2-norm; twice that.
+@pytest.mark.parametrize("dtype,tol", [(torch.bfloat16, 6.4e-3), (torch.float16, 8e-4)])
+@pytest.mark.parametrize("B,H,Sq,Sk", [(2, 32, 1024, 1024), (1, 57, 128, 1152), (4, 128, 128, 128)])
+def test_gradients_against_float64(gpu, dtype, tol, B, H, Sq, Sk):
+    assert _native.load().sa_bwd_workspace_bytes_ex(B, H, Sq, Sk, 128) > B * H * Sq * Sk * 2
+    g = torch.Generator().manual_seed(Sq + Sk)
+    q, k, v, do = (torch.randn(B, H, S, 128, generator=g).to(gpu, dtype) for S in (Sq, Sk, Sk, Sq))
+    mask = torch.rand(B, 1, Sq, Sk, generator=g) < 0.6
+    mask[..., : Sk // 2] = True                       # FULL tiles
+    mask[:, :, Sq // 2:, Sk // 4: Sk // 2] = False    # EMPTY ones
+    mask[:, :, :64, Sk - 128:] = False                # empty for the key pass, half of a PARTIAL tile for the query pass
+    mask[0, 0, 3] = False                             # a query without a key
+    mask[0, 0, :, 5] = False                          # a key without a query
+    mask = mask.to(gpu).expand(B, H, Sq, Sk)
+    o, lse = sparse_attention(q, k, v, mask, 128, 64, return_lse=True)
+    bmd = compute_backward_metadata(mask)
+    _poison(_native.load().sa_bwd_workspace_bytes_ex(B, H, Sq, Sk, 128), gpu)
+    got = sparse_attention_backward(do, q, k, v, o, lse, None, bmd)
+
+    q64, k64, v64 = (t.double().requires_grad_(True) for t in (q, k, v))
+    s = (q64 @ k64.transpose(-1, -2).contiguous()) * 128 ** -0.5
+    (torch.softmax(s.masked_fill(~mask, float("-inf")), -1).nan_to_num() @ v64).backward(do.double())
+    for x, t in zip(got, (q64, k64, v64)):
+        assert torch.isfinite(x).all()
+        assert _rel(x, t.grad.nan_to_num()) <= tol
+
+
+def test_planes_in_groups(gpu):
+    """9 planes of 512 MiB of dS: groups of five and four through one workspace, against the passes that store nothing."""
+    B, H, S = 1, 9, 16384
+    assert 5 * S * S * 2 <= _native.load().sa_bwd_workspace_bytes_ex(B, H, S, S, 128) <= 5 * S * S * 2 + B * H * S * 8 + 1024
+    g = torch.Generator(device=gpu).manual_seed(1)
+    q, k, v, do = (torch.randn(B, S, H, 128, device=gpu, generator=g, dtype=torch.bfloat16).transpose(1, 2) for _ in range(4))
+    i = torch.arange(S, device=gpu)
+    mask = ((i[None] <= i[:, None]) & (i[:, None] - i[None] < 300))[None, None].expand(B, H, S, S)
+    o, lse = sparse_attention(q, k, v, mask, 128, 64, compute_mask_kernel(mask, 128, 64), return_lse=True)
+    _poison(5 * S * S * 2 + B * H * S * 8, gpu)
+    got = sparse_attention_backward(do, q, k, v, o, lse, None, compute_backward_metadata(mask))
+    want = sparse_attention_backward(do, q, k, v, o, lse, mask, compute_backward_metadata(mask, pack_partial=False))
+    for x, y in zip(got, want):
+        assert torch.isfinite(x).all()
+        assert _rel(x, y) <= 6.4e-3
