@@ -179,6 +179,16 @@ int sa_validate_metadata(const int32_t *full_ids, const int64_t full_ids_strides
                          int BQ, int BK, int32_t *flag, void *stream);
 
 /*
+ * sa_mask_classify and sa_mask_pack_partial (below) of its lists in one call: the same results, in one launch where the
+ * mask holds few bytes per Q tile.
+ */
+int sa_mask_classify_packed(const uint8_t *mask, const int64_t mask_strides[4], int B, int H, int Sq, int Sk, int BQ,
+                            int BK, int32_t *full_ids, const int64_t full_ids_strides[4], int32_t *full_lens,
+                            const int64_t full_lens_strides[3], int32_t *part_ids, const int64_t part_ids_strides[4],
+                            int32_t *part_lens, const int64_t part_lens_strides[3], uint8_t *packed,
+                            const int64_t packed_strides[2], void *workspace, size_t workspace_bytes, void *stream);
+
+/*
  * Bytes of the buffer sa_mask_pack_partial fills: Sq*Sk/8 for every DISTINCT mask plane (room for every
  * tile being PARTIAL, so that no count has to be read back to the host).  Returns 0 on invalid arguments
  * (BK must be a multiple of 8).

@@ -39,6 +39,7 @@ EXPORTS = (
     "sa_sparse_attention_fwd",
     "sa_mask_pack_partial_bytes",
     "sa_mask_pack_partial",
+    "sa_mask_classify_packed",
     "sa_fwd_schedule_bytes",
     "sa_fwd_schedule",
     "sa_sparse_attention_fwd_ex",
@@ -105,6 +106,8 @@ def load() -> ctypes.CDLL:
     )
     lib.sa_mask_pack_partial_bytes.restype = ctypes.c_size_t
     lib.sa_mask_pack_partial_bytes.argtypes = [_i64p] + [ctypes.c_int] * 6
+    lib.sa_mask_classify_packed.restype = ctypes.c_int
+    lib.sa_mask_classify_packed.argtypes = [_vp, _i64p] + [ctypes.c_int] * 6 + [_vp, _i64p] * 5 + [_vp, ctypes.c_size_t, _vp]
     lib.sa_mask_pack_partial.restype = ctypes.c_int
     lib.sa_mask_pack_partial.argtypes = [_vp, _i64p] + [ctypes.c_int] * 6 + [_vp, _i64p] * 3 + [_vp]
     lib.sa_fwd_schedule_bytes.restype = ctypes.c_size_t

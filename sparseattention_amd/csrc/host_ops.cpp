@@ -199,11 +199,13 @@ Lists classify_lists(const Tensor &mask, int64_t BQ, int64_t BK, std::optional<b
     const size_t need = sa_mask_classify_workspace_bytes(st(mask), B, H, Sq, Sk, BQ, BK);
     // (dropped at the end of this call: the allocator hands the block out again only behind these launches on the stream)
     const Tensor ws = at::empty({(int64_t)std::max<size_t>(need, 1)}, at::TensorOptions().dtype(at::kByte).device(mask.device()));
-    check_rc(sa_mask_classify(ptr<uint8_t>(mask), st(mask), B, H, Sq, Sk, BQ, BK, ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl),
-                              ptr<int32_t>(l.pid), st(l.pid), ptr<int32_t>(l.pl), st(l.pl), ws.data_ptr(), ws.numel(), stream));
     if (pack)
-        check_rc(sa_mask_pack_partial(ptr<uint8_t>(mask), st(mask), B, H, Sq, Sk, BQ, BK, ptr<int32_t>(l.pid), st(l.pid), ptr<int32_t>(l.pl),
-                                      st(l.pl), ptr<uint8_t>(*l.packed), st(*l.packed), stream));
+        check_rc(sa_mask_classify_packed(ptr<uint8_t>(mask), st(mask), B, H, Sq, Sk, BQ, BK, ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl),
+                                         ptr<int32_t>(l.pid), st(l.pid), ptr<int32_t>(l.pl), st(l.pl), ptr<uint8_t>(*l.packed), st(*l.packed),
+                                         ws.data_ptr(), ws.numel(), stream));
+    else
+        check_rc(sa_mask_classify(ptr<uint8_t>(mask), st(mask), B, H, Sq, Sk, BQ, BK, ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl),
+                                  ptr<int32_t>(l.pid), st(l.pid), ptr<int32_t>(l.pl), st(l.pl), ws.data_ptr(), ws.numel(), stream));
     return l;
 }
 

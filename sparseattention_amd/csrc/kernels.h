@@ -40,6 +40,17 @@ struct PackParams {
     int vec8;  // 1: key stride 1 and every row segment 8-byte aligned, so 8 entries load as one qword
 };
 
+// Classification, compaction and (packed not null) packing in one launch, a workgroup per Q tile (classify_rows_kernel).
+struct ClassifyRowsParams {
+    ClassifyParams c;  // (cls unused)
+    CompactParams l;
+    uint8_t *packed;
+    int64_t ob, oh;
+};
+// The rule: mask_classify.hip.  The mask must suit the wide kernel, `packed` and its plane strides even addresses.
+bool classify_rows_has(const ClassifyParams &p);
+hipError_t launch_classify_rows(const ClassifyRowsParams &p, hipStream_t stream);
+
 // Q tiles dealt out to G persistent workgroups (G a multiple of 8, G/8 <= 64).  Workgroup g = 8*j + x is taken
 // to run on XCD x (hardware hands consecutive workgroup ids to the XCDs in turn) and gets Q tiles of the x-th
 // eighth of the (b,h)-major order, so that the tiles sharing a K/V plane meet in one L2.

@@ -13,6 +13,8 @@
 //   pack_partial_kernel (optional, no counterpart in the reference)
 //       one bit per entry of every PARTIAL tile, so that the forward reads BQ*BK/8 contiguous bytes per
 //       partial tile instead of BQ row segments of the mask (sparse_attn_kernel.py:42-46).
+//   classify_rows_kernel
+//       all three in one launch, for masks of few bytes per Q tile.
 //
 // A byte != 0 counts as "attend", so masks that were viewed from uint8 storage behave like torch.sum.
 #include <hip/hip_runtime.h>
@@ -191,6 +193,103 @@ __global__ __launch_bounds__(256) void pack_partial_kernel(const PackParams p) {
     }
 }
 
+// The three steps above in one launch for masks of few bytes per Q tile, where each is a launch's latency: grid (nQ,
+// distinct planes), a workgroup of eight waves makes everything of one Q tile and the tiles' states stay in LDS.
+//   rows     16 bytes per lane and row, as classify_wide_kernel; column blocks of 64 lanes are dealt to the waves, and where
+//            there are fewer than eight of them the rows of one are shared by several waves.  Rows of 16, 32 .. 512 bytes
+//            go several to a wave instruction.
+//   lists    wave 0 writes the FULL list, wave 1 the PARTIAL one, wave 2 + 3 the next output plane's ...
+//   packing  16 mask bytes, just read and in L2, become 16 bits per thread and step.
+constexpr int kRowsThreads = 512, kRowsWaves = kRowsThreads / 64;
+constexpr int kRowsTiles = 2048;  // KV tiles of a Q tile that LDS holds
+__global__ __launch_bounds__(kRowsThreads) void classify_rows_kernel(const ClassifyRowsParams a) {
+    __shared__ unsigned state[kRowsTiles];  // bit 0: some entry attends, bit 1: some entry does not
+    __shared__ uint16_t part[kRowsTiles];   // the PARTIAL tiles, in order
+    __shared__ int sh_np;
+    const ClassifyParams &p = a.c;
+    const CompactParams &l = a.l;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int qt = blockIdx.x, plane = blockIdx.y;
+    const int ub = plane / p.uH, uh = plane - ub * p.uH;
+    const uint8_t *rows = p.mask + (int64_t)ub * p.sb + (int64_t)uh * p.sh + (int64_t)qt * p.BQ * p.sq;
+    for (int i = tid; i < p.nK; i += kRowsThreads) state[i] = 0u;
+    __syncthreads();
+    {
+        const int pieces = p.Sk >> 4;  // 16-byte pieces of a row
+        const int per_row = pieces < 64 && (pieces & (pieces - 1)) == 0 ? pieces : 64;
+        const int rpi = 64 / per_row, sub = lane / per_row;  // rows of one wave instruction, and this lane's
+        const int blocks = (pieces + per_row - 1) / per_row;
+        const int groups = min(blocks, kRowsWaves), share = kRowsWaves / groups;  // waves that share a column block
+        if (wave < groups * share) {
+            const int step = share * rpi;
+            for (int cb = wave / share; cb < blocks; cb += groups) {
+                const int piece = cb * per_row + lane % per_row;
+                if (piece >= pieces) continue;
+                const uint8_t *base = rows + 16 * piece;
+                uint32_t any = 0u, all = 0x80808080u;
+                int r = (wave % share) * rpi + sub;
+                const bool mine = r < p.BQ;
+                for (; r + step * (kRowUnroll - 1) < p.BQ; r += step * kRowUnroll) {
+                    u32x4 v[kRowUnroll];
+#pragma unroll
+                    for (int u = 0; u < kRowUnroll; u++) v[u] = *(const u32x4 *)(base + (int64_t)(r + step * u) * p.sq);
+#pragma unroll
+                    for (int u = 0; u < kRowUnroll; u++) {
+                        any |= v[u].x | v[u].y | v[u].z | v[u].w;
+                        all &= nonzero_bytes(v[u].x) & nonzero_bytes(v[u].y) & nonzero_bytes(v[u].z) & nonzero_bytes(v[u].w);
+                    }
+                }
+                for (; r < p.BQ; r += step) {
+                    const u32x4 v = *(const u32x4 *)(base + (int64_t)r * p.sq);
+                    any |= v.x | v.y | v.z | v.w;
+                    all &= nonzero_bytes(v.x) & nonzero_bytes(v.y) & nonzero_bytes(v.z) & nonzero_bytes(v.w);
+                }
+                if (mine) atomicOr(&state[(16 * piece) >> p.lbk], (any != 0u ? 1u : 0u) | (all != 0x80808080u ? 2u : 0u));
+            }
+        }
+    }
+    __syncthreads();
+    // even waves the FULL list, odd ones the PARTIAL list, of every fourth output plane each
+    {
+        const int nb = l.bcast_b ? l.oB : 1, nh = l.bcast_h ? l.oH : 1;
+        const unsigned want = (wave & 1) ? 3u : 1u;
+        const unsigned long long below = (1ull << lane) - 1ull;
+        for (int pl = wave >> 1; pl < nb * nh; pl += kRowsWaves / 2) {
+            const int b = l.bcast_b ? pl / nh : ub, h = l.bcast_h ? pl % nh : uh;
+            int32_t *ids = (wave & 1) ? l.part_ids + b * l.pis[0] + h * l.pis[1] + qt * l.pis[2] : l.full_ids + b * l.fis[0] + h * l.fis[1] + qt * l.fis[2];
+            const int64_t step = (wave & 1) ? l.pis[3] : l.fis[3];
+            int found = 0;
+            for (int k0 = 0; k0 < p.nK; k0 += 64) {
+                const bool is = k0 + lane < p.nK && state[k0 + lane] == want;
+                const unsigned long long bits = __ballot(is);
+                const int at = found + __popcll(bits & below);
+                if (is) ids[(int64_t)at * step] = k0 + lane;
+                if (is && wave == 1 && pl == 0) part[at] = (uint16_t)(k0 + lane);
+                found += __popcll(bits);
+            }
+            if (lane == 0) {
+                if (wave & 1) l.part_lens[b * l.pls[0] + h * l.pls[1] + qt * l.pls[2]] = found;
+                else l.full_lens[b * l.fls[0] + h * l.fls[1] + qt * l.fls[2]] = found;
+                if (wave == 1 && pl == 0) sh_np = found;
+            }
+        }
+    }
+    if (a.packed == nullptr) return;
+    __syncthreads();
+    const int per_tile = p.BQ << (p.lbk - 4);  // 16-byte pieces of a tile
+    const int64_t total = (int64_t)sh_np * per_tile;
+    uint16_t *out = (uint16_t *)(a.packed + (int64_t)ub * a.ob + (int64_t)uh * a.oh + (int64_t)qt * p.nK * per_tile * 2);
+    for (int64_t i = tid; i < total; i += kRowsThreads) {
+        const int slot = (int)i / per_tile, w = (int)i - slot * per_tile;
+        const int r = w >> (p.lbk - 4), c = w & ((1 << (p.lbk - 4)) - 1);
+        const u32x4 v = *(const u32x4 *)(rows + (int64_t)r * p.sq + (int64_t)part[slot] * p.BK + 16 * c);
+        unsigned bits = 0u;
+#pragma unroll
+        for (int e = 0; e < 4; e++) bits |= ((((nonzero_bytes(v[e]) >> 7) * 0x00204081u) >> 21) & 0xfu) << (4 * e);
+        out[i] = (uint16_t)bits;
+    }
+}
+
 // One wave per (b, h, Q tile) row of the lists: bit 0 of *flag when a count is negative or the two counts exceed nK,
 // bit 1 when a FULL index inside its count lies outside [0, nK), bit 2 the same for a PARTIAL index.
 __global__ __launch_bounds__(256) void validate_lists_kernel(const ValidateParams p) {
@@ -224,6 +323,23 @@ hipError_t launch_validate(const ValidateParams &p, hipStream_t stream) {
 hipError_t launch_pack(const PackParams &p, hipStream_t stream) {
     const int lanes = p.nK < 8 ? p.nK : 8;
     hipLaunchKernelGGL(pack_partial_kernel, dim3(lanes, p.nQ, p.uB * p.uH), dim3(256), 0, stream, p);
+    return hipGetLastError();
+}
+
+// One workgroup reads a Q tile's whole slab of the mask, so the slab must be small, or there must be many of them.  us for
+// lists and packed tiles, three launches | one (launches back to back in a graph):
+//   slab 2 KiB x 4 workgroups (decode, four lengths)  6.2 | 4.0    32 KiB x 8 (Sk 32768)      7.4 | 5.4
+//   128 KiB x 8 (causal S1024)                        9.4 | 5.7    128 KiB x 8, all PARTIAL  12.1 | 9.6
+//   512 KiB x 128 (causal S8192)                     19.0 | 13.5   512 KiB x 256, all PARTIAL 97 | 51
+//   256 KiB x 64, all PARTIAL                        17.7 | 15.9   256 KiB x 512, all PARTIAL 76 | 42
+// and beyond the rule 256 KiB x 16 causal 9.8 | 6.9 but all PARTIAL 12.5 | 15.6, 2 MiB x 4 10.3 | 23.5.
+bool classify_rows_has(const ClassifyParams &p) {
+    const int64_t slab = (int64_t)p.BQ * p.Sk, workgroups = (int64_t)p.nQ * p.uB * p.uH;
+    return p.nK <= kRowsTiles && slab <= 512 * 1024 && (slab <= 128 * 1024 || slab <= workgroups * 8192);
+}
+
+hipError_t launch_classify_rows(const ClassifyRowsParams &p, hipStream_t stream) {
+    hipLaunchKernelGGL(classify_rows_kernel, dim3(p.c.nQ, p.c.uB * p.c.uH), dim3(kRowsThreads), 0, stream, p);
     return hipGetLastError();
 }
 

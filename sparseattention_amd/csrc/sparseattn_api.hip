@@ -37,13 +37,15 @@ int check_tiling(int B, int H, int Sq, int Sk, int BQ, int BK) {
     return SA_OK;
 }
 
-// The two launches of the classification (class bytes, then compaction into the lists), after the argument checks
-// the entry points share.  `workspace` holds one class byte per tile of every distinct plane; the caller has checked
+// The launches of the classification (class bytes, then compaction into the lists; or one that does both, and packs the
+// PARTIAL tiles into `packed` too, which it says in *packed_done), after the argument checks the entry points share.
+// `workspace` holds one class byte per tile of every distinct plane; the caller has checked
 // its size.  `who` names the entry point in error messages.
 int classify_impl(const char *who, const uint8_t *mask, const int64_t mask_strides[4], int B, int H, int Sq, int Sk,
                   int BQ, int BK, int32_t *full_ids, const int64_t full_ids_strides[4], int32_t *full_lens,
                   const int64_t full_lens_strides[3], int32_t *part_ids, const int64_t part_ids_strides[4],
-                  int32_t *part_lens, const int64_t part_lens_strides[3], void *workspace, void *stream) {
+                  int32_t *part_lens, const int64_t part_lens_strides[3], void *workspace, void *stream,
+                  uint8_t *packed = nullptr, const int64_t *packed_strides = nullptr, bool *packed_done = nullptr) {
     const int nQ = Sq / BQ, nK = Sk / BK;
     const bool bcast_b = mask_strides[0] == 0 || B == 1;
     const bool bcast_h = mask_strides[1] == 0 || H == 1;
@@ -82,9 +84,6 @@ int classify_impl(const char *who, const uint8_t *mask, const int64_t mask_strid
     // Wide kernel: 16-byte loads along a contiguous, aligned key dimension; a tile spans 1..64 lanes.
     const bool wide = cp.lbk >= 4 && BK <= 1024 && (cp.sk == 1 || Sk == 1) && aligned(mask, 16) && cp.sq % 16 == 0 &&
                       (cp.uB == 1 || cp.sb % 16 == 0) && (cp.uH == 1 || cp.sh % 16 == 0);
-    hipError_t e = sa::launch_classify(cp, wide, static_cast<hipStream_t>(stream));
-    if (e != hipSuccess) return fail(SA_ERR_HIP, "%s: classify launch failed: %s", who, hipGetErrorString(e));
-
     sa::CompactParams kp{};
     kp.cls = cp.cls;
     kp.uH = cp.uH;
@@ -106,6 +105,23 @@ int classify_impl(const char *who, const uint8_t *mask, const int64_t mask_strid
         kp.fls[i] = full_lens_strides[i];
         kp.pls[i] = part_lens_strides[i];
     }
+    hipError_t e;
+    if (wide && sa::classify_rows_has(cp)) {
+        sa::ClassifyRowsParams rp{};
+        rp.c = cp;
+        rp.l = kp;
+        if (packed && aligned(packed, 2) && (cp.uB == 1 || packed_strides[0] % 2 == 0) && (cp.uH == 1 || packed_strides[1] % 2 == 0)) {
+            rp.packed = packed;
+            rp.ob = packed_strides[0];
+            rp.oh = packed_strides[1];
+            *packed_done = true;
+        }
+        e = sa::launch_classify_rows(rp, static_cast<hipStream_t>(stream));
+        if (e != hipSuccess) return fail(SA_ERR_HIP, "%s: classify launch failed: %s", who, hipGetErrorString(e));
+        return SA_OK;
+    }
+    e = sa::launch_classify(cp, wide, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(SA_ERR_HIP, "%s: classify launch failed: %s", who, hipGetErrorString(e));
     e = sa::launch_compact(kp, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail(SA_ERR_HIP, "%s: compaction launch failed: %s", who, hipGetErrorString(e));
     return SA_OK;
@@ -648,10 +664,48 @@ int sa_fwd_schedule(const int32_t *full_lens, const int64_t full_lens_strides[3]
     return SA_OK;
 }
 
+// What the two entry points that pack check of their output.
+static int check_pack(const char *who, const int64_t mask_strides[4], int B, int H, int Sq, int Sk, int BQ, int BK, const int64_t packed_strides[2]) {
+    if (BK % 8) return fail(SA_ERR_UNSUPPORTED, "%s: BLOCK_K %d (must be a multiple of 8)", who, BK);
+    const Planes pl = planes_of(mask_strides, B, H);
+    const int64_t plane_bytes = (int64_t)Sq * Sk / 8;
+    if ((pl.uB > 1 && packed_strides[0] < plane_bytes) || (pl.uH > 1 && packed_strides[1] < plane_bytes))
+        return fail(SA_ERR_INVALID_ARGUMENT, "%s: packed planes overlap (strides %lld, %lld; %lld bytes per plane)", who,
+                    (long long)packed_strides[0], (long long)packed_strides[1], (long long)plane_bytes);
+    if (Sq / BQ > 65535 || (int64_t)pl.uB * pl.uH > 65535)
+        return fail(SA_ERR_UNSUPPORTED, "%s: more than 65535 Q tiles or distinct mask planes", who);
+    return SA_OK;
+}
+
 size_t sa_mask_pack_partial_bytes(const int64_t mask_strides[4], int B, int H, int Sq, int Sk, int BQ, int BK) {
     if (!mask_strides || check_tiling(B, H, Sq, Sk, BQ, BK) != SA_OK || BK % 8) return 0;
     const Planes pl = planes_of(mask_strides, B, H);
     return (size_t)pl.uB * pl.uH * (size_t)Sq * (size_t)Sk / 8;
+}
+
+int sa_mask_classify_packed(const uint8_t *mask, const int64_t mask_strides[4], int B, int H, int Sq, int Sk, int BQ,
+                            int BK, int32_t *full_ids, const int64_t full_ids_strides[4], int32_t *full_lens,
+                            const int64_t full_lens_strides[3], int32_t *part_ids, const int64_t part_ids_strides[4],
+                            int32_t *part_lens, const int64_t part_lens_strides[3], uint8_t *packed,
+                            const int64_t packed_strides[2], void *workspace, size_t workspace_bytes, void *stream) {
+    g_error[0] = 0;
+    if (!mask || !mask_strides || !full_ids || !full_ids_strides || !full_lens || !full_lens_strides || !part_ids ||
+        !part_ids_strides || !part_lens || !part_lens_strides || !packed || !packed_strides)
+        return fail(SA_ERR_INVALID_ARGUMENT, "sa_mask_classify_packed: null pointer argument");
+    if (const int rc = check_tiling(B, H, Sq, Sk, BQ, BK)) return rc;
+    if (const int rc = check_pack("sa_mask_classify_packed", mask_strides, B, H, Sq, Sk, BQ, BK, packed_strides)) return rc;
+    const size_t need = sa_mask_classify_workspace_bytes(mask_strides, B, H, Sq, Sk, BQ, BK);
+    if (!workspace || workspace_bytes < need)
+        return fail(SA_ERR_WORKSPACE, "sa_mask_classify_packed: workspace of %zu bytes required, %zu given", need,
+                    workspace ? workspace_bytes : (size_t)0);
+    bool done = false;
+    if (const int rc = classify_impl("sa_mask_classify_packed", mask, mask_strides, B, H, Sq, Sk, BQ, BK, full_ids, full_ids_strides,
+                                     full_lens, full_lens_strides, part_ids, part_ids_strides, part_lens, part_lens_strides,
+                                     workspace, stream, packed, packed_strides, &done))
+        return rc;
+    return done ? SA_OK
+                : sa_mask_pack_partial(mask, mask_strides, B, H, Sq, Sk, BQ, BK, part_ids, part_ids_strides, part_lens,
+                                       part_lens_strides, packed, packed_strides, stream);
 }
 
 int sa_mask_pack_partial(const uint8_t *mask, const int64_t mask_strides[4], int B, int H, int Sq, int Sk, int BQ,
@@ -663,15 +717,9 @@ int sa_mask_pack_partial(const uint8_t *mask, const int64_t mask_strides[4], int
         !packed_strides)
         return fail(SA_ERR_INVALID_ARGUMENT, "sa_mask_pack_partial: null pointer argument");
     if (const int rc = check_tiling(B, H, Sq, Sk, BQ, BK)) return rc;
-    if (BK % 8) return fail(SA_ERR_UNSUPPORTED, "sa_mask_pack_partial: BLOCK_K %d (must be a multiple of 8)", BK);
+    if (const int rc = check_pack("sa_mask_pack_partial", mask_strides, B, H, Sq, Sk, BQ, BK, packed_strides)) return rc;
     const Planes pl = planes_of(mask_strides, B, H);
-    const int64_t plane_bytes = (int64_t)Sq * Sk / 8;
-    if ((pl.uB > 1 && packed_strides[0] < plane_bytes) || (pl.uH > 1 && packed_strides[1] < plane_bytes))
-        return fail(SA_ERR_INVALID_ARGUMENT, "sa_mask_pack_partial: packed planes overlap (strides %lld, %lld; %lld bytes per plane)",
-                    (long long)packed_strides[0], (long long)packed_strides[1], (long long)plane_bytes);
     const int nQ = Sq / BQ, nK = Sk / BK;
-    if (nQ > 65535 || (int64_t)pl.uB * pl.uH > 65535)
-        return fail(SA_ERR_UNSUPPORTED, "sa_mask_pack_partial: more than 65535 Q tiles or distinct mask planes");
 
     sa::PackParams pp{};
     pp.mask = mask;
