@@ -26,6 +26,7 @@ namespace {
 [[noreturn]] void value_error(const std::string &m) { throw py::value_error(m); }
 [[noreturn]] void type_error(const std::string &m) { throw py::type_error(m); }
 [[noreturn]] void assertion(const char *m) {
+    const py::gil_scoped_acquire gil;
     PyErr_SetString(PyExc_AssertionError, m);
     throw py::error_already_set();
 }
@@ -561,16 +562,15 @@ py::object backward(const Tensor &do_, const Tensor &q, const Tensor &k, const T
 struct AttentionFunction : public torch::autograd::Function<AttentionFunction> {
     static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &mask, const Out &r,
                           const std::optional<BackwardLists> &lists) {
-        std::vector<at::Tensor> keep = {q, k, v, r.o, *r.lse, mask.value_or(Tensor())};
-        // (the lists are no outputs or inputs of the function: kept as they are, in the order backward() takes them)
-        std::vector<at::Tensor> l;
+        // (the lists are the program's own, kept as an attribute would be: hooks on saved tensors see what they always saw)
         if (lists) {
+            c10::List<OptTensor> l;
             for (const Lists *p : {&lists->by_query, &lists->by_key})
-                for (const Tensor &t : {p->fid, p->fl, p->pid, p->pl, p->packed.value_or(Tensor())}) l.push_back(t);
-            l.push_back(lists->transposed_mask.value_or(Tensor()));
+                for (const OptTensor &t : {OptTensor(p->fid), OptTensor(p->fl), OptTensor(p->pid), OptTensor(p->pl), p->packed}) l.push_back(t);
+            l.push_back(lists->transposed_mask);
+            ctx->saved_data["lists"] = std::move(l);
         }
-        for (const Tensor &t : l) keep.push_back(t);
-        ctx->save_for_backward(keep);
+        ctx->save_for_backward({q, k, v, r.o, *r.lse, mask.value_or(Tensor())});
         return r.o;
     }
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
@@ -578,10 +578,11 @@ struct AttentionFunction : public torch::autograd::Function<AttentionFunction> {
         const Tensor &q = s[0], &k = s[1];
         OptTensor mask;
         if (s[5].defined()) mask = s[5];
-        auto opt = [](const Tensor &t) -> OptTensor { return t.defined() ? OptTensor(t) : std::nullopt; };
         BackwardLists l;
-        if (s.size() > 6) {
-            l = {{s[6], s[7], s[8], s[9], opt(s[10])}, {s[11], s[12], s[13], s[14], opt(s[15])}, opt(s[16])};
+        if (const auto it = ctx->saved_data.find("lists"); it != ctx->saved_data.end()) {
+            const auto t = it->second.toOptionalTensorList();
+            const auto at_ = [&](size_t i) { return OptTensor(t.get(i)); };
+            l = {{*at_(0), *at_(1), *at_(2), *at_(3), at_(4)}, {*at_(5), *at_(6), *at_(7), *at_(8), at_(9)}, at_(10)};
         } else {
             l = backward_lists_from(*mask);
         }
