@@ -48,18 +48,18 @@ PEAK_FP32_TFLOPS = 157.3   # MI355X dense fp32 MFMA peak, TFLOP/s
 # `bench.py --traffic-probe` and scaled by what the same counters read for the 1 GiB device copy of the same run
 # (`bench.py --traffic-summary` does the arithmetic).  profiles/hbm_traffic_all_kernels.txt holds the commands.
 TRAFFIC_BYTES = {
-    "forward, causal": (850642198, 268435456),
-    "forward, dense": (807990383, 268435456),
-    "forward, p=0.25": (1342766238, 268435456),
-    "forward, p=0.5": (2866683417, 268435456),
-    "forward, p=0.75": (2937911497, 268435456),
-    "forward, p=0.9": (1421786017, 268435456),
-    "backward, causal": (8302542627, 5242880085),
-    "forward, documents": (1773818346, 536870912),
-    "forward, composed": (1632119461, 268435456),
-    "mask_classify, composed mask 1 GiB": (1074097997, 308736),
-    "decode, 1": (4295535603, 344064),
-    "decode, 16": (1617161242, 5308725),
+    "forward, causal": (853735343, 268435456),
+    "forward, dense": (807993712, 268435541),
+    "forward, p=0.25": (1353390346, 268435456),
+    "forward, p=0.5": (2851538520, 268435456),
+    "forward, p=0.75": (2937622647, 268435456),
+    "forward, p=0.9": (1419725872, 268435456),
+    "backward, causal": (8111131484, 5242880000),
+    "forward, documents": (1725168346, 536870912),
+    "forward, composed": (1614240091, 268435456),
+    "mask_classify, composed mask 1 GiB": (1074098168, 308736),
+    "decode, 1": (4295523657, 344064),
+    "decode, 16": (1617161712, 5308416),
 }
 TRAFFIC_SOURCE = "profiles/hbm_traffic_all_kernels.txt"
 # The sources each kernel is built from.  The counters were read with kernels built from sources of the digests in
@@ -71,8 +71,8 @@ KERNEL_FILES = {
     "decode": ("sparse_decode.hip", "fwd_common.h", "kernels.h"),
     "backward": ("sparse_bwd.hip", "fwd_common.h", "kernels.h"),
 }
-TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "3e69e41a4e196f13", "mask_classify": "f01d28ab108dfb99", "decode": "b9a665fe6b1983dc",
-                                "backward": "c1e3e4678de61b29"}
+TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "94c7ca3577a858fc", "mask_classify": "ae1679520463a44b", "decode": "b496d7a3ade7b9fa",
+                                "backward": "560c0c46d711d9f9"}
 
 
 def kernel_sources_sha16(which=None):

@@ -439,6 +439,19 @@ int sa_sparse_attention_decode_ex(const void *q, const int64_t q_strides[4], con
                                   const int64_t lse_strides[3], void *stream);
 
 /*
+ * sa_sparse_attention_decode for a mask that is new at every call: no lists.  Every workgroup reads the mask of its (b, h) and
+ * makes its lists, which costs less than a launch for them; results are bit-identical.  For the masks that
+ * sa_decode_mask_fits says 1 of (else SA_ERR_UNSUPPORTED): Sq <= 32, BK a power of two from 32 to 256, Sq * Sk <= 32768,
+ * contiguous rows, base and strides multiples of 16 bytes.  num_splits and the workspace as above.
+ */
+int sa_decode_mask_fits(const uint8_t *mask, const int64_t mask_strides[4], int B, int H, int Sq, int Sk, int BK);
+int sa_sparse_attention_decode_mask(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
+                                    const void *v, const int64_t v_strides[4], void *o, const int64_t o_strides[4],
+                                    const uint8_t *mask, const int64_t mask_strides[4], int B, int H, int Sq, int Sk, int D,
+                                    int BK, int dtype, float sm_scale_log2, int num_splits, void *workspace, size_t workspace_bytes,
+                                    float *lse, const int64_t lse_strides[3], void *stream);
+
+/*
  * Merge of n attention results over disjoint key ranges of the same queries (what sharding the key axis over
  * devices, or over launches, ends with; the reference has no counterpart - it never hands out the row statistics):
  *   o = sum_i exp(lse_i - lse) o_i,   lse = log sum_i exp(lse_i)     (rows with every lse_i = -inf give 0 and -inf)

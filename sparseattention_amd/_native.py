@@ -52,6 +52,8 @@ EXPORTS = (
     "sa_decode_workspace_bytes",
     "sa_sparse_attention_decode",
     "sa_sparse_attention_decode_ex",
+    "sa_decode_mask_fits",
+    "sa_sparse_attention_decode_mask",
     "sa_merge_attention_parts",
     "sa_bwd_workspace_bytes",
     "sa_bwd_workspace_bytes_ex",
@@ -153,6 +155,12 @@ def load() -> ctypes.CDLL:
     lib.sa_sparse_attention_decode_ex.argtypes = (
         [_vp, _i64p] * 4 + [_vp, _i64p] + [_vp, _i64p] * 4 + [_vp, _i64p] + [ctypes.c_int] * 7 + [ctypes.c_float, ctypes.c_int]
         + [_vp, ctypes.c_size_t] + [_vp, _i64p] + [_vp]
+    )
+    lib.sa_decode_mask_fits.restype = ctypes.c_int
+    lib.sa_decode_mask_fits.argtypes = [_vp, _i64p] + [ctypes.c_int] * 5
+    lib.sa_sparse_attention_decode_mask.restype = ctypes.c_int
+    lib.sa_sparse_attention_decode_mask.argtypes = (
+        [_vp, _i64p] * 5 + [ctypes.c_int] * 7 + [ctypes.c_float, ctypes.c_int] + [_vp, ctypes.c_size_t] + [_vp, _i64p] + [_vp]
     )
     lib.sa_merge_attention_parts.restype = ctypes.c_int
     lib.sa_merge_attention_parts.argtypes = [_vp, _i64p] * 4 + [ctypes.c_int] * 6 + [_vp]

@@ -260,10 +260,13 @@ Out decode_impl(const Tensor &q, const Tensor &k, const Tensor &v, const OptTens
     OptTensor mask = mask_in;
     if (mask) mask = mask->expand({B, H, Sq, Sk});
     Lists l;
-    if (md.is_none()) {
+    // (a small mask without lists: the decode kernel finds its tiles in it; what the classification refuses goes there)
+    const bool direct = md.is_none() && mask && mask->scalar_type() == at::kBool && BK > 0 && BK <= Sk &&
+                        sa_decode_mask_fits(ptr<uint8_t>(*mask), st(*mask), B, H, Sq, Sk, BK);
+    if (md.is_none() && !direct) {
         if (!mask) value_error("sparse_attention_decode needs the mask or mask_metadata with packed_masks");
         l = classify_lists(*mask, Sq, BK, std::nullopt);
-    } else {
+    } else if (!direct) {
         l = lists_of(md);
         if (BK <= 0) value_error("BLOCK_K must be positive");
         check_lists(l, q, B, H, 1, Sk / BK, "mask_metadata");
@@ -287,6 +290,12 @@ Out decode_impl(const Tensor &q, const Tensor &k, const Tensor &v, const OptTens
     if (ws_bytes) ws = at::empty({(int64_t)(ws_bytes / 4)}, f32);
     OptTensor lse;
     if (return_lse) lse = at::empty({B, H, Sq}, f32);
+    if (direct) {
+        check_rc(sa_sparse_attention_decode_mask(qc.data_ptr(), st(qc), kc.data_ptr(), st(kc), vc.data_ptr(), st(vc), o.data_ptr(), st(o),
+                                                 ptr<uint8_t>(*mask), st(*mask), B, H, Sq, Sk, Dk, BK, dt, (float)scale_log2(D), num_splits,
+                                                 ws_bytes ? ws.data_ptr() : nullptr, ws_bytes, ptr<float>(lse), st(lse), stream_of(q)));
+        return {cut_head_dim(o, D), lse};
+    }
     check_rc(sa_sparse_attention_decode_ex(qc.data_ptr(), st(qc), kc.data_ptr(), st(kc), vc.data_ptr(), st(vc), o.data_ptr(), st(o), ptr<uint8_t>(mask),
                                            st(mask), ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl), ptr<int32_t>(l.pid), st(l.pid),
                                            ptr<int32_t>(l.pl), st(l.pl), ptr<uint8_t>(l.packed), st(l.packed), B, H, Sq, Sk, Dk, BK, dt,

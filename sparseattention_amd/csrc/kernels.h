@@ -186,11 +186,15 @@ hipError_t launch_fwd_f32_mfma(const FwdParams &p, int D, int BQ, hipStream_t st
 
 // Few query rows against a long K/V (decode): one Q tile of Sq <= 32 rows per (b, h), its list of KV tiles split
 // over `nsplit` workgroups whose partial results a second kernel merges.
+// The most entries a plane's mask may have for a decode without lists, and the widest tiles: bits and lists lie in LDS, every
+// workgroup of the plane reads the whole mask, and a lane goes over a tile.
+constexpr int kDecodeDirectEntries = 32768;
+constexpr int kDecodeDirectBK = 256;
 struct DecodeParams {
     const uint16_t *q, *k, *v;
     uint16_t *o;
     const uint8_t *mask;
-    const int32_t *full_ids, *full_lens, *part_ids, *part_lens;
+    const int32_t *full_ids, *full_lens, *part_ids, *part_lens;  // all null: the tiles are found in the mask
     int64_t qs[3], ks[3], vs[3], os[3];  // b, h, s strides in elements (d stride is 1)
     int64_t ms[4];                        // mask strides in bytes
     int64_t fis[3], fls[2], pis[3], pls[2];  // b, h (and entry) strides of the lists of the one Q tile

@@ -50,10 +50,27 @@ __device__ __forceinline__ void merge_parts(const float *part, int n, int64_t st
     }
 }
 
+// DM: the workgroup's own lists, behind the V stages: a bit per mask entry, then FULL and PARTIAL tiles (16 bit each).
+constexpr int kDirectBits = kDecodeDirectEntries / 8;
+constexpr int kDirectList = kDecodeDirectEntries / 32;  // entries of one list at most
+constexpr int kDirectBytes = kDirectBits + 2 * 2 * kDirectList;
+
+// The byte of a bool mask as a bit: bits 0..3 for the four bytes of w (any non-zero byte attends).
+__device__ __forceinline__ uint32_t bits_of4(uint32_t w) {
+    w |= w >> 4;
+    w |= w >> 2;
+    w |= w >> 1;
+    return ((w & 0x01010101u) * 0x01020408u >> 24) & 15u;
+}
+
 // PK: the mask entries of PARTIAL tiles come bit-packed from p.packed (sa_mask_pack_partial with BQ = Sq) instead of from
 // the bool mask.  B16: BLOCK_K = 16, two list entries per chunk of 32 keys (else BLOCK_K >= 32, BLOCK_K/32 chunks per
-// entry).
-template <int DT, int D, bool PK, bool B16>
+// entry).  DM: no lists given; every workgroup reads the plane's mask (at most kDecodeDirectEntries bytes, mostly from a
+// cache) and makes the lists that the classification would have made in LDS, in the same order: results are bit-identical.
+// One launch instead of two where both are mostly latency, and three allocations less: with the lists made first / here, bf16,
+// D = 128, three quarters of the keys attended: B4 H32 Sq1 Sk2048 28.0 / 24.1 us, B1 H8 Sq1 Sk512 12.5 / 10.3, at the bound
+// B8 H32 Sq1 Sk32768 496 / 477, B8 H16 Sq32 Sk1024 26.3 / 25.1; nowhere slower than the runs differ.
+template <int DT, int D, bool PK, bool B16, bool DM>
 __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(const DecodeParams p) {
     using E = Elem<DT>;
     constexpr int ROWB = D * 2;
@@ -71,14 +88,58 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
 
     const uint16_t *kbase = p.k + b * p.ks[0] + h * p.ks[1];
     const uint16_t *vbase = p.v + b * p.vs[0] + h * p.vs[1];
-    const int32_t *fid = p.full_ids + b * p.fis[0] + h * p.fis[1];
-    const int32_t *pid = p.part_ids + b * p.pis[0] + h * p.pis[1];
+    const int32_t *fid = DM ? nullptr : p.full_ids + b * p.fis[0] + h * p.fis[1];
+    const int32_t *pid = DM ? nullptr : p.part_ids + b * p.pis[0] + h * p.pis[1];
     // Counts and tile indices are clamped to what Sk holds (the reference guards every K/V and mask load with
     // kv_offset < SEQLEN_K, sparse_attn_kernel.py:35,39,60): stale or foreign metadata then gives wrong numbers, never
     // an access outside K, V or the mask.
     const int nKt = p.Sk >> p.lbk;
-    const int F = min(max(p.full_lens[b * p.fls[0] + h * p.fls[1]], 0), nKt);
-    const int NE = F + min(max(p.part_lens[b * p.pls[0] + h * p.pls[1]], 0), nKt - F);
+    int F = DM ? 0 : min(max(p.full_lens[b * p.fls[0] + h * p.fls[1]], 0), nKt);
+    int NE = DM ? 0 : F + min(max(p.part_lens[b * p.pls[0] + h * p.pls[1]], 0), nKt - F);
+    const int nCh = p.Sk >> 5;  // (DM) chunks of a row
+    uint32_t *const bits = reinterpret_cast<uint32_t *>(smem + decode_smem_bytes<D>());  // (DM) [Sq][nCh]
+    uint16_t *const list = reinterpret_cast<uint16_t *>(smem + decode_smem_bytes<D>() + kDirectBits);  // FULL, then PARTIAL
+    if constexpr (DM) {
+        const uint8_t *m0 = p.mask + b * p.ms[0] + h * p.ms[1];
+        const int ppr = 2 * nCh, pieces = p.Sq * ppr;  // of 16 entries
+        for (int i0 = tid; i0 < pieces; i0 += 4 * 256) {
+            u32x4 x[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int i = min(i0 + 256 * j, pieces - 1), r = i / ppr;
+                x[j] = *(const u32x4 *)(m0 + r * p.ms[2] + 16 * (i - r * ppr));
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (i0 + 256 * j < pieces)
+                    reinterpret_cast<uint16_t *>(bits)[i0 + 256 * j] = (uint16_t)(bits_of4(x[j].x) | (bits_of4(x[j].y) << 4) |
+                                                                                  (bits_of4(x[j].z) << 8) | (bits_of4(x[j].w) << 12));
+        }
+        __syncthreads();
+        // a lane per tile; every wave counts, the first one writes
+        const int words = p.BK >> 5;  // of a row of a tile
+        int P = 0;
+        for (int c0 = 0; c0 < nKt; c0 += 64) {
+            const int c = c0 + lane;
+            uint32_t any = 0u, all = ~0u;
+            if (c < nKt)
+                for (int r = 0; r < p.Sq; r++)
+                    for (int w = 0; w < words; w++) {
+                        const uint32_t x = bits[r * nCh + c * words + w];
+                        any |= x;
+                        all &= x;
+                    }
+            const bool is_part = any != 0u && all != ~0u, is_full = any != 0u && !is_part;
+            const uint64_t full = __builtin_amdgcn_ballot_w64(is_full), part = __builtin_amdgcn_ballot_w64(is_part);
+            const uint64_t below = (1ull << lane) - 1ull;
+            if (wave == 0 && is_full) list[F + __popcll(full & below)] = (uint16_t)c;
+            if (wave == 0 && is_part) list[kDirectList + P + __popcll(part & below)] = (uint16_t)c;
+            F += __popcll(full);
+            P += __popcll(part);
+        }
+        NE = F + P;
+        __syncthreads();
+    }
     constexpr int EPC = B16 ? 2 : 1;   // list entries per chunk
     const int sh = B16 ? 0 : p.lbk - 5;  // chunks per list entry, log2
     const int T = B16 ? (NE + 1) >> 1 : NE << sh;
@@ -90,7 +151,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
     // query row of this lane (rows past Sq are padding: zero queries, row 0's mask, never stored)
     const bool live = l32 < p.Sq;
     const int qrow = live ? l32 : 0;
-    const uint8_t *mrow = PK ? nullptr : p.mask + b * p.ms[0] + h * p.ms[1] + (int64_t)qrow * p.ms[2];
+    const uint8_t *mrow = PK || DM ? nullptr : p.mask + b * p.ms[0] + h * p.ms[1] + (int64_t)qrow * p.ms[2];
     // this row's bits in the packed tile of a PARTIAL slot: BK/8 bytes per row, Sq rows per tile
     const int64_t tile_bytes = (int64_t)p.Sq * (p.BK >> 3);
     const uint8_t *prow = PK ? p.packed + b * p.pks[0] + h * p.pks[1] + (int64_t)qrow * (p.BK >> 3) : nullptr;
@@ -144,6 +205,11 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
 
     // list entries of chunk t (clamped into the row of tiles; an entry past the count reads as entry 0 and is masked out)
     auto idx_load = [&](int t, int(&idx)[EPC]) {
+        if constexpr (DM) {
+            const int e = t >> sh;
+            idx[0] = list[e < F ? e : kDirectList + e - F];
+            return;
+        }
 #pragma unroll
         for (int j = 0; j < EPC; j++) {
             const int e0 = B16 ? 2 * t + j : (t >> sh);
@@ -169,7 +235,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
         return f;
     };
     constexpr unsigned ALL = (1u << EPC) - 1u;
-    constexpr int NMW = PK ? EPC : 4;  // mask words per lane and chunk
+    constexpr int NMW = PK || DM ? EPC : 4;  // mask words per lane and chunk
     // everything chunk t needs from memory: K into registers, V into LDS stage `st`, mask words if it has a PARTIAL entry
     auto issue = [&](int t, const int(&col)[EPC], int st, u32x4(&kf)[NC], uint32_t(&mk)[NMW]) {
         const int kcol = B16 ? ((l32 < 16 ? col[0] : col[EPC - 1]) - (l32 & 16)) : col[0];  // (+ l32: this lane's key)
@@ -184,7 +250,9 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
         }
         const unsigned fl = flags_of(t);
         if (fl >> 4) {
-            if constexpr (PK) {
+            if constexpr (DM) {
+                mk[0] = bits[qrow * nCh + (col[0] >> 5)];
+            } else if constexpr (PK) {
 #pragma unroll
                 for (int j = 0; j < EPC; j++) {
                     const int e = B16 ? 2 * t + j : (t >> sh);
@@ -216,7 +284,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
         for (int c = 0; c < NC; c++) s = E::mfma(kf[c], qf[c], s);
         const unsigned fl = flags_of(t);
         if (fl != ALL) {  // a PARTIAL entry, or (BLOCK_K = 16) a second entry past the end of the list
-            if constexpr (PK) {
+            if constexpr (PK || DM) {
                 // bit k of w: key k of the chunk; FULL entries count as all ones, missing ones as zero
                 uint32_t w;
                 if constexpr (B16) {
@@ -433,10 +501,10 @@ __global__ __launch_bounds__(256) void merge_parts_kernel(const MergeParams p) {
         p.lse[b * p.lses[0] + h * p.lses[1] + (int64_t)q * p.lses[2]] = L > 0.f ? M + __logf(L) : kNegInf;
 }
 
-template <int DT, int D, bool PK, bool B16>
+template <int DT, int D, bool PK, bool B16, bool DM = false>
 hipError_t launch_decode_kind(const DecodeParams &p, hipStream_t stream) {
-    constexpr int smem = decode_smem_bytes<D>();
-    auto kern = sparse_decode_kernel<DT, D, PK, B16>;
+    constexpr int smem = decode_smem_bytes<D>() + (DM ? kDirectBytes : 0);
+    auto kern = sparse_decode_kernel<DT, D, PK, B16, DM>;
     static unsigned long long attr_done = 0;  // devices on which this kernel may use `smem` bytes of LDS
     if (const hipError_t e0 = allow_dynamic_smem(kern, smem, attr_done); e0 != hipSuccess) return e0;
     hipLaunchKernelGGL(kern, dim3(p.nsplit, p.B * p.H), dim3(kDecodeWaves * 64), smem, stream, p);
@@ -448,6 +516,7 @@ hipError_t launch_decode_kind(const DecodeParams &p, hipStream_t stream) {
 
 template <int DT, int D>
 hipError_t launch_decode_one(const DecodeParams &p, hipStream_t stream) {
+    if (p.full_ids == nullptr) return launch_decode_kind<DT, D, false, false, true>(p, stream);
     const bool pk = p.packed != nullptr, b16 = p.BK == 16;
     if (pk) return b16 ? launch_decode_kind<DT, D, true, true>(p, stream) : launch_decode_kind<DT, D, true, false>(p, stream);
     return b16 ? launch_decode_kind<DT, D, false, true>(p, stream) : launch_decode_kind<DT, D, false, false>(p, stream);

@@ -893,11 +893,13 @@ int decode_impl(const void *q, const int64_t q_strides[4], const void *k, const 
                 const int64_t part_ids_strides[4], const int32_t *part_lens, const int64_t part_lens_strides[3],
                 const uint8_t *packed, const int64_t packed_strides[2], int B, int H, int Sq, int Sk, int D, int BK,
                 int dtype, float sm_scale_log2, int num_splits, void *workspace, size_t workspace_bytes, float *lse,
-                const int64_t lse_strides[3], void *stream) {
+                const int64_t lse_strides[3], void *stream, bool direct = false) {
     g_error[0] = 0;
-    if (!q || !k || !v || !o || !q_strides || !k_strides || !v_strides || !o_strides ||
-        !full_ids || !full_ids_strides || !full_lens || !full_lens_strides || !part_ids || !part_ids_strides ||
-        !part_lens || !part_lens_strides)
+    // (direct: no lists at all, see sa_sparse_attention_decode_mask, which has looked at the mask)
+    if (!q || !k || !v || !o || !q_strides || !k_strides || !v_strides || !o_strides)
+        return fail(SA_ERR_INVALID_ARGUMENT, "sa_sparse_attention_decode: null pointer argument");
+    if (!direct && (!full_ids || !full_ids_strides || !full_lens || !full_lens_strides || !part_ids || !part_ids_strides ||
+        !part_lens || !part_lens_strides))
         return fail(SA_ERR_INVALID_ARGUMENT, "sa_sparse_attention_decode: null pointer argument");
     if (packed ? !packed_strides : (!mask || !mask_strides))
         return fail(SA_ERR_INVALID_ARGUMENT, "sa_sparse_attention_decode: null pointer argument (%s)", packed ? "packed_strides" : "mask");
@@ -958,16 +960,18 @@ int decode_impl(const void *q, const int64_t q_strides[4], const void *k, const 
     }
     for (int i = 0; i < 4; i++) dp.ms[i] = packed ? 0 : mask_strides[i];
     // the lists of the one Q tile: b and h strides, and the stride along the entries
-    dp.fis[0] = full_ids_strides[0];
-    dp.fis[1] = full_ids_strides[1];
-    dp.fis[2] = full_ids_strides[3];
-    dp.pis[0] = part_ids_strides[0];
-    dp.pis[1] = part_ids_strides[1];
-    dp.pis[2] = part_ids_strides[3];
-    dp.fls[0] = full_lens_strides[0];
-    dp.fls[1] = full_lens_strides[1];
-    dp.pls[0] = part_lens_strides[0];
-    dp.pls[1] = part_lens_strides[1];
+    if (!direct) {
+        dp.fis[0] = full_ids_strides[0];
+        dp.fis[1] = full_ids_strides[1];
+        dp.fis[2] = full_ids_strides[3];
+        dp.pis[0] = part_ids_strides[0];
+        dp.pis[1] = part_ids_strides[1];
+        dp.pis[2] = part_ids_strides[3];
+        dp.fls[0] = full_lens_strides[0];
+        dp.fls[1] = full_lens_strides[1];
+        dp.pls[0] = part_lens_strides[0];
+        dp.pls[1] = part_lens_strides[1];
+    }
     dp.B = B;
     dp.H = H;
     dp.Sq = Sq;
@@ -1026,6 +1030,31 @@ int sa_sparse_attention_decode_ex(const void *q, const int64_t q_strides[4], con
                        full_ids_strides, full_lens, full_lens_strides, part_ids, part_ids_strides, part_lens,
                        part_lens_strides, packed, packed_strides, B, H, Sq, Sk, D, BK, dtype, sm_scale_log2, num_splits,
                        workspace, workspace_bytes, lse, lse_strides, stream);
+}
+
+int sa_decode_mask_fits(const uint8_t *mask, const int64_t mask_strides[4], int B, int H, int Sq, int Sk, int BK) {
+    if (!mask || !mask_strides || B <= 0 || H <= 0 || Sq <= 0 || Sq > 32 || Sk <= 0) return 0;
+    if (BK < 32 || BK > sa::kDecodeDirectBK || log2_exact(BK) < 0 || Sk % BK) return 0;
+    if ((int64_t)Sq * Sk > sa::kDecodeDirectEntries || mask_strides[3] != 1 || !aligned(mask, 16)) return 0;
+    const int n[3] = {B, H, Sq};
+    for (int i = 0; i < 3; i++)
+        if (n[i] > 1 && mask_strides[i] % 16) return 0;
+    return 1;
+}
+
+int sa_sparse_attention_decode_mask(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
+                                    const void *v, const int64_t v_strides[4], void *o, const int64_t o_strides[4],
+                                    const uint8_t *mask, const int64_t mask_strides[4], int B, int H, int Sq, int Sk, int D,
+                                    int BK, int dtype, float sm_scale_log2, int num_splits, void *workspace, size_t workspace_bytes,
+                                    float *lse, const int64_t lse_strides[3], void *stream) {
+    g_error[0] = 0;
+    if (!sa_decode_mask_fits(mask, mask_strides, B, H, Sq, Sk, BK))
+        return fail(SA_ERR_UNSUPPORTED,
+                    "sa_sparse_attention_decode_mask: needs BLOCK_K 32..%d, at most %d mask entries per (b, h), contiguous mask rows, and a base and strides that are multiples of 16 bytes",
+                    sa::kDecodeDirectBK, sa::kDecodeDirectEntries);
+    return decode_impl(q, q_strides, k, k_strides, v, v_strides, o, o_strides, mask, mask_strides, nullptr, nullptr, nullptr,
+                       nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, B, H, Sq, Sk, D, BK, dtype, sm_scale_log2,
+                       num_splits, workspace, workspace_bytes, lse, lse_strides, stream, true);
 }
 
 size_t sa_bwd_workspace_bytes(int B, int H, int Sq) {
