@@ -48,18 +48,18 @@ PEAK_FP32_TFLOPS = 157.3   # MI355X dense fp32 MFMA peak, TFLOP/s
 # `bench.py --traffic-probe` and scaled by what the same counters read for the 1 GiB device copy of the same run
 # (`bench.py --traffic-summary` does the arithmetic).  profiles/hbm_traffic_all_kernels.txt holds the commands.
 TRAFFIC_BYTES = {
-    "forward, causal": (853735343, 268435456),
-    "forward, dense": (807993712, 268435541),
-    "forward, p=0.25": (1353390346, 268435456),
-    "forward, p=0.5": (2851538520, 268435456),
-    "forward, p=0.75": (2937622647, 268435456),
-    "forward, p=0.9": (1419725872, 268435456),
-    "backward, causal": (8111131484, 5242880000),
-    "forward, documents": (1725168346, 536870912),
-    "forward, composed": (1614240091, 268435456),
-    "mask_classify, composed mask 1 GiB": (1074098168, 308736),
-    "decode, 1": (4295523657, 344064),
-    "decode, 16": (1617161712, 5308416),
+    "forward, causal": (854423687, 268435456),
+    "forward, dense": (808001455, 268435797),
+    "forward, p=0.25": (1347283834, 268435456),
+    "forward, p=0.5": (2861761172, 268435456),
+    "forward, p=0.75": (2934045149, 268435456),
+    "forward, p=0.9": (1414350219, 268435456),
+    "backward, causal": (8130115082, 5242880213),
+    "forward, documents": (1723502198, 536870912),
+    "forward, composed": (1613264454, 268440320),
+    "mask_classify, composed mask 1 GiB": (1074098083, 308736),
+    "decode, 1": (4295523998, 344064),
+    "decode, 16": (1617158640, 5308587),
 }
 TRAFFIC_SOURCE = "profiles/hbm_traffic_all_kernels.txt"
 # The sources each kernel is built from.  The counters were read with kernels built from sources of the digests in
@@ -71,7 +71,7 @@ KERNEL_FILES = {
     "decode": ("sparse_decode.hip", "fwd_common.h", "kernels.h"),
     "backward": ("sparse_bwd.hip", "fwd_common.h", "kernels.h"),
 }
-TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "94c7ca3577a858fc", "mask_classify": "ae1679520463a44b", "decode": "b496d7a3ade7b9fa",
+TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "94c7ca3577a858fc", "mask_classify": "ae1679520463a44b", "decode": "9ae1240b96559893",
                                 "backward": "560c0c46d711d9f9"}
 
 

@@ -454,6 +454,77 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(const DecodeParams p)
     for (int j = 0; j < NV; j += 2) *(uint32_t *)(orow + j) = E::pack2(out[j] * inv, out[j + 1] * inv);
 }
 
+// The same for more than kMergeFew parts: one wave per query row, four per workgroup.  Eight lanes share a part (two
+// neighbouring floats of every 16 each, so a part is read in runs of 64 bytes), eight parts go side by side and kMergeBatch
+// reads of each are in flight.  The parts lie in a cache and are few: all of this is latency, and the kernel above, which
+// walks them one after the other, took most of a call with many (bf16, D = 128, Sq1; classification, decode and merge):
+// 128 parts (B1 H4 Sk32768) 76.9 -> 19.5 us, 22 parts (B2 H12 Sq4 Sk8192) 40.6 -> 31.1, 16 parts (B1 H32 Sk32768) 78.7 -> 72.5.
+// With 2 ... 4 parts the exchanges between lanes cost more than they save: 2 parts (B1 H8 Sk512) 12.5 -> 14.4, 4 parts (B8 H16
+// Sq32 Sk1024) 26.3 -> 29.6.
+constexpr int kMergeFew = 8;
+constexpr int kMergeBatch = 4;
+template <int DT, int D>
+__global__ __launch_bounds__(256) void decode_merge_many_kernel(const DecodeParams p) {
+    using E = Elem<DT>;
+    constexpr int NP = D / 16, PST = D + 2;
+    const int lane = threadIdx.x & 63, l8 = lane & 7, grp = lane >> 3;
+    const int64_t row = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (row >= (int64_t)p.B * p.H * p.Sq) return;
+    const int bh = (int)(row / p.Sq), q = (int)(row - (int64_t)bh * p.Sq);
+    const int b = bh / p.H, h = bh - b * p.H;
+    const int64_t stride = (int64_t)p.Sq * PST;
+    const float *const part = p.ws + ((int64_t)bh * p.nsplit * p.Sq + q) * PST;
+    float M = kNegInf;
+    for (int i = lane; i < p.nsplit; i += 64) M = fmaxf(M, part[i * stride + D]);
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) M = fmaxf(M, __shfl_xor(M, s));
+    float L = 0.f;
+    f32x2 out[NP];
+#pragma unroll
+    for (int c = 0; c < NP; c++) out[c] = f32x2{0.f, 0.f};
+    if (M != kNegInf) {  // else no part saw an attended key
+        for (int i0 = grp; i0 < p.nsplit; i0 += 8 * kMergeBatch) {
+            f32x2 ml[kMergeBatch], x[kMergeBatch][NP];
+#pragma unroll
+            for (int i = 0; i < kMergeBatch; i++) {
+                // (past the last part: the last one again, with weight 0)
+                const float *pp = part + min(i0 + 8 * i, p.nsplit - 1) * stride;
+                ml[i] = *(const f32x2 *)(pp + D);
+#pragma unroll
+                for (int c = 0; c < NP; c++) x[i][c] = *(const f32x2 *)(pp + 16 * c + 2 * l8);
+            }
+#pragma unroll
+            for (int i = 0; i < kMergeBatch; i++) {
+                // 0 for parts without an attended key (m = -inf)
+                const float w = i0 + 8 * i < p.nsplit ? __builtin_amdgcn_exp2f(ml[i].x - M) : 0.f;
+                L += w * ml[i].y;
+#pragma unroll
+                for (int c = 0; c < NP; c++) {
+                    out[c].x += w * x[i][c].x;
+                    out[c].y += w * x[i][c].y;
+                }
+            }
+        }
+#pragma unroll
+        for (int s = 8; s < 64; s <<= 1) {
+            L += __shfl_xor(L, s);
+#pragma unroll
+            for (int c = 0; c < NP; c++) {
+                out[c].x += __shfl_xor(out[c].x, s);
+                out[c].y += __shfl_xor(out[c].y, s);
+            }
+        }
+    }
+    if (grp != 0) return;
+    const float inv = L > 0.f ? 1.f / L : 0.f;
+    if (p.lse != nullptr && l8 == 0)
+        p.lse[b * p.lses[0] + h * p.lses[1] + q * p.lses[2]] =
+            L > 0.f ? (M + __builtin_amdgcn_logf(L)) * 0.69314718056f : kNegInf;
+    uint16_t *orow = p.o + b * p.os[0] + h * p.os[1] + (int64_t)q * p.os[2] + 2 * l8;
+#pragma unroll
+    for (int c = 0; c < NP; c++) *(uint32_t *)(orow + 16 * c) = E::pack2(out[c].x * inv, out[c].y * inv);
+}
+
 // Merge of n attention results over disjoint key ranges: o = sum_i exp(lse_i - lse) o_i, lse = log sum_i exp(lse_i).
 // One thread per 8 output elements.
 template <int DT>
@@ -510,7 +581,9 @@ hipError_t launch_decode_kind(const DecodeParams &p, hipStream_t stream) {
     hipLaunchKernelGGL(kern, dim3(p.nsplit, p.B * p.H), dim3(kDecodeWaves * 64), smem, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || p.nsplit == 1) return e;
-    hipLaunchKernelGGL((decode_merge_kernel<DT, D>), dim3(p.B * p.H), dim3(256), 0, stream, p);
+    const unsigned rows = (unsigned)p.B * p.H * p.Sq;  // (at most 65535 planes of 32 rows)
+    if (p.nsplit > kMergeFew) hipLaunchKernelGGL((decode_merge_many_kernel<DT, D>), dim3((rows + 3) / 4), dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL((decode_merge_kernel<DT, D>), dim3(p.B * p.H), dim3(256), 0, stream, p);
     return hipGetLastError();
 }
 
