@@ -204,17 +204,15 @@ def time_launches(fn, steps, warmup):
 
 
 def forward_case(name, mask2d, q, k, v, steps, warmup, schedule=None, pack_partial=None, block_k=BK, block_q=BQ):
-    import torch
-    from sparseattention_amd import compute_mask_kernel, sparse_attention
+    from sparseattention_amd import _native, compute_mask_kernel, sparse_attention
 
     B, H, S, D = q.shape
     BQ = block_q
     me = mask2d[None, None].expand(B, H, S, S)
     md = compute_mask_kernel(me, BQ, block_k, pack_partial=pack_partial, schedule=schedule, list_stats=True)
-    from sparseattention_amd.sparse_attn_kernel import _short_list_kernel
-    kernel = ("sparse_fwd_c32_kernel" if _short_list_kernel(md, q.dtype, D, BQ, block_k, None)
-              else "sparse_fwd_kernel" + (" (FULL entries walked from a start that depends on the Q tile)"
-                                          if md.list_rotation and schedule is None else ""))
+    which = _native.host().forward_kernel(q, BQ, block_k, md, "auto")
+    kernel = {"short": "sparse_fwd_c32_kernel", "default": "sparse_fwd_kernel",
+              "rotated": "sparse_fwd_kernel (FULL entries walked from a start that depends on the Q tile)"}[which]
     tiles_plane = int(md.unmasked_lens[0, 0].sum()) + int(md.masked_lens[0, 0].sum())
     partial_plane = int(md.masked_lens[0, 0].sum())
     # mean of the mask in row slabs (a [32768,32768] float copy would take 4 GiB)
@@ -319,9 +317,11 @@ def classify_small_case(steps, warmup):
 def backward_case(q, k, v, steps, warmup):
     """dq, dk, dv of the headline workload (causal, B8 H32 S4096 D128 bf16); the backward tiles the mask 128 x 64
     both ways.  Algorithmic work per executed tile: the five products of the derivative (S, dP, dQ, dK, dV) of
-    2*128*64*128 flop each; the three passes of the kernel recompute S twice and dP once, eight products in all."""
+    2*128*64*128 flop each.  Where dS goes through memory (sa_bwd_workspace_bytes_ex) those five are what is executed: S, dP,
+    dK and dV by the pass over the keys, dQ by the one over the queries; else three passes in one launch recompute S
+    twice and dP once, eight products in all."""
     import torch
-    from sparseattention_amd import (compute_backward_metadata, compute_mask_kernel, sparse_attention,
+    from sparseattention_amd import (_native, compute_backward_metadata, compute_mask_kernel, sparse_attention,
                                      sparse_attention_backward, workloads as W)
 
     me = W.causal_mask(S, "cuda")[None, None].expand(B, H, S, S)
@@ -334,7 +334,9 @@ def backward_case(q, k, v, steps, warmup):
     tk = int(bmd.by_key.unmasked_lens[0, 0].sum()) + int(bmd.by_key.masked_lens[0, 0].sum())
     per_product = 2 * 128 * 64 * D
     algorithmic = (3 * tq + 2 * tk) * per_product * B * H  # S, dP, dQ once per query-side tile; dK, dV per key-side tile
-    executed = (3 * tq + 5 * tk) * per_product * B * H
+    lib = _native.load()
+    stored = lib.sa_bwd_workspace_bytes_ex(B, H, S, S, D) > lib.sa_bwd_workspace_bytes(B, H, S)
+    executed = ((tq + 4 * tk) if stored else (3 * tq + 5 * tk)) * per_product * B * H
     achieved = algorithmic / (ev_ms * 1e-3) / 1e12
     return {
         "workload": "dq, dk, dv of configs[1] (causal, B=8 H=32 S=4096 D=128 bf16), tiles 128x64 of the mask and of "
@@ -344,7 +346,9 @@ def backward_case(q, k, v, steps, warmup):
         "executed_tflops": round(executed / (ev_ms * 1e-3) / 1e12, 1),
         "roofline": {"bound": "mfma", "achieved": round(achieved, 1), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(achieved / PEAK_BF16_TFLOPS, 4), **traffic_of("backward, causal", "backward"),
-                     "kernel": "sparse_bwd_kernel x3 (+ bwd_prepare_kernel)", "flop_per_launch": algorithmic},
+                     "kernel": ("sparse_bwd_keys_kernel, sparse_bwd_queries_kernel" if stored else "sparse_bwd_kernel")
+                               + " (+ bwd_prepare_kernel)",
+                     "flop_per_launch": algorithmic},
     }
 
 

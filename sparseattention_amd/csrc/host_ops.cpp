@@ -325,6 +325,54 @@ bool tiles_as_asked(int64_t Sq, int64_t Sk, int64_t D, int64_t BQ, int64_t BK, b
 // 2100 keys and more +5 ... +8 %: the third workgroup per compute unit pays for itself on the shortest lists only.
 constexpr double kShortListKeys = 512;
 
+// What a metadata object says besides its lists.
+struct Hints {
+    OptTensor sched;
+    int sched_mode = 0;
+    bool stats = false;  // list_stats: mean and longest number of listed tiles per Q tile
+    double mean_list = 0;
+    int64_t longest_list = 0, rotation = 0;
+};
+Hints hints_of(py::handle md) {
+    Hints h;
+    h.sched = opt_tensor_attr(md, "schedule");
+    if (h.sched)
+        if (const py::object m = attr(md, "schedule_mode")) h.sched_mode = m.cast<int>();
+    if (const py::object s = attr(md, "list_stats")) {
+        h.stats = true;
+        h.mean_list = s[py::int_(0)].cast<double>();
+        h.longest_list = s[py::int_(1)].cast<int64_t>();
+    }
+    if (const py::object r = attr(md, "list_rotation")) h.rotation = r.cast<int64_t>();
+    return h;
+}
+
+// Which of the forward kernels a call runs, as a code of the C ABI.
+int choose_kernel(const std::string &kernel, bool f32, int64_t Dk, int64_t BQ, int64_t BK, bool packed, const Hints &h) {
+    if (kernel != "auto" && kernel != "default" && kernel != "short" && kernel != "rotated")
+        value_error("kernel must be 'auto', 'default', 'rotated' or 'short' (got '" + kernel + "')");
+    if (kernel == "rotated" && (h.sched || f32)) value_error("kernel='rotated' needs bf16/fp16 and mask_metadata without a schedule");
+    const bool short_has = !f32 && Dk == 128 && BQ == 128 && pow2_from_16(BK) && packed && !h.sched;
+    const bool short_fits = h.stats && h.longest_list <= SA_FWD_SHORT_LISTS_MAX_ENTRIES;
+    if (kernel == "short") {
+        if (!(short_has && short_fits))
+            value_error("kernel='short' needs bf16/fp16, head dim 128, BLOCK_Q 128, mask_metadata with packed_masks, no schedule, and list_stats whose longest list has at most " +
+                        std::to_string(SA_FWD_SHORT_LISTS_MAX_ENTRIES) + " entries");
+        return SA_FWD_KERNEL_SHORT_LISTS;
+    }
+    if (kernel == "auto" && short_has && short_fits && h.mean_list * (double)BK < kShortListKeys) return SA_FWD_KERNEL_SHORT_LISTS;
+    // the default kernel with the FULL entries of Q tile qt walked from a start that depends on qt
+    if (!h.sched && !f32 && (kernel == "rotated" || (kernel == "auto" && h.rotation > 0)))
+        return SA_FWD_KERNEL_ROTATED | ((int)(h.rotation ? h.rotation : 16) << 8);
+    return SA_FWD_KERNEL_DEFAULT;
+}
+// The same by name ("default", "short" or "rotated"), for reports on what a call with this metadata runs.
+std::string forward_kernel(const Tensor &q, int64_t BQ, int64_t BK, py::object md, const std::string &kernel) {
+    const bool packed = (bool)attr(md, "packed_masks");
+    const int code = choose_kernel(kernel, q.scalar_type() == at::kFloat, kernel_head_dim(q.size(-1), true), BQ, BK, packed, hints_of(md)) & 0xff;
+    return code == SA_FWD_KERNEL_SHORT_LISTS ? "short" : code == SA_FWD_KERNEL_ROTATED ? "rotated" : "default";
+}
+
 // Whether tensors of these sizes run on a larger tile grid as they are (sa_sparse_attention_fwd_ragged): nothing is padded.
 bool ragged_has(const Tensor &q, int64_t BQ, int64_t BK, const Lists &l) {
     const int dt = dtype_code(q.scalar_type());
@@ -365,11 +413,7 @@ std::optional<Out> forward_impl(const Tensor &q, const Tensor &k, const Tensor &
 
     const int64_t nQ = Sq / BQ, nK = Sk / BK;
     Lists l;
-    OptTensor sched;
-    int sched_mode = 0;
-    double mean_list = 0;
-    int64_t longest_list = 0, rotation = 0;
-    bool stats = false;
+    Hints hints;
     if (!has_md) {
         l = classify_lists(*mask, BQ, BK, std::nullopt);
     } else {
@@ -377,40 +421,15 @@ std::optional<Out> forward_impl(const Tensor &q, const Tensor &k, const Tensor &
         check_lists(l, q, B, H, nQ, nK, "mask_metadata");
         checked_metadata(md, l, Sk, BK);
         if (l.packed) check_packed(*l.packed, q, B, H, nQ, nK, BQ * BK / 8, "mask_metadata");
-        sched = opt_tensor_attr(md, "schedule");
-        if (sched) {
-            if (sched->scalar_type() != at::kInt || sched->device() != q.device() || !sched->is_contiguous())
-                value_error("mask_metadata.schedule: expected a contiguous int32 tensor on q's device");
-            if (const py::object m = attr(md, "schedule_mode")) sched_mode = m.cast<int>();
-        }
-        if (const py::object s = attr(md, "list_stats")) {
-            stats = true;
-            mean_list = s[py::int_(0)].cast<double>();
-            longest_list = s[py::int_(1)].cast<int64_t>();
-        }
-        if (const py::object r = attr(md, "list_rotation")) rotation = r.cast<int64_t>();
+        hints = hints_of(md);
+        if (hints.sched && (hints.sched->scalar_type() != at::kInt || hints.sched->device() != q.device() || !hints.sched->is_contiguous()))
+            value_error("mask_metadata.schedule: expected a contiguous int32 tensor on q's device");
     }
     if (mask && mask->scalar_type() != at::kBool) assertion("mask must be a torch.bool tensor");
 
     const int64_t Dk = kernel_head_dim(D, true);
-    // which of the forward kernels: 0 default, otherwise the code of the C ABI
-    if (kernel != "auto" && kernel != "default" && kernel != "short" && kernel != "rotated")
-        value_error("kernel must be 'auto', 'default', 'rotated' or 'short' (got '" + kernel + "')");
-    if (kernel == "rotated" && (sched || f32)) value_error("kernel='rotated' needs bf16/fp16 and mask_metadata without a schedule");
-    int code = SA_FWD_KERNEL_DEFAULT;
-    const bool short_has = !f32 && Dk == 128 && BQ == 128 && pow2_from_16(BK) && l.packed && !sched;
-    const bool short_fits = stats && longest_list <= SA_FWD_SHORT_LISTS_MAX_ENTRIES;
-    if (kernel == "short") {
-        if (!(short_has && short_fits))
-            value_error("kernel='short' needs bf16/fp16, head dim 128, BLOCK_Q 128, mask_metadata with packed_masks, no schedule, and list_stats whose longest list has at most " +
-                        std::to_string(SA_FWD_SHORT_LISTS_MAX_ENTRIES) + " entries");
-        code = SA_FWD_KERNEL_SHORT_LISTS;
-    } else if (kernel == "auto" && short_has && short_fits && mean_list * (double)BK < kShortListKeys) {
-        code = SA_FWD_KERNEL_SHORT_LISTS;
-    } else if (!sched && !f32 && (kernel == "rotated" || (kernel == "auto" && rotation > 0))) {
-        // the default kernel with the FULL entries of Q tile qt walked from a start that depends on qt
-        code = SA_FWD_KERNEL_ROTATED | ((int)(rotation ? rotation : 16) << 8);
-    }
+    const OptTensor &sched = hints.sched;
+    const int code = choose_kernel(kernel, f32, Dk, BQ, BK, l.packed.has_value(), hints);
 
     if (D != Dk && !sched && code == SA_FWD_KERNEL_DEFAULT && ragged_has(q, BQ, BK, l))
         return ragged_forward(q, k, v, l, BQ, BK, 0, 0, Sq, Sk, return_lse);
@@ -427,7 +446,7 @@ std::optional<Out> forward_impl(const Tensor &q, const Tensor &k, const Tensor &
         check_rc(sa_sparse_attention_fwd_lse(qc.data_ptr(), st(qc), kc.data_ptr(), st(kc), vc.data_ptr(), st(vc), o.data_ptr(), st(o), ptr<uint8_t>(mask),
                                              st(mask), ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl), ptr<int32_t>(l.pid), st(l.pid),
                                              ptr<int32_t>(l.pl), st(l.pl), ptr<uint8_t>(l.packed), st(l.packed), ptr<int32_t>(*sched),
-                                             sched->numel() * 4, sched_mode, ptr<float>(lse), st(lse), B, H, Sq, Sk, Dk, BQ, BK, dt, scale, stream));
+                                             sched->numel() * 4, hints.sched_mode, ptr<float>(lse), st(lse), B, H, Sq, Sk, Dk, BQ, BK, dt, scale, stream));
     } else if (code != SA_FWD_KERNEL_DEFAULT) {
         check_rc(sa_sparse_attention_fwd_kernel(qc.data_ptr(), st(qc), kc.data_ptr(), st(kc), vc.data_ptr(), st(vc), o.data_ptr(), st(o),
                                                 ptr<uint8_t>(mask), st(mask), ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl),
@@ -624,6 +643,7 @@ py::object trainable(const Tensor &q, const Tensor &k, const Tensor &v, const Op
 PYBIND11_MODULE(_host, m) {
     m.doc() = "Checks, allocations and launches of the wrappers in sparse_attn_kernel.py and mask_utils.py.";
     m.def("forward", &forward);
+    m.def("forward_kernel", &forward_kernel);
     m.def("forward_tiled", &forward_tiled);
     m.def("decode", &decode);
     m.def("classify", &classify);
