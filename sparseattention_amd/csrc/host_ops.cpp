@@ -585,57 +585,70 @@ py::object backward(const Tensor &do_, const Tensor &q, const Tensor &k, const T
 }
 
 // ---- autograd -----------------------------------------------------------------------------------------------------
-// Everything the backward needs is taken out of the Python objects in the forward: autograd runs backwards on a thread of
-// its own, without the interpreter's lock.
+// What the caller passed is kept as it was passed: the mask unexpanded, so that hooks on saved tensors see the tensor the
+// program has and not B * H planes of it, and the metadata object itself, whose lists are looked at (and checked) when the
+// backward runs.  Autograd runs that on a thread of its own, without the interpreter's lock.
+struct Metadata : torch::CustomClassHolder {
+    PyObject *object;
+    explicit Metadata(py::object o) : object(o.release().ptr()) {}
+    ~Metadata() override {
+        if (!Py_IsInitialized()) return;
+        const py::gil_scoped_acquire gil;
+        Py_DECREF(object);
+    }
+};
+
+// Runs f; its exceptions become Python's own, which alone keep their type on the way out of a backward.
+template <class F>
+auto with_python_errors(F &&f) {
+    try {
+        return f();
+    } catch (const py::builtin_exception &e) {
+        const py::gil_scoped_acquire gil;
+        e.set_error();
+        throw py::error_already_set();
+    }
+}
+
 struct AttentionFunction : public torch::autograd::Function<AttentionFunction> {
     static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &mask, const Out &r,
-                          const std::optional<BackwardLists> &lists) {
-        // (the lists are the program's own, kept as an attribute would be: hooks on saved tensors see what they always saw)
-        if (lists) {
-            c10::List<OptTensor> l;
-            for (const Lists *p : {&lists->by_query, &lists->by_key})
-                for (const OptTensor &t : {OptTensor(p->fid), OptTensor(p->fl), OptTensor(p->pid), OptTensor(p->pl), p->packed}) l.push_back(t);
-            l.push_back(lists->transposed_mask);
-            ctx->saved_data["lists"] = std::move(l);
-        }
+                          const py::object &bmd) {
+        if (!bmd.is_none()) ctx->saved_data["bwd_metadata"] = c10::IValue::make_capsule(c10::make_intrusive<Metadata>(bmd));
         ctx->save_for_backward({q, k, v, r.o, *r.lse, mask.value_or(Tensor())});
         return r.o;
     }
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
         const auto s = ctx->get_saved_variables();
         const Tensor &q = s[0], &k = s[1];
-        OptTensor mask;
-        if (s[5].defined()) mask = s[5];
-        BackwardLists l;
-        if (const auto it = ctx->saved_data.find("lists"); it != ctx->saved_data.end()) {
-            const auto t = it->second.toOptionalTensorList();
-            const auto at_ = [&](size_t i) { return OptTensor(t.get(i)); };
-            l = {{*at_(0), *at_(1), *at_(2), *at_(3), at_(4)}, {*at_(5), *at_(6), *at_(7), *at_(8), at_(9)}, at_(10)};
-        } else {
-            l = backward_lists_from(*mask);
-        }
-        check_backward(grads[0], q, k, s[2], s[3], s[4], mask);
-        const auto g = backward_impl(grads[0], q, k, s[2], s[3], s[4], mask, l);
+        const auto g = with_python_errors([&] {
+            OptTensor mask;
+            if (s[5].defined()) mask = s[5].expand({q.size(0), q.size(1), q.size(2), k.size(2)});
+            check_backward(grads[0], q, k, s[2], s[3], s[4], mask);
+            BackwardLists l;
+            if (const auto it = ctx->saved_data.find("bwd_metadata"); it != ctx->saved_data.end()) {
+                const auto kept = it->second.toCapsule();
+                const py::gil_scoped_acquire gil;
+                l = backward_lists_of(static_cast<const Metadata &>(*kept).object, q, k.size(2));
+            } else {
+                l = backward_lists_from(*mask);
+            }
+            return backward_impl(grads[0], q, k, s[2], s[3], s[4], mask, l);
+        });
         return {std::get<0>(g), std::get<1>(g), std::get<2>(g), Tensor(), Tensor(), Tensor()};
     }
 };
 
 // sparse_attention_trainable, or None where the wrapper has to pad or to make other tiles
-py::object trainable(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &mask_in, int64_t BQ, int64_t BK, py::object md, py::object bmd) {
-    if (q.dim() != 4 || k.dim() != 4 || q.size(2) % 128 || k.size(2) % 128 || q.scalar_type() == at::kFloat || (bmd.is_none() && !mask_in))
+py::object trainable(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &mask, int64_t BQ, int64_t BK, py::object md, py::object bmd) {
+    if (q.dim() != 4 || k.dim() != 4 || q.size(2) % 128 || k.size(2) % 128 || q.scalar_type() == at::kFloat || (bmd.is_none() && !mask))
         return py::none();
     std::optional<Out> r;
     {
         const at::NoGradGuard no_grad;
-        r = forward_impl(q, k, v, mask_in, BQ, BK, md, true, "auto");
+        r = forward_impl(q, k, v, mask, BQ, BK, md, true, "auto");
     }
     if (!r) return py::none();
-    const int64_t Sq = q.size(2), Sk = k.size(2);
-    OptTensor mask = mask_in;
-    if (mask) mask = mask->expand({q.size(0), q.size(1), Sq, Sk});
-    std::optional<BackwardLists> lists;
-    if (!bmd.is_none()) lists = backward_lists_of(bmd, q, Sk);
-    return py::cast(AttentionFunction::apply(q, k, v, mask, *r, lists));
+    return py::cast(AttentionFunction::apply(q, k, v, mask, *r, bmd));
 }
 
 }  // namespace
