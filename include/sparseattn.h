@@ -480,10 +480,13 @@ int sa_merge_attention_parts(const void *o_parts, const int64_t o_parts_strides[
  *                   BK = 64 and the q_* lists; the transposed mask with BQ = 128, BK = 64 and the k_* lists), or
  *                   NULL.  A pass that has its packed buffer reads no mask; with both, `mask` and `mask_t` may be
  *                   NULL, so the bool tensors can be released after preprocessing.
- *   workspace       sa_bwd_workspace_bytes(B, H, Sq) bytes of device memory, 16-byte aligned.  With
- *                   sa_bwd_workspace_bytes_ex(B, H, Sq, Sk, D) bytes (never less; at most 4 GiB more) and both packed
- *                   buffers, dS is kept between the passes where that is faster: dQ is then made from it by one
- *                   product instead of three.  Memory only: the sums are the same, of the same rounded dS.
+ *   workspace       sa_bwd_workspace_bytes(B, H, Sq) bytes of device memory, 16-byte aligned: dQ follows the q_* lists, dK and
+ *                   dV the k_* lists, whatever the others say.  With sa_bwd_workspace_bytes_ex(B, H, Sq, Sk, D) bytes (never
+ *                   less; at most 4 GiB more) and both packed buffers, dS is kept between the passes where that is faster,
+ *                   and dQ is made from it by one product instead of three.  The larger workspace is for lists that agree,
+ *                   made of one mask and its transpose: where an entry attends by the q_* lists and the k_* lists
+ *                   leave its tile out, dQ takes what the memory held.  dS is rounded as it is on its way into the products either way; the scores are
+ *                   scaled in float32 there and in the rounded operand here, so that results differ within rounding.
  * D = 64 or 128, bf16 or fp16, Sq and Sk multiples of 128; tensors as for the forward (last dimension contiguous).
  * The tile sizes of the backward are its own: they need not be those the forward ran with.
  */

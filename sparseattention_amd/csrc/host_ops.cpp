@@ -125,24 +125,26 @@ Lists lists_of(py::handle md) {
             tensor_attr(md, "masked_lens"), opt_tensor_attr(md, "packed_masks")};
 }
 
-// Whether md._validated_for is mask_utils.validation_key(md, Sk, BK): the sizes, then address and version counter of the
-// four list tensors.
-bool validated(py::handle md, const Lists &l, int64_t Sk, int64_t BK) {
-    const py::object key = attr(md, "_validated_for");
-    if (!key || !PyTuple_Check(key.ptr()) || PyTuple_GET_SIZE(key.ptr()) != 6) return false;
-    auto is = [](PyObject *o, unsigned long long want) {
-        const unsigned long long got = PyLong_Check(o) ? PyLong_AsUnsignedLongLongMask(o) : ~want;
-        return got == want;
-    };
-    if (!is(PyTuple_GET_ITEM(key.ptr(), 0), (unsigned long long)Sk) || !is(PyTuple_GET_ITEM(key.ptr(), 1), (unsigned long long)BK)) return false;
+bool int_is(PyObject *o, unsigned long long want) { return (PyLong_Check(o) ? PyLong_AsUnsignedLongLongMask(o) : ~want) == want; }
+
+// Whether `key`, a mask_utils.validation_key, holds address and version counter of the four list tensors as they are.
+bool unedited(PyObject *key, const Lists &l) {
+    if (!PyTuple_Check(key) || PyTuple_GET_SIZE(key) != 6) return false;
     const Tensor *t[4] = {&l.fid, &l.fl, &l.pid, &l.pl};
     for (int i = 0; i < 4; i++) {
-        PyObject *e = PyTuple_GET_ITEM(key.ptr(), 2 + i);
-        if (!PyTuple_Check(e) || PyTuple_GET_SIZE(e) != 2 || !is(PyTuple_GET_ITEM(e, 0), (unsigned long long)(uintptr_t)t[i]->data_ptr()) ||
-            !is(PyTuple_GET_ITEM(e, 1), (unsigned long long)t[i]->_version()))
+        PyObject *e = PyTuple_GET_ITEM(key, 2 + i);
+        if (!PyTuple_Check(e) || PyTuple_GET_SIZE(e) != 2 || !int_is(PyTuple_GET_ITEM(e, 0), (unsigned long long)(uintptr_t)t[i]->data_ptr()) ||
+            !int_is(PyTuple_GET_ITEM(e, 1), (unsigned long long)t[i]->_version()))
             return false;
     }
     return true;
+}
+
+// Whether md._validated_for is mask_utils.validation_key(md, Sk, BK).
+bool validated(py::handle md, const Lists &l, int64_t Sk, int64_t BK) {
+    const py::object key = attr(md, "_validated_for");
+    return key && unedited(key.ptr(), l) && int_is(PyTuple_GET_ITEM(key.ptr(), 0), (unsigned long long)Sk) &&
+           int_is(PyTuple_GET_ITEM(key.ptr(), 1), (unsigned long long)BK);
 }
 void checked_metadata(py::handle md, const Lists &l, int64_t Sk, int64_t BK) {
     if (!validated(md, l, Sk, BK))
@@ -490,13 +492,35 @@ py::object forward_tiled(const Tensor &q, const Tensor &k, const Tensor &v, int6
 struct BackwardLists {
     Lists by_query, by_key;
     OptTensor transposed_mask;
+    bool agree = false;  // both are known to say the same of every entry
 };
+
+// Whether the ten tensors are the ones, unedited, that this package made of one mask: bmd._agreeing holds them, with the
+// addresses and in-place versions they had then, and keeps them alive, so that nothing else can stand in their place.
+bool lists_agree(py::handle bmd, const BackwardLists &l) {
+    const py::object made = attr(bmd, "_agreeing");
+    if (!made || !PyTuple_Check(made.ptr()) || PyTuple_GET_SIZE(made.ptr()) != 2) return false;
+    for (int i = 0; i < 2; i++) {
+        const Lists &a = i ? l.by_key : l.by_query;
+        PyObject *const e = PyTuple_GET_ITEM(made.ptr(), i);
+        if (!a.packed || !PyTuple_Check(e) || PyTuple_GET_SIZE(e) != 8) return false;
+        const Tensor *const t[5] = {&a.fid, &a.fl, &a.pid, &a.pl, &*a.packed};
+        for (int j = 0; j < 5; j++) {
+            PyObject *const o = PyTuple_GET_ITEM(e, j);
+            if (!THPVariable_Check(o) || THPVariable_Unpack(o).unsafeGetTensorImpl() != t[j]->unsafeGetTensorImpl() || t[j]->is_inference()) return false;
+        }
+        if (!unedited(PyTuple_GET_ITEM(e, 5), a) || !int_is(PyTuple_GET_ITEM(e, 6), (unsigned long long)(uintptr_t)a.packed->data_ptr()) ||
+            !int_is(PyTuple_GET_ITEM(e, 7), (unsigned long long)a.packed->_version()))
+            return false;
+    }
+    return true;
+}
 
 BackwardLists backward_lists_of(py::handle bmd, const Tensor &q, int64_t Sk) {
     const int64_t B = q.size(0), H = q.size(1), Sq = q.size(2);
     const py::object mq = attr(bmd, "by_query"), mk = attr(bmd, "by_key");
     if (!mq || !mk) type_error("bwd_metadata has no by_query / by_key lists");
-    BackwardLists l{lists_of(mq), lists_of(mk), opt_tensor_attr(bmd, "transposed_mask")};
+    BackwardLists l{lists_of(mq), lists_of(mk), opt_tensor_attr(bmd, "transposed_mask"), false};
     check_lists(l.by_query, q, B, H, Sq / 128, Sk / 64, "bwd_metadata");
     checked_metadata(mq, l.by_query, Sk, 64);
     check_lists(l.by_key, q, B, H, Sk / 128, Sq / 64, "bwd_metadata");
@@ -508,6 +532,7 @@ BackwardLists backward_lists_of(py::handle bmd, const Tensor &q, int64_t Sk) {
         if (mt->sizes() != at::IntArrayRef(want, 4) || mt->scalar_type() != at::kBool || mt->device() != q.device())
             value_error("bwd_metadata.transposed_mask: expected bool " + str(at::IntArrayRef(want, 4)) + " on " + q.device().str());
     }
+    l.agree = lists_agree(bmd, l);
     return l;
 }
 
@@ -516,7 +541,7 @@ BackwardLists backward_lists_from(const Tensor &mask) {
     const int64_t B = mask.size(0), H = mask.size(1);
     const Tensor distinct = mask.narrow(0, 0, mask.stride(0) == 0 ? 1 : B).narrow(1, 0, mask.stride(1) == 0 ? 1 : H);
     const Tensor transposed = distinct.transpose(-1, -2).contiguous().expand({B, H, mask.size(3), mask.size(2)});
-    return {classify_lists(mask, 128, 64, true), classify_lists(transposed, 128, 64, true), std::nullopt};
+    return {classify_lists(mask, 128, 64, true), classify_lists(transposed, 128, 64, true), std::nullopt, true};
 }
 
 std::tuple<Tensor, Tensor, Tensor> backward_impl(const Tensor &do_, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &o, const Tensor &lse,
@@ -531,7 +556,8 @@ std::tuple<Tensor, Tensor, Tensor> backward_impl(const Tensor &do_, const Tensor
     const Tensor dq = at::empty_like(qc), dk = at::empty_like(kc), dv = at::empty_like(vc);
     const Lists &a = l.by_query, &b = l.by_key;
     const auto workspace = [&](size_t bytes) { return at::empty({(int64_t)bytes}, at::TensorOptions().dtype(at::kByte).device(q.device())); };
-    size_t ws_bytes = a.packed && b.packed ? sa_bwd_workspace_bytes_ex(B, H, Sq, Sk, Dk) : sa_bwd_workspace_bytes(B, H, Sq);
+    // dQ from stored dS takes a dS of every entry of by_query that attends, which lists that do not agree do not give
+    size_t ws_bytes = a.packed && b.packed && l.agree ? sa_bwd_workspace_bytes_ex(B, H, Sq, Sk, Dk) : sa_bwd_workspace_bytes(B, H, Sq);
     Tensor ws;
     try {
         ws = workspace(ws_bytes);

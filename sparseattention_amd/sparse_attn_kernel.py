@@ -211,13 +211,29 @@ class BackwardMetadata:
     mask per 128 keys (tiles of 64 queries).  Built once per mask by :func:`compute_backward_metadata`.
 
     When both lists carry ``packed_masks`` (the PARTIAL tiles at one bit per entry), the backward reads those and
-    neither the mask nor its transposed copy, so both bool tensors can be released after this preprocessing."""
+    neither the mask nor its transposed copy, so both bool tensors can be released after this preprocessing.
+
+    Lists put together by the caller need not agree with each other: dQ follows ``by_query`` alone, dK and dV ``by_key``.
+    Lists of one mask from the functions below are known to agree (``_agreeing``: their tensors with the addresses and
+    in-place versions they had) until they are edited or replaced, and then dQ may be made from the dS of the pass over the keys."""
 
     def __init__(self, by_query: MaskMetadata, by_key: MaskMetadata, transposed_mask: torch.Tensor | None = None):
         self.by_query = by_query
         self.by_key = by_key
         #: bool [B,H,Sk,Sq], the mask transposed as a tensor of its own (distinct planes, expanded), or None
         self.transposed_mask = transposed_mask
+        self._agreeing = None
+
+    def __getstate__(self):
+        return {**self.__dict__, "_agreeing": None}  # (addresses and versions are this process's own)
+
+
+def _of_one_mask(bmd: BackwardMetadata) -> BackwardMetadata:
+    """Notes that both lists of ``bmd``, with packed tiles, were made from one mask."""
+    bmd._agreeing = tuple((md.unmasked_kv_ids, md.unmasked_lens, md.masked_kv_ids, md.masked_lens, md.packed_masks,
+                           md._validated_for, md.packed_masks.data_ptr(), md.packed_masks._version)
+                          for md in (bmd.by_query, bmd.by_key))
+    return bmd
 
 
 def compute_backward_metadata(mask: torch.Tensor, pack_partial: bool = True) -> BackwardMetadata:
@@ -234,9 +250,10 @@ def compute_backward_metadata(mask: torch.Tensor, pack_partial: bool = True) -> 
     B, H = mask.shape[:2]
     distinct = mask[: 1 if mask.stride(0) == 0 else B, : 1 if mask.stride(1) == 0 else H]
     transposed = distinct.transpose(-1, -2).contiguous().expand(B, H, mask.shape[3], mask.shape[2])
-    return BackwardMetadata(compute_mask_kernel(mask, 128, 64, pack_partial=pack_partial),
-                            compute_mask_kernel(transposed, 128, 64, pack_partial=pack_partial),
-                            None if pack_partial else transposed)
+    bmd = BackwardMetadata(compute_mask_kernel(mask, 128, 64, pack_partial=pack_partial),
+                           compute_mask_kernel(transposed, 128, 64, pack_partial=pack_partial),
+                           None if pack_partial else transposed)
+    return _of_one_mask(bmd) if pack_partial else bmd
 
 
 def compute_backward_metadata_terms(terms, B: int, H: int, Sq: int, Sk: int, doc_q=None, doc_k=None,
@@ -245,9 +262,9 @@ def compute_backward_metadata_terms(terms, B: int, H: int, Sq: int, Sk: int, doc
     their packed PARTIAL tiles, the key-major one from the transposed terms, so that
     ``sparse_attention_backward(..., mask=None, bwd_metadata=...)`` runs without any mask tensor."""
     terms = list(terms)
-    return BackwardMetadata(
+    return _of_one_mask(BackwardMetadata(
         compute_mask_terms(terms, B, H, Sq, Sk, 128, 64, doc_q, doc_k, device),
-        compute_mask_terms([t.transposed() for t in terms], B, H, Sk, Sq, 128, 64, doc_k, doc_q, device), None)
+        compute_mask_terms([t.transposed() for t in terms], B, H, Sk, Sq, 128, 64, doc_k, doc_q, device), None))
 
 
 def sparse_attention_backward(do: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
