@@ -38,7 +38,7 @@
 extern "C" {
 #endif
 
-#define SA_ABI_VERSION 16
+#define SA_ABI_VERSION 17
 
 enum sa_status {
     SA_OK = 0,
@@ -492,6 +492,9 @@ int sa_merge_attention_parts(const void *o_parts, const int64_t o_parts_strides[
  */
 size_t sa_bwd_workspace_bytes(int B, int H, int Sq);
 size_t sa_bwd_workspace_bytes_ex(int B, int H, int Sq, int Sk, int D);
+/* The most bytes up to `limit` that a workspace between these two has a use for (never less than the first): fewer planes
+ * of dS at a time, or none. */
+size_t sa_bwd_workspace_bytes_within(int B, int H, int Sq, int Sk, int D, size_t limit);
 int sa_sparse_attention_bwd(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
                             const void *v, const int64_t v_strides[4], const void *o, const int64_t o_strides[4],
                             const void *d_o, const int64_t do_strides[4], const float *lse,

@@ -10,7 +10,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libsparseattn_hip.so")
 
-SA_ABI_VERSION = 16
+SA_ABI_VERSION = 17
 SA_OK = 0
 SA_ERR_INVALID_ARGUMENT = -1
 SA_ERR_UNSUPPORTED = -2
@@ -57,6 +57,7 @@ EXPORTS = (
     "sa_merge_attention_parts",
     "sa_bwd_workspace_bytes",
     "sa_bwd_workspace_bytes_ex",
+    "sa_bwd_workspace_bytes_within",
     "sa_sparse_attention_bwd",
     "sa_mask_terms_workspace_bytes",
     "sa_mask_classify_terms",
@@ -168,6 +169,8 @@ def load() -> ctypes.CDLL:
     lib.sa_bwd_workspace_bytes.argtypes = [ctypes.c_int] * 3
     lib.sa_bwd_workspace_bytes_ex.restype = ctypes.c_size_t
     lib.sa_bwd_workspace_bytes_ex.argtypes = [ctypes.c_int] * 5
+    lib.sa_bwd_workspace_bytes_within.restype = ctypes.c_size_t
+    lib.sa_bwd_workspace_bytes_within.argtypes = [ctypes.c_int] * 5 + [ctypes.c_size_t]
     lib.sa_sparse_attention_bwd.restype = ctypes.c_int
     lib.sa_sparse_attention_bwd.argtypes = (
         [_vp, _i64p] * 13 + [_vp, _i64p] * 8 + [_vp, ctypes.c_size_t] + [ctypes.c_int] * 6 + [ctypes.c_float, _vp]

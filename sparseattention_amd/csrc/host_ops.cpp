@@ -9,6 +9,7 @@
 // SparseAttnError for the library's own error codes.
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <torch/extension.h>
 
 #include <cmath>
@@ -544,6 +545,25 @@ BackwardLists backward_lists_from(const Tensor &mask) {
     return {classify_lists(mask, 128, 64, true), classify_lists(transposed, 128, 64, true), std::nullopt, true};
 }
 
+// What the backward takes of `room` bytes of device memory: a quarter, so that a program near the card's capacity keeps its
+// room, and its allocator need not give back what it holds (which waits for the device) to find a block of this size.
+int64_t backward_workspace_bytes(int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D, int64_t room) {
+    return (int64_t)sa_bwd_workspace_bytes_within(B, H, Sq, Sk, D, (size_t)room / 4);
+}
+// Bytes that this process can still get on `dev`: free ones, and those its allocator holds without a use for them.
+int64_t device_room(const at::Device &dev) {
+    int64_t idle = 0;
+    try {
+        const auto s = c10::hip::HIPCachingAllocator::getDeviceStats(dev.index());
+        constexpr auto all = static_cast<size_t>(c10::CachingAllocator::StatType::AGGREGATE);
+        idle = s.reserved_bytes[all].current - s.allocated_bytes[all].current;
+    } catch (const c10::Error &) {  // an allocator without statistics
+    }
+    size_t free = 0, total = 0;
+    if (hipMemGetInfo(&free, &total) != hipSuccess) free = 0;
+    return idle + (int64_t)free;
+}
+
 std::tuple<Tensor, Tensor, Tensor> backward_impl(const Tensor &do_, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &o, const Tensor &lse,
                                                  const OptTensor &mask, const BackwardLists &l) {
     const int64_t B = q.size(0), H = q.size(1), Sq = q.size(2), D = q.size(3), Sk = k.size(2);
@@ -557,11 +577,13 @@ std::tuple<Tensor, Tensor, Tensor> backward_impl(const Tensor &do_, const Tensor
     const Lists &a = l.by_query, &b = l.by_key;
     const auto workspace = [&](size_t bytes) { return at::empty({(int64_t)bytes}, at::TensorOptions().dtype(at::kByte).device(q.device())); };
     // dQ from stored dS takes a dS of every entry of by_query that attends, which lists that do not agree do not give
-    size_t ws_bytes = a.packed && b.packed && l.agree ? sa_bwd_workspace_bytes_ex(B, H, Sq, Sk, Dk) : sa_bwd_workspace_bytes(B, H, Sq);
+    size_t ws_bytes = sa_bwd_workspace_bytes(B, H, Sq);
+    if (a.packed && b.packed && l.agree && sa_bwd_workspace_bytes_ex(B, H, Sq, Sk, Dk) > ws_bytes)
+        ws_bytes = backward_workspace_bytes(B, H, Sq, Sk, Dk, device_room(q.device()));
     Tensor ws;
     try {
         ws = workspace(ws_bytes);
-    } catch (const c10::OutOfMemoryError &) {  // dS finds no place: the passes that make it anew
+    } catch (const c10::OutOfMemoryError &) {  // dS finds no place after all: the passes that make it anew
         ws_bytes = sa_bwd_workspace_bytes(B, H, Sq);
         ws = workspace(ws_bytes);
     }
@@ -688,5 +710,6 @@ PYBIND11_MODULE(_host, m) {
     m.def("classify", &classify);
     m.def("classify_terms", &classify_terms);
     m.def("backward", &backward);
+    m.def("backward_workspace_bytes", &backward_workspace_bytes);
     m.def("trainable", &trainable);
 }

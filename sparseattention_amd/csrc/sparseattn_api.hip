@@ -1072,6 +1072,14 @@ size_t sa_bwd_workspace_bytes_ex(int B, int H, int Sq, int Sk, int D) {
     return ds ? ds_offset(stats) + ds : stats;
 }
 
+size_t sa_bwd_workspace_bytes_within(int B, int H, int Sq, int Sk, int D, size_t limit) {
+    const size_t stats = sa_bwd_workspace_bytes(B, H, Sq), most = sa_bwd_workspace_bytes_ex(B, H, Sq, Sk, D);
+    if (most <= limit || most == stats) return most;
+    if (limit <= ds_offset(stats)) return stats;
+    const int group = sa::bwd_ds_group(B, H, Sq, Sk, D, limit - ds_offset(stats));
+    return group > 0 ? ds_offset(stats) + (size_t)group * Sq * Sk * 2 : stats;
+}
+
 int sa_sparse_attention_bwd(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
                             const void *v, const int64_t v_strides[4], const void *o, const int64_t o_strides[4],
                             const void *d_o, const int64_t do_strides[4], const float *lse,
