@@ -263,6 +263,8 @@ class Tiling:
     metadata: MaskMetadata
     padded_mask: torch.Tensor
     report: list
+    #: keys of the mask itself (None: not known)
+    Sk: Optional[int] = None
 
 
 def select_tiling(mask: torch.Tensor, candidates=DEFAULT_TILE_CANDIDATES, offsets: Sequence[Tuple[int, int]] = ((0, 0),),
@@ -297,7 +299,7 @@ def select_tiling(mask: torch.Tensor, candidates=DEFAULT_TILE_CANDIDATES, offset
                 best = (cost, BQ, BK, qo, ko, md, padded)
     if best is None:
         raise ValueError("no candidate tile size / offset pair fits")
-    return Tiling(best[1], best[2], best[3], best[4], best[5], best[6], report)
+    return Tiling(best[1], best[2], best[3], best[4], best[5], best[6], report, Sk)
 
 
 # ---- masks given by a formula -----------------------------------------------------------------------------------

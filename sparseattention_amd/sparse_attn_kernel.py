@@ -168,13 +168,15 @@ def sparse_attention_tiled(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, ti
     lets nothing attend to or from, and the rows of the result that belong to the caller's queries are returned.  With
     both offsets 0 and sizes that are whole tiles this is sparse_attention itself.  In bf16 and fp16 with packed tiles,
     BLOCK_Q up to 128 and head dims that are multiples of 8 up to 128 the kernel leaves the rows out that do not exist;
-    otherwise it costs a copy of q, k, v."""
+    otherwise, and for k and v of fewer keys than the mask, it costs a copy of q, k, v."""
     Sq, Sk = q.shape[-2], k.shape[-2]
     Pq, Pk = tiling.padded_mask.shape[-2:]
     qo, ko = tiling.q_offset, tiling.k_offset
     if not (qo + Sq <= Pq and ko + Sk <= Pk):
         raise ValueError(f"tiling for a mask of {Pq - qo}x{Pk - ko} or smaller, got Sq={Sq}, Sk={Sk}")
-    if (qo, Pq, ko, Pk) != (0, Sq, 0, Sk):
+    # (the kernel reads no key that the tensors do not have, so it needs a mask that has none there either; with fewer keys
+    # than the mask the missing ones are zeros, as below)
+    if (qo, Pq, ko, Pk) != (0, Sq, 0, Sk) and Sk == tiling.Sk:
         out = _native.host().forward_tiled(q, k, v, tiling.BLOCK_Q, tiling.BLOCK_K, qo, ko, Pq, Pk, tiling.metadata, return_lse)
         if out is not None:
             return out

@@ -63,3 +63,16 @@ def test_head_dims_between_the_kernels(gpu, D):
     # through padding, as without the packed tiles
     p = sparse_attention(q, k, v, mask, 64, 32, compute_mask_kernel(mask, 64, 32, pack_partial=False))
     assert torch.equal(o, p)
+
+
+@pytest.mark.parametrize("Sk", [257, 299])
+def test_tensors_with_fewer_keys_than_the_mask(gpu, Sk):
+    """Keys that the mask has and the tensors do not are keys of zeros."""
+    B, H, S, D, qo, ko = 1, 2, 300, 80, 3, 5
+    q, k, v = (inside(B, H, n, D, torch.bfloat16, 30 + i, gpu) for i, n in enumerate((S, Sk, Sk)))
+    t = select_tiling(torch.ones(B, H, S, S, dtype=torch.bool, device=gpu), candidates=((64, 32),), offsets=((qo, ko),))
+    Pq, Pk = t.padded_mask.shape[-2:]
+    pad = torch.nn.functional.pad
+    want = sparse_attention(pad(q, (0, 0, qo, Pq - qo - S)), *(pad(x, (0, 0, ko, Pk - ko - Sk)) for x in (k, v)), t.padded_mask,
+                            64, 32, t.metadata)[:, :, qo:qo + S]
+    assert torch.equal(sparse_attention_tiled(q, k, v, t), want)
