@@ -487,7 +487,7 @@ __global__ __launch_bounds__(256) void decode_merge_many_kernel(const DecodePara
             f32x2 ml[kMergeBatch], x[kMergeBatch][NP];
 #pragma unroll
             for (int i = 0; i < kMergeBatch; i++) {
-                // (past the last part: the last one again, with weight 0)
+                // (past the last part: the last one again, left out below: a weight of 0 would turn an infinity into NaN)
                 const float *pp = part + min(i0 + 8 * i, p.nsplit - 1) * stride;
                 ml[i] = *(const f32x2 *)(pp + D);
 #pragma unroll
@@ -495,8 +495,9 @@ __global__ __launch_bounds__(256) void decode_merge_many_kernel(const DecodePara
             }
 #pragma unroll
             for (int i = 0; i < kMergeBatch; i++) {
+                if (i0 + 8 * i >= p.nsplit) break;
                 // 0 for parts without an attended key (m = -inf)
-                const float w = i0 + 8 * i < p.nsplit ? __builtin_amdgcn_exp2f(ml[i].x - M) : 0.f;
+                const float w = __builtin_amdgcn_exp2f(ml[i].x - M);
                 L += w * ml[i].y;
 #pragma unroll
                 for (int c = 0; c < NP; c++) {

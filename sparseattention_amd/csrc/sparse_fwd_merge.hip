@@ -32,7 +32,7 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(const FwdParams p, int l
 #pragma unroll
     for (int g = 0; g < 4; g++) sum[g] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int i0 = 0; i0 < share; i0 += kBatch) {
-        // (past the last part: the last one again, with weight 0)
+        // (past the last part: the last one again, left out of the sums below: a weight of 0 would turn an infinity into NaN)
         f32x2 st[kBatch];
         f32x4 x[kBatch][4];
 #pragma unroll
@@ -54,7 +54,8 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(const FwdParams p, int l
             for (int e = 0; e < 4; e++) sum[g][e] *= keep;
 #pragma unroll
         for (int i = 0; i < kBatch; i++) {
-            const float w = i0 + i < share ? __builtin_amdgcn_exp2f(st[i].x - M0) : 0.f;
+            if (i0 + i >= share) break;
+            const float w = __builtin_amdgcn_exp2f(st[i].x - M0);
             L += w * st[i].y;
 #pragma unroll
             for (int g = 0; g < 4; g++)
