@@ -5,6 +5,9 @@
 // with metadata, 68 us with the mask classified on the way and 220 us for a training step, so the device waited for the
 // host.  Nothing is kept between calls; every workspace is a tensor of the caching allocator, ordered by the stream.
 //
+// The interpreter's lock is held while Python objects are read (arguments, metadata) and let go of for the rest, so that a
+// launch that waits for room in a queue, or an allocation that waits for the device, stops no other thread.
+//
 // Errors are the Python exceptions the wrappers document: ValueError, TypeError, AssertionError, RuntimeError, and
 // SparseAttnError for the library's own error codes.
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -42,8 +45,7 @@ std::string str(const Tensor &t) { return std::string(c10::toString(t.scalar_typ
 void check_rc(int rc) {
     if (rc == SA_OK) return;
     if (rc == SA_ERR_INVALID_ARGUMENT) value_error(std::string("libsparseattn_hip: ") + sa_last_error());
-    // (the backward of the autograd function runs on a thread of its own, without the interpreter's lock)
-    py::gil_scoped_acquire gil;
+    const py::gil_scoped_acquire gil;
     const py::object cls = py::module_::import("sparseattention_amd._native").attr("SparseAttnError");
     const py::object err = cls(rc, py::str(sa_last_error()));
     PyErr_SetObject(cls.ptr(), err.ptr());
@@ -217,7 +219,12 @@ py::tuple as_tuple(const Lists &l) { return py::make_tuple(l.fid, l.fl, l.pid, l
 
 // compute_mask_kernel: (unmasked_kv_ids, unmasked_lens, masked_kv_ids, masked_lens, packed_masks or None)
 py::tuple classify(const Tensor &mask, int64_t BQ, int64_t BK, std::optional<bool> pack_partial) {
-    return as_tuple(classify_lists(mask, BQ, BK, pack_partial));
+    Lists l;
+    {
+        const py::gil_scoped_release unlocked;
+        l = classify_lists(mask, BQ, BK, pack_partial);
+    }
+    return as_tuple(l);
 }
 
 // compute_mask_terms: the same from terms, eight int32 each (their and the documents' shapes are checked by the caller)
@@ -226,13 +233,17 @@ py::tuple classify_terms(const std::vector<int32_t> &terms, int64_t B, int64_t H
     const int64_t nQ = Sq / BQ, nK = Sk / BK;
     const bool per_batch = B > 1 && ((doc_q && doc_q->stride(0) != 0) || (doc_k && doc_k->stride(0) != 0));
     const int64_t uB = per_batch ? B : 1;
-    const c10::DeviceGuard guard(dev);
-    Lists l = empty_lists(uB, 1, B, H, nQ, nK, BQ * BK / 8, pack, dev);
-    const size_t need = sa_mask_terms_workspace_bytes(uB, Sq, Sk, BQ, BK);
-    const Tensor ws = at::empty({(int64_t)std::max<size_t>(need, 1)}, at::TensorOptions().dtype(at::kByte).device(dev));
-    check_rc(sa_mask_classify_terms(terms.data(), (int)(terms.size() / 8), ptr<int32_t>(doc_q), st(doc_q), ptr<int32_t>(doc_k), st(doc_k), B, H, Sq, Sk,
-                                    BQ, BK, ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl), ptr<int32_t>(l.pid), st(l.pid),
-                                    ptr<int32_t>(l.pl), st(l.pl), ptr<uint8_t>(l.packed), st(l.packed), ws.data_ptr(), ws.numel(), stream_of(l.fid)));
+    Lists l;
+    {
+        const py::gil_scoped_release unlocked;
+        const c10::DeviceGuard guard(dev);
+        l = empty_lists(uB, 1, B, H, nQ, nK, BQ * BK / 8, pack, dev);
+        const size_t need = sa_mask_terms_workspace_bytes(uB, Sq, Sk, BQ, BK);
+        const Tensor ws = at::empty({(int64_t)std::max<size_t>(need, 1)}, at::TensorOptions().dtype(at::kByte).device(dev));
+        check_rc(sa_mask_classify_terms(terms.data(), (int)(terms.size() / 8), ptr<int32_t>(doc_q), st(doc_q), ptr<int32_t>(doc_k), st(doc_k), B, H, Sq,
+                                        Sk, BQ, BK, ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl), ptr<int32_t>(l.pid), st(l.pid),
+                                        ptr<int32_t>(l.pl), st(l.pl), ptr<uint8_t>(l.packed), st(l.packed), ws.data_ptr(), ws.numel(), stream_of(l.fid)));
+    }
     return as_tuple(l);
 }
 
@@ -263,18 +274,21 @@ Out decode_impl(const Tensor &q, const Tensor &k, const Tensor &v, const OptTens
     OptTensor mask = mask_in;
     if (mask) mask = mask->expand({B, H, Sq, Sk});
     Lists l;
-    // (a small mask without lists: the decode kernel finds its tiles in it; what the classification refuses goes there)
-    const bool direct = md.is_none() && mask && mask->scalar_type() == at::kBool && BK > 0 && BK <= Sk &&
-                        sa_decode_mask_fits(ptr<uint8_t>(*mask), st(*mask), B, H, Sq, Sk, BK);
-    if (md.is_none() && !direct) {
-        if (!mask) value_error("sparse_attention_decode needs the mask or mask_metadata with packed_masks");
-        l = classify_lists(*mask, Sq, BK, std::nullopt);
-    } else if (!direct) {
+    const bool has_md = !md.is_none();
+    if (has_md) {
         l = lists_of(md);
         if (BK <= 0) value_error("BLOCK_K must be positive");
         check_lists(l, q, B, H, 1, Sk / BK, "mask_metadata");
         checked_metadata(md, l, Sk, BK);
         if (l.packed) check_packed(*l.packed, q, B, H, 1, Sk / BK, Sq * BK / 8, "mask_metadata");
+    }
+    const py::gil_scoped_release unlocked;
+    // (a small mask without lists: the decode kernel finds its tiles in it; what the classification refuses goes there)
+    const bool direct = !has_md && mask && mask->scalar_type() == at::kBool && BK > 0 && BK <= Sk &&
+                        sa_decode_mask_fits(ptr<uint8_t>(*mask), st(*mask), B, H, Sq, Sk, BK);
+    if (!has_md && !direct) {
+        if (!mask) value_error("sparse_attention_decode needs the mask or mask_metadata with packed_masks");
+        l = classify_lists(*mask, Sq, BK, std::nullopt);
     }
     if (l.packed && BK == 16 && Sq % 2) l.packed.reset();  // (halfword rows: the kernels want an even number of them)
     if (!l.packed) {
@@ -382,6 +396,7 @@ bool ragged_has(const Tensor &q, int64_t BQ, int64_t BK, const Lists &l) {
     return (dt == SA_DTYPE_BF16 || dt == SA_DTYPE_FP16) && q.size(3) % 8 == 0 && q.size(3) <= 128 && (BQ == 32 || BQ == 64 || BQ == 128) &&
            pow2_from_16(BK) && l.packed.has_value();
 }
+// (called without the interpreter's lock)
 Out ragged_forward(const Tensor &q, const Tensor &k, const Tensor &v, const Lists &l, int64_t BQ, int64_t BK, int64_t q0, int64_t k0, int64_t Pq,
                    int64_t Pk, bool return_lse) {
     const int64_t B = q.size(0), H = q.size(1), Sq = q.size(2), D = q.size(3), Sk = k.size(2);
@@ -417,9 +432,7 @@ std::optional<Out> forward_impl(const Tensor &q, const Tensor &k, const Tensor &
     const int64_t nQ = Sq / BQ, nK = Sk / BK;
     Lists l;
     Hints hints;
-    if (!has_md) {
-        l = classify_lists(*mask, BQ, BK, std::nullopt);
-    } else {
+    if (has_md) {
         l = lists_of(md);
         check_lists(l, q, B, H, nQ, nK, "mask_metadata");
         checked_metadata(md, l, Sk, BK);
@@ -428,6 +441,8 @@ std::optional<Out> forward_impl(const Tensor &q, const Tensor &k, const Tensor &
         if (hints.sched && (hints.sched->scalar_type() != at::kInt || hints.sched->device() != q.device() || !hints.sched->is_contiguous()))
             value_error("mask_metadata.schedule: expected a contiguous int32 tensor on q's device");
     }
+    const py::gil_scoped_release unlocked;
+    if (!has_md) l = classify_lists(*mask, BQ, BK, std::nullopt);
     if (mask && mask->scalar_type() != at::kBool) assertion("mask must be a torch.bool tensor");
 
     const int64_t Dk = kernel_head_dim(D, true);
@@ -485,7 +500,12 @@ py::object forward_tiled(const Tensor &q, const Tensor &k, const Tensor &v, int6
     check_lists(l, q, q.size(0), q.size(1), Pq / BQ, Pk / BK, "tiling.metadata");
     checked_metadata(md, l, Pk, BK);
     check_packed(*l.packed, q, q.size(0), q.size(1), Pq / BQ, Pk / BK, BQ * BK / 8, "tiling.metadata");
-    return as_object(ragged_forward(q, k, v, l, BQ, BK, q0, k0, Pq, Pk, return_lse));
+    Out r;
+    {
+        const py::gil_scoped_release unlocked;
+        r = ragged_forward(q, k, v, l, BQ, BK, q0, k0, Pq, Pk, return_lse);
+    }
+    return as_object(r);
 }
 
 // ---- backward -----------------------------------------------------------------------------------------------------
@@ -628,7 +648,15 @@ py::object backward(const Tensor &do_, const Tensor &q, const Tensor &k, const T
     if (mask) mask = mask->expand({q.size(0), q.size(1), Sq, Sk});
     if (Sq % 128 || Sk % 128) return py::none();
     if (bmd.is_none() && !mask) value_error("sparse_attention_backward needs the mask or a BackwardMetadata with packed tiles");
-    const auto g = backward_impl(do_, q, k, v, o, lse, mask, bmd.is_none() ? backward_lists_from(*mask) : backward_lists_of(bmd, q, Sk));
+    const bool has_bmd = !bmd.is_none();
+    BackwardLists l;
+    if (has_bmd) l = backward_lists_of(bmd, q, Sk);
+    std::tuple<Tensor, Tensor, Tensor> g;
+    {
+        const py::gil_scoped_release unlocked;
+        if (!has_bmd) l = backward_lists_from(*mask);
+        g = backward_impl(do_, q, k, v, o, lse, mask, l);
+    }
     return py::make_tuple(std::get<0>(g), std::get<1>(g), std::get<2>(g));
 }
 
