@@ -142,6 +142,7 @@ struct FwdParams {
     //   ws    [B*H*nQ][nsplit][BQ/32][D/8][64 lanes][4] floats: unnormalised rows in the order the registers hold them
     //   ws_ml [B*H*nQ][nsplit][BQ][2] floats: reference value (-inf: no attended key) and sum of every row
     int nsplit, split_chunks;  // split_chunks: chunks of one part (the last ones may be shorter)
+    int split_least;           // lists of up to this many chunks are not shared
     float *ws, *ws_ml;
     // Ragged sizes: the tile grid (Sq, Sk, nQ, nK, lists, packed tiles) is that of a padded mask, the tensors have Sq_in
     // and Sk_in rows, which stand q0 and k0 rows into the grid, of D_in elements (a multiple of 8, at most the kernel's D).
@@ -151,9 +152,10 @@ struct FwdParams {
 
 // How many workgroups share a list of NE entries of 2^lbk keys, walked in chunks of 2^lck keys, and the first entry of
 // part s of them (s = share: the end of the list).  Entries of one chunk stay together.
-__host__ __device__ inline int fwd_split_share(int NE, int lbk, int lck, int split_chunks, int nsplit) {
+__host__ __device__ inline int fwd_split_share(int NE, int lbk, int lck, int split_least, int split_chunks, int nsplit) {
     const int le = lck > lbk ? lck - lbk : 0, lc = lbk > lck ? lbk - lck : 0;
     const int groups = (NE + (1 << le) - 1) >> le;
+    if ((groups << lc) <= split_least) return 1;
     const int parts = ((groups << lc) + split_chunks - 1) / split_chunks;
     const int most = groups < nsplit ? groups : nsplit;
     return parts < most ? (parts > 1 ? parts : 1) : (most > 1 ? most : 1);
@@ -164,8 +166,11 @@ __host__ __device__ inline int fwd_split_first(int NE, int lbk, int lck, int s, 
     const int e = (int)(groups * (unsigned)s / (unsigned)share) << le;
     return e < NE ? e : NE;
 }
-// The rule for nsplit and split_chunks: sparse_fwd_merge.hip.
-void fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus, int *nsplit, int *split_chunks);
+// The rule for nsplit, split_chunks and split_least: sparse_fwd_merge.hip.
+struct FwdSplitPlan {
+    int nsplit = 1, chunks = 1 << 30, least = 0;
+};
+FwdSplitPlan fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus);
 // Adds up the parts of shared lists (dtype 2: float32 output).
 hipError_t launch_fwd_merge(const FwdParams &p, int dtype, int D, int BQ, hipStream_t stream);
 

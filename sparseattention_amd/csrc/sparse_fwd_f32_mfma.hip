@@ -88,7 +88,7 @@ __global__ __launch_bounds__(NW * 64, NW >= 4 ? 2 : 1) void sparse_fwd_f32_mfma_
     int NE = F + min(min(max(p.part_lens[b * p.pls[0] + h * p.pls[1] + qt * p.pls[2]], 0), p.nK - F), kF32ListCap - F);
     int share = 1, p_lo = 0;
     if (p.nsplit > 1) {
-        share = fwd_split_share(NE, p.lbk, 5, p.split_chunks, p.nsplit);
+        share = fwd_split_share(NE, p.lbk, 5, p.split_least, p.split_chunks, p.nsplit);
         if (s0 >= share) return;
         const int e_lo = fwd_split_first(NE, p.lbk, 5, s0, share), e_hi = fwd_split_first(NE, p.lbk, 5, s0 + 1, share);
         fid += (int64_t)min(e_lo, F) * p.fis[3];

@@ -234,7 +234,7 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
             const int32_t *const cnt_addr[2] = {fl0, pl0};
             scalar_gather(cnt_addr, cnt);
             set_item(b0, h0, qt0, cnt[0], cnt[1]);
-            share = fwd_split_share(NE, p.lbk, 6, p.split_chunks, p.nsplit);
+            share = fwd_split_share(NE, p.lbk, 6, p.split_least, p.split_chunks, p.nsplit);
             share_part = s0;
             if (s0 >= share) return;
             const int e_lo = fwd_split_first(NE, p.lbk, 6, s0, share), e_hi = fwd_split_first(NE, p.lbk, 6, s0 + 1, share);

@@ -21,7 +21,7 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(const FwdParams p, int l
     const int b = bh / p.H, h = bh - b * p.H;
     const int F = min(max(p.full_lens[b * p.fls[0] + h * p.fls[1] + qt * p.fls[2]], 0), p.nK);
     const int NE = F + min(max(p.part_lens[b * p.pls[0] + h * p.pls[1] + qt * p.pls[2]], 0), p.nK - F);
-    const int share = fwd_split_share(NE, p.lbk, lck, p.split_chunks, p.nsplit);
+    const int share = fwd_split_share(NE, p.lbk, lck, p.split_least, p.split_chunks, p.nsplit);
     if (share <= 1) return;  // written by the workgroup that had the whole list
 
     const int64_t part0 = (int64_t)tile * p.nsplit;
@@ -85,30 +85,39 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(const FwdParams p, int l
 
 // When lists are shared.  A compute unit takes two workgroups of these kernels, so up to 2 * cus of them run at once, and a
 // launch of half as many or fewer Q tiles leaves slots empty while each list is walked by one workgroup.  A chunk of 64
-// keys takes a workgroup 0.95 us while it has its compute unit to itself and 1.5 us beside another one (D = 128); the
-// partial results and their merge cost 4 us plus 12 ns per part.  With few tiles parts of 8 chunks pay for that (64 tiles
-// of 16 chunks: 20.4 -> 18.7 us; 8 tiles of 256: 240 -> 31), up to 128 tiles 24 chunks do (128 tiles of 32: 38 -> 33 us,
-// of 64: 69 -> 47, of 256: 255 -> 142; parts of 8 made lists of 18 slower, 25 -> 31 us), and between 128 and 256 tiles,
-// where a second workgroup per compute unit is all there is to gain, only long lists (256 tiles of 64: 82 -> 75 us, of
-// 256: 288 -> 239; of 16: 21 -> 28).  From 257 tiles on every slot has work.  The lengths are on the device: the host
-// goes by Sk, and where the lists turn out short (a window) a launch pays 3 to 4 us for the merge that finds nothing.
+// keys takes a workgroup 0.95 us while it has its compute unit to itself and 1.5 us beside another one (D = 128).  The host
+// goes by Sk; the lengths are on the device, and a launch pays 2 to 3 us for a merge that finds nothing to do.  us at D = 128,
+// bf16, every list as long as stated, one workgroup per list | shared (and "alone" in such a launch: with that merge):
+//   parts of 8 chunks, up to cus / 4 tiles
+//       8 tiles   8 chunks  12.1 | alone 14.0    12  15.9 | 14.2    32  34.1 | 17.3    256  240 | 31
+//      64 tiles   4 chunks   9.0 | alone 11.5    12  16.7 | 19.9    16  20.0 | 21.2    24  27.4 | 24.1    64  63.9 | 32.6
+//   parts of 16 chunks, up to cus / 2 tiles, lists of more than 8 + tiles / 8 chunks (beside each other workgroups take half as
+//   long again: two of 9 chunks are no faster than one of 18)
+//      65 tiles  16 chunks  19.8 | alone 22.8    17  21.1 | 22.6    20  23.5 | 23.6    64  63.8 | 36.2
+//      96 tiles  17 chunks  21.2 | 25.1          20  23.6 | 26.3    24  27.4 | 28.2    64  64.1 | 39.4
+//     128 tiles  16 chunks  20.3 | alone 22.9    17  21.1 | 27.2    24  27.2 | 30.5    28  31.0 | 32.1    64  64.8 | 46.3
+//   parts of 48 chunks, up to cus tiles, where a second workgroup per compute unit is all there is to gain
+//     192 tiles  32 chunks  35.1 | alone 38.2    49  51.8 | 52.0    64  67.3 | 62.4   128 125.5 | 107.5
+//     256 tiles  48 chunks  55.9 | alone 58.0    49  56.9 | 62.0    64  72.7 | 74.8   128 135.3 | 130.1   256  288 | 239
+// From 257 tiles on every slot has work.  Sk below 32 chunks is not shared, whatever the lists (32 chunks, Sk = 2048: 8 tiles
+// 33.6 | 17.0, 64 tiles 34.7 | 26.3, 128 tiles 35.2 | 33.6; 16 chunks: the tables above, as lists of a longer Sk).
 // float32: a chunk of 32 keys keeps the matrix unit busy for 1.7 us (D = 64) or 3.4 us, so two chunks are worth a part
-// (32 tiles of 16 chunks at D = 64: 46 -> 16 us, 256 of 32 at D = 128: 158 -> 95 us).  There the keys of a row are added
-// up one after the other, which costs 1.2e-6 of the result at 4096 keys and 3.3e-6 at 32768, shared lists 4e-7 and
-// 7e-7; longer rows than 4096 keys stay with the one order of addition, so that a result does not move by more than
-// float32 sums may (1.5e-6).
-void fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus, int *nsplit, int *split_chunks) {
-    *nsplit = 1;
-    *split_chunks = 1 << 30;
-    if (D > 128 || (BQ != 32 && BQ != 64 && BQ != 128) || (dtype == 2 && ((D == 128 && BQ == 32) || Sk > 4096))) return;
+// (32 tiles of 16 chunks at D = 64: 46 -> 16 us, 256 of 32 at D = 128: 158 -> 95 us).  Sk above 4096 is not shared there: a row's
+// keys are added up one after the other in one workgroup, 1.2e-6 from the result at 4096 keys and 3.3e-6 at 32768, and shared
+// lists (4e-7 and 7e-7) would move the result by that much.
+FwdSplitPlan fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus) {
+    FwdSplitPlan plan;
+    if (D > 128 || (BQ != 32 && BQ != 64 && BQ != 128) || (dtype == 2 && ((D == 128 && BQ == 32) || Sk > 4096))) return plan;
     const int lck = dtype == 2 ? 5 : 6;
     const int chunks = (Sk + (1 << lck) - 1) >> lck;  // of the longest list there can be
     const int part = dtype == 2 ? 2 : (4 * tiles <= cus ? 8 : (2 * tiles <= cus ? 16 : 48));
     const int most = 2 * cus / tiles, parts = (chunks + part - 1) / part;
     const int n = parts < most ? parts : most;
-    if (n < 2 || chunks < (dtype == 2 ? 4 : 32)) return;
-    *nsplit = n < 32 ? n : 32;
-    *split_chunks = part;
+    if (n < 2 || chunks < (dtype == 2 ? 4 : 32)) return plan;
+    plan.nsplit = n < 32 ? n : 32;
+    plan.chunks = part;
+    plan.least = part == 16 ? 8 + tiles / 8 : part;
+    return plan;
 }
 
 hipError_t launch_fwd_merge(const FwdParams &p, int dtype, int D, int BQ, hipStream_t stream) {

@@ -255,18 +255,17 @@ size_t schedule_shape(int B, int H, int Sq, int Sk, int BQ, int BK, int mode, in
     return (size_t)G * (size_t)(R + 1) * 16;
 }
 
-// Parts of a shared list and chunks per part on the current device (1: no sharing), and the bytes of the partial results.
-size_t split_shape(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype, int *nsplit, int *split_chunks) {
-    *nsplit = 1;
-    *split_chunks = 1 << 30;
+// How lists are shared on the current device, and the bytes of the partial results (0: they are not).
+size_t split_shape(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype, sa::FwdSplitPlan *plan) {
+    *plan = sa::FwdSplitPlan();
     if (B <= 0 || H <= 0 || Sq <= 0 || Sk <= 0 || BQ <= 0 || BK <= 0 || Sq % BQ || Sk % BK || log2_exact(BK) < 4) return 0;
     const int64_t tiles = (int64_t)B * H * (Sq / BQ);
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
     if (tiles > 2 * cus) return 0;
-    sa::fwd_split_plan((int)tiles, Sk, BQ, D, dtype, cus, nsplit, split_chunks);
-    return *nsplit > 1 ? (size_t)tiles * (size_t)*nsplit * (size_t)BQ * (size_t)(D + 2) * 4 : 0;
+    *plan = sa::fwd_split_plan((int)tiles, Sk, BQ, D, dtype, cus);
+    return plan->nsplit > 1 ? (size_t)tiles * (size_t)plan->nsplit * (size_t)BQ * (size_t)(D + 2) * 4 : 0;
 }
 
 // Tensors that are smaller than the tile grid of their mask (FwdParams::ragged).
@@ -412,7 +411,11 @@ int forward_impl(const void *q, const int64_t q_strides[4], const void *k, const
     }
     fp.nsplit = 1;
     if (workspace && kernel == SA_FWD_KERNEL_DEFAULT && !fp.sched) {
-        const size_t need = split_shape(B, H, Sq, Sk, D, BQ, BK, dtype, &fp.nsplit, &fp.split_chunks);
+        sa::FwdSplitPlan plan;
+        const size_t need = split_shape(B, H, Sq, Sk, D, BQ, BK, dtype, &plan);
+        fp.nsplit = plan.nsplit;
+        fp.split_chunks = plan.chunks;
+        fp.split_least = plan.least;
         if (need != 0 && (workspace_bytes < need || !aligned(workspace, 16)))
             return fail(SA_ERR_WORKSPACE, "sa_sparse_attention_fwd_split: a 16-byte aligned workspace of %zu bytes required, %zu given", need, workspace_bytes);
         fp.ws = static_cast<float *>(workspace);
@@ -535,9 +538,9 @@ int sa_sparse_attention_fwd_kernel(const void *q, const int64_t q_strides[4], co
 }
 
 size_t sa_fwd_split_workspace_bytes(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype) {
-    int nsplit, split_chunks;
+    sa::FwdSplitPlan plan;
     if ((D != 64 && D != 128) || dtype < SA_DTYPE_BF16 || dtype > SA_DTYPE_FP32) return 0;
-    return split_shape(B, H, Sq, Sk, D, BQ, BK, dtype, &nsplit, &split_chunks);
+    return split_shape(B, H, Sq, Sk, D, BQ, BK, dtype, &plan);
 }
 
 int sa_sparse_attention_fwd_split(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],

@@ -71,3 +71,19 @@ def test_caller_lists_are_clamped_in_shared_lists(gpu):
     clean[..., 20 * BK:21 * BK] = False
     want = torch.nn.functional.scaled_dot_product_attention(q.float(), k.float(), v.float(), attn_mask=clean)
     assert float((got.float() - want).abs().max()) <= 2e-2
+
+
+@pytest.mark.parametrize("tiles,chunks", [(65, 16), (96, 20), (128, 17), (128, 24)])
+def test_lists_too_short_to_be_shared(gpu, tiles, chunks):
+    """Half the device's slots taken: two workgroups beside each other are no faster on such a list than one (results as
+    of one, bit for bit)."""
+    B, H, D, BQ, BK, Sk = 1, 1, 128, 128, 64, 8192
+    q, _, _ = W.qkv(B, H, BQ * tiles, D, torch.bfloat16, seed=3, device=gpu)
+    _, k, v = W.qkv(B, H, Sk, D, torch.bfloat16, seed=4, device=gpu)
+    mask = (torch.arange(Sk, device=gpu) >= Sk - BK * chunks).expand(B, H, BQ * tiles, Sk)
+    md = compute_mask_kernel(mask, BQ, BK)
+    assert _native.load().sa_fwd_split_workspace_bytes(B, H, BQ * tiles, Sk, D, BQ, BK, 0) > 0
+    got = sparse_attention(q, k, v, None, BQ, BK, md)
+    many = torch.cat([q] * 4, 2)  # (enough Q tiles to fill the device: nothing is shared)
+    more = compute_mask_kernel(mask[:, :, :1].expand(B, H, 4 * BQ * tiles, Sk), BQ, BK)
+    assert torch.equal(got, sparse_attention(many, k, v, None, BQ, BK, more)[:, :, :BQ * tiles])
