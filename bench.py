@@ -48,18 +48,18 @@ PEAK_FP32_TFLOPS = 157.3   # MI355X dense fp32 MFMA peak, TFLOP/s
 # `bench.py --traffic-probe` and scaled by what the same counters read for the 1 GiB device copy of the same run
 # (`bench.py --traffic-summary` does the arithmetic).  profiles/hbm_traffic_all_kernels.txt holds the commands.
 TRAFFIC_BYTES = {
-    "forward, causal": (854423687, 268435456),
-    "forward, dense": (808001455, 268435797),
-    "forward, p=0.25": (1347283834, 268435456),
-    "forward, p=0.5": (2861761172, 268435456),
-    "forward, p=0.75": (2934045149, 268435456),
-    "forward, p=0.9": (1414350219, 268435456),
-    "backward, causal": (8130115082, 5242880213),
-    "forward, documents": (1723502198, 536870912),
-    "forward, composed": (1613264454, 268440320),
-    "mask_classify, composed mask 1 GiB": (1074098083, 308736),
-    "decode, 1": (4295523998, 344064),
-    "decode, 16": (1617158640, 5308587),
+    "forward, causal": (852370416, 268435456),
+    "forward, dense": (808004591, 268436267),
+    "forward, p=0.25": (1355455323, 268435456),
+    "forward, p=0.5": (2852664399, 268435456),
+    "forward, p=0.75": (2933578494, 268435456),
+    "forward, p=0.9": (1418451520, 268435456),
+    "backward, causal": (8119310878, 5242880171),
+    "forward, documents": (1725412717, 536870912),
+    "forward, composed": (1628726469, 268435456),
+    "mask_classify, composed mask 1 GiB": (1074097997, 308736),
+    "decode, 1": (4295522505, 344064),
+    "decode, 16": (1617160474, 5308416),
 }
 TRAFFIC_SOURCE = "profiles/hbm_traffic_all_kernels.txt"
 # The sources each kernel is built from.  The counters were read with kernels built from sources of the digests in
@@ -71,8 +71,8 @@ KERNEL_FILES = {
     "decode": ("sparse_decode.hip", "fwd_common.h", "kernels.h"),
     "backward": ("sparse_bwd.hip", "fwd_common.h", "kernels.h"),
 }
-TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "94c7ca3577a858fc", "mask_classify": "ae1679520463a44b", "decode": "9ae1240b96559893",
-                                "backward": "560c0c46d711d9f9"}
+TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "9bd94683c78ce4fc", "mask_classify": "830b3fd448915572", "decode": "c64f677817bb3a89",
+                                "backward": "d4e8132a37e81df4"}
 
 
 def kernel_sources_sha16(which=None):
@@ -604,6 +604,7 @@ def power_trace(seconds):
         time.sleep(0.3)  # (a gap in the samples between workloads)
 
     masks = [("causal", W.causal_mask(S, "cuda")), ("dense", torch.ones(S, S, dtype=torch.bool, device="cuda")),
+             ("random blocks p=0.75", W.random_block_mask(S, 128, 0.75, seed=75, device="cuda")),
              ("random blocks p=0.9", W.random_block_mask(S, 128, 0.9, seed=90, device="cuda")),
              ("no tile attended (q read, zeros written)", torch.zeros(S, S, dtype=torch.bool, device="cuda"))]
     for name, m in masks:

@@ -5,7 +5,12 @@
 // log-sum-exp the forward hands out (FwdParams::lse):
 //     P = exp(S - lse),  dV = P^T dO,  dP = dO V^T,  dS = P o (dP - rowsum(dO o O)),  dQ = scale dS K,  dK = scale dS^T Q.
 //
-// One kernel serves the three gradients.  A workgroup owns a tile of 128 RESIDENT rows (queries for dQ, keys for dK
+// Three ways to the gradients, by head dim and size (launch_bwd):
+//   D = 64                      sparse_bwd_kernel: a pass for dK and dV together and one for dQ, in one launch
+//   D = 128                     sparse_bwd_kernel: a pass each for dK, dQ and dV, in one launch
+//   D = 128, bwd_ds_group > 0   sparse_bwd_keys_kernel: dK, dV and dS from one pass over the keys, dS stored;
+//                               sparse_bwd_queries_kernel: dQ from the stored dS (bwd_dq_tile)
+// All but the last are forms of bwd_tile.  A workgroup owns a tile of 128 RESIDENT rows (queries for dQ, keys for dK
 // and dV), 32 per wave, whose operands stay in registers, and walks the list of 64-row tiles of the STREAMED side
 // (keys for dQ, queries for dK/dV) that the mask leaves for it: FULL tiles, then PARTIAL ones, as in the forward; for
 // dK/dV the lists are those of the transposed mask.  Per 32 streamed rows:
@@ -16,8 +21,7 @@
 // are streamed.  Streamed chunks of 64 rows arrive by direct loads global -> LDS in two stages, one barrier per chunk.
 // A chunk buffer is read both ways - row-wise as MFMA A operand (ds_read_b128) and transposed (ds_read_b64_tr_b16) -
 // so the 16-byte pieces of a row are swizzled with a function of the row that keeps both patterns free of bank
-// conflicts (bwd_swizzle).  Where there is enough work at D = 128 the pass over the keys makes dK, dV and dS at once and
-// dQ is made from the stored dS (bwd_ds_group, bwd_dq_tile).
+// conflicts (bwd_swizzle).
 #include "fwd_common.h"
 
 namespace sa {
@@ -54,7 +58,7 @@ constexpr int kDQ = 0;   // queries resident
 constexpr int kDK = 1;   // keys resident, as for the following
 constexpr int kDV = 2;
 constexpr int kDKV = 3;  // both from one walk: S and P once instead of twice (D = 64, where two accumulators leave room for
-                         // two waves per SIMD)
+                         // more waves per SIMD, and D = 128 where dS is stored)
 
 // LDS, two stages of each: [Y][Z][stats: 64 L then 64 Delta floats][mask: 8 bytes per resident row][list]
 template <int D, bool PK>

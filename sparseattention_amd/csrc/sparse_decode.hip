@@ -459,6 +459,12 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(const DecodeParams p)
 // reads of each are in flight.  The parts lie in a cache and are few: all of this is latency, and the kernel above, which
 // walks them one after the other, took most of a call with many (bf16, D = 128, Sq1; classification, decode and merge):
 // 128 parts (B1 H4 Sk32768) 76.9 -> 19.5 us, 22 parts (B2 H12 Sq4 Sk8192) 40.6 -> 31.1, 16 parts (B1 H32 Sk32768) 78.7 -> 72.5.
+// Around the line (decode and merge in a graph, us, kernel above | this one):
+//   parts                2             4             5             6             8             9            16
+//   B1 H8  Sq1  Sk4096   30.3 | 30.9   20.2 | 19.7   18.9 | 17.8   18.9 | 17.3   17.5 | 14.8   17.8 | 14.5   18.5 | 12.0
+//   B4 H16 Sq1  Sk4096   39.8 | 40.6   28.6 | 28.2   34.6 | 33.3   32.3 | 30.3   30.9 | 27.8   36.7 | 33.4   39.2 | 31.6
+//   B4 H8  Sq16 Sk4096   39.1 | 39.8   26.0 | 25.4   24.1 | 23.0   23.1 | 21.3   22.6 | 19.6   26.9 | 23.7   28.0 | 20.5
+// so from five parts on this one is faster at these sizes; the line stands at eight, where the order of the sum has been so far.
 // With 2 ... 4 parts the exchanges between lanes cost more than they save: 2 parts (B1 H8 Sk512) 12.5 -> 14.4, 4 parts (B8 H16
 // Sq32 Sk1024) 26.3 -> 29.6.
 constexpr int kMergeFew = 8;
