@@ -38,7 +38,7 @@
 extern "C" {
 #endif
 
-#define SA_ABI_VERSION 17
+#define SA_ABI_VERSION 18
 
 enum sa_status {
     SA_OK = 0,
@@ -361,8 +361,11 @@ int sa_sparse_attention_fwd_kernel(const void *q, const int64_t q_strides[4], co
  *               which says that the launch has no use for it (the call is then sa_sparse_attention_fwd_kernel with the
  *               default kernel).  The bytes depend on the current device.
  * Results agree with the default kernel within rounding (a row's keys are added up in other groups).
+ * sa_fwd_split_least_keys: lists of up to that many keys are walked by one workgroup all the same (Sk where all are); a caller
+ * who knows that no list is longer does without the workspace and saves the second launch.
  */
 size_t sa_fwd_split_workspace_bytes(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype);
+int sa_fwd_split_least_keys(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype);
 int sa_sparse_attention_fwd_split(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
                                   const void *v, const int64_t v_strides[4], void *o, const int64_t o_strides[4],
                                   const uint8_t *mask, const int64_t mask_strides[4], const int32_t *full_ids,

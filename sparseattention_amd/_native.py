@@ -10,7 +10,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libsparseattn_hip.so")
 
-SA_ABI_VERSION = 17
+SA_ABI_VERSION = 18
 SA_OK = 0
 SA_ERR_INVALID_ARGUMENT = -1
 SA_ERR_UNSUPPORTED = -2
@@ -46,6 +46,7 @@ EXPORTS = (
     "sa_sparse_attention_fwd_lse",
     "sa_sparse_attention_fwd_kernel",
     "sa_fwd_split_workspace_bytes",
+    "sa_fwd_split_least_keys",
     "sa_sparse_attention_fwd_split",
     "sa_sparse_attention_fwd_ragged",
     "sa_decode_num_splits",
@@ -139,6 +140,8 @@ def load() -> ctypes.CDLL:
     )
     lib.sa_fwd_split_workspace_bytes.restype = ctypes.c_size_t
     lib.sa_fwd_split_workspace_bytes.argtypes = [ctypes.c_int] * 8
+    lib.sa_fwd_split_least_keys.restype = ctypes.c_int
+    lib.sa_fwd_split_least_keys.argtypes = [ctypes.c_int] * 8
     lib.sa_sparse_attention_fwd_split.restype = ctypes.c_int
     lib.sa_sparse_attention_fwd_split.argtypes = (
         [_vp, _i64p] * 4 + [_vp, _i64p] + [_vp, _i64p] * 4 + [_vp, _i64p] + [_vp, _i64p] + [ctypes.c_int] * 8

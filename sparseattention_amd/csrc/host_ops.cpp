@@ -472,7 +472,9 @@ std::optional<Out> forward_impl(const Tensor &q, const Tensor &k, const Tensor &
                                                 ptr<float>(lse), st(lse), B, H, Sq, Sk, Dk, BQ, BK, dt, scale, code, stream));
     } else {
         // (too few Q tiles to fill the device: their lists are shared by several workgroups, which need a workspace)
-        const size_t ws_bytes = sa_fwd_split_workspace_bytes(B, H, Sq, Sk, Dk, BQ, BK, dt);
+        size_t ws_bytes = sa_fwd_split_workspace_bytes(B, H, Sq, Sk, Dk, BQ, BK, dt);
+        // (metadata that says that no list is long enough: 128 tiles of 16 chunks 22.9 -> 20.0 us, no merge that finds nothing)
+        if (ws_bytes && hints.stats && hints.longest_list * BK <= sa_fwd_split_least_keys(B, H, Sq, Sk, Dk, BQ, BK, dt)) ws_bytes = 0;
         Tensor ws;
         if (ws_bytes) ws = at::empty({(int64_t)(ws_bytes / 4)}, opt_f32);
         check_rc(sa_sparse_attention_fwd_split(qc.data_ptr(), st(qc), kc.data_ptr(), st(kc), vc.data_ptr(), st(vc), o.data_ptr(), st(o),

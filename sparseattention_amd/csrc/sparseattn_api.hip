@@ -543,6 +543,12 @@ size_t sa_fwd_split_workspace_bytes(int B, int H, int Sq, int Sk, int D, int BQ,
     return split_shape(B, H, Sq, Sk, D, BQ, BK, dtype, &plan);
 }
 
+int sa_fwd_split_least_keys(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype) {
+    sa::FwdSplitPlan plan;
+    if ((D != 64 && D != 128) || dtype < SA_DTYPE_BF16 || dtype > SA_DTYPE_FP32 || split_shape(B, H, Sq, Sk, D, BQ, BK, dtype, &plan) == 0) return Sk;
+    return plan.least << (dtype == SA_DTYPE_FP32 ? 5 : 6);  // (a plan's lists may be longer than this: less than Sk)
+}
+
 int sa_sparse_attention_fwd_split(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
                                   const void *v, const int64_t v_strides[4], void *o, const int64_t o_strides[4],
                                   const uint8_t *mask, const int64_t mask_strides[4], const int32_t *full_ids,

@@ -87,3 +87,22 @@ def test_lists_too_short_to_be_shared(gpu, tiles, chunks):
     many = torch.cat([q] * 4, 2)  # (enough Q tiles to fill the device: nothing is shared)
     more = compute_mask_kernel(mask[:, :, :1].expand(B, H, 4 * BQ * tiles, Sk), BQ, BK)
     assert torch.equal(got, sparse_attention(many, k, v, None, BQ, BK, more)[:, :, :BQ * tiles])
+
+
+@pytest.mark.parametrize("keys", [512, 576])
+def test_no_parts_where_the_metadata_says_that_no_list_is_long(gpu, keys):
+    B, H, Sq, Sk, D, BQ, BK = 1, 4, 128, 8192, 64, 128, 64
+    q, _, _ = W.qkv(B, H, Sq, D, torch.bfloat16, seed=3, device=gpu)
+    _, k, v = W.qkv(B, H, Sk, D, torch.bfloat16, seed=4, device=gpu)
+    mask = (torch.arange(Sk, device=gpu) >= Sk - keys).expand(B, H, Sq, Sk)
+    md = compute_mask_kernel(mask, BQ, BK)
+    want = sparse_attention(q, k, v, None, BQ, BK, md)
+    taken = _native.load().sa_fwd_split_workspace_bytes(B, H, Sq, Sk, D, BQ, BK, 0)
+    assert taken > 0
+    md = compute_mask_kernel(mask, BQ, BK, list_stats=True)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    got = sparse_attention(q, k, v, None, BQ, BK, md)
+    assert (torch.cuda.max_memory_allocated() - before < taken) == (keys == 512)  # (lists of eight chunks and of nine)
+    assert torch.equal(got, want)
