@@ -82,6 +82,9 @@ Tensor kernel_ready(const Tensor &t) {
     for (int64_t d = 0; d + 1 < t.dim(); d++) ok = ok && t.stride(d) % per16 == 0;
     return ok ? t : t.contiguous();
 }
+// The head dim the kernels run a request for D with: the smallest that holds it (q, k, v are then padded with zero columns,
+// which change neither the scores nor the first D columns of the result; the softmax scale stays that of D).  A D beyond
+// all of them is passed on, for the library to refuse.
 int64_t kernel_head_dim(int64_t D, bool has256) { return D <= 64 ? 64 : D <= 128 ? 128 : has256 && D <= 256 ? 256 : D; }
 Tensor pad_head_dim(const Tensor &t, int64_t Dk) {
     return t.size(-1) == Dk ? t : at::constant_pad_nd(t, {0, Dk - t.size(-1)});
@@ -741,5 +744,6 @@ PYBIND11_MODULE(_host, m) {
     m.def("classify_terms", &classify_terms);
     m.def("backward", &backward);
     m.def("backward_workspace_bytes", &backward_workspace_bytes);
+    m.def("kernel_head_dim", &kernel_head_dim);
     m.def("trainable", &trainable);
 }

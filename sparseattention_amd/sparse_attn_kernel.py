@@ -12,13 +12,6 @@ from .mask_utils import MaskMetadata, Tiling, compute_mask_kernel, compute_mask_
 _DTYPES = {torch.bfloat16: _native.SA_DTYPE_BF16, torch.float16: _native.SA_DTYPE_FP16}
 
 
-def _kernel_head_dim(D: int, sizes) -> int:
-    """The head dim the kernels run a request for ``D`` with: the smallest of ``sizes`` that holds it (q, k, v are then
-    padded with zero columns, which change neither the scores nor the first D columns of the result; the softmax scale
-    stays that of D).  A D beyond all of them is passed on, for the library to refuse."""
-    return next((s for s in sizes if D <= s), D)
-
-
 def _pad_mask(mask: torch.Tensor, q_multiple: int, k_multiple: int) -> torch.Tensor:
     """``mask`` [B,H,Sq,Sk] with all-False rows and columns added up to multiples of the two numbers; only the
     distinct planes of a broadcast view are copied."""

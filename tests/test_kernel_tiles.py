@@ -1,7 +1,8 @@
 """Host logic that maps a request for tile sizes and head dims onto what the kernels have (no GPU)."""
 import pytest
 
-from sparseattention_amd.sparse_attn_kernel import _kernel_head_dim, kernel_tiles
+from sparseattention_amd import _native
+from sparseattention_amd.sparse_attn_kernel import kernel_tiles
 
 
 @pytest.mark.parametrize("args,want", [
@@ -28,6 +29,7 @@ def test_kernel_tiles(args, want):
 
 
 def test_kernel_head_dim():
-    sizes = (64, 128, 256)
-    assert [_kernel_head_dim(d, sizes) for d in (16, 64, 65, 96, 128, 192, 256)] == [64, 64, 128, 128, 128, 256, 256]
-    assert _kernel_head_dim(320, sizes) == 320  # passed on, for the library to refuse
+    of = _native.host().kernel_head_dim
+    assert [of(d, True) for d in (16, 64, 65, 96, 128, 192, 256)] == [64, 64, 128, 128, 128, 256, 256]
+    assert of(320, True) == 320  # passed on, for the library to refuse
+    assert [of(d, False) for d in (16, 64, 65, 128, 192)] == [64, 64, 128, 128, 192]  # few rows, backward: no 256
