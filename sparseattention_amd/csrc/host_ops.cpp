@@ -13,6 +13,7 @@
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPCachingAllocator.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/extension.h>
 
 #include <cmath>
@@ -719,9 +720,11 @@ struct AttentionFunction : public torch::autograd::Function<AttentionFunction> {
     }
 };
 
-// sparse_attention_trainable, or None where the wrapper has to pad or to make other tiles
+// sparse_attention_trainable, or None where the wrapper has to pad or to make other tiles.  Under torch.jit.trace too: a
+// trace records the wrapper's Python function as one step, of this one it would keep the allocations and not the launches.
 py::object trainable(const Tensor &q, const Tensor &k, const Tensor &v, const OptTensor &mask, int64_t BQ, int64_t BK, py::object md, py::object bmd) {
-    if (q.dim() != 4 || k.dim() != 4 || q.size(2) % 128 || k.size(2) % 128 || q.scalar_type() == at::kFloat || (bmd.is_none() && !mask))
+    if (q.dim() != 4 || k.dim() != 4 || q.size(2) % 128 || k.size(2) % 128 || q.scalar_type() == at::kFloat || (bmd.is_none() && !mask) ||
+        torch::jit::tracer::isTracing())
         return py::none();
     std::optional<Out> r;
     {

@@ -309,7 +309,7 @@ def sparse_attention_trainable(q, k, v, mask, BLOCK_Q, BLOCK_K, mask_metadata: M
     """:func:`sparse_attention` as a differentiable torch function (gradients for q, k, v through
     :func:`sparse_attention_backward`)."""
     out = _native.host().trainable(q, k, v, mask, int(BLOCK_Q), int(BLOCK_K), mask_metadata, bwd_metadata)
-    if out is None:  # sizes that the wrappers pad or tile anew
+    if out is None:  # sizes that the wrappers pad or tile anew, and under torch.jit.trace
         out = _SparseAttentionFunction.apply(q, k, v, mask, BLOCK_Q, BLOCK_K, mask_metadata, bwd_metadata)
     return out
 

@@ -49,3 +49,18 @@ def test_metadata_is_looked_at_in_the_backward(gpu):
     bmd.by_key.unmasked_lens.fill_(S)
     with pytest.raises(ValueError):
         torch.autograd.grad(o, (q, k, v), do)
+
+
+def test_trace(gpu):
+    """A trace keeps the call itself, so that other inputs and their gradients go through it."""
+    q, k, v, mask, do = case(gpu)
+    bmd = compute_backward_metadata(mask.expand(B, H, S, S))
+    call = lambda *t: sparse_attention_trainable(*t, mask, 128, 64, None, bmd)  # noqa: E731
+    traced = torch.jit.trace(call, (q, k, v))
+    other = tuple(t.requires_grad_(True) for t in W.qkv(B, H, S, D, torch.bfloat16, seed=4, device=gpu))
+    want = call(*other)
+    for _ in range(2):
+        got = traced(*other)
+        assert torch.equal(got, want)
+        grads = torch.autograd.grad(got, other, do)
+        assert all(torch.equal(a, b) for a, b in zip(grads, torch.autograd.grad(want, other, do, retain_graph=True)))
