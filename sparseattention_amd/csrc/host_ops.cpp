@@ -17,6 +17,7 @@
 #include <torch/extension.h>
 
 #include <cmath>
+#include <memory>
 #include <optional>
 #include <string>
 
@@ -101,9 +102,15 @@ struct Lists {
     OptTensor packed;
 };
 
-// Attribute of a metadata object: a new reference, or an empty object where there is none or it is None.
-py::object attr(py::handle o, const char *name) {
-    PyObject *v = PyObject_GetAttrString(o.ptr(), name);
+// Attribute of a metadata object: a new reference, or an empty object where there is none or it is None.  Names are interned
+// once, or every look-up would make a string and miss the type's cache of attributes.
+struct Name {
+    const char *text;
+    mutable PyObject *str = nullptr;
+};
+py::object attr(py::handle o, const Name &name) {
+    if (!name.str) name.str = PyUnicode_InternFromString(name.text);
+    PyObject *v = name.str ? PyObject_GetAttr(o.ptr(), name.str) : nullptr;
     if (!v) {
         if (!PyErr_ExceptionMatches(PyExc_AttributeError)) throw py::error_already_set();
         PyErr_Clear();
@@ -115,43 +122,43 @@ py::object attr(py::handle o, const char *name) {
     }
     return py::reinterpret_steal<py::object>(v);
 }
-Tensor tensor_attr(py::handle o, const char *name) {
+// (read under the interpreter's lock)
+const Name kFullIds{"unmasked_kv_ids"}, kFullLens{"unmasked_lens"}, kPartIds{"masked_kv_ids"}, kPartLens{"masked_lens"}, kPacked{"packed_masks"},
+    kValidatedFor{"_validated_for"}, kSchedule{"schedule"}, kScheduleMode{"schedule_mode"}, kListStats{"list_stats"}, kListRotation{"list_rotation"},
+    kByQuery{"by_query"}, kByKey{"by_key"}, kTransposedMask{"transposed_mask"}, kAgreeing{"_agreeing"};
+Tensor tensor_attr(py::handle o, const Name &name) {
     const py::object v = attr(o, name);
-    if (!v || !THPVariable_Check(v.ptr())) type_error(std::string("mask_metadata.") + name + " is not a tensor");
+    if (!v || !THPVariable_Check(v.ptr())) type_error(std::string("mask_metadata.") + name.text + " is not a tensor");
     return THPVariable_Unpack(v.ptr());
 }
-OptTensor opt_tensor_attr(py::handle o, const char *name) {
+OptTensor opt_tensor_attr(py::handle o, const Name &name) {
     const py::object v = attr(o, name);
     if (!v) return std::nullopt;
-    if (!THPVariable_Check(v.ptr())) type_error(std::string("mask_metadata.") + name + " is not a tensor");
+    if (!THPVariable_Check(v.ptr())) type_error(std::string("mask_metadata.") + name.text + " is not a tensor");
     return THPVariable_Unpack(v.ptr());
 }
 
 Lists lists_of(py::handle md) {
-    return {tensor_attr(md, "unmasked_kv_ids"), tensor_attr(md, "unmasked_lens"), tensor_attr(md, "masked_kv_ids"),
-            tensor_attr(md, "masked_lens"), opt_tensor_attr(md, "packed_masks")};
+    return {tensor_attr(md, kFullIds), tensor_attr(md, kFullLens), tensor_attr(md, kPartIds),
+            tensor_attr(md, kPartLens), opt_tensor_attr(md, kPacked)};
 }
 
 bool int_is(PyObject *o, unsigned long long want) { return (PyLong_Check(o) ? PyLong_AsUnsignedLongLongMask(o) : ~want) == want; }
 
-// Whether `key`, a mask_utils.validation_key, holds address and version counter of the four list tensors as they are.
-bool unedited(PyObject *key, const Lists &l) {
-    if (!PyTuple_Check(key) || PyTuple_GET_SIZE(key) != 6) return false;
+// Whether md._validated_for is mask_utils.validation_key(md, Sk, BK): the sizes, then address and version counter of the
+// four list tensors.
+bool validated(py::handle md, const Lists &l, int64_t Sk, int64_t BK) {
+    const py::object key = attr(md, kValidatedFor);
+    if (!key || !PyTuple_Check(key.ptr()) || PyTuple_GET_SIZE(key.ptr()) != 6) return false;
+    if (!int_is(PyTuple_GET_ITEM(key.ptr(), 0), (unsigned long long)Sk) || !int_is(PyTuple_GET_ITEM(key.ptr(), 1), (unsigned long long)BK)) return false;
     const Tensor *t[4] = {&l.fid, &l.fl, &l.pid, &l.pl};
     for (int i = 0; i < 4; i++) {
-        PyObject *e = PyTuple_GET_ITEM(key, 2 + i);
+        PyObject *e = PyTuple_GET_ITEM(key.ptr(), 2 + i);
         if (!PyTuple_Check(e) || PyTuple_GET_SIZE(e) != 2 || !int_is(PyTuple_GET_ITEM(e, 0), (unsigned long long)(uintptr_t)t[i]->data_ptr()) ||
             !int_is(PyTuple_GET_ITEM(e, 1), (unsigned long long)t[i]->_version()))
             return false;
     }
     return true;
-}
-
-// Whether md._validated_for is mask_utils.validation_key(md, Sk, BK).
-bool validated(py::handle md, const Lists &l, int64_t Sk, int64_t BK) {
-    const py::object key = attr(md, "_validated_for");
-    return key && unedited(key.ptr(), l) && int_is(PyTuple_GET_ITEM(key.ptr(), 0), (unsigned long long)Sk) &&
-           int_is(PyTuple_GET_ITEM(key.ptr(), 1), (unsigned long long)BK);
 }
 void checked_metadata(py::handle md, const Lists &l, int64_t Sk, int64_t BK) {
     if (!validated(md, l, Sk, BK))
@@ -356,15 +363,15 @@ struct Hints {
 };
 Hints hints_of(py::handle md) {
     Hints h;
-    h.sched = opt_tensor_attr(md, "schedule");
+    h.sched = opt_tensor_attr(md, kSchedule);
     if (h.sched)
-        if (const py::object m = attr(md, "schedule_mode")) h.sched_mode = m.cast<int>();
-    if (const py::object s = attr(md, "list_stats")) {
+        if (const py::object m = attr(md, kScheduleMode)) h.sched_mode = m.cast<int>();
+    if (const py::object s = attr(md, kListStats)) {
         h.stats = true;
         h.mean_list = s[py::int_(0)].cast<double>();
         h.longest_list = s[py::int_(1)].cast<int64_t>();
     }
-    if (const py::object r = attr(md, "list_rotation")) h.rotation = r.cast<int64_t>();
+    if (const py::object r = attr(md, kListRotation)) h.rotation = r.cast<int64_t>();
     return h;
 }
 
@@ -389,7 +396,7 @@ int choose_kernel(const std::string &kernel, bool f32, int64_t Dk, int64_t BQ, i
 }
 // The same by name ("default", "short" or "rotated"), for reports on what a call with this metadata runs.
 std::string forward_kernel(const Tensor &q, int64_t BQ, int64_t BK, py::object md, const std::string &kernel) {
-    const bool packed = (bool)attr(md, "packed_masks");
+    const bool packed = (bool)attr(md, kPacked);
     const int code = choose_kernel(kernel, q.scalar_type() == at::kFloat, kernel_head_dim(q.size(-1), true), BQ, BK, packed, hints_of(md)) & 0xff;
     return code == SA_FWD_KERNEL_SHORT_LISTS ? "short" : code == SA_FWD_KERNEL_ROTATED ? "rotated" : "default";
 }
@@ -425,7 +432,7 @@ std::optional<Out> forward_impl(const Tensor &q, const Tensor &k, const Tensor &
         type_error(std::string("q, k, v must share dtype bfloat16, float16 or float32 (got ") + c10::toString(q.scalar_type()) + ", " +
                    c10::toString(k.scalar_type()) + ", " + c10::toString(v.scalar_type()) + ")");
     const bool f32 = dt == SA_DTYPE_FP32, has_md = !md.is_none();
-    if (!mask_in && !(has_md && attr(md, "packed_masks")))
+    if (!mask_in && !(has_md && attr(md, kPacked)))
         value_error("sparse_attention without a mask tensor needs mask_metadata with packed_masks");
     OptTensor mask = mask_in;
     if (mask) mask = mask->expand({B, H, Sq, Sk});
@@ -502,7 +509,7 @@ py::object forward_tiled(const Tensor &q, const Tensor &k, const Tensor &v, int6
     check_qkv(q, k, v, std::nullopt, "sparse_attention");
     if (k.scalar_type() != q.scalar_type() || v.scalar_type() != q.scalar_type() || BQ < 1 || BK < 1 || Pq % BQ || Pk % BK) return py::none();
     const Lists l = lists_of(md);
-    if (!ragged_has(q, BQ, BK, l) || attr(md, "schedule")) return py::none();
+    if (!ragged_has(q, BQ, BK, l) || attr(md, kSchedule)) return py::none();
     check_lists(l, q, q.size(0), q.size(1), Pq / BQ, Pk / BK, "tiling.metadata");
     checked_metadata(md, l, Pk, BK);
     check_packed(*l.packed, q, q.size(0), q.size(1), Pq / BQ, Pk / BK, BQ * BK / 8, "tiling.metadata");
@@ -522,45 +529,91 @@ struct BackwardLists {
     bool agree = false;  // both are known to say the same of every entry
 };
 
-// Whether the ten tensors are the ones, unedited, that this package made of one mask: bmd._agreeing holds them, with the
-// addresses and in-place versions they had then, and keeps them alive, so that nothing else can stand in their place.
-bool lists_agree(py::handle bmd, const BackwardLists &l) {
-    const py::object made = attr(bmd, "_agreeing");
-    if (!made || !PyTuple_Check(made.ptr()) || PyTuple_GET_SIZE(made.ptr()) != 2) return false;
-    for (int i = 0; i < 2; i++) {
-        const Lists &a = i ? l.by_key : l.by_query;
-        PyObject *const e = PyTuple_GET_ITEM(made.ptr(), i);
-        if (!a.packed || !PyTuple_Check(e) || PyTuple_GET_SIZE(e) != 8) return false;
-        const Tensor *const t[5] = {&a.fid, &a.fl, &a.pid, &a.pl, &*a.packed};
-        for (int j = 0; j < 5; j++) {
-            PyObject *const o = PyTuple_GET_ITEM(e, j);
-            if (!THPVariable_Check(o) || THPVariable_Unpack(o).unsafeGetTensorImpl() != t[j]->unsafeGetTensorImpl() || t[j]->is_inference()) return false;
-        }
-        if (!unedited(PyTuple_GET_ITEM(e, 5), a) || !int_is(PyTuple_GET_ITEM(e, 6), (unsigned long long)(uintptr_t)a.packed->data_ptr()) ||
-            !int_is(PyTuple_GET_ITEM(e, 7), (unsigned long long)a.packed->_version()))
-            return false;
+// The note that a BackwardMetadata carries (_agreeing) when this package made both its lists of one mask: the ten tensors, with
+// the addresses and in-place versions they had then.  It keeps them alive, so that nothing else can stand in their place.
+// Native, and looked at without a reference taken to any of them, its lists used as they stand: the backward does so on the
+// autograd thread, where every object whose count of references changes is a cache line that the two threads take from
+// each other.
+const Name *const kListNames[5] = {&kFullIds, &kFullLens, &kPartIds, &kPartLens, &kPacked};
+struct OneMask {
+    BackwardLists lists;
+    struct {
+        py::object object;
+        const void *data;
+        int64_t version;
+    } was[10];
+
+    const Tensor &tensor(int i) const {
+        const Lists &l = i < 5 ? lists.by_query : lists.by_key;
+        const Tensor *const t[5] = {&l.fid, &l.fl, &l.pid, &l.pl, &*l.packed};
+        return *t[i % 5];
     }
-    return true;
+};
+// (None for lists without packed tiles, which no path needs it for, and for tensors that do not count their edits)
+std::shared_ptr<OneMask> of_one_mask(py::object by_query, py::object by_key) {
+    auto n = std::make_shared<OneMask>();
+    n->lists = {lists_of(by_query), lists_of(by_key), std::nullopt, true};
+    if (!n->lists.by_query.packed || !n->lists.by_key.packed) return nullptr;
+    for (int i = 0; i < 10; i++) {
+        const Tensor &t = n->tensor(i);
+        if (t.is_inference()) return nullptr;
+        n->was[i] = {attr(i < 5 ? by_query : by_key, *kListNames[i % 5]), t.data_ptr(), (int64_t)t._version()};
+    }
+    return n;
+}
+// The note of bmd where its lists are still those tensors, unedited, or nothing.
+std::shared_ptr<OneMask> lists_agree(py::handle bmd, py::handle by_query, py::handle by_key) {
+    const py::object made = attr(bmd, kAgreeing);
+    if (!made || !py::isinstance<OneMask>(made)) return nullptr;
+    auto n = made.cast<std::shared_ptr<OneMask>>();
+    for (int l = 0; l < 2; l++) {
+        const py::object dict = py::reinterpret_steal<py::object>(PyObject_GenericGetDict((l ? by_key : by_query).ptr(), nullptr));
+        if (!dict || !PyDict_Check(dict.ptr())) {
+            PyErr_Clear();
+            return nullptr;
+        }
+        for (int i = 5 * l; i < 5 * l + 5; i++) {
+            const Tensor &t = n->tensor(i);
+            if (PyDict_GetItem(dict.ptr(), kListNames[i % 5]->str) != n->was[i].object.ptr() || t.data_ptr() != n->was[i].data ||
+                (int64_t)t._version() != n->was[i].version)
+                return nullptr;
+        }
+    }
+    return n;
 }
 
-BackwardLists backward_lists_of(py::handle bmd, const Tensor &q, int64_t Sk) {
+// The lists of a BackwardMetadata: those of its note, or else its own.
+struct ReadLists {
+    std::shared_ptr<const OneMask> note;
+    BackwardLists own;
+    const BackwardLists &get() const { return note ? note->lists : own; }
+};
+ReadLists backward_lists_of(py::handle bmd, const Tensor &q, int64_t Sk) {
     const int64_t B = q.size(0), H = q.size(1), Sq = q.size(2);
-    const py::object mq = attr(bmd, "by_query"), mk = attr(bmd, "by_key");
+    const py::object mq = attr(bmd, kByQuery), mk = attr(bmd, kByKey);
     if (!mq || !mk) type_error("bwd_metadata has no by_query / by_key lists");
-    BackwardLists l{lists_of(mq), lists_of(mk), opt_tensor_attr(bmd, "transposed_mask"), false};
+    ReadLists r;
+    r.note = lists_agree(bmd, mq, mk);
+    const OptTensor mt = opt_tensor_attr(bmd, kTransposedMask);
+    if (!r.note || mt) {
+        r.own = {lists_of(mq), lists_of(mk), mt, r.note != nullptr};
+        r.note.reset();
+    }
+    const BackwardLists &l = r.get();
     check_lists(l.by_query, q, B, H, Sq / 128, Sk / 64, "bwd_metadata");
-    checked_metadata(mq, l.by_query, Sk, 64);
     check_lists(l.by_key, q, B, H, Sk / 128, Sq / 64, "bwd_metadata");
-    checked_metadata(mk, l.by_key, Sq, 64);
+    if (!r.note) {  // (lists of this package fit the sizes that their shapes have)
+        checked_metadata(mq, l.by_query, Sk, 64);
+        checked_metadata(mk, l.by_key, Sq, 64);
+    }
     if (l.by_query.packed) check_packed(*l.by_query.packed, q, B, H, Sq / 128, Sk / 64, 1024, "bwd_metadata");
     if (l.by_key.packed) check_packed(*l.by_key.packed, q, B, H, Sk / 128, Sq / 64, 1024, "bwd_metadata");
-    if (const OptTensor &mt = l.transposed_mask) {
+    if (mt) {
         const int64_t want[4] = {B, H, Sk, Sq};
         if (mt->sizes() != at::IntArrayRef(want, 4) || mt->scalar_type() != at::kBool || mt->device() != q.device())
             value_error("bwd_metadata.transposed_mask: expected bool " + str(at::IntArrayRef(want, 4)) + " on " + q.device().str());
     }
-    l.agree = lists_agree(bmd, l);
-    return l;
+    return r;
 }
 
 // The lists made from the mask itself (compute_backward_metadata with packed tiles; Sq and Sk multiples of 128).
@@ -655,13 +708,13 @@ py::object backward(const Tensor &do_, const Tensor &q, const Tensor &k, const T
     if (Sq % 128 || Sk % 128) return py::none();
     if (bmd.is_none() && !mask) value_error("sparse_attention_backward needs the mask or a BackwardMetadata with packed tiles");
     const bool has_bmd = !bmd.is_none();
-    BackwardLists l;
+    ReadLists l;
     if (has_bmd) l = backward_lists_of(bmd, q, Sk);
     std::tuple<Tensor, Tensor, Tensor> g;
     {
         const py::gil_scoped_release unlocked;
-        if (!has_bmd) l = backward_lists_from(*mask);
-        g = backward_impl(do_, q, k, v, o, lse, mask, l);
+        if (!has_bmd) l.own = backward_lists_from(*mask);
+        g = backward_impl(do_, q, k, v, o, lse, mask, l.get());
     }
     return py::make_tuple(std::get<0>(g), std::get<1>(g), std::get<2>(g));
 }
@@ -706,15 +759,15 @@ struct AttentionFunction : public torch::autograd::Function<AttentionFunction> {
             OptTensor mask;
             if (s[5].defined()) mask = s[5].expand({q.size(0), q.size(1), q.size(2), k.size(2)});
             check_backward(grads[0], q, k, s[2], s[3], s[4], mask);
-            BackwardLists l;
-            if (const auto it = ctx->saved_data.find("bwd_metadata"); it != ctx->saved_data.end()) {
-                const auto kept = it->second.toCapsule();
-                const py::gil_scoped_acquire gil;
-                l = backward_lists_of(static_cast<const Metadata &>(*kept).object, q, k.size(2));
-            } else {
-                l = backward_lists_from(*mask);
-            }
-            return backward_impl(grads[0], q, k, s[2], s[3], s[4], mask, l);
+            const auto run = [&](const BackwardLists &l) { return backward_impl(grads[0], q, k, s[2], s[3], s[4], mask, l); };
+            const auto it = ctx->saved_data.find("bwd_metadata");
+            if (it == ctx->saved_data.end()) return run(backward_lists_from(*mask));
+            const auto kept = it->second.toCapsule();
+            const py::gil_scoped_acquire gil;
+            // (let go of with the lock: tensors that the program has too would each take it for themselves)
+            const ReadLists l = backward_lists_of(static_cast<const Metadata &>(*kept).object, q, k.size(2));
+            const py::gil_scoped_release unlocked;
+            return run(l.get());
         });
         return {std::get<0>(g), std::get<1>(g), std::get<2>(g), Tensor(), Tensor(), Tensor()};
     }
@@ -739,6 +792,8 @@ py::object trainable(const Tensor &q, const Tensor &k, const Tensor &v, const Op
 
 PYBIND11_MODULE(_host, m) {
     m.doc() = "Checks, allocations and launches of the wrappers in sparse_attn_kernel.py and mask_utils.py.";
+    py::class_<OneMask, std::shared_ptr<OneMask>>(m, "OneMask");
+    m.def("of_one_mask", &of_one_mask);
     m.def("forward", &forward);
     m.def("forward_kernel", &forward_kernel);
     m.def("forward_tiled", &forward_tiled);

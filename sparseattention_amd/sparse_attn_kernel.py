@@ -225,9 +225,7 @@ class BackwardMetadata:
 
 def _of_one_mask(bmd: BackwardMetadata) -> BackwardMetadata:
     """Notes that both lists of ``bmd``, with packed tiles, were made from one mask."""
-    bmd._agreeing = tuple((md.unmasked_kv_ids, md.unmasked_lens, md.masked_kv_ids, md.masked_lens, md.packed_masks,
-                           md._validated_for, md.packed_masks.data_ptr(), md.packed_masks._version)
-                          for md in (bmd.by_query, bmd.by_key))
+    bmd._agreeing = _native.host().of_one_mask(bmd.by_query, bmd.by_key)
     return bmd
 
 

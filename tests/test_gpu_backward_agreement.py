@@ -57,3 +57,16 @@ def test_lists_changed_later(gpu, how):
     got = sparse_attention_backward(do, q, k, v, o, lse, None, bmd)
     want = sparse_attention_backward(do, q, k, v, o, lse, None, BackwardMetadata(bmd.by_query, bmd.by_key))
     assert all(torch.isfinite(x).all() and torch.equal(x, y) for x, y in zip(got, want))
+
+
+def test_lists_of_one_mask_with_a_transposed_mask_beside_them(gpu):
+    """The packed tiles are what is read, as without it; a transposed mask of other sizes is refused as ever."""
+    do, q, k, v, o, lse, mask = _inputs(gpu)
+    bmd = compute_backward_metadata(mask)
+    want = sparse_attention_backward(do, q, k, v, o, lse, None, bmd)
+    bmd.transposed_mask = mask.transpose(-1, -2).contiguous()
+    got = sparse_attention_backward(do, q, k, v, o, lse, None, bmd)
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
+    bmd.transposed_mask = mask[..., :128]
+    with pytest.raises(ValueError):
+        sparse_attention_backward(do, q, k, v, o, lse, None, bmd)
