@@ -407,12 +407,15 @@ int sa_sparse_attention_fwd_ragged(const void *q, const int64_t q_strides[4], co
  *   BK           power of two >= 16
  *   num_splits   workgroups per (b, h), 1..256, or 0 for sa_decode_num_splits(...)
  *   workspace    sa_decode_workspace_bytes(...) bytes of device memory, 16-byte aligned (may be NULL when that is 0,
- *                i.e. for one split); contents on return are unspecified
+ *                i.e. for one split); contents on return are unspecified.  With sa_decode_workspace_bytes_ex(...) bytes
+ *                (never fewer) the partial results are merged by the launch that makes them, to the same sums in another
+ *                order; contents on entry are unspecified either way
  *   lse, lse_strides   optional second output as in sa_sparse_attention_fwd_lse, or NULL
  * q, k, v, o, D, dtype, sm_scale_log2, stream: as for sa_sparse_attention_fwd.
  */
 int sa_decode_num_splits(int B, int H, int Sq, int Sk, int BK);
 size_t sa_decode_workspace_bytes(int B, int H, int Sq, int D, int num_splits);
+size_t sa_decode_workspace_bytes_ex(int B, int H, int Sq, int D, int num_splits);
 int sa_sparse_attention_decode(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
                                const void *v, const int64_t v_strides[4], void *o, const int64_t o_strides[4],
                                const uint8_t *mask, const int64_t mask_strides[4], const int32_t *full_ids,

@@ -51,6 +51,7 @@ EXPORTS = (
     "sa_sparse_attention_fwd_ragged",
     "sa_decode_num_splits",
     "sa_decode_workspace_bytes",
+    "sa_decode_workspace_bytes_ex",
     "sa_sparse_attention_decode",
     "sa_sparse_attention_decode_ex",
     "sa_decode_mask_fits",
@@ -132,6 +133,8 @@ def load() -> ctypes.CDLL:
     lib.sa_decode_num_splits.argtypes = [ctypes.c_int] * 5
     lib.sa_decode_workspace_bytes.restype = ctypes.c_size_t
     lib.sa_decode_workspace_bytes.argtypes = [ctypes.c_int] * 5
+    lib.sa_decode_workspace_bytes_ex.restype = ctypes.c_size_t
+    lib.sa_decode_workspace_bytes_ex.argtypes = [ctypes.c_int] * 5
     lib.sa_sparse_attention_decode.restype = ctypes.c_int
     lib.sa_sparse_attention_fwd_kernel.restype = ctypes.c_int
     lib.sa_sparse_attention_fwd_kernel.argtypes = (

@@ -103,7 +103,8 @@ constexpr float kNegInf = -__builtin_inff();
 // copy, and a build of that form ended in a GPU memory fault.
 // STREAM: the bytes are read once by the whole launch (the K/V rows of the few-rows kernels): the load carries the
 // non-temporal hint, with which a streaming read runs at 7.1 TB/s on this device against 6.3 TB/s without.
-template <bool STREAM = false>
+// DEVICE: what another workgroup of this launch has handed over (HandOver).
+template <bool STREAM = false, bool DEVICE = false>
 __device__ __forceinline__ void dma16(const void *base, uint32_t lane_offset, uint32_t lds_addr) {
     // the base is wave-uniform by construction; say so in a way the register allocator cannot miss
     const uint64_t b = (uint64_t)(uintptr_t)base;
@@ -111,7 +112,15 @@ __device__ __forceinline__ void dma16(const void *base, uint32_t lane_offset, ui
     const uint64_t ub = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b) |
                         ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) << 32);
     lds_addr = __builtin_amdgcn_readfirstlane(lds_addr);
-    if constexpr (STREAM) {
+    if constexpr (DEVICE) {
+        asm volatile(
+            "s_mov_b32 m0, %2\n\t"
+            "s_nop 0\n\t"
+            "global_load_lds_dwordx4 %0, %1 sc1"
+            :
+            : "v"(lane_offset), "s"(ub), "s"(lds_addr)
+            : "memory");
+    } else if constexpr (STREAM) {
         asm volatile(
             "s_mov_b32 m0, %2\n\t"
             "s_nop 0\n\t"
@@ -232,6 +241,60 @@ __device__ __forceinline__ int k_swizzle(int row) {
 template <int D>
 __device__ __forceinline__ int v_swizzle(int row) {
     return D >= 128 ? 4 * (row & 3) : 4 * ((row >> 1) & 1);
+}
+
+// Several workgroups leave parts of one result in memory; the last of them to arrive adds the parts up, in the same launch.
+// What one workgroup hands to another goes by stores and loads of device scope (sc1): they pass the L2 of their XCD by, so
+// nothing has to be written back or invalidated there, where other workgroups keep their operands (a release and an
+// acquire of device scope take 5.6 us of a workgroup, the counter alone 0.4).  512 workgroups, parts of 8 KiB of which four meet: stores
+// 1.6 us (0.9 where the four run on one XCD), counter 0.4, loads 1.2 ... 1.6.
+constexpr int kDeviceScope = 16;  // (the sc1 bit of a buffer instruction's modifiers)
+struct HandOver {
+    __amdgpu_buffer_rsrc_t rsrc;
+    // `bytes` (less than 2 GiB) from a wave-uniform base; accesses outside them do nothing
+    __device__ __forceinline__ HandOver(void *base, uint32_t bytes) {
+        const uint64_t b = (uint64_t)(uintptr_t)base;
+        const uint64_t ub = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b) |
+                            ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) << 32);
+        rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(uintptr_t)ub, 0, (int)bytes, 0x00027000);
+    }
+    __device__ __forceinline__ void put(uint32_t at, f32x4 x) const {
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, x), rsrc, (int)at, 0, kDeviceScope);
+    }
+    __device__ __forceinline__ void put(uint32_t at, f32x2 x) const {
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), rsrc, (int)at, 0, kDeviceScope);
+    }
+    __device__ __forceinline__ f32x4 get4(uint32_t at) const {
+        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)at, 0, kDeviceScope));
+    }
+    __device__ __forceinline__ f32x2 get2(uint32_t at) const {
+        return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)at, 0, kDeviceScope));
+    }
+};
+// One thread of each of n <= kArrivalMost workgroups, after what the workgroup hands over has been stored (every wave: vmcnt(0),
+// then a barrier): true for the last one.  The word needs no first value: its upper 56 bits are the launch's number
+// (next_launch_tag, no two launches of a process share one), its low 8 bits count.  A word with other upper bits, whatever the memory held, counts
+// as zero.  The last one leaves zero, so that a replay of a captured launch, which brings the same number, finds no count.
+constexpr int kArrivalMost = 255;
+__device__ __forceinline__ bool arrives_last(uint64_t *word, uint64_t tag, int n) {
+    uint64_t old = __hip_atomic_fetch_add(word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if ((old & ~0xffull) != tag) {
+        // (the count was added to what the memory held: harmless, and never more than n times)
+        uint64_t seen = old + 1;
+        for (;;) {
+            if ((seen & ~0xffull) == tag) {  // another one has put the number there meanwhile
+                old = __hip_atomic_fetch_add(word, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                break;
+            }
+            if (__hip_atomic_compare_exchange_strong(word, &seen, tag | 1ull, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+                old = tag;
+                break;
+            }
+        }
+    }
+    if ((int)(old & 0xff) + 1 != n) return false;
+    __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
 }
 
 // log2-domain slack before the running maximum is raised (and the accumulator rescaled).  Scores are

@@ -313,7 +313,7 @@ Out decode_impl(const Tensor &q, const Tensor &k, const Tensor &v, const OptTens
     const Tensor o = at::empty_like(qc);
     const auto f32 = at::TensorOptions().dtype(at::kFloat).device(q.device());
     if (num_splits == 0) num_splits = sa_decode_num_splits(B, H, Sq, Sk, BK);
-    const size_t ws_bytes = sa_decode_workspace_bytes(B, H, Sq, Dk, num_splits);
+    const size_t ws_bytes = sa_decode_workspace_bytes_ex(B, H, Sq, Dk, num_splits);
     Tensor ws;
     if (ws_bytes) ws = at::empty({(int64_t)(ws_bytes / 4)}, f32);
     OptTensor lse;

@@ -195,6 +195,7 @@ hipError_t launch_fwd_f32_mfma(const FwdParams &p, int D, int BQ, hipStream_t st
 // workgroup of the plane reads the whole mask, and a lane goes over a tile.
 constexpr int kDecodeDirectEntries = 32768;
 constexpr int kDecodeDirectBK = 256;
+constexpr int kDecodeMergeRows = 128;  // partial rows (parts x query rows) of a plane that its last workgroup merges: LDS holds them
 struct DecodeParams {
     const uint16_t *q, *k, *v;
     uint16_t *o;
@@ -211,6 +212,10 @@ struct DecodeParams {
     int64_t pks[2];  // bytes between packed planes along b and h
     int nsplit;     // workgroups per (b, h)
     float *ws;      // [B*H][nsplit][Sq][D + 2] floats: unnormalised rows, then reference value and row sum
+    // [B*H] words by which the last workgroup of a plane to arrive knows that it is the one to merge (arrives_last), or null:
+    // then a second launch merges.
+    uint64_t *arrivals;
+    uint64_t tag;   // the launch's number
     float scale;    // softmax scale / ln 2
     float *lse;     // optional second output as in FwdParams, or null
     int64_t lses[3];

@@ -22,11 +22,12 @@ namespace sa {
 namespace {
 
 constexpr int kDecodeWaves = 4;
+constexpr int kMergeFew = 8;  // parts up to which a row's are added up one after the other
 
 template <int D>
 constexpr int decode_smem_bytes() {
     constexpr int stream = kDecodeWaves * 2 * 32 * D * 2;         // per wave two V stages of 32 rows
-    constexpr int merge = kDecodeWaves * 32 * (D + 2) * 4;        // per wave 32 rows of D + 2 floats
+    constexpr int merge = kDecodeWaves * 32 * (D + 2) * 4 + 16;   // per wave 32 rows of D + 2 floats (kDecodeMergeRows)
     return stream > merge ? stream : merge;
 }
 
@@ -83,7 +84,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l32 = lane & 31, hh = lane >> 5;
-    const int split = blockIdx.x, bh = blockIdx.y;
+    const int bh = (int)(blockIdx.x / (unsigned)p.nsplit), split = (int)(blockIdx.x - (unsigned)bh * (unsigned)p.nsplit);
     const int b = bh / p.H, h = bh - b * p.H;
 
     const uint16_t *kbase = p.k + b * p.ks[0] + h * p.ks[1];
@@ -407,34 +408,75 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
         }
     }
     __syncthreads();
-    {
-        constexpr int NV = D / 8;  // 8 threads per query row
-        const int q = tid >> 3, d0 = (tid & 7) * NV;
-        if (q < p.Sq) {
-            float out[NV], M, L;
-            merge_parts<NV>(part + q * PST, kDecodeWaves, 32 * PST, D, d0, out, M, L);
-            if (p.nsplit == 1) {
-                const float inv = L > 0.f ? 1.f / L : 0.f;
-                if (p.lse != nullptr && (tid & 7) == 0)
-                    p.lse[b * p.lses[0] + h * p.lses[1] + q * p.lses[2]] =
-                        L > 0.f ? (M + __builtin_amdgcn_logf(L)) * 0.69314718056f : kNegInf;
-                uint16_t *orow = p.o + b * p.os[0] + h * p.os[1] + (int64_t)q * p.os[2] + d0;
-#pragma unroll
-                for (int j = 0; j < NV; j += 2) *(uint32_t *)(orow + j) = E::pack2(out[j] * inv, out[j + 1] * inv);
-            } else {
-                float *w = p.ws + (((int64_t)bh * p.nsplit + split) * p.Sq + q) * PST;
-#pragma unroll
-                for (int j = 0; j < NV; j++) w[d0 + j] = out[j];
-                if ((tid & 7) == 0) {
-                    w[D] = M;
-                    w[D + 1] = L;
-                }
-            }
+    // n parts in LDS, `stride` floats apart, added up: a wave takes rows, four floats per lane
+    constexpr int LPR = D / 4, RPW = 64 / LPR;  // lanes per row, rows side by side
+    const int l = lane & (LPR - 1), r0 = lane / LPR;
+    auto add_up = [&](const float *parts, int n, int stride, int first, int step, auto &&leave) {
+#pragma unroll 1
+        for (int row = first; row < p.Sq; row += step) {
+            float out[4], M, L;
+            merge_parts<4>(parts + row * PST, n, stride, D, 4 * l, out, M, L);
+            leave(row, f32x4{out[0], out[1], out[2], out[3]}, M, L);
         }
+    };
+    const int first = wave_u * RPW + r0, step = kDecodeWaves * RPW;
+    auto to_output = [&](int row, f32x4 x, float M, float L) {
+        const float inv = L > 0.f ? 1.f / L : 0.f;
+        if (p.lse != nullptr && l == 0)
+            p.lse[b * p.lses[0] + h * p.lses[1] + row * p.lses[2]] =
+                L > 0.f ? (M + __builtin_amdgcn_logf(L)) * 0.69314718056f : kNegInf;
+        *(u32x2 *)(p.o + b * p.os[0] + h * p.os[1] + (int64_t)row * p.os[2] + 4 * l) =
+            u32x2{E::pack2(x.x * inv, x.y * inv), E::pack2(x.z * inv, x.w * inv)};
+    };
+    if (p.nsplit == 1) {
+        add_up(part, kDecodeWaves, 32 * PST, first, step, to_output);
+        return;
     }
+    const uint32_t part_bytes = (uint32_t)(p.Sq * PST * 4);
+    uint8_t *const plane_parts = reinterpret_cast<uint8_t *>(p.ws) + (int64_t)bh * p.nsplit * part_bytes;
+    const HandOver mine(plane_parts + (int64_t)split * part_bytes, part_bytes);
+    add_up(part, kDecodeWaves, 32 * PST, first, step, [&](int row, f32x4 x, float M, float L) {
+        mine.put((uint32_t)(4 * (row * PST + 4 * l)), x);
+        if (l == 0) mine.put((uint32_t)(4 * (row * PST + D)), f32x2{M, L});
+    });
+    if (p.arrivals == nullptr) return;
+
+    // ---- the last workgroup of the plane brings all parts to LDS as they lie in memory, and adds them up ----
+    // A launch of its own for that costs its 3 us on an idle device and two more memory round trips: B4 H32 Sq1 Sk2048 with a new mask
+    // 25.8 -> 23.3 us a call, B8 H16 Sq16 Sk16384 gathered 86.4 -> 85.3, B8 H32 Sq1 Sk32768 651 -> 649 (D = 128, bf16).  With the parts
+    // read into registers row by row instead, in unrolled code that every compute unit fetches for the first time here: 24.3, 92.2.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();  // every wave's rows have been handed over, and LDS has been read
+    if (tid == 0) *reinterpret_cast<int *>(smem) = arrives_last(p.arrivals + bh, p.tag, p.nsplit);
+    __syncthreads();
+    const bool last = __builtin_amdgcn_readfirstlane(*reinterpret_cast<int *>(smem)) != 0;
+    if (!last) return;
+    __syncthreads();
+    // (rows are a multiple of 8 bytes; the 8 in front of a plane that starts between two pieces of 16 are the plane's before it,
+    // the up to 8 behind the last plane the counters')
+    const uint32_t lead = (uint32_t)(uintptr_t)plane_parts & 8u, bytes = p.nsplit * part_bytes + lead;
+    for (uint32_t at = 1024u * wave_u; at < bytes; at += 1024u * kDecodeWaves)
+        if (at + 16u * lane < bytes) dma16<false, true>(plane_parts - lead + at, 16u * lane, lds0 + at);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    float *const all = part + lead / 4;
+    const int stride = p.Sq * PST;
+    int n = p.nsplit;
+    if (n > kMergeFew) {  // the waves share the parts first, each into the first one of its own
+        float *const own = all + wave_u * stride;
+        add_up(own, (n - wave_u + kDecodeWaves - 1) / kDecodeWaves, kDecodeWaves * stride, r0, RPW, [&](int row, f32x4 x, float M, float L) {
+            *(f32x2 *)(own + row * PST + 4 * l) = f32x2{x.x, x.y};
+            *(f32x2 *)(own + row * PST + 4 * l + 2) = f32x2{x.z, x.w};
+            if (l == 0) *(f32x2 *)(own + row * PST + D) = f32x2{M, L};
+        });
+        n = kDecodeWaves;
+        __syncthreads();
+    }
+    add_up(all, n, stride, first, step, to_output);
 }
 
-// Merge of the nsplit partial results of every (b, h): grid B*H, 256 threads, 8 per query row.
+// Merge of the nsplit partial results of every (b, h) in a launch of its own, where LDS does not hold them or the workspace has no
+// place for the counters: grid B*H, 256 threads, 8 per query row.
 template <int DT, int D>
 __global__ __launch_bounds__(256) void decode_merge_kernel(const DecodeParams p) {
     using E = Elem<DT>;
@@ -467,7 +509,6 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(const DecodeParams p)
 // so from five parts on this one is faster at these sizes; the line stands at eight, where the order of the sum has been so far.
 // With 2 ... 4 parts the exchanges between lanes cost more than they save: 2 parts (B1 H8 Sk512) 12.5 -> 14.4, 4 parts (B8 H16
 // Sq32 Sk1024) 26.3 -> 29.6.
-constexpr int kMergeFew = 8;
 constexpr int kMergeBatch = 4;
 template <int DT, int D>
 __global__ __launch_bounds__(256) void decode_merge_many_kernel(const DecodeParams p) {
@@ -585,9 +626,9 @@ hipError_t launch_decode_kind(const DecodeParams &p, hipStream_t stream) {
     auto kern = sparse_decode_kernel<DT, D, PK, B16, DM>;
     static unsigned long long attr_done = 0;  // devices on which this kernel may use `smem` bytes of LDS
     if (const hipError_t e0 = allow_dynamic_smem(kern, smem, attr_done); e0 != hipSuccess) return e0;
-    hipLaunchKernelGGL(kern, dim3(p.nsplit, p.B * p.H), dim3(kDecodeWaves * 64), smem, stream, p);
+    hipLaunchKernelGGL(kern, dim3((unsigned)p.nsplit * (unsigned)(p.B * p.H)), dim3(kDecodeWaves * 64), smem, stream, p);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess || p.nsplit == 1) return e;
+    if (e != hipSuccess || p.nsplit == 1 || p.arrivals != nullptr) return e;
     const unsigned rows = (unsigned)p.B * p.H * p.Sq;  // (at most 65535 planes of 32 rows)
     if (p.nsplit > kMergeFew) hipLaunchKernelGGL((decode_merge_many_kernel<DT, D>), dim3((rows + 3) / 4), dim3(256), 0, stream, p);
     else hipLaunchKernelGGL((decode_merge_kernel<DT, D>), dim3(p.B * p.H), dim3(256), 0, stream, p);

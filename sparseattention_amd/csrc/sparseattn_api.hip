@@ -4,6 +4,8 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <chrono>
+
 #include "kernels.h"
 #include "sparseattn.h"
 
@@ -24,6 +26,18 @@ int log2_exact(int x) {  // -1 unless x is a power of two
     int l = 0;
     while ((1 << l) < x) l++;
     return l;
+}
+
+// The number of a launch whose workgroups count their arrivals (arrives_last): its upper 56 bits, no two in a process alike.
+// The first one depends on the time the process took it and on where it lies in memory, so that memory which another
+// process left behind holds none of them.
+uint64_t next_launch_tag() {
+    static uint64_t last = [] {
+        uint64_t x = (uint64_t)std::chrono::steady_clock::now().time_since_epoch().count() ^ (uint64_t)(uintptr_t)&g_error;
+        for (int i = 0; i < 2; i++) x = (x ^ (x >> 31)) * 0x9e3779b97f4a7c15ull;
+        return x << 8;
+    }();
+    return __atomic_add_fetch(&last, 256, __ATOMIC_RELAXED);
 }
 
 bool aligned(const void *p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
@@ -892,6 +906,11 @@ size_t sa_decode_workspace_bytes(int B, int H, int Sq, int D, int num_splits) {
     return (size_t)B * H * num_splits * Sq * (size_t)(D + 2) * sizeof(float);
 }
 
+size_t sa_decode_workspace_bytes_ex(int B, int H, int Sq, int D, int num_splits) {
+    const size_t least = sa_decode_workspace_bytes(B, H, Sq, D, num_splits);
+    return least != 0 && num_splits * Sq <= sa::kDecodeMergeRows ? (least + 7) / 8 * 8 + (size_t)B * H * 8 : least;
+}
+
 }  // extern "C"
 
 namespace {
@@ -993,6 +1012,10 @@ int decode_impl(const void *q, const int64_t q_strides[4], const void *k, const 
                        : 0;
     dp.nsplit = num_splits;
     dp.ws = static_cast<float *>(workspace);
+    if (need != 0 && num_splits * Sq <= sa::kDecodeMergeRows && workspace_bytes >= sa_decode_workspace_bytes_ex(B, H, Sq, D, num_splits)) {
+        dp.arrivals = reinterpret_cast<uint64_t *>(static_cast<uint8_t *>(workspace) + (need + 7) / 8 * 8);
+        dp.tag = next_launch_tag();
+    }
     dp.scale = sm_scale_log2;
     dp.lse = nullptr;
     if (lse) {
