@@ -249,6 +249,32 @@ int sa_mask_classify_terms(const int32_t *terms, int n_terms, const int32_t *doc
                            int32_t *part_lens, const int64_t part_lens_strides[3], uint8_t *packed,
                            const int64_t packed_strides[2], void *workspace, size_t workspace_bytes, void *stream);
 
+/* Two masks by one launch, each as by sa_mask_classify_terms with the arguments of its call (host structures, read before the
+ * function returns): the two tilings of a backward have few Q tiles each.  Outputs must not overlap. */
+typedef struct sa_mask_terms_call {
+    const int32_t *terms;
+    int n_terms;
+    const int32_t *doc_q;
+    const int64_t *doc_q_strides;
+    const int32_t *doc_k;
+    const int64_t *doc_k_strides;
+    int B, H, Sq, Sk, BQ, BK;
+    int32_t *full_ids;
+    const int64_t *full_ids_strides;
+    int32_t *full_lens;
+    const int64_t *full_lens_strides;
+    int32_t *part_ids;
+    const int64_t *part_ids_strides;
+    int32_t *part_lens;
+    const int64_t *part_lens_strides;
+    uint8_t *packed;
+    const int64_t *packed_strides;
+    void *workspace;
+    size_t workspace_bytes;
+} sa_mask_terms_call;
+int sa_mask_classify_terms_pair(const sa_mask_terms_call *first, const sa_mask_terms_call *second, void *stream);
+
+
 /*
  * Schedule of the forward: which Q tiles a workgroup processes, in order.  No counterpart in the reference, whose
  * grid is one program per Q tile (sparse_attn_kernel.py:167).  A workgroup that walks several Q tiles runs one

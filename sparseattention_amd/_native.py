@@ -63,6 +63,7 @@ EXPORTS = (
     "sa_sparse_attention_bwd",
     "sa_mask_terms_workspace_bytes",
     "sa_mask_classify_terms",
+    "sa_mask_classify_terms_pair",
 )
 
 _lib = None

@@ -239,11 +239,15 @@ py::tuple classify(const Tensor &mask, int64_t BQ, int64_t BK, std::optional<boo
 }
 
 // compute_mask_terms: the same from terms, eight int32 each (their and the documents' shapes are checked by the caller)
+int64_t terms_planes(int64_t B, const OptTensor &doc_q, const OptTensor &doc_k) {
+    const bool per_batch = B > 1 && ((doc_q && doc_q->stride(0) != 0) || (doc_k && doc_k->stride(0) != 0));
+    return per_batch ? B : 1;
+}
+
 py::tuple classify_terms(const std::vector<int32_t> &terms, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t BQ, int64_t BK,
                          const OptTensor &doc_q, const OptTensor &doc_k, bool pack, const at::Device &dev) {
     const int64_t nQ = Sq / BQ, nK = Sk / BK;
-    const bool per_batch = B > 1 && ((doc_q && doc_q->stride(0) != 0) || (doc_k && doc_k->stride(0) != 0));
-    const int64_t uB = per_batch ? B : 1;
+    const int64_t uB = terms_planes(B, doc_q, doc_k);
     Lists l;
     {
         const py::gil_scoped_release unlocked;
@@ -256,6 +260,33 @@ py::tuple classify_terms(const std::vector<int32_t> &terms, int64_t B, int64_t H
                                         ptr<int32_t>(l.pl), st(l.pl), ptr<uint8_t>(l.packed), st(l.packed), ws.data_ptr(), ws.numel(), stream_of(l.fid)));
     }
     return as_tuple(l);
+}
+
+// compute_backward_metadata_terms: the mask by query rows and, from its transposed terms, by keys (tiles of 128 x 64 both), packed
+py::tuple classify_terms_backward(const std::vector<int32_t> &terms, const std::vector<int32_t> &transposed, int64_t B, int64_t H, int64_t Sq,
+                                  int64_t Sk, const OptTensor &doc_q, const OptTensor &doc_k, const at::Device &dev) {
+    constexpr int64_t BQ = 128, BK = 64;
+    const int64_t uB = terms_planes(B, doc_q, doc_k);
+    Lists l[2];
+    {
+        const py::gil_scoped_release unlocked;
+        const c10::DeviceGuard guard(dev);
+        const size_t need[2] = {sa_mask_terms_workspace_bytes(uB, Sq, Sk, BQ, BK), sa_mask_terms_workspace_bytes(uB, Sk, Sq, BQ, BK)};
+        const Tensor ws = at::empty({(int64_t)std::max<size_t>(need[0] + need[1], 1)}, at::TensorOptions().dtype(at::kByte).device(dev));
+        sa_mask_terms_call call[2];
+        for (int i = 0; i < 2; i++) {
+            const int64_t rows = i == 0 ? Sq : Sk, keys = i == 0 ? Sk : Sq;
+            const std::vector<int32_t> &t = i == 0 ? terms : transposed;
+            const OptTensor &dr = i == 0 ? doc_q : doc_k, &dk = i == 0 ? doc_k : doc_q;
+            l[i] = empty_lists(uB, 1, B, H, rows / BQ, keys / BK, BQ * BK / 8, true, dev);
+            call[i] = {t.data(), (int)(t.size() / 8), ptr<int32_t>(dr), st(dr), ptr<int32_t>(dk), st(dk), (int)B, (int)H, (int)rows, (int)keys,
+                       (int)BQ, (int)BK, ptr<int32_t>(l[i].fid), st(l[i].fid), ptr<int32_t>(l[i].fl), st(l[i].fl), ptr<int32_t>(l[i].pid),
+                       st(l[i].pid), ptr<int32_t>(l[i].pl), st(l[i].pl), ptr<uint8_t>(l[i].packed), st(l[i].packed),
+                       ptr<uint8_t>(ws) + (i == 0 ? 0 : need[0]), need[i]};
+        }
+        check_rc(sa_mask_classify_terms_pair(&call[0], &call[1], stream_of(l[0].fid)));
+    }
+    return py::make_tuple(as_tuple(l[0]), as_tuple(l[1]));
 }
 
 // ---- decode -------------------------------------------------------------------------------------------------------
@@ -800,6 +831,7 @@ PYBIND11_MODULE(_host, m) {
     m.def("decode", &decode);
     m.def("classify", &classify);
     m.def("classify_terms", &classify_terms);
+    m.def("classify_terms_backward", &classify_terms_backward);
     m.def("backward", &backward);
     m.def("backward_workspace_bytes", &backward_workspace_bytes);
     m.def("kernel_head_dim", &kernel_head_dim);

@@ -109,7 +109,11 @@ struct TermsParams {
     uint8_t *packed;  // PackParams layout, or null
     int64_t ob;       // bytes between packed planes along b
 };
-hipError_t launch_mask_terms(const TermsParams &p, hipStream_t stream);
+// Masks made by one launch: the two tilings of a backward are short of workgroups one by one.
+struct TermsBatch {
+    TermsParams of[2];
+};
+hipError_t launch_mask_terms(const TermsBatch &b, int n, hipStream_t stream);
 
 // ---- block-sparse forward ------------------------------------------------------------------------
 struct FwdParams {

@@ -72,7 +72,7 @@ __device__ __forceinline__ uint64_t row_word(const TermsParams &p, int q, int ks
     return word & bit_range(0, n);
 }
 
-// grid (nQ, distinct planes), 512 threads: a workgroup makes everything of one Q tile, so nothing goes through memory
+// grid (nQ, distinct planes, masks), 512 threads: a workgroup makes everything of one Q tile, so nothing goes through memory
 // between classification, lists and packed tiles.  Per round of at most kTiles tiles:
 //   A  a strip of 64 keys is decided from the first and the last row of the Q tile where it can be (both ends of a
 //      row's interval move right, or stay, as q grows): no term reaches it, or one term covers it from every row,
@@ -86,7 +86,11 @@ __device__ __forceinline__ uint64_t row_word(const TermsParams &p, int q, int ks
 // classification with one key per lane and one row per step, compaction and packing as three kernels that evaluated the
 // terms per entry (launches back to back in a graph): causal documents B4 S2048 tiles 128x64 71 -> 10.3 us, B4 S16384
 // tiles 128x32 352 -> 44 us, window and prefix at S32768 149 -> 9.5 us.  1024 threads: 10.4 / 49 / 10.5 us.
-__global__ __launch_bounds__(kThreads) void mask_terms_kernel(const TermsParams p) {
+// The two tilings of a backward come from one launch: few Q tiles each (B4 S2048: 64 workgroups), and most of a launch is the start
+// of a compute unit that has none of the code yet.  Causal documents B4 S2048 20.0 -> 10.6 us, B8 S4096 24.5 -> 14.8, B1 S32768 53 -> 33.
+__global__ __launch_bounds__(kThreads) void mask_terms_kernel(const TermsBatch batch) {
+    const TermsParams &p = batch.of[blockIdx.z];
+    if ((int)blockIdx.x >= p.nQ || (int)blockIdx.y >= p.uB) return;
     __shared__ unsigned state[kTiles];  // bit 0: some entry attends, bit 1: some entry does not
     __shared__ uint16_t part[kTiles];   // the PARTIAL tiles of the round, in order
     __shared__ uint16_t todo[kStrips];  // strips that step A left open
@@ -293,8 +297,13 @@ __global__ __launch_bounds__(kThreads) void mask_terms_kernel(const TermsParams 
 
 }  // namespace
 
-hipError_t launch_mask_terms(const TermsParams &p, hipStream_t stream) {
-    hipLaunchKernelGGL(mask_terms_kernel, dim3(p.nQ, p.uB), dim3(kThreads), 0, stream, p);
+hipError_t launch_mask_terms(const TermsBatch &b, int n, hipStream_t stream) {
+    unsigned nQ = 0, planes = 0;
+    for (int i = 0; i < n; i++) {
+        nQ = b.of[i].nQ > (int)nQ ? b.of[i].nQ : nQ;
+        planes = b.of[i].uB > (int)planes ? b.of[i].uB : planes;
+    }
+    hipLaunchKernelGGL(mask_terms_kernel, dim3(nQ, planes, n), dim3(kThreads), 0, stream, b);
     return hipGetLastError();
 }
 

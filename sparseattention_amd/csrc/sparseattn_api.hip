@@ -777,32 +777,32 @@ size_t sa_mask_terms_workspace_bytes(int distinct_b, int Sq, int Sk, int BQ, int
     return (size_t)distinct_b * (size_t)(Sq / BQ) * (size_t)(Sk / BK);
 }
 
-int sa_mask_classify_terms(const int32_t *terms, int n_terms, const int32_t *doc_q, const int64_t doc_q_strides[2],
-                           const int32_t *doc_k, const int64_t doc_k_strides[2], int B, int H, int Sq, int Sk, int BQ,
-                           int BK, int32_t *full_ids, const int64_t full_ids_strides[4], int32_t *full_lens,
-                           const int64_t full_lens_strides[3], int32_t *part_ids, const int64_t part_ids_strides[4],
-                           int32_t *part_lens, const int64_t part_lens_strides[3], uint8_t *packed,
-                           const int64_t packed_strides[2], void *workspace, size_t workspace_bytes, void *stream) {
-    g_error[0] = 0;
+// The checks of a mask given by terms, and what its launch needs.
+static int terms_params(const char *who, sa::TermsParams &tp, const int32_t *terms, int n_terms, const int32_t *doc_q,
+                        const int64_t doc_q_strides[2], const int32_t *doc_k, const int64_t doc_k_strides[2], int B, int H,
+                        int Sq, int Sk, int BQ, int BK, int32_t *full_ids, const int64_t full_ids_strides[4], int32_t *full_lens,
+                        const int64_t full_lens_strides[3], int32_t *part_ids, const int64_t part_ids_strides[4],
+                        int32_t *part_lens, const int64_t part_lens_strides[3], uint8_t *packed,
+                        const int64_t packed_strides[2], void *workspace, size_t workspace_bytes) {
     if (!terms || !full_ids || !full_ids_strides || !full_lens || !full_lens_strides || !part_ids ||
         !part_ids_strides || !part_lens || !part_lens_strides || (doc_q && !doc_q_strides) ||
         (doc_k && !doc_k_strides) || (packed && !packed_strides))
-        return fail(SA_ERR_INVALID_ARGUMENT, "sa_mask_classify_terms: null pointer argument");
+        return fail(SA_ERR_INVALID_ARGUMENT, "%s: null pointer argument", who);
     if (n_terms < 1 || n_terms > sa::kMaxMaskTerms)
-        return fail(SA_ERR_INVALID_ARGUMENT, "sa_mask_classify_terms: %d terms (1..%d)", n_terms, sa::kMaxMaskTerms);
+        return fail(SA_ERR_INVALID_ARGUMENT, "%s: %d terms (1..%d)", who, n_terms, sa::kMaxMaskTerms);
     if (const int rc = check_tiling(B, H, Sq, Sk, BQ, BK)) return rc;
     const int lbk = log2_exact(BK);
-    if (lbk < 4) return fail(SA_ERR_UNSUPPORTED, "sa_mask_classify_terms: BLOCK_K %d (supported: powers of two >= 16)", BK);
+    if (lbk < 4) return fail(SA_ERR_UNSUPPORTED, "%s: BLOCK_K %d (supported: powers of two >= 16)", who, BK);
     if ((int64_t)BQ * BK > 0x7fffffffLL)
-        return fail(SA_ERR_UNSUPPORTED, "sa_mask_classify_terms: tiles of more than 2^31-1 entries");
+        return fail(SA_ERR_UNSUPPORTED, "%s: tiles of more than 2^31-1 entries", who);
 
-    sa::TermsParams tp{};
+    tp = sa::TermsParams{};
     tp.n_terms = n_terms;
     for (int t = 0; t < n_terms; t++) {
         const int32_t *w = terms + 8 * t;
-        if (w[0] < 0 || w[0] > 31) return fail(SA_ERR_INVALID_ARGUMENT, "sa_mask_classify_terms: term %d has unknown flags %d", t, w[0]);
+        if (w[0] < 0 || w[0] > 31) return fail(SA_ERR_INVALID_ARGUMENT, "%s: term %d has unknown flags %d", who, t, w[0]);
         if ((w[0] & SA_TERM_SAME_DOC) && !(doc_q && doc_k))
-            return fail(SA_ERR_INVALID_ARGUMENT, "sa_mask_classify_terms: term %d compares documents, doc_q and doc_k are needed", t);
+            return fail(SA_ERR_INVALID_ARGUMENT, "%s: term %d compares documents, doc_q and doc_k are needed", who, t);
         // the term as an interval of keys per query row (sa::MaskTerm), in 64 bits before clamping
         const int64_t big = (int64_t)1 << 30;
         auto clamp = [](int64_t x, int64_t lo, int64_t hi) { return x < lo ? lo : (x > hi ? hi : x); };
@@ -816,17 +816,17 @@ int sa_mask_classify_terms(const int32_t *terms, int n_terms, const int32_t *doc
         m.doc = (w[0] & SA_TERM_SAME_DOC) ? 1 : 0;
     }
     if (Sq > (1 << 29) || Sk > (1 << 29))
-        return fail(SA_ERR_UNSUPPORTED, "sa_mask_classify_terms: more than 2^29 queries or keys");
+        return fail(SA_ERR_UNSUPPORTED, "%s: more than 2^29 queries or keys", who);
     // the mask depends on the batch element only through the document numbers
     const bool per_batch = B > 1 && ((doc_q && doc_q_strides[0] != 0) || (doc_k && doc_k_strides[0] != 0));
     const int uB = per_batch ? B : 1;
     const int nQ = Sq / BQ, nK = Sk / BK;
     if (nQ > 65535 || uB > 65535)
-        return fail(SA_ERR_UNSUPPORTED, "sa_mask_classify_terms: more than 65535 Q tiles or distinct mask planes");
+        return fail(SA_ERR_UNSUPPORTED, "%s: more than 65535 Q tiles or distinct mask planes", who);
     // (part of the contract; the kernel keeps the tiles' states in LDS and does not touch it)
     const size_t need = sa_mask_terms_workspace_bytes(uB, Sq, Sk, BQ, BK);
     if (!workspace || workspace_bytes < need)
-        return fail(SA_ERR_WORKSPACE, "sa_mask_classify_terms: workspace of %zu bytes required, %zu given", need,
+        return fail(SA_ERR_WORKSPACE, "%s: workspace of %zu bytes required, %zu given", who, need,
                     workspace ? workspace_bytes : (size_t)0);
     const int64_t ob[4] = {full_ids_strides[0], full_lens_strides[0], part_ids_strides[0], part_lens_strides[0]};
     const int64_t oh[4] = {full_ids_strides[1], full_lens_strides[1], part_ids_strides[1], part_lens_strides[1]};
@@ -836,18 +836,18 @@ int sa_mask_classify_terms(const int32_t *terms, int n_terms, const int32_t *doc
         zh += oh[i] == 0;
     }
     if (B > 1 && zb != 0 && (zb != 4 || per_batch))
-        return fail(SA_ERR_INVALID_ARGUMENT, "sa_mask_classify_terms: output batch stride 0 needs a mask shared by the batch and must be 0 on all four outputs");
+        return fail(SA_ERR_INVALID_ARGUMENT, "%s: output batch stride 0 needs a mask shared by the batch and must be 0 on all four outputs", who);
     if (H > 1 && zh != 0 && zh != 4)
-        return fail(SA_ERR_INVALID_ARGUMENT, "sa_mask_classify_terms: output head stride 0 must be 0 on all four outputs");
+        return fail(SA_ERR_INVALID_ARGUMENT, "%s: output head stride 0 must be 0 on all four outputs", who);
     if (packed) {
         const int64_t plane_bytes = (int64_t)Sq * Sk / 8;
         if (!aligned(packed, 4) || packed_strides[0] % 4)
-            return fail(SA_ERR_UNSUPPORTED, "sa_mask_classify_terms: packed needs a 4-byte aligned base and batch stride");
+            return fail(SA_ERR_UNSUPPORTED, "%s: packed needs a 4-byte aligned base and batch stride", who);
         if (uB > 1 && packed_strides[0] < plane_bytes)
-            return fail(SA_ERR_INVALID_ARGUMENT, "sa_mask_classify_terms: packed planes overlap (stride %lld, %lld bytes per plane)",
+            return fail(SA_ERR_INVALID_ARGUMENT, "%s: packed planes overlap (stride %lld, %lld bytes per plane)", who,
                         (long long)packed_strides[0], (long long)plane_bytes);
         if (H > 1 && packed_strides[1] != 0)
-            return fail(SA_ERR_INVALID_ARGUMENT, "sa_mask_classify_terms: the mask is the same for every head: packed_strides[1] must be 0");
+            return fail(SA_ERR_INVALID_ARGUMENT, "%s: the mask is the same for every head: packed_strides[1] must be 0", who);
     }
 
     tp.doc_q = doc_q;
@@ -881,8 +881,41 @@ int sa_mask_classify_terms(const int32_t *terms, int n_terms, const int32_t *doc
     }
     tp.packed = packed;
     tp.ob = packed ? packed_strides[0] : 0;
-    const hipError_t e = sa::launch_mask_terms(tp, static_cast<hipStream_t>(stream));
+    return SA_OK;
+}
+
+int sa_mask_classify_terms(const int32_t *terms, int n_terms, const int32_t *doc_q, const int64_t doc_q_strides[2],
+                           const int32_t *doc_k, const int64_t doc_k_strides[2], int B, int H, int Sq, int Sk, int BQ,
+                           int BK, int32_t *full_ids, const int64_t full_ids_strides[4], int32_t *full_lens,
+                           const int64_t full_lens_strides[3], int32_t *part_ids, const int64_t part_ids_strides[4],
+                           int32_t *part_lens, const int64_t part_lens_strides[3], uint8_t *packed,
+                           const int64_t packed_strides[2], void *workspace, size_t workspace_bytes, void *stream) {
+    g_error[0] = 0;
+    sa::TermsBatch b;
+    if (const int rc = terms_params("sa_mask_classify_terms", b.of[0], terms, n_terms, doc_q, doc_q_strides, doc_k, doc_k_strides, B, H, Sq,
+                                    Sk, BQ, BK, full_ids, full_ids_strides, full_lens, full_lens_strides, part_ids, part_ids_strides,
+                                    part_lens, part_lens_strides, packed, packed_strides, workspace, workspace_bytes))
+        return rc;
+    b.of[1] = b.of[0];
+    const hipError_t e = sa::launch_mask_terms(b, 1, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail(SA_ERR_HIP, "sa_mask_classify_terms: launch failed: %s", hipGetErrorString(e));
+    return SA_OK;
+}
+
+int sa_mask_classify_terms_pair(const sa_mask_terms_call *first, const sa_mask_terms_call *second, void *stream) {
+    g_error[0] = 0;
+    if (!first || !second) return fail(SA_ERR_INVALID_ARGUMENT, "sa_mask_classify_terms_pair: null pointer argument");
+    sa::TermsBatch b;
+    for (int i = 0; i < 2; i++) {
+        const sa_mask_terms_call &c = i == 0 ? *first : *second;
+        if (const int rc = terms_params("sa_mask_classify_terms_pair", b.of[i], c.terms, c.n_terms, c.doc_q, c.doc_q_strides, c.doc_k,
+                                        c.doc_k_strides, c.B, c.H, c.Sq, c.Sk, c.BQ, c.BK, c.full_ids, c.full_ids_strides, c.full_lens,
+                                        c.full_lens_strides, c.part_ids, c.part_ids_strides, c.part_lens, c.part_lens_strides, c.packed,
+                                        c.packed_strides, c.workspace, c.workspace_bytes))
+            return rc;
+    }
+    const hipError_t e = sa::launch_mask_terms(b, 2, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return fail(SA_ERR_HIP, "sa_mask_classify_terms_pair: launch failed: %s", hipGetErrorString(e));
     return SA_OK;
 }
 

@@ -388,16 +388,7 @@ def materialize_mask_terms(terms: Sequence[MaskTerm], B: int, Sq: int, Sk: int, 
     return out
 
 
-def compute_mask_terms(terms: Sequence[MaskTerm], B: int, H: int, Sq: int, Sk: int, BLOCK_Q: int, BLOCK_K: int,
-                       doc_q: Optional[torch.Tensor] = None, doc_k: Optional[torch.Tensor] = None, device=None,
-                       pack_partial: bool = True, schedule=None) -> MaskMetadata:
-    """:func:`compute_mask_kernel` for a mask given by terms: the same lists (and packed PARTIAL tiles, schedule) as
-    for ``materialize_mask_terms(...)``, computed on the GPU from the formula without the Sq x Sk tensor.
-
-    With ``pack_partial`` the result carries everything the forward needs: ``sparse_attention(q, k, v, None, BLOCK_Q,
-    BLOCK_K, mask_metadata=md)``.  ``doc_q`` / ``doc_k``: int32 document numbers [B,Sq] / [B,Sk] (or [Sq] / [Sk]) on
-    the GPU for terms with ``same_doc``.  ``device``: where to compute when there are no documents.
-    """
+def _check_terms(terms, B, Sq, Sk, BLOCK_Q, BLOCK_K, doc_q, doc_k, device):
     terms = list(terms)
     if not 1 <= len(terms) <= MAX_MASK_TERMS:
         raise ValueError(f"1..{MAX_MASK_TERMS} terms (got {len(terms)})")
@@ -410,6 +401,34 @@ def compute_mask_terms(terms: Sequence[MaskTerm], B: int, H: int, Sq: int, Sk: i
     if dev.type != "cuda" or any(d is not None and d.device != dev for d in (doc_q, doc_k)):
         raise RuntimeError("compute_mask_terms runs on a ROCm GPU (documents on the same device); "
                            "materialize_mask_terms + compute_mask_slow run anywhere")
+    return terms, doc_q, doc_k, dev
+
+
+def compute_mask_terms_backward(terms: Sequence[MaskTerm], B: int, H: int, Sq: int, Sk: int, doc_q=None, doc_k=None,
+                                device=None) -> tuple[MaskMetadata, MaskMetadata]:
+    """:func:`compute_mask_terms` for the backward's two tilings (128 x 64, by query rows and by keys) in one launch."""
+    terms, doc_q, doc_k, dev = _check_terms(terms, B, Sq, Sk, 128, 64, doc_q, doc_k, device)
+    assert Sk % 128 == 0, "Sk must be a multiple of 128"
+    flat, turned = ([w for t in ts for w in t.encode()] for ts in (terms, [t.transposed() for t in terms]))
+    out = []
+    for lists, keys in zip(_native.host().classify_terms_backward(flat, turned, B, H, Sq, Sk, doc_q, doc_k, dev), (Sk, Sq)):
+        md = MaskMetadata(*lists, None, 0)
+        md._validated_for = validation_key(md, keys, 64)  # (as in compute_mask_terms)
+        out.append(md)
+    return tuple(out)
+
+
+def compute_mask_terms(terms: Sequence[MaskTerm], B: int, H: int, Sq: int, Sk: int, BLOCK_Q: int, BLOCK_K: int,
+                       doc_q: Optional[torch.Tensor] = None, doc_k: Optional[torch.Tensor] = None, device=None,
+                       pack_partial: bool = True, schedule=None) -> MaskMetadata:
+    """:func:`compute_mask_kernel` for a mask given by terms: the same lists (and packed PARTIAL tiles, schedule) as
+    for ``materialize_mask_terms(...)``, computed on the GPU from the formula without the Sq x Sk tensor.
+
+    With ``pack_partial`` the result carries everything the forward needs: ``sparse_attention(q, k, v, None, BLOCK_Q,
+    BLOCK_K, mask_metadata=md)``.  ``doc_q`` / ``doc_k``: int32 document numbers [B,Sq] / [B,Sk] (or [Sq] / [Sk]) on
+    the GPU for terms with ``same_doc``.  ``device``: where to compute when there are no documents.
+    """
+    terms, doc_q, doc_k, dev = _check_terms(terms, B, Sq, Sk, BLOCK_Q, BLOCK_K, doc_q, doc_k, device)
     flat = [w for t in terms for w in t.encode()]
     fid, fl, pid, pl, packed = _native.host().classify_terms(flat, B, H, Sq, Sk, BLOCK_Q, BLOCK_K, doc_q, doc_k, bool(pack_partial), dev)
     sched, mode = None, 0

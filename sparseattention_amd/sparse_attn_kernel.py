@@ -7,7 +7,7 @@ from __future__ import annotations
 import torch
 
 from . import _native
-from .mask_utils import MaskMetadata, Tiling, compute_mask_kernel, compute_mask_terms, validation_key
+from .mask_utils import MaskMetadata, Tiling, compute_mask_kernel, compute_mask_terms_backward, validation_key
 
 _DTYPES = {torch.bfloat16: _native.SA_DTYPE_BF16, torch.float16: _native.SA_DTYPE_FP16}
 
@@ -254,10 +254,7 @@ def compute_backward_metadata_terms(terms, B: int, H: int, Sq: int, Sk: int, doc
     """:func:`compute_backward_metadata` for a mask given by terms (:func:`compute_mask_terms`): both tilings with
     their packed PARTIAL tiles, the key-major one from the transposed terms, so that
     ``sparse_attention_backward(..., mask=None, bwd_metadata=...)`` runs without any mask tensor."""
-    terms = list(terms)
-    return _of_one_mask(BackwardMetadata(
-        compute_mask_terms(terms, B, H, Sq, Sk, 128, 64, doc_q, doc_k, device),
-        compute_mask_terms([t.transposed() for t in terms], B, H, Sk, Sq, 128, 64, doc_k, doc_q, device), None))
+    return _of_one_mask(BackwardMetadata(*compute_mask_terms_backward(terms, B, H, Sq, Sk, doc_q, doc_k, device), None))
 
 
 def sparse_attention_backward(do: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
