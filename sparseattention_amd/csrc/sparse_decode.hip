@@ -9,8 +9,8 @@
 // read once, 2 flop per byte and query row.
 //
 // Per chunk of 32 keys a wave
-//   * holds K as MFMA operand straight from global memory (lane = key, 8 x 16 bytes of its row half; the
-//     contraction order is permuted the same way in Q, which costs nothing),
+//   * holds K as MFMA operand (lane = key, 8 x 16 bytes of its row half; the contraction order is permuted the same way in Q, which
+//     costs nothing), from whole rows after a way through LDS or, where decode_key_rows says so, straight from global memory,
 //   * receives V in its own LDS stage by direct loads (swizzled rows, transposing reads: fwd_common.h),
 //   * computes S^T = K . Q^T (32 keys x 32 query rows, rows past Sq are padding), masks PARTIAL tiles from the bool
 //     mask, updates the lagging reference value, P = exp2(S^T - m), O^T += V^T . P^T, row sums by a small MFMA,
@@ -24,9 +24,19 @@ namespace {
 constexpr int kDecodeWaves = 4;
 constexpr int kMergeFew = 8;  // parts up to which a row's are added up one after the other
 
-template <int D>
+// Where K comes as whole rows.  Two workgroups with the 16 rows that this takes of each wave's share have all of a compute unit's LDS,
+// none is left for lists made in the kernel.  us, K per lane | as rows, K and V not in a cache (a call's own are a layer's of many):
+//   D = 128  B1 H32 Sk8192 Sq1 36.5 | 33.1  Sq8 38.3 | 34.4   B4 H16 Sk8192 Sq1 50.6 | 48.0   B4 H16 Sk32768 Sq1 165.8 | 163.1
+//            B8 H32 Sk32768 Sq1 647 | 624 (6.9 TB/s; a linear streaming read runs at 7.1)   B8 H16 Sk16384 Sq16 gathered 90.3 | 83.6
+//   D = 64   B1 H32 Sk2048 Sq8 13.5 | 11.9   B4 H16 Sk32768 Sq1 90.3 | 85.9   Sq32 97.3 | 93.3
+// and nowhere slower but at BLOCK_K = 16 (B8 H32 Sk4096 Sq1 87.7 | 90.2), whose rows come from two places.  (Called again and again
+// on the same K and V, no more than the memory-side cache and L2 hold, K per lane is up to 6 % faster: B8 H32 Sk4096 78.8 | 82.9.)
+constexpr bool decode_key_rows(bool b16, bool dm) { return !b16 && !dm; }
+
+template <int D, bool KR>
 constexpr int decode_smem_bytes() {
-    constexpr int stream = kDecodeWaves * 2 * 32 * D * 2;         // per wave two V stages of 32 rows
+    // per wave two V stages of 32 rows and, where K comes as whole rows, 16 rows of it
+    constexpr int stream = kDecodeWaves * (2 * 32 + (KR ? 16 : 0)) * D * 2;
     constexpr int merge = kDecodeWaves * 32 * (D + 2) * 4 + 16;   // per wave 32 rows of D + 2 floats (kDecodeMergeRows)
     return stream > merge ? stream : merge;
 }
@@ -80,6 +90,7 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
     constexpr int NLD = 32 / RPI;     // direct loads per chunk
     constexpr int PPR = ROWB / 16;
     constexpr int NC = D / 16, NDB = D / 32;
+    constexpr bool KR = decode_key_rows(B16, DM);  // K comes as whole rows
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -98,8 +109,8 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
     int F = DM ? 0 : min(max(p.full_lens[b * p.fls[0] + h * p.fls[1]], 0), nKt);
     int NE = DM ? 0 : F + min(max(p.part_lens[b * p.pls[0] + h * p.pls[1]], 0), nKt - F);
     const int nCh = p.Sk >> 5;  // (DM) chunks of a row
-    uint32_t *const bits = reinterpret_cast<uint32_t *>(smem + decode_smem_bytes<D>());  // (DM) [Sq][nCh]
-    uint16_t *const list = reinterpret_cast<uint16_t *>(smem + decode_smem_bytes<D>() + kDirectBits);  // FULL, then PARTIAL
+    uint32_t *const bits = reinterpret_cast<uint32_t *>(smem + decode_smem_bytes<D, KR>());  // (DM) [Sq][nCh]
+    uint16_t *const list = reinterpret_cast<uint16_t *>(smem + decode_smem_bytes<D, KR>() + kDirectBits);  // FULL, then PARTIAL
     if constexpr (DM) {
         const uint8_t *m0 = p.mask + b * p.ms[0] + h * p.ms[1];
         const int ppr = 2 * nCh, pieces = p.Sq * ppr;  // of 16 entries
@@ -202,7 +213,11 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const SA_LDS uint8_t *)smem);
     uint8_t *const vmine = smem + wave_u * 2 * VBUF;
     const uint32_t vmine_lds = lds0 + wave_u * 2 * VBUF;
-    const int64_t koff_lane = (int64_t)l32 * p.ks[2] + (D / 2) * hh;
+    // KR: K is read as whole rows like V, 1 KiB per wave instruction, so that its loads can carry the streaming hint too (a lane
+    // that reads its own key's row takes 16 bytes of a line at a time, and with the hint the line is gone after the first ones), and
+    // crosses the lanes through 16 rows of LDS: the same operand, so results are bit-identical (decode_key_rows).
+    uint8_t *const kmine = smem + kDecodeWaves * 2 * VBUF + wave_u * 16 * ROWB;
+    const int64_t kr_lane = (int64_t)ld_r0 * p.ks[2] + 8 * ld_slot;
 
     // list entries of chunk t (clamped into the row of tiles; an entry past the count reads as entry 0 and is masked out)
     auto idx_load = [&](int t, int(&idx)[EPC]) {
@@ -239,10 +254,18 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
     constexpr int NMW = PK || DM ? EPC : 4;  // mask words per lane and chunk
     // everything chunk t needs from memory: K into registers, V into LDS stage `st`, mask words if it has a PARTIAL entry
     auto issue = [&](int t, const int(&col)[EPC], int st, u32x4(&kf)[NC], uint32_t(&mk)[NMW]) {
-        const int kcol = B16 ? ((l32 < 16 ? col[0] : col[EPC - 1]) - (l32 & 16)) : col[0];  // (+ l32: this lane's key)
-        const uint16_t *kp = kbase + (int64_t)kcol * p.ks[2] + koff_lane;
+        if constexpr (KR) {
+            static_assert(NLD == NC, "a chunk of K is as many registers either way");
 #pragma unroll
-        for (int c = 0; c < NC; c++) kf[c] = *(const u32x4 *)(kp + 8 * c);
+            for (int i = 0; i < NLD; i++) {
+                kf[i] = __builtin_nontemporal_load((const u32x4 *)(kbase + (int64_t)(col[0] + RPI * i) * p.ks[2] + kr_lane));
+            }
+        } else {
+            const int kcol = B16 ? ((l32 < 16 ? col[0] : col[EPC - 1]) - (l32 & 16)) : col[0];  // (+ l32: this lane's key)
+            const uint16_t *kp = kbase + (int64_t)(kcol + l32) * p.ks[2] + (D / 2) * hh;
+#pragma unroll
+            for (int c = 0; c < NC; c++) kf[c] = *(const u32x4 *)(kp + 8 * c);
+        }
 #pragma unroll
         for (int i = 0; i < NLD; i++) {
             // rows [RPI i, RPI i + RPI) of the chunk: with BLOCK_K = 16 the second half belongs to the second entry
@@ -277,12 +300,37 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
         }
     };
     // one chunk: scores, mask, softmax update, O^T += V^T . P^T
-    auto compute = [&](int t, int st, const u32x4(&kf)[NC], const uint32_t(&mk)[NMW]) {
+    auto compute = [&](int t, int st, const u32x4(&kf)[NC], const uint32_t(&mk)[NMW]) __attribute__((always_inline)) {
         f32x16 s;
 #pragma unroll
         for (int i = 0; i < 16; i++) s[i] = 0.f;
+        u32x4 ka[NC];  // the A operand: lane (l32, hh) holds d = (D/2) hh + 8c .. +7 of key l32
+        if constexpr (KR) {
+            // (the operations of a wave on LDS take effect in their order)
+            const int r = l32 & 15;
 #pragma unroll
-        for (int c = 0; c < NC; c++) s = E::mfma(kf[c], qf[c], s);
+            for (int i = 0; i < NLD / 2; i++) {
+                const int w = RPI * i + ld_r0;
+                *(u32x4 *)(kmine + w * ROWB + 16 * (ld_slot ^ k_swizzle<D>(w))) = kf[i];
+            }
+#pragma unroll
+            for (int c = 0; c < NC; c++) ka[c] = *(const u32x4 *)(kmine + r * ROWB + 16 * ((NC * hh + c) ^ k_swizzle<D>(r)));
+#pragma unroll
+            for (int i = 0; i < NLD / 2; i++) {
+                const int w = RPI * i + ld_r0;
+                *(u32x4 *)(kmine + w * ROWB + 16 * (ld_slot ^ k_swizzle<D>(w))) = kf[NLD / 2 + i];
+            }
+#pragma unroll
+            for (int c = 0; c < NC; c++) {
+                const u32x4 x = *(const u32x4 *)(kmine + r * ROWB + 16 * ((NC * hh + c) ^ k_swizzle<D>(r)));
+                ka[c] = l32 < 16 ? ka[c] : x;
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < NC; c++) ka[c] = kf[c];
+        }
+#pragma unroll
+        for (int c = 0; c < NC; c++) s = E::mfma(ka[c], qf[c], s);
         const unsigned fl = flags_of(t);
         if (fl != ALL) {  // a PARTIAL entry, or (BLOCK_K = 16) a second entry past the end of the list
             if constexpr (PK || DM) {
@@ -622,7 +670,7 @@ __global__ __launch_bounds__(256) void merge_parts_kernel(const MergeParams p) {
 
 template <int DT, int D, bool PK, bool B16, bool DM = false>
 hipError_t launch_decode_kind(const DecodeParams &p, hipStream_t stream) {
-    constexpr int smem = decode_smem_bytes<D>() + (DM ? kDirectBytes : 0);
+    constexpr int smem = decode_smem_bytes<D, decode_key_rows(B16, DM)>() + (DM ? kDirectBytes : 0);
     auto kern = sparse_decode_kernel<DT, D, PK, B16, DM>;
     static unsigned long long attr_done = 0;  // devices on which this kernel may use `smem` bytes of LDS
     if (const hipError_t e0 = allow_dynamic_smem(kern, smem, attr_done); e0 != hipSuccess) return e0;
