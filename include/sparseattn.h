@@ -385,7 +385,8 @@ int sa_sparse_attention_fwd_kernel(const void *q, const int64_t q_strides[4], co
  * list of a Q tile is shared by several workgroups and their partial results are added up by a second launch.
  *   workspace   sa_fwd_split_workspace_bytes(...) bytes of device memory, 16-byte aligned; may be NULL when that is 0,
  *               which says that the launch has no use for it (the call is then sa_sparse_attention_fwd_kernel with the
- *               default kernel).  The bytes depend on the current device.
+ *               default kernel, or a kernel that walks a list in two halves by the waves of one workgroup).  The bytes depend
+ *               on the current device.
  * Results agree with the default kernel within rounding (a row's keys are added up in other groups).
  * sa_fwd_split_least_keys: lists of up to that many keys are walked by one workgroup all the same (Sk where all are); a caller
  * who knows that no list is longer does without the workspace and saves the second launch.

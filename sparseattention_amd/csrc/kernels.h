@@ -148,6 +148,7 @@ struct FwdParams {
     int nsplit, split_chunks;  // split_chunks: chunks of one part (the last ones may be shorter)
     int split_least;           // lists of up to this many chunks are not shared
     float *ws, *ws_ml;
+    int halves;                // 1: every list in two halves by the waves of one workgroup (fwd_in_halves)
     // Ragged sizes: the tile grid (Sq, Sk, nQ, nK, lists, packed tiles) is that of a padded mask, the tensors have Sq_in
     // and Sk_in rows, which stand q0 and k0 rows into the grid, of D_in elements (a multiple of 8, at most the kernel's D).
     int ragged;
@@ -175,6 +176,8 @@ struct FwdSplitPlan {
     int nsplit = 1, chunks = 1 << 30, least = 0;
 };
 FwdSplitPlan fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus);
+// Whether a launch walks its lists in two halves (sparse_fwd_kernel<..., TW>) where they are not shared: sparse_fwd_merge.hip.
+bool fwd_in_halves(int64_t tiles, int Sk, int BQ, int BK, int D, int dtype, int cus);
 // Adds up the parts of shared lists (dtype 2: float32 output).
 hipError_t launch_fwd_merge(const FwdParams &p, int dtype, int D, int BQ, hipStream_t stream);
 

@@ -10,6 +10,7 @@ hipError_t launch_fwd_variant(const FwdParams &p, int D, int BQ, hipStream_t str
     extern template hipError_t launch_fwd_variant<DT, PK, HOW>(const FwdParams &, int, int, hipStream_t);
 SA_DECL(0, false, 0) SA_DECL(0, false, 1) SA_DECL(0, false, 2) SA_DECL(0, true, 0) SA_DECL(0, true, 1) SA_DECL(0, true, 2)
 SA_DECL(0, true, 3) SA_DECL(1, true, 3)
+SA_DECL(0, false, 4) SA_DECL(0, true, 4) SA_DECL(1, false, 4) SA_DECL(1, true, 4)
 SA_DECL(1, false, 0) SA_DECL(1, false, 1) SA_DECL(1, false, 2) SA_DECL(1, true, 0) SA_DECL(1, true, 1) SA_DECL(1, true, 2)
 #undef SA_DECL
 
@@ -21,6 +22,7 @@ hipError_t by_hand_out(const FwdParams &p, int D, int BQ, hipStream_t stream) {
         if constexpr (PK) return launch_fwd_variant<DT, PK, 3>(p, D, BQ, stream);
         else return hipErrorInvalidValue;
     }
+    if (p.halves) return launch_fwd_variant<DT, PK, 4>(p, D, BQ, stream);
     if (p.nsplit <= 1) return launch_fwd_variant<DT, PK, 0>(p, D, BQ, stream);
     const hipError_t e = launch_fwd_variant<DT, PK, 2>(p, D, BQ, stream);
     return e != hipSuccess ? e : launch_fwd_merge(p, DT, D, BQ, stream);

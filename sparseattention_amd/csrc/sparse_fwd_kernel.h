@@ -36,6 +36,7 @@ namespace {
 // then do their vector and scalar work together, with the pipe idle.  Letting the wave in its P.V phase (MFMAs
 // with exponentials between them) go ahead of one in its S phase (MFMAs only), and either ahead of the
 // bookkeeping between chunks, keeps them apart: 3 % on the causal and 2 % on the dense workload at D = 128.
+constexpr int kHalvesSync = 256;  // (TW) bytes for the count of a half's arrivals
 constexpr int kPrioS = 1;
 constexpr int kPrioPV = 2;
 
@@ -76,11 +77,17 @@ __device__ __forceinline__ void wait_vm_at_most(int n, int step) {
 // every lane 16 bytes), keys before the first and behind the last one as that one, which the mask of their tile leaves
 // out, and what has no place in the output is not stored.  The address of a direct load is formed per lane then, some six
 // instructions each.  B2 H16 S1499 D80 against padding q, k, v and cutting the result (14 launches): 82 -> 22 us.
-template <int DT, int D, int NW, int MODE, int NS, bool PP, bool PK, bool PS, bool SP, bool RG>
-__global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse_fwd_kernel(const FwdParams p) {
+// TW: the list of a Q tile is walked in two halves by two times NW waves of one workgroup, for launches of no more Q tiles than
+// compute units (fwd_in_halves, with times): the second half takes the registers and the LDS that a second workgroup would.  Each
+// half has its own stages and its own copy of its part of the list; the second one leaves its rows in LDS, the first one adds
+// them up.  Two waves per SIMD are bound by the matrix pipe (1.8 us for a chunk of each, at D = 128), a lone one by its own
+// serial phases (0.95 us a chunk), so what halves gain is the shorter tail of an uneven launch and, at BLOCK_Q = 64, the idle SIMDs.
+template <int DT, int D, int NW, int MODE, int NS, bool PP, bool PK, bool PS, bool SP, bool RG, bool TW>
+__global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 : 1) void sparse_fwd_kernel(const FwdParams p) {
     static_assert(!PS || (!PP && NS == 2), "persistent workgroups use the two-stage loop");
     static_assert(!SP || (!PS && !PP && D <= 128), "shared lists use the plain loop");
     static_assert(!RG || (PK && !SP && !PS && !PP && D <= 128), "ragged sizes use the plain loop and packed tiles");
+    static_assert(!TW || (!SP && !PS && !PP && !RG && NS == 2 && D <= 128), "two halves use the plain loop");
     using E = Elem<DT>;
     constexpr int ROWB = D * 2;                   // bytes per K/V row in LDS
     constexpr int KBUF = 64 * ROWB, VBUF = 64 * ROWB;
@@ -91,13 +98,26 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
     constexpr int LBKC = MODE == 0 ? 4 : 5;                   // log2(BK) when MODE < 2
     static_assert(64 % (RPI * NW) == 0, "staging layout");
 
-    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem0[];
     static_assert(NS == 2 || NS == 4, "stage count");
-    // [K stage 0..NS-1][V stage 0..NS-1][first key column of every list entry, kListCap ints]
+    // [K stage 0..NS-1][V stage 0..NS-1][first key column of every list entry, kListCap ints]; TW: a set per half
+    constexpr int HALF_BYTES = NS * KBUF + NS * VBUF + kListCap * 4 + (TW ? kHalvesSync : 0);
+    const int half = TW ? __builtin_amdgcn_readfirstlane(threadIdx.x / (NW * 64)) : 0;  // which half this wave belongs to
+    // (TW) lists of up to this many chunks are walked by the first half alone: of 13 on (BLOCK_Q 128) or 5 (64) two are faster
+    constexpr int LEAST = NW == 4 ? 10 : 4;
+    uint8_t *const smem = smem0 + half * HALF_BYTES;
     int *const ent = reinterpret_cast<int *>(smem + NS * KBUF + NS * VBUF);
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = TW ? threadIdx.x % (NW * 64) : threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l32 = lane & 31, hh = lane >> 5;
+    uint32_t *const arrived = reinterpret_cast<uint32_t *>(smem + HALF_BYTES - kHalvesSync);  // (TW, see meet)
+    if (TW && tid == 0) __hip_atomic_store(arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    // (once per half, behind the counts' round trip: the counts of arrivals are 0; no wait for loads under way)
+    auto both_start = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    };
 
     // Workgroup -> (b, h, Q tile).  Hardware hands consecutive workgroup ids to the 8 XCDs in turn; the
     // remap gives each XCD whole planes (every eighth pair of the (b,h)-major order) so that the Q tiles sharing one
@@ -227,16 +247,23 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
         // past a count hold anything; early_entry() picks the ones that count.
         const int32_t *const fl0 = p.full_lens + (b0 * p.fls[0] + h0 * p.fls[1] + qt0 * p.fls[2]);
         const int32_t *const pl0 = p.part_lens + (b0 * p.pls[0] + h0 * p.pls[1] + qt0 * p.pls[2]);
-        if constexpr (SP) {
+        if (SP || half == 1) {
             // (the counts say where this workgroup's part of the list begins, so they come by a round trip of their own)
             load_q(b0, h0, qt0);
             int cnt[2];
             const int32_t *const cnt_addr[2] = {fl0, pl0};
             scalar_gather(cnt_addr, cnt);
             set_item(b0, h0, qt0, cnt[0], cnt[1]);
-            share = fwd_split_share(NE, p.lbk, 6, p.split_least, p.split_chunks, p.nsplit);
-            share_part = s0;
-            if (s0 >= share) return;
+            if constexpr (TW) {
+                both_start();
+                if (T <= LEAST) return;  // (the first half has it all)
+                share = 2;
+                s0 = 1;
+            } else {
+                share = fwd_split_share(NE, p.lbk, 6, p.split_least, p.split_chunks, p.nsplit);
+                share_part = s0;
+                if (s0 >= share) return;
+            }
             const int e_lo = fwd_split_first(NE, p.lbk, 6, s0, share), e_hi = fwd_split_first(NE, p.lbk, 6, s0 + 1, share);
             const int f_lo = min(e_lo, F), p_lo = max(e_lo - F, 0);
             fid += f_lo * p.fis[3];
@@ -280,6 +307,13 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
                 early_p[i] = got[2 + EPC + i];
             });
             set_item(b0, h0, qt0, got[0], got[1]);
+            if constexpr (TW) both_start();
+            if (TW && T > LEAST) {
+                share = 2;
+                NE = fwd_split_first(NE, p.lbk, 6, 1, 2);
+                F = min(F, NE);
+                T = chunks_of(NE);
+            }
         } else {
             set_item(b0, h0, qt0, *fl0, *pl0);
         }
@@ -414,6 +448,22 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
         int x = e - rot_first - rot_by;
         if (x < 0) x += rot_n;
         return rot_first + x;
+    };
+    // A barrier among the waves that share stages.  TW: the halves do not wait for each other at every chunk; in step they want the
+    // matrix pipe together and leave it together (kPrioS; 64 chunks 66.3 us so, 63.1 apart).  So each half counts its own waves'
+    // arrivals in LDS.  All waves of a half are resident and meet equally often (T is one value), so every wait ends.
+    // (A lone first half takes the workgroup's barrier, which waits for the waves there still are: a count costs 0.1 us more.)
+    uint32_t met = 0;
+    auto meet = [&]() {
+        if (TW && share == 2) {
+            met += NW;
+            asm volatile("" ::: "memory");
+            if (lane == 0) __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+            while (__hip_atomic_load(arrived, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < met) {}
+            asm volatile("" ::: "memory");
+        } else {
+            __syncthreads();
+        }
     };
     auto copy_list = [&]() {
         if (list_in_lds) {
@@ -1152,7 +1202,7 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
         } else {
             copy_list();
         }
-        __syncthreads();  // the list in LDS is complete
+        meet();  // the list in LDS is complete
         if constexpr (kEarlyFirstChunk) {
             scale_q();
         } else {
@@ -1174,7 +1224,7 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
         for (int c = 0; c < D / 16; c++) asm volatile("" ::"v"(qf[c]));
         settle(mk[0]);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
+        meet();
         // Two chunks per trip so that the LDS stage is a compile-time constant.  Iteration tc computes chunk tc
         // while chunk tc+1 is fetched (its pieces go out between the S bundles) and, during the P.V phase, turns
         // the list entries of chunk tc+2 into the fetch plan of the next iteration.  Indices past the last chunk
@@ -1216,7 +1266,7 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
                     sp[cur] = sp2;
                     vl[cur] = valid2;
                     pt[cur] = part2;
-                    __syncthreads();
+                    meet();
                 }
             });
         }
@@ -1239,28 +1289,63 @@ __global__ __launch_bounds__(NW * 64, (NW >= 4 && D <= 128) ? 2 : 1) void sparse
             return;
         }
     }
+    if (TW && share == 2) {
+        // The second half's rows go through its own stages, which nobody reads any more, their state through its list.
+        static_assert(!TW || (NW * 32 * D * 4 <= NS * (KBUF + VBUF) && NW * 32 * 8 <= kListCap * 4), "the rows of a half fit its stages");
+        uint8_t *const second = smem0 + HALF_BYTES;
+        float *const rows = reinterpret_cast<float *>(second) + wave_u * (32 * D) + 4 * lane;
+        f32x2 *const state = reinterpret_cast<f32x2 *>(second + NS * KBUF + NS * VBUF) + wave * 32 + l32;
+        const float m = raise_above == kMaxSlack ? m_ref : kNegInf, l = l32 < 16 ? acc_l[0] : acc_l[1];
+        if (half == 1) {
+#pragma unroll
+            for (int db = 0; db < D / 32; db++)
+#pragma unroll
+                for (int g = 0; g < 4; g++)
+                    *(f32x4 *)(rows + 256 * (4 * db + g)) = f32x4{acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]};
+            if (hh == 0) *state = f32x2{m, l};
+        }
+        __syncthreads();
+        if (half == 1) return;
+        const f32x2 other = *state;
+        const float M = fmaxf(m, other.x), M0 = M == kNegInf ? 0.f : M;  // (no half saw an attended key: both weights are 0)
+        const float w0 = __builtin_amdgcn_exp2f(m - M0), w1 = __builtin_amdgcn_exp2f(other.x - M0);
+#pragma unroll
+        for (int db = 0; db < D / 32; db++)
+#pragma unroll
+            for (int g = 0; g < 4; g++) {
+                const f32x4 x = *(const f32x4 *)(rows + 256 * (4 * db + g));
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[db][4 * g + e] = __builtin_fmaf(acc[db][4 * g + e], w0, w1 * x[e]);
+            }
+        acc_l[0] = acc_l[1] = __builtin_fmaf(l, w0, w1 * other.y);
+        m_ref = M0;
+    }
     store_o_rows();
 }
 
-// HOW 0: one workgroup per Q tile, 1: persistent workgroups, 2: lists shared by workgroups (SP), 3: ragged sizes (RG)
+// HOW 0: one workgroup per Q tile, 1: persistent workgroups, 2: lists shared by workgroups (SP), 3: ragged sizes (RG),
+// 4: lists walked in two halves (TW)
 template <int DT, int D, int NW, int MODE, bool PK, int HOW>
 hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
     // Eight waves fill a CU's register file on their own, so that workgroup can have most of the LDS: 4 stages.
     constexpr int NS = NW == 8 ? 4 : 2;
     static_assert(kListCap == 2 * kPsListCap, "one long list or two short ones in the same LDS");
-    constexpr int smem = 2 * NS * 64 * D * 2 + kListCap * 4;  // NS stages of 64 rows for K and for V + the list(s)
-    auto kern = sparse_fwd_kernel<DT, D, NW, MODE, NS, NW == 8, PK, HOW == 1, HOW == 2, HOW == 3>;
+    constexpr int HALVES = HOW == 4 ? 2 : 1;
+    constexpr int smem = HALVES * (2 * NS * 64 * D * 2 + kListCap * 4 + (HOW == 4 ? kHalvesSync : 0));  // NS stages of 64 rows for K and for V + the list(s)
+    auto kern = sparse_fwd_kernel<DT, D, NW, MODE, NS, NW == 8, PK, HOW == 1, HOW == 2, HOW == 3, HOW == 4>;
     static unsigned long long attr_done = 0;  // devices on which this kernel may use `smem` bytes of LDS
     if (const hipError_t e0 = allow_dynamic_smem(kern, smem, attr_done); e0 != hipSuccess) return e0;
     const unsigned grid = HOW == 1 ? (unsigned)p.sched_G
                                    : (unsigned)p.nQ * (unsigned)p.B * (unsigned)p.H * (HOW == 2 ? (unsigned)p.nsplit : 1u);
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(NW * 64), smem, stream, p);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(HALVES * NW * 64), smem, stream, p);
     return hipGetLastError();
 }
 
 template <int DT, int D, int NW, bool PK, int HOW>
 hipError_t launch_mode(const FwdParams &p, hipStream_t stream) {
-    if (p.BK == 16) return launch_one<DT, D, NW, 0, PK, HOW>(p, stream);
+    if constexpr (HOW == 4) {  // (four entries a chunk and two halves take more scalar registers than there are)
+        if (p.BK == 16) return hipErrorInvalidValue;
+    } else if (p.BK == 16) return launch_one<DT, D, NW, 0, PK, HOW>(p, stream);
     if (p.BK == 32) return launch_one<DT, D, NW, 1, PK, HOW>(p, stream);
     return launch_one<DT, D, NW, 2, PK, HOW>(p, stream);
 }
@@ -1269,13 +1354,13 @@ template <int DT, int D, bool PK, int HOW>
 hipError_t launch_bq(const FwdParams &p, int BQ, hipStream_t stream) {
     switch (BQ) {
         case 32:
-            if constexpr (D > 128) return hipErrorInvalidValue;  // a lone wave would spill its registers there
+            if constexpr (D > 128 || HOW == 4) return hipErrorInvalidValue;  // a lone wave would spill its registers there
             else return launch_mode<DT, D, 1, PK, HOW>(p, stream);
         case 64: return launch_mode<DT, D, 2, PK, HOW>(p, stream);
         case 128: return launch_mode<DT, D, 4, PK, HOW>(p, stream);
         case 256:
             // 8-wave workgroups have the plain form only, and their four stages do not fit the LDS at D = 256
-            if constexpr (HOW != 0 || D > 128) return hipErrorInvalidValue;
+            if constexpr (HOW != 0 || D > 128) return hipErrorInvalidValue;  // (HOW 4 too: it has eight waves at BLOCK_Q 128)
             else return launch_mode<DT, D, 8, PK, 0>(p, stream);
         default: return hipErrorInvalidValue;
     }

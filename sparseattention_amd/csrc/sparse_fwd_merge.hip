@@ -98,7 +98,8 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(const FwdParams p, int l
 //      65 tiles  16 chunks  19.8 | alone 22.8    17  21.1 | 22.6    20  23.5 | 23.6    64  63.8 | 36.2
 //      96 tiles  17 chunks  21.2 | 25.1          20  23.6 | 26.3    24  27.4 | 28.2    64  64.1 | 39.4
 //     128 tiles  16 chunks  20.3 | alone 22.9    17  21.1 | 27.2    24  27.2 | 30.5    28  31.0 | 32.1    64  64.8 | 46.3
-//   parts of 48 chunks, up to cus tiles, where a second workgroup per compute unit is all there is to gain
+//   parts of 48 chunks, up to cus tiles, where a second workgroup per compute unit is all there is to gain (and lists are not
+//   walked in halves, see fwd_in_halves)
 //     192 tiles  32 chunks  35.1 | alone 38.2    49  51.8 | 52.0    64  67.3 | 62.4   128 125.5 | 107.5
 //     256 tiles  48 chunks  55.9 | alone 58.0    49  56.9 | 62.0    64  72.7 | 74.8   128 135.3 | 130.1   256  288 | 239
 // From 257 tiles on every slot has work.  Sk below 32 chunks is not shared, whatever the lists (32 chunks, Sk = 2048: 8 tiles
@@ -120,6 +121,26 @@ FwdSplitPlan fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus
     plan.chunks = part;
     plan.least = part == 16 ? 8 + tiles / 8 : part;
     return plan;
+}
+
+// When a list is walked in two halves by one workgroup of twice the waves (sparse_fwd_kernel<..., TW>): from half as many Q tiles
+// as compute units on, up to as many.  A compute unit has one workgroup then, which leaves half of its registers and LDS
+// idle, at BLOCK_Q = 64 two of its four SIMDs too.  No workspace, no second launch.  bf16 and fp16, us, one workgroup per list or
+// shared by two with a merge, as it was | halves:
+//   BLOCK_Q 128, Sk of more than 48 chunks, where lists were shared by two workgroups before
+//       256 tiles  causal Sk 4096  59.5 | 51.7   every key 4096  72.7 | 64.7   16384  239 | 236   D 64, 16384  143.2 | 142.5
+//                  window 64  12.5 | 10.5   256  15.1 | 13.1   900, BLOCK_K 32  26.6 | 22.9
+//   (with shorter rows the launch had no merge to save, and lists of up to 7 chunks would pay 1.4 us for the wider workgroup: 9.2 |
+//   10.6, 11.8 | 13.2; 13 and more gain: causal Sk 1024 21.4 | 20.2, every key of 2048 39.2 | 36.7)
+//   BLOCK_Q 64
+//       256 tiles  causal Sk 1024  24.5 | 17.8   causal Sk 4096, D 64  51.1 | 34.8   every key 8192  104.1 | 97.9
+//                  window 256  12.2 | 12.0   window 64 (lists of two chunks)  9.1 | 9.5
+//       160 tiles  causal Sk 1280  30.7 | 20.6   window 500  17.6 | 14.7
+// Up to two thirds as many tiles as compute units long lists are shared by three workgroups (136 tiles of 8192 keys: 78.1 | 88.9).
+bool fwd_in_halves(int64_t tiles, int Sk, int BQ, int BK, int D, int dtype, int cus) {
+    if (dtype == 2 || (D != 64 && D != 128) || BK < 32 || 2 * tiles <= cus || tiles > cus) return false;
+    if (3 * tiles <= 2 * cus && Sk > 96 * 64) return false;
+    return (BQ == 64 && Sk >= 1024) || (BQ == 128 && Sk > 48 * 64);
 }
 
 hipError_t launch_fwd_merge(const FwdParams &p, int dtype, int D, int BQ, hipStream_t stream) {

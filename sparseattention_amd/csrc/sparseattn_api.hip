@@ -269,6 +269,15 @@ size_t schedule_shape(int B, int H, int Sq, int Sk, int BQ, int BK, int mode, in
     return (size_t)G * (size_t)(R + 1) * 16;
 }
 
+// Whether lists are walked in two halves on the current device.
+bool in_halves(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype) {
+    if (B <= 0 || H <= 0 || Sq <= 0 || BQ <= 0 || Sq % BQ) return false;
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return false;
+    return sa::fwd_in_halves((int64_t)B * H * (Sq / BQ), Sk, BQ, BK, D, dtype, cus);
+}
+
 // How lists are shared on the current device, and the bytes of the partial results (0: they are not).
 size_t split_shape(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype, sa::FwdSplitPlan *plan) {
     *plan = sa::FwdSplitPlan();
@@ -277,7 +286,7 @@ size_t split_shape(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtyp
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-    if (tiles > 2 * cus) return 0;
+    if (tiles > 2 * cus || sa::fwd_in_halves(tiles, Sk, BQ, BK, D, dtype, cus)) return 0;
     *plan = sa::fwd_split_plan((int)tiles, Sk, BQ, D, dtype, cus);
     return plan->nsplit > 1 ? (size_t)tiles * (size_t)plan->nsplit * (size_t)BQ * (size_t)(D + 2) * 4 : 0;
 }
@@ -296,7 +305,7 @@ int forward_impl(const void *q, const int64_t q_strides[4], const void *k, const
                  size_t schedule_bytes, int schedule_mode, float *lse, const int64_t lse_strides[3], int B, int H,
                  int Sq, int Sk, int D, int BQ, int BK, int dtype, float sm_scale_log2, void *stream,
                  int kernel = SA_FWD_KERNEL_DEFAULT, void *workspace = nullptr, size_t workspace_bytes = 0,
-                 const Ragged *ragged = nullptr) {
+                 const Ragged *ragged = nullptr, bool other_order = false) {
     g_error[0] = 0;
     const int rot_group = kernel >> 8;
     kernel &= 0xff;
@@ -424,7 +433,8 @@ int forward_impl(const void *q, const int64_t q_strides[4], const void *k, const
         fp.D_in = ragged->D;
     }
     fp.nsplit = 1;
-    if (workspace && kernel == SA_FWD_KERNEL_DEFAULT && !fp.sched) {
+    fp.halves = other_order && in_halves(B, H, Sq, Sk, D, BQ, BK, dtype);
+    if (workspace && !fp.halves && kernel == SA_FWD_KERNEL_DEFAULT && !fp.sched) {
         sa::FwdSplitPlan plan;
         const size_t need = split_shape(B, H, Sq, Sk, D, BQ, BK, dtype, &plan);
         fp.nsplit = plan.nsplit;
@@ -583,7 +593,7 @@ int sa_sparse_attention_fwd_split(const void *q, const int64_t q_strides[4], con
     return forward_impl(q, q_strides, k, k_strides, v, v_strides, o, o_strides, mask, mask_strides, full_ids,
                         full_ids_strides, full_lens, full_lens_strides, part_ids, part_ids_strides, part_lens,
                         part_lens_strides, packed, packed_strides, use_packed, nullptr, 0, 0, lse, lse_strides, B, H, Sq,
-                        Sk, D, BQ, BK, dtype, sm_scale_log2, stream, SA_FWD_KERNEL_DEFAULT, workspace, workspace_bytes);
+                        Sk, D, BQ, BK, dtype, sm_scale_log2, stream, SA_FWD_KERNEL_DEFAULT, workspace, workspace_bytes, nullptr, true);
 }
 
 int sa_sparse_attention_fwd_ragged(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
