@@ -48,18 +48,18 @@ PEAK_FP32_TFLOPS = 157.3   # MI355X dense fp32 MFMA peak, TFLOP/s
 # `bench.py --traffic-probe` and scaled by what the same counters read for the 1 GiB device copy of the same run
 # (`bench.py --traffic-summary` does the arithmetic).  profiles/hbm_traffic_all_kernels.txt holds the commands.
 TRAFFIC_BYTES = {
-    "forward, causal": (852025685, 268435456),
-    "forward, dense": (808001520, 268435840),
-    "forward, p=0.25": (1352330401, 268435456),
-    "forward, p=0.5": (2847766570, 268435456),
-    "forward, p=0.75": (2943479415, 268435456),
-    "forward, p=0.9": (1418357710, 268435456),
-    "backward, causal": (8120977198, 5242880043),
-    "forward, documents": (1724719289, 536870912),
-    "forward, composed": (1614155656, 268435456),
-    "mask_classify, composed mask 1 GiB": (1074098168, 308736),
-    "decode, 1": (4295566835, 399904),
-    "decode, 16": (1617199728, 5680725),
+    "forward, causal": (831941342, 268435456),
+    "forward, dense": (807995205, 268435755),
+    "forward, p=0.25": (1368186604, 268435456),
+    "forward, p=0.5": (2837988926, 268435456),
+    "forward, p=0.75": (2940366482, 268435456),
+    "forward, p=0.9": (1384485039, 268435456),
+    "backward, causal": (8164298086, 5242880299),
+    "forward, documents": (1754596627, 536870912),
+    "forward, composed": (1612859641, 268435456),
+    "mask_classify, composed mask 1 GiB": (1074097997, 308736),
+    "decode, 1": (4295554888, 397312),
+    "decode, 16": (1617191364, 5677056),
 }
 TRAFFIC_SOURCE = "profiles/hbm_traffic_all_kernels.txt"
 # The sources each kernel is built from.  The counters were read with kernels built from sources of the digests in
@@ -71,8 +71,8 @@ KERNEL_FILES = {
     "decode": ("sparse_decode.hip", "fwd_common.h", "kernels.h"),
     "backward": ("sparse_bwd.hip", "fwd_common.h", "kernels.h"),
 }
-TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "347a6f7c4714fe47", "mask_classify": "f4df084b45a608b0", "decode": "90bacfebd04c22ca",
-                                "backward": "25028ac99815136a"}
+TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "8396152b14eeae54", "mask_classify": "bb816487f407821e", "decode": "4ae22d844fc72b96",
+                                "backward": "bafce1103391b245"}
 
 
 def kernel_sources_sha16(which=None):
