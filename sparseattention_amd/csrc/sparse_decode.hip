@@ -306,20 +306,30 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
         for (int i = 0; i < 16; i++) s[i] = 0.f;
         u32x4 ka[NC];  // the A operand: lane (l32, hh) holds d = (D/2) hh + 8c .. +7 of key l32
         if constexpr (KR) {
-            // (the operations of a wave on LDS take effect in their order)
+            // Lanes read what others have written and overwrite what others have read.  A wave's operations on LDS take effect in
+            // their order, so nothing waits here; the fence keeps the compiler, which sees one lane, to that order.
             const int r = l32 & 15;
+            auto in_order = [] {
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            };
+            in_order();
 #pragma unroll
             for (int i = 0; i < NLD / 2; i++) {
                 const int w = RPI * i + ld_r0;
                 *(u32x4 *)(kmine + w * ROWB + 16 * (ld_slot ^ k_swizzle<D>(w))) = kf[i];
             }
+            in_order();
 #pragma unroll
             for (int c = 0; c < NC; c++) ka[c] = *(const u32x4 *)(kmine + r * ROWB + 16 * ((NC * hh + c) ^ k_swizzle<D>(r)));
+            in_order();
 #pragma unroll
             for (int i = 0; i < NLD / 2; i++) {
                 const int w = RPI * i + ld_r0;
                 *(u32x4 *)(kmine + w * ROWB + 16 * (ld_slot ^ k_swizzle<D>(w))) = kf[NLD / 2 + i];
             }
+            in_order();
 #pragma unroll
             for (int c = 0; c < NC; c++) {
                 const u32x4 x = *(const u32x4 *)(kmine + r * ROWB + 16 * ((NC * hh + c) ^ k_swizzle<D>(r)));
