@@ -48,15 +48,15 @@ PEAK_FP32_TFLOPS = 157.3   # MI355X dense fp32 MFMA peak, TFLOP/s
 # `bench.py --traffic-probe` and scaled by what the same counters read for the 1 GiB device copy of the same run
 # (`bench.py --traffic-summary` does the arithmetic).  profiles/hbm_traffic_all_kernels.txt holds the commands.
 TRAFFIC_BYTES = {
-    "forward, causal": (831941342, 268435456),
-    "forward, dense": (807995205, 268435755),
-    "forward, p=0.25": (1368186604, 268435456),
-    "forward, p=0.5": (2837988926, 268435456),
-    "forward, p=0.75": (2940366482, 268435456),
-    "forward, p=0.9": (1384485039, 268435456),
+    "forward, causal": (850532316, 268435456),
+    "forward, dense": (807997573, 268436011),
+    "forward, p=0.25": (1347340537, 268435456),
+    "forward, p=0.5": (2865887374, 268435456),
+    "forward, p=0.75": (2932038323, 268435456),
+    "forward, p=0.9": (1422602923, 268435456),
     "backward, causal": (8164298086, 5242880299),
-    "forward, documents": (1754596627, 536870912),
-    "forward, composed": (1612859641, 268435456),
+    "forward, documents": (1727509875, 536870912),
+    "forward, composed": (1617125617, 268435456),
     "mask_classify, composed mask 1 GiB": (1074097997, 308736),
     "decode, 1": (4295555827, 397312),
     "decode, 16": (1617191706, 5677056),
@@ -71,7 +71,7 @@ KERNEL_FILES = {
     "decode": ("sparse_decode.hip", "fwd_common.h", "kernels.h"),
     "backward": ("sparse_bwd.hip", "fwd_common.h", "kernels.h"),
 }
-TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "8396152b14eeae54", "mask_classify": "bb816487f407821e", "decode": "602ae92e0769dce7",
+TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "ae96e018d98d7867", "mask_classify": "bb816487f407821e", "decode": "602ae92e0769dce7",
                                 "backward": "bafce1103391b245"}
 
 

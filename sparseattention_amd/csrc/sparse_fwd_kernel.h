@@ -451,15 +451,18 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
     };
     // A barrier among the waves that share stages.  TW: the halves do not wait for each other at every chunk; in step they want the
     // matrix pipe together and leave it together (kPrioS; 64 chunks 66.3 us so, 63.1 apart).  So each half counts its own waves'
-    // arrivals in LDS.  All waves of a half are resident and meet equally often (T is one value), so every wait ends.
+    // arrivals in LDS.  All waves of a half are resident and meet equally often: each has read the same counts.  Counts that someone
+    // writes while the kernel runs can differ from wave to wave; the result is worth nothing then, but as with a barrier, which
+    // does not wait for waves that have ended, the waiting ends: a wave looks at the count kMeetLooks times at most (seconds).
     // (A lone first half takes the workgroup's barrier, which waits for the waves there still are: a count costs 0.1 us more.)
-    uint32_t met = 0;
+    constexpr uint32_t kMeetLooks = 1u << 26;
+    uint32_t met = 0, looks = kMeetLooks;
     auto meet = [&]() {
         if (TW && share == 2) {
             met += NW;
             asm volatile("" ::: "memory");
             if (lane == 0) __hip_atomic_fetch_add(arrived, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-            while (__hip_atomic_load(arrived, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < met) {}
+            while (__hip_atomic_load(arrived, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < met && looks != 0) looks--;
             asm volatile("" ::: "memory");
         } else {
             __syncthreads();
