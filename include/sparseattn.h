@@ -427,16 +427,17 @@ int sa_sparse_attention_fwd_ragged(const void *q, const int64_t q_strides[4], co
  * BLOCK_Q = Sq; the reference has no kernel of its own for this shape ("Backwards pass + decode kernels" is item 3
  * of its README's list of what could come next, README.md:65), and its one-program-per-Q-tile launch
  * (sparse_attn_kernel.py:166) would leave one program per (b, h).  Here the list of every (b, h) is cut into
- * num_splits ranges of 32-key chunks, one workgroup each, and a second kernel merges the partial results.
+ * num_splits ranges of 32-key chunks, one workgroup each, whose partial results are merged by the last of them or by a
+ * second kernel (see workspace).
  *
  *   lists        output of sa_mask_classify for the same mask with BQ = Sq: shapes [B,H,1,Sk/BK] and [B,H,1]
  *                (stride entry 2 is ignored)
  *   BK           power of two >= 16
  *   num_splits   workgroups per (b, h), 1..256, or 0 for sa_decode_num_splits(...)
  *   workspace    sa_decode_workspace_bytes(...) bytes of device memory, 16-byte aligned (may be NULL when that is 0,
- *                i.e. for one split); contents on return are unspecified.  With sa_decode_workspace_bytes_ex(...) bytes
- *                (never fewer) the partial results are merged by the launch that makes them, to the same sums in another
- *                order; contents on entry are unspecified either way
+ *                i.e. for one split); contents on entry and on return are unspecified.  sa_decode_workspace_bytes_ex(...) is
+ *                more where the launch that makes the partial results can merge them sooner than a second one (few parts,
+ *                few rows) and needs counters for it; a call that has so many bytes does so, with the same bits
  *   lse, lse_strides   optional second output as in sa_sparse_attention_fwd_lse, or NULL
  * q, k, v, o, D, dtype, sm_scale_log2, stream: as for sa_sparse_attention_fwd.
  */

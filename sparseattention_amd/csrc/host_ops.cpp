@@ -344,13 +344,7 @@ Out decode_impl(const Tensor &q, const Tensor &k, const Tensor &v, const OptTens
     const Tensor o = at::empty_like(qc);
     const auto f32 = at::TensorOptions().dtype(at::kFloat).device(q.device());
     if (num_splits == 0) num_splits = sa_decode_num_splits(B, H, Sq, Sk, BK);
-    // The last workgroup of a plane merges where it does so sooner than a second launch: the workgroups of a plane count in one word,
-    // half a microsecond each, and one workgroup adds up all rows.  us, second launch -> last workgroup, lists made in the call:
-    //   parts of one row  8  14.5 -> 12.3   16  29.0 -> 34.8   32  14.6 -> 23.6   64  33.4 -> 53.8
-    //   rows, D = 128     8 x 4 16.8 -> 15.2   8 x 8 18.7 -> 16.1   8 x 16 26.7 -> 23.6   2 x 16 13.7 -> 13.5   2 x 32 15.4 -> 16.0
-    //   rows, D = 64      8 x 4 12.2 -> 10.6   8 x 8 12.7 -> 13.5   8 x 16 14.5 -> 15.2   2 x 16 10.4 -> 10.3   2 x 32 12.0 -> 12.4
-    const bool last_merges = num_splits <= 8 && Sq <= 16 && num_splits * Sq <= (Dk == 128 ? 128 : 32);
-    const size_t ws_bytes = last_merges ? sa_decode_workspace_bytes_ex(B, H, Sq, Dk, num_splits) : sa_decode_workspace_bytes(B, H, Sq, Dk, num_splits);
+    const size_t ws_bytes = sa_decode_workspace_bytes_ex(B, H, Sq, Dk, num_splits);
     Tensor ws;
     if (ws_bytes) ws = at::empty({(int64_t)(ws_bytes / 4)}, f32);
     OptTensor lse;

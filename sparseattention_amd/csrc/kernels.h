@@ -202,7 +202,18 @@ hipError_t launch_fwd_f32_mfma(const FwdParams &p, int D, int BQ, hipStream_t st
 // workgroup of the plane reads the whole mask, and a lane goes over a tile.
 constexpr int kDecodeDirectEntries = 32768;
 constexpr int kDecodeDirectBK = 256;
-constexpr int kDecodeMergeRows = 128;  // partial rows (parts x query rows) of a plane that its last workgroup merges: LDS holds them
+// Whether the last workgroup of a plane to arrive merges its parts (else a second launch does).  It does where that is sooner: the
+// workgroups of a plane count in one word, half a microsecond each, and one workgroup adds up all rows.  us, second launch -> last
+// workgroup, lists made in the call:
+//   parts of one row  8  14.5 -> 12.3   16  29.0 -> 34.8   32  14.6 -> 23.6   64  33.4 -> 53.8
+//   rows, D = 128     8 x 4 16.8 -> 15.2   8 x 8 18.7 -> 16.1   8 x 16 26.7 -> 23.6   2 x 16 13.7 -> 13.5   2 x 32 15.4 -> 16.0
+//   rows, D = 64      8 x 4 12.2 -> 10.6   8 x 8 12.7 -> 13.5   8 x 16 14.5 -> 15.2   2 x 16 10.4 -> 10.3   2 x 32 12.0 -> 12.4
+// Up to kDecodeMergeFew parts both add a row's parts up one after the other: the same bits.
+constexpr int kDecodeMergeFew = 8;
+constexpr int kDecodeMergeRows = 128;  // partial rows of a plane that LDS holds
+inline bool decode_merges_in_launch(int64_t nsplit, int64_t Sq, int D) {
+    return nsplit > 1 && nsplit <= kDecodeMergeFew && Sq <= 16 && nsplit * Sq <= (D == 128 ? kDecodeMergeRows : 32);
+}
 struct DecodeParams {
     const uint16_t *q, *k, *v;
     uint16_t *o;

@@ -22,7 +22,6 @@ namespace sa {
 namespace {
 
 constexpr int kDecodeWaves = 4;
-constexpr int kMergeFew = 8;  // parts up to which a row's are added up one after the other
 
 // Where K comes as whole rows.  Two workgroups with the 16 rows that this takes of each wave's share have all of a compute unit's LDS,
 // none is left for lists made in the kernel.  us, K per lane | as rows, K and V not in a cache (a call's own are a layer's of many):
@@ -37,7 +36,8 @@ template <int D, bool KR>
 constexpr int decode_smem_bytes() {
     // per wave two V stages of 32 rows and, where K comes as whole rows, 16 rows of it
     constexpr int stream = kDecodeWaves * (2 * 32 + (KR ? 16 : 0)) * D * 2;
-    constexpr int merge = kDecodeWaves * 32 * (D + 2) * 4 + 16;   // per wave 32 rows of D + 2 floats (kDecodeMergeRows)
+    constexpr int merge = kDecodeWaves * 32 * (D + 2) * 4 + 16;   // per wave 32 rows of D + 2 floats; the parts of a plane
+    static_assert(kDecodeMergeRows <= kDecodeWaves * 32, "LDS holds the parts that the last workgroup merges");
     return stream > merge ? stream : merge;
 }
 
@@ -518,23 +518,11 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     float *const all = part + lead / 4;
-    const int stride = p.Sq * PST;
-    int n = p.nsplit;
-    if (n > kMergeFew) {  // the waves share the parts first, each into the first one of its own
-        float *const own = all + wave_u * stride;
-        add_up(own, (n - wave_u + kDecodeWaves - 1) / kDecodeWaves, kDecodeWaves * stride, r0, RPW, [&](int row, f32x4 x, float M, float L) {
-            *(f32x2 *)(own + row * PST + 4 * l) = f32x2{x.x, x.y};
-            *(f32x2 *)(own + row * PST + 4 * l + 2) = f32x2{x.z, x.w};
-            if (l == 0) *(f32x2 *)(own + row * PST + D) = f32x2{M, L};
-        });
-        n = kDecodeWaves;
-        __syncthreads();
-    }
-    add_up(all, n, stride, first, step, to_output);
+    add_up(all, p.nsplit, p.Sq * PST, first, step, to_output);
 }
 
-// Merge of the nsplit partial results of every (b, h) in a launch of its own, where LDS does not hold them or the workspace has no
-// place for the counters: grid B*H, 256 threads, 8 per query row.
+// Merge of the nsplit partial results of every (b, h) in a launch of its own, where that is sooner (decode_merges_in_launch) or the
+// workspace has no place for the counters: grid B*H, 256 threads, 8 per query row.
 template <int DT, int D>
 __global__ __launch_bounds__(256) void decode_merge_kernel(const DecodeParams p) {
     using E = Elem<DT>;
@@ -554,7 +542,7 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(const DecodeParams p)
     for (int j = 0; j < NV; j += 2) *(uint32_t *)(orow + j) = E::pack2(out[j] * inv, out[j + 1] * inv);
 }
 
-// The same for more than kMergeFew parts: one wave per query row, four per workgroup.  Eight lanes share a part (two
+// The same for more than kDecodeMergeFew parts: one wave per query row, four per workgroup.  Eight lanes share a part (two
 // neighbouring floats of every 16 each, so a part is read in runs of 64 bytes), eight parts go side by side and kMergeBatch
 // reads of each are in flight.  The parts lie in a cache and are few: all of this is latency, and the kernel above, which
 // walks them one after the other, took most of a call with many (bf16, D = 128, Sq1; classification, decode and merge):
@@ -688,7 +676,7 @@ hipError_t launch_decode_kind(const DecodeParams &p, hipStream_t stream) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || p.nsplit == 1 || p.arrivals != nullptr) return e;
     const unsigned rows = (unsigned)p.B * p.H * p.Sq;  // (at most 65535 planes of 32 rows)
-    if (p.nsplit > kMergeFew) hipLaunchKernelGGL((decode_merge_many_kernel<DT, D>), dim3((rows + 3) / 4), dim3(256), 0, stream, p);
+    if (p.nsplit > kDecodeMergeFew) hipLaunchKernelGGL((decode_merge_many_kernel<DT, D>), dim3((rows + 3) / 4), dim3(256), 0, stream, p);
     else hipLaunchKernelGGL((decode_merge_kernel<DT, D>), dim3(p.B * p.H), dim3(256), 0, stream, p);
     return hipGetLastError();
 }

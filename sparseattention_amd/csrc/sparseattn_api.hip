@@ -951,7 +951,7 @@ size_t sa_decode_workspace_bytes(int B, int H, int Sq, int D, int num_splits) {
 
 size_t sa_decode_workspace_bytes_ex(int B, int H, int Sq, int D, int num_splits) {
     const size_t least = sa_decode_workspace_bytes(B, H, Sq, D, num_splits);
-    return least != 0 && num_splits * Sq <= sa::kDecodeMergeRows ? (least + 7) / 8 * 8 + (size_t)B * H * 8 : least;
+    return least != 0 && sa::decode_merges_in_launch(num_splits, Sq, D) ? (least + 7) / 8 * 8 + (size_t)B * H * 8 : least;
 }
 
 }  // extern "C"
@@ -1055,7 +1055,7 @@ int decode_impl(const void *q, const int64_t q_strides[4], const void *k, const 
                        : 0;
     dp.nsplit = num_splits;
     dp.ws = static_cast<float *>(workspace);
-    if (need != 0 && num_splits * Sq <= sa::kDecodeMergeRows && workspace_bytes >= sa_decode_workspace_bytes_ex(B, H, Sq, D, num_splits)) {
+    if (need != 0 && sa::decode_merges_in_launch(num_splits, Sq, D) && workspace_bytes >= sa_decode_workspace_bytes_ex(B, H, Sq, D, num_splits)) {
         dp.arrivals = reinterpret_cast<uint64_t *>(static_cast<uint8_t *>(workspace) + (need + 7) / 8 * 8);
         dp.tag = next_launch_tag();
     }
