@@ -125,22 +125,33 @@ FwdSplitPlan fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus
 
 // When a list is walked in two halves by one workgroup of twice the waves (sparse_fwd_kernel<..., TW>): from half as many Q tiles
 // as compute units on, up to as many.  A compute unit has one workgroup then, which leaves half of its registers and LDS
-// idle, at BLOCK_Q = 64 two of its four SIMDs too.  No workspace, no second launch.  bf16 and fp16, us, one workgroup per list or
-// shared by two with a merge, as it was | halves:
-//   BLOCK_Q 128, Sk of more than 48 chunks, where lists were shared by two workgroups before
-//       256 tiles  causal Sk 4096  59.5 | 51.7   every key 4096  72.7 | 64.7   16384  239 | 236   D 64, 16384  143.2 | 142.5
-//                  window 64  12.5 | 10.5   256  15.1 | 13.1   900, BLOCK_K 32  26.6 | 22.9
-//   (with shorter rows the launch had no merge to save, and lists of up to 7 chunks would pay 1.4 us for the wider workgroup: 9.2 |
-//   10.6, 11.8 | 13.2; 13 and more gain: causal Sk 1024 21.4 | 20.2, every key of 2048 39.2 | 36.7)
-//   BLOCK_Q 64
-//       256 tiles  causal Sk 1024  24.5 | 17.8   causal Sk 4096, D 64  51.1 | 34.8   every key 8192  104.1 | 97.9
+// idle, at BLOCK_Q = 64 two of its four SIMDs too.  No workspace, no second launch; but a long list stays on its compute unit,
+// where parts of it would go to units whose own lists are short.  bf16 and fp16, us, D = 128 where not said:
+//   BLOCK_Q 128, Sk of 49 to 72 chunks, or 96 where every compute unit has a tile.  Shared by two with a merge | halves, lists that
+//   grow evenly from an eighth of the keys to all ("causal") and lists of all keys:
+//       136 tiles  causal  64 chunks 63.0 | 51.6   72 60.5 | 56.6   80 61.3 | 61.7    96 70.8 | 72.3    all  96 73.6 | 73.4
+//       192 tiles  causal  64        58.9 | 51.7   72 57.5 | 57.4   96 71.7 | 73.0   192 122.6 | 138.4  all  96 83.3 | 79.0   192 148.8 | 148.8
+//       240 tiles  causal  64        62.1 | 54.0   72 61.1 | 60.3   88 69.8 | 72.5   192 134.7 | 147.2  all  96 95.9 | 90.8
+//       256 tiles  causal  64        62.0 | 54.9   80 69.3 | 67.4   96 79.0 | 78.9   192 146.6 | 149.5  all  96 99.9 | 94.2   192 178.9 | 178.9
+//       D = 64     causal  224 tiles 72 chunks 41.5 | 41.8   88 45.9 | 49.0    256 tiles  72 41.9 | 42.1   96 52.9 | 53.3
+//       256 tiles  window 64  12.5 | 10.5   256  15.1 | 13.1   900, BLOCK_K 32  26.6 | 22.9
+//   (with shorter rows the launch had no merge to save, and lists of up to 12 chunks would pay 1.1 us for the wider workgroup: 9.2 |
+//   10.6, 11.8 | 13.2; longer ones gain little: causal Sk 1024 21.4 | 20.2, every key of 2048 39.2 | 36.7)
+//   BLOCK_Q 64, one workgroup per list (Sk up to 48 chunks) or shared by two with a merge | halves
+//       256 tiles  causal  16 chunks 24.5 | 17.8   64, D = 64 51.1 | 34.8   256 203.0 | 197.4   all 128 104.6 | 96.6
 //                  window 256  12.2 | 12.0   window 64 (lists of two chunks)  9.1 | 9.5
 //       160 tiles  causal Sk 1280  30.7 | 20.6   window 500  17.6 | 14.7
-// Up to two thirds as many tiles as compute units long lists are shared by three workgroups (136 tiles of 8192 keys: 78.1 | 88.9).
+//       192 tiles  causal  128 100.6 | 96.5   256 191.0 | 185.4         (D = 64: 77.3 | 72.6, 145.9 | 139.5)
+//       224 tiles  causal   96  76.1 | 74.3   128  98.3 | 99.8   256 188.3 | 193.0   (D = 64: 80.2 | 72.4, 141.3 | 140.3)
+//       240 tiles  causal   96  76.2 | 75.5   128  99.2 | 104.2  256 188.2 | 201.3
+// Up to two thirds as many tiles as compute units lists of more than 96 chunks are shared by three workgroups (BLOCK_Q 128, 136 tiles of
+// 8192 keys: 78.1 | 88.9).
 bool fwd_in_halves(int64_t tiles, int Sk, int BQ, int BK, int D, int dtype, int cus) {
     if (dtype == 2 || (D != 64 && D != 128) || BK < 32 || 2 * tiles <= cus || tiles > cus) return false;
-    if (3 * tiles <= 2 * cus && Sk > 96 * 64) return false;
-    return (BQ == 64 && Sk >= 1024) || (BQ == 128 && Sk > 48 * 64);
+    if (BQ == 128) return Sk > 48 * 64 && Sk <= (tiles == cus ? 96 : 72) * 64;
+    if (BQ != 64 || Sk < 1024) return false;
+    if (Sk <= 96 * 64) return true;
+    return 3 * tiles > 2 * cus && (D == 64 || 4 * tiles <= 3 * cus || tiles == cus);
 }
 
 hipError_t launch_fwd_merge(const FwdParams &p, int dtype, int D, int BQ, hipStream_t stream) {

@@ -58,6 +58,18 @@ def test_halves_against_float64(gpu, dtype, B, H, Sq, Sk, D, BQ, BK, packed):
             assert (lse[b, :3] - want_lse)[live[b, :3]].abs().max() <= 16 * eps
 
 
+# (tiles in 1/256 of the compute units: lists that differ in length finish sooner in parts than in halves there, and were shared before)
+@pytest.mark.parametrize("tiles,chunks,D,BQ", [(136, 73, 128, 128), (136, 96, 64, 128), (176, 128, 128, 128), (192, 192, 128, 128), (224, 80, 64, 128),
+                                               (240, 256, 128, 128), (255, 96, 128, 128), (256, 97, 128, 128), (256, 256, 64, 128),
+                                               (136, 97, 64, 64), (170, 97, 128, 64), (224, 128, 128, 64), (240, 256, 128, 64), (255, 97, 128, 64)])
+def test_long_uneven_lists_are_shared(gpu, tiles, chunks, D, BQ):
+    cus = torch.cuda.get_device_properties(gpu).multi_processor_count
+    if cus % 256:
+        pytest.skip("the numbers are those of 256 compute units")
+    lib = _native.load()
+    assert lib.sa_fwd_split_workspace_bytes(1, tiles * cus // 256, BQ, 64 * chunks, D, BQ, 64, 0) > 0
+
+
 def test_halves_with_infinite_values_and_entries_out_of_range(gpu):
     """What a list does not name does not reach the result; an entry outside K leaves other Q tiles alone and is left out."""
     B, H, Sq, Sk, D, BQ, BK = 1, 32, 1024, 3200, 128, 128, 64
