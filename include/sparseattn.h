@@ -388,8 +388,9 @@ int sa_sparse_attention_fwd_kernel(const void *q, const int64_t q_strides[4], co
  *               default kernel, or a kernel that walks a list in two halves by the waves of one workgroup).  The bytes depend
  *               on the current device.
  * Results agree with the default kernel within rounding (a row's keys are added up in other groups).
- * sa_fwd_split_least_keys: lists of up to that many keys are walked by one workgroup all the same (Sk where all are); a caller
- * who knows that no list is longer does without the workspace and saves the second launch.
+ * sa_fwd_split_least_keys: this entry gains nothing on lists of up to that many keys (Sk: on none); a caller who knows that no
+ * list is longer calls sa_sparse_attention_fwd_kernel with the default kernel and saves the workspace, the second launch or the
+ * wider workgroups.
  */
 size_t sa_fwd_split_workspace_bytes(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype);
 int sa_fwd_split_least_keys(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype);

@@ -432,6 +432,28 @@ std::string forward_kernel(const Tensor &q, int64_t BQ, int64_t BK, py::object m
     return code == SA_FWD_KERNEL_SHORT_LISTS ? "short" : code == SA_FWD_KERNEL_ROTATED ? "rotated" : "default";
 }
 
+// How a call with the default kernel hands its lists out: one workgroup each, or as sa_sparse_attention_fwd_split does (which needs
+// ws_bytes).  Metadata that says that no list is long enough to gain by it (list_stats) keeps them whole: 128 tiles of 16 chunks
+// 22.9 -> 20.0 us, no merge that finds nothing; 256 tiles of 64 rows, lists of 4 chunks 10.9 -> 10.2, of 128 rows and 8 chunks
+// 14.9 -> 13.6, no workgroups of twice the waves.
+struct ListsShared {
+    bool whole;
+    size_t ws_bytes = 0;
+};
+ListsShared lists_shared(const Hints &h, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t Dk, int64_t BQ, int64_t BK, int dt) {
+    if (h.stats && h.longest_list * BK <= sa_fwd_split_least_keys(B, H, Sq, Sk, Dk, BQ, BK, dt)) return {true};
+    return {false, sa_fwd_split_workspace_bytes(B, H, Sq, Sk, Dk, BQ, BK, dt)};
+}
+// The same by name, for reports on what a call without a schedule runs: "whole", "halves" or "shared".
+std::string forward_lists(const Tensor &q, int64_t Sk, int64_t BQ, int64_t BK, py::object md) {
+    const c10::DeviceGuard guard(q.device());
+    const int64_t B = q.size(0), H = q.size(1), Sq = q.size(2), Dk = kernel_head_dim(q.size(3), true);
+    const int dt = dtype_code(q.scalar_type());
+    const ListsShared s = lists_shared(hints_of(md), B, H, Sq, Sk, Dk, BQ, BK, dt);
+    if (s.whole || (s.ws_bytes == 0 && sa_fwd_split_least_keys(B, H, Sq, Sk, Dk, BQ, BK, dt) == Sk)) return "whole";
+    return s.ws_bytes ? "shared" : "halves";
+}
+
 // Whether tensors of these sizes run on a larger tile grid as they are (sa_sparse_attention_fwd_ragged): nothing is padded.
 bool ragged_has(const Tensor &q, int64_t BQ, int64_t BK, const Lists &l) {
     const int dt = dtype_code(q.scalar_type());
@@ -507,16 +529,18 @@ std::optional<Out> forward_impl(const Tensor &q, const Tensor &k, const Tensor &
                                              st(mask), ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl), ptr<int32_t>(l.pid), st(l.pid),
                                              ptr<int32_t>(l.pl), st(l.pl), ptr<uint8_t>(l.packed), st(l.packed), ptr<int32_t>(*sched),
                                              sched->numel() * 4, hints.sched_mode, ptr<float>(lse), st(lse), B, H, Sq, Sk, Dk, BQ, BK, dt, scale, stream));
-    } else if (code != SA_FWD_KERNEL_DEFAULT) {
+        return Out{cut_head_dim(o, D), lse};
+    }
+    ListsShared shared{true};
+    if (code == SA_FWD_KERNEL_DEFAULT) shared = lists_shared(hints, B, H, Sq, Sk, Dk, BQ, BK, dt);
+    if (shared.whole) {
         check_rc(sa_sparse_attention_fwd_kernel(qc.data_ptr(), st(qc), kc.data_ptr(), st(kc), vc.data_ptr(), st(vc), o.data_ptr(), st(o),
                                                 ptr<uint8_t>(mask), st(mask), ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl),
                                                 ptr<int32_t>(l.pid), st(l.pid), ptr<int32_t>(l.pl), st(l.pl), ptr<uint8_t>(l.packed), st(l.packed),
                                                 ptr<float>(lse), st(lse), B, H, Sq, Sk, Dk, BQ, BK, dt, scale, code, stream));
     } else {
-        // (too few Q tiles to fill the device: their lists are shared by several workgroups, which need a workspace)
-        size_t ws_bytes = sa_fwd_split_workspace_bytes(B, H, Sq, Sk, Dk, BQ, BK, dt);
-        // (metadata that says that no list is long enough: 128 tiles of 16 chunks 22.9 -> 20.0 us, no merge that finds nothing)
-        if (ws_bytes && hints.stats && hints.longest_list * BK <= sa_fwd_split_least_keys(B, H, Sq, Sk, Dk, BQ, BK, dt)) ws_bytes = 0;
+        // (too few Q tiles to fill the device: lists are shared by several workgroups, which need a workspace, or walked in halves)
+        const size_t ws_bytes = shared.ws_bytes;
         Tensor ws;
         if (ws_bytes) ws = at::empty({(int64_t)(ws_bytes / 4)}, opt_f32);
         check_rc(sa_sparse_attention_fwd_split(qc.data_ptr(), st(qc), kc.data_ptr(), st(kc), vc.data_ptr(), st(vc), o.data_ptr(), st(o),
@@ -826,6 +850,7 @@ PYBIND11_MODULE(_host, m) {
     py::class_<OneMask, std::shared_ptr<OneMask>>(m, "OneMask");
     m.def("of_one_mask", &of_one_mask);
     m.def("forward", &forward);
+    m.def("forward_lists", &forward_lists);
     m.def("forward_kernel", &forward_kernel);
     m.def("forward_tiled", &forward_tiled);
     m.def("decode", &decode);

@@ -178,6 +178,8 @@ struct FwdSplitPlan {
 FwdSplitPlan fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus);
 // Whether a launch walks its lists in two halves (sparse_fwd_kernel<..., TW>) where they are not shared: sparse_fwd_merge.hip.
 bool fwd_in_halves(int64_t tiles, int Sk, int BQ, int BK, int D, int dtype, int cus);
+// There: chunks up to which the form without halves is no slower, if every list is known to be as short.
+int fwd_halves_least(int BQ, int D);
 // Adds up the parts of shared lists (dtype 2: float32 output).
 hipError_t launch_fwd_merge(const FwdParams &p, int dtype, int D, int BQ, hipStream_t stream);
 

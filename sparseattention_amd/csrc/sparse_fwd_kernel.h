@@ -103,7 +103,8 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
     // [K stage 0..NS-1][V stage 0..NS-1][first key column of every list entry, kListCap ints]; TW: a set per half
     constexpr int HALF_BYTES = NS * KBUF + NS * VBUF + kListCap * 4 + (TW ? kHalvesSync : 0);
     const int half = TW ? __builtin_amdgcn_readfirstlane(threadIdx.x / (NW * 64)) : 0;  // which half this wave belongs to
-    // (TW) lists of up to this many chunks are walked by the first half alone: of 13 on (BLOCK_Q 128) or 5 (64) two are faster
+    // (TW) Lists of up to this many chunks are walked by the first half alone.  us at this many for all, 10 | 12 (BLOCK_Q 128): 11 chunks
+    // 18.2 | 18.3, 12 chunks 19.0 | 19.3, D = 64 12.5 | 12.6, 12.9 | 13.1; 4 | 6 (BLOCK_Q 64): 5 chunks 11.5 | 12.1, 6 chunks 11.6 | 13.2.
     constexpr int LEAST = NW == 4 ? 10 : 4;
     uint8_t *const smem = smem0 + half * HALF_BYTES;
     int *const ent = reinterpret_cast<int *>(smem + NS * KBUF + NS * VBUF);

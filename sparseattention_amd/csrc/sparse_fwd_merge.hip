@@ -135,8 +135,8 @@ FwdSplitPlan fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus
 //       256 tiles  causal  64        62.0 | 54.9   80 69.3 | 67.4   96 79.0 | 78.9   192 146.6 | 149.5  all  96 99.9 | 94.2   192 178.9 | 178.9
 //       D = 64     causal  224 tiles 72 chunks 41.5 | 41.8   88 45.9 | 49.0    256 tiles  72 41.9 | 42.1   96 52.9 | 53.3
 //       256 tiles  window 64  12.5 | 10.5   256  15.1 | 13.1   900, BLOCK_K 32  26.6 | 22.9
-//   (with shorter rows the launch had no merge to save, and lists of up to 12 chunks would pay 1.1 us for the wider workgroup: 9.2 |
-//   10.6, 11.8 | 13.2; longer ones gain little: causal Sk 1024 21.4 | 20.2, every key of 2048 39.2 | 36.7)
+//   (with shorter rows the launch had no merge to save, and lists of up to 16 chunks would pay up to 1.4 us for the wider workgroup,
+//   fwd_halves_least; longer ones gain little: causal Sk 1024 21.4 | 20.2, every key of 2048 39.2 | 36.7)
 //   BLOCK_Q 64, one workgroup per list (Sk up to 48 chunks) or shared by two with a merge | halves
 //       256 tiles  causal  16 chunks 24.5 | 17.8   64, D = 64 51.1 | 34.8   256 203.0 | 197.4   all 128 104.6 | 96.6
 //                  window 256  12.2 | 12.0   window 64 (lists of two chunks)  9.1 | 9.5
@@ -153,6 +153,14 @@ bool fwd_in_halves(int64_t tiles, int Sk, int BQ, int BK, int D, int dtype, int 
     if (Sk <= 96 * 64) return true;
     return 3 * tiles > 2 * cus && (D == 64 || 4 * tiles <= 3 * cus || tiles == cus);
 }
+
+// A caller who knows that all lists are short does without the wider workgroup: us, one workgroup of half the waves | halves, 256 tiles,
+// every list as long as stated (kept whole by the first half up to 10 chunks, at BLOCK_Q 64 up to 4: sparse_fwd_kernel's LEAST)
+//   BLOCK_Q 128          4 chunks  9.7 | 10.8    8 13.6 | 14.9   12 18.0 | 19.0   14 20.5 | 21.1   16 22.4 | 22.6   20 26.6 | 26.2
+//                D = 64  4 chunks  7.5 |  8.2    8 10.4 | 10.7   13 13.2 | 13.5   14 13.9 | 13.8   16 15.3 | 15.0   20 18.1 | 17.2
+//   BLOCK_Q 64           2 chunks  7.8 |  8.4    4 10.2 | 10.9    5 11.4 | 11.5    6 12.5 | 11.6    8 15.0 | 12.9
+//                D = 64  2 chunks  6.0 |  6.6    4  7.8 |  8.4    5  8.7 |  9.1    6  9.4 |  9.0    8 11.1 | 10.0
+int fwd_halves_least(int BQ, int D) { return BQ == 64 ? 5 : (D == 64 ? 13 : 16); }
 
 hipError_t launch_fwd_merge(const FwdParams &p, int dtype, int D, int BQ, hipStream_t stream) {
     const int NW = BQ / 32, lck = dtype == 2 ? 5 : 6;

@@ -569,7 +569,9 @@ size_t sa_fwd_split_workspace_bytes(int B, int H, int Sq, int Sk, int D, int BQ,
 
 int sa_fwd_split_least_keys(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype) {
     sa::FwdSplitPlan plan;
-    if ((D != 64 && D != 128) || dtype < SA_DTYPE_BF16 || dtype > SA_DTYPE_FP32 || split_shape(B, H, Sq, Sk, D, BQ, BK, dtype, &plan) == 0) return Sk;
+    if ((D != 64 && D != 128) || dtype < SA_DTYPE_BF16 || dtype > SA_DTYPE_FP32) return Sk;
+    if (in_halves(B, H, Sq, Sk, D, BQ, BK, dtype)) return sa::fwd_halves_least(BQ, D) << 6;
+    if (split_shape(B, H, Sq, Sk, D, BQ, BK, dtype, &plan) == 0) return Sk;
     return plan.least << (dtype == SA_DTYPE_FP32 ? 5 : 6);  // (a plan's lists may be longer than this: less than Sk)
 }
 
