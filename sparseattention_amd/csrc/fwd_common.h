@@ -264,12 +264,6 @@ struct HandOver {
     __device__ __forceinline__ void put(uint32_t at, f32x2 x) const {
         __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), rsrc, (int)at, 0, kDeviceScope);
     }
-    __device__ __forceinline__ f32x4 get4(uint32_t at) const {
-        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)at, 0, kDeviceScope));
-    }
-    __device__ __forceinline__ f32x2 get2(uint32_t at) const {
-        return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)at, 0, kDeviceScope));
-    }
 };
 // One thread of each of n <= kArrivalMost workgroups, after what the workgroup hands over has been stored (every wave: vmcnt(0),
 // then a barrier): true for the last one.  The word needs no first value: its upper 56 bits are the launch's number

@@ -28,8 +28,12 @@ constexpr int kDecodeWaves = 4;
 //   D = 128  B1 H32 Sk8192 Sq1 36.5 | 33.1  Sq8 38.3 | 34.4   B4 H16 Sk8192 Sq1 50.6 | 48.0   B4 H16 Sk32768 Sq1 165.8 | 163.1
 //            B8 H32 Sk32768 Sq1 647 | 624 (6.9 TB/s; a linear streaming read runs at 7.1)   B8 H16 Sk16384 Sq16 gathered 90.3 | 83.6
 //   D = 64   B1 H32 Sk2048 Sq8 13.5 | 11.9   B4 H16 Sk32768 Sq1 90.3 | 85.9   Sq32 97.3 | 93.3
-// and nowhere slower but at BLOCK_K = 16 (B8 H32 Sk4096 Sq1 87.7 | 90.2), whose rows come from two places.  (Called again and again
-// on the same K and V, no more than the memory-side cache and L2 hold, K per lane is up to 6 % faster: B8 H32 Sk4096 78.8 | 82.9.)
+// and nowhere slower but at BLOCK_K = 16 (B8 H32 Sk4096 Sq1 87.7 | 90.2), whose rows come from two places.
+// Called again and again on the same K and V, which nothing else has pushed out, K per lane is faster up to 512 MiB of them (D = 128, Sq1,
+// per lane | rows; behind it the same call on K and V from a rotation of 1.5 GiB): B1 H32 Sk2048 14.1 | 14.6 (16.0 | 15.9),
+// B4 H16 Sk8192 45.8 | 47.9 (51.8 | 50.2), B8 H32 Sk2048 45.8 | 48.0 (51.0 | 49.4), Sk4096 83.1 | 90.2 (93.8 | 91.4), Sk8192 174 |
+// 170 (176.6 | 173): loads with the streaming hint find less of what the last call left.  A program's layers have K and V of
+// their own, so the rule goes by the rotation.
 constexpr bool decode_key_rows(bool b16, bool dm) { return !b16 && !dm; }
 
 template <int D, bool KR>
@@ -38,6 +42,7 @@ constexpr int decode_smem_bytes() {
     constexpr int stream = kDecodeWaves * (2 * 32 + (KR ? 16 : 0)) * D * 2;
     constexpr int merge = kDecodeWaves * 32 * (D + 2) * 4 + 16;   // per wave 32 rows of D + 2 floats; the parts of a plane
     static_assert(kDecodeMergeRows <= kDecodeWaves * 32, "LDS holds the parts that the last workgroup merges");
+    static_assert(kDecodeMergeFew <= kArrivalMost, "a plane's workgroups have place in its count");
     return stream > merge ? stream : merge;
 }
 
