@@ -21,11 +21,14 @@ def exact(q, k, v, mask):
     (torch.float16, 1, 13, 640, 1088, 64, 64, 32),      # 130 Q tiles
     (torch.float16, 2, 33, 256, 3104, 128, 128, 32),    # a last chunk that is not full
     (torch.bfloat16, 1, 3, 4096, 2048, 64, 64, 1024),   # fewer entries than chunks
+    (torch.bfloat16, 2, 3, 1920, 1216, 128, 64, 64),    # 180 Q tiles of 64 rows at D = 128, 19 chunks
+    (torch.float16, 1, 17, 1024, 3168, 64, 128, 32),    # 136 Q tiles of 128 rows at D = 64
 ])
 @pytest.mark.parametrize("packed", [True, False])
 def test_halves_against_float64(gpu, dtype, B, H, Sq, Sk, D, BQ, BK, packed):
     assert _native.load().sa_fwd_split_workspace_bytes(B, H, Sq, Sk, D, BQ, BK, {torch.bfloat16: 0, torch.float16: 1}[dtype]) == 0
     q, _, _ = W.qkv(B, H, Sq, D, dtype, seed=1, device=gpu)
+    assert _native.host().forward_lists(q, Sk, BQ, BK, None) == "halves"
     _, k, v = W.qkv(B, H, Sk, D, dtype, seed=2, device=gpu)
     g = torch.Generator(device=gpu).manual_seed(BK)
     nq, nk = Sq // BQ, Sk // BK
@@ -68,6 +71,31 @@ def test_long_uneven_lists_are_shared(gpu, tiles, chunks, D, BQ):
         pytest.skip("the numbers are those of 256 compute units")
     lib = _native.load()
     assert lib.sa_fwd_split_workspace_bytes(1, tiles * cus // 256, BQ, 64 * chunks, D, BQ, 64, 0) > 0
+
+
+@pytest.mark.parametrize("D,BQ", [(128, 128), (64, 128), (128, 64), (64, 64)])
+def test_infinite_values_that_lists_name(gpu, D, BQ):
+    """An infinity or a NaN in V reaches its column of the result whichever half holds it, and no other column."""
+    B, H, Sk, BK = 1, 32, 3200, 64
+    Sq = 8 * BQ
+    q, _, _ = W.qkv(B, H, Sq, D, torch.bfloat16, seed=5, device=gpu)
+    _, k, v = W.qkv(B, H, Sk, D, torch.bfloat16, seed=6, device=gpu)
+    mask = torch.ones(B, 1, Sq, Sk, dtype=torch.bool, device=gpu)
+    mask[..., : BQ + 5, 2 * Sk // 3:] = False  # (rows that attend to none of the second infinity)
+    me = mask.expand(B, H, Sq, Sk)
+    want, _ = exact(q[0], k[0], v[0], mask[0])
+    v[..., 70, 3], v[..., -70, 9] = float("inf"), float("-inf")  # (the first half's, the second half's)
+    v[..., 300, 17], v[..., -300, 31] = float("nan"), float("nan")
+    assert _native.host().forward_lists(q, Sk, BQ, BK, None) == "halves"
+    o = sparse_attention(q, k, v, me, BQ, BK, mask_metadata=compute_mask_kernel(me, BQ, BK))[0].double()
+    # (where a tile is listed, the keys of it that a row does not attend to have a weight of 0: 0 times these is NaN)
+    far = slice(2 * BQ, Sq)
+    assert torch.isposinf(o[..., 3]).all() and torch.isneginf(o[:, far, 9]).all()
+    assert torch.isnan(o[..., 17]).all() and torch.isnan(o[:, far, 31]).all()
+    near = slice(0, BQ)  # (their lists end before the second ones)
+    assert torch.isfinite(o[:, near, 9]).all() and torch.isfinite(o[:, near, 31]).all()
+    rest = [d for d in range(D) if d not in (3, 9, 17, 31)]
+    assert ((o[..., rest] - want[..., rest]).norm() / want[..., rest].norm()) <= 2.0 ** -7
 
 
 def test_halves_with_infinite_values_and_entries_out_of_range(gpu):
