@@ -380,7 +380,7 @@ def decode_case(steps, warmup):
                          "unit": "GB/s", "frac": round(nbytes / (ev_ms * 1e-3) / 1e9 / PEAK_HBM_GBS, 4),
                          **traffic_of("decode, %d" % Sq, "decode"),
                          "algorithmic_bytes": nbytes,
-                         "kernel": "sparse_decode_kernel (+ decode_merge_kernel)"},
+                         "kernel": "sparse_decode_kernel"},
         })
     return rows
 
