@@ -220,12 +220,12 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
     }
     __syncthreads();
 
-    // where this wave's keys' dS of the 64 queries from ent[t] goes: two pieces of 2 KiB, 4 KiB apart
+    // where this wave's keys' dS of the 64 queries from ent[t] goes: 4 KiB in a row
     const int64_t ds_row = (int64_t)p.nR * 2 * 16384;  // all keys of 128 queries
-    uint8_t *const ds0 = DS ? p.ds + (int64_t)plane * (p.nS >> 1) * ds_row + (2 * rt + (wave_u >> 1)) * 16384 + (wave_u & 1) * 2048 : nullptr;
+    uint8_t *const ds0 = DS ? p.ds + (int64_t)plane * (p.nS >> 1) * ds_row + (2 * rt + (wave_u >> 1)) * 16384 + (wave_u & 1) * 8192 : nullptr;
     auto ds_out = [&](int t) {
         const int row = __builtin_amdgcn_readfirstlane(ent[t]);
-        return ds0 + (row >> 7) * ds_row + ((row & 64) << 7);
+        return ds0 + (row >> 7) * ds_row + ((row & 64) << 6);
     };
 
     // everything chunk t needs from memory, into stage st
@@ -359,9 +359,10 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
             }
             if constexpr (DS) {  // (the order of the pieces: bwd_dq_tile)
 #pragma unroll
-                for (int c = 0; c < 2; c++)
-                    *(u32x4 *)(ds_out(t) + 4096 * kb + 1024 * c + (uint32_t)((32 * (ln & 31) + 16 * (ln >> 5)) ^ (128 * c))) =
-                        u32x4{pw[4 * c], pw[4 * c + 1], pw[4 * c + 2], pw[4 * c + 3]};
+                for (int c = 0; c < 2; c++) {
+                    uint8_t *const to = ds_out(t) + 2048 * kb + 1024 * c + (uint32_t)((32 * (ln & 31) + 16 * (ln >> 5)) ^ (128 * c));
+                    __builtin_nontemporal_store(u32x4{pw[4 * c], pw[4 * c + 1], pw[4 * c + 2], pw[4 * c + 3]}, (u32x4 *)to);
+                }
             }
             phase();
             const uint32_t tb = (OUT_P ? zb : yb) + 32 * kb * ROWB;
@@ -446,10 +447,16 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
 }
 
 // dQ from the dS that the pass over the keys stored: dQ^T += K^T . dS^T, one product instead of three, bound by the reads
-// of dS (B8 H16 S4096 causal: 2.15 GB in 505 us, 4.3 TB/s; 312 us with the same dS from L2, so neither the products nor the
-// loads into LDS bound it; two stages and four workgroups per compute unit: 535 us).  128 queries per workgroup, 32 per wave; a chunk of 64 keys is 16 KiB of K, shared, and 4 KiB of dS per wave.
-// dS lies as [plane][128 queries][64 keys][32 queries][32 keys]: what a workgroup here reads is contiguous.  In the 2 KiB of
-// the last two,
+// of dS (B8 H16 S4096 causal: 2.2 GB in 487 us, 4.5 TB/s, and 312 us with the same dS from L2, so neither the products nor the
+// loads into LDS bound it; every key: 4.3 GB in 741 us, 5.8 TB/s).  128 queries per workgroup, 32 per wave; a chunk of 64 keys is
+// 16 KiB of K, shared, and 4 KiB of dS per wave.  More of dS on its way does not help (causal: a fifth wave for K, which leaves
+// LDS for 80 instead of 48 KiB of dS per compute unit, +9 us; dS through registers, 96 ... 160 KiB, +30 ... +100 us; the next
+// step's requests behind this one's LDS reads +5 us; two stages and four workgroups per compute unit +30 us).
+// dS lies as [plane][128 queries][64 keys][halves of 32 keys][32 queries][32 keys]: what a workgroup here reads in a step is 8 KiB
+// in a row, and what a wave of the key pass stores of a chunk 4 KiB (pieces of 2 KiB 4 KiB apart before: causal 498 -> 493 us).  It is
+// stored past L2, where Q and dO are read again and again (key pass 1156 -> 1141 us, reads from beyond L2 1.4 -> 0.76 GB;
+// this pass 493 -> 487), and the planes are walked from the last one the key pass wrote, whose dS the memory-side cache still
+// holds (520 -> 498).  All three together: every key 941 -> 741 us.  In the 2 KiB of the last two,
 // key k's queries 8g + 4h .. + 3 are the 8 bytes at 1024 (g / 2) + ((32 k + 16 h) ^ 128 (g / 2)) + 8 (g & 1): the key
 // pass stores 1 KiB per instruction, and a transposing read (four keys, two groups of 16 queries) meets no bank twice.
 // A block that the key pass did not visit holds whatever the memory held: none of its entries attends, so it lies in
@@ -469,13 +476,13 @@ __device__ __forceinline__ void bwd_dq_tile(const BwdParams &p, int lin, int tot
     const int tid = threadIdx.x, lane = tid & 63, wave_u = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, hh = lane >> 5;
     const BwdPlace at = bwd_place(p, lin, total);
-    const int plane = at.plane, rt = at.rt, bh = p.plane0 + plane;
+    const int plane = p.planes - 1 - at.plane /* (last written first) */, rt = at.rt, bh = p.plane0 + plane;
     const int b = bh / p.H, h = bh - b * p.H;
     const uint16_t *ybase = p.y + b * p.ys[0] + h * p.ys[1];
     const int32_t *fid = p.full_ids + b * p.fis[0] + h * p.fis[1] + rt * p.fis[2];
     const int32_t *pid = p.part_ids + b * p.pis[0] + h * p.pis[1] + rt * p.pis[2];
     const uint8_t *prow = p.packed + b * p.pks[0] + h * p.pks[1] + (int64_t)rt * p.nS * 1024 + wave_u * 256;
-    const uint8_t *dsbase = p.ds + ((int64_t)plane * p.nR + rt) * p.nS * 16384 + wave_u * 4096;
+    const uint8_t *dsbase = p.ds + ((int64_t)plane * p.nR + rt) * p.nS * 16384 + wave_u * 2048;
     int cnt[2];  // (clamped as in bwd_tile)
     const int32_t *const cnt_addr[2] = {p.full_lens + (b * p.fls[0] + h * p.fls[1] + rt * p.fls[2]),
                                         p.part_lens + (b * p.pls[0] + h * p.pls[1] + rt * p.pls[2])};
@@ -502,7 +509,7 @@ __device__ __forceinline__ void bwd_dq_tile(const BwdParams &p, int lin, int tot
     const int64_t ytile = 64 * p.ys[2], yhalf = 32 * p.ys[2], yload = 4 * RPI * p.ys[2];
     auto issue = [&](int u, int st) {
         const int t = u >> 1, kt = __builtin_amdgcn_readfirstlane(ent[t]);
-        const uint8_t *dsp = dsbase + (int64_t)kt * 16384 + (u & 1) * 2048;
+        const uint8_t *dsp = dsbase + (int64_t)kt * 16384 + (u & 1) * 8192;
         if (t >= F && (u & 1) == 0) dma4(prow + (int64_t)(t - F) * 1024, 4 * lane, lds0 + MASK0 + (t & 3) * 1024 + wave_u * 256);
 #pragma unroll
         for (int i = 0; i < 2; i++) dma16<true>(dsp + 1024 * i, 16 * lane, lds0 + DS0 + st * 8192 + wave_u * 2048 + 1024 * i);
