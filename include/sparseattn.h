@@ -382,7 +382,7 @@ int sa_sparse_attention_fwd_kernel(const void *q, const int64_t q_strides[4], co
 
 /*
  * The same forward for launches with too few Q tiles to fill the device (a chunk of a prompt against a long cache): the
- * list of a Q tile is shared by several workgroups and their partial results are added up by a second launch.
+ * list of a Q tile is shared by several workgroups and their partial results are added up by the last of them or by a second launch.
  *   workspace   sa_fwd_split_workspace_bytes(...) bytes of device memory, 16-byte aligned; may be NULL when that is 0,
  *               which says that the launch has no use for it (the call is then sa_sparse_attention_fwd_kernel with the
  *               default kernel, or a kernel that walks a list in two halves by the waves of one workgroup).  The bytes depend

@@ -264,6 +264,12 @@ struct HandOver {
     __device__ __forceinline__ void put(uint32_t at, f32x2 x) const {
         __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x), rsrc, (int)at, 0, kDeviceScope);
     }
+    __device__ __forceinline__ f32x4 get4(uint32_t at) const {
+        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)at, 0, kDeviceScope));
+    }
+    __device__ __forceinline__ f32x2 get2(uint32_t at) const {
+        return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rsrc, (int)at, 0, kDeviceScope));
+    }
 };
 // One thread of each of n <= kArrivalMost workgroups, after what the workgroup hands over has been stored (every wave: vmcnt(0),
 // then a barrier): true for the last one.  The word needs no first value: its upper 56 bits are the launch's number
@@ -289,6 +295,75 @@ __device__ __forceinline__ bool arrives_last(uint64_t *word, uint64_t tag, int n
     if ((int)(old & 0xff) + 1 != n) return false;
     __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return true;
+}
+
+// The same without a common word, whose atomics go through one place one after the other (0.5 us each: seven workgroups 3.4 us, this
+// way 1.2): each of n <= 64 workgroups has a word of its own.  One wave of each, after what its workgroup hands over has been stored: it
+// sets its word to the launch's number, waits until that is in memory and looks at all n.  Whoever's word gets there last sees all set, so at
+// least one workgroup is told true; more than one may be, and then each does the same work and leaves the same bits.  Who
+// is told true clears the words (all have been set then), so that a replay of a captured launch, which brings the same number, finds none.
+__device__ __forceinline__ bool all_arrived(uint64_t *words, uint64_t tag, int mine, int n) {
+    const int lane = threadIdx.x & 63;
+    const HandOver h(words, 8u * (uint32_t)n);
+    const u32x2 set = {(uint32_t)tag, (uint32_t)(tag >> 32)};
+    if (lane == 0) h.put(8u * (uint32_t)mine, __builtin_bit_cast(f32x2, set));
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const u32x2 seen = __builtin_bit_cast(u32x2, h.get2(8u * (uint32_t)min(lane, n - 1)));
+    const bool all = __builtin_amdgcn_ballot_w64(seen.x == set.x && seen.y == set.y) == ~0ull;
+    if (all && lane < n) h.put(8u * (uint32_t)lane, f32x2{0.f, 0.f});
+    return all;
+}
+
+// The sum of n parts that workgroups have handed over: this wave's N blocks of 32 x 32 values, 16 a lane, the lane's four of run g of a
+// block at rows_at + part * rows_step + 1024 (4 block + g) (where a wave leaves its accumulators, 1 KiB a store), with reference value
+// (-inf: no attended key) and sum of the lane's row at state_at + part * state_step.  In the order of the parts, whoever adds.  The
+// first B parts are under way while the largest reference value is looked for: one round trip for up to B parts.
+template <int N, int B>
+__device__ __forceinline__ void add_parts(const HandOver &rows, uint32_t rows_at, uint32_t rows_step, const HandOver &state, uint32_t state_at,
+                                          uint32_t state_step, int n, f32x16 (&acc)[N], float &M, float &L) {
+    f32x4 x[B][4 * N];
+    f32x2 st[B];
+    auto request = [&](int i0) {
+#pragma unroll
+        for (int i = 0; i < B; i++) {
+            const uint32_t part = (uint32_t)min(i0 + i, n - 1);  // (past the last one: that one again, left out below)
+            st[i] = state.get2(state_at + part * state_step);
+#pragma unroll
+            for (int g = 0; g < 4 * N; g++) x[i][g] = rows.get4(rows_at + part * rows_step + 1024u * g);
+        }
+    };
+    request(0);
+    float m = kNegInf;
+    for (int i0 = 0; i0 < n; i0 += 4) {
+        f32x2 s4[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) s4[i] = state.get2(state_at + (uint32_t)min(i0 + i, n - 1) * state_step);
+#pragma unroll
+        for (int i = 0; i < 4; i++) m = fmaxf(m, s4[i].x);
+    }
+    M = m;
+    L = 0.f;
+    const float M0 = m == kNegInf ? 0.f : m;  // (no part saw an attended key: every weight is 0)
+#pragma unroll
+    for (int d = 0; d < N; d++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) acc[d][e] = 0.f;
+#pragma unroll 1
+    for (int i0 = 0;;) {
+#pragma unroll
+        for (int i = 0; i < B; i++) {
+            if (i0 + i >= n) break;
+            const float w = __builtin_amdgcn_exp2f(st[i].x - M0);
+            L = __builtin_fmaf(w, st[i].y, L);
+#pragma unroll
+            for (int g = 0; g < 4 * N; g++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[g / 4][4 * (g % 4) + e] = __builtin_fmaf(w, x[i][g][e], acc[g / 4][4 * (g % 4) + e]);
+        }
+        i0 += B;
+        if (i0 >= n) break;
+        request(i0);
+    }
 }
 
 // log2-domain slack before the running maximum is raised (and the accumulator rescaled).  Scores are

@@ -148,6 +148,10 @@ struct FwdParams {
     int nsplit, split_chunks;  // split_chunks: chunks of one part (the last ones may be shorter)
     int split_least;           // lists of up to this many chunks are not shared
     float *ws, *ws_ml;
+    // [B*H*nQ][nsplit] words by which the last workgroup of a shared list to arrive knows that it is the one to add the parts up
+    // (all_arrived), or null: then a second launch does (launch_fwd_merge).  tag: the launch's number.
+    uint64_t *arrivals;
+    uint64_t tag;
     int halves;                // 1: every list in two halves by the waves of one workgroup (fwd_in_halves)
     // Ragged sizes: the tile grid (Sq, Sk, nQ, nK, lists, packed tiles) is that of a padded mask, the tensors have Sq_in
     // and Sk_in rows, which stand q0 and k0 rows into the grid, of D_in elements (a multiple of 8, at most the kernel's D).
@@ -171,6 +175,8 @@ __host__ __device__ inline int fwd_split_first(int NE, int lbk, int lck, int s, 
     const int e = (int)(groups * (unsigned)s / (unsigned)share) << le;
     return e < NE ? e : NE;
 }
+// Whether the last workgroup of a shared list to arrive adds up its parts (all_arrived), else a second launch does: sparse_fwd_merge.hip.
+bool fwd_merges_in_launch(int nsplit, int BQ, int D, int dtype);
 // The rule for nsplit, split_chunks and split_least: sparse_fwd_merge.hip.
 struct FwdSplitPlan {
     int nsplit = 1, chunks = 1 << 30, least = 0;

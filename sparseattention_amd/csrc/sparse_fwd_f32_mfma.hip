@@ -30,26 +30,42 @@ namespace sa {
 namespace {
 
 constexpr int kF32ListCap = 1024;  // list entries kept in LDS (the launcher refuses longer rows of tiles)
+constexpr int f32_groups(int NW, bool SP) { return SP && NW <= 2 ? 2 : 1; }
+// LDS of a group of NW waves: [K, two stages][V, two stages][mask words, two stages][list]
+template <int D, int NW>
+constexpr int f32_group_bytes = 4 * 32 * D * 4 + 2 * NW * 1024 + kF32ListCap * 4;
 
 // MODE 0: BK = 16 (two list entries per chunk), MODE 1: BK = 32, MODE 2: BK >= 64 (BK/32 chunks per entry).
 // PK: mask entries of PARTIAL tiles from the bit-packed tiles; else from the bool mask (key stride 1, rows and base
 // 16-byte aligned: checked by the launcher).
-template <int D, int NW, int MODE, bool PK>
-__global__ __launch_bounds__(NW * 64, NW >= 4 ? 2 : 1) void sparse_fwd_f32_mfma_kernel(const FwdParams p) {
+// SP: lists shared by up to p.nsplit workgroups (fwd_split_share).
+// KG: groups of NW waves that share out a list, each with stages of its own, in step; their rows meet in LDS.  Two where lists are
+// shared and NW <= 2 would leave two of the four SIMDs idle.
+// A small launch is a chain: B1 H4 S512 D64 with half of the 32 x 32 blocks (32 Q tiles, about 9 chunks each, parts of two) takes 10.9 us a
+// pass, where two waves per part, reads of the list behind the counts and a second launch for the merge took 16.0.  Time stamps: queries,
+// counts and lists 1.2 us, first K and V at 2.3, products and softmax 3.0, the groups' rows 0.4, parts handed over 0.7, all arrived 0.8,
+// parts read and added 2.1.
+// Registers for two waves per SIMD (D = 64: results stay out of the accumulation registers; causal B2 H16 S2048 235 -> 226 us), but not at
+// D = 128 with two waves a workgroup: registers that fill a SIMD keep the waves of two workgroups on different ones (339 us against 592).
+template <int D, int NW, int MODE, bool PK, bool SP>
+__global__ __launch_bounds__(NW * f32_groups(NW, SP) * 64, D == 128 && NW * f32_groups(NW, SP) <= 2 ? 1 : 2) void sparse_fwd_f32_mfma_kernel(const FwdParams p) {
+    constexpr int KG = f32_groups(NW, SP);
     constexpr int ROWB = D * 4, PPR = ROWB / 16;  // bytes and 16-byte pieces per K/V row
     constexpr int KBUF = 32 * ROWB;               // one stage of K (or V): 32 rows
     constexpr int MBUF = NW * 1024;               // one stage of mask words: 64 lanes x 16 bytes per wave
-    constexpr int OFF_V = 2 * KBUF, OFF_M = 4 * KBUF, OFF_L = OFF_M + 2 * MBUF;
+    constexpr int OFF_V = 2 * KBUF, OFF_M = 4 * KBUF, OFF_L = OFF_M + 2 * MBUF, GROUP = f32_group_bytes<D, NW>;
     constexpr int EPC = MODE == 0 ? 2 : 1;
     constexpr int LBKC = MODE == 0 ? 4 : 5;
     constexpr int RPI = 1024 / ROWB;   // rows per direct load
     constexpr int NLD = 32 / RPI / NW; // direct loads per wave and chunk, each for K and for V
     static_assert(32 % (RPI * NW) == 0, "staging layout");
 
-    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem0[];
+    const int grp = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / (NW * 64));
+    uint8_t *const smem = smem0 + grp * GROUP;
     int *const ring = reinterpret_cast<int *>(smem + OFF_L);
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = KG == 1 ? threadIdx.x : threadIdx.x % (NW * 64), lane = tid & 63, wave = tid >> 6;
     const int l32 = lane & 31, hh = lane >> 5;
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     // Workgroup -> (b, h, Q tile) as in sparse_fwd_kernel: the hardware hands consecutive workgroup ids to the 8 XCDs
@@ -60,7 +76,7 @@ __global__ __launch_bounds__(NW * 64, NW >= 4 ? 2 : 1) void sparse_fwd_f32_mfma_
     {
         const int total = p.nQ * p.B * p.H, per = total >> 3;
         int lin = blockIdx.x;
-        if (p.nsplit > 1) {  // the first parts of all tiles, then the second ones, ...
+        if constexpr (SP) {  // the first parts of all tiles, then the second ones, ...
             s0 = lin / total;
             lin -= s0 * total;
         }
@@ -84,33 +100,53 @@ __global__ __launch_bounds__(NW * 64, NW >= 4 ? 2 : 1) void sparse_fwd_f32_mfma_
     const float *const vbase = reinterpret_cast<const float *>(p.v) + b * p.vs[0] + h * p.vs[1];
     const int32_t *fid = p.full_ids + b * p.fis[0] + h * p.fis[1] + qt * p.fis[2];
     const int32_t *pid = p.part_ids + b * p.pis[0] + h * p.pis[1] + qt * p.pis[2];
-    int F = min(min(max(p.full_lens[b * p.fls[0] + h * p.fls[1] + qt * p.fls[2]], 0), p.nK), kF32ListCap);
-    int NE = F + min(min(max(p.part_lens[b * p.pls[0] + h * p.pls[1] + qt * p.pls[2]], 0), p.nK - F), kF32ListCap - F);
-    int share = 1, p_lo = 0;
-    if (p.nsplit > 1) {
-        share = fwd_split_share(NE, p.lbk, 5, p.split_least, p.split_chunks, p.nsplit);
-        if (s0 >= share) return;
-        const int e_lo = fwd_split_first(NE, p.lbk, 5, s0, share), e_hi = fwd_split_first(NE, p.lbk, 5, s0 + 1, share);
-        fid += (int64_t)min(e_lo, F) * p.fis[3];
-        p_lo = max(e_lo - F, 0);
-        pid += (int64_t)p_lo * p.pis[3];
-        F = min(max(F - e_lo, 0), e_hi - e_lo);
-        NE = e_hi - e_lo;
-    }
-    const int T = MODE == 2 ? (NE << (p.lbk - 5)) : ((NE + EPC - 1) / EPC);
-    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const SA_LDS uint8_t *)smem);
-
-    // Q^T operand: d = (D/2) hh + c for step c, scaled once (softmax scale / ln 2)
-    float qf[D / 2];
+    // The memory round trips of the start side by side: queries, counts, and (SP, rows of at most 64 tiles) both lists whole, a slot
+    // per lane.  Slots past a count hold anything and are not looked at.
+    f32x4 q_in[D / 8];
     {
         const float *qp = reinterpret_cast<const float *>(p.q) + b * p.qs[0] + h * p.qs[1] + (int64_t)qrow * p.qs[2] + (D / 2) * hh;
 #pragma unroll
-        for (int c = 0; c < D / 2; c += 4) {
-            const f32x4 x = *(const f32x4 *)(qp + c);
-#pragma unroll
-            for (int e = 0; e < 4; e++) qf[c + e] = x[e] * p.scale;
-        }
+        for (int c = 0; c < D / 8; c++) q_in[c] = *(const f32x4 *)(qp + 4 * c);
     }
+    const bool in_lanes = SP && p.nK <= 64;
+    int lane_full = 0, lane_part = 0;
+    if (in_lanes) {
+        const int slot = min(lane, p.nK - 1);
+        lane_full = fid[(int64_t)slot * p.fis[3]];
+        lane_part = pid[(int64_t)slot * p.pis[3]];
+    }
+    int cnt[2];
+    const int32_t *const cnt_addr[2] = {p.full_lens + (b * p.fls[0] + h * p.fls[1] + qt * p.fls[2]),
+                                        p.part_lens + (b * p.pls[0] + h * p.pls[1] + qt * p.pls[2])};
+    scalar_gather(cnt_addr, cnt);
+    int F = min(min(max(cnt[0], 0), p.nK), kF32ListCap);
+    int NE = F + min(min(max(cnt[1], 0), p.nK - F), kF32ListCap - F);
+    int share = 1, f_lo = 0, p_lo = 0, T_all = 0;  // T_all (KG > 1): chunks of the longest group
+    auto part_of = [&](int s, int n) {  // the s-th of n runs of what is left of the list
+        const int e_lo = fwd_split_first(NE, p.lbk, 5, s, n), e_hi = fwd_split_first(NE, p.lbk, 5, s + 1, n);
+        f_lo += min(e_lo, F);
+        p_lo += max(e_lo - F, 0);
+        F = min(max(F - e_lo, 0), e_hi - e_lo);
+        NE = e_hi - e_lo;
+    };
+    auto chunks_of = [&](int ne) { return MODE == 2 ? (ne << (p.lbk - 5)) : ((ne + EPC - 1) / EPC); };
+    if constexpr (SP) {
+        share = fwd_split_share(NE, p.lbk, 5, p.split_least, p.split_chunks, p.nsplit);
+        if (s0 >= share) return;
+        part_of(s0, share);
+    }
+    if constexpr (KG > 1) {
+        const int all = NE;
+        part_of(grp, KG);
+#pragma unroll
+        for (int i = 0; i < KG; i++)
+            T_all = max(T_all, chunks_of(fwd_split_first(all, p.lbk, 5, i + 1, KG) - fwd_split_first(all, p.lbk, 5, i, KG)));
+    }
+    fid += (int64_t)f_lo * p.fis[3];
+    pid += (int64_t)p_lo * p.pis[3];
+    const int T = chunks_of(NE);
+    if constexpr (KG == 1) T_all = T;
+    const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const SA_LDS uint8_t *)smem);
 
     // ---- per-lane constants ------------------------------------------------------------------------------------
     const int koff0 = l32 * ROWB + 16 * ((hh * (PPR / 2)) ^ (l32 & 15));  // read i of the row half: koff0 ^ (16 i)
@@ -141,7 +177,10 @@ __global__ __launch_bounds__(NW * 64, NW >= 4 ? 2 : 1) void sparse_fwd_f32_mfma_
         for (int j = 0; j < EPC; j++) {
             const int e = MODE == 2 ? (t >> (p.lbk - 5)) : t * EPC + j;
             const int sub = MODE == 2 ? (t & ((1 << (p.lbk - 5)) - 1)) : 0;
-            plan_entry(pl, j, e, __builtin_amdgcn_readfirstlane(ring[min(e, kF32ListCap - 1)]), sub);
+            int idx;
+            if (in_lanes) idx = e < F ? __builtin_amdgcn_readlane(lane_full, min(f_lo + e, 63)) : __builtin_amdgcn_readlane(lane_part, min(p_lo + max(e - F, 0), 63));
+            else idx = __builtin_amdgcn_readfirstlane(ring[min(e, kF32ListCap - 1)]);
+            plan_entry(pl, j, e, idx, sub);
         }
     };
     // all direct loads of a chunk into stage `buf`
@@ -188,29 +227,45 @@ __global__ __launch_bounds__(NW * 64, NW >= 4 ? 2 : 1) void sparse_fwd_f32_mfma_
 #pragma unroll
         for (int i = 0; i < 16; i++) acc[db][i] = 0.f;
 
-    if (T > 0) {
-        // the list: wave w brings entries 64 w + lane, 64 (w + NW) + lane, ...
-        for (int base = 64 * wave_u; base < NE; base += 64 * NW) {
-            const int e = min(base + lane, NE - 1);
-            const int32_t *src = e < F ? fid + (int64_t)e * p.fis[3] : pid + (int64_t)(e - F) * p.pis[3];
-            dma4_lane(src, lds0 + OFF_L + 4 * base);
+    // Q^T operand: d = (D/2) hh + c for step c, scaled once (softmax scale / ln 2)
+    float qf[D / 2];
+    auto scale_q = [&]() {
+#pragma unroll
+        for (int c = 0; c < D / 2; c++) qf[c] = q_in[c / 4][c % 4] * p.scale;
+    };
+    if (T_all > 0) {
+        if (!in_lanes) {
+            // the list: wave w brings entries 64 w + lane, 64 (w + NW) + lane, ...
+            for (int base = 64 * wave_u; base < NE; base += 64 * NW) {
+                const int e = min(base + lane, NE - 1);
+                const int32_t *src = e < F ? fid + (int64_t)e * p.fis[3] : pid + (int64_t)(e - F) * p.pis[3];
+                dma4_lane(src, lds0 + OFF_L + 4 * base);
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
         }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
         Plan pl;
-        plan_of(0, pl);
-        stage_chunk(0, pl, 0);
-        unsigned fl_cur = pl.flags;
+        if (T > 0) {  // (KG > 1: another group may have entries where this one has none)
+            plan_of(0, pl);
+            stage_chunk(0, pl, 0);
+        }
+        unsigned fl_cur = T > 0 ? pl.flags : 0u;
+        scale_q();
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
 
         auto chunk = [&](auto buf_c, int tc) {
             constexpr int BUF = decltype(buf_c)::value;
-            // the next chunk goes to the other stage (past the last chunk: the last one once more, harmless)
-            Plan pn;
-            const int tn = tc + 1 < T ? tc + 1 : T - 1;
-            plan_of(tn, pn);
-            stage_chunk(BUF ^ 1, pn, tn);
+            // the next chunk goes to the other stage (past the last chunk the last one once more: in a long loop cheaper than the
+            // branch, 1 %, but a part of one chunk would wait for it)
+            unsigned fl_next = 0u;
+            if (!SP || tc + 1 < T) {
+                const int tn = tc + 1 < T ? tc + 1 : T - 1;
+                Plan pn;
+                plan_of(tn, pn);
+                stage_chunk(BUF ^ 1, pn, tn);
+                fl_next = pn.flags;
+            }
 
             // ---- S^T = K . Q^T ----
             const uint8_t *kb_ = smem + BUF * KBUF;
@@ -219,11 +274,20 @@ __global__ __launch_bounds__(NW * 64, NW >= 4 ? 2 : 1) void sparse_fwd_f32_mfma_
             for (int i = 0; i < 16; i++) s[i] = 0.f;
             int kbo = koff0;
             asm volatile("" : "+v"(kbo));
+            // (SP: operand reads three bundles ahead, pinned, where each was waited for as it was issued: the products and softmax of a lone
+            // chunk 3.2 -> 2.95 us; in the plain form, whose waves cover for each other, 1 % slower)
+            constexpr int kAheadK = SP ? 3 : 0;
+            f32x4 kf[PPR / 2];
+            auto k_read = [&](int i) { kf[i] = *(const f32x4 *)(kb_ + (kbo ^ (16 * i))); };
+#pragma unroll
+            for (int i = 0; i < kAheadK; i++) k_read(i);
+            if constexpr (SP) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < PPR / 2; i++) {
-                const f32x4 kv = *(const f32x4 *)(kb_ + (kbo ^ (16 * i)));
+                if (i + kAheadK < PPR / 2) k_read(i + kAheadK);
 #pragma unroll
-                for (int e = 0; e < 4; e++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv[e], qf[4 * i + e], s, 0, 0, 0);
+                for (int e = 0; e < 4; e++) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[i][e], qf[4 * i + e], s, 0, 0, 0);
+                if constexpr (SP) __builtin_amdgcn_sched_barrier(0);
             }
 
             // ---- mask (chunks with a PARTIAL or missing entry only) ----
@@ -299,57 +363,109 @@ __global__ __launch_bounds__(NW * 64, NW >= 4 ? 2 : 1) void sparse_fwd_f32_mfma_
                         const float vv = *(const float *)(vb_ + (8 * g + j) * ROWB + (vbo ^ (128 * db)));
                         acc[db] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv, s[4 * g + j], acc[db], 0, 0, 0);
                     }
-            fl_cur = pn.flags;
+            fl_cur = fl_next;
+        };
+        auto step = [&](auto buf_c, int tc) {
+            if (KG == 1 || tc < T) chunk(buf_c, tc);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the next chunk has landed
             __syncthreads();                                   // and every wave is done with this one
         };
-        for (int t = 0; t < T; t += 2) {
-            chunk(std::integral_constant<int, 0>{}, t);
-            if (t + 1 < T) chunk(std::integral_constant<int, 1>{}, t + 1);
+        for (int t = 0; t < T_all; t += 2) {
+            step(std::integral_constant<int, 0>{}, t);
+            if (t + 1 < T_all) step(std::integral_constant<int, 1>{}, t + 1);
         }
     }
 
-    // ---- O = acc / l (sparse_attn_kernel.py:144); rows without a key give 0 ----
-    {
-        const uint32_t lu = __float_as_uint(l_i);
-        const auto sw = __builtin_amdgcn_permlane32_swap(lu, lu, false, false);
-        const float l_tot = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
-        if (share > 1) {
-            const int64_t part_id = ((int64_t)(b * p.H + h) * p.nQ + qt) * p.nsplit + s0;
-            float *const wo = p.ws + (part_id * NW + wave_u) * (32 * D) + 4 * lane;
+    // ---- the groups' rows, the parts' rows, O = acc / l (sparse_attn_kernel.py:144); rows without a key give 0 ----
+    const uint32_t lu = __float_as_uint(l_i);
+    const auto sw = __builtin_amdgcn_permlane32_swap(lu, lu, false, false);
+    float l_tot = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+    auto finish = [&](auto g_c) {
+        constexpr int G = decltype(g_c)::value, NB = D / 32 / KG;  // this group's blocks of 32 columns: G NB ...
+        f32x16 o[NB];
 #pragma unroll
-            for (int db = 0; db < D / 32; db++)
+        for (int d = 0; d < NB; d++) o[d] = acc[G * NB + d];
+        if constexpr (KG > 1) {
+            // each group leaves the other's columns in its own stages, which nobody reads any more, its rows' state in its list
+            static_assert(KG == 2 && NW * 32 * D * 2 <= 4 * KBUF && NW * 32 * 8 <= kF32ListCap * 4, "what a group leaves fits its LDS");
+            const uint32_t at = wave_u * (NB * 4096) + 16 * lane, st_at = OFF_L + (wave_u * 32 + l32) * 8;
+#pragma unroll
+            for (int d = 0; d < NB; d++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const f32x16 &a = acc[(1 - G) * NB + d];
+                    *(f32x4 *)(smem + at + 1024 * (4 * d + g)) = f32x4{a[4 * g], a[4 * g + 1], a[4 * g + 2], a[4 * g + 3]};
+                }
+            if (hh == 0) *(f32x2 *)(smem + st_at) = f32x2{m_i, l_tot};
+            __syncthreads();
+            const uint8_t *const other = smem0 + (1 - G) * GROUP;
+            const f32x2 st = *(const f32x2 *)(other + st_at);
+            const float M = fmaxf(m_i, st.x), M0 = M == kNegInf ? 0.f : M;
+            const float mine = __builtin_amdgcn_exp2f(m_i - M0), its = __builtin_amdgcn_exp2f(st.x - M0);
+            // (the first group's values first, whichever group adds)
+            auto add = [&](float a, float x) { return G == 0 ? __builtin_fmaf(a, mine, its * x) : __builtin_fmaf(x, its, mine * a); };
+            l_tot = add(l_tot, st.y);
+#pragma unroll
+            for (int d = 0; d < NB; d++)
+#pragma unroll
+                for (int g = 0; g < 4; g++) {
+                    const f32x4 x = *(const f32x4 *)(other + at + 1024 * (4 * d + g));
+#pragma unroll
+                    for (int e = 0; e < 4; e++) o[d][4 * g + e] = add(o[d][4 * g + e], x[e]);
+                }
+            m_i = M;
+        }
+        if (SP && share > 1) {
+            const int64_t tile = (int64_t)(b * p.H + h) * p.nQ + qt, first = tile * p.nsplit;
+            constexpr uint32_t rows_step = NW * 32 * D * 4, state_step = NW * 32 * 8;
+            const HandOver rows(p.ws + first * (rows_step / 4), p.nsplit * rows_step), state(p.ws_ml + first * (state_step / 4), p.nsplit * state_step);
+            const uint32_t rows_at = wave_u * (32 * D * 4) + G * NB * 4096 + 16 * lane, state_at = (wave_u * 32 + l32) * 8;
+#pragma unroll
+            for (int d = 0; d < NB; d++)
 #pragma unroll
                 for (int g = 0; g < 4; g++)
-                    *(f32x4 *)(wo + 256 * (4 * db + g)) = f32x4{acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]};
-            if (hh == 0) *(f32x2 *)(p.ws_ml + 2 * (part_id * (NW * 32) + wave * 32 + l32)) = f32x2{m_i, l_tot};
-            return;
+                    rows.put(s0 * rows_step + rows_at + 1024 * (4 * d + g), f32x4{o[d][4 * g], o[d][4 * g + 1], o[d][4 * g + 2], o[d][4 * g + 3]});
+            if (G == 0 && hh == 0) state.put(s0 * state_step + state_at, f32x2{m_i, l_tot});
+            if (p.arrivals == nullptr) return;
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();  // every wave's rows have been handed over, and LDS has been read
+            if (threadIdx.x < 64) {
+                const bool all = all_arrived(p.arrivals + first, p.tag, s0, share);
+                if (threadIdx.x == 0) *reinterpret_cast<int *>(smem0) = all;
+            }
+            __syncthreads();
+            if (__builtin_amdgcn_readfirstlane(*reinterpret_cast<int *>(smem0)) == 0) return;
+            add_parts<NB, NB == 1 ? 8 : (NB == 2 ? 3 : 2)>(rows, rows_at, rows_step, state, state_at, state_step, share, o, m_i, l_tot);
         }
         const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
-        if (p.lse != nullptr && hh == 0)
+        if (G == 0 && p.lse != nullptr && hh == 0)
             p.lse[b * p.lses[0] + h * p.lses[1] + (int64_t)qrow * p.lses[2]] =
                 l_tot > 0.f ? (m_i + __builtin_amdgcn_logf(l_tot)) * 0.69314718056f : kNegInf;
-        float *orow = reinterpret_cast<float *>(p.o) + b * p.os[0] + h * p.os[1] + (int64_t)qrow * p.os[2] + 4 * hh;
+        float *orow = reinterpret_cast<float *>(p.o) + b * p.os[0] + h * p.os[1] + (int64_t)qrow * p.os[2] + 4 * hh + 32 * G * NB;
 #pragma unroll
-        for (int db = 0; db < D / 32; db++)
+        for (int d = 0; d < NB; d++)
 #pragma unroll
-            for (int g = 0; g < 4; g++) {
-                const f32x4 w = {acc[db][4 * g] * inv, acc[db][4 * g + 1] * inv, acc[db][4 * g + 2] * inv,
-                                 acc[db][4 * g + 3] * inv};
-                *(f32x4 *)(orow + 32 * db + 8 * g) = w;
-            }
-    }
+            for (int g = 0; g < 4; g++)
+                *(f32x4 *)(orow + 32 * d + 8 * g) = f32x4{o[d][4 * g] * inv, o[d][4 * g + 1] * inv, o[d][4 * g + 2] * inv, o[d][4 * g + 3] * inv};
+    };
+    if (KG == 1 || grp == 0) finish(std::integral_constant<int, 0>{});
+    else finish(std::integral_constant<int, KG - 1>{});
+}
+
+template <int D, int NW, int MODE, bool PK, bool SP>
+hipError_t launch_lists(const FwdParams &p, hipStream_t stream) {
+    constexpr int smem = f32_groups(NW, SP) * f32_group_bytes<D, NW>;
+    auto kern = sparse_fwd_f32_mfma_kernel<D, NW, MODE, PK, SP>;
+    static unsigned long long attr_done = 0;
+    if (const hipError_t e0 = allow_dynamic_smem(kern, smem, attr_done); e0 != hipSuccess) return e0;
+    hipLaunchKernelGGL(kern, dim3((unsigned)p.nQ * (unsigned)(p.B * p.H) * (unsigned)(SP ? p.nsplit : 1)),
+                       dim3(f32_groups(NW, SP) * NW * 64), smem, stream, p);
+    return hipGetLastError();
 }
 
 template <int D, int NW, int MODE, bool PK>
 hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
-    constexpr int smem = 4 * 32 * D * 4 + 2 * NW * 1024 + kF32ListCap * 4;
-    auto kern = sparse_fwd_f32_mfma_kernel<D, NW, MODE, PK>;
-    static unsigned long long attr_done = 0;
-    if (const hipError_t e0 = allow_dynamic_smem(kern, smem, attr_done); e0 != hipSuccess) return e0;
-    hipLaunchKernelGGL(kern, dim3((unsigned)p.nQ * (unsigned)(p.B * p.H) * (unsigned)(p.nsplit > 1 ? p.nsplit : 1)),
-                       dim3(NW * 64), smem, stream, p);
-    return hipGetLastError();
+    return p.nsplit > 1 ? launch_lists<D, NW, MODE, PK, true>(p, stream) : launch_lists<D, NW, MODE, PK, false>(p, stream);
 }
 
 template <int D, int NW, bool PK>
@@ -391,7 +507,7 @@ hipError_t launch_fwd_f32_mfma(const FwdParams &p, int D, int BQ, hipStream_t st
     if (!fwd_f32_mfma_has(p, D, BQ)) return hipErrorInvalidValue;
     const hipError_t e = p.packed != nullptr ? (D == 64 ? launch_bq<64, true>(p, BQ, stream) : launch_bq<128, true>(p, BQ, stream))
                                              : (D == 64 ? launch_bq<64, false>(p, BQ, stream) : launch_bq<128, false>(p, BQ, stream));
-    return e != hipSuccess || p.nsplit <= 1 ? e : launch_fwd_merge(p, 2, D, BQ, stream);
+    return e != hipSuccess || p.nsplit <= 1 || p.arrivals != nullptr ? e : launch_fwd_merge(p, 2, D, BQ, stream);
 }
 
 }  // namespace sa

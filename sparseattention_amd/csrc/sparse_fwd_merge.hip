@@ -105,7 +105,7 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(const FwdParams p, int l
 // From 257 tiles on every slot has work.  Sk below 32 chunks is not shared, whatever the lists (32 chunks, Sk = 2048: 8 tiles
 // 33.6 | 17.0, 64 tiles 34.7 | 26.3, 128 tiles 35.2 | 33.6; 16 chunks: the tables above, as lists of a longer Sk).
 // float32: a chunk of 32 keys keeps the matrix unit busy for 1.7 us (D = 64) or 3.4 us, so two chunks are worth a part
-// (32 tiles of 16 chunks at D = 64: 46 -> 16 us, 256 of 32 at D = 128: 158 -> 95 us).  Sk above 4096 is not shared there: a row's
+// (32 tiles of 16 chunks at D = 64: 46 -> 11.7 us, 256 of 32 at D = 128: 158 -> 95 us).  Sk above 4096 is not shared there: a row's
 // keys are added up one after the other in one workgroup, 1.2e-6 from the result at 4096 keys and 3.3e-6 at 32768, and shared
 // lists (4e-7 and 7e-7) would move the result by that much.
 FwdSplitPlan fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus) {
@@ -122,6 +122,13 @@ FwdSplitPlan fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus
     plan.least = part == 16 ? 8 + tiles / 8 : part;
     return plan;
 }
+
+// One workgroup reads all parts of its Q tile, where a second launch spreads them over the device: in the launch up to 256 KiB a tile.
+// float32, us, second launch | last workgroup (parts x KiB a part, every list that long):
+//   8 x 16  32 tiles 13.3 | 11.7    32 x 8  8 tiles 19.8 | 17.5    8 x 32  32 tiles 18.5 | 17.3
+//   32 x 16  16 tiles 25.2 | 24.9, 8 tiles 21.0 | 20.7, 4 tiles 20.2 | 20.4    16 x 32  16 tiles 20.1 | 20.0    8 x 64  16 tiles 21.9 | 23.6
+//   32 x 32  8 tiles 29.2 | 33.6, 4 tiles 25.0 | 29.6    16 x 64  16 tiles 28.9 | 30.6    32 x 64  4 tiles 38.0 | 50.7
+bool fwd_merges_in_launch(int nsplit, int BQ, int D, int dtype) { return dtype == 2 && (int64_t)nsplit * BQ * D * 4 <= 256 * 1024; }
 
 // When a list is walked in two halves by one workgroup of twice the waves (sparse_fwd_kernel<..., TW>): from half as many Q tiles
 // as compute units on, up to as many.  A compute unit has one workgroup then, which leaves half of its registers and LDS

@@ -278,7 +278,8 @@ bool in_halves(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype) {
     return sa::fwd_in_halves((int64_t)B * H * (Sq / BQ), Sk, BQ, BK, D, dtype, cus);
 }
 
-// How lists are shared on the current device, and the bytes of the partial results (0: they are not).
+// How lists are shared on the current device, and the bytes of the partial results (0: they are not).  Where the last workgroup to
+// arrive adds them up (fwd_merges_in_launch), 8 bytes per part follow, in which its workgroup says that it is done.
 size_t split_shape(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype, sa::FwdSplitPlan *plan) {
     *plan = sa::FwdSplitPlan();
     if (B <= 0 || H <= 0 || Sq <= 0 || Sk <= 0 || BQ <= 0 || BK <= 0 || Sq % BQ || Sk % BK || log2_exact(BK) < 4) return 0;
@@ -444,6 +445,11 @@ int forward_impl(const void *q, const int64_t q_strides[4], const void *k, const
             return fail(SA_ERR_WORKSPACE, "sa_sparse_attention_fwd_split: a 16-byte aligned workspace of %zu bytes required, %zu given", need, workspace_bytes);
         fp.ws = static_cast<float *>(workspace);
         fp.ws_ml = fp.ws + (need / 4 / (size_t)(D + 2)) * (size_t)D;
+        // (a caller who asked an earlier library for the size has no place for them: a second launch then)
+        if (need != 0 && sa::fwd_merges_in_launch(plan.nsplit, BQ, D, dtype) && workspace_bytes >= need + (size_t)8 * B * H * fp.nQ * plan.nsplit) {
+            fp.arrivals = reinterpret_cast<uint64_t *>(static_cast<uint8_t *>(workspace) + need);
+            fp.tag = next_launch_tag();
+        }
     }
     if (kernel == SA_FWD_KERNEL_SHORT_LISTS) {
         if (f32 || !sa::fwd_c32_has(fp, dtype, D, BQ))
@@ -564,7 +570,8 @@ int sa_sparse_attention_fwd_kernel(const void *q, const int64_t q_strides[4], co
 size_t sa_fwd_split_workspace_bytes(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype) {
     sa::FwdSplitPlan plan;
     if ((D != 64 && D != 128) || dtype < SA_DTYPE_BF16 || dtype > SA_DTYPE_FP32) return 0;
-    return split_shape(B, H, Sq, Sk, D, BQ, BK, dtype, &plan);
+    const size_t parts = split_shape(B, H, Sq, Sk, D, BQ, BK, dtype, &plan);
+    return parts != 0 && sa::fwd_merges_in_launch(plan.nsplit, BQ, D, dtype) ? parts + (size_t)8 * B * H * (Sq / BQ) * plan.nsplit : parts;
 }
 
 int sa_fwd_split_least_keys(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype) {

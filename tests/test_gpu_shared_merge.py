@@ -1,0 +1,113 @@
+"""Shared lists whose last workgroup adds the parts up (the whole workspace) against the merge by a second launch (a workspace without
+place for the workgroups' words) and against the definition."""
+import ctypes
+import math
+
+import pytest
+import torch
+
+from sparseattention_amd import _native, compute_mask_kernel, workloads as W
+
+pytestmark = pytest.mark.gpu
+
+CODE = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
+# a result's own rounding (2^-9, 2^-12 of values up to 4) with that of P, twice; float32: a row's sum of 4096 terms in another order
+TOL = {torch.bfloat16: 2e-2, torch.float16: 4e-3, torch.float32: 1e-5}
+
+
+def forward(q, k, v, md, BQ, BK, ws, ws_bytes, o, lse):
+    S, (B, H, Sq, D), Sk = _native.strides, q.shape, k.shape[2]
+    args = []
+    for t in (q, k, v, o):
+        args += [t.data_ptr(), S(t.stride())]
+    args += [None, None]
+    for t in (md.unmasked_kv_ids, md.unmasked_lens, md.masked_kv_ids, md.masked_lens):
+        args += [t.data_ptr(), S(t.stride())]
+    args += [md.packed_masks.data_ptr(), S(md.packed_masks.stride()[:2]), lse.data_ptr(), S(lse.stride())]
+    rc = _native.load().sa_sparse_attention_fwd_split(*args, B, H, Sq, Sk, D, BQ, BK, CODE[q.dtype], D ** -0.5 / math.log(2), ws.data_ptr(),
+                                                      ws_bytes, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0, _native.load().sa_last_error()
+
+
+def sizes(q, Sk, BQ, BK):
+    """(bytes with the words, bytes of the parts alone)"""
+    B, H, Sq, D = q.shape
+    full = _native.load().sa_fwd_split_workspace_bytes(B, H, Sq, Sk, D, BQ, BK, CODE[q.dtype])
+    tiles, part = B * H * (Sq // BQ), BQ * (D + 2) * 4
+    assert full > 0 and full % (tiles * (part + 8)) == 0
+    return full, full // (part + 8) * part
+
+
+def uneven(B, H, Sq, Sk, BQ, gpu):
+    """Lists from none to all tiles, FULL, PARTIAL and EMPTY ones in turn; rows that attend to nothing."""
+    mask = torch.rand(B, 1, Sq, Sk, generator=torch.Generator().manual_seed(Sk)) < 0.5
+    for c in range(0, Sk, 256):
+        mask[..., c:c + 64] = True
+        mask[..., c + 64:c + 128] = False
+    mask[:, :, 3] = False
+    mask[0, 0, :BQ, Sk // 2 + 5:] = False  # (parts without a key)
+    mask[-1, 0, Sq - BQ:, 33:] = False     # one short list
+    mask[-1, 0, Sq - BQ:, :33] = True
+    return mask.to(gpu).expand(B, H, Sq, Sk)
+
+
+@pytest.mark.parametrize("dtype,B,H,Sq,Sk,D,BQ,BK", [
+    (torch.float32, 1, 4, 512, 512, 64, 64, 32),      # two groups of waves
+    (torch.float32, 1, 3, 192, 160, 64, 64, 16),      # an odd number of chunks: one group has one more
+    (torch.float32, 1, 2, 64, 1280, 64, 32, 16),      # lists that come by way of LDS; one wave a group
+    (torch.float32, 1, 2, 128, 1024, 64, 64, 256),    # entries of several chunks: a group without any
+    (torch.float32, 1, 2, 128, 256, 128, 64, 32),
+    (torch.float32, 2, 16, 512, 160, 128, 128, 32),   # one group of four waves
+])
+def test_the_last_workgroup_adds_up(gpu, dtype, B, H, Sq, Sk, D, BQ, BK):
+    q, _, _ = W.qkv(B, H, Sq, D, dtype, seed=1, device=gpu)
+    _, k, v = W.qkv(B, H, Sk, D, dtype, seed=2, device=gpu)
+    mask = uneven(B, H, Sq, Sk, BQ, gpu)
+    md = compute_mask_kernel(mask, BQ, BK)
+    full, parts = sizes(q, Sk, BQ, BK)
+    out = lambda: (torch.empty_like(q), torch.empty(B, H, Sq, device=gpu))  # noqa: E731
+    ws = torch.empty(full + 64, dtype=torch.uint8, device=gpu)
+    two, one = out(), out()
+    forward(q, k, v, md, BQ, BK, ws, parts, *two)
+    for fill in (255, 0, None):  # whatever the memory held; last, what a call left
+        if fill is not None:
+            ws.fill_(fill)
+        got = out()
+        forward(q, k, v, md, BQ, BK, ws, full, *got)
+        torch.cuda.synchronize()
+        if fill == 255:
+            one = got
+        assert torch.equal(got[0], one[0]) and torch.equal(got[1], one[1])  # (the parts in their order, whoever adds)
+    s = ((q.double() @ k.double().transpose(-1, -2).contiguous()) * D ** -0.5).masked_fill(~mask, float("-inf"))
+    want, want_lse = torch.nan_to_num(torch.softmax(s, -1)) @ v.double(), torch.logsumexp(s, -1)
+    live = torch.isfinite(want_lse)
+    for o, lse in (one, two):
+        assert float((o.double() - want).abs().max()) <= TOL[dtype]
+        assert torch.equal(torch.isfinite(lse), live)
+        assert float((lse.double() - want_lse)[live].abs().max()) <= (1e-5 if dtype == torch.float32 else 6e-3 + 2 ** -9 * 5)
+
+
+@pytest.mark.parametrize("dtype,B,H,Sq,Sk,D,BQ,BK", [(torch.float32, 1, 4, 256, 512, 64, 64, 32)])
+def test_replays_bring_the_same_launch_number(gpu, dtype, B, H, Sq, Sk, D, BQ, BK):
+    q, _, _ = W.qkv(B, H, Sq, D, dtype, seed=1, device=gpu)
+    _, k, v = W.qkv(B, H, Sk, D, dtype, seed=2, device=gpu)
+    md = compute_mask_kernel(uneven(B, H, Sq, Sk, BQ, gpu), BQ, BK)
+    full, _ = sizes(q, Sk, BQ, BK)
+    ws = torch.zeros(full, dtype=torch.uint8, device=gpu)
+    o, lse = torch.empty_like(q), torch.empty(B, H, Sq, device=gpu)
+    forward(q, k, v, md, BQ, BK, ws, full, o, lse)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        forward(q, k, v, md, BQ, BK, ws, full, o, lse)
+    for i in range(4):
+        q.copy_(torch.randn_like(q))
+        want, wlse = torch.empty_like(q), torch.empty_like(lse)
+        if i == 2:
+            ws.fill_(37)
+        graph.replay()
+        torch.cuda.synchronize()
+        got, glse = o.clone(), lse.clone()
+        forward(q, k, v, md, BQ, BK, torch.empty_like(ws), full, want, wlse)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and torch.equal(glse, wlse)
