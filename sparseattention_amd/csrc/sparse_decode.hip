@@ -103,6 +103,20 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
     const int bh = (int)(blockIdx.x / (unsigned)p.nsplit), split = (int)(blockIdx.x - (unsigned)bh * (unsigned)p.nsplit);
     const int b = bh / p.H, h = bh - b * p.H;
 
+    // query row of this lane (rows past Sq are padding: zero queries, row 0's mask, never stored)
+    const bool live = l32 < p.Sq;
+    const int qrow = live ? l32 : 0;
+    // Q^T operand: lane (l32, hh) keeps d = (D/2) hh + 8c .. +7 of its row for step c (K uses the same order, so each lane's K
+    // bytes are contiguous).  Requested first of all, with the counts or the mask, and scaled once behind the requests for the first chunk:
+    // requested and scaled in front of them it was a memory round trip of its own (B4 H32 Sq1 Sk2048 with a new mask 22.6 -> 21.8 us a
+    // call, B8 H16 Sq16 Sk16384 gathered 90.5 -> 89.4).
+    u32x4 qf[NC];
+    {
+        const uint16_t *qp = p.q + b * p.qs[0] + h * p.qs[1] + (int64_t)qrow * p.qs[2] + (D / 2) * hh;
+#pragma unroll
+        for (int c = 0; c < NC; c++) qf[c] = *(const u32x4 *)(qp + 8 * c);
+    }
+
     const uint16_t *kbase = p.k + b * p.ks[0] + h * p.ks[1];
     const uint16_t *vbase = p.v + b * p.vs[0] + h * p.vs[1];
     const int32_t *fid = DM ? nullptr : p.full_ids + b * p.fis[0] + h * p.fis[1];
@@ -165,26 +179,11 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
               t_hi = (int)((unsigned)T * (unsigned)(split + 1) / (unsigned)p.nsplit);  // T * nsplit < 2^31 (checked by the caller)
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
 
-    // query row of this lane (rows past Sq are padding: zero queries, row 0's mask, never stored)
-    const bool live = l32 < p.Sq;
-    const int qrow = live ? l32 : 0;
     const uint8_t *mrow = PK || DM ? nullptr : p.mask + b * p.ms[0] + h * p.ms[1] + (int64_t)qrow * p.ms[2];
     // this row's bits in the packed tile of a PARTIAL slot: BK/8 bytes per row, Sq rows per tile
     const int64_t tile_bytes = (int64_t)p.Sq * (p.BK >> 3);
     const uint8_t *prow = PK ? p.packed + b * p.pks[0] + h * p.pks[1] + (int64_t)qrow * (p.BK >> 3) : nullptr;
 
-    // Q^T operand, scaled once: lane (l32, hh) keeps d = (D/2) hh + 8c .. +7 of its row for step c (K uses the same
-    // order, so each lane's K bytes are contiguous)
-    u32x4 qf[NC];
-    {
-        const uint16_t *qp = p.q + b * p.qs[0] + h * p.qs[1] + (int64_t)qrow * p.qs[2] + (D / 2) * hh;
-#pragma unroll
-        for (int c = 0; c < NC; c++) {
-            qf[c] = *(const u32x4 *)(qp + 8 * c);
-#pragma unroll
-            for (int e = 0; e < 4; e++) qf[c][e] = live ? E::scale2(qf[c][e], p.scale) : 0u;
-        }
-    }
 
     // online-softmax state of this lane's query row (see sparse_fwd_kernel.h); scores start from 0 here and the
     // reference value is subtracted before the exponential
@@ -427,6 +426,10 @@ __global__ __launch_bounds__(kDecodeWaves * 64, 2) void sparse_decode_kernel(con
             cols_of(t, idxs[0], col);
             issue(t, col, 0, kf[0], mk[0]);
         }
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) qf[c][e] = live ? E::scale2(qf[c][e], p.scale) : 0u;
         for (; t < t_hi; t += 2 * kDecodeWaves) {
             static_for<2>([&](auto jc) {
                 constexpr int j = decltype(jc)::value;
