@@ -69,8 +69,8 @@ __device__ __forceinline__ void wait_vm_at_most(int n, int step) {
 // the other (arguments, counts, lists, first K/V chunk) are paid once per workgroup instead of once per tile.
 // SP: the list of a Q tile is shared by up to p.nsplit workgroups (fwd_split_share), for launches with too few Q tiles to
 // fill the device: a chunk of a prompt against a long cache.  Every workgroup walks a range of its own and leaves
-// unnormalised rows with their reference values and sums in p.ws, which fwd_merge_kernel adds up; a tile whose list is
-// too short to be shared is written as by the plain kernel.
+// unnormalised rows with their reference values and sums in p.ws; the last of a few (fwd_merges_in_launch) to arrive adds them up, else
+// fwd_merge_kernel does.  A tile whose list is too short to be shared is written as by the plain kernel.
 // RG: the tile grid is larger than the tensors (p.q0, p.k0: rows of it in front of the first query and key; p.Sq_in, p.Sk_in:
 // rows there are) and the head dim may be smaller than D (p.D_in, a multiple of 8).  Nothing is padded in memory: queries
 // and pieces of rows that do not exist enter as zeros (pieces from a zero in device memory, since a direct load brings
@@ -1279,18 +1279,34 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
     if constexpr (PP) __syncthreads();  // the late waves of the ping-pong schedule have read their last stage
     if constexpr (SP) {
         if (share > 1) {
-            // in the order the registers hold them: whole 1 KiB runs per store instruction (fwd_merge_kernel reads them so)
-            const int64_t part_id = ((int64_t)(b * p.H + h) * p.nQ + qt) * p.nsplit + share_part;
-            float *const wo = p.ws + (part_id * NW + wave_u) * (32 * D) + 4 * lane;
+            // in the order the registers hold them: whole 1 KiB runs per store instruction (add_parts, fwd_merge_kernel)
+            const int64_t tile = (int64_t)(b * p.H + h) * p.nQ + qt, first = tile * p.nsplit;
+            constexpr uint32_t rows_step = NW * 32 * D * 4, state_step = NW * 32 * 8;
+            const HandOver rows(p.ws + first * (rows_step / 4), p.nsplit * rows_step), state(p.ws_ml + first * (state_step / 4), p.nsplit * state_step);
+            const uint32_t rows_at = wave_u * (32 * D * 4) + 16 * lane, state_at = (wave_u * 32 + l32) * 8;
 #pragma unroll
             for (int db = 0; db < D / 32; db++)
 #pragma unroll
                 for (int g = 0; g < 4; g++)
-                    *(f32x4 *)(wo + 256 * (4 * db + g)) = f32x4{acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]};
+                    rows.put(share_part * rows_step + rows_at + 1024 * (4 * db + g),
+                             f32x4{acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]});
             if (hh == 0)
-                *(f32x2 *)(p.ws_ml + 2 * (part_id * (NW * 32) + wave * 32 + l32)) =
-                    f32x2{raise_above == kMaxSlack ? m_ref : kNegInf, l32 < 16 ? acc_l[0] : acc_l[1]};
-            return;
+                state.put(share_part * state_step + state_at, f32x2{raise_above == kMaxSlack ? m_ref : kNegInf, l32 < 16 ? acc_l[0] : acc_l[1]});
+            if (p.arrivals == nullptr) return;
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();  // every wave's rows have been handed over
+            int *const last = reinterpret_cast<int *>(smem);  // (a stage nobody reads any more)
+            if (tid < 64) {
+                const bool all = all_arrived(p.arrivals + first, p.tag, share_part, share);
+                if (tid == 0) *last = all;
+            }
+            __syncthreads();
+            if (__builtin_amdgcn_readfirstlane(*last) == 0) return;
+            __syncthreads();  // (the stages are about to hold output rows)
+            float M, L;
+            add_parts<D / 32, D == 128 ? 2 : 4>(rows, rows_at, rows_step, state, state_at, state_step, share, acc, M, L);
+            acc_l[0] = acc_l[1] = L;
+            m_ref = M == kNegInf ? 0.f : M;
         }
     }
     if (TW && share == 2) {

@@ -128,7 +128,13 @@ FwdSplitPlan fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus
 //   8 x 16  32 tiles 13.3 | 11.7    32 x 8  8 tiles 19.8 | 17.5    8 x 32  32 tiles 18.5 | 17.3
 //   32 x 16  16 tiles 25.2 | 24.9, 8 tiles 21.0 | 20.7, 4 tiles 20.2 | 20.4    16 x 32  16 tiles 20.1 | 20.0    8 x 64  16 tiles 21.9 | 23.6
 //   32 x 32  8 tiles 29.2 | 33.6, 4 tiles 25.0 | 29.6    16 x 64  16 tiles 28.9 | 30.6    32 x 64  4 tiles 38.0 | 50.7
-bool fwd_merges_in_launch(int nsplit, int BQ, int D, int dtype) { return dtype == 2 && (int64_t)nsplit * BQ * D * 4 <= 256 * 1024; }
+// bf16, where one wave reads 32 rows of every part: up to four parts
+//   4 x 64  128 tiles of up to 256 chunks 136.0 | 132.8, 128 72.3 | 68.8, 64 45.3 | 42.0, 25 28.7 | 25.8; 64 tiles of 32 22.7 | 21.3, 32 tiles 20.6 | 18.7
+//   4 x 32  128 tiles, D = 64, of up to 256 79.3 | 76.8, BLOCK_Q 64 of up to 128 58.3 | 58.1    4 x 16  128 tiles of up to 128 45.9 | 41.5
+//   8 x 32  8 tiles of 64, D = 64 14.4 | 14.8, 64 tiles of up to 128 29.4 | 29.3, BLOCK_Q 64 36.8 | 38.2, 16 tiles of 64 21.0 | 21.9
+bool fwd_merges_in_launch(int nsplit, int BQ, int D, int dtype) {
+    return (int64_t)nsplit * BQ * D * 4 <= 256 * 1024 && (dtype == 2 || nsplit <= 4);
+}
 
 // When a list is walked in two halves by one workgroup of twice the waves (sparse_fwd_kernel<..., TW>): from half as many Q tiles
 // as compute units on, up to as many.  A compute unit has one workgroup then, which leaves half of its registers and LDS

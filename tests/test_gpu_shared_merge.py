@@ -58,6 +58,11 @@ def uneven(B, H, Sq, Sk, BQ, gpu):
     (torch.float32, 1, 2, 128, 1024, 64, 64, 256),    # entries of several chunks: a group without any
     (torch.float32, 1, 2, 128, 256, 128, 64, 32),
     (torch.float32, 2, 16, 512, 160, 128, 128, 32),   # one group of four waves
+    (torch.bfloat16, 4, 8, 512, 4096, 128, 128, 64),  # four parts of four waves
+    (torch.bfloat16, 1, 3, 256, 2048, 128, 128, 32),
+    (torch.float16, 3, 8, 256, 2560, 64, 64, 16),     # parts that do not divide the list
+    (torch.float16, 1, 2, 96, 2048, 64, 32, 64),      # one wave
+    (torch.bfloat16, 1, 2, 64, 2048, 128, 64, 1024),  # entries of several chunks, fewer than parts
 ])
 def test_the_last_workgroup_adds_up(gpu, dtype, B, H, Sq, Sk, D, BQ, BK):
     q, _, _ = W.qkv(B, H, Sq, D, dtype, seed=1, device=gpu)
@@ -87,7 +92,7 @@ def test_the_last_workgroup_adds_up(gpu, dtype, B, H, Sq, Sk, D, BQ, BK):
         assert float((lse.double() - want_lse)[live].abs().max()) <= (1e-5 if dtype == torch.float32 else 6e-3 + 2 ** -9 * 5)
 
 
-@pytest.mark.parametrize("dtype,B,H,Sq,Sk,D,BQ,BK", [(torch.float32, 1, 4, 256, 512, 64, 64, 32)])
+@pytest.mark.parametrize("dtype,B,H,Sq,Sk,D,BQ,BK", [(torch.float32, 1, 4, 256, 512, 64, 64, 32), (torch.bfloat16, 1, 8, 256, 2048, 128, 128, 64)])
 def test_replays_bring_the_same_launch_number(gpu, dtype, B, H, Sq, Sk, D, BQ, BK):
     q, _, _ = W.qkv(B, H, Sq, D, dtype, seed=1, device=gpu)
     _, k, v = W.qkv(B, H, Sk, D, dtype, seed=2, device=gpu)
