@@ -179,12 +179,6 @@ __device__ __forceinline__ void dma4_lane(const void *lane_addr, uint32_t lds_ad
 // What a lane whose 16 bytes do not exist fetches.
 __device__ const uint32_t kZeros[4] __attribute__((aligned(16))) = {0u, 0u, 0u, 0u};
 
-// A wave-uniform pointer that the compiler may have formed in vector registers.
-__device__ __forceinline__ const int32_t *scalar_pointer(const int32_t *p) {
-    const uint64_t b = (uint64_t)(uintptr_t)p;
-    return reinterpret_cast<const int32_t *>((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)b) |
-                                             ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(b >> 32)) << 32));
-}
 // N dwords from N wave-uniform addresses by scalar loads that are issued back to back and share ONE wait.  Left to
 // the compiler, loads whose addresses it forms one after the other are waited for one after the other as well, a
 // memory round trip each; at the start of a Q tile that is most of the time before the first K/V request.

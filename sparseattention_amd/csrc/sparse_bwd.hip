@@ -91,50 +91,6 @@ __device__ __forceinline__ BwdPlace bwd_place(const BwdParams &p, int lin, int t
     return {2 * pair + (paired ? (pr & 1) : 0), p.first_tile_first ? order : p.nR - 1 - order};
 }
 
-// The start of a tile: its list's slots, a FULL and a PARTIAL one per thread, travel with the counts and with the first slot of each
-// list, so that the first chunk is requested one memory round trip after the arguments, before the list has made its way to LDS.
-// Slots past a count hold anything and are not looked at.
-struct BwdList {
-    const int32_t *fid, *pid;
-    int64_t fs, ps;
-    int lane_full, lane_part, first, F, T;  // first: the tile that leads the list (0 .. nS - 1, also where there is none)
-    __device__ __forceinline__ void request(const BwdParams &p, int b, int h, int rt, int tid) {
-        fid = p.full_ids + b * p.fis[0] + h * p.fis[1] + rt * p.fis[2];
-        pid = p.part_ids + b * p.pis[0] + h * p.pis[1] + rt * p.pis[2];
-        fs = p.fis[3];
-        ps = p.pis[3];
-        const int slot = min(tid, p.nS - 1);
-        lane_full = fid[(int64_t)slot * fs];
-        lane_part = pid[(int64_t)slot * ps];
-    }
-    // Counts and tile indices are clamped to the nS streamed tiles there are (the reference guards every K/V and mask
-    // load with kv_offset < SEQLEN_K, sparse_attn_kernel.py:35,39,60): stale or foreign metadata then gives wrong
-    // numbers, never an access outside the tensors or past the list's LDS copy (nS <= kBwdListCap, checked by the host).
-    __device__ __forceinline__ void counts(const BwdParams &p, int b, int h, int rt) {
-        int got[4];
-        const int32_t *const addr[4] = {p.full_lens + (b * p.fls[0] + h * p.fls[1] + rt * p.fls[2]),
-                                        p.part_lens + (b * p.pls[0] + h * p.pls[1] + rt * p.pls[2]), scalar_pointer(fid), scalar_pointer(pid)};
-        scalar_gather(addr, got);
-        F = min(max(got[0], 0), p.nS);
-        T = F + min(max(got[1], 0), p.nS - F);
-        int f0 = got[2], p0 = got[3];
-        asm volatile("" : "+s"(f0), "+s"(p0));  // (no elements of an array any more: the select would become one load at a variable index)
-        first = min(max(F > 0 ? f0 : p0, 0), p.nS - 1);
-    }
-    // FULL entries, then PARTIAL ones, by 256 threads: those past the first 256 of a kind (before the first chunk is requested: the
-    // pointers are not needed any more then), and those that came with the counts
-    template <class E>
-    __device__ __forceinline__ void deposit(int nS, int tid, E &&put) const {
-        if (tid < F) put(tid, min(max(lane_full, 0), nS - 1));
-        if (tid < T - F) put(F + tid, min(max(lane_part, 0), nS - 1));
-    }
-    template <class E>
-    __device__ __forceinline__ void deposit_rest(int nS, int tid, E &&put) const {
-        for (int e = tid + 256; e < F; e += 256) put(e, min(max(fid[(int64_t)e * fs], 0), nS - 1));
-        for (int e = tid + 256; e < T - F; e += 256) put(F + e, min(max(pid[(int64_t)e * ps], 0), nS - 1));
-    }
-};
-
 // out = acc * scale; acc holds the transposed tile: lane (row l32, hh), register 4g + jj of block db is
 // d = 32 db + 8g + 4hh + jj.  A lane's 8-byte pieces would make every store instruction touch 32 rows, so the wave's 32
 // rows go through a private slice `ob` of the (now idle) chunk buffers, rows 16 bytes apart from the banks' period, and
@@ -193,8 +149,8 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
 
     const uint16_t *ybase = p.y + b * p.ys[0] + h * p.ys[1];
     const uint16_t *zbase = p.z + b * p.zs[0] + h * p.zs[1];
-    BwdList list;
-    list.request(p, b, h, rt, tid);
+    const int32_t *fid = p.full_ids + b * p.fis[0] + h * p.fis[1] + rt * p.fis[2];
+    const int32_t *pid = p.part_ids + b * p.pis[0] + h * p.pis[1] + rt * p.pis[2];
     const uint8_t *mrow = PK ? nullptr : p.mask + b * p.ms[0] + h * p.ms[1] + (int64_t)rrow * p.mrs;
     // packed tiles: 8 bytes per row, 1024 per tile, nS tiles per resident tile; a lane's four bytes of its wave's 32 rows
     const uint8_t *prow = PK ? p.packed + b * p.pks[0] + h * p.pks[1] + (int64_t)rt * p.nS * 1024 : nullptr;
@@ -203,13 +159,17 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
     // bytes from a query's L to its Delta (both live in one workspace, less than 4 GiB apart)
     const uint32_t stat_gap = (uint32_t)((const uint8_t *)p.stat_d - (const uint8_t *)p.stat_l);
 
-    // resident operands: lane (l32, hh) keeps d = 16c + 8hh .. +7 of its row; X carries the softmax scale / ln 2 (below, when the first
-    // chunk has been requested: scaled here they were waited for first)
+    // resident operands: lane (l32, hh) keeps d = 16c + 8hh .. +7 of its row; X carries the softmax scale / ln 2
     u32x4 xf[NC], gf[OUT_P ? 1 : NC];
     {
         const uint16_t *xp = p.x + b * p.xs[0] + h * p.xs[1] + (int64_t)rrow * p.xs[2] + 8 * hh;
 #pragma unroll
-        for (int c = 0; c < NC; c++) xf[c] = *(const u32x4 *)(xp + 16 * c);
+        for (int c = 0; c < NC; c++) {
+            xf[c] = *(const u32x4 *)(xp + 16 * c);
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if constexpr (!DS) xf[c][e] = E::scale2(xf[c][e], p.scale);
+        }
         if constexpr (!OUT_P) {
             const uint16_t *gp = p.g + b * p.gs[0] + h * p.gs[1] + (int64_t)rrow * p.gs[2] + 8 * hh;
 #pragma unroll
@@ -221,8 +181,15 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
         laneL = statL[(int64_t)rrow * p.sts[2]];
         laneD = statD[(int64_t)rrow * p.sts[2]];
     }
-    list.counts(p, b, h, rt);
-    const int F = list.F, T = list.T;  // chunks = list entries
+    // Counts and tile indices are clamped to the nS streamed tiles there are (the reference guards every K/V and mask
+    // load with kv_offset < SEQLEN_K, sparse_attn_kernel.py:35,39,60): stale or foreign metadata then gives wrong
+    // numbers, never an access outside the tensors or past the list's LDS copy (nS <= kBwdListCap, checked by the host).
+    int cnt[2];
+    const int32_t *const cnt_addr[2] = {p.full_lens + (b * p.fls[0] + h * p.fls[1] + rt * p.fls[2]),
+                                        p.part_lens + (b * p.pls[0] + h * p.pls[1] + rt * p.pls[2])};
+    scalar_gather(cnt_addr, cnt);
+    const int F = min(max(cnt[0], 0), p.nS);
+    const int T = F + min(max(cnt[1], 0), p.nS - F);  // chunks = list entries
     f32x16 acc[NDB], acc2[BOTH ? NDB : 1];  // acc2: dV beside dK
 #pragma unroll
     for (int db = 0; db < NDB; db++)
@@ -246,6 +213,13 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
     const uint32_t ld_yoff = (uint32_t)((ld_row * p.ys[2] + 8 * ld_piece) * 2);
     const uint32_t ld_zoff = (uint32_t)((ld_row * p.zs[2] + 8 * ld_piece) * 2);
 
+    // the tile's list (FULL entries, then PARTIAL ones) as first streamed rows
+    for (int e = tid; e < T; e += 256) {
+        const int idx = e < F ? fid[(int64_t)e * p.fis[3]] : pid[(int64_t)(e - F) * p.pis[3]];
+        ent[e] = min(max(idx, 0), p.nS - 1) << 6;
+    }
+    __syncthreads();
+
     // where this wave's keys' dS of the 64 queries from ent[t] goes: 4 KiB in a row
     const int64_t ds_row = (int64_t)p.nR * 2 * 16384;  // all keys of 128 queries
     uint8_t *const ds0 = DS ? p.ds + (int64_t)plane * (p.nS >> 1) * ds_row + (2 * rt + (wave_u >> 1)) * 16384 + (wave_u & 1) * 8192 : nullptr;
@@ -255,9 +229,10 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
     };
 
     // everything chunk t needs from memory, into stage st
-    auto issue_at = [&](int col, int t, int st, uint32_t(&mk)[NMW]) {
+    auto issue = [&](int t, int st, uint32_t(&mk)[NMW]) {
         int ln = lane;
         if constexpr (DS) asm volatile("" : "+v"(ln));
+        const int col = __builtin_amdgcn_readfirstlane(ent[t]);
 #pragma unroll
         for (int i = 0; i < NLD; i++) {
             const uint32_t dst = 1024 * (4 * i + wave_u);  // RPI rows per load
@@ -290,8 +265,6 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
             }
         }
     };
-
-    auto issue = [&](int t, int st, uint32_t(&mk)[NMW]) { issue_at(__builtin_amdgcn_readfirstlane(ent[t]), t, st, mk); };
 
     auto compute = [&](int t, int st, const uint32_t(&mk)[NMW]) {
         // Two accumulators of D = 128 leave no register over: the offsets are made anew from their bases per phase (kept,
@@ -424,25 +397,17 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
         for (int j = 0; j < NS; j++)
 #pragma unroll
             for (int i = 0; i < NMW; i++) mk[j][i] = 0u;
-        list.deposit_rest(p.nS, tid, [&](int e, int idx) { ent[e] = idx << 6; });
-        if (T > 0) issue_at(list.first << 6, 0, 0, mk[0]);
-        // the tile's list (FULL entries, then PARTIAL ones) as first streamed rows
-        list.deposit(p.nS, tid, [&](int e, int idx) { ent[e] = idx << 6; });
-        // The resident operands are waited for here: "used", they are no loads any more to the compiler, whose wait in front of
-        // their first use in the loop would take the direct loads of the chunks behind along, in every trip.
+        // The resident operands were requested before the list and have landed with it.  "Used" here, they are no loads any
+        // more to the compiler, whose wait in front of their first use in the loop would take the direct loads of the
+        // chunks behind along, in every trip.
 #pragma unroll
-        for (int c = 0; c < NC; c++) {
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                if constexpr (!DS) xf[c][e] = E::scale2(xf[c][e], p.scale);
-            asm volatile("" : "+v"(xf[c]));
-        }
+        for (int c = 0; c < NC; c++) asm volatile("" : "+v"(xf[c]));
         if constexpr (!OUT_P) {
 #pragma unroll
             for (int c = 0; c < NC; c++) asm volatile("" : "+v"(gf[c]));
         }
         if constexpr (LANE_STATS) asm volatile("" : "+v"(laneL), "+v"(laneD));
-        __syncthreads();  // the list in LDS is complete
+        if (T > 0) issue(0, 0, mk[0]);
         if constexpr (DS) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         for (int t0 = 0; t0 < T; t0 += NS) {
             static_for<NS>([&](auto jc) {
@@ -514,12 +479,16 @@ __device__ __forceinline__ void bwd_dq_tile(const BwdParams &p, int lin, int tot
     const int plane = p.planes - 1 - at.plane /* (last written first) */, rt = at.rt, bh = p.plane0 + plane;
     const int b = bh / p.H, h = bh - b * p.H;
     const uint16_t *ybase = p.y + b * p.ys[0] + h * p.ys[1];
-    BwdList list;
-    list.request(p, b, h, rt, tid);
+    const int32_t *fid = p.full_ids + b * p.fis[0] + h * p.fis[1] + rt * p.fis[2];
+    const int32_t *pid = p.part_ids + b * p.pis[0] + h * p.pis[1] + rt * p.pis[2];
     const uint8_t *prow = p.packed + b * p.pks[0] + h * p.pks[1] + (int64_t)rt * p.nS * 1024 + wave_u * 256;
     const uint8_t *dsbase = p.ds + ((int64_t)plane * p.nR + rt) * p.nS * 16384 + wave_u * 2048;
-    list.counts(p, b, h, rt);
-    const int F = list.F, T = list.T;
+    int cnt[2];  // (clamped as in bwd_tile)
+    const int32_t *const cnt_addr[2] = {p.full_lens + (b * p.fls[0] + h * p.fls[1] + rt * p.fls[2]),
+                                        p.part_lens + (b * p.pls[0] + h * p.pls[1] + rt * p.pls[2])};
+    scalar_gather(cnt_addr, cnt);
+    const int F = min(max(cnt[0], 0), p.nS);
+    const int T = F + min(max(cnt[1], 0), p.nS - F);
     f32x16 acc[NDB];
 #pragma unroll
     for (int db = 0; db < NDB; db++)
@@ -531,10 +500,15 @@ __device__ __forceinline__ void bwd_dq_tile(const BwdParams &p, int lin, int tot
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const SA_LDS uint8_t *)smem);
     const int ld_row = RPI * wave_u + lane / PPR, ld_piece = (lane % PPR) ^ bwd_swizzle<D>(ld_row);
     const uint32_t ld_yoff = (uint32_t)((ld_row * p.ys[2] + 8 * ld_piece) * 2);
+    for (int e = tid; e < T; e += 256) {
+        const int idx = e < F ? fid[(int64_t)e * p.fis[3]] : pid[(int64_t)(e - F) * p.pis[3]];
+        ent[e] = (uint16_t)min(max(idx, 0), p.nS - 1);
+    }
+    __syncthreads();
     // Steps of 32 keys, two per list entry.
     const int64_t ytile = 64 * p.ys[2], yhalf = 32 * p.ys[2], yload = 4 * RPI * p.ys[2];
-    auto issue_at = [&](int kt, int u, int st) {
-        const int t = u >> 1;
+    auto issue = [&](int u, int st) {
+        const int t = u >> 1, kt = __builtin_amdgcn_readfirstlane(ent[t]);
         const uint8_t *dsp = dsbase + (int64_t)kt * 16384 + (u & 1) * 8192;
         if (t >= F && (u & 1) == 0) dma4(prow + (int64_t)(t - F) * 1024, 4 * lane, lds0 + MASK0 + (t & 3) * 1024 + wave_u * 256);
 #pragma unroll
@@ -543,7 +517,6 @@ __device__ __forceinline__ void bwd_dq_tile(const BwdParams &p, int lin, int tot
 #pragma unroll
         for (int i = 0; i < SLD; i++) dma16(yp + i * yload, ld_yoff, lds0 + st * SBUF + 1024 * (4 * i + wave_u));
     };
-    auto issue = [&](int u, int st) { issue_at(__builtin_amdgcn_readfirstlane(ent[u >> 1]), u, st); };
     auto compute = [&](int u, int st) {
         const uint8_t *yb = smem + st * SBUF, *db_ = smem + DS0 + st * 8192 + wave_u * 2048 + dbase;
         u32x4 x[2];  // dS^T of keys 16kc ..
@@ -574,15 +547,8 @@ __device__ __forceinline__ void bwd_dq_tile(const BwdParams &p, int lin, int tot
             }
     };
     const int U = 2 * T;
-    list.deposit_rest(p.nS, tid, [&](int e, int idx) { ent[e] = (uint16_t)idx; });
-    if (U > 0) {  // (the two steps of the first entry)
-        issue_at(list.first, 0, 0);
-        issue_at(list.first, 1, 1);
-    }
-    list.deposit(p.nS, tid, [&](int e, int idx) { ent[e] = (uint16_t)idx; });
-    __syncthreads();  // the list in LDS is complete
 #pragma unroll
-    for (int u = 2; u < NST - 1; u++)
+    for (int u = 0; u < NST - 1; u++)
         if (u < U) issue(u, u);
     for (int u0 = 0; u0 < U; u0 += NST) {
         static_for<NST>([&](auto jc) {
