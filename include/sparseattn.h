@@ -530,6 +530,9 @@ size_t sa_bwd_workspace_bytes_ex(int B, int H, int Sq, int Sk, int D);
 /* The most bytes up to `limit` that a workspace between these two has a use for (never less than the first): fewer planes
  * of dS at a time, or none. */
 size_t sa_bwd_workspace_bytes_within(int B, int H, int Sq, int Sk, int D, size_t limit);
+/* Bytes behind the first of these sizes that a call without dS has a use for (0: for none): the order of its tiles by the lengths of
+ * their lists, longest first, for launches that would end with a few long lists that started late.  The same bits either way. */
+size_t sa_bwd_order_bytes(int B, int H, int Sq, int Sk, int D);
 int sa_sparse_attention_bwd(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
                             const void *v, const int64_t v_strides[4], const void *o, const int64_t o_strides[4],
                             const void *d_o, const int64_t do_strides[4], const float *lse,

@@ -60,6 +60,7 @@ EXPORTS = (
     "sa_bwd_workspace_bytes",
     "sa_bwd_workspace_bytes_ex",
     "sa_bwd_workspace_bytes_within",
+    "sa_bwd_order_bytes",
     "sa_sparse_attention_bwd",
     "sa_mask_terms_workspace_bytes",
     "sa_mask_classify_terms",
@@ -176,6 +177,8 @@ def load() -> ctypes.CDLL:
     lib.sa_bwd_workspace_bytes.argtypes = [ctypes.c_int] * 3
     lib.sa_bwd_workspace_bytes_ex.restype = ctypes.c_size_t
     lib.sa_bwd_workspace_bytes_ex.argtypes = [ctypes.c_int] * 5
+    lib.sa_bwd_order_bytes.restype = ctypes.c_size_t
+    lib.sa_bwd_order_bytes.argtypes = [ctypes.c_int] * 5
     lib.sa_bwd_workspace_bytes_within.restype = ctypes.c_size_t
     lib.sa_bwd_workspace_bytes_within.argtypes = [ctypes.c_int] * 5 + [ctypes.c_size_t]
     lib.sa_sparse_attention_bwd.restype = ctypes.c_int

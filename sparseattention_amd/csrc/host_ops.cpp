@@ -714,6 +714,7 @@ std::tuple<Tensor, Tensor, Tensor> backward_impl(const Tensor &do_, const Tensor
     size_t ws_bytes = sa_bwd_workspace_bytes(B, H, Sq);
     if (a.packed && b.packed && l.agree && sa_bwd_workspace_bytes_ex(B, H, Sq, Sk, Dk) > ws_bytes)
         ws_bytes = backward_workspace_bytes(B, H, Sq, Sk, Dk, device_room(q.device()));
+    if (ws_bytes == sa_bwd_workspace_bytes(B, H, Sq)) ws_bytes += sa_bwd_order_bytes(B, H, Sq, Sk, Dk);
     Tensor ws;
     try {
         ws = workspace(ws_bytes);

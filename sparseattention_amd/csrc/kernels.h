@@ -294,9 +294,27 @@ struct BwdParams {
 struct BwdLaunch {
     BwdParams pass[3];
     int first[3], tiles[3];
+    // null, or [8][slots]: workgroup 8 j + x has the j-th of XCD x's tiles by falling cost: pass << 24 | its place in the XCD's share
+    const int32_t *order;
+    int slots;
 };
+// How the tiles of a launch come by falling cost (bwd_prepare_kernel makes the order from the lists' lengths).
+struct BwdOrderParams {
+    int n;  // passes, or 0: no order
+    struct Pass {
+        const int32_t *full_lens, *part_lens;
+        int64_t fls[3], pls[3];
+        int nR, nS, planes, H, first_tile_first;
+        int fixed, per_entry;  // cost of a tile, and of an entry of its list
+    } pass[3];
+    int slots;
+    int32_t *order;
+};
+// The rule for it (sparse_bwd.hip): bytes of `order`, 0 where the tiles stay in the order of planes.
+size_t bwd_order_bytes(int B, int H, int Sq, int Sk, int D);
+BwdOrderParams bwd_order(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, int D, int32_t *order);
 // group > 0 (D = 128 and both packed buffers): dS of that many planes at a time goes through `ds`, and dQ is made from it.
-hipError_t launch_bwd(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, int dtype, int D, uint8_t *ds, int group, hipStream_t stream);
+hipError_t launch_bwd(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, int dtype, int D, uint8_t *ds, int group, const BwdOrderParams &order, hipStream_t stream);
 // The rule for group: sparse_bwd.hip.  bytes: what the workspace holds besides the statistics.
 int bwd_ds_group(int B, int H, int Sq, int Sk, int D, size_t bytes);
 // Bytes of dS that are worth their place, 0 where none are.
@@ -309,6 +327,7 @@ struct BwdPrepParams {
     float *stat_l, *stat_d;  // [B*H*Sq] each, contiguous
     float l_mul;             // stat_l = lse * l_mul: -1 / ln 2, or -1 / (ln 2 scale) where the kernel scales S - L
     int B, H, Sq;
+    BwdOrderParams order;
 };
 hipError_t launch_bwd_prepare(const BwdPrepParams &p, int dtype, int D, hipStream_t stream);
 

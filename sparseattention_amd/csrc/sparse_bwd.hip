@@ -76,9 +76,8 @@ struct BwdLds {
 struct BwdPlace {
     int plane, rt;
 };
-__device__ __forceinline__ BwdPlace bwd_place(const BwdParams &p, int lin, int total) {
-    const int per = total >> 3;
-    if (lin < (per << 3)) lin = (lin & 7) * per + (lin >> 3);
+template <class P>
+__device__ __forceinline__ BwdPlace bwd_place_in_order(const P &p, int lin) {  // lin: in the plane-major order
     int pair = lin / (2 * p.nR);
     const int pr = lin - pair * 2 * p.nR;
     if ((p.planes & 15) == 0) {  // every eighth pair of planes to an XCD: masks that differ per batch element load them alike
@@ -89,6 +88,10 @@ __device__ __forceinline__ BwdPlace bwd_place(const BwdParams &p, int lin, int t
     const bool paired = 2 * pair + 1 < p.planes;
     const int order = paired ? (pr >> 1) : pr;
     return {2 * pair + (paired ? (pr & 1) : 0), p.first_tile_first ? order : p.nR - 1 - order};
+}
+__device__ __forceinline__ BwdPlace bwd_place(const BwdParams &p, int lin, int total) {
+    const int per = total >> 3;
+    return bwd_place_in_order(p, lin < (per << 3) ? (lin & 7) * per + (lin >> 3) : lin);
 }
 
 // out = acc * scale; acc holds the transposed tile: lane (row l32, hh), register 4g + jj of block db is
@@ -576,24 +579,29 @@ __device__ __forceinline__ void bwd_dq_tile(const BwdParams &p, int lin, int tot
 // than workgroup slots would run one after the other (B2 H8 S1024: 128 tiles a pass on 512 slots).  The passes whose
 // tiles take longest come first; every pass starts at a multiple of eight workgroups, so that the plane-to-XCD mapping of
 // bwd_tile holds for each.
-template <int DT, int D, bool PK>
+// ORD: the tiles come by falling cost (l.order).
+template <int DT, int D, bool PK, bool ORD>
 __global__ __launch_bounds__(256, D == 64 && PK ? 3 : 2) void sparse_bwd_kernel(const BwdLaunch l) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     const int id = blockIdx.x;
-    if constexpr (D == 64) {
-        if (id < l.first[1]) {
-            if (id < l.tiles[0]) bwd_tile<DT, D, kDKV, PK, 0>(l.pass[0], id, l.tiles[0], smem);
-        } else {
-            bwd_tile<DT, D, kDQ, PK, 1>(l.pass[1], id - l.first[1], l.tiles[1], smem);
-        }
+    int pass = 0, lin = id;  // lin: workgroup of its pass, as bwd_place takes it
+    if constexpr (ORD) {
+        const int e = l.order[(id & 7) * l.slots + (id >> 3)];
+        pass = e >> 24;
+        lin = (e & 0xffffff) * 8 + (id & 7);
+    } else if (D != 64 && id >= l.first[2]) {
+        pass = 2;
+        lin = id - l.first[2];
+    } else if (id >= l.first[1]) {
+        pass = 1;
+        lin = id - l.first[1];
+    }
+    if (pass == 0) {
+        if (lin < l.tiles[0]) bwd_tile<DT, D, D == 64 ? kDKV : kDK, PK, 0>(l.pass[0], lin, l.tiles[0], smem);
+    } else if (D == 64 || pass == 1) {
+        if (lin < l.tiles[1]) bwd_tile<DT, D, kDQ, PK, 1>(l.pass[1], lin, l.tiles[1], smem);
     } else {
-        if (id < l.first[1]) {
-            if (id < l.tiles[0]) bwd_tile<DT, D, kDK, PK, 0>(l.pass[0], id, l.tiles[0], smem);
-        } else if (id < l.first[2]) {
-            if (id - l.first[1] < l.tiles[1]) bwd_tile<DT, D, kDQ, PK, 1>(l.pass[1], id - l.first[1], l.tiles[1], smem);
-        } else {
-            bwd_tile<DT, D, kDV, PK, 2>(l.pass[2], id - l.first[2], l.tiles[2], smem);
-        }
+        if constexpr (D != 64) bwd_tile<DT, D, kDV, PK, 2>(l.pass[2], lin, l.tiles[2], smem);
     }
 }
 
@@ -613,10 +621,84 @@ __global__ __launch_bounds__(256, 2) void sparse_bwd_queries_kernel(const BwdPar
 
 // Per query row: -Delta = -sum_d dO o O, and -L = -lse / ln 2 (-inf for rows that attended to nothing, so that their
 // P = exp2(S - L) is 0).  D/8 lanes per row, 8 elements each.
-template <int DT, int D>
+// In front of them, where the passes take their tiles by falling cost, eight workgroups sort one XCD's tiles each: a counting sort over
+// 32 classes of cost by eighths of the order of planes (whose neighbours share operands; within one in any order: each tile's result
+// is its own).
+constexpr int kCosts = 256, kOrderMost = 2048;
+__device__ __forceinline__ void bwd_sort_tiles(const BwdOrderParams &o, int xcd) {
+    __shared__ uint16_t cost[kOrderMost];
+    __shared__ int most, count[kCosts], of_wave[4], least_of[3], most_of[3];
+    const int tid = threadIdx.x;
+    if (tid == 0) most = 1;
+    if (tid < 3) {
+        least_of[tid] = 0x7fffffff;
+        most_of[tid] = 0;
+    }
+    count[tid] = 0;
+    __syncthreads();
+    auto which = [&](int i, int &pass, int &k) {  // slot i of the XCD before sorting
+        pass = 0;
+        k = i;
+        for (int n = 0; n + 1 < o.n && k >= (o.pass[n].planes * o.pass[n].nR >> 3); n++) {
+            k -= o.pass[n].planes * o.pass[n].nR >> 3;
+            pass = n + 1;
+        }
+    };
+    for (int i = tid; i < o.slots; i += 256) {
+        int pass, k;
+        which(i, pass, k);
+        const BwdOrderParams::Pass &q = o.pass[pass];
+        const BwdPlace at = bwd_place_in_order(q, xcd * (q.planes * q.nR >> 3) + k);
+        const int b = at.plane / q.H, h = at.plane - b * q.H;
+        const int F = min(max(q.full_lens[b * q.fls[0] + h * q.fls[1] + at.rt * q.fls[2]], 0), q.nS);
+        const int T = F + min(max(q.part_lens[b * q.pls[0] + h * q.pls[1] + at.rt * q.pls[2]], 0), q.nS - F);
+        const int c = min(q.fixed + q.per_entry * T, 0xffff);
+        cost[i] = (uint16_t)c;
+        atomicMax(&most, c);
+        atomicMin(&least_of[pass], c);
+        atomicMax(&most_of[pass], c);
+    }
+    __syncthreads();
+    bool alike = true;  // lists of about one length: the order of planes, whose neighbours share operands, is the better one
+    for (int n = 0; n < o.n; n++) alike = alike && 4 * (most_of[n] - least_of[n]) <= most_of[n];
+    if (alike) {
+        for (int i = tid; i < o.slots; i += 256) {
+            int pass, k;
+            which(i, pass, k);
+            o.order[xcd * o.slots + i] = pass << 24 | k;
+        }
+        return;
+    }
+    auto cls = [&](int i) { return 8 * (31 - (int)((unsigned)cost[i] * 31u / (unsigned)most)) + 8 * i / o.slots; };
+    for (int i = tid; i < o.slots; i += 256) atomicAdd(&count[cls(i)], 1);
+    __syncthreads();
+    const int mine = count[tid], lane = tid & 63;
+    int upto = mine;  // of the wave's classes up to this one
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) {
+        const int x = __shfl_up(upto, s);
+        if (lane >= s) upto += x;
+    }
+    if (lane == 63) of_wave[tid >> 6] = upto;
+    __syncthreads();
+    for (int w = 0; w < tid >> 6; w++) upto += of_wave[w];
+    count[tid] = upto - mine;
+    __syncthreads();
+    for (int i = tid; i < o.slots; i += 256) {
+        int pass, k;
+        which(i, pass, k);
+        o.order[xcd * o.slots + atomicAdd(&count[cls(i)], 1)] = pass << 24 | k;
+    }
+}
+template <int DT, int D, bool ORD>
 __global__ __launch_bounds__(256) void bwd_prepare_kernel(const BwdPrepParams p) {
     constexpr int LPR = D / 8;  // lanes per row
-    const int64_t row = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
+    int block = blockIdx.x;
+    if constexpr (ORD) {
+        if (block < 8) return bwd_sort_tiles(p.order, block);
+        block -= 8;
+    }
+    const int64_t row = (int64_t)block * (256 / LPR) + threadIdx.x / LPR;
     const int part = threadIdx.x % LPR;
     if (row >= (int64_t)p.B * p.H * p.Sq) return;
     const int q = (int)(row % p.Sq);
@@ -646,10 +728,10 @@ __global__ __launch_bounds__(256) void bwd_prepare_kernel(const BwdPrepParams p)
     }
 }
 
-template <int DT, int D, bool PK>
-hipError_t launch_bwd_one(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, hipStream_t stream) {
+template <int DT, int D, bool PK, bool ORD>
+hipError_t launch_bwd_one(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, const BwdOrderParams &ord, hipStream_t stream) {
     constexpr int smem = BwdLds<D, PK>::bytes;
-    auto kern = sparse_bwd_kernel<DT, D, PK>;
+    auto kern = sparse_bwd_kernel<DT, D, PK, ORD>;
     static unsigned long long attr_done = 0;
     if (const hipError_t e0 = allow_dynamic_smem(kern, smem, attr_done); e0 != hipSuccess) return e0;
     BwdLaunch l{};
@@ -666,7 +748,11 @@ hipError_t launch_bwd_one(const BwdParams &dq, const BwdParams &dk, const BwdPar
         l.pass[0].out2 = dv.out;
         for (int i = 0; i < 3; i++) l.pass[0].outs2[i] = dv.outs[i];
     }
-    hipLaunchKernelGGL(kern, dim3((unsigned)(l.first[n - 1] + l.tiles[n - 1])), dim3(256), smem, stream, l);
+    if constexpr (ORD) {
+        l.order = ord.order;
+        l.slots = ord.slots;
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned)(ORD ? 8 * l.slots : l.first[n - 1] + l.tiles[n - 1])), dim3(256), smem, stream, l);
     return hipGetLastError();
 }
 
@@ -706,7 +792,9 @@ template <int DT, int D>
 hipError_t launch_prepare_one(const BwdPrepParams &p, hipStream_t stream) {
     const int64_t rows = (int64_t)p.B * p.H * p.Sq;
     constexpr int RPB = 256 / (D / 8);  // rows per workgroup
-    hipLaunchKernelGGL((bwd_prepare_kernel<DT, D>), dim3((unsigned)((rows + RPB - 1) / RPB)), dim3(256), 0, stream, p);
+    const unsigned blocks = (unsigned)((rows + RPB - 1) / RPB);
+    if (p.order.n > 0) hipLaunchKernelGGL((bwd_prepare_kernel<DT, D, true>), dim3(8 + blocks), dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL((bwd_prepare_kernel<DT, D, false>), dim3(blocks), dim3(256), 0, stream, p);
     return hipGetLastError();
 }
 
@@ -738,7 +826,49 @@ size_t bwd_ds_bytes(int B, int H, int Sq, int Sk, int D) {
     return (size_t)Sq * Sk * 2 * bwd_ds_group(B, H, Sq, Sk, D, (size_t)4 << 30);
 }
 
-hipError_t launch_bwd(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, int dtype, int D, uint8_t *ds, int group, hipStream_t stream) {
+// Tiles by falling cost.  In the order of planes the last ones to start are as likely long as short: of 1536 tiles (B4 H12 S2048 D64, packed
+// documents) on 768 slots one of 15 entries started at 31 us and ended the launch at 60, where the work is 40 us of every slot.  More
+// workgroups than run at once by a quarter (three per compute unit at D = 64, else two), lists of eight entries or more (the sort
+// is 4 us beside the statistics, which take as long from there on), eighths of equal size, at most kOrderMost tiles a XCD, and planes of a
+// XCD that its L2 nearly holds (8 MiB), since the tiles at work are of all of them.  Backward with statistics, us, planes | cost:
+//   D = 64   documents B4 H12 S2048 71.3 | 63.9, B8 H12 S1024 67.9 | 58.1, B4 H17 S1024 51.3 | 46.4, B8 H24 S512 51.7 | 48.5   blocks p = 0.75 82 | 73.5
+//            causal B4 H12 S2048 124.6 | 112.2, B4 H17 S1024 60.2 | 53.4   every key 177.7 | 177.8   (S256 29.5 | 32.2: left as it is)
+//   D = 128  documents B4 H8 S1024 51.2 | 47.5, B1 H28 S1024 47.4 | 43.2 (B3 H8, 576 tiles 43.7 | 44.4: left as it is)
+//            causal B2 H8 S2048 91.9 | 87.4, B1 H32 S1024 57.2 | 55.6   every key B1 H28 S1024 79.0 | 80.4
+size_t bwd_order_bytes(int B, int H, int Sq, int Sk, int D) {
+    const int64_t planes = (int64_t)B * H, tq = planes * (Sq / 128), tk = planes * (Sk / 128), all = tq + tk * (D == 64 ? 1 : 2);
+    if (tq % 8 || tk % 8 || all <= (D == 64 ? 960 : 640) || all > 8 * kOrderMost || Sq < 512 || Sk < 512) return 0;
+    if ((planes + 7) / 8 * 2 * ((int64_t)Sq + Sk) * D * 2 > (8 << 20)) return 0;
+    return (size_t)all * 4;
+}
+BwdOrderParams bwd_order(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, int D, int32_t *order) {
+    BwdOrderParams o{};
+    const BwdParams *passes[3] = {&dk, &dq, &dv};  // (as launch_bwd_one has them)
+    o.n = D == 64 ? 2 : 3;
+    o.order = order;
+    for (int i = 0; i < o.n; i++) {
+        const BwdParams &p = *passes[i];
+        BwdOrderParams::Pass &q = o.pass[i];
+        q.full_lens = p.full_lens;
+        q.part_lens = p.part_lens;
+        for (int c = 0; c < 3; c++) {
+            q.fls[c] = p.fls[c];
+            q.pls[c] = p.pls[c];
+        }
+        q.nR = p.nR;
+        q.nS = p.nS;
+        q.planes = p.planes;
+        q.H = p.H;
+        q.first_tile_first = p.first_tile_first;
+        // (quarters of a microsecond: of the pass that makes dK and dV 2.5 an entry and 5 besides, of dQ 1.75 and 3.5; products 4 : 3 : 2)
+        q.per_entry = D == 64 ? (i == 0 ? 10 : 7) : (i == 2 ? 6 : 9);
+        q.fixed = 2 * q.per_entry;
+        o.slots += p.planes * p.nR / 8;
+    }
+    return o;
+}
+
+hipError_t launch_bwd(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, int dtype, int D, uint8_t *ds, int group, const BwdOrderParams &order, hipStream_t stream) {
     if (group > 0) {
         if (dtype == 0) return launch_bwd_ds<0>(dq, dk, dv, ds, group, stream);
         return launch_bwd_ds<1>(dq, dk, dv, ds, group, stream);
@@ -746,7 +876,8 @@ hipError_t launch_bwd(const BwdParams &dq, const BwdParams &dk, const BwdParams 
     const bool pk = dq.packed != nullptr && dk.packed != nullptr;  // (with only one of them the mask is there too)
 #define SA_BWD(DT, DD) \
     if (dtype == DT && D == DD) \
-        return pk ? launch_bwd_one<DT, DD, true>(dq, dk, dv, stream) : launch_bwd_one<DT, DD, false>(dq, dk, dv, stream)
+        return pk ? (order.n > 0 ? launch_bwd_one<DT, DD, true, true>(dq, dk, dv, order, stream) : launch_bwd_one<DT, DD, true, false>(dq, dk, dv, order, stream)) \
+                  : (order.n > 0 ? launch_bwd_one<DT, DD, false, true>(dq, dk, dv, order, stream) : launch_bwd_one<DT, DD, false, false>(dq, dk, dv, order, stream))
     SA_BWD(0, 128);
     SA_BWD(0, 64);
     SA_BWD(1, 128);

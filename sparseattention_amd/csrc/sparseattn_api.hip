@@ -1156,6 +1156,11 @@ size_t sa_bwd_workspace_bytes_ex(int B, int H, int Sq, int Sk, int D) {
     return ds ? ds_offset(stats) + ds : stats;
 }
 
+size_t sa_bwd_order_bytes(int B, int H, int Sq, int Sk, int D) {
+    if (B <= 0 || H <= 0 || Sq <= 0 || Sk <= 0 || Sq % 128 || Sk % 128 || (D != 64 && D != 128)) return 0;
+    return sa::bwd_order_bytes(B, H, Sq, Sk, D);
+}
+
 size_t sa_bwd_workspace_bytes_within(int B, int H, int Sq, int Sk, int D, size_t limit) {
     const size_t stats = sa_bwd_workspace_bytes(B, H, Sq), most = sa_bwd_workspace_bytes_ex(B, H, Sq, Sk, D);
     if (most <= limit || most == stats) return most;
@@ -1244,9 +1249,6 @@ int sa_sparse_attention_bwd(const void *q, const int64_t q_strides[4], const voi
     pp.B = B;
     pp.H = H;
     pp.Sq = Sq;
-    hipError_t e = sa::launch_bwd_prepare(pp, dtype, D, hs);
-    if (e != hipSuccess) return fail(SA_ERR_HIP, "sa_sparse_attention_bwd: launch failed: %s", hipGetErrorString(e));
-
     auto set3 = [](int64_t(&dst)[3], const int64_t *src) {
         for (int i = 0; i < 3; i++) dst[i] = src[i];
     };
@@ -1355,7 +1357,12 @@ int sa_sparse_attention_bwd(const void *q, const int64_t q_strides[4], const voi
     bp.out = static_cast<uint16_t *>(dv);
     set3(bp.outs, dv_strides);
     bp.out_scale = 1.f;
-    e = sa::launch_bwd(dq_pass, dk_pass, bp, dtype, D, ds, group, hs);
+    // where nothing else is behind the statistics, the order of the tiles may be
+    const size_t order_bytes = group > 0 ? 0 : sa_bwd_order_bytes(B, H, Sq, Sk, D);
+    if (order_bytes != 0 && workspace_bytes >= need + order_bytes)
+        pp.order = sa::bwd_order(dq_pass, dk_pass, bp, D, reinterpret_cast<int32_t *>(static_cast<uint8_t *>(workspace) + need));
+    hipError_t e = sa::launch_bwd_prepare(pp, dtype, D, hs);
+    if (e == hipSuccess) e = sa::launch_bwd(dq_pass, dk_pass, bp, dtype, D, ds, group, pp.order, hs);
     if (e != hipSuccess) return fail(SA_ERR_HIP, "sa_sparse_attention_bwd: launch failed: %s", hipGetErrorString(e));
     return SA_OK;
 }
