@@ -14,7 +14,7 @@
 //       one bit per entry of every PARTIAL tile, so that the forward reads BQ*BK/8 contiguous bytes per
 //       partial tile instead of BQ row segments of the mask (sparse_attn_kernel.py:42-46).
 //   classify_rows_kernel
-//       all three in one launch, for masks of few bytes per Q tile.
+//       all three in one launch, for masks of few bytes per Q tile and for large ones of many Q tiles.
 //
 // A byte != 0 counts as "attend", so masks that were viewed from uint8 storage behave like torch.sum.
 #include <hip/hip_runtime.h>
@@ -193,16 +193,21 @@ __global__ __launch_bounds__(256) void pack_partial_kernel(const PackParams p) {
     }
 }
 
-// The three steps above in one launch for masks of few bytes per Q tile, where each is a launch's latency: grid (nQ,
-// distinct planes), a workgroup of eight waves makes everything of one Q tile and the tiles' states stay in LDS.
+// The three steps above in one launch, a launch's latency each for masks of few bytes per Q tile: grid (nQ, distinct planes),
+// a workgroup of eight waves makes everything of one Q tile and the tiles' states stay in LDS.
 //   rows     16 bytes per lane and row, as classify_wide_kernel; column blocks of 64 lanes are dealt to the waves, and where
 //            there are fewer than eight of them the rows of one are shared by several waves.  Rows of 16, 32 .. 512 bytes
 //            go several to a wave instruction.
 //   lists    wave 0 writes the FULL list, wave 1 the PARTIAL one, wave 2 + 3 the next output plane's ...
 //   packing  16 mask bytes, just read and in L2, become 16 bits per thread and step.
-constexpr int kRowsThreads = 512, kRowsWaves = kRowsThreads / 64;
-constexpr int kRowsTiles = 2048;  // KV tiles of a Q tile that LDS holds
-__global__ __launch_bounds__(kRowsThreads) void classify_rows_kernel(const ClassifyRowsParams a) {
+// SLAB is the form for slabs of megabytes, bound by HBM: sixteen waves, each with two column blocks side by side and eight rows of
+// both in flight, so that a workgroup has up to 256 KiB requested and reads its slab from front to back, by streaming loads.  1 GiB
+// of a window's mask with lists and packed tiles 190 -> 166 us (6.5 TB/s), all PARTIAL 816 -> 434 us: its bits come out of the L2s.
+constexpr int kRowsTiles = 2048;           // KV tiles of a Q tile that LDS holds
+constexpr int64_t kSmallSlab = 512 * 1024;  // mask bytes of a Q tile past which it is the SLAB form
+template <bool SLAB>
+__global__ __launch_bounds__(SLAB ? 1024 : 512) void classify_rows_kernel(const ClassifyRowsParams a) {
+    constexpr int kRowsThreads = SLAB ? 1024 : 512, kRowsWaves = kRowsThreads / 64;
     __shared__ unsigned state[kRowsTiles];  // bit 0: some entry attends, bit 1: some entry does not
     __shared__ uint16_t part[kRowsTiles];   // the PARTIAL tiles, in order
     __shared__ int sh_np;
@@ -214,7 +219,41 @@ __global__ __launch_bounds__(kRowsThreads) void classify_rows_kernel(const Class
     const uint8_t *rows = p.mask + (int64_t)ub * p.sb + (int64_t)uh * p.sh + (int64_t)qt * p.BQ * p.sq;
     for (int i = tid; i < p.nK; i += kRowsThreads) state[i] = 0u;
     __syncthreads();
-    {
+    if constexpr (SLAB) {
+        const int pieces = p.Sk >> 4, blocks = (pieces + 63) >> 6;
+        for (int cb = wave; cb < blocks; cb += 2 * kRowsWaves) {
+            // (a lane without a piece of its own, or a wave without a second block, reads the row's last one again)
+            const int piece[2] = {cb * 64 + lane, (cb + kRowsWaves) * 64 + lane};
+            const uint8_t *const base[2] = {rows + 16 * min(piece[0], pieces - 1), rows + 16 * min(piece[1], pieces - 1)};
+            uint32_t any[2] = {0u, 0u}, all[2] = {0x80808080u, 0x80808080u};
+            const bool two = cb + kRowsWaves < blocks;
+            auto fold = [&](int i, const u32x4 &v) {
+                any[i] |= v.x | v.y | v.z | v.w;
+                all[i] &= nonzero_bytes(v.x) & nonzero_bytes(v.y) & nonzero_bytes(v.z) & nonzero_bytes(v.w);
+            };
+            int r = 0;
+            for (; r + kRowUnroll <= p.BQ; r += kRowUnroll) {
+                u32x4 v[2][kRowUnroll];
+#pragma unroll
+                for (int u = 0; u < kRowUnroll; u++) {
+                    v[0][u] = __builtin_nontemporal_load((const u32x4 *)(base[0] + (int64_t)(r + u) * p.sq));
+                    if (two) v[1][u] = __builtin_nontemporal_load((const u32x4 *)(base[1] + (int64_t)(r + u) * p.sq));
+                }
+#pragma unroll
+                for (int u = 0; u < kRowUnroll; u++) {
+                    fold(0, v[0][u]);
+                    if (two) fold(1, v[1][u]);
+                }
+            }
+            for (; r < p.BQ; r++) {
+                fold(0, __builtin_nontemporal_load((const u32x4 *)(base[0] + (int64_t)r * p.sq)));
+                if (two) fold(1, __builtin_nontemporal_load((const u32x4 *)(base[1] + (int64_t)r * p.sq)));
+            }
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                if (piece[i] < pieces) atomicOr(&state[(16 * piece[i]) >> p.lbk], (any[i] != 0u ? 1u : 0u) | (all[i] != 0x80808080u ? 2u : 0u));
+        }
+    } else {
         const int pieces = p.Sk >> 4;  // 16-byte pieces of a row
         const int per_row = pieces < 64 && (pieces & (pieces - 1)) == 0 ? pieces : 64;
         const int rpi = 64 / per_row, sub = lane / per_row;  // rows of one wave instruction, and this lane's
@@ -333,13 +372,23 @@ hipError_t launch_pack(const PackParams &p, hipStream_t stream) {
 //   512 KiB x 128 (causal S8192)                     19.0 | 13.5   512 KiB x 256, all PARTIAL 97 | 51
 //   256 KiB x 64, all PARTIAL                        17.7 | 15.9   256 KiB x 512, all PARTIAL 76 | 42
 // and beyond the rule 256 KiB x 16 causal 9.8 | 6.9 but all PARTIAL 12.5 | 15.6, 2 MiB x 4 10.3 | 23.5.
+// Larger slabs (the SLAB form; a call at a time, with its allocations) need 128 workgroups, half of the chip's CUs:
+//   1 MiB x 128 (S8192, causal)     34.5 | 27    all PARTIAL 82 | 72     x 192 46.3 | 31.5    x 512 107.6 | 81
+//   2 MiB x 128 (S16384, causal)    66.6 | 49    all PARTIAL 174 | 143   4 MiB x 256 (S32768, window) 190 | 166, all PARTIAL 816 | 434
+//   8 MiB x 128 (256 x 1024 tiles)   333 | 199
+// and lose below: 1 MiB x 64 21.0 | 23.1, x 86 28.5 | 34.6, 4 MiB x 32 34 | 79, x 64 59 | 85.  A wave takes 1024 columns, so the rows
+// must be long enough for at least half of the sixteen waves.
 bool classify_rows_has(const ClassifyParams &p) {
     const int64_t slab = (int64_t)p.BQ * p.Sk, workgroups = (int64_t)p.nQ * p.uB * p.uH;
-    return p.nK <= kRowsTiles && slab <= 512 * 1024 && (slab <= 128 * 1024 || slab <= workgroups * 8192);
+    if (p.nK > kRowsTiles) return false;
+    if (slab <= kSmallSlab) return slab <= 128 * 1024 || slab <= workgroups * 8192;
+    return workgroups >= 128 && p.Sk >= 8 * kWideCols && slab <= INT32_MAX;
 }
 
 hipError_t launch_classify_rows(const ClassifyRowsParams &p, hipStream_t stream) {
-    hipLaunchKernelGGL(classify_rows_kernel, dim3(p.c.nQ, p.c.uB * p.c.uH), dim3(kRowsThreads), 0, stream, p);
+    const dim3 grid(p.c.nQ, p.c.uB * p.c.uH);
+    if ((int64_t)p.c.BQ * p.c.Sk > kSmallSlab) hipLaunchKernelGGL(classify_rows_kernel<true>, grid, dim3(1024), 0, stream, p);
+    else hipLaunchKernelGGL(classify_rows_kernel<false>, grid, dim3(512), 0, stream, p);
     return hipGetLastError();
 }
 
