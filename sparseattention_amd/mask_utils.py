@@ -355,9 +355,10 @@ def _check_docs(doc, B, S, name):
         return None
     if doc.dim() == 1:
         doc = doc[None]
-    if doc.dim() != 2 or doc.shape[-1] != S or doc.shape[0] not in (1, B) or doc.dtype != torch.int32:
-        raise ValueError(f"{name}: expected int32 [{B},{S}] or [{S}], got {doc.dtype} {tuple(doc.shape)}")
-    return doc.expand(B, S)
+    shape = doc.shape
+    if len(shape) != 2 or shape[1] != S or shape[0] not in (1, B) or doc.dtype != torch.int32:
+        raise ValueError(f"{name}: expected int32 [{B},{S}] or [{S}], got {doc.dtype} {tuple(shape)}")
+    return doc if shape[0] == B else doc.expand(B, S)
 
 
 def materialize_mask_terms(terms: Sequence[MaskTerm], B: int, Sq: int, Sk: int, doc_q=None, doc_k=None, device=None):
