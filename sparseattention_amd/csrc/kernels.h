@@ -147,16 +147,17 @@ struct FwdParams {
     //   ws_ml [B*H*nQ][nsplit][BQ][2] floats: reference value (-inf: no attended key) and sum of every row
     int nsplit, split_chunks;  // split_chunks: chunks of one part (the last ones may be shorter)
     int split_least;           // lists of up to this many chunks are not shared
-    float *ws, *ws_ml;
-    // [B*H*nQ][nsplit] words by which the last workgroup of a shared list to arrive knows that it is the one to add the parts up
-    // (all_arrived), or null: then a second launch does (launch_fwd_merge).  tag: the launch's number.
-    uint64_t *arrivals;
-    uint64_t tag;
     int halves;                // 1: every list in two halves by the waves of one workgroup (fwd_in_halves)
+    float *ws, *ws_ml;
     // Ragged sizes: the tile grid (Sq, Sk, nQ, nK, lists, packed tiles) is that of a padded mask, the tensors have Sq_in
     // and Sk_in rows, which stand q0 and k0 rows into the grid, of D_in elements (a multiple of 8, at most the kernel's D).
     int ragged;
     int q0, k0, Sq_in, Sk_in, D_in;
+    // The launch's number where the last workgroup of a shared list to arrive adds the parts up (all_arrived), or 0: then a second
+    // launch does (launch_fwd_merge).  The words it knows that by, [B*H*nQ][nsplit], lie behind ws_ml.  (The arguments stay within
+    // 512 bytes with the grid's size behind them: 16 more, and one more miss at the start made a launch of 22.5 us 0.3 us longer.)
+    uint64_t tag;
+    __host__ __device__ uint64_t *arrivals(int BQ) const { return reinterpret_cast<uint64_t *>(ws_ml + (int64_t)B * H * nQ * nsplit * BQ * 2); }
 };
 
 // How many workgroups share a list of NE entries of 2^lbk keys, walked in chunks of 2^lck keys, and the first entry of

@@ -25,7 +25,7 @@ hipError_t by_hand_out(const FwdParams &p, int D, int BQ, hipStream_t stream) {
     if (p.halves) return launch_fwd_variant<DT, PK, 4>(p, D, BQ, stream);
     if (p.nsplit <= 1) return launch_fwd_variant<DT, PK, 0>(p, D, BQ, stream);
     const hipError_t e = launch_fwd_variant<DT, PK, 2>(p, D, BQ, stream);
-    return e != hipSuccess || p.arrivals != nullptr ? e : launch_fwd_merge(p, DT, D, BQ, stream);
+    return e != hipSuccess || p.tag != 0 ? e : launch_fwd_merge(p, DT, D, BQ, stream);
 }
 }  // namespace
 

@@ -426,11 +426,11 @@ __global__ __launch_bounds__(NW * f32_groups(NW, SP) * 64, D == 128 && NW * f32_
                 for (int g = 0; g < 4; g++)
                     rows.put(s0 * rows_step + rows_at + 1024 * (4 * d + g), f32x4{o[d][4 * g], o[d][4 * g + 1], o[d][4 * g + 2], o[d][4 * g + 3]});
             if (G == 0 && hh == 0) state.put(s0 * state_step + state_at, f32x2{m_i, l_tot});
-            if (p.arrivals == nullptr) return;
+            if (p.tag == 0) return;
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();  // every wave's rows have been handed over, and LDS has been read
             if (threadIdx.x < 64) {
-                const bool all = all_arrived(p.arrivals + first, p.tag, s0, share);
+                const bool all = all_arrived(p.arrivals(NW * 32) + first, p.tag, s0, share);
                 if (threadIdx.x == 0) *reinterpret_cast<int *>(smem0) = all;
             }
             __syncthreads();
@@ -507,7 +507,7 @@ hipError_t launch_fwd_f32_mfma(const FwdParams &p, int D, int BQ, hipStream_t st
     if (!fwd_f32_mfma_has(p, D, BQ)) return hipErrorInvalidValue;
     const hipError_t e = p.packed != nullptr ? (D == 64 ? launch_bq<64, true>(p, BQ, stream) : launch_bq<128, true>(p, BQ, stream))
                                              : (D == 64 ? launch_bq<64, false>(p, BQ, stream) : launch_bq<128, false>(p, BQ, stream));
-    return e != hipSuccess || p.nsplit <= 1 || p.arrivals != nullptr ? e : launch_fwd_merge(p, 2, D, BQ, stream);
+    return e != hipSuccess || p.nsplit <= 1 || p.tag != 0 ? e : launch_fwd_merge(p, 2, D, BQ, stream);
 }
 
 }  // namespace sa

@@ -1292,12 +1292,12 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
                              f32x4{acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]});
             if (hh == 0)
                 state.put(share_part * state_step + state_at, f32x2{raise_above == kMaxSlack ? m_ref : kNegInf, l32 < 16 ? acc_l[0] : acc_l[1]});
-            if (p.arrivals == nullptr) return;
+            if (p.tag == 0) return;
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();  // every wave's rows have been handed over
             int *const last = reinterpret_cast<int *>(smem);  // (a stage nobody reads any more)
             if (tid < 64) {
-                const bool all = all_arrived(p.arrivals + first, p.tag, share_part, share);
+                const bool all = all_arrived(p.arrivals(NW * 32) + first, p.tag, share_part, share);
                 if (tid == 0) *last = all;
             }
             __syncthreads();

@@ -446,10 +446,8 @@ int forward_impl(const void *q, const int64_t q_strides[4], const void *k, const
         fp.ws = static_cast<float *>(workspace);
         fp.ws_ml = fp.ws + (need / 4 / (size_t)(D + 2)) * (size_t)D;
         // (a caller who asked an earlier library for the size has no place for them: a second launch then)
-        if (need != 0 && sa::fwd_merges_in_launch(plan.nsplit, BQ, D, dtype) && workspace_bytes >= need + (size_t)8 * B * H * fp.nQ * plan.nsplit) {
-            fp.arrivals = reinterpret_cast<uint64_t *>(static_cast<uint8_t *>(workspace) + need);
-            fp.tag = next_launch_tag();
-        }
+        if (need != 0 && sa::fwd_merges_in_launch(plan.nsplit, BQ, D, dtype) && workspace_bytes >= need + (size_t)8 * B * H * fp.nQ * plan.nsplit)
+            fp.tag = next_launch_tag() | 1;  // (never 0)
     }
     if (kernel == SA_FWD_KERNEL_SHORT_LISTS) {
         if (f32 || !sa::fwd_c32_has(fp, dtype, D, BQ))
