@@ -48,18 +48,18 @@ PEAK_FP32_TFLOPS = 157.3   # MI355X dense fp32 MFMA peak, TFLOP/s
 # `bench.py --traffic-probe` and scaled by what the same counters read for the 1 GiB device copy of the same run
 # (`bench.py --traffic-summary` does the arithmetic).  profiles/hbm_traffic_all_kernels.txt holds the commands.
 TRAFFIC_BYTES = {
-    "forward, causal": (851555764, 268435456),
-    "forward, dense": (807997466, 268436224),
-    "forward, p=0.25": (1353367819, 268435456),
-    "forward, p=0.5": (2861066972, 268435456),
-    "forward, p=0.75": (2939201279, 268435456),
-    "forward, p=0.9": (1418611315, 268435456),
-    "backward, causal": (6764364779, 5242880128),
-    "forward, documents": (1725892383, 536870912),
-    "forward, composed": (1617152625, 268435456),
-    "mask_classify, composed mask 1 GiB": (1073825790, 58880),
-    "decode, 1": (4295549641, 397312),
-    "decode, 16": (1617185562, 5677056),
+    "forward, causal": (851685571, 268435456),
+    "forward, dense": (807998895, 268435456),
+    "forward, p=0.25": (1375509304, 268435456),
+    "forward, p=0.5": (2870573991, 268435456),
+    "forward, p=0.75": (2943998167, 268435456),
+    "forward, p=0.9": (1415445150, 268435456),
+    "backward, causal": (6760299478, 5242880171),
+    "forward, documents": (1726078013, 536870912),
+    "forward, composed": (1618993437, 268435456),
+    "mask_classify, composed mask 1 GiB": (1073825705, 58880),
+    "decode, 1": (4295549086, 397312),
+    "decode, 16": (1617185349, 5677056),
 }
 TRAFFIC_SOURCE = "profiles/hbm_traffic_all_kernels.txt"
 # The sources each kernel is built from.  The counters were read with kernels built from sources of the digests in
@@ -71,7 +71,7 @@ KERNEL_FILES = {
     "decode": ("sparse_decode.hip", "fwd_common.h", "kernels.h"),
     "backward": ("sparse_bwd.hip", "fwd_common.h", "kernels.h"),
 }
-TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "b60bd59c36e4ffe1", "mask_classify": "ecc32103cd758d6a", "decode": "1a84164e00e548fe",
+TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "db3a0a081cbbd2ae", "mask_classify": "ecc32103cd758d6a", "decode": "1a84164e00e548fe",
                                 "backward": "47c8255cb462b3db"}
 
 

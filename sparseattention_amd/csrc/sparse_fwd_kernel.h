@@ -71,21 +71,27 @@ __device__ __forceinline__ void wait_vm_at_most(int n, int step) {
 // fill the device: a chunk of a prompt against a long cache.  Every workgroup walks a range of its own and leaves
 // unnormalised rows with their reference values and sums in p.ws; the last of a few (fwd_merges_in_launch) to arrive adds them up, else
 // fwd_merge_kernel does.  A tile whose list is too short to be shared is written as by the plain kernel.
-// RG: the tile grid is larger than the tensors (p.q0, p.k0: rows of it in front of the first query and key; p.Sq_in, p.Sk_in:
+// RG (RGD 1 or 2): the tile grid is larger than the tensors (p.q0, p.k0: rows of it in front of the first query and key; p.Sq_in, p.Sk_in:
 // rows there are) and the head dim may be smaller than D (p.D_in, a multiple of 8).  Nothing is padded in memory: queries
 // and pieces of rows that do not exist enter as zeros (pieces from a zero in device memory, since a direct load brings
 // every lane 16 bytes), keys before the first and behind the last one as that one, which the mask of their tile leaves
 // out, and what has no place in the output is not stored.  The address of a direct load is formed per lane then, some six
 // instructions each.  B2 H16 S1499 D80 against padding q, k, v and cutting the result (14 launches): 82 -> 22 us.
+// RGD 2: D = 128 of which at most 96 elements exist: a quarter of both products, and of the operand reads from LDS, is left out (the same bits:
+// what it added was 0).  S1499 D80 documents B2 H16 20.7 -> 19.6 us, causal 38.4 -> 34.9, B4 H16 S2999 161 -> 144.  (Half of them, D <= 64, is the
+// kernel of D = 64; an eighth would be two of sixteen MFMAs of one product alone.)
 // TW: the list of a Q tile is walked in two halves by two times NW waves of one workgroup, for launches of no more Q tiles than
 // compute units (fwd_in_halves, with times): the second half takes the registers and the LDS that a second workgroup would.  Each
 // half has its own stages and its own copy of its part of the list; the second one leaves its rows in LDS, the first one adds
 // them up.  Two waves per SIMD are bound by the matrix pipe (1.8 us for a chunk of each, at D = 128), a lone one by its own
 // serial phases (0.95 us a chunk), so what halves gain is the shorter tail of an uneven launch and, at BLOCK_Q = 64, the idle SIMDs.
-template <int DT, int D, int NW, int MODE, int NS, bool PP, bool PK, bool PS, bool SP, bool RG, bool TW>
+template <int DT, int D, int NW, int MODE, int NS, bool PP, bool PK, bool PS, bool SP, int RGD, bool TW>
 __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 : 1) void sparse_fwd_kernel(const FwdParams p) {
     static_assert(!PS || (!PP && NS == 2), "persistent workgroups use the two-stage loop");
     static_assert(!SP || (!PS && !PP && D <= 128), "shared lists use the plain loop");
+    constexpr bool RG = RGD != 0;
+    constexpr int DE = RGD == 2 ? 96 : D;  // elements of a row that take part
+    static_assert(RGD != 2 || D == 128, "three quarters of the larger head dim");
     static_assert(!RG || (PK && !SP && !PS && !PP && D <= 128), "ragged sizes use the plain loop and packed tiles");
     static_assert(!TW || (!SP && !PS && !PP && !RG && NS == 2 && D <= 128), "two halves use the plain loop");
     using E = Elem<DT>;
@@ -737,7 +743,7 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
 
         // S^T = K . Q^T in bundles of two MFMAs (the two key blocks of d step c), operand reads kPfS bundles
         // ahead.  Within a bundle the MFMA that uses the younger read goes first, so one wait covers both.
-        constexpr int NC = D / 16;
+        constexpr int NC = DE / 16;
         constexpr int kPfS = 3;
         u32x4 kf0[NC], kf1[NC];
         auto k_read = [&](int c) {
@@ -837,6 +843,7 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
 #pragma unroll
             for (int u = 0; u < 2; u++) {
                 const int kc = b / BPK, db = 2 * (b % BPK) + u;
+                if (32 * db >= DE) continue;
                 const uint8_t *vp = vb_ + 16 * kc * ROWB + voff[db];
                 vlo[2 * b + u] = E::tr_read(vp);
                 vhi[2 * b + u] = E::tr_read(vp + 8 * ROWB);
@@ -855,6 +862,7 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
 #pragma unroll
             for (int u = 1; u >= 0; u--) {
                 const int db = 2 * (b % BPK) + u, i = 2 * b + u;
+                if (32 * db >= DE) continue;  // (those accumulators stay 0 and are not stored)
                 acc[db] = E::mfma(u32x4{vlo[i].x, vlo[i].y, vhi[i].x, vhi[i].y}, pk4, acc[db]);
             }
             if (b % BPK == BPK - 1) acc_l = E::mfma16(sum_sel, pk4, acc_l);
@@ -1343,22 +1351,30 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
     store_o_rows();
 }
 
-// HOW 0: one workgroup per Q tile, 1: persistent workgroups, 2: lists shared by workgroups (SP), 3: ragged sizes (RG),
+// HOW 0: one workgroup per Q tile, 1: persistent workgroups, 2: lists shared by workgroups (SP), 3: ragged sizes (RG; its form by the head dim),
 // 4: lists walked in two halves (TW)
-template <int DT, int D, int NW, int MODE, bool PK, int HOW>
-hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
+template <int DT, int D, int NW, int MODE, bool PK, int HOW, int RGD>
+hipError_t launch_form(const FwdParams &p, hipStream_t stream) {
     // Eight waves fill a CU's register file on their own, so that workgroup can have most of the LDS: 4 stages.
     constexpr int NS = NW == 8 ? 4 : 2;
     static_assert(kListCap == 2 * kPsListCap, "one long list or two short ones in the same LDS");
     constexpr int HALVES = HOW == 4 ? 2 : 1;
     constexpr int smem = HALVES * (2 * NS * 64 * D * 2 + kListCap * 4 + (HOW == 4 ? kHalvesSync : 0));  // NS stages of 64 rows for K and for V + the list(s)
-    auto kern = sparse_fwd_kernel<DT, D, NW, MODE, NS, NW == 8, PK, HOW == 1, HOW == 2, HOW == 3, HOW == 4>;
+    auto kern = sparse_fwd_kernel<DT, D, NW, MODE, NS, NW == 8, PK, HOW == 1, HOW == 2, RGD, HOW == 4>;
     static unsigned long long attr_done = 0;  // devices on which this kernel may use `smem` bytes of LDS
     if (const hipError_t e0 = allow_dynamic_smem(kern, smem, attr_done); e0 != hipSuccess) return e0;
     const unsigned grid = HOW == 1 ? (unsigned)p.sched_G
                                    : (unsigned)p.nQ * (unsigned)p.B * (unsigned)p.H * (HOW == 2 ? (unsigned)p.nsplit : 1u);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(HALVES * NW * 64), smem, stream, p);
     return hipGetLastError();
+}
+
+template <int DT, int D, int NW, int MODE, bool PK, int HOW>
+hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
+    if constexpr (HOW == 3 && D == 128) {  // (D_in 112: 38.9 us, as before; 96 and less: 34.9 against 38.3)
+        if (p.D_in <= 96) return launch_form<DT, D, NW, MODE, PK, HOW, 2>(p, stream);
+    }
+    return launch_form<DT, D, NW, MODE, PK, HOW, HOW == 3 ? 1 : 0>(p, stream);
 }
 
 template <int DT, int D, int NW, bool PK, int HOW>
