@@ -136,7 +136,8 @@ int sa_mask_classify_static(const uint8_t *mask, const int64_t mask_strides[4], 
  *   q,o  [B,H,Sq,D]; k,v [B,H,Sk,D]; dtype selects bf16 or fp16 for all four.  The last
  *   dimension must be contiguous (stride 1), every other stride a multiple of 8 elements and
  *   the base pointers 16-byte aligned; otherwise SA_ERR_UNSUPPORTED (copy to a contiguous tensor).
- *   mask and the four metadata tensors are as in sa_mask_classify; only ids[..., :len] are read.
+ *   mask and the four metadata tensors are as in sa_mask_classify; only ids[..., :len] take part.  float32 reads nothing
+ *   else of ids; bf16 and fp16 may also read, without looking at them, up to four slots past a count, of the Sk/BK of the row.
  *   sm_scale_log2 = softmax scale divided by ln 2 (the reference uses D^-0.5 / ln 2,
  *   sparse_attn_kernel.py:152); scores are exponentiated with exp2.
  *

@@ -41,10 +41,10 @@ constexpr int f32_group_bytes = 4 * 32 * D * 4 + 2 * NW * 1024 + kF32ListCap * 4
 // SP: lists shared by up to p.nsplit workgroups (fwd_split_share).
 // KG: groups of NW waves that share out a list, each with stages of its own, in step; their rows meet in LDS.  Two where lists are
 // shared and NW <= 2 would leave two of the four SIMDs idle.
-// A small launch is a chain: B1 H4 S512 D64 with half of the 32 x 32 blocks (32 Q tiles, about 9 chunks each, parts of two) takes 10.9 us a
-// pass, where two waves per part, reads of the list behind the counts and a second launch for the merge took 16.0.  Time stamps: queries,
-// counts and lists 1.2 us, first K and V at 2.3, products and softmax 3.0, the groups' rows 0.4, parts handed over 0.7, all arrived 0.8,
-// parts read and added 2.1.
+// A small launch is a chain: B1 H4 S512 D64 with half of the 32 x 32 blocks (32 Q tiles, about 9 chunks each, parts of two) takes 11.1 us a
+// pass, where two waves per part, lists by way of LDS and a second launch for the merge took 15.7.  Time stamps with both lists read whole
+// beside the counts (11.2 us; callers' rows may end with the list): queries, counts and lists 1.2 us, first K and V at 2.3, products and
+// softmax 3.0, the groups' rows 0.4, parts handed over 0.7, all arrived 0.8, parts read and added 2.1.
 // Registers for two waves per SIMD (D = 64: results stay out of the accumulation registers; causal B2 H16 S2048 235 -> 226 us), but not at
 // D = 128 with two waves a workgroup: registers that fill a SIMD keep the waves of two workgroups on different ones (339 us against 592).
 template <int D, int NW, int MODE, bool PK, bool SP>
@@ -100,20 +100,12 @@ __global__ __launch_bounds__(NW * f32_groups(NW, SP) * 64, D == 128 && NW * f32_
     const float *const vbase = reinterpret_cast<const float *>(p.v) + b * p.vs[0] + h * p.vs[1];
     const int32_t *fid = p.full_ids + b * p.fis[0] + h * p.fis[1] + qt * p.fis[2];
     const int32_t *pid = p.part_ids + b * p.pis[0] + h * p.pis[1] + qt * p.pis[2];
-    // The memory round trips of the start side by side: queries, counts, and (SP, rows of at most 64 tiles) both lists whole, a slot
-    // per lane.  Slots past a count hold anything and are not looked at.
+    // Queries and counts travel together.
     f32x4 q_in[D / 8];
     {
         const float *qp = reinterpret_cast<const float *>(p.q) + b * p.qs[0] + h * p.qs[1] + (int64_t)qrow * p.qs[2] + (D / 2) * hh;
 #pragma unroll
         for (int c = 0; c < D / 8; c++) q_in[c] = *(const f32x4 *)(qp + 4 * c);
-    }
-    const bool in_lanes = SP && p.nK <= 64;
-    int lane_full = 0, lane_part = 0;
-    if (in_lanes) {
-        const int slot = min(lane, p.nK - 1);
-        lane_full = fid[(int64_t)slot * p.fis[3]];
-        lane_part = pid[(int64_t)slot * p.pis[3]];
     }
     int cnt[2];
     const int32_t *const cnt_addr[2] = {p.full_lens + (b * p.fls[0] + h * p.fls[1] + qt * p.fls[2]),
@@ -135,6 +127,7 @@ __global__ __launch_bounds__(NW * f32_groups(NW, SP) * 64, D == 128 && NW * f32_
         if (s0 >= share) return;
         part_of(s0, share);
     }
+    const bool in_lanes = SP && NE <= 64;  // a part of at most 64 entries: one per lane, no way by LDS
     if constexpr (KG > 1) {
         const int all = NE;
         part_of(grp, KG);
@@ -146,6 +139,8 @@ __global__ __launch_bounds__(NW * f32_groups(NW, SP) * 64, D == 128 && NW * f32_
     pid += (int64_t)p_lo * p.pis[3];
     const int T = chunks_of(NE);
     if constexpr (KG == 1) T_all = T;
+    int lane_entry = 0;
+    if (in_lanes && lane < NE) lane_entry = lane < F ? fid[(int64_t)lane * p.fis[3]] : pid[(int64_t)(lane - F) * p.pis[3]];
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const SA_LDS uint8_t *)smem);
 
     // ---- per-lane constants ------------------------------------------------------------------------------------
@@ -177,10 +172,7 @@ __global__ __launch_bounds__(NW * f32_groups(NW, SP) * 64, D == 128 && NW * f32_
         for (int j = 0; j < EPC; j++) {
             const int e = MODE == 2 ? (t >> (p.lbk - 5)) : t * EPC + j;
             const int sub = MODE == 2 ? (t & ((1 << (p.lbk - 5)) - 1)) : 0;
-            int idx;
-            if (in_lanes) idx = e < F ? __builtin_amdgcn_readlane(lane_full, min(f_lo + e, 63)) : __builtin_amdgcn_readlane(lane_part, min(p_lo + max(e - F, 0), 63));
-            else idx = __builtin_amdgcn_readfirstlane(ring[min(e, kF32ListCap - 1)]);
-            plan_entry(pl, j, e, idx, sub);
+            plan_entry(pl, j, e, in_lanes ? __builtin_amdgcn_readlane(lane_entry, min(e, 63)) : __builtin_amdgcn_readfirstlane(ring[min(e, kF32ListCap - 1)]), sub);
         }
     };
     // all direct loads of a chunk into stage `buf`

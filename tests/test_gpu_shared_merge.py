@@ -1,6 +1,7 @@
 """Shared lists whose last workgroup adds the parts up (the whole workspace) against the merge by a second launch (a workspace without
 place for the workgroups' words) and against the definition."""
 import ctypes
+import dataclasses
 import math
 
 import pytest
@@ -116,3 +117,25 @@ def test_replays_bring_the_same_launch_number(gpu, dtype, B, H, Sq, Sk, D, BQ, B
         forward(q, k, v, md, BQ, BK, torch.empty_like(ws), full, want, wlse)
         torch.cuda.synchronize()
         assert torch.equal(got, want) and torch.equal(glse, wlse)
+
+
+@pytest.mark.parametrize("B,H,Sq,Sk,D,BQ,BK", [
+    (1, 4, 512, 512, 64, 64, 32),     # two groups of waves, 16 slots a row
+    (1, 2, 64, 1280, 64, 32, 16),     # 80 slots: lists of more entries than lanes
+    (1, 2, 128, 1024, 64, 64, 256),   # entries of several chunks
+    (1, 4, 256, 160, 128, 128, 32),   # one group
+])
+def test_rows_that_end_with_the_longest_list(gpu, B, H, Sq, Sk, D, BQ, BK):
+    """float32 reads ids[..., :len] alone: lists in rows of as many slots as the longest has, the last one at the end of its memory."""
+    q, _, _ = W.qkv(B, H, Sq, D, torch.float32, seed=1, device=gpu)
+    _, k, v = W.qkv(B, H, Sk, D, torch.float32, seed=2, device=gpu)
+    md = compute_mask_kernel(uneven(B, H, Sq, Sk, BQ, gpu), BQ, BK)
+    full, _ = sizes(q, Sk, BQ, BK)
+    ws = torch.empty(full, dtype=torch.uint8, device=gpu)
+    want, got = ((torch.empty_like(q), torch.empty(B, H, Sq, device=gpu)) for _ in range(2))
+    forward(q, k, v, md, BQ, BK, ws, full, *want)
+    ids = [(md.unmasked_kv_ids, md.unmasked_lens), (md.masked_kv_ids, md.masked_lens)]
+    cut = [t[..., :max(1, int(n.max()))].contiguous() for t, n in ids]
+    forward(q, k, v, dataclasses.replace(md, unmasked_kv_ids=cut[0], masked_kv_ids=cut[1]), BQ, BK, ws, full, *got)
+    torch.cuda.synchronize()
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
