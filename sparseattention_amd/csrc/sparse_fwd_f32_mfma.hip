@@ -39,8 +39,9 @@ constexpr int f32_group_bytes = 4 * 32 * D * 4 + 2 * NW * 1024 + kF32ListCap * 4
 // PK: mask entries of PARTIAL tiles from the bit-packed tiles; else from the bool mask (key stride 1, rows and base
 // 16-byte aligned: checked by the launcher).
 // SP: lists shared by up to p.nsplit workgroups (fwd_split_share).
-// KG: groups of NW waves that share out a list, each with stages of its own, in step; their rows meet in LDS.  Two where lists are
-// shared and NW <= 2 would leave two of the four SIMDs idle.
+// KG: groups of NW waves that share out a part's chunks, each with stages of its own, in step; their rows meet in LDS.  Two where lists are
+// shared and NW <= 2 would leave two of the four SIMDs idle (144 KiB of LDS at D = 128, one workgroup a compute unit: fwd_split_plan).
+// By chunks, not by entries: of an entry of two chunks (BLOCK_K 64) one group had both, 8 tiles of 32 chunks at D = 64 15.2 -> 12.6 us.
 // A small launch is a chain: B1 H4 S512 D64 with half of the 32 x 32 blocks (32 Q tiles, about 9 chunks each, parts of two) takes 11.1 us a
 // pass, where two waves per part, lists by way of LDS and a second launch for the merge took 15.7.  Time stamps with both lists read whole
 // beside the counts (11.2 us; callers' rows may end with the list): queries, counts and lists 1.2 us, first K and V at 2.3, products and
@@ -113,32 +114,21 @@ __global__ __launch_bounds__(NW * f32_groups(NW, SP) * 64, D == 128 && NW * f32_
     scalar_gather(cnt_addr, cnt);
     int F = min(min(max(cnt[0], 0), p.nK), kF32ListCap);
     int NE = F + min(min(max(cnt[1], 0), p.nK - F), kF32ListCap - F);
-    int share = 1, f_lo = 0, p_lo = 0, T_all = 0;  // T_all (KG > 1): chunks of the longest group
-    auto part_of = [&](int s, int n) {  // the s-th of n runs of what is left of the list
-        const int e_lo = fwd_split_first(NE, p.lbk, 5, s, n), e_hi = fwd_split_first(NE, p.lbk, 5, s + 1, n);
-        f_lo += min(e_lo, F);
-        p_lo += max(e_lo - F, 0);
-        F = min(max(F - e_lo, 0), e_hi - e_lo);
-        NE = e_hi - e_lo;
-    };
-    auto chunks_of = [&](int ne) { return MODE == 2 ? (ne << (p.lbk - 5)) : ((ne + EPC - 1) / EPC); };
+    int share = 1, p_lo = 0;
     if constexpr (SP) {
         share = fwd_split_share(NE, p.lbk, 5, p.split_least, p.split_chunks, p.nsplit);
         if (s0 >= share) return;
-        part_of(s0, share);
+        const int e_lo = fwd_split_first(NE, p.lbk, 5, s0, share), e_hi = fwd_split_first(NE, p.lbk, 5, s0 + 1, share);
+        p_lo = max(e_lo - F, 0);
+        fid += (int64_t)min(e_lo, F) * p.fis[3];
+        pid += (int64_t)p_lo * p.pis[3];
+        F = min(max(F - e_lo, 0), e_hi - e_lo);
+        NE = e_hi - e_lo;
     }
     const bool in_lanes = SP && NE <= 64;  // a part of at most 64 entries: one per lane, no way by LDS
-    if constexpr (KG > 1) {
-        const int all = NE;
-        part_of(grp, KG);
-#pragma unroll
-        for (int i = 0; i < KG; i++)
-            T_all = max(T_all, chunks_of(fwd_split_first(all, p.lbk, 5, i + 1, KG) - fwd_split_first(all, p.lbk, 5, i, KG)));
-    }
-    fid += (int64_t)f_lo * p.fis[3];
-    pid += (int64_t)p_lo * p.pis[3];
-    const int T = chunks_of(NE);
-    if constexpr (KG == 1) T_all = T;
+    // this group's chunks, t_lo .. t_lo + T - 1 of the part's (an entry of several chunks is shared out too), and those of the longest group
+    const int T_part = MODE == 2 ? (NE << (p.lbk - 5)) : ((NE + EPC - 1) / EPC);
+    const int t_lo = T_part * grp / KG, T = T_part * (grp + 1) / KG - t_lo, T_all = (T_part + KG - 1) / KG;
     int lane_entry = 0;
     if (in_lanes && lane < NE) lane_entry = lane < F ? fid[(int64_t)lane * p.fis[3]] : pid[(int64_t)(lane - F) * p.pis[3]];
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(const SA_LDS uint8_t *)smem);
@@ -166,7 +156,7 @@ __global__ __launch_bounds__(NW * f32_groups(NW, SP) * 64, D == 128 && NW * f32_
         pl.slot[j] = partial ? e - F : 0;
         pl.flags |= (exists ? 1u : 0u) << j | (partial ? 16u : 0u) << j;
     };
-    auto plan_of = [&](int t, Plan &pl) {  // chunk t (t < T) from the LDS copy of the list
+    auto plan_of = [&](int t, Plan &pl) {  // chunk t of the part
         pl.flags = 0u;
 #pragma unroll
         for (int j = 0; j < EPC; j++) {
@@ -237,9 +227,9 @@ __global__ __launch_bounds__(NW * f32_groups(NW, SP) * 64, D == 128 && NW * f32_
             __syncthreads();
         }
         Plan pl;
-        if (T > 0) {  // (KG > 1: another group may have entries where this one has none)
-            plan_of(0, pl);
-            stage_chunk(0, pl, 0);
+        if (T > 0) {  // (KG > 1: a part of one chunk is the other group's)
+            plan_of(t_lo, pl);
+            stage_chunk(0, pl, t_lo);
         }
         unsigned fl_cur = T > 0 ? pl.flags : 0u;
         scale_q();
@@ -252,7 +242,7 @@ __global__ __launch_bounds__(NW * f32_groups(NW, SP) * 64, D == 128 && NW * f32_
             // branch, 1 %, but a part of one chunk would wait for it)
             unsigned fl_next = 0u;
             if (!SP || tc + 1 < T) {
-                const int tn = tc + 1 < T ? tc + 1 : T - 1;
+                const int tn = t_lo + (tc + 1 < T ? tc + 1 : T - 1);
                 Plan pn;
                 plan_of(tn, pn);
                 stage_chunk(BUF ^ 1, pn, tn);

@@ -105,7 +105,12 @@ __global__ __launch_bounds__(256) void fwd_merge_kernel(const FwdParams p, int l
 // From 257 tiles on every slot has work.  Sk below 32 chunks is not shared, whatever the lists (32 chunks, Sk = 2048: 8 tiles
 // 33.6 | 17.0, 64 tiles 34.7 | 26.3, 128 tiles 35.2 | 33.6; 16 chunks: the tables above, as lists of a longer Sk).
 // float32: a chunk of 32 keys keeps the matrix unit busy for 1.7 us (D = 64) or 3.4 us, so two chunks are worth a part
-// (32 tiles of 16 chunks at D = 64: 46 -> 11.7 us, 256 of 32 at D = 128: 158 -> 95 us).  Sk above 4096 is not shared there: a row's
+// (32 tiles of 16 chunks at D = 64: 46 -> 11.4 us, 256 of 32 at D = 128, BLOCK_Q 64: 158 -> 93 us).  At D = 128, BLOCK_Q 64 the two groups of
+// a workgroup take a compute unit's LDS: parts for one workgroup a unit where those fill seven eighths of the units.  Every list that
+// long, us, parts for two workgroups a unit | one:
+//    16 tiles of 64 chunks 35.8 | 23.7   32 of 16 16.8 | 16.6, of 32 30.0 | 21.4, of 128 56.7 | 50.9   48 of 32 39.1 | 28.9   64 of 64 55.8 | 49.0
+//   128 of 32 55.2 | 48.2, of 128 166 | 161   and three quarters of them: 96 of 16 35.5 | 28.5, of 64 81.6 | 85.0, of 128 138 | 160
+// Sk above 4096 is not shared there: a row's
 // keys are added up one after the other in one workgroup, 1.2e-6 from the result at 4096 keys and 3.3e-6 at 32768, and shared
 // lists (4e-7 and 7e-7) would move the result by that much.
 FwdSplitPlan fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus) {
@@ -114,7 +119,8 @@ FwdSplitPlan fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus
     const int lck = dtype == 2 ? 5 : 6;
     const int chunks = (Sk + (1 << lck) - 1) >> lck;  // of the longest list there can be
     const int part = dtype == 2 ? 2 : (4 * tiles <= cus ? 8 : (2 * tiles <= cus ? 16 : 48));
-    const int most = 2 * cus / tiles, parts = (chunks + part - 1) / part;
+    const bool lone = dtype == 2 && D == 128 && BQ == 64 && 2 * tiles <= cus && 8 * (cus / tiles * tiles) >= 7 * cus;
+    const int most = lone ? cus / tiles : 2 * cus / tiles, parts = (chunks + part - 1) / part;
     const int n = parts < most ? parts : most;
     if (n < 2 || chunks < (dtype == 2 ? 4 : 32)) return plan;
     plan.nsplit = n < 32 ? n : 32;

@@ -30,13 +30,19 @@ def forward(q, k, v, md, BQ, BK, ws, ws_bytes, o, lse):
     assert rc == 0, _native.load().sa_last_error()
 
 
-def sizes(q, Sk, BQ, BK):
-    """(bytes with the words, bytes of the parts alone)"""
+def sizes_of(q, Sk, BQ, BK):
+    """(bytes with the words, where the launch has them; bytes of the parts alone)"""
     B, H, Sq, D = q.shape
     full = _native.load().sa_fwd_split_workspace_bytes(B, H, Sq, Sk, D, BQ, BK, CODE[q.dtype])
     tiles, part = B * H * (Sq // BQ), BQ * (D + 2) * 4
-    assert full > 0 and full % (tiles * (part + 8)) == 0
-    return full, full // (part + 8) * part
+    return full, full if full % (tiles * (part + 8)) else full // (part + 8) * part
+
+
+def sizes(q, Sk, BQ, BK):
+    """(bytes with the words, bytes of the parts alone)"""
+    full, parts = sizes_of(q, Sk, BQ, BK)
+    assert 0 < parts < full
+    return full, parts
 
 
 def uneven(B, H, Sq, Sk, BQ, gpu):
@@ -56,7 +62,7 @@ def uneven(B, H, Sq, Sk, BQ, gpu):
     (torch.float32, 1, 4, 512, 512, 64, 64, 32),      # two groups of waves
     (torch.float32, 1, 3, 192, 160, 64, 64, 16),      # an odd number of chunks: one group has one more
     (torch.float32, 1, 2, 64, 1280, 64, 32, 16),      # lists that come by way of LDS; one wave a group
-    (torch.float32, 1, 2, 128, 1024, 64, 64, 256),    # entries of several chunks: a group without any
+    (torch.float32, 1, 2, 128, 1024, 64, 64, 256),    # entries of several chunks, shared out between the groups
     (torch.float32, 1, 2, 128, 256, 128, 64, 32),
     (torch.float32, 2, 16, 512, 160, 128, 128, 32),   # one group of four waves
     (torch.bfloat16, 4, 8, 512, 4096, 128, 128, 64),  # four parts of four waves
@@ -139,3 +145,14 @@ def test_rows_that_end_with_the_longest_list(gpu, B, H, Sq, Sk, D, BQ, BK):
     forward(q, k, v, dataclasses.replace(md, unmasked_kv_ids=cut[0], masked_kv_ids=cut[1]), BQ, BK, ws, full, *got)
     torch.cuda.synchronize()
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("tiles", [8, 16, 32, 48, 64, 80, 128])
+def test_no_more_parts_than_run_at_once(gpu, tiles):
+    """float32, D = 128, BLOCK_Q 64: a workgroup takes the LDS of its compute unit, so the launch has one for each; elsewhere two."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    D, Sk = 128, 4096
+    for BQ, most in ((64, cus), (128, 2 * cus)):
+        q = torch.empty(1, 1, tiles * BQ, D, dtype=torch.float32, device=gpu)
+        _, parts = sizes_of(q, Sk, BQ, 32)
+        assert parts // (tiles * BQ * (D + 2) * 4) == min(64, 32, most // tiles)
