@@ -317,7 +317,8 @@ __device__ __forceinline__ bool all_arrived(uint64_t *words, uint64_t tag, int m
 // The sum of n parts that workgroups have handed over: this wave's N blocks of 32 x 32 values, 16 a lane, the lane's four of run g of a
 // block at rows_at + part * rows_step + 1024 (4 block + g) (where a wave leaves its accumulators, 1 KiB a store), with reference value
 // (-inf: no attended key) and sum of the lane's row at state_at + part * state_step.  In the order of the parts, whoever adds.  The
-// first B parts are under way while the largest reference value is looked for: one round trip for up to B parts.
+// first B parts are under way while the largest reference value is looked for, by fours: one round trip for up to four parts, one more for every four
+// beyond them and for every B parts behind the first B.
 template <int N, int B>
 __device__ __forceinline__ void add_parts(const HandOver &rows, uint32_t rows_at, uint32_t rows_step, const HandOver &state, uint32_t state_at,
                                           uint32_t state_step, int n, f32x16 (&acc)[N], float &M, float &L) {

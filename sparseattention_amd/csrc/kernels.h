@@ -177,7 +177,7 @@ __host__ __device__ inline int fwd_split_first(int NE, int lbk, int lck, int s, 
     return e < NE ? e : NE;
 }
 // Whether the last workgroup of a shared list to arrive adds up its parts (all_arrived), else a second launch does: sparse_fwd_merge.hip.
-bool fwd_merges_in_launch(int nsplit, int BQ, int D, int dtype);
+bool fwd_merges_in_launch(int tiles, int nsplit, int BQ, int D, int dtype);
 // The rule for nsplit, split_chunks and split_least: sparse_fwd_merge.hip.
 struct FwdSplitPlan {
     int nsplit = 1, chunks = 1 << 30, least = 0;

@@ -7,7 +7,7 @@ namespace {
 
 // One wave per (Q tile, 32 rows, 32 of the D columns), four per workgroup: the parts' rows in the register order they were
 // left in (lane (l32, hh): row l32, columns 8g + 4hh + j), so every read is a run of 1 KiB.  The rows are the launch's
-// own output of a moment ago and mostly still in a cache; the reads of kBatch parts are in flight together.
+// own output of a moment ago, past the L2s and mostly still in the memory-side cache; the reads of kBatch parts are in flight together.
 constexpr int kBatch = 4;
 template <int DT, int D>
 __global__ __launch_bounds__(256) void fwd_merge_kernel(const FwdParams p, int lck, int NW) {
@@ -134,12 +134,17 @@ FwdSplitPlan fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus
 //   8 x 16  32 tiles 13.3 | 11.7    32 x 8  8 tiles 19.8 | 17.5    8 x 32  32 tiles 18.5 | 17.3
 //   32 x 16  16 tiles 25.2 | 24.9, 8 tiles 21.0 | 20.7, 4 tiles 20.2 | 20.4    16 x 32  16 tiles 20.1 | 20.0    8 x 64  16 tiles 21.9 | 23.6
 //   32 x 32  8 tiles 29.2 | 33.6, 4 tiles 25.0 | 29.6    16 x 64  16 tiles 28.9 | 30.6    32 x 64  4 tiles 38.0 | 50.7
-// bf16, where one wave reads 32 rows of every part: up to four parts
+// bf16, where one wave reads 32 rows of every part: up to four parts, of 64 KiB only where there are more than 16 tiles to add up side by side
 //   4 x 64  128 tiles of up to 256 chunks 136.0 | 132.8, 128 72.3 | 68.8, 64 45.3 | 42.0, 25 28.7 | 25.8; 64 tiles of 32 22.7 | 21.3, 32 tiles 20.6 | 18.7
 //   4 x 32  128 tiles, D = 64, of up to 256 79.3 | 76.8, BLOCK_Q 64 of up to 128 58.3 | 58.1    4 x 16  128 tiles of up to 128 45.9 | 41.5
 //   8 x 32  8 tiles of 64, D = 64 14.4 | 14.8, 64 tiles of up to 128 29.4 | 29.3, BLOCK_Q 64 36.8 | 38.2, 16 tiles of 64 21.0 | 21.9
-bool fwd_merges_in_launch(int nsplit, int BQ, int D, int dtype) {
-    return (int64_t)nsplit * BQ * D * 4 <= 256 * 1024 && (dtype == 2 || nsplit <= 4);
+//   4 x 64  of 32 chunks  8 tiles 16.4 | 17.6   16 tiles 17.5 | 17.9   32 tiles 20.4 | 18.7   64 tiles 25.2 | 21.2
+// For a second launch too parts are stored past L2 (HandOver): a launch whose parts lie in the L2s ends with writing them back.  bf16, us, a kernel
+// of its own without the adding up and with stores through L2 | this one: 64 tiles of 64 chunks, BLOCK_Q 64, D = 64 22.5 | 20.6, D = 128
+// 27.0 | 25.7; 32 tiles of 256, D = 64 30.5 | 27.6; 16 tiles of 128, BLOCK_Q 128 24.8 | 23.7; it loses at 8 tiles of 128, BLOCK_Q 64, D = 64 16.3 | 17.3.
+bool fwd_merges_in_launch(int tiles, int nsplit, int BQ, int D, int dtype) {
+    const int64_t bytes = (int64_t)nsplit * BQ * D * 4;
+    return bytes <= 256 * 1024 && (dtype == 2 || (nsplit <= 4 && (bytes <= 128 * 1024 || tiles > 16)));
 }
 
 // When a list is walked in two halves by one workgroup of twice the waves (sparse_fwd_kernel<..., TW>): from half as many Q tiles

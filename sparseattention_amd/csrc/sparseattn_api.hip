@@ -446,7 +446,7 @@ int forward_impl(const void *q, const int64_t q_strides[4], const void *k, const
         fp.ws = static_cast<float *>(workspace);
         fp.ws_ml = fp.ws + (need / 4 / (size_t)(D + 2)) * (size_t)D;
         // (a caller who asked an earlier library for the size has no place for them: a second launch then)
-        if (need != 0 && sa::fwd_merges_in_launch(plan.nsplit, BQ, D, dtype) && workspace_bytes >= need + (size_t)8 * B * H * fp.nQ * plan.nsplit)
+        if (need != 0 && sa::fwd_merges_in_launch(B * H * fp.nQ, plan.nsplit, BQ, D, dtype) && workspace_bytes >= need + (size_t)8 * B * H * fp.nQ * plan.nsplit)
             fp.tag = next_launch_tag() | 1;  // (never 0)
     }
     if (kernel == SA_FWD_KERNEL_SHORT_LISTS) {
@@ -569,7 +569,7 @@ size_t sa_fwd_split_workspace_bytes(int B, int H, int Sq, int Sk, int D, int BQ,
     sa::FwdSplitPlan plan;
     if ((D != 64 && D != 128) || dtype < SA_DTYPE_BF16 || dtype > SA_DTYPE_FP32) return 0;
     const size_t parts = split_shape(B, H, Sq, Sk, D, BQ, BK, dtype, &plan);
-    return parts != 0 && sa::fwd_merges_in_launch(plan.nsplit, BQ, D, dtype) ? parts + (size_t)8 * B * H * (Sq / BQ) * plan.nsplit : parts;
+    return parts != 0 && sa::fwd_merges_in_launch(B * H * (Sq / BQ), plan.nsplit, BQ, D, dtype) ? parts + (size_t)8 * B * H * (Sq / BQ) * plan.nsplit : parts;
 }
 
 int sa_fwd_split_least_keys(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype) {

@@ -66,7 +66,7 @@ def uneven(B, H, Sq, Sk, BQ, gpu):
     (torch.float32, 1, 2, 128, 256, 128, 64, 32),
     (torch.float32, 2, 16, 512, 160, 128, 128, 32),   # one group of four waves
     (torch.bfloat16, 4, 8, 512, 4096, 128, 128, 64),  # four parts of four waves
-    (torch.bfloat16, 1, 3, 256, 2048, 128, 128, 32),
+    (torch.bfloat16, 1, 9, 256, 2048, 128, 128, 32),
     (torch.float16, 3, 8, 256, 2560, 64, 64, 16),     # parts that do not divide the list
     (torch.float16, 1, 2, 96, 2048, 64, 32, 64),      # one wave
     (torch.bfloat16, 1, 2, 64, 2048, 128, 64, 1024),  # entries of several chunks, fewer than parts
@@ -99,7 +99,7 @@ def test_the_last_workgroup_adds_up(gpu, dtype, B, H, Sq, Sk, D, BQ, BK):
         assert float((lse.double() - want_lse)[live].abs().max()) <= (1e-5 if dtype == torch.float32 else 6e-3 + 2 ** -9 * 5)
 
 
-@pytest.mark.parametrize("dtype,B,H,Sq,Sk,D,BQ,BK", [(torch.float32, 1, 4, 256, 512, 64, 64, 32), (torch.bfloat16, 1, 8, 256, 2048, 128, 128, 64)])
+@pytest.mark.parametrize("dtype,B,H,Sq,Sk,D,BQ,BK", [(torch.float32, 1, 4, 256, 512, 64, 64, 32), (torch.bfloat16, 1, 9, 256, 2048, 128, 128, 64)])
 def test_replays_bring_the_same_launch_number(gpu, dtype, B, H, Sq, Sk, D, BQ, BK):
     q, _, _ = W.qkv(B, H, Sq, D, dtype, seed=1, device=gpu)
     _, k, v = W.qkv(B, H, Sk, D, dtype, seed=2, device=gpu)
@@ -156,3 +156,13 @@ def test_no_more_parts_than_run_at_once(gpu, tiles):
         q = torch.empty(1, 1, tiles * BQ, D, dtype=torch.float32, device=gpu)
         _, parts = sizes_of(q, Sk, BQ, 32)
         assert parts // (tiles * BQ * (D + 2) * 4) == min(64, 32, most // tiles)
+
+
+@pytest.mark.parametrize("dtype,tiles,BQ,Sk,in_launch", [
+    (torch.bfloat16, 8, 128, 2048, False), (torch.bfloat16, 16, 128, 2048, False), (torch.bfloat16, 17, 128, 2048, True),
+    (torch.bfloat16, 8, 64, 2048, True), (torch.bfloat16, 8, 64, 4096, False), (torch.float32, 8, 128, 256, True), (torch.float32, 8, 128, 512, False)])
+def test_which_launch_adds_up(gpu, dtype, tiles, BQ, Sk, in_launch):
+    """One workgroup adds up 256 KiB of 16-bit types' parts only where enough of them do so side by side."""
+    q = torch.empty(1, 1, tiles * BQ, 128, dtype=dtype, device=gpu)
+    full, parts = sizes_of(q, Sk, BQ, 64)
+    assert (full > parts) == in_launch
