@@ -295,7 +295,8 @@ struct BwdParams {
 struct BwdLaunch {
     BwdParams pass[3];
     int first[3], tiles[3];
-    // null, or [8][slots]: workgroup 8 j + x has the j-th of XCD x's tiles by falling cost: pass << 24 | its place in the XCD's share
+    // null, or [8][slots]: workgroup 8 j + x has the j-th of XCD x's tiles by falling cost: pass << 29 | its place in the XCD's share << 18 |
+    // its FULL entries << 9 | all its entries
     const int32_t *order;
     int slots;
 };

@@ -126,8 +126,9 @@ __device__ __forceinline__ void bwd_store_rows(const f32x16 (&a)[D / 32], float 
 // enters dK's product, is stored for bwd_dq_tile too (D = 128: both accumulators, K and V take 192 of 256 registers, so that
 // S, dP and the reads on their way share the rest: see `phase`).  K then stays unscaled and S - L is scaled in float32 (a rounded
 // scale K would give dQ another P than the rounded scale Q of the forward: 3 % more error, this is less than before).
-template <int DT, int D, int KIND, bool PK, int PASS, bool DS = false>
-__device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, uint8_t *smem) {
+// ORD: the counts come with the tile's place in the order (bwd_sort_tiles), F << 9 | T.
+template <int DT, int D, int KIND, bool PK, int PASS, bool DS = false, bool ORD = false>
+__device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, uint8_t *smem, int counts = 0) {
     using E = Elem<DT>;
     static_assert(D == 128 || D == 64, "head dim");
     constexpr int ROWB = D * 2;
@@ -187,12 +188,18 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
     // Counts and tile indices are clamped to the nS streamed tiles there are (the reference guards every K/V and mask
     // load with kv_offset < SEQLEN_K, sparse_attn_kernel.py:35,39,60): stale or foreign metadata then gives wrong
     // numbers, never an access outside the tensors or past the list's LDS copy (nS <= kBwdListCap, checked by the host).
-    int cnt[2];
-    const int32_t *const cnt_addr[2] = {p.full_lens + (b * p.fls[0] + h * p.fls[1] + rt * p.fls[2]),
-                                        p.part_lens + (b * p.pls[0] + h * p.pls[1] + rt * p.pls[2])};
-    scalar_gather(cnt_addr, cnt);
-    const int F = min(max(cnt[0], 0), p.nS);
-    const int T = F + min(max(cnt[1], 0), p.nS - F);  // chunks = list entries
+    int F, T;  // chunks = list entries
+    if constexpr (ORD) {
+        F = counts >> 9;
+        T = counts & 511;
+    } else {
+        int cnt[2];
+        const int32_t *const cnt_addr[2] = {p.full_lens + (b * p.fls[0] + h * p.fls[1] + rt * p.fls[2]),
+                                            p.part_lens + (b * p.pls[0] + h * p.pls[1] + rt * p.pls[2])};
+        scalar_gather(cnt_addr, cnt);
+        F = min(max(cnt[0], 0), p.nS);
+        T = F + min(max(cnt[1], 0), p.nS - F);
+    }
     f32x16 acc[NDB], acc2[BOTH ? NDB : 1];  // acc2: dV beside dK
 #pragma unroll
     for (int db = 0; db < NDB; db++)
@@ -584,11 +591,12 @@ template <int DT, int D, bool PK, bool ORD>
 __global__ __launch_bounds__(256, D == 64 && PK ? 3 : 2) void sparse_bwd_kernel(const BwdLaunch l) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     const int id = blockIdx.x;
-    int pass = 0, lin = id;  // lin: workgroup of its pass, as bwd_place takes it
+    int pass = 0, lin = id, counts = 0;  // lin: workgroup of its pass, as bwd_place takes it
     if constexpr (ORD) {
-        const int e = l.order[(id & 7) * l.slots + (id >> 3)];
-        pass = e >> 24;
-        lin = (e & 0xffffff) * 8 + (id & 7);
+        const int e = __builtin_amdgcn_readfirstlane(l.order[(id & 7) * l.slots + (id >> 3)]);
+        pass = e >> 29;
+        lin = (e >> 18 & 2047) * 8 + (id & 7);
+        counts = e & 0x3ffff;
     } else if (D != 64 && id >= l.first[2]) {
         pass = 2;
         lin = id - l.first[2];
@@ -597,11 +605,11 @@ __global__ __launch_bounds__(256, D == 64 && PK ? 3 : 2) void sparse_bwd_kernel(
         lin = id - l.first[1];
     }
     if (pass == 0) {
-        if (lin < l.tiles[0]) bwd_tile<DT, D, D == 64 ? kDKV : kDK, PK, 0>(l.pass[0], lin, l.tiles[0], smem);
+        if (lin < l.tiles[0]) bwd_tile<DT, D, D == 64 ? kDKV : kDK, PK, 0, false, ORD>(l.pass[0], lin, l.tiles[0], smem, counts);
     } else if (D == 64 || pass == 1) {
-        if (lin < l.tiles[1]) bwd_tile<DT, D, kDQ, PK, 1>(l.pass[1], lin, l.tiles[1], smem);
+        if (lin < l.tiles[1]) bwd_tile<DT, D, kDQ, PK, 1, false, ORD>(l.pass[1], lin, l.tiles[1], smem, counts);
     } else {
-        if constexpr (D != 64) bwd_tile<DT, D, kDV, PK, 2>(l.pass[2], lin, l.tiles[2], smem);
+        if constexpr (D != 64) bwd_tile<DT, D, kDV, PK, 2, false, ORD>(l.pass[2], lin, l.tiles[2], smem, counts);
     }
 }
 
@@ -622,57 +630,59 @@ __global__ __launch_bounds__(256, 2) void sparse_bwd_queries_kernel(const BwdPar
 // Per query row: -Delta = -sum_d dO o O, and -L = -lse / ln 2 (-inf for rows that attended to nothing, so that their
 // P = exp2(S - L) is 0).  D/8 lanes per row, 8 elements each.
 // In front of them, where the passes take their tiles by falling cost, eight workgroups sort one XCD's tiles each: a counting sort over
-// 32 classes of cost by eighths of the order of planes (whose neighbours share operands; within one in any order: each tile's result
-// is its own).
+// 32 classes of cost by eighths of the XCD's tiles, the passes one after the other in the order of planes (neighbours share operands; within
+// one in any order: each tile's result is its own).  A tile's counts go with its place, so that its start is no read longer.
 constexpr int kCosts = 256, kOrderMost = 2048;
 __device__ __forceinline__ void bwd_sort_tiles(const BwdOrderParams &o, int xcd) {
+    __shared__ int32_t entry[kOrderMost];
     __shared__ uint16_t cost[kOrderMost];
-    __shared__ int most, count[kCosts], of_wave[4], least_of[3], most_of[3];
-    const int tid = threadIdx.x;
-    if (tid == 0) most = 1;
+    __shared__ int count[kCosts], of_wave[4], least_of[3], most_of[3];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (tid < 3) {
         least_of[tid] = 0x7fffffff;
         most_of[tid] = 0;
     }
     count[tid] = 0;
     __syncthreads();
-    auto which = [&](int i, int &pass, int &k) {  // slot i of the XCD before sorting
-        pass = 0;
-        k = i;
-        for (int n = 0; n + 1 < o.n && k >= (o.pass[n].planes * o.pass[n].nR >> 3); n++) {
-            k -= o.pass[n].planes * o.pass[n].nR >> 3;
-            pass = n + 1;
-        }
-    };
-    for (int i = tid; i < o.slots; i += 256) {
-        int pass, k;
-        which(i, pass, k);
+    {  // one pass per wave (its arguments are scalars then), the passes' tiles one after the other
+        const int pass = wave % o.n, waves = (4 - pass + o.n - 1) / o.n;
         const BwdOrderParams::Pass &q = o.pass[pass];
-        const BwdPlace at = bwd_place_in_order(q, xcd * (q.planes * q.nR >> 3) + k);
-        const int b = at.plane / q.H, h = at.plane - b * q.H;
-        const int F = min(max(q.full_lens[b * q.fls[0] + h * q.fls[1] + at.rt * q.fls[2]], 0), q.nS);
-        const int T = F + min(max(q.part_lens[b * q.pls[0] + h * q.pls[1] + at.rt * q.pls[2]], 0), q.nS - F);
-        const int c = min(q.fixed + q.per_entry * T, 0xffff);
-        cost[i] = (uint16_t)c;
-        atomicMax(&most, c);
-        atomicMin(&least_of[pass], c);
-        atomicMax(&most_of[pass], c);
+        const int tiles = q.planes * q.nR >> 3;
+        int first = 0, least = 0x7fffffff, most = 0;
+        for (int n = 0; n < pass; n++) first += o.pass[n].planes * o.pass[n].nR >> 3;
+        for (int k = 64 * (wave / o.n) + lane; k < tiles; k += 64 * waves) {
+            const BwdPlace at = bwd_place_in_order(q, xcd * tiles + k);
+            const int b = at.plane / q.H, h = at.plane - b * q.H;
+            const int f = q.full_lens[b * q.fls[0] + h * q.fls[1] + at.rt * q.fls[2]], m = q.part_lens[b * q.pls[0] + h * q.pls[1] + at.rt * q.pls[2]];
+            const int F = min(max(f, 0), q.nS), T = F + min(max(m, 0), q.nS - F);  // (clamped as in bwd_tile; below 512: bwd_order_bytes)
+            const int c = min(q.fixed + q.per_entry * T, 0xffff);
+            cost[first + k] = (uint16_t)c;
+            entry[first + k] = pass << 29 | k << 18 | F << 9 | T;
+            least = min(least, c);
+            most = max(most, c);
+        }
+#pragma unroll
+        for (int s = 1; s < 64; s <<= 1) {
+            least = min(least, __shfl_xor(least, s));
+            most = max(most, __shfl_xor(most, s));
+        }
+        if (lane == 0) {
+            atomicMin(&least_of[pass], least);
+            atomicMax(&most_of[pass], most);
+        }
     }
     __syncthreads();
     bool alike = true;  // lists of about one length: the order of planes, whose neighbours share operands, is the better one
     for (int n = 0; n < o.n; n++) alike = alike && 4 * (most_of[n] - least_of[n]) <= most_of[n];
     if (alike) {
-        for (int i = tid; i < o.slots; i += 256) {
-            int pass, k;
-            which(i, pass, k);
-            o.order[xcd * o.slots + i] = pass << 24 | k;
-        }
+        for (int i = tid; i < o.slots; i += 256) o.order[xcd * o.slots + i] = entry[i];
         return;
     }
+    const int most = max(max(most_of[0], most_of[1]), most_of[2]);
     auto cls = [&](int i) { return 8 * (31 - (int)((unsigned)cost[i] * 31u / (unsigned)most)) + 8 * i / o.slots; };
     for (int i = tid; i < o.slots; i += 256) atomicAdd(&count[cls(i)], 1);
     __syncthreads();
-    const int mine = count[tid], lane = tid & 63;
+    const int mine = count[tid];
     int upto = mine;  // of the wave's classes up to this one
 #pragma unroll
     for (int s = 1; s < 64; s <<= 1) {
@@ -684,11 +694,7 @@ __device__ __forceinline__ void bwd_sort_tiles(const BwdOrderParams &o, int xcd)
     for (int w = 0; w < tid >> 6; w++) upto += of_wave[w];
     count[tid] = upto - mine;
     __syncthreads();
-    for (int i = tid; i < o.slots; i += 256) {
-        int pass, k;
-        which(i, pass, k);
-        o.order[xcd * o.slots + atomicAdd(&count[cls(i)], 1)] = pass << 24 | k;
-    }
+    for (int i = tid; i < o.slots; i += 256) o.order[xcd * o.slots + atomicAdd(&count[cls(i)], 1)] = entry[i];
 }
 template <int DT, int D, bool ORD>
 __global__ __launch_bounds__(256) void bwd_prepare_kernel(const BwdPrepParams p) {
@@ -827,17 +833,23 @@ size_t bwd_ds_bytes(int B, int H, int Sq, int Sk, int D) {
 }
 
 // Tiles by falling cost.  In the order of planes the last ones to start are as likely long as short: of 1536 tiles (B4 H12 S2048 D64, packed
-// documents) on 768 slots one of 15 entries started at 31 us and ended the launch at 60, where the work is 40 us of every slot.  More
-// workgroups than run at once by a quarter (three per compute unit at D = 64, else two), lists of eight entries or more (the sort
-// is 4 us beside the statistics, which take as long from there on), eighths of equal size, at most kOrderMost tiles a XCD, and planes of a
-// XCD that its L2 nearly holds (8 MiB), since the tiles at work are of all of them.  Backward with statistics, us, planes | cost:
-//   D = 64   documents B4 H12 S2048 71.3 | 63.9, B8 H12 S1024 67.9 | 58.1, B4 H17 S1024 51.3 | 46.4, B8 H24 S512 51.7 | 48.5   blocks p = 0.75 82 | 73.5
-//            causal B4 H12 S2048 124.6 | 112.2, B4 H17 S1024 60.2 | 53.4   every key 177.7 | 177.8   (S256 29.5 | 32.2: left as it is)
-//   D = 128  documents B4 H8 S1024 51.2 | 47.5, B1 H28 S1024 47.4 | 43.2 (B3 H8, 576 tiles 43.7 | 44.4: left as it is)
-//            causal B2 H8 S2048 91.9 | 87.4, B1 H32 S1024 57.2 | 55.6   every key B1 H28 S1024 79.0 | 80.4
+// documents) on 768 slots one of 15 entries started at 31 us and ended the launch at 60, where the work is 40 us of every slot.
+// More workgroups than run at once by a quarter (256 compute units; three each at D = 64 with packed tiles, else two), lists of eight entries
+// or more, at D = 128 of sixteen, eighths of equal size, at most kOrderMost tiles a XCD.  So many query tiles that their statistics take as
+// long as the sort (prepare 5.1 -> 6.1 us at 256 query tiles of D = 128, 7.1 -> 7.3 at 768 of D = 64).  Planes of a XCD that its L2 nearly holds
+// (8 MiB), since the tiles at work are of all of them; and two planes or more, three where they are long, since a XCD with one has all its
+// long tiles at work on one part of it.  Backward with statistics, us, planes | cost:
+//   D = 64   documents B4 H12 S2048 70.7 | 57.9, B8 H12 S1024 70.9 | 57.7, B4 H17 S1024 58.2 | 44.7, B8 H24 S512 50.7 | 46.8, B2 H12 S4096 74.0 | 62.7
+//            causal B4 H12 S2048 120 | 105, B4 H17 S1024 56.5 | 48.0   blocks B4 H12 S2048 111 | 101   every key 177 | 179, B8 H12 S1024 96.5 | 97.7
+//            window of a quarter B4 H12 S2048 68.5 | 65.8, B8 H12 S1024 49.6 | 49.4, B8 H24 S512 40.1 | 40.4, of 64 keys there 35.2 | 37.1
+//            left as it is: causal B1 H8 S8192 301 | 348, window of half B2 H8 S4096 97.7 | 102
+//   D = 128  documents B4 H8 S1024 51.6 | 47.3, B2 H12 S2048 70.8 | 65.3   causal B4 H8 S1024 54.1 | 49.9, B2 H12 S2048 134 | 120   blocks 132 | 123
+//            every key B4 H8 S1024 74.2 | 74.1, window of a quarter 39.2 | 40.2   (B1 H64 S512, left as it is: 45.0 | 46.1, window 32.3 | 33.9)
 size_t bwd_order_bytes(int B, int H, int Sq, int Sk, int D) {
     const int64_t planes = (int64_t)B * H, tq = planes * (Sq / 128), tk = planes * (Sk / 128), all = tq + tk * (D == 64 ? 1 : 2);
-    if (tq % 8 || tk % 8 || all <= (D == 64 ? 960 : 640) || all > 8 * kOrderMost || Sq < 512 || Sk < 512) return 0;
+    const int shortest = Sq < Sk ? Sq : Sk, longest = Sq < Sk ? Sk : Sq;
+    if (tq % 8 || tk % 8 || all <= (D == 64 ? 960 : 640) || all > 8 * kOrderMost) return 0;
+    if (shortest < (D == 64 ? 512 : 1024) || tq < (D == 64 ? 384 : 192) || planes < (longest > 2048 ? 24 : 16)) return 0;
     if ((planes + 7) / 8 * 2 * ((int64_t)Sq + Sk) * D * 2 > (8 << 20)) return 0;
     return (size_t)all * 4;
 }
