@@ -290,6 +290,7 @@ struct BwdParams {
     int64_t outs2[3];
     int plane0, planes;            // the pass covers planes plane0 .. plane0 + planes - 1 of the B * H
     uint8_t *ds;                   // workspace of dS of these planes (bwd_dq_tile), Sq * Sk elements each
+    int far;                       // 1: dS of these planes is larger than the caches (kDsFar)
 };
 // The passes of one launch: workgroup first[i] + t has tile t of pass i.
 struct BwdLaunch {

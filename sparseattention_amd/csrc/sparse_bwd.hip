@@ -122,15 +122,16 @@ __device__ __forceinline__ void bwd_store_rows(const f32x16 (&a)[D / 32], float 
     }
 }
 
-// PK: the mask entries of PARTIAL tiles come bit-packed from p.packed, else from the bool mask.  DS: dS, rounded as it
+// PK: the mask entries of PARTIAL tiles come bit-packed from p.packed, else from the bool mask.  DS (DSM 1; 2: past L2): dS, rounded as it
 // enters dK's product, is stored for bwd_dq_tile too (D = 128: both accumulators, K and V take 192 of 256 registers, so that
 // S, dP and the reads on their way share the rest: see `phase`).  K then stays unscaled and S - L is scaled in float32 (a rounded
 // scale K would give dQ another P than the rounded scale Q of the forward: 3 % more error, this is less than before).
 // ORD: the counts come with the tile's place in the order (bwd_sort_tiles), F << 9 | T.
-template <int DT, int D, int KIND, bool PK, int PASS, bool DS = false, bool ORD = false>
+template <int DT, int D, int KIND, bool PK, int PASS, int DSM = 0, bool ORD = false>
 __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, uint8_t *smem, int counts = 0) {
     using E = Elem<DT>;
     static_assert(D == 128 || D == 64, "head dim");
+    constexpr bool DS = DSM != 0;
     constexpr int ROWB = D * 2;
     using Lds = BwdLds<D, PK>;
     constexpr int NS = Lds::NS, CBUF = Lds::CBUF, Z0 = Lds::Z0, STAT0 = Lds::STAT0, MASK0 = Lds::MASK0;
@@ -371,7 +372,9 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
 #pragma unroll
                 for (int c = 0; c < 2; c++) {
                     uint8_t *const to = ds_out(t) + 2048 * kb + 1024 * c + (uint32_t)((32 * (ln & 31) + 16 * (ln >> 5)) ^ (128 * c));
-                    __builtin_nontemporal_store(u32x4{pw[4 * c], pw[4 * c + 1], pw[4 * c + 2], pw[4 * c + 3]}, (u32x4 *)to);
+                    const u32x4 x = {pw[4 * c], pw[4 * c + 1], pw[4 * c + 2], pw[4 * c + 3]};
+                    if constexpr (DSM == 2) __builtin_nontemporal_store(x, (u32x4 *)to);
+                    else *(u32x4 *)to = x;
                 }
             }
             phase();
@@ -463,10 +466,10 @@ __device__ __forceinline__ void bwd_tile(const BwdParams p, int lin, int total, 
 // LDS for 80 instead of 48 KiB of dS per compute unit, +9 us; dS through registers, 96 ... 160 KiB, +30 ... +100 us; the next
 // step's requests behind this one's LDS reads +5 us; two stages and four workgroups per compute unit +30 us).
 // dS lies as [plane][128 queries][64 keys][halves of 32 keys][32 queries][32 keys]: what a workgroup here reads in a step is 8 KiB
-// in a row, and what a wave of the key pass stores of a chunk 4 KiB (pieces of 2 KiB 4 KiB apart before: causal 498 -> 493 us).  It is
-// stored past L2, where Q and dO are read again and again (key pass 1156 -> 1141 us, reads from beyond L2 1.4 -> 0.76 GB;
-// this pass 493 -> 487), and the planes are walked from the last one the key pass wrote, whose dS the memory-side cache still
-// holds (520 -> 498).  All three together: every key 941 -> 741 us.  In the 2 KiB of the last two,
+// in a row, and what a wave of the key pass stores of a chunk 4 KiB (pieces of 2 KiB 4 KiB apart before: causal 498 -> 493 us).  Where
+// there is more of it than the caches hold (kDsFar) it is stored past L2, where Q and dO are read again and again (key pass 1156 -> 1141 us,
+// reads from beyond L2 1.4 -> 0.76 GB; this pass 493 -> 487), and the planes are walked from the last one the key pass wrote, whose dS the
+// memory-side cache still holds (520 -> 498).  All three together: every key 941 -> 741 us.  In the 2 KiB of the last two,
 // key k's queries 8g + 4h .. + 3 are the 8 bytes at 1024 (g / 2) + ((32 k + 16 h) ^ 128 (g / 2)) + 8 (g & 1): the key
 // pass stores 1 KiB per instruction, and a transposing read (four keys, two groups of 16 queries) meets no bank twice.
 // A block that the key pass did not visit holds whatever the memory held: none of its entries attends, so it lies in
@@ -486,7 +489,7 @@ __device__ __forceinline__ void bwd_dq_tile(const BwdParams &p, int lin, int tot
     const int tid = threadIdx.x, lane = tid & 63, wave_u = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, hh = lane >> 5;
     const BwdPlace at = bwd_place(p, lin, total);
-    const int plane = p.planes - 1 - at.plane /* (last written first) */, rt = at.rt, bh = p.plane0 + plane;
+    const int plane = p.far ? p.planes - 1 - at.plane /* (last written first) */ : at.plane, rt = at.rt, bh = p.plane0 + plane;
     const int b = bh / p.H, h = bh - b * p.H;
     const uint16_t *ybase = p.y + b * p.ys[0] + h * p.ys[1];
     const int32_t *fid = p.full_ids + b * p.fis[0] + h * p.fis[1] + rt * p.fis[2];
@@ -605,19 +608,19 @@ __global__ __launch_bounds__(256, D == 64 && PK ? 3 : 2) void sparse_bwd_kernel(
         lin = id - l.first[1];
     }
     if (pass == 0) {
-        if (lin < l.tiles[0]) bwd_tile<DT, D, D == 64 ? kDKV : kDK, PK, 0, false, ORD>(l.pass[0], lin, l.tiles[0], smem, counts);
+        if (lin < l.tiles[0]) bwd_tile<DT, D, D == 64 ? kDKV : kDK, PK, 0, 0, ORD>(l.pass[0], lin, l.tiles[0], smem, counts);
     } else if (D == 64 || pass == 1) {
-        if (lin < l.tiles[1]) bwd_tile<DT, D, kDQ, PK, 1, false, ORD>(l.pass[1], lin, l.tiles[1], smem, counts);
+        if (lin < l.tiles[1]) bwd_tile<DT, D, kDQ, PK, 1, 0, ORD>(l.pass[1], lin, l.tiles[1], smem, counts);
     } else {
-        if constexpr (D != 64) bwd_tile<DT, D, kDV, PK, 2, false, ORD>(l.pass[2], lin, l.tiles[2], smem, counts);
+        if constexpr (D != 64) bwd_tile<DT, D, kDV, PK, 2, 0, ORD>(l.pass[2], lin, l.tiles[2], smem, counts);
     }
 }
 
-// dK, dV and dS from one walk over the keys' lists.
-template <int DT>
+// dK, dV and dS from one walk over the keys' lists.  FAR: dS is larger than the caches (kDsFar) and stored past L2.
+template <int DT, bool FAR>
 __global__ __launch_bounds__(256, 2) void sparse_bwd_keys_kernel(const BwdLaunch l) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
-    bwd_tile<DT, 128, kDKV, true, 0, true>(l.pass[0], blockIdx.x, l.tiles[0], smem);
+    bwd_tile<DT, 128, kDKV, true, 0, FAR ? 2 : 1>(l.pass[0], blockIdx.x, l.tiles[0], smem);
 }
 
 // dQ from the stored dS.  LDS: [K, four stages][dS, four stages][mask words of four entries][list]
@@ -764,10 +767,10 @@ hipError_t launch_bwd_one(const BwdParams &dq, const BwdParams &dk, const BwdPar
 
 // The planes in groups of `group`, whose dS takes its turn in the workspace.  (The key tiles of a group in one launch with the
 // query tiles of the group before, dealt out evenly: 2 ... 15 % slower than launches of their own, with 2 ... 8 groups.)
-template <int DT>
+template <int DT, bool FAR>
 hipError_t launch_bwd_ds(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, uint8_t *ds, int group, hipStream_t stream) {
     constexpr int smem = BwdLds<128, true>::bytes;
-    auto kern = sparse_bwd_keys_kernel<DT>;
+    auto kern = sparse_bwd_keys_kernel<DT, FAR>;
     static unsigned long long attr_done = 0;
     if (const hipError_t e0 = allow_dynamic_smem(kern, smem, attr_done); e0 != hipSuccess) return e0;
     auto kern_q = sparse_bwd_queries_kernel<DT, 128>;
@@ -784,6 +787,7 @@ hipError_t launch_bwd_ds(const BwdParams &dq, const BwdParams &dk, const BwdPara
             p->plane0 = p0;
             p->planes = planes - p0 < group ? planes - p0 : group;
             p->ds = ds;
+            p->far = FAR;
         }
         l.tiles[0] = l.pass[0].planes * dk.nR;
         hipLaunchKernelGGL(kern, dim3((unsigned)l.tiles[0]), dim3(256), smem, stream, l);
@@ -826,6 +830,14 @@ int bwd_ds_group(int B, int H, int Sq, int Sk, int D, size_t bytes) {
     n = (planes + groups - 1) / groups;  // groups of even size
     return n * (Sk / 128) < kLeastTiles ? 0 : (int)n;
 }
+
+// dS of a group of more bytes, four times the memory-side cache, goes past L2 and is read from the planes written last (bwd_dq_tile).  Backward
+// with prepare in us, dS through the caches in the order of planes | past them:
+//   0.27 GB  B2 H16 S2048 causal 154 | 172, every key 209 | 206     0.54  B1 H16 S4096 causal 248 | 258, window of 1024 keys 116 | 123
+//   1.07     B1 H8 S8192 window of 2048 205 | 209, B2 H16 S4096 causal 438 | 421, documents 153 | 158, every key 846 | 820
+//   1.6      B3 H16 S4096 causal 691 | 660, documents 234 | 226     2.1  B4 H16 S4096 causal 884 | 859, documents 299 | 287
+//   4.3      B8 H16 S4096 causal 1743 | 1700, documents 557 | 547, every key 3103 | 2935
+constexpr int64_t kDsFar = (int64_t)1 << 30;
 
 // At most 4 GiB, a seventieth of the device's memory.
 size_t bwd_ds_bytes(int B, int H, int Sq, int Sk, int D) {
@@ -882,8 +894,9 @@ BwdOrderParams bwd_order(const BwdParams &dq, const BwdParams &dk, const BwdPara
 
 hipError_t launch_bwd(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, int dtype, int D, uint8_t *ds, int group, const BwdOrderParams &order, hipStream_t stream) {
     if (group > 0) {
-        if (dtype == 0) return launch_bwd_ds<0>(dq, dk, dv, ds, group, stream);
-        return launch_bwd_ds<1>(dq, dk, dv, ds, group, stream);
+        const bool far = (int64_t)group * dq.nR * dk.nR * (128 * 128 * 2) > kDsFar;
+        if (dtype == 0) return far ? launch_bwd_ds<0, true>(dq, dk, dv, ds, group, stream) : launch_bwd_ds<0, false>(dq, dk, dv, ds, group, stream);
+        return far ? launch_bwd_ds<1, true>(dq, dk, dv, ds, group, stream) : launch_bwd_ds<1, false>(dq, dk, dv, ds, group, stream);
     }
     const bool pk = dq.packed != nullptr && dk.packed != nullptr;  // (with only one of them the mask is there too)
 #define SA_BWD(DT, DD) \

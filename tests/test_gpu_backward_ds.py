@@ -1,5 +1,7 @@
 """The backward whose dQ comes from stored dS (D = 128, packed tiles, 512 key tiles and more): masks with blocks no pass visits,
 a query without a key and a key without a query, one group of planes and several."""
+import math
+
 import pytest
 import torch
 
@@ -60,3 +62,37 @@ def test_planes_in_groups(gpu):
     for x, y in zip(got, want):
         assert torch.isfinite(x).all()
         assert _rel(x, y) <= 6.4e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_past_the_caches_or_through_them(gpu, dtype):
+    """33 planes of 32 MiB of dS: more than 1 GiB in one group, which goes past the caches from the last plane on, or in groups of
+    seventeen and sixteen, which do not.  The same bits."""
+    B, H, S, D = 1, 33, 4096, 128
+    lib, st, plane = _native.load(), _native.strides, S * S * 2
+    g = torch.Generator(device=gpu).manual_seed(2)
+    q, k, v, do = (torch.randn(B, H, S, D, device=gpu, generator=g, dtype=dtype) for _ in range(4))
+    i = torch.arange(S, device=gpu)
+    mask = ((i[None] <= i[:, None]) & (i[:, None] - i[None] < 900))[None, None].expand(B, H, S, S)
+    o, lse = sparse_attention(q, k, v, mask, 128, 64, return_lse=True)
+    bmd = compute_backward_metadata(mask)
+    lists, packs = [], []
+    for md in (bmd.by_query, bmd.by_key):
+        for t in (md.unmasked_kv_ids, md.unmasked_lens, md.masked_kv_ids, md.masked_lens):
+            lists += [t.data_ptr(), st(t.stride())]
+        packs += [md.packed_masks.data_ptr(), st(md.packed_masks.stride()[:2])]
+
+    def gradients(planes):
+        nbytes = lib.sa_bwd_workspace_bytes_within(B, H, S, S, D, planes * plane + B * H * S * 8 + 1024)
+        assert planes * plane < nbytes <= planes * plane + B * H * S * 8 + 1024
+        out, ws = [torch.full_like(t, float("nan")) for t in (q, k, v)], torch.full((nbytes,), 0xFF, dtype=torch.uint8, device=gpu)
+        tensors = [x for t in (q, k, v, o, do, lse, *out) for x in (t.data_ptr(), st(t.stride()))]
+        _native.check(lib.sa_sparse_attention_bwd(*tensors, None, None, None, None, *packs, *lists, ws.data_ptr(), nbytes, B, H, S, S, D,
+                                                  _native.SA_DTYPE_BF16 if dtype == torch.bfloat16 else _native.SA_DTYPE_FP16,
+                                                  D ** -0.5 / math.log(2), torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        return out
+
+    want = gradients(33)
+    assert not any(torch.isnan(t).any() for t in want)
+    assert all(torch.equal(a, b) for a, b in zip(gradients(17), want))
