@@ -854,14 +854,15 @@ size_t bwd_ds_bytes(int B, int H, int Sq, int Sk, int D) {
 //   D = 64   documents B4 H12 S2048 70.7 | 57.9, B8 H12 S1024 70.9 | 57.7, B4 H17 S1024 58.2 | 44.7, B8 H24 S512 50.7 | 46.8, B2 H12 S4096 74.0 | 62.7
 //            causal B4 H12 S2048 120 | 105, B4 H17 S1024 56.5 | 48.0   blocks B4 H12 S2048 111 | 101   every key 177 | 179, B8 H12 S1024 96.5 | 97.7
 //            window of a quarter B4 H12 S2048 68.5 | 65.8, B8 H12 S1024 49.6 | 49.4, B8 H24 S512 40.1 | 40.4, of 64 keys there 35.2 | 37.1
-//            left as it is: causal B1 H8 S8192 301 | 348, window of half B2 H8 S4096 97.7 | 102
-//   D = 128  documents B4 H8 S1024 51.6 | 47.3, B2 H12 S2048 70.8 | 65.3   causal B4 H8 S1024 54.1 | 49.9, B2 H12 S2048 134 | 120   blocks 132 | 123
+//            from a bool mask (with a transposed copy) documents B2 H12 S4096 91.5 | 76.4, causal 232 | 216
+//            left as it is: causal B1 H8 S8192 301 | 348, window of half B2 H8 S4096 97.7 | 102, documents from a bool mask there 79.1 | 90.3
+//   D = 128  documents B4 H8 S1024 51.6 | 47.3, B2 H12 S2048 70.8 | 65.3   causal B4 H8 S1024 54.1 | 49.9, B2 H12 S2048 134 | 120, B1 H16 S3072 175 | 161
 //            every key B4 H8 S1024 74.2 | 74.1, window of a quarter 39.2 | 40.2   (B1 H64 S512, left as it is: 45.0 | 46.1, window 32.3 | 33.9)
 size_t bwd_order_bytes(int B, int H, int Sq, int Sk, int D) {
     const int64_t planes = (int64_t)B * H, tq = planes * (Sq / 128), tk = planes * (Sk / 128), all = tq + tk * (D == 64 ? 1 : 2);
     const int shortest = Sq < Sk ? Sq : Sk, longest = Sq < Sk ? Sk : Sq;
     if (tq % 8 || tk % 8 || all <= (D == 64 ? 960 : 640) || all > 8 * kOrderMost) return 0;
-    if (shortest < (D == 64 ? 512 : 1024) || tq < (D == 64 ? 384 : 192) || planes < (longest > 2048 ? 24 : 16)) return 0;
+    if (shortest < (D == 64 ? 512 : 1024) || tq < (D == 64 ? 384 : 192) || planes < (longest > 3072 ? 24 : 16)) return 0;
     if ((planes + 7) / 8 * 2 * ((int64_t)Sq + Sk) * D * 2 > (8 << 20)) return 0;
     return (size_t)all * 4;
 }

@@ -1357,9 +1357,7 @@ int sa_sparse_attention_bwd(const void *q, const int64_t q_strides[4], const voi
     bp.out_scale = 1.f;
     // where nothing else is behind the statistics, the order of the tiles may be
     const size_t order_bytes = group > 0 ? 0 : sa_bwd_order_bytes(B, H, Sq, Sk, D);
-    // (from a bool mask long planes stay in their order, where neighbouring tiles read the same lines of it: bwd_order_bytes)
-    const bool pays = (q_packed && k_packed) || (Sq <= 2048 && Sk <= 2048);
-    if (order_bytes != 0 && pays && workspace_bytes >= need + order_bytes)
+    if (order_bytes != 0 && workspace_bytes >= need + order_bytes)
         pp.order = sa::bwd_order(dq_pass, dk_pass, bp, D, reinterpret_cast<int32_t *>(static_cast<uint8_t *>(workspace) + need));
     hipError_t e = sa::launch_bwd_prepare(pp, dtype, D, hs);
     if (e == hipSuccess) e = sa::launch_bwd(dq_pass, dk_pass, bp, dtype, D, ds, group, pp.order, hs);

@@ -58,7 +58,7 @@ def backward(gpu, D, B, H, Sq, Sk, packed, kind, dtype):
     (64, 4, 32, 512, 512, True, "all", torch.bfloat16), (64, 4, 32, 512, 512, True, "documents", torch.float16),
     (64, 1, 128, 512, 512, False, "random", torch.float16), (128, 4, 8, 1024, 1024, True, "documents", torch.bfloat16),
     (128, 1, 32, 1024, 1280, False, "random", torch.bfloat16), (128, 1, 32, 1024, 1024, True, "random", torch.float16),
-    (128, 2, 8, 2048, 2048, False, "documents", torch.float16)])
+    (128, 2, 8, 2048, 2048, False, "documents", torch.float16), (64, 2, 12, 4096, 4096, False, "documents", torch.bfloat16)])
 def test_tiles_by_length(gpu, D, B, H, Sq, Sk, packed, kind, dtype):
     gradients = backward(gpu, D, B, H, Sq, Sk, packed, kind, dtype)
     want, _ = gradients(False, 0)
@@ -70,13 +70,6 @@ def test_tiles_by_length(gpu, D, B, H, Sq, Sk, packed, kind, dtype):
     assert not any(torch.isnan(t).any() for t in want)
 
 
-def test_long_planes_from_a_bool_mask_stay_in_the_order_of_planes(gpu):
-    gradients = backward(gpu, 64, 2, 12, 4096, 4096, False, "documents", torch.bfloat16)
-    got, order = gradients(True, 255)
-    assert (order == 255).all()
-    assert all(torch.equal(a, b) for a, b in zip(got, gradients(False, 0)[0]))
-
-
 def test_what_stays_in_the_order_of_planes():
     f = _native.load().sa_bwd_order_bytes
     assert f(4, 12, 2048, 2048, 64) == 4 * 1536
@@ -86,6 +79,6 @@ def test_what_stays_in_the_order_of_planes():
     assert f(8, 32, 256, 256, 64) == 0     # lists of four entries at most
     assert f(2, 8, 2048, 2048, 128) > 0 and f(1, 64, 512, 512, 128) == 0  # D = 128: of eight at most
     assert f(1, 8, 8192, 8192, 64) == 0 and f(1, 8, 4096, 4096, 128) == 0  # a XCD has one plane
-    assert f(2, 12, 4096, 4096, 64) > 0 and f(2, 8, 4096, 4096, 64) == 0  # two long ones
+    assert f(2, 12, 4096, 4096, 64) > 0 and f(2, 8, 4096, 4096, 64) == 0 and f(1, 16, 3072, 3072, 128) > 0  # two long ones
     assert f(1, 48, 1024, 4096, 64) > 0 and f(1, 32, 512, 4096, 64) == 0  # the sort takes longer than the statistics
     assert f(0, 1, 128, 128, 64) == 0 and f(1, 64, 1000, 1024, 64) == 0 and f(1, 64, 1024, 1024, 96) == 0
