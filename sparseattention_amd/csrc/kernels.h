@@ -48,7 +48,7 @@ struct ClassifyRowsParams {
     int64_t ob, oh;
 };
 // The rule: mask_classify.hip.  The mask must suit the wide kernel, `packed` and its plane strides even addresses.
-bool classify_rows_has(const ClassifyParams &p);
+bool classify_rows_has(const ClassifyParams &p, int copies, bool packing);
 hipError_t launch_classify_rows(const ClassifyRowsParams &p, hipStream_t stream);
 
 // Q tiles dealt out to G persistent workgroups (G a multiple of 8, G/8 <= 64).  Workgroup g = 8*j + x is taken

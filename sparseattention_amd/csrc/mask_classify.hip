@@ -194,15 +194,16 @@ __global__ __launch_bounds__(256) void pack_partial_kernel(const PackParams p) {
 }
 
 // The three steps above in one launch, a launch's latency each for masks of few bytes per Q tile: grid (nQ, distinct planes),
-// a workgroup of eight waves makes everything of one Q tile and the tiles' states stay in LDS.
+// a workgroup of eight waves (SLAB: sixteen) makes everything of one Q tile and the tiles' states stay in LDS.
 //   rows     16 bytes per lane and row, as classify_wide_kernel; column blocks of 64 lanes are dealt to the waves, and where
 //            there are fewer than eight of them the rows of one are shared by several waves.  Rows of 16, 32 .. 512 bytes
 //            go several to a wave instruction.
 //   lists    wave 0 writes the FULL list, wave 1 the PARTIAL one, wave 2 + 3 the next output plane's ...
-//   packing  16 mask bytes, just read and in L2, become 16 bits per thread and step.
+//   packing  16 mask bytes (just read and in L2, in the form for small slabs) become 16 bits per thread and step.
 // SLAB is the form for slabs of megabytes, bound by HBM: sixteen waves, each with two column blocks side by side and eight rows of
 // both in flight, so that a workgroup has up to 256 KiB requested and reads its slab from front to back, by streaming loads.  1 GiB
-// of a window's mask with lists and packed tiles 190 -> 166 us (6.5 TB/s), all PARTIAL 816 -> 434 us: its bits come out of the L2s.
+// of a window's mask with lists and packed tiles 190 -> 166 us (6.5 TB/s), all PARTIAL 816 -> 434 us: PARTIAL tiles are read a second
+// time, when the whole slab has been read, from beyond the L2s (a slab is as large as one, and some 32 workgroups share it).
 constexpr int kRowsTiles = 2048;           // KV tiles of a Q tile that LDS holds
 constexpr int64_t kSmallSlab = 512 * 1024;  // mask bytes of a Q tile past which it is the SLAB form
 template <bool SLAB>
@@ -288,7 +289,7 @@ __global__ __launch_bounds__(SLAB ? 1024 : 512) void classify_rows_kernel(const 
         }
     }
     __syncthreads();
-    // even waves the FULL list, odd ones the PARTIAL list, of every fourth output plane each
+    // even waves the FULL list, odd ones the PARTIAL list, of every (kRowsWaves / 2)-th output plane each
     {
         const int nb = l.bcast_b ? l.oB : 1, nh = l.bcast_h ? l.oH : 1;
         const unsigned want = (wave & 1) ? 3u : 1u;
@@ -372,17 +373,30 @@ hipError_t launch_pack(const PackParams &p, hipStream_t stream) {
 //   512 KiB x 128 (causal S8192)                     19.0 | 13.5   512 KiB x 256, all PARTIAL 97 | 51
 //   256 KiB x 64, all PARTIAL                        17.7 | 15.9   256 KiB x 512, all PARTIAL 76 | 42
 // and beyond the rule 256 KiB x 16 causal 9.8 | 6.9 but all PARTIAL 12.5 | 15.6, 2 MiB x 4 10.3 | 23.5.
-// Larger slabs (the SLAB form; a call at a time, with its allocations) need 128 workgroups, half of the chip's CUs:
-//   1 MiB x 128 (S8192, causal)     34.5 | 27    all PARTIAL 82 | 72     x 192 46.3 | 31.5    x 512 107.6 | 81
-//   2 MiB x 128 (S16384, causal)    66.6 | 49    all PARTIAL 174 | 143   4 MiB x 256 (S32768, window) 190 | 166, all PARTIAL 816 | 434
-//   8 MiB x 128 (256 x 1024 tiles)   333 | 199
-// and lose below: 1 MiB x 64 21.0 | 23.1, x 86 28.5 | 34.6, 4 MiB x 32 34 | 79, x 64 59 | 85.  A wave takes 1024 columns, so the rows
-// must be long enough for at least half of the sixteen waves.
-bool classify_rows_has(const ClassifyParams &p) {
+// Larger slabs (the SLAB form).  A compute unit runs one workgroup, so a launch takes rounds of 256, and one that is hardly begun costs as
+// much as a full one; a wave takes 1024 columns, so rows must be long enough for half of the sixteen waves.  Lists alone:
+//   1 MiB (128 x 8192)  x 192 35.5 | 30.3   x 256 46.0 | 40.5   x 272 49.7 | 58.8   x 320 57.1 | 62.1   x 384 67.6 | 65.7   x 768 128.7 | 120.6
+//   2 MiB (128 x 16384) x 192 76.2 | 63.8   x 257 100 | 113     x 320 121 | 125     x 384 143 | 132
+//   4 MiB (128 x 32768) x 192 136 | 148     x 240 168 | 172     x 256 182 | 169     and packed: causal 196 | 171, all PARTIAL 833 | 432
+//   64 rows: 1 MiB x 512 84.1 | 86.3        2 MiB x 300 112 | 127   x 512 182 | 170     4 MiB x 192 135 | 147   x 256 169 | 167
+// Half a round reads as fast as three launches read a mask from the memory-side cache (256 MiB), and saves two of them:
+//   1 MiB x 128 24.9 | 25.5, packed, causal 31.4 | 26.2   2 MiB x 128 54.0 | 52.4, packed 62.1 | 52.9   4 MiB x 128 93.3 | 97.4
+// (with lists of 32 planes each its own, which three launches spread over the device, 2 MiB x 128 55.2 | 58.0).  Packed tiles of 64 Ki entries
+// and more: a Q tile has few PARTIAL ones, and each is one workgroup's in the packing launch, so the one launch is always the faster one where
+// there are some: 256 x 1024 tiles of 32768 keys x 128, causal 255 | 190, window 334 | 209, of 16384 keys x 300, causal 408 | 265; where there
+// are none, or all are, up to 13 % slower (176 | 184, 538 | 562; 207 | 234).
+bool classify_rows_has(const ClassifyParams &p, int copies, bool packing) {
     const int64_t slab = (int64_t)p.BQ * p.Sk, workgroups = (int64_t)p.nQ * p.uB * p.uH;
     if (p.nK > kRowsTiles) return false;
     if (slab <= kSmallSlab) return slab <= 128 * 1024 || slab <= workgroups * 8192;
-    return workgroups >= 128 && p.Sk >= 8 * kWideCols && slab <= INT32_MAX;
+    if (slab > INT32_MAX || p.Sk < 8 * kWideCols || workgroups < 128) return false;
+    constexpr int64_t kMiB = 1 << 20;
+    const int64_t slots = (workgroups + 255) / 256 * 256;  // of the rounds the launch takes
+    if (packing && p.BQ * p.BK >= 64 * 1024) return true;
+    if (slab >= 4 * kMiB) return workgroups >= 256 && 10 * workgroups >= 9 * slots;
+    if (p.BQ < 128) return slab >= 2 * kMiB && 10 * workgroups >= 9 * slots;
+    if (workgroups >= 192) return 4 * workgroups >= 3 * slots;
+    return copies <= 8 && (slab <= kMiB ? packing : slab <= 2 * kMiB && workgroups * slab >= 256 * kMiB);
 }
 
 hipError_t launch_classify_rows(const ClassifyRowsParams &p, hipStream_t stream) {

@@ -120,7 +120,8 @@ int classify_impl(const char *who, const uint8_t *mask, const int64_t mask_strid
         kp.pls[i] = part_lens_strides[i];
     }
     hipError_t e;
-    if (wide && sa::classify_rows_has(cp)) {
+    const int copies = (bcast_b ? kp.oB : 1) * (bcast_h ? kp.oH : 1);  // planes of lists that a distinct plane of the mask gives
+    if (wide && sa::classify_rows_has(cp, copies, packed != nullptr)) {
         sa::ClassifyRowsParams rp{};
         rp.c = cp;
         rp.l = kp;
