@@ -48,18 +48,18 @@ PEAK_FP32_TFLOPS = 157.3   # MI355X dense fp32 MFMA peak, TFLOP/s
 # `bench.py --traffic-probe` and scaled by what the same counters read for the 1 GiB device copy of the same run
 # (`bench.py --traffic-summary` does the arithmetic).  profiles/hbm_traffic_all_kernels.txt holds the commands.
 TRAFFIC_BYTES = {
-    "forward, causal": (851685571, 268435456),
-    "forward, dense": (807998895, 268435456),
-    "forward, p=0.25": (1375509304, 268435456),
-    "forward, p=0.5": (2870573991, 268435456),
-    "forward, p=0.75": (2943998167, 268435456),
-    "forward, p=0.9": (1415445150, 268435456),
-    "backward, causal": (6760299478, 5242880171),
-    "forward, documents": (1726078013, 536870912),
-    "forward, composed": (1618993437, 268435456),
-    "mask_classify, composed mask 1 GiB": (1073825705, 58880),
-    "decode, 1": (4295549086, 397312),
-    "decode, 16": (1617185349, 5677056),
+    "forward, causal": (853633236, 268435456),
+    "forward, dense": (808007578, 268435456),
+    "forward, p=0.25": (1368278762, 268435456),
+    "forward, p=0.5": (2857154369, 268435456),
+    "forward, p=0.75": (2931945634, 268435456),
+    "forward, p=0.9": (1417183708, 268435456),
+    "backward, causal": (6768688003, 5242880299),
+    "forward, documents": (1726500309, 536870912),
+    "forward, composed": (1614452310, 268435669),
+    "mask_classify, composed mask 1 GiB": (1073825619, 58880),
+    "decode, 1": (4295548872, 397312),
+    "decode, 16": (1617185220, 5677056),
 }
 TRAFFIC_SOURCE = "profiles/hbm_traffic_all_kernels.txt"
 # The sources each kernel is built from.  The counters were read with kernels built from sources of the digests in
@@ -71,8 +71,8 @@ KERNEL_FILES = {
     "decode": ("sparse_decode.hip", "fwd_common.h", "kernels.h"),
     "backward": ("sparse_bwd.hip", "fwd_common.h", "kernels.h"),
 }
-TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "db3a0a081cbbd2ae", "mask_classify": "ecc32103cd758d6a", "decode": "1a84164e00e548fe",
-                                "backward": "47c8255cb462b3db"}
+TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "1aaab1fd0fe78028", "mask_classify": "2f127cde56abac51", "decode": "19b4fa5c1254a162",
+                                "backward": "c96bd3bf11bf9723"}
 
 
 def kernel_sources_sha16(which=None):

@@ -159,6 +159,7 @@ struct FwdParams {
     uint64_t tag;
     __host__ __device__ uint64_t *arrivals(int BQ) const { return reinterpret_cast<uint64_t *>(ws_ml + (int64_t)B * H * nQ * nsplit * BQ * 2); }
 };
+static_assert(sizeof(FwdParams) + 3 * sizeof(uint32_t) <= 512, "the forward's arguments with the grid's size behind them");
 
 // How many workgroups share a list of NE entries of 2^lbk keys, walked in chunks of 2^lck keys, and the first entry of
 // part s of them (s = share: the end of the list).  Entries of one chunk stay together.

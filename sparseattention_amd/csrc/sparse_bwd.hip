@@ -812,11 +812,12 @@ hipError_t launch_prepare_one(const BwdPrepParams &p, hipStream_t stream) {
 
 // dS through memory: a pass over the keys (S, dP, dK, dV) and one over the queries (dQ), against one launch of three passes
 // and 8 products.  It needs the device filled twice over by the key tiles alone (two workgroups on each of 256 compute units):
-// causal, D = 128, backward with prepare in us, dS | three passes:
+// causal, D = 128, backward with prepare in us, dS | three passes (by falling cost where that is their order):
 //   256 key tiles  B1 H32 S1024  68 |  58   B1 H8  S4096  206 |  191   B2 H8 S2048 113 | 93
-//   512            B8 H32 S256   49 |  52   B2 H16 S2048  158 |  166   B1 H16 S4096 256 | 292   B1 H8 S8192 500 | 629
-//   1024           B8 H32 S512  113 | 127   B4 H16 S2048  263 |  313   B2 H16 S4096 443 | 546
-//   4096           B8 H16 S4096 1792 | 2195;  documents of 512 B4 H16 S8192 452 | 560;  random blocks B1 H16 S4096 132 | 162
+//   512            B8 H32 S256   48 |  55   B4 H16 S1024   98 |   97   B2 H16 S2048 165 | 154   B1 H16 S4096 259 | 283   B1 H8 S8192 511 | 666
+//                  there every key B2 H16 S2048 212 | 262, random blocks 128 | 158, a window of 512 82 | 99, documents of 64 to 1024 103 | 85
+//   1024           B8 H32 S512  116 | 134   B4 H16 S2048  266 |  317   B2 H16 S4096 434 | 541
+//   4096           B8 H16 S4096 1719 | 2148, documents 551 | 747
 // D = 64 stays with its two passes: dS is as large there and its two products half as long.
 int bwd_ds_group(int B, int H, int Sq, int Sk, int D, size_t bytes) {
     constexpr int64_t kLeastTiles = 512;  // key tiles of a group
