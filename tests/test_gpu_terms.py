@@ -200,3 +200,25 @@ def test_long_rows_wide_tiles_and_odd_row_counts(gpu, Sq, Sk, BQ, BK):
     want = compute_mask_kernel(mask, BQ, BK, pack_partial=True)
     assert int(want.masked_lens.sum()) > 0
     same_metadata(md, want, BQ, BK)
+
+
+@pytest.mark.parametrize("view", ["rows", "shifted", "every other"])
+@pytest.mark.parametrize("BQ,BK,lo,hi,both_ways", [(128, 64, 64, 1024, False), (128, 16, 40, 300, False), (128, 32, 700, 2500, True),
+                                                   (128, 128, 1, 90, True), (256, 64, 64, 1024, False), (48, 64, 5, 700, True)])
+def test_one_term_with_documents(gpu, BQ, BK, lo, hi, both_ways, view):
+    """Strips of one document against rows of several, which a single term decides without their entries; more than 2048 keys, so that
+    some of the documents are read from memory again; more open strips than have their words kept; documents whose rows
+    are not aligned for wide loads, or strided."""
+    B, H, Sq, Sk = 2, 2, BQ * 3, 4608
+    dk = docs(B, Sk, BQ + hi, gpu, lo, hi)
+    if view == "shifted":
+        dk = torch.cat([dk.new_full((B, 1), -1), dk], 1)[:, 1:]
+    elif view == "every other":
+        dk = dk.repeat_interleave(2, 1)[:, ::2]
+    dq = dk[:, Sk // 2: Sk // 2 + Sq]
+    terms = [MaskTerm(same_doc=True) if both_ways else causal_term(offset=Sk // 2, same_doc=True)]
+    md = compute_mask_terms(terms, B, H, Sq, Sk, BQ, BK, dq, dk)
+    mask = materialize_mask_terms(terms, B, Sq, Sk, dq, dk, device=gpu).expand(B, H, Sq, Sk)
+    want = compute_mask_kernel(mask, BQ, BK, pack_partial=True)
+    assert int(want.masked_lens.sum()) > 0
+    same_metadata(md, want, BQ, BK)
