@@ -131,6 +131,7 @@ struct FwdParams {
     const uint8_t *packed;
     int64_t pks[2];  // bytes between packed planes along b and h (0 where the mask is broadcast)
     int nK;          // KV tiles per row of tiles (slots per Q tile in `packed`)
+    int spread;      // planes an XCD takes together, their Q tiles side by side from the last one down (fwd_spread), or 0: two by two
     // Schedule of persistent workgroups (ScheduleParams layout), or null: then one workgroup per Q tile.
     const int32_t *sched;
     int sched_G, sched_R;  // workgroups, and entries per row after the header entry
@@ -184,6 +185,8 @@ struct FwdSplitPlan {
     int nsplit = 1, chunks = 1 << 30, least = 0;
 };
 FwdSplitPlan fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus);
+// FwdParams::spread of a launch: sparse_fwd_merge.hip.
+int fwd_spread(int64_t planes, int nQ, int BQ, int64_t plane_bytes, int cus);
 // Whether a launch walks its lists in two halves (sparse_fwd_kernel<..., TW>) where they are not shared: sparse_fwd_merge.hip.
 bool fwd_in_halves(int64_t tiles, int Sk, int BQ, int BK, int D, int dtype, int cus);
 // There: chunks up to which the form without halves is no slower, if every list is known to be as short.

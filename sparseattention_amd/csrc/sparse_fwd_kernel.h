@@ -85,7 +85,8 @@ __device__ __forceinline__ void wait_vm_at_most(int n, int step) {
 // half has its own stages and its own copy of its part of the list; the second one leaves its rows in LDS, the first one adds
 // them up.  Two waves per SIMD are bound by the matrix pipe (1.8 us for a chunk of each, at D = 128), a lone one by its own
 // serial phases (0.95 us a chunk), so what halves gain is the shorter tail of an uneven launch and, at BLOCK_Q = 64, the idle SIMDs.
-template <int DT, int D, int NW, int MODE, int NS, bool PP, bool PK, bool PS, bool SP, int RGD, bool TW>
+// SD: planes of an XCD side by side (fwd_spread), in a form of its own: a launch of 20 us pays 0.3 us for another branch at its start.
+template <int DT, int D, int NW, int MODE, int NS, bool PP, bool PK, bool PS, bool SP, int RGD, bool TW, bool SD>
 __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 : 1) void sparse_fwd_kernel(const FwdParams p) {
     static_assert(!PS || (!PP && NS == 2), "persistent workgroups use the two-stage loop");
     static_assert(!SP || (!PS && !PP && D <= 128), "shared lists use the plain loop");
@@ -93,6 +94,7 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
     constexpr int DE = RGD == 2 ? 96 : D;  // elements of a row that take part
     static_assert(RGD != 2 || D == 128, "three quarters of the larger head dim");
     static_assert(!RG || (PK && !SP && !PS && !PP && D <= 128), "ragged sizes use the plain loop and packed tiles");
+    static_assert(!SD || (!SP && !PS && !PP && !TW && D <= 128 && (NW == 2 || NW == 4)), "side by side: the plain loop");
     static_assert(!TW || (!SP && !PS && !PP && !RG && NS == 2 && D <= 128), "two halves use the plain loop");
     using E = Elem<DT>;
     constexpr int ROWB = D * 2;                   // bytes per K/V row in LDS
@@ -130,7 +132,8 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
     // remap gives each XCD whole planes (every eighth pair of the (b,h)-major order) so that the Q tiles sharing one
     // K/V plane run on the XCD whose L2 already holds it.  Planes are taken two at a time with their Q tiles
     // interleaved, last Q tile first (under causal-like masks it has the longest list): the slots that finish
-    // the short tiles of one pair then pick up the long tiles of the next, which evens out the load.
+    // the short tiles of one pair then pick up the long tiles of the next, which evens out the load; or more planes at a
+    // time, side by side, which spreads the long tiles over the compute units (fwd_spread).
     // The Q tile at hand: plane (b, h), tile qt, F FULL and NE - F PARTIAL entries, T chunks.  A persistent
     // workgroup moves from tile to tile; the others keep the values they start with.
     int b, h, qt, F, NE, T;
@@ -233,20 +236,34 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
             s0 = lin / total;
             lin -= s0 * total;
         }
-        if (lin < (per << 3)) lin = (lin & 7) * per + (lin >> 3);
-        int pair = lin / (2 * p.nQ);
-        const int r = lin - pair * 2 * p.nQ;
-        // Which pairs of planes an XCD gets: every eighth one, so that a mask that differs between batch elements
-        // (whose planes are neighbours in this order) loads the XCDs alike; a contiguous range when the pairs do
-        // not divide evenly.
-        if (((p.B * p.H) & 15) == 0) {
-            const int ppx = (p.B * p.H) >> 4;  // pairs per XCD
-            const int x = pair / ppx;
-            pair = (pair - x * ppx) * 8 + x;
+        int bh, qt0;
+        if constexpr (SD) {
+            // (planes of an XCD: every eighth one, see below)
+            int i = blockIdx.x >> 3, group = 0;
+            if ((i >> 5) == 1 && (i | 31) < per) i ^= 31;  // (the second workgroups of its 32 compute units)
+            if (8 * p.spread != p.B * p.H) {
+                group = i / (p.spread * p.nQ);
+                i -= group * (p.spread * p.nQ);
+            }
+            const int below = i / p.spread;
+            bh = (group * p.spread + i - below * p.spread) * 8 + (blockIdx.x & 7);
+            qt0 = p.nQ - 1 - below;
+        } else {
+            if (lin < (per << 3)) lin = (lin & 7) * per + (lin >> 3);
+            int pair = lin / (2 * p.nQ);
+            const int r = lin - pair * 2 * p.nQ;
+            // Which pairs of planes an XCD gets: every eighth one, so that a mask that differs between batch elements
+            // (whose planes are neighbours in this order) loads the XCDs alike; a contiguous range when the pairs do
+            // not divide evenly.
+            if (((p.B * p.H) & 15) == 0) {
+                const int ppx = (p.B * p.H) >> 4;  // pairs per XCD
+                const int x = pair / ppx;
+                pair = (pair - x * ppx) * 8 + x;
+            }
+            const bool paired = 2 * pair + 1 < p.B * p.H;  // the last plane of an odd count goes alone
+            bh = 2 * pair + (paired ? (r & 1) : 0);
+            qt0 = p.nQ - 1 - (paired ? (r >> 1) : r);
         }
-        const bool paired = 2 * pair + 1 < p.B * p.H;  // the last plane of an odd count goes alone
-        const int bh = 2 * pair + (paired ? (r & 1) : 0);
-        const int qt0 = p.nQ - 1 - (paired ? (r >> 1) : r);
         const int b0 = bh / p.H, h0 = bh - b0 * p.H;
         // The queries come from HBM, the longest wait of a tile's start: requested first of all.  Then the counts and,
         // with them, the first slots of both lists (uniform addresses: scalar loads under one wait), so that the first
@@ -1353,14 +1370,14 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
 
 // HOW 0: one workgroup per Q tile, 1: persistent workgroups, 2: lists shared by workgroups (SP), 3: ragged sizes (RG; its form by the head dim),
 // 4: lists walked in two halves (TW)
-template <int DT, int D, int NW, int MODE, bool PK, int HOW, int RGD>
+template <int DT, int D, int NW, int MODE, bool PK, int HOW, int RGD, bool SD>
 hipError_t launch_form(const FwdParams &p, hipStream_t stream) {
     // Eight waves fill a CU's register file on their own, so that workgroup can have most of the LDS: 4 stages.
     constexpr int NS = NW == 8 ? 4 : 2;
     static_assert(kListCap == 2 * kPsListCap, "one long list or two short ones in the same LDS");
     constexpr int HALVES = HOW == 4 ? 2 : 1;
     constexpr int smem = HALVES * (2 * NS * 64 * D * 2 + kListCap * 4 + (HOW == 4 ? kHalvesSync : 0));  // NS stages of 64 rows for K and for V + the list(s)
-    auto kern = sparse_fwd_kernel<DT, D, NW, MODE, NS, NW == 8, PK, HOW == 1, HOW == 2, RGD, HOW == 4>;
+    auto kern = sparse_fwd_kernel<DT, D, NW, MODE, NS, NW == 8, PK, HOW == 1, HOW == 2, RGD, HOW == 4, SD>;
     static unsigned long long attr_done = 0;  // devices on which this kernel may use `smem` bytes of LDS
     if (const hipError_t e0 = allow_dynamic_smem(kern, smem, attr_done); e0 != hipSuccess) return e0;
     const unsigned grid = HOW == 1 ? (unsigned)p.sched_G
@@ -1371,10 +1388,16 @@ hipError_t launch_form(const FwdParams &p, hipStream_t stream) {
 
 template <int DT, int D, int NW, int MODE, bool PK, int HOW>
 hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
+    const auto form = [&](auto rgd) {
+        if constexpr ((HOW == 0 || HOW == 3) && D <= 128 && (NW == 2 || NW == 4)) {
+            if (p.spread != 0) return launch_form<DT, D, NW, MODE, PK, HOW, decltype(rgd)::value, true>(p, stream);
+        }
+        return launch_form<DT, D, NW, MODE, PK, HOW, decltype(rgd)::value, false>(p, stream);
+    };
     if constexpr (HOW == 3 && D == 128) {  // (D_in 112: 38.9 us, as before; 96 and less: 34.9 against 38.3)
-        if (p.D_in <= 96) return launch_form<DT, D, NW, MODE, PK, HOW, 2>(p, stream);
+        if (p.D_in <= 96) return form(std::integral_constant<int, 2>{});
     }
-    return launch_form<DT, D, NW, MODE, PK, HOW, HOW == 3 ? 1 : 0>(p, stream);
+    return form(std::integral_constant<int, HOW == 3 ? 1 : 0>{});
 }
 
 template <int DT, int D, int NW, bool PK, int HOW>

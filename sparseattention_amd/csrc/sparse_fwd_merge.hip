@@ -186,6 +186,32 @@ bool fwd_in_halves(int64_t tiles, int Sk, int BQ, int BK, int D, int dtype, int 
 //                D = 64  2 chunks  6.0 |  6.6    4  7.8 |  8.4    5  8.7 |  9.1    6  9.4 |  9.0    8 11.1 | 10.0
 int fwd_halves_least(int BQ, int D) { return BQ == 64 ? 5 : (D == 64 ? 13 : 16); }
 
+// How many of an XCD's planes are walked together, their Q tiles side by side from the last one down.  An XCD's first 32 workgroups
+// go to its 32 compute units, the next 32 to the same ones: with planes two by two and 16 Q tiles a plane the second workgroup of a unit has
+// the first one's Q tile in another plane, under a causal mask (or the documents of one batch element) a list as long, and the
+// units of the longest lists finish last, alone.  Side by side the longest lists of all planes go to different units, and the second 32 the
+// other way round (sparse_fwd_kernel), so that a unit's two lists add up to about the same.  us, two by two | side by side:
+//   causal      512 tiles  B2 H16 S2048 52.0 | 46.7   D = 64 34.7 | 30.0   B1 H16 S4096 86.5 | 80.6   B1 H8 S8192 158.4 | 147.4
+//               768  B4 H12 S2048 66.7 | 59.5, D = 64 44.8 | 36.5     1024  B4 H16 S2048 85.1 | 75.8   B8 H16 S1024 56.1 | 47.8
+//   documents   768  54.8 | 51.0, D = 64 28.5 | 23.1   1024  65.8 | 62.6   B8 H16 S1024, D = 64 32.1 | 25.8   B2 H32, BLOCK_Q 64 41.6 | 31.9
+//   every key   512  67.5 | 66.7   768 102.6 | 103.5   1024  123.3 | 123.7   blocks  512 43.7 | 45.1   768 64.0 | 64.6   1024 80.1 | 80.0
+// As many as leave their K and V in the XCD's 4 MiB of L2, two by two | those | more of them:
+//   1024 tiles, 1 MiB a plane, causal 85.1 | 75.8 | 73.3, blocks 80.1 | 80.0 | 82.9, every key 123.3 | 123.7 | 125.0
+//   2048 tiles, 1 MiB, causal 151.9 | 145.0 | 147.9, blocks 105.0 | 101.0 | 113.0, documents 137.3 | 135.8 | 140.8
+//   2048 tiles, 1/2 MiB, causal 96.6 | 92.0 | 99.2, documents 87.3 | 84.4 | 87.7; D = 64 91.8 | 85.0 | 84.2, documents 84.1 | 81.0 | 80.0
+//   4096 tiles, 2 MiB (two fit), causal 493.9 | - | 499.4, blocks 316.8 | - | 338.9, documents 315.2 | - | 348.1
+// An odd number of planes an XCD cannot be taken two by two (two XCDs shared a pair, one its long lists): then up to 6 MiB, else one by one.
+//   B1 H24 S4096 causal 113.9 | 105.5, blocks 114.7 | 113.9, documents 62.3 | 57.8   B3 H24 311 | 282, 276 | 280, 137 | 124
+//   one by one  B5 H8 S4096 187 | 179, blocks 166.3 | 166.2, documents 87.8 | 82.3   B1 H8 S16384 537 | 460, documents 69 | 75
+int fwd_spread(int64_t planes, int nQ, int BQ, int64_t plane_bytes, int cus) {
+    if (planes % 8 != 0 || planes * nQ <= cus || (BQ != 64 && BQ != 128)) return 0;  // (BLOCK_Q 32 B4 H8 S2048 causal 106.9 | 108.1)
+    const int64_t each = planes / 8, most = (each % 2 != 0 ? 6 << 20 : 4 << 20) / (plane_bytes > 0 ? plane_bytes : 1);
+    if (each <= 2) return (int)each;
+    int64_t n = most < each ? most : each;
+    while (n > 1 && each % n != 0) n--;
+    return n > 2 ? (int)n : (each % 2 != 0 ? 1 : 0);
+}
+
 hipError_t launch_fwd_merge(const FwdParams &p, int dtype, int D, int BQ, hipStream_t stream) {
     const int NW = BQ / 32, lck = dtype == 2 ? 5 : 6;
     const int64_t waves = (int64_t)p.B * p.H * p.nQ * NW * (D / 32);

@@ -479,3 +479,17 @@ def test_lists_longer_than_the_lds_copy(gpu, BK):
         assert int(md.unmasked_lens[0, 0, 0] + md.masked_lens[0, 0, 0]) > 2048
         o = sparse_attention(q, k, v, me, 128, BK, mask_metadata=md)
         assert (o.float() - want).abs().max() <= TOL
+
+
+@pytest.mark.parametrize("B,H,nQ,BQ,D", [(2, 8, 17, 64, 64), (8, 5, 8, 64, 128), (3, 8, 11, 64, 64), (16, 12, 6, 64, 64),
+                                         (24, 16, 4, 64, 128), (1, 8, 33, 128, 128), (3, 8, 12, 128, 64)])
+def test_planes_of_an_xcd_side_by_side(gpu, B, H, nQ, BQ, D):
+    """More than 256 Q tiles over planes that divide evenly over the XCDs (fwd_spread): one, two, an odd number and more planes to an
+    XCD, groups of them, a last block of 32 workgroups that is not full.  Every tile is the masked softmax of its own plane."""
+    S = nQ * BQ
+    q, k, v = W.qkv(B, H, S, D, torch.bfloat16, seed=nQ, device=gpu)
+    mask = torch.stack([W.random_block_mask(S, 32, 0.6, seed=b, device=gpu) for b in range(B)])[:, None].expand(B, H, S, S)
+    o = sparse_attention(q, k, v, mask, BQ, 32)
+    want = sdpa32(q, k, v, mask)
+    want = torch.where(mask.any(-1, keepdim=True), want, torch.zeros_like(want))
+    assert float((o.float() - want).abs().max()) <= TOL
