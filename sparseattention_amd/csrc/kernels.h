@@ -295,6 +295,7 @@ struct BwdParams {
     int plane0, planes;            // the pass covers planes plane0 .. plane0 + planes - 1 of the B * H
     uint8_t *ds;                   // workspace of dS of these planes (bwd_dq_tile), Sq * Sk elements each
     int far;                       // 1: dS of these planes is larger than the caches (kDsFar)
+    int spread;                    // planes an XCD takes together, their tiles side by side (bwd_spread), or 0: two by two
 };
 // The passes of one launch: workgroup first[i] + t has tile t of pass i.
 struct BwdLaunch {

@@ -91,6 +91,16 @@ __device__ __forceinline__ BwdPlace bwd_place_in_order(const P &p, int lin) {  /
 }
 __device__ __forceinline__ BwdPlace bwd_place(const BwdParams &p, int lin, int total) {
     const int per = total >> 3;
+    if (p.spread != 0) {  // (as in sparse_fwd_kernel<..., SD>)
+        int i = lin >> 3, group = 0;
+        if ((i >> 5) == 1 && (i | 31) < per) i ^= 31;
+        if (8 * p.spread != p.planes) {
+            group = i / (p.spread * p.nR);
+            i -= group * (p.spread * p.nR);
+        }
+        const int order = i / p.spread;
+        return {(group * p.spread + i - order * p.spread) * 8 + (lin & 7), p.first_tile_first ? order : p.nR - 1 - order};
+    }
     return bwd_place_in_order(p, lin < (per << 3) ? (lin & 7) * per + (lin >> 3) : lin);
 }
 
@@ -767,6 +777,22 @@ hipError_t launch_bwd_one(const BwdParams &dq, const BwdParams &dk, const BwdPar
 
 // The planes in groups of `group`, whose dS takes its turn in the workspace.  (The key tiles of a group in one launch with the
 // query tiles of the group before, dealt out evenly: 2 ... 15 % slower than launches of their own, with 2 ... 8 groups.)
+// How many of an XCD's planes the passes with dS walk together, their tiles side by side, heaviest under causal-like masks first: as in the forward
+// (fwd_spread) the longest lists go to different compute units then.  Up to nine planes: the caches mind it less here, where a chunk carries twice
+// the products.  An odd number that has no such divisor goes one by one, since two by two two XCDs would share a pair.  Backward with prepare, us,
+// two by two | side by side (four, where it says so, of eight or more):
+//   causal     B4 H16 S1024 97.2 | 86.4   B2 H16 S2048 169 | 154   B4 H16 S2048 268 | 254   B8 H16 S2048 523 | 483 (490)   B1 H16 S4096 264 | 256
+//              B8 H16 S4096 1675 | 1598 (1615)   B2 H16 S4096 431 | 435   B2 H16 S8192 1507 | 1480   B1 H8 S8192 516 | 481   B3 H24 S2048 320 | 278 (three 297)
+//   documents  B4 H16 S1024 97.0 | 84.5   B2 H16 S2048 140 | 131   B8 H16 S2048 373 | 346 (369)   B8 H16 S4096 734 | 713 (726)   B3 H24 S2048 253 | 188
+//   every key  B4 H16 S1024 122.5 | 119.7   B8 H16 S2048 827 | 822 (822)   B8 H16 S4096 2938 | 2967 (2947)   B3 H8 S4096 596 | 599
+// The three passes in one launch and the two at D = 64 gain nothing by it (D = 64 causal B1 H16 S4096 144 | 138, B8 H16 S1024 92.8 | 94.4).
+int bwd_spread(int planes) {
+    if (planes % 8 != 0) return 0;
+    const int each = planes / 8;
+    int n = each < 9 ? each : 9;
+    while (each % n != 0) n--;
+    return n;
+}
 template <int DT, bool FAR>
 hipError_t launch_bwd_ds(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, uint8_t *ds, int group, hipStream_t stream) {
     constexpr int smem = BwdLds<128, true>::bytes;
@@ -788,6 +814,7 @@ hipError_t launch_bwd_ds(const BwdParams &dq, const BwdParams &dk, const BwdPara
             p->planes = planes - p0 < group ? planes - p0 : group;
             p->ds = ds;
             p->far = FAR;
+            p->spread = bwd_spread(p->planes);
         }
         l.tiles[0] = l.pass[0].planes * dk.nR;
         hipLaunchKernelGGL(kern, dim3((unsigned)l.tiles[0]), dim3(256), smem, stream, l);
