@@ -30,7 +30,7 @@ UNITS = [("sparseattn_api.hip", "sparseattn_api.o", []), ("mask_classify.hip", "
          ("sparse_decode.hip", "sparse_decode.o", []), ("sparse_bwd.hip", "sparse_bwd.o", [])]
 UNITS += [("sparse_fwd_inst.hip", f"sparse_fwd_dt{dt}_pk{pk}_how{how}.o",
            [f"-DSA_FWD_DT={dt}", f"-DSA_FWD_PK={pk}", f"-DSA_FWD_HOW={how}"])
-          for dt in (0, 1) for pk in (0, 1) for how in (0, 1, 2, 3, 4) if pk or how != 3]
+          for dt in (0, 1) for pk in (0, 1) for how in (0, 1, 2, 3, 4, 5) if pk or how != 3]
 
 # -packed-fp32-ops is switched off on purpose: the compiler must not form v_pk_*_f32 from float code.
 HIPCC_FLAGS = [

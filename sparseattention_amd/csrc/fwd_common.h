@@ -314,6 +314,13 @@ __device__ __forceinline__ bool all_arrived(uint64_t *words, uint64_t tag, int m
     return all;
 }
 
+// Whether the workgroup of this word has handed over what it has.  One wave.
+__device__ __forceinline__ bool other_arrived(uint64_t *words, uint64_t tag, int other) {
+    const HandOver h(words, 8u * (uint32_t)(other + 1));
+    const u32x2 seen = __builtin_bit_cast(u32x2, h.get2(8u * (uint32_t)other));
+    return __builtin_amdgcn_readfirstlane(seen.x == (uint32_t)tag && seen.y == (uint32_t)(tag >> 32));
+}
+
 // The sum of n parts that workgroups have handed over: this wave's N blocks of 32 x 32 values, 16 a lane, the lane's four of run g of a
 // block at rows_at + part * rows_step + 1024 (4 block + g) (where a wave leaves its accumulators, 1 KiB a store), with reference value
 // (-inf: no attended key) and sum of the lane's row at state_at + part * state_step.  In the order of the parts, whoever adds.  The

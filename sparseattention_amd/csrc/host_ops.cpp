@@ -533,6 +533,14 @@ std::optional<Out> forward_impl(const Tensor &q, const Tensor &k, const Tensor &
     }
     ListsShared shared{true};
     if (code == SA_FWD_KERNEL_DEFAULT) shared = lists_shared(hints, B, H, Sq, Sk, Dk, BQ, BK, dt);
+    Tensor ws;
+    if (!shared.whole && shared.ws_bytes != 0) {
+        try {
+            ws = at::empty({(int64_t)(shared.ws_bytes / 4)}, opt_f32);
+        } catch (const c10::OutOfMemoryError &) {  // (no place for parts: one workgroup a list)
+            shared.whole = true;
+        }
+    }
     if (shared.whole) {
         check_rc(sa_sparse_attention_fwd_kernel(qc.data_ptr(), st(qc), kc.data_ptr(), st(kc), vc.data_ptr(), st(vc), o.data_ptr(), st(o),
                                                 ptr<uint8_t>(mask), st(mask), ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl),
@@ -541,8 +549,6 @@ std::optional<Out> forward_impl(const Tensor &q, const Tensor &k, const Tensor &
     } else {
         // (too few Q tiles to fill the device: lists are shared by several workgroups, which need a workspace, or walked in halves)
         const size_t ws_bytes = shared.ws_bytes;
-        Tensor ws;
-        if (ws_bytes) ws = at::empty({(int64_t)(ws_bytes / 4)}, opt_f32);
         check_rc(sa_sparse_attention_fwd_split(qc.data_ptr(), st(qc), kc.data_ptr(), st(kc), vc.data_ptr(), st(vc), o.data_ptr(), st(o),
                                                ptr<uint8_t>(mask), st(mask), ptr<int32_t>(l.fid), st(l.fid), ptr<int32_t>(l.fl), st(l.fl),
                                                ptr<int32_t>(l.pid), st(l.pid), ptr<int32_t>(l.pl), st(l.pl), ptr<uint8_t>(l.packed), st(l.packed),

@@ -181,9 +181,12 @@ __host__ __device__ inline int fwd_split_first(int NE, int lbk, int lck, int s, 
 // Whether the last workgroup of a shared list to arrive adds up its parts (all_arrived), else a second launch does: sparse_fwd_merge.hip.
 bool fwd_merges_in_launch(int tiles, int nsplit, int BQ, int D, int dtype);
 // The rule for nsplit, split_chunks and split_least: sparse_fwd_merge.hip.
+// chunks 0: every list has one assistant (fwd_assists, sparse_fwd_kernel<..., AS>), which takes the end of it where it is `least` longer.
 struct FwdSplitPlan {
     int nsplit = 1, chunks = 1 << 30, least = 0;
 };
+bool fwd_assists(int64_t planes, int nQ, int Sk, int BQ, int BK, int D, int dtype, int cus);
+constexpr int kAssistLeast = 8;
 FwdSplitPlan fwd_split_plan(int tiles, int Sk, int BQ, int D, int dtype, int cus);
 // FwdParams::spread of a launch: sparse_fwd_merge.hip.
 int fwd_spread(int64_t planes, int nQ, int BQ, int64_t plane_bytes, int cus);

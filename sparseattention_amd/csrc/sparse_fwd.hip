@@ -11,6 +11,7 @@ hipError_t launch_fwd_variant(const FwdParams &p, int D, int BQ, hipStream_t str
 SA_DECL(0, false, 0) SA_DECL(0, false, 1) SA_DECL(0, false, 2) SA_DECL(0, true, 0) SA_DECL(0, true, 1) SA_DECL(0, true, 2)
 SA_DECL(0, true, 3) SA_DECL(1, true, 3)
 SA_DECL(0, false, 4) SA_DECL(0, true, 4) SA_DECL(1, false, 4) SA_DECL(1, true, 4)
+SA_DECL(0, false, 5) SA_DECL(0, true, 5) SA_DECL(1, false, 5) SA_DECL(1, true, 5)
 SA_DECL(1, false, 0) SA_DECL(1, false, 1) SA_DECL(1, false, 2) SA_DECL(1, true, 0) SA_DECL(1, true, 1) SA_DECL(1, true, 2)
 #undef SA_DECL
 
@@ -24,6 +25,7 @@ hipError_t by_hand_out(const FwdParams &p, int D, int BQ, hipStream_t stream) {
     }
     if (p.halves) return launch_fwd_variant<DT, PK, 4>(p, D, BQ, stream);
     if (p.nsplit <= 1) return launch_fwd_variant<DT, PK, 0>(p, D, BQ, stream);
+    if (p.split_chunks == 0) return p.tag != 0 ? launch_fwd_variant<DT, PK, 5>(p, D, BQ, stream) : hipErrorInvalidValue;
     const hipError_t e = launch_fwd_variant<DT, PK, 2>(p, D, BQ, stream);
     return e != hipSuccess || p.tag != 0 ? e : launch_fwd_merge(p, DT, D, BQ, stream);
 }

@@ -85,8 +85,11 @@ __device__ __forceinline__ void wait_vm_at_most(int n, int step) {
 // half has its own stages and its own copy of its part of the list; the second one leaves its rows in LDS, the first one adds
 // them up.  Two waves per SIMD are bound by the matrix pipe (1.8 us for a chunk of each, at D = 128), a lone one by its own
 // serial phases (0.95 us a chunk), so what halves gain is the shorter tail of an uneven launch and, at BLOCK_Q = 64, the idle SIMDs.
+// AS: for launches of no more Q tiles than compute units (fwd_assists): every Q tile has a second workgroup, which takes the end of its list
+// where that is longer than the list of the tile whose compute unit it is started on, so that both units come to about the same; else
+// it ends.  The parts meet as those of shared lists do.
 // SD: planes of an XCD side by side (fwd_spread), in a form of its own: a launch of 20 us pays 0.3 us for another branch at its start.
-template <int DT, int D, int NW, int MODE, int NS, bool PP, bool PK, bool PS, bool SP, int RGD, bool TW, bool SD>
+template <int DT, int D, int NW, int MODE, int NS, bool PP, bool PK, bool PS, bool SP, int RGD, bool TW, bool SD, bool AS>
 __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 : 1) void sparse_fwd_kernel(const FwdParams p) {
     static_assert(!PS || (!PP && NS == 2), "persistent workgroups use the two-stage loop");
     static_assert(!SP || (!PS && !PP && D <= 128), "shared lists use the plain loop");
@@ -94,7 +97,8 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
     constexpr int DE = RGD == 2 ? 96 : D;  // elements of a row that take part
     static_assert(RGD != 2 || D == 128, "three quarters of the larger head dim");
     static_assert(!RG || (PK && !SP && !PS && !PP && D <= 128), "ragged sizes use the plain loop and packed tiles");
-    static_assert(!SD || (!SP && !PS && !PP && !TW && D <= 128 && (NW == 2 || NW == 4)), "side by side: the plain loop");
+    static_assert(!AS || (SP && SD && !TW && RGD == 0), "assisted: parts of two, planes side by side");
+    static_assert(!SD || ((!SP || AS) && !PS && !PP && !TW && D <= 128 && (NW == 2 || NW == 4)), "side by side: the plain loop");
     static_assert(!TW || (!SP && !PS && !PP && !RG && NS == 2 && D <= 128), "two halves use the plain loop");
     using E = Elem<DT>;
     constexpr int ROWB = D * 2;                   // bytes per K/V row in LDS
@@ -232,22 +236,45 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
         // (shared lists: the first parts of all tiles, then the second ones, ...; parts that turn out empty come last)
         const int total = SP ? p.nQ * p.B * p.H : gridDim.x, per = total >> 3;
         int lin = blockIdx.x, s0 = 0;
-        if constexpr (SP) {
+        if constexpr (SP && !AS) {
             s0 = lin / total;
             lin -= s0 * total;
         }
+        // (AS) The second workgroups of an XCD: the first of them find compute units without a tile and take the ends of the longest lists, the
+        // others come to the units in their order and go from the shortest list to the longest, that of the unit `per - 1 - tile`.
+        const int idle = 32 - per;
+        auto tile_of = [&](int i, int &second) {
+            second = i >= per;
+            if (!second) return i;
+            const int k = i - per;
+            return k < idle ? k : per - 1 - (k - idle);
+        };
         int bh, qt0;
-        if constexpr (SD) {
-            // (planes of an XCD: every eighth one, see below)
-            int i = blockIdx.x >> 3, group = 0;
-            if ((i >> 5) == 1 && (i | 31) < per) i ^= 31;  // (the second workgroups of its 32 compute units)
-            if (8 * p.spread != p.B * p.H) {
+        // (AS) Tile of the XCD whose list this one's is held against: the one on whose compute unit its second workgroup is, or where that has a
+        // unit of its own (`alone`), the first one that has to share.
+        int partner = 0;
+        bool alone = false;
+        auto side_by_side = [&](int i, int &bh_, int &qt_) {
+            int group = 0;
+            if (!AS && 8 * p.spread != p.B * p.H) {
                 group = i / (p.spread * p.nQ);
                 i -= group * (p.spread * p.nQ);
             }
             const int below = i / p.spread;
-            bh = (group * p.spread + i - below * p.spread) * 8 + (blockIdx.x & 7);
-            qt0 = p.nQ - 1 - below;
+            bh_ = (group * p.spread + i - below * p.spread) * 8 + (blockIdx.x & 7);
+            qt_ = p.nQ - 1 - below;
+        };
+        if constexpr (SD) {
+            // (planes of an XCD: every eighth one, see below)
+            int i = blockIdx.x >> 3;
+            if constexpr (AS) {
+                i = tile_of(i, s0);
+                alone = i < idle;
+                partner = alone ? min(idle, per - 1) : per - 1 - i;
+            } else if ((i >> 5) == 1 && (i | 31) < per) {
+                i ^= 31;  // (the second workgroups of its 32 compute units)
+            }
+            side_by_side(i, bh, qt0);
         } else {
             if (lin < (per << 3)) lin = (lin & 7) * per + (lin >> 3);
             int pair = lin / (2 * p.nQ);
@@ -271,7 +298,71 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
         // past a count hold anything; early_entry() picks the ones that count.
         const int32_t *const fl0 = p.full_lens + (b0 * p.fls[0] + h0 * p.fls[1] + qt0 * p.fls[2]);
         const int32_t *const pl0 = p.part_lens + (b0 * p.pls[0] + h0 * p.pls[1] + qt0 * p.pls[2]);
-        if (SP || half == 1) {
+        if constexpr (AS) {
+            // (the counts of both tiles and the first slots in one round trip; the second workgroup's slots by another, when it stays)
+            int pbh, pqt;
+            if (alone) {
+                side_by_side(partner, pbh, pqt);
+            } else {  // (partner and tile add up to `per - 1`: the other end of the Q tiles, of the planes)
+                pbh = 8 * (p.spread - 1) + 2 * (int)(blockIdx.x & 7) - bh;
+                pqt = p.nQ - 1 - qt0;
+            }
+            const int pb = pbh / p.H, ph = pbh - pb * p.H;
+            if (s0 == 0) load_q(b0, h0, qt0);
+            const int32_t *addr[4 + 2 * EPC];
+            int got[4 + 2 * EPC];
+            addr[0] = fl0;
+            addr[1] = pl0;
+            addr[2] = p.full_lens + (pb * p.fls[0] + ph * p.fls[1] + pqt * p.fls[2]);
+            addr[3] = p.part_lens + (pb * p.pls[0] + ph * p.pls[1] + pqt * p.pls[2]);
+            static_for<EPC>([&](auto i_c) {
+                constexpr int i = decltype(i_c)::value;
+                const int slot = i < p.nK ? i : p.nK - 1;
+                addr[4 + i] = p.full_ids + b0 * p.fis[0] + h0 * p.fis[1] + qt0 * p.fis[2] + (int64_t)slot * p.fis[3];
+                addr[4 + EPC + i] = p.part_ids + b0 * p.pis[0] + h0 * p.pis[1] + qt0 * p.pis[2] + (int64_t)slot * p.pis[3];
+            });
+            scalar_gather(addr, got);
+            static_for<EPC>([&](auto i_c) {
+                constexpr int i = decltype(i_c)::value;
+                early_f[i] = got[4 + i];
+                early_p[i] = got[4 + EPC + i];
+            });
+            set_item(b0, h0, qt0, got[0], got[1]);
+            const int other = chunks_of(clamp_full(got[2]) + clamp_part(got[2], got[3]));
+            // chunks that go to the second workgroup
+            const int end = alone ? (T > other && T >= p.split_least ? T >> 1 : 0) : (T - other >= p.split_least ? (T - other) >> 1 : 0);
+            const int mid = MODE == 2 ? NE - (end >> (p.lbk - 6)) : min((T - end) * EPC, NE);
+            share = mid < NE ? 2 : 1;
+            share_part = s0;
+            if (s0 >= share) return;
+            if (s0 == 0) {
+                F = min(F, mid);
+                NE = mid;
+            } else {
+                load_q(b0, h0, qt0);
+                const int f_lo = min(mid, F), p_lo = max(mid - F, 0);
+                fid += f_lo * p.fis[3];
+                pid += p_lo * p.pis[3];
+                prow += p_lo * tile_bytes;
+                const int f_left = p.nK - 1 - f_lo, p_left = p.nK - 1 - p_lo;
+                F = max(F - mid, 0);
+                NE -= mid;
+                const int32_t *addr2[2 * EPC];
+                int got2[2 * EPC];
+                static_for<EPC>([&](auto i_c) {
+                    constexpr int i = decltype(i_c)::value;
+                    addr2[i] = fid + (int64_t)min(i, f_left) * p.fis[3];
+                    addr2[EPC + i] = pid + (int64_t)min(i, p_left) * p.pis[3];
+                });
+                scalar_gather(addr2, got2);
+                static_for<EPC>([&](auto i_c) {
+                    constexpr int i = decltype(i_c)::value;
+                    early_f[i] = got2[i];
+                    early_p[i] = got2[EPC + i];
+                });
+            }
+            T = chunks_of(NE);
+        } else if (SP || half == 1) {
             // (the counts say where this workgroup's part of the list begins, so they come by a round trip of their own)
             load_q(b0, h0, qt0);
             int cnt[2];
@@ -1302,7 +1393,60 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
     }
 
     if constexpr (PP) __syncthreads();  // the late waves of the ping-pong schedule have read their last stage
-    if constexpr (SP) {
+    if constexpr (AS) {
+        if (share > 1) {
+            // The parts meet as in the form below, with two differences: who finds the other part there keeps its own in registers (nothing
+            // stored: the longest wait of the one that is last), and reads one part instead of two.
+            const int64_t first = ((int64_t)(b * p.H + h) * p.nQ + qt) * 2;
+            constexpr uint32_t rows_step = NW * 32 * D * 4, state_step = NW * 32 * 8;
+            const HandOver rows(p.ws + first * (rows_step / 4), 2 * rows_step), state(p.ws_ml + first * (state_step / 4), 2 * state_step);
+            uint64_t *const words = p.arrivals(NW * 32) + first;
+            const uint32_t rows_at = wave_u * (32 * D * 4) + 16 * lane, state_at = (wave_u * 32 + l32) * 8;
+            const float m = raise_above == kMaxSlack ? m_ref : kNegInf, l = l32 < 16 ? acc_l[0] : acc_l[1];
+            int *const there = reinterpret_cast<int *>(smem);  // (a stage nobody reads any more)
+            if (tid < 64) {
+                const bool is = other_arrived(words, p.tag, share_part ^ 1);
+                if (tid == 0) *there = is;
+            }
+            __syncthreads();
+            bool last = __builtin_amdgcn_readfirstlane(*there) != 0;
+            if (!last) {
+#pragma unroll
+                for (int db = 0; db < D / 32; db++)
+#pragma unroll
+                    for (int g = 0; g < 4; g++)
+                        rows.put(share_part * rows_step + rows_at + 1024 * (4 * db + g),
+                                 f32x4{acc[db][4 * g], acc[db][4 * g + 1], acc[db][4 * g + 2], acc[db][4 * g + 3]});
+                if (hh == 0) state.put(share_part * state_step + state_at, f32x2{m, l});
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                __syncthreads();  // every wave's rows have been handed over (and everyone has read *there)
+                if (tid < 64) {
+                    const bool all = all_arrived(words, p.tag, share_part, 2);
+                    if (tid == 0) *there = all;
+                }
+                __syncthreads();
+                last = __builtin_amdgcn_readfirstlane(*there) != 0;
+                if (!last) return;
+            } else if (tid == 0) {
+                HandOver(words, 16).put(8 * (share_part ^ 1), f32x2{0.f, 0.f});  // (its own was never set)
+            }
+            __syncthreads();  // (the stages are about to hold output rows)
+            f32x4 x[D / 8];
+            const f32x2 st = state.get2((share_part ^ 1) * state_step + state_at);
+#pragma unroll
+            for (int g = 0; g < D / 8; g++) x[g] = rows.get4((share_part ^ 1) * rows_step + rows_at + 1024u * g);
+            const float M = fmaxf(m, st.x), M0 = M == kNegInf ? 0.f : M;  // (neither saw an attended key: both weights are 0)
+            const float w = __builtin_amdgcn_exp2f(m - M0), wx = __builtin_amdgcn_exp2f(st.x - M0);
+            // in the order of the parts, whoever adds
+            auto add = [&](float mine, float other) { return share_part == 0 ? __builtin_fmaf(wx, other, w * mine) : __builtin_fmaf(w, mine, wx * other); };
+#pragma unroll
+            for (int g = 0; g < D / 8; g++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) acc[g / 4][4 * (g % 4) + e] = add(acc[g / 4][4 * (g % 4) + e], x[g][e]);
+            acc_l[0] = acc_l[1] = add(l, st.y);
+            m_ref = M0;
+        }
+    } else if constexpr (SP) {
         if (share > 1) {
             // in the order the registers hold them: whole 1 KiB runs per store instruction (add_parts, fwd_merge_kernel)
             const int64_t tile = (int64_t)(b * p.H + h) * p.nQ + qt, first = tile * p.nsplit;
@@ -1377,11 +1521,11 @@ hipError_t launch_form(const FwdParams &p, hipStream_t stream) {
     static_assert(kListCap == 2 * kPsListCap, "one long list or two short ones in the same LDS");
     constexpr int HALVES = HOW == 4 ? 2 : 1;
     constexpr int smem = HALVES * (2 * NS * 64 * D * 2 + kListCap * 4 + (HOW == 4 ? kHalvesSync : 0));  // NS stages of 64 rows for K and for V + the list(s)
-    auto kern = sparse_fwd_kernel<DT, D, NW, MODE, NS, NW == 8, PK, HOW == 1, HOW == 2, RGD, HOW == 4, SD>;
+    auto kern = sparse_fwd_kernel<DT, D, NW, MODE, NS, NW == 8, PK, HOW == 1, HOW == 2 || HOW == 5, RGD, HOW == 4, SD || HOW == 5, HOW == 5>;
     static unsigned long long attr_done = 0;  // devices on which this kernel may use `smem` bytes of LDS
     if (const hipError_t e0 = allow_dynamic_smem(kern, smem, attr_done); e0 != hipSuccess) return e0;
     const unsigned grid = HOW == 1 ? (unsigned)p.sched_G
-                                   : (unsigned)p.nQ * (unsigned)p.B * (unsigned)p.H * (HOW == 2 ? (unsigned)p.nsplit : 1u);
+                                   : (unsigned)p.nQ * (unsigned)p.B * (unsigned)p.H * (HOW == 2 || HOW == 5 ? (unsigned)p.nsplit : 1u);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(HALVES * NW * 64), smem, stream, p);
     return hipGetLastError();
 }
@@ -1402,7 +1546,7 @@ hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
 
 template <int DT, int D, int NW, bool PK, int HOW>
 hipError_t launch_mode(const FwdParams &p, hipStream_t stream) {
-    if constexpr (HOW == 4) {  // (four entries a chunk and two halves take more scalar registers than there are)
+    if constexpr (HOW >= 4) {  // (four entries a chunk and two halves take more scalar registers than there are)
         if (p.BK == 16) return hipErrorInvalidValue;
     } else if (p.BK == 16) return launch_one<DT, D, NW, 0, PK, HOW>(p, stream);
     if (p.BK == 32) return launch_one<DT, D, NW, 1, PK, HOW>(p, stream);
@@ -1413,9 +1557,11 @@ template <int DT, int D, bool PK, int HOW>
 hipError_t launch_bq(const FwdParams &p, int BQ, hipStream_t stream) {
     switch (BQ) {
         case 32:
-            if constexpr (D > 128 || HOW == 4) return hipErrorInvalidValue;  // a lone wave would spill its registers there
+            if constexpr (D > 128 || HOW >= 4) return hipErrorInvalidValue;  // a lone wave would spill its registers there
             else return launch_mode<DT, D, 1, PK, HOW>(p, stream);
-        case 64: return launch_mode<DT, D, 2, PK, HOW>(p, stream);
+        case 64:
+            if constexpr (HOW == 5) return hipErrorInvalidValue;
+            else return launch_mode<DT, D, 2, PK, HOW>(p, stream);
         case 128: return launch_mode<DT, D, 4, PK, HOW>(p, stream);
         case 256:
             // 8-wave workgroups have the plain form only, and their four stages do not fit the LDS at D = 256

@@ -178,6 +178,25 @@ bool fwd_in_halves(int64_t tiles, int Sk, int BQ, int BK, int D, int dtype, int 
     return 3 * tiles > 2 * cus && (D == 64 || 4 * tiles <= 3 * cus || tiles == cus);
 }
 
+// When every list has an assistant (sparse_fwd_kernel<..., AS>): up to one Q tile of 128 rows a compute unit, more than half as many, where neither
+// parts by the length of Sk nor halves serve.  A unit has one workgroup then, which takes 0.95 us a chunk, and the longest list ends the
+// launch.  The second workgroups of the grid land on the units in the order of the first ones, so which tile an assistant sits beside is known, and
+// the two lists' lengths say what it takes: half the difference, from eight chunks on (less does not pay for the meeting of the parts, 3 us), or
+// on a unit of its own half the list, where that is longer than the longest that has to share.  Both workgroups decide alike from the same
+// counts.  us, one workgroup a list | with assistants, bf16:
+//   causal     256 tiles  D = 128  16 chunks 22.5 | 21.1   20 24.2 | 20.2 (160 tiles)   32 36.8 | 29.0   D = 64  32 26.2 | 20.6
+//              192 tiles  16 20.7 | 18.4   48 50.3 | 35.1
+//   documents of 64 ... 1024  256 tiles 32 chunks 22.2 | 20.1, D = 64 16.5 | 14.7   192 tiles 16 17.5 | 15.9   160 tiles 20 17.4 | 15.8
+//   every key  256 tiles 16 24.9 | 25.4   32 41.5 | 41.3, D = 64 27.0 | 27.4   192 tiles 16 21.6 | 22.2   48 52.3 | 52.6
+//   blocks     256 tiles 16 24.0 | 24.3   32 36.5 | 36.8   window of 200 keys 16 13.6 | 14.2   32 13.0 | 13.7   (nothing to assist: the second tile's counts)
+//   16 chunks at D = 64: causal 16.7 | 15.9, every key 17.7 | 18.4.  12 chunks: causal 17.1 | 17.5.
+// From 49 chunks on halves stay: causal 64 chunks of S4096 54.1 | 46.6, but every key 68.0 | 77.6, causal Sq 2048 Sk 4096 61.0 | 66.9.
+bool fwd_assists(int64_t planes, int nQ, int Sk, int BQ, int BK, int D, int dtype, int cus) {
+    const int64_t tiles = planes * nQ;
+    const int chunks = (Sk + 63) / 64;
+    return dtype != 2 && (D == 64 || D == 128) && BQ == 128 && BK >= 32 && cus == 256 && planes % 8 == 0 && 2 * tiles > cus && tiles <= cus && chunks >= (D == 64 ? 24 : 16) && chunks <= 48;
+}
+
 // A caller who knows that all lists are short does without the wider workgroup: us, one workgroup of half the waves | halves, 256 tiles,
 // every list as long as stated (kept whole by the first half up to 10 chunks, at BLOCK_Q 64 up to 4: sparse_fwd_kernel's LEAST)
 //   BLOCK_Q 128          4 chunks  9.7 | 10.8    8 13.6 | 14.9   12 18.0 | 19.0   14 20.5 | 21.1   16 22.4 | 22.6   20 26.6 | 26.2

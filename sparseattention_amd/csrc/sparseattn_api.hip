@@ -289,7 +289,13 @@ size_t split_shape(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtyp
     if (hipGetDevice(&dev) != hipSuccess) return 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
     if (tiles > 2 * cus || sa::fwd_in_halves(tiles, Sk, BQ, BK, D, dtype, cus)) return 0;
-    *plan = sa::fwd_split_plan((int)tiles, Sk, BQ, D, dtype, cus);
+    if (sa::fwd_assists((int64_t)B * H, Sq / BQ, Sk, BQ, BK, D, dtype, cus)) {
+        plan->nsplit = 2;
+        plan->chunks = 0;
+        plan->least = sa::kAssistLeast;
+    } else {
+        *plan = sa::fwd_split_plan((int)tiles, Sk, BQ, D, dtype, cus);
+    }
     return plan->nsplit > 1 ? (size_t)tiles * (size_t)plan->nsplit * (size_t)BQ * (size_t)(D + 2) * 4 : 0;
 }
 
@@ -455,6 +461,10 @@ int forward_impl(const void *q, const int64_t q_strides[4], const void *k, const
         // (a caller who asked an earlier library for the size has no place for them: a second launch then)
         if (need != 0 && sa::fwd_merges_in_launch(B * H * fp.nQ, plan.nsplit, BQ, D, dtype) && workspace_bytes >= need + (size_t)8 * B * H * fp.nQ * plan.nsplit)
             fp.tag = next_launch_tag() | 1;  // (never 0)
+        if (plan.nsplit > 1 && plan.chunks == 0) {
+            if (fp.tag != 0) fp.spread = B * H / 8;
+            else fp.nsplit = 1;
+        }
     }
     if (kernel == SA_FWD_KERNEL_SHORT_LISTS) {
         if (f32 || !sa::fwd_c32_has(fp, dtype, D, BQ))
