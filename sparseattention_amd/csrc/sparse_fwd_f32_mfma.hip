@@ -48,7 +48,7 @@ constexpr int f32_group_bytes = 4 * 32 * D * 4 + 2 * NW * 1024 + kF32ListCap * 4
 // softmax 3.0, the groups' rows 0.4, parts handed over 0.7, all arrived 0.8, parts read and added 2.1.
 // Registers for two waves per SIMD (D = 64: results stay out of the accumulation registers; causal B2 H16 S2048 235 -> 226 us), but not at
 // D = 128 with two waves a workgroup: registers that fill a SIMD keep the waves of two workgroups on different ones (339 us against 592).
-template <int D, int NW, int MODE, bool PK, bool SP>
+template <int D, int NW, int MODE, bool PK, bool SP, bool SD>
 __global__ __launch_bounds__(NW * f32_groups(NW, SP) * 64, D == 128 && NW * f32_groups(NW, SP) <= 2 ? 1 : 2) void sparse_fwd_f32_mfma_kernel(const FwdParams p) {
     constexpr int KG = f32_groups(NW, SP);
     constexpr int ROWB = D * 4, PPR = ROWB / 16;  // bytes and 16-byte pieces per K/V row
@@ -72,7 +72,7 @@ __global__ __launch_bounds__(NW * f32_groups(NW, SP) * 64, D == 128 && NW * f32_
     // Workgroup -> (b, h, Q tile) as in sparse_fwd_kernel: the hardware hands consecutive workgroup ids to the 8 XCDs
     // in turn; the remap gives every XCD whole planes (so that the Q tiles sharing a K/V plane meet in one L2 and every
     // XCD gets the same mix of long and short lists), planes two at a time with their Q tiles interleaved, last Q tile
-    // first.
+    // first; or more planes side by side (SD, fwd_spread).
     int b, h, qt, s0 = 0;  // s0: this workgroup's part of a shared list
     {
         const int total = p.nQ * p.B * p.H, per = total >> 3;
@@ -81,17 +81,30 @@ __global__ __launch_bounds__(NW * f32_groups(NW, SP) * 64, D == 128 && NW * f32_
             s0 = lin / total;
             lin -= s0 * total;
         }
-        if (lin < (per << 3)) lin = (lin & 7) * per + (lin >> 3);
-        int pair = lin / (2 * p.nQ);
-        const int r = lin - pair * 2 * p.nQ;
-        if (((p.B * p.H) & 15) == 0) {
-            const int ppx = (p.B * p.H) >> 4;
-            const int x = pair / ppx;
-            pair = (pair - x * ppx) * 8 + x;
+        int bh;
+        if constexpr (SD) {
+            int i = blockIdx.x >> 3, group = 0;
+            if ((i >> 5) == 1 && (i | 31) < per) i ^= 31;
+            if (8 * p.spread != p.B * p.H) {
+                group = i / (p.spread * p.nQ);
+                i -= group * (p.spread * p.nQ);
+            }
+            const int below = i / p.spread;
+            bh = (group * p.spread + i - below * p.spread) * 8 + (blockIdx.x & 7);
+            qt = p.nQ - 1 - below;
+        } else {
+            if (lin < (per << 3)) lin = (lin & 7) * per + (lin >> 3);
+            int pair = lin / (2 * p.nQ);
+            const int r = lin - pair * 2 * p.nQ;
+            if (((p.B * p.H) & 15) == 0) {
+                const int ppx = (p.B * p.H) >> 4;
+                const int x = pair / ppx;
+                pair = (pair - x * ppx) * 8 + x;
+            }
+            const bool paired = 2 * pair + 1 < p.B * p.H;
+            bh = 2 * pair + (paired ? (r & 1) : 0);
+            qt = p.nQ - 1 - (paired ? (r >> 1) : r);
         }
-        const bool paired = 2 * pair + 1 < p.B * p.H;
-        const int bh = 2 * pair + (paired ? (r & 1) : 0);
-        qt = p.nQ - 1 - (paired ? (r >> 1) : r);
         b = bh / p.H;
         h = bh - b * p.H;
     }
@@ -434,10 +447,10 @@ __global__ __launch_bounds__(NW * f32_groups(NW, SP) * 64, D == 128 && NW * f32_
     else finish(std::integral_constant<int, KG - 1>{});
 }
 
-template <int D, int NW, int MODE, bool PK, bool SP>
+template <int D, int NW, int MODE, bool PK, bool SP, bool SD>
 hipError_t launch_lists(const FwdParams &p, hipStream_t stream) {
     constexpr int smem = f32_groups(NW, SP) * f32_group_bytes<D, NW>;
-    auto kern = sparse_fwd_f32_mfma_kernel<D, NW, MODE, PK, SP>;
+    auto kern = sparse_fwd_f32_mfma_kernel<D, NW, MODE, PK, SP, SD>;
     static unsigned long long attr_done = 0;
     if (const hipError_t e0 = allow_dynamic_smem(kern, smem, attr_done); e0 != hipSuccess) return e0;
     hipLaunchKernelGGL(kern, dim3((unsigned)p.nQ * (unsigned)(p.B * p.H) * (unsigned)(SP ? p.nsplit : 1)),
@@ -447,7 +460,11 @@ hipError_t launch_lists(const FwdParams &p, hipStream_t stream) {
 
 template <int D, int NW, int MODE, bool PK>
 hipError_t launch_one(const FwdParams &p, hipStream_t stream) {
-    return p.nsplit > 1 ? launch_lists<D, NW, MODE, PK, true>(p, stream) : launch_lists<D, NW, MODE, PK, false>(p, stream);
+    if (p.nsplit > 1) return launch_lists<D, NW, MODE, PK, true, false>(p, stream);
+    if constexpr (NW > 1) {
+        if (p.spread != 0) return launch_lists<D, NW, MODE, PK, false, true>(p, stream);
+    }
+    return launch_lists<D, NW, MODE, PK, false, false>(p, stream);
 }
 
 template <int D, int NW, bool PK>

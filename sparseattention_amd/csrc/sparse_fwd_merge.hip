@@ -222,6 +222,8 @@ int fwd_halves_least(int BQ, int D) { return BQ == 64 ? 5 : (D == 64 ? 13 : 16);
 // An odd number of planes an XCD cannot be taken two by two (two XCDs shared a pair, one its long lists): then up to 6 MiB, else one by one.
 //   B1 H24 S4096 causal 113.9 | 105.5, blocks 114.7 | 113.9, documents 62.3 | 57.8   B3 H24 311 | 282, 276 | 280, 137 | 124
 //   one by one  B5 H8 S4096 187 | 179, blocks 166.3 | 166.2, documents 87.8 | 82.3   B1 H8 S16384 537 | 460, documents 69 | 75
+// float32, whose chunks keep the matrix unit busy four to eight times as long: causal B2 H16 S1024 D64 144.2 | 88.9, B4 H12 148.8 | 108.0,
+// B1 H8 S4096 479 | 321, BLOCK_Q 128 B3 H8 S2048 281 | 199; documents B2 H16 S1024 120.7 | 89.2; every key 144.5 | 144.3; D = 128 B1 H16 S2048 313 | 311.
 int fwd_spread(int64_t planes, int nQ, int BQ, int64_t plane_bytes, int cus) {
     if (planes % 8 != 0 || planes * nQ <= cus || (BQ != 64 && BQ != 128)) return 0;  // (BLOCK_Q 32 B4 H8 S2048 causal 106.9 | 108.1)
     const int64_t each = planes / 8, most = (each % 2 != 0 ? 6 << 20 : 4 << 20) / (plane_bytes > 0 ? plane_bytes : 1);

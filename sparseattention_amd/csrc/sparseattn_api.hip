@@ -445,7 +445,7 @@ int forward_impl(const void *q, const int64_t q_strides[4], const void *k, const
     {
         int dev = 0, cus = 0;
         if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
-            fp.spread = sa::fwd_spread((int64_t)B * H, fp.nQ, BQ, (int64_t)Sk * D * 4, cus);  // (K and V of 16 bits)
+            fp.spread = sa::fwd_spread((int64_t)B * H, fp.nQ, BQ, (int64_t)Sk * D * (f32 ? 8 : 4), cus);
     }
     fp.halves = other_order && in_halves(B, H, Sq, Sk, D, BQ, BK, dtype);
     if (workspace && !fp.halves && kernel == SA_FWD_KERNEL_DEFAULT && !fp.sched) {

@@ -154,3 +154,15 @@ def test_sizes_of_the_matrix_unit_kernel(gpu, D, BQ, BK):
         assert torch.equal(o[:, :, 9].cpu(), torch.zeros(B, H, D))
         live = ~torch.isneginf(want_lse)
         assert torch.isneginf(lse.cpu()[~live]).all() and (lse.cpu().double()[live] - want_lse[live]).abs().max() <= 1e-5
+
+
+@pytest.mark.parametrize("B,H,nQ,BQ,D", [(2, 8, 17, 64, 64), (3, 8, 11, 64, 128), (8, 5, 8, 64, 64), (3, 8, 12, 128, 64), (1, 8, 33, 64, 64)])
+def test_planes_of_an_xcd_side_by_side(gpu, B, H, nQ, BQ, D):
+    """More than 256 Q tiles over planes that divide evenly over the XCDs (fwd_spread)."""
+    S = nQ * BQ
+    q, k, v = W.qkv(B, H, S, D, torch.float32, seed=nQ, device=gpu)
+    mask = torch.stack([W.random_block_mask(S, 32, 0.6, seed=b, device=gpu) for b in range(B)])[:, None].expand(B, H, S, S)
+    o = sparse_attention(q, k, v, mask, BQ, 32)
+    want = F.scaled_dot_product_attention(q.double(), k.double(), v.double(), attn_mask=mask)
+    want = torch.where(mask.any(-1, keepdim=True), want, torch.zeros_like(want))
+    assert float((o - want).abs().max()) <= 1e-5
