@@ -131,7 +131,7 @@ struct FwdParams {
     const uint8_t *packed;
     int64_t pks[2];  // bytes between packed planes along b and h (0 where the mask is broadcast)
     int nK;          // KV tiles per row of tiles (slots per Q tile in `packed`)
-    int spread;      // planes an XCD takes together, their Q tiles side by side from the last one down (fwd_spread), or 0: two by two
+    int spread;      // planes taken together, their Q tiles side by side from the last one down (fwd_spread), or 0: two by two
     // Schedule of persistent workgroups (ScheduleParams layout), or null: then one workgroup per Q tile.
     const int32_t *sched;
     int sched_G, sched_R;  // workgroups, and entries per row after the header entry
@@ -298,7 +298,7 @@ struct BwdParams {
     int plane0, planes;            // the pass covers planes plane0 .. plane0 + planes - 1 of the B * H
     uint8_t *ds;                   // workspace of dS of these planes (bwd_dq_tile), Sq * Sk elements each
     int far;                       // 1: dS of these planes is larger than the caches (kDsFar)
-    int spread;                    // planes an XCD takes together, their tiles side by side (bwd_spread), or 0: two by two
+    int spread;                    // planes taken together, their tiles side by side (bwd_spread), or 0: two by two
 };
 // The passes of one launch: workgroup first[i] + t has tile t of pass i.
 struct BwdLaunch {

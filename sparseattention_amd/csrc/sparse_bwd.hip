@@ -94,12 +94,13 @@ __device__ __forceinline__ BwdPlace bwd_place(const BwdParams &p, int lin, int t
     if (p.spread != 0) {  // (as in sparse_fwd_kernel<..., SD>)
         int i = lin >> 3, group = 0;
         if ((i >> 5) == 1 && (i | 31) < per) i ^= 31;
-        if (8 * p.spread != p.planes) {
-            group = i / (p.spread * p.nR);
-            i -= group * (p.spread * p.nR);
+        int n = 8 * i + (lin & 7);
+        if (p.spread != p.planes) {
+            group = n / (p.spread * p.nR);
+            n -= group * (p.spread * p.nR);
         }
-        const int order = i / p.spread;
-        return {(group * p.spread + i - order * p.spread) * 8 + (lin & 7), p.first_tile_first ? order : p.nR - 1 - order};
+        const int order = n / p.spread;
+        return {group * p.spread + n - order * p.spread, p.first_tile_first ? order : p.nR - 1 - order};
     }
     return bwd_place_in_order(p, lin < (per << 3) ? (lin & 7) * per + (lin >> 3) : lin);
 }
@@ -784,14 +785,15 @@ hipError_t launch_bwd_one(const BwdParams &dq, const BwdParams &dk, const BwdPar
 //   causal     B4 H16 S1024 97.2 | 86.4   B2 H16 S2048 169 | 154   B4 H16 S2048 268 | 254   B8 H16 S2048 523 | 483 (490)   B1 H16 S4096 264 | 256
 //              B8 H16 S4096 1675 | 1598 (1615)   B2 H16 S4096 431 | 435   B2 H16 S8192 1507 | 1480   B1 H8 S8192 516 | 481   B3 H24 S2048 320 | 278 (three 297)
 //   documents  B4 H16 S1024 97.0 | 84.5   B2 H16 S2048 140 | 131   B8 H16 S2048 373 | 346 (369)   B8 H16 S4096 734 | 713 (726)   B3 H24 S2048 253 | 188
+//   odd fours  causal B1 H12 S8192 737 | 625   B3 H12 S2048 186 | 163   B1 H4 S16384 1083 | 919   documents B3 H12 S2048 110 | 96   every key 282 | 289
 //   every key  B4 H16 S1024 122.5 | 119.7   B8 H16 S2048 827 | 822 (822)   B8 H16 S4096 2938 | 2967 (2947)   B3 H8 S4096 596 | 599
 // The three passes in one launch and the two at D = 64 gain nothing by it (D = 64 causal B1 H16 S4096 144 | 138, B8 H16 S1024 92.8 | 94.4).
 int bwd_spread(int planes) {
-    if (planes % 8 != 0) return 0;
-    const int each = planes / 8;
+    if (planes % 4 != 0) return 0;
+    const int unit = planes % 8 != 0 ? 4 : 8, each = planes / unit;
     int n = each < 9 ? each : 9;
     while (each % n != 0) n--;
-    return n;
+    return unit * n;
 }
 template <int DT, bool FAR>
 hipError_t launch_bwd_ds(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, uint8_t *ds, int group, hipStream_t stream) {

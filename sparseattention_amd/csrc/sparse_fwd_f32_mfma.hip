@@ -85,12 +85,14 @@ __global__ __launch_bounds__(NW * f32_groups(NW, SP) * 64, D == 128 && NW * f32_
         if constexpr (SD) {
             int i = blockIdx.x >> 3, group = 0;
             if ((i >> 5) == 1 && (i | 31) < per) i ^= 31;
-            if (8 * p.spread != p.B * p.H) {
-                group = i / (p.spread * p.nQ);
-                i -= group * (p.spread * p.nQ);
+            int n = 8 * i + (blockIdx.x & 7);
+            if (p.spread != p.B * p.H) {
+                group = n / (p.spread * p.nQ);
+                n -= group * (p.spread * p.nQ);
             }
-            const int below = i / p.spread;
-            bh = (group * p.spread + i - below * p.spread) * 8 + (blockIdx.x & 7);
+            int below = n / p.spread;
+            bh = group * p.spread + n - below * p.spread;
+            if ((p.spread & 4) != 0 && (below | 1) < p.nQ) below ^= (below >> 1) & 1;
             qt = p.nQ - 1 - below;
         } else {
             if (lin < (per << 3)) lin = (lin & 7) * per + (lin >> 3);

@@ -254,18 +254,22 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
         // unit of its own (`alone`), the first one that has to share.
         int partner = 0;
         bool alone = false;
-        auto side_by_side = [&](int i, int &bh_, int &qt_) {
-            int group = 0;
-            if (!AS && 8 * p.spread != p.B * p.H) {
-                group = i / (p.spread * p.nQ);
-                i -= group * (p.spread * p.nQ);
+        auto side_by_side = [&](int i, int &bh_, int &qt_) {  // i: the XCD's i-th
+            int n = 8 * i + (blockIdx.x & 7), group = 0;
+            if (!AS && p.spread != p.B * p.H) {
+                group = n / (p.spread * p.nQ);
+                n -= group * (p.spread * p.nQ);
             }
-            const int below = i / p.spread;
-            bh_ = (group * p.spread + i - below * p.spread) * 8 + (blockIdx.x & 7);
+            int below = n / p.spread;
+            // (an odd number of fours: Q tiles 0, 3, 4, 7, 8 ... of a plane on one XCD and 1, 2, 5, 6 ... on another: as much work, and neighbours, which
+            // share keys under a window, by twos)
+            const int kept = below * p.spread;
+            if (!AS && (p.spread & 4) != 0 && (below | 1) < p.nQ) below ^= (below >> 1) & 1;
+            bh_ = group * p.spread + n - kept;
             qt_ = p.nQ - 1 - below;
         };
         if constexpr (SD) {
-            // (planes of an XCD: every eighth one, see below)
+            // (the planes of a group in turn: an XCD has every eighth one, or where they are an odd number of fours every second Q tile of every fourth)
             int i = blockIdx.x >> 3;
             if constexpr (AS) {
                 i = tile_of(i, s0);
@@ -304,7 +308,7 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
             if (alone) {
                 side_by_side(partner, pbh, pqt);
             } else {  // (partner and tile add up to `per - 1`: the other end of the Q tiles, of the planes)
-                pbh = 8 * (p.spread - 1) + 2 * (int)(blockIdx.x & 7) - bh;
+                pbh = p.spread - 8 + 2 * (int)(blockIdx.x & 7) - bh;
                 pqt = p.nQ - 1 - qt0;
             }
             const int pb = pbh / p.H, ph = pbh - pb * p.H;

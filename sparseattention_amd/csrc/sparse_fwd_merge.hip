@@ -205,7 +205,7 @@ bool fwd_assists(int64_t planes, int nQ, int Sk, int BQ, int BK, int D, int dtyp
 //                D = 64  2 chunks  6.0 |  6.6    4  7.8 |  8.4    5  8.7 |  9.1    6  9.4 |  9.0    8 11.1 | 10.0
 int fwd_halves_least(int BQ, int D) { return BQ == 64 ? 5 : (D == 64 ? 13 : 16); }
 
-// How many of an XCD's planes are walked together, their Q tiles side by side from the last one down.  An XCD's first 32 workgroups
+// How many planes are walked together (an XCD has an eighth of them, see below), their Q tiles side by side from the last one down.  An XCD's first 32 workgroups
 // go to its 32 compute units, the next 32 to the same ones: with planes two by two and 16 Q tiles a plane the second workgroup of a unit has
 // the first one's Q tile in another plane, under a causal mask (or the documents of one batch element) a list as long, and the
 // units of the longest lists finish last, alone.  Side by side the longest lists of all planes go to different units, and the second 32 the
@@ -222,15 +222,22 @@ int fwd_halves_least(int BQ, int D) { return BQ == 64 ? 5 : (D == 64 ? 13 : 16);
 // An odd number of planes an XCD cannot be taken two by two (two XCDs shared a pair, one its long lists): then up to 6 MiB, else one by one.
 //   B1 H24 S4096 causal 113.9 | 105.5, blocks 114.7 | 113.9, documents 62.3 | 57.8   B3 H24 311 | 282, 276 | 280, 137 | 124
 //   one by one  B5 H8 S4096 187 | 179, blocks 166.3 | 166.2, documents 87.8 | 82.3   B1 H8 S16384 537 | 460, documents 69 | 75
+// Planes that are an odd number of fours (12 heads, 4 heads) took two by two leave one XCD the long lists of a pair and another its short ones; side
+// by side a plane's Q tiles go to two XCDs in turn, by twos:
+//   causal B3 H12 S2048 60.9 | 54.4   B1 H4 S16384 347 | 304   B1 H12 S8192 D = 64 137 | 132   B1 H12 S4096 84.3 | 81.4   B5 H12 S1024 31.3 | 30.9
+//   documents B3 H12 S2048 37.2 | 34.3   B5 H12 S1024 29.8 | 27.9   blocks 87.5 | 86.0, 36.3 | 38.1   every key 98.8 | 99.3
+//   window of 500 keys B3 H12 S2048 37.4 | 38.4   B1 H12 S8192 D = 64 25.3 | 27.4 (one by one, not by twos: 24.1 | 25.8 for 25.0 | 25.8 at S4096)
+//   float32 B3 H12 S1152 D = 64 causal 154.5 | 110.8, documents 125.6 | 108.5
 // float32, whose chunks keep the matrix unit busy four to eight times as long: causal B2 H16 S1024 D64 144.2 | 88.9, B4 H12 148.8 | 108.0,
 // B1 H8 S4096 479 | 321, BLOCK_Q 128 B3 H8 S2048 281 | 199; documents B2 H16 S1024 120.7 | 89.2; every key 144.5 | 144.3; D = 128 B1 H16 S2048 313 | 311.
 int fwd_spread(int64_t planes, int nQ, int BQ, int64_t plane_bytes, int cus) {
-    if (planes % 8 != 0 || planes * nQ <= cus || (BQ != 64 && BQ != 128)) return 0;  // (BLOCK_Q 32 B4 H8 S2048 causal 106.9 | 108.1)
-    const int64_t each = planes / 8, most = (each % 2 != 0 ? 6 << 20 : 4 << 20) / (plane_bytes > 0 ? plane_bytes : 1);
-    if (each <= 2) return (int)each;
+    if (planes % 4 != 0 || planes * nQ <= cus || (BQ != 64 && BQ != 128)) return 0;  // (BLOCK_Q 32 B4 H8 S2048 causal 106.9 | 108.1)
+    const int unit = planes % 8 != 0 ? 4 : 8;
+    const int64_t each = planes / unit, most = (each % 2 != 0 ? 6 << 20 : 4 << 20) / (plane_bytes > 0 ? plane_bytes : 1);
+    if (each <= 2) return (int)planes;
     int64_t n = most < each ? most : each;
     while (n > 1 && each % n != 0) n--;
-    return n > 2 ? (int)n : (each % 2 != 0 ? 1 : 0);
+    return n > 2 ? (int)(unit * n) : (each % 2 != 0 ? unit : 0);
 }
 
 hipError_t launch_fwd_merge(const FwdParams &p, int dtype, int D, int BQ, hipStream_t stream) {

@@ -462,7 +462,7 @@ int forward_impl(const void *q, const int64_t q_strides[4], const void *k, const
         if (need != 0 && sa::fwd_merges_in_launch(B * H * fp.nQ, plan.nsplit, BQ, D, dtype) && workspace_bytes >= need + (size_t)8 * B * H * fp.nQ * plan.nsplit)
             fp.tag = next_launch_tag() | 1;  // (never 0)
         if (plan.nsplit > 1 && plan.chunks == 0) {
-            if (fp.tag != 0) fp.spread = B * H / 8;
+            if (fp.tag != 0) fp.spread = B * H;
             else fp.nsplit = 1;
         }
     }

@@ -98,7 +98,9 @@ def test_past_the_caches_or_through_them(gpu, dtype):
     assert all(torch.equal(a, b) for a, b in zip(gradients(17), want))
 
 
-@pytest.mark.parametrize("B,H,Sq,Sk", [(2, 8, 384, 4096), (9, 8, 128, 1024), (11, 8, 256, 768), (16, 8, 384, 512), (8, 8, 1152, 1024)])
+@pytest.mark.parametrize("B,H,Sq,Sk", [(2, 8, 384, 4096), (9, 8, 128, 1024), (11, 8, 256, 768), (16, 8, 384, 512), (8, 8, 1152, 1024),
+                                         (3, 12, 384, 1920), (1, 4, 128, 16384)])
 def test_planes_of_an_xcd_side_by_side(gpu, B, H, Sq, Sk):
-    """Two, nine, eleven (one by one), sixteen (by eights) and eight planes to an XCD; last blocks of 32 workgroups that are not full."""
+    """Two, nine, eleven (one by one), sixteen (by eights) and eight planes to an XCD; last blocks of 32 workgroups that are not full; planes
+    shared by two XCDs."""
     test_gradients_against_float64(gpu, torch.bfloat16, 6.4e-3, B, H, Sq, Sk)

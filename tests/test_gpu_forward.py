@@ -482,10 +482,12 @@ def test_lists_longer_than_the_lds_copy(gpu, BK):
 
 
 @pytest.mark.parametrize("B,H,nQ,BQ,D", [(2, 8, 17, 64, 64), (8, 5, 8, 64, 128), (3, 8, 11, 64, 64), (16, 12, 6, 64, 64),
-                                         (24, 16, 4, 64, 128), (1, 8, 33, 128, 128), (3, 8, 12, 128, 64)])
+                                         (24, 16, 4, 64, 128), (1, 8, 33, 128, 128), (3, 8, 12, 128, 64),
+                                         (1, 4, 67, 64, 64), (3, 12, 10, 64, 128), (1, 12, 22, 128, 64), (5, 28, 9, 64, 64)])
 def test_planes_of_an_xcd_side_by_side(gpu, B, H, nQ, BQ, D):
     """More than 256 Q tiles over planes that divide evenly over the XCDs (fwd_spread): one, two, an odd number and more planes to an
-    XCD, groups of them, a last block of 32 workgroups that is not full.  Every tile is the masked softmax of its own plane."""
+    XCD, groups of them, a last block of 32 workgroups that is not full; and planes shared by two XCDs, with Q tiles that are no
+    multiple of two or of four.  Every tile is the masked softmax of its own plane."""
     S = nQ * BQ
     q, k, v = W.qkv(B, H, S, D, torch.bfloat16, seed=nQ, device=gpu)
     mask = torch.stack([W.random_block_mask(S, 32, 0.6, seed=b, device=gpu) for b in range(B)])[:, None].expand(B, H, S, S)

@@ -156,7 +156,8 @@ def test_sizes_of_the_matrix_unit_kernel(gpu, D, BQ, BK):
         assert torch.isneginf(lse.cpu()[~live]).all() and (lse.cpu().double()[live] - want_lse[live]).abs().max() <= 1e-5
 
 
-@pytest.mark.parametrize("B,H,nQ,BQ,D", [(2, 8, 17, 64, 64), (3, 8, 11, 64, 128), (8, 5, 8, 64, 64), (3, 8, 12, 128, 64), (1, 8, 33, 64, 64)])
+@pytest.mark.parametrize("B,H,nQ,BQ,D", [(2, 8, 17, 64, 64), (3, 8, 11, 64, 128), (8, 5, 8, 64, 64), (3, 8, 12, 128, 64), (1, 8, 33, 64, 64),
+                                         (1, 4, 67, 64, 64), (3, 12, 10, 64, 64)])
 def test_planes_of_an_xcd_side_by_side(gpu, B, H, nQ, BQ, D):
     """More than 256 Q tiles over planes that divide evenly over the XCDs (fwd_spread)."""
     S = nQ * BQ
