@@ -48,18 +48,18 @@ PEAK_FP32_TFLOPS = 157.3   # MI355X dense fp32 MFMA peak, TFLOP/s
 # `bench.py --traffic-probe` and scaled by what the same counters read for the 1 GiB device copy of the same run
 # (`bench.py --traffic-summary` does the arithmetic).  profiles/hbm_traffic_all_kernels.txt holds the commands.
 TRAFFIC_BYTES = {
-    "forward, causal": (853633236, 268435456),
-    "forward, dense": (808007578, 268435456),
-    "forward, p=0.25": (1368278762, 268435456),
-    "forward, p=0.5": (2857154369, 268435456),
-    "forward, p=0.75": (2931945634, 268435456),
-    "forward, p=0.9": (1417183708, 268435456),
-    "backward, causal": (6768688003, 5242880299),
-    "forward, documents": (1726500309, 536870912),
-    "forward, composed": (1614452310, 268435669),
-    "mask_classify, composed mask 1 GiB": (1073825619, 58880),
-    "decode, 1": (4295548872, 397312),
-    "decode, 16": (1617185220, 5677056),
+    "forward, causal": (852181457, 268435456),
+    "forward, dense": (808008901, 268435499),
+    "forward, p=0.25": (1337445864, 268435456),
+    "forward, p=0.5": (2840242682, 268435456),
+    "forward, p=0.75": (2935913032, 268435456),
+    "forward, p=0.9": (1417311077, 268435456),
+    "backward, causal": (8335721843, 5242880171),
+    "forward, documents": (1724013299, 536870912),
+    "forward, composed": (1618501032, 268435456),
+    "mask_classify, composed mask 1 GiB": (1073825790, 58880),
+    "decode, 1": (4295549427, 397312),
+    "decode, 16": (1617185392, 5677056),
 }
 TRAFFIC_SOURCE = "profiles/hbm_traffic_all_kernels.txt"
 # The sources each kernel is built from.  The counters were read with kernels built from sources of the digests in
@@ -71,8 +71,8 @@ KERNEL_FILES = {
     "decode": ("sparse_decode.hip", "fwd_common.h", "kernels.h"),
     "backward": ("sparse_bwd.hip", "fwd_common.h", "kernels.h"),
 }
-TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "1aaab1fd0fe78028", "mask_classify": "2f127cde56abac51", "decode": "19b4fa5c1254a162",
-                                "backward": "c96bd3bf11bf9723"}
+TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "846297b992b895ac", "mask_classify": "ceddea2e80ec4703", "decode": "bfb067ef9a00552d",
+                                "backward": "3770c2296d22f013"}
 
 
 def kernel_sources_sha16(which=None):

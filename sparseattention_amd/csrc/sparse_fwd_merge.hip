@@ -190,6 +190,7 @@ bool fwd_in_halves(int64_t tiles, int Sk, int BQ, int BK, int D, int dtype, int 
 //   every key  256 tiles 16 24.9 | 25.4   32 41.5 | 41.3, D = 64 27.0 | 27.4   192 tiles 16 21.6 | 22.2   48 52.3 | 52.6
 //   blocks     256 tiles 16 24.0 | 24.3   32 36.5 | 36.8   window of 200 keys 16 13.6 | 14.2   32 13.0 | 13.7   (nothing to assist: the second tile's counts)
 //   16 chunks at D = 64: causal 16.7 | 15.9, every key 17.7 | 18.4.  12 chunks: causal 17.1 | 17.5.
+// The error against float64 is the same or less: causal S1024 bf16 2.4582e-3 | 2.4574e-3, S2048 fp16 3.1558e-4 | 3.1554e-4.
 // From 49 chunks on halves stay: causal 64 chunks of S4096 54.1 | 46.6, but every key 68.0 | 77.6, causal Sq 2048 Sk 4096 61.0 | 66.9.
 bool fwd_assists(int64_t planes, int nQ, int Sk, int BQ, int BK, int D, int dtype, int cus) {
     const int64_t tiles = planes * nQ;
