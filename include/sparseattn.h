@@ -384,6 +384,8 @@ int sa_sparse_attention_fwd_kernel(const void *q, const int64_t q_strides[4], co
 /*
  * The same forward for launches with too few Q tiles to fill the device (a chunk of a prompt against a long cache): the
  * list of a Q tile is shared by several workgroups and their partial results are added up by the last of them or by a second launch.
+ * Launches of up to one Q tile a compute unit may give every list an assistant instead, where the workspace has room for it (all of the bytes
+ * asked for); with less they run without.
  *   workspace   sa_fwd_split_workspace_bytes(...) bytes of device memory, 16-byte aligned; may be NULL when that is 0,
  *               which says that the launch has no use for it (the call is then sa_sparse_attention_fwd_kernel with the
  *               default kernel, or a kernel that walks a list in two halves by the waves of one workgroup).  The bytes depend

@@ -451,20 +451,20 @@ int forward_impl(const void *q, const int64_t q_strides[4], const void *k, const
     if (workspace && !fp.halves && kernel == SA_FWD_KERNEL_DEFAULT && !fp.sched) {
         sa::FwdSplitPlan plan;
         const size_t need = split_shape(B, H, Sq, Sk, D, BQ, BK, dtype, &plan);
+        // (assistants: a workspace that does not hold parts and words, as callers have whose size was 0 in an earlier library, goes without them)
+        const bool assists = need != 0 && plan.chunks == 0;
+        if (assists && (workspace_bytes < need + (size_t)16 * B * H * fp.nQ || !aligned(workspace, 16))) plan = sa::FwdSplitPlan();
         fp.nsplit = plan.nsplit;
         fp.split_chunks = plan.chunks;
         fp.split_least = plan.least;
-        if (need != 0 && (workspace_bytes < need || !aligned(workspace, 16)))
+        if (need != 0 && !assists && (workspace_bytes < need || !aligned(workspace, 16)))
             return fail(SA_ERR_WORKSPACE, "sa_sparse_attention_fwd_split: a 16-byte aligned workspace of %zu bytes required, %zu given", need, workspace_bytes);
         fp.ws = static_cast<float *>(workspace);
         fp.ws_ml = fp.ws + (need / 4 / (size_t)(D + 2)) * (size_t)D;
         // (a caller who asked an earlier library for the size has no place for them: a second launch then)
-        if (need != 0 && sa::fwd_merges_in_launch(B * H * fp.nQ, plan.nsplit, BQ, D, dtype) && workspace_bytes >= need + (size_t)8 * B * H * fp.nQ * plan.nsplit)
+        if (need != 0 && plan.nsplit > 1 && sa::fwd_merges_in_launch(B * H * fp.nQ, plan.nsplit, BQ, D, dtype) && workspace_bytes >= need + (size_t)8 * B * H * fp.nQ * plan.nsplit)
             fp.tag = next_launch_tag() | 1;  // (never 0)
-        if (plan.nsplit > 1 && plan.chunks == 0) {
-            if (fp.tag != 0) fp.spread = B * H;
-            else fp.nsplit = 1;
-        }
+        if (plan.nsplit > 1 && plan.chunks == 0) fp.spread = B * H;
     }
     if (kernel == SA_FWD_KERNEL_SHORT_LISTS) {
         if (f32 || !sa::fwd_c32_has(fp, dtype, D, BQ))

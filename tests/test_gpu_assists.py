@@ -1,5 +1,8 @@
 """Lists with assistants (up to one Q tile of 128 rows a compute unit): a second workgroup takes the end of a list that is longer than that
 of the tile it shares a compute unit with, and the last of the two to finish adds the parts up."""
+import ctypes
+import math
+
 import pytest
 import torch
 
@@ -61,3 +64,33 @@ def test_replays_of_a_captured_launch(gpu):
         torch.cuda.synchronize()
         assert torch.equal(o, want)
         assert torch.equal(sparse_attention(q, k, v, mask, 128, 64, mask_metadata=md), want)
+
+
+def test_a_workspace_without_room_goes_without_assistants(gpu):
+    """None, one that is too small, one whose address does not suit: the plain form, as for callers of a library that asked for none."""
+    B, H, S = 1, 32, 1024
+    q, k, v = W.qkv(B, H, S, 128, torch.bfloat16, seed=4, device=gpu)
+    mask = _masks(S, B, gpu)["causal"][:, None].expand(B, H, S, S)
+    md = compute_mask_kernel(mask, 128, 64)
+    lib, st = _native.load(), lambda t: _native.strides(t.stride())
+    need = lib.sa_fwd_split_workspace_bytes(B, H, S, S, 128, 128, 64, 0)
+    assert need >= 2 * 256 * 128 * 130 * 4 + 16 * 256
+
+    def call(ws, nbytes):
+        o = torch.empty_like(q)
+        pk = (md.packed_masks.data_ptr(), _native.strides(md.packed_masks.stride()[:2]))
+        rc = lib.sa_sparse_attention_fwd_split(
+            q.data_ptr(), st(q), k.data_ptr(), st(k), v.data_ptr(), st(v), o.data_ptr(), st(o), None, None, md.unmasked_kv_ids.data_ptr(),
+            st(md.unmasked_kv_ids), md.unmasked_lens.data_ptr(), st(md.unmasked_lens), md.masked_kv_ids.data_ptr(), st(md.masked_kv_ids),
+            md.masked_lens.data_ptr(), st(md.masked_lens), *pk, None, None, B, H, S, S, 128, 128, 64, 0, 128 ** -0.5 / math.log(2), ws, nbytes,
+            ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert rc == 0, lib.sa_last_error()
+        return o
+
+    ws = torch.empty(need + 32, dtype=torch.uint8, device=gpu)
+    plain = call(None, 0)
+    assert torch.equal(call(ws.data_ptr(), 64), plain) and torch.equal(call(ws.data_ptr(), need - 8), plain)
+    assert torch.equal(call(ws.data_ptr() + 8, need), plain)
+    o = call(ws.data_ptr(), need)
+    assert torch.equal(o, sparse_attention(q, k, v, mask, 128, 64, mask_metadata=md)) and not torch.equal(o, plain)
+    assert float((o.float() - plain.float()).abs().max()) <= 2e-2
