@@ -66,12 +66,13 @@ TRAFFIC_SOURCE = "profiles/hbm_traffic_all_kernels.txt"
 # TRAFFIC_KERNEL_SOURCES_SHA16; the line carries those beside the digests of the sources in the tree, per kernel, so a
 # reader sees whether a traffic figure belongs to the kernel that was timed.
 KERNEL_FILES = {
-    "forward": ("sparse_fwd_kernel.h", "sparse_fwd_c32.hip", "fwd_common.h", "kernels.h", "sparse_fwd.hip", "sparse_fwd_inst.hip"),
+    "forward": ("sparse_fwd_kernel.h", "sparse_fwd_c32.hip", "fwd_common.h", "kernels.h", "sparse_fwd.hip", "sparse_fwd_inst.hip",
+                "sparse_fwd_merge.hip"),  # (the last one: which order the workgroups take, fwd_spread, and with it what is read past L2)
     "mask_classify": ("mask_classify.hip", "kernels.h"),
     "decode": ("sparse_decode.hip", "fwd_common.h", "kernels.h"),
     "backward": ("sparse_bwd.hip", "fwd_common.h", "kernels.h"),
 }
-TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "846297b992b895ac", "mask_classify": "ceddea2e80ec4703", "decode": "bfb067ef9a00552d",
+TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "03a779714c1c5b97", "mask_classify": "ceddea2e80ec4703", "decode": "bfb067ef9a00552d",
                                 "backward": "3770c2296d22f013"}
 
 

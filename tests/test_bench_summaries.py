@@ -77,3 +77,14 @@ def test_traffic_digests_name_the_sources_in_the_tree():
     # the traffic constants were read with the kernels that are in the tree (a kernel edit must re-run the probe)
     for which, digest in bench.TRAFFIC_KERNEL_SOURCES_SHA16.items():
         assert bench.kernel_sources_sha16(which) == digest, which
+
+
+def test_rules_that_decide_traffic_are_in_the_digests():
+    # the order of a launch's workgroups, and with it what it reads past L2, comes from these rules
+    csrc = os.path.join(ROOT, "sparseattention_amd", "csrc")
+    for which, rules in {"forward": ("int fwd_spread(", "bool fwd_assists(", "FwdSplitPlan fwd_split_plan(", "bool fwd_in_halves("),
+                         "backward": ("int bwd_spread(", "int bwd_ds_group(", "size_t bwd_order_bytes(")}.items():
+        for rule in rules:
+            files = [n for n in sorted(os.listdir(csrc)) if n.endswith((".hip", ".h", ".cpp"))
+                     and any(rule in ln and ln.rstrip().endswith("{") for ln in open(os.path.join(csrc, n)))]
+            assert files and all(f in bench.KERNEL_FILES[which] for f in files), (rule, files)
