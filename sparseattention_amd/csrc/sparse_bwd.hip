@@ -23,6 +23,7 @@
 // so the 16-byte pieces of a row are swizzled with a function of the row that keeps both patterns free of bank
 // conflicts (bwd_swizzle).
 #include "fwd_common.h"
+#include "places.h"
 
 namespace sa {
 
@@ -91,16 +92,9 @@ __device__ __forceinline__ BwdPlace bwd_place_in_order(const P &p, int lin) {  /
 }
 __device__ __forceinline__ BwdPlace bwd_place(const BwdParams &p, int lin, int total) {
     const int per = total >> 3;
-    if (p.spread != 0) {  // (as in sparse_fwd_kernel<..., SD>)
-        int i = lin >> 3, group = 0;
-        if ((i >> 5) == 1 && (i | 31) < per) i ^= 31;
-        int n = 8 * i + (lin & 7);
-        if (p.spread != p.planes) {
-            group = n / (p.spread * p.nR);
-            n -= group * (p.spread * p.nR);
-        }
-        const int order = n / p.spread;
-        return {group * p.spread + n - order * p.spread, p.first_tile_first ? order : p.nR - 1 - order};
+    if (p.spread != 0) {
+        const SidePlace at = side_place(8 * side_turn(lin >> 3, per) + (lin & 7), p.spread, p.planes, p.nR);
+        return {at.plane, p.first_tile_first ? at.order : p.nR - 1 - at.order};
     }
     return bwd_place_in_order(p, lin < (per << 3) ? (lin & 7) * per + (lin >> 3) : lin);
 }
