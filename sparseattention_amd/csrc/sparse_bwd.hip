@@ -772,23 +772,6 @@ hipError_t launch_bwd_one(const BwdParams &dq, const BwdParams &dk, const BwdPar
 
 // The planes in groups of `group`, whose dS takes its turn in the workspace.  (The key tiles of a group in one launch with the
 // query tiles of the group before, dealt out evenly: 2 ... 15 % slower than launches of their own, with 2 ... 8 groups.)
-// How many of an XCD's planes the passes with dS walk together, their tiles side by side, heaviest under causal-like masks first: as in the forward
-// (fwd_spread) the longest lists go to different compute units then.  Up to nine planes: the caches mind it less here, where a chunk carries twice
-// the products.  An odd number that has no such divisor goes one by one, since two by two two XCDs would share a pair.  Backward with prepare, us,
-// two by two | side by side (four, where it says so, of eight or more):
-//   causal     B4 H16 S1024 97.2 | 86.4   B2 H16 S2048 169 | 154   B4 H16 S2048 268 | 254   B8 H16 S2048 523 | 483 (490)   B1 H16 S4096 264 | 256
-//              B8 H16 S4096 1675 | 1598 (1615)   B2 H16 S4096 431 | 435   B2 H16 S8192 1507 | 1480   B1 H8 S8192 516 | 481   B3 H24 S2048 320 | 278 (three 297)
-//   documents  B4 H16 S1024 97.0 | 84.5   B2 H16 S2048 140 | 131   B8 H16 S2048 373 | 346 (369)   B8 H16 S4096 734 | 713 (726)   B3 H24 S2048 253 | 188
-//   odd fours  causal B1 H12 S8192 737 | 625   B3 H12 S2048 186 | 163   B1 H4 S16384 1083 | 919   documents B3 H12 S2048 110 | 96   every key 282 | 289
-//   every key  B4 H16 S1024 122.5 | 119.7   B8 H16 S2048 827 | 822 (822)   B8 H16 S4096 2938 | 2967 (2947)   B3 H8 S4096 596 | 599
-// The three passes in one launch and the two at D = 64 gain nothing by it (D = 64 causal B1 H16 S4096 144 | 138, B8 H16 S1024 92.8 | 94.4).
-int bwd_spread(int planes) {
-    if (planes % 4 != 0) return 0;
-    const int unit = planes % 8 != 0 ? 4 : 8, each = planes / unit;
-    int n = each < 9 ? each : 9;
-    while (each % n != 0) n--;
-    return unit * n;
-}
 template <int DT, bool FAR>
 hipError_t launch_bwd_ds(const BwdParams &dq, const BwdParams &dk, const BwdParams &dv, uint8_t *ds, int group, hipStream_t stream) {
     constexpr int smem = BwdLds<128, true>::bytes;
@@ -799,6 +782,7 @@ hipError_t launch_bwd_ds(const BwdParams &dq, const BwdParams &dk, const BwdPara
     static unsigned long long attr_done_q = 0;
     if (const hipError_t e0 = allow_dynamic_smem(kern_q, BwdDqLds<128>::bytes, attr_done_q); e0 != hipSuccess) return e0;
     const int planes = dq.B * dq.H;
+    const int64_t plane_bytes = (int64_t)(dq.nR > dk.nR ? dq.nR : dk.nR) * (128 * 2 * 128 * 2);
     for (int p0 = 0; p0 < planes; p0 += group) {
         BwdLaunch l{};
         l.pass[0] = dk;
@@ -810,7 +794,7 @@ hipError_t launch_bwd_ds(const BwdParams &dq, const BwdParams &dk, const BwdPara
             p->planes = planes - p0 < group ? planes - p0 : group;
             p->ds = ds;
             p->far = FAR;
-            p->spread = bwd_spread(p->planes);
+            p->spread = bwd_spread(p->planes, plane_bytes);
         }
         l.tiles[0] = l.pass[0].planes * dk.nR;
         hipLaunchKernelGGL(kern, dim3((unsigned)l.tiles[0]), dim3(256), smem, stream, l);
