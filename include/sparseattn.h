@@ -394,9 +394,12 @@ int sa_sparse_attention_fwd_kernel(const void *q, const int64_t q_strides[4], co
  * sa_fwd_split_least_keys: this entry gains nothing on lists of up to that many keys (Sk: on none); a caller who knows that no
  * list is longer calls sa_sparse_attention_fwd_kernel with the default kernel and saves the workspace, the second launch or the
  * wider workgroups.
+ * sa_fwd_split_uneven_keys: where lists have assistants, the keys by which the longest list has to exceed the mean for this entry to gain by
+ * them, with less a caller who knows the lists calls the default kernel; 0 where they have none.
  */
 size_t sa_fwd_split_workspace_bytes(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype);
 int sa_fwd_split_least_keys(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype);
+int sa_fwd_split_uneven_keys(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype);
 int sa_sparse_attention_fwd_split(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
                                   const void *v, const int64_t v_strides[4], void *o, const int64_t o_strides[4],
                                   const uint8_t *mask, const int64_t mask_strides[4], const int32_t *full_ids,

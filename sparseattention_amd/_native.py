@@ -47,6 +47,7 @@ EXPORTS = (
     "sa_sparse_attention_fwd_kernel",
     "sa_fwd_split_workspace_bytes",
     "sa_fwd_split_least_keys",
+    "sa_fwd_split_uneven_keys",
     "sa_sparse_attention_fwd_split",
     "sa_sparse_attention_fwd_ragged",
     "sa_decode_num_splits",
@@ -147,6 +148,8 @@ def load() -> ctypes.CDLL:
     lib.sa_fwd_split_workspace_bytes.argtypes = [ctypes.c_int] * 8
     lib.sa_fwd_split_least_keys.restype = ctypes.c_int
     lib.sa_fwd_split_least_keys.argtypes = [ctypes.c_int] * 8
+    lib.sa_fwd_split_uneven_keys.restype = ctypes.c_int
+    lib.sa_fwd_split_uneven_keys.argtypes = [ctypes.c_int] * 8
     lib.sa_sparse_attention_fwd_split.restype = ctypes.c_int
     lib.sa_sparse_attention_fwd_split.argtypes = (
         [_vp, _i64p] * 4 + [_vp, _i64p] + [_vp, _i64p] * 4 + [_vp, _i64p] + [_vp, _i64p] + [ctypes.c_int] * 8

@@ -435,14 +435,16 @@ std::string forward_kernel(const Tensor &q, int64_t BQ, int64_t BK, py::object m
 // How a call with the default kernel hands its lists out: one workgroup each, or as sa_sparse_attention_fwd_split does (which needs
 // ws_bytes).  Metadata that says that no list is long enough to gain by it (list_stats) keeps them whole: 128 tiles of 16 chunks
 // 22.9 -> 20.0 us, no merge that finds nothing; 256 tiles of 64 rows, lists of 4 chunks 10.9 -> 10.2, of 128 rows and 8 chunks
-// 14.9 -> 13.6, no workgroups of twice the waves.
+// 14.9 -> 13.6, no workgroups of twice the waves.  So does metadata that says that they are too much alike for assistants.
 struct ListsShared {
     bool whole;
     size_t ws_bytes = 0;
 };
 ListsShared lists_shared(const Hints &h, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t Dk, int64_t BQ, int64_t BK, int dt) {
     if (h.stats && h.longest_list * BK <= sa_fwd_split_least_keys(B, H, Sq, Sk, Dk, BQ, BK, dt)) return {true};
-    return {false, sa_fwd_split_workspace_bytes(B, H, Sq, Sk, Dk, BQ, BK, dt)};
+    const size_t bytes = sa_fwd_split_workspace_bytes(B, H, Sq, Sk, Dk, BQ, BK, dt);
+    if (h.stats && bytes != 0 && ((double)h.longest_list - h.mean_list) * (double)BK < sa_fwd_split_uneven_keys(B, H, Sq, Sk, Dk, BQ, BK, dt)) return {true};
+    return {false, bytes};
 }
 // The same by name, for reports on what a call without a schedule runs: "whole", "halves" or "shared".
 std::string forward_lists(const Tensor &q, int64_t Sk, int64_t BQ, int64_t BK, py::object md) {

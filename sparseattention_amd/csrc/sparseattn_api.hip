@@ -597,6 +597,18 @@ int sa_fwd_split_least_keys(int B, int H, int Sq, int Sk, int D, int BQ, int BK,
     return plan.least << (dtype == SA_DTYPE_FP32 ? 5 : 6);  // (a plan's lists may be longer than this: less than Sk)
 }
 
+// Six chunks.  An assistant takes half of what a list is longer than the one beside it, from eight chunks on, and lists that lie evenly about their
+// mean reach as far below it as above.  One workgroup a list | with assistants, by how much the longest list exceeds the mean, 130 masks at 192 to
+// 256 Q tiles of S1024 ... 3072: less than two chunks -2 ... +7 %, two to four -3 ... +6 %, four to six -5 ... +7 % (at S1024 and 2048 +2 % in the
+// mean), six to seven -6 ... 0 %, seven and eight -13 ... +5 % (causal S1024 -7 %), more -39 ... +3 %.  us: every key S1024 22.5 | 23.4, window of 1000 keys
+// S2048 23.5 | 25.2, random blocks S1024 18.3 | 19.2.
+int sa_fwd_split_uneven_keys(int B, int H, int Sq, int Sk, int D, int BQ, int BK, int dtype) {
+    constexpr int kAssistUneven = 6;
+    sa::FwdSplitPlan plan;
+    if ((D != 64 && D != 128) || dtype < SA_DTYPE_BF16 || dtype > SA_DTYPE_FP32) return 0;
+    return split_shape(B, H, Sq, Sk, D, BQ, BK, dtype, &plan) != 0 && plan.chunks == 0 ? kAssistUneven << 6 : 0;
+}
+
 int sa_sparse_attention_fwd_split(const void *q, const int64_t q_strides[4], const void *k, const int64_t k_strides[4],
                                   const void *v, const int64_t v_strides[4], void *o, const int64_t o_strides[4],
                                   const uint8_t *mask, const int64_t mask_strides[4], const int32_t *full_ids,

@@ -94,3 +94,21 @@ def test_a_workspace_without_room_goes_without_assistants(gpu):
     o = call(ws.data_ptr(), need)
     assert torch.equal(o, sparse_attention(q, k, v, mask, 128, 64, mask_metadata=md)) and not torch.equal(o, plain)
     assert float((o.float() - plain.float()).abs().max()) <= 2e-2
+
+
+@pytest.mark.parametrize("BK", [32, 64, 128])
+def test_lists_known_to_be_alike_have_no_assistants(gpu, BK):
+    """Statistics that say by how much the longest list exceeds the mean: less than six chunks of 64 keys stay with one workgroup each."""
+    B, H, S = 1, 16, 2048
+    q, k, v = W.qkv(B, H, S, 128, torch.bfloat16, seed=5, device=gpu)
+    assert _native.load().sa_fwd_split_uneven_keys(B, H, S, S, 128, 128, BK, 0) == 6 * 64
+    tile = torch.arange(S, device=gpu) // 128
+    for longer in (0, 3, 4, 8):  # blocks of 128 keys that one of the 16 Q tiles has beyond the others' eight: 15/16 of them is what it exceeds the mean by
+        mask = ((tile[None] < 8) | ((tile[:, None] == 15) & (tile[None] < 8 + longer)))[None, None].expand(B, H, S, S)
+        known, unknown = compute_mask_kernel(mask, 128, BK, list_stats=True), compute_mask_kernel(mask, 128, BK)
+        assert (known.list_stats[1] - known.list_stats[0]) * BK == longer * 120
+        assert _native.host().forward_lists(q, S, 128, BK, unknown) == "shared"
+        assert _native.host().forward_lists(q, S, 128, BK, known) == ("whole" if longer * 120 < 384 else "shared")
+        o = sparse_attention(q, k, v, mask, 128, BK, mask_metadata=known, kernel="default")
+        want = torch.softmax((q.float() @ k.float().transpose(-1, -2).contiguous() * 128 ** -0.5).masked_fill(~mask, float("-inf")), -1) @ v.float()
+        assert float((o.float() - want).abs().max()) <= 2e-2
