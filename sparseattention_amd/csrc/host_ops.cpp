@@ -439,12 +439,14 @@ std::string forward_kernel(const Tensor &q, int64_t BQ, int64_t BK, py::object m
 struct ListsShared {
     bool whole;
     size_t ws_bytes = 0;
+    bool assistants = false;  // only they need the workspace: a call whose parts find no place goes without
 };
 ListsShared lists_shared(const Hints &h, int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t Dk, int64_t BQ, int64_t BK, int dt) {
     if (h.stats && h.longest_list * BK <= sa_fwd_split_least_keys(B, H, Sq, Sk, Dk, BQ, BK, dt)) return {true};
     const size_t bytes = sa_fwd_split_workspace_bytes(B, H, Sq, Sk, Dk, BQ, BK, dt);
-    if (h.stats && bytes != 0 && ((double)h.longest_list - h.mean_list) * (double)BK < sa_fwd_split_uneven_keys(B, H, Sq, Sk, Dk, BQ, BK, dt)) return {true};
-    return {false, bytes};
+    const int uneven = bytes != 0 ? sa_fwd_split_uneven_keys(B, H, Sq, Sk, Dk, BQ, BK, dt) : 0;
+    if (h.stats && ((double)h.longest_list - h.mean_list) * (double)BK < uneven) return {true};
+    return {false, bytes, uneven > 0};
 }
 // The same by name, for reports on what a call without a schedule runs: "whole", "halves" or "shared".
 std::string forward_lists(const Tensor &q, int64_t Sk, int64_t BQ, int64_t BK, py::object md) {
@@ -539,7 +541,8 @@ std::optional<Out> forward_impl(const Tensor &q, const Tensor &k, const Tensor &
     if (!shared.whole && shared.ws_bytes != 0) {
         try {
             ws = at::empty({(int64_t)(shared.ws_bytes / 4)}, opt_f32);
-        } catch (const c10::OutOfMemoryError &) {  // (no place for parts: one workgroup a list)
+        } catch (const c10::OutOfMemoryError &) {  // (shared lists of one workgroup each would be several times as long: for the caller to know)
+            if (!shared.assistants) throw;
             shared.whole = true;
         }
     }

@@ -112,3 +112,41 @@ def test_lists_known_to_be_alike_have_no_assistants(gpu, BK):
         o = sparse_attention(q, k, v, mask, 128, BK, mask_metadata=known, kernel="default")
         want = torch.softmax((q.float() @ k.float().transpose(-1, -2).contiguous() * 128 ** -0.5).masked_fill(~mask, float("-inf")), -1) @ v.float()
         assert float((o.float() - want).abs().max()) <= 2e-2
+
+
+def _without_room(fn, spare):
+    """fn() with `spare` more bytes than are held already for it to allocate."""
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + spare) / total)
+    try:
+        return fn()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+def test_no_memory_for_parts(gpu):
+    """Assistants are done without where their parts find no place, as such launches asked for none once.  A launch whose lists are shared
+    for their length says that it has no memory."""
+    B, H, S = 1, 32, 1024
+    q, k, v = W.qkv(B, H, S, 128, torch.bfloat16, seed=6, device=gpu)
+    mask = _masks(S, B, gpu)["causal"][:, None].expand(B, H, S, S)
+    md = compute_mask_kernel(mask, 128, 64)
+    assert _native.load().sa_fwd_split_workspace_bytes(B, H, S, S, 128, 128, 64, 0) > 32 << 20
+    with_parts = sparse_attention(q, k, v, mask, 128, 64, mask_metadata=md)
+    got = _without_room(lambda: sparse_attention(q, k, v, mask, 128, 64, mask_metadata=md), 24 << 20)
+    even = compute_mask_kernel(mask, 128, 64)
+    even.list_stats = (16.0, 16)  # (statistics that keep the lists whole)
+    assert torch.equal(got, sparse_attention(q, k, v, mask, 128, 64, mask_metadata=even, kernel="default"))
+    assert not torch.equal(got, with_parts) and float((got.float() - with_parts.float()).abs().max()) <= 2e-2
+
+    q, k, v = (torch.randn(1, 32, s, 128, device=gpu, dtype=torch.bfloat16) for s in (512, 8192, 8192))
+    mask = torch.ones(1, 1, 512, 8192, dtype=torch.bool, device=gpu).expand(1, 32, 512, 8192)
+    md = compute_mask_kernel(mask, 128, 64)
+    lib = _native.load()
+    assert lib.sa_fwd_split_workspace_bytes(1, 32, 512, 8192, 128, 128, 64, 0) > 24 << 20 and lib.sa_fwd_split_uneven_keys(1, 32, 512, 8192, 128, 128, 64, 0) == 0
+    want = sparse_attention(q, k, v, mask, 128, 64, mask_metadata=md)
+    with pytest.raises(torch.OutOfMemoryError):
+        _without_room(lambda: sparse_attention(q, k, v, mask, 128, 64, mask_metadata=md), 16 << 20)
+    assert torch.equal(sparse_attention(q, k, v, mask, 128, 64, mask_metadata=md), want)
