@@ -442,7 +442,7 @@ int forward_impl(const void *q, const int64_t q_strides[4], const void *k, const
     }
     fp.nsplit = 1;
     fp.spread = 0;
-    {
+    if (!fp.sched && D <= 128 && (BQ == 64 || BQ == 128) && kernel != SA_FWD_KERNEL_SHORT_LISTS) {  // (no other form has planes side by side)
         int dev = 0, cus = 0;
         if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
             fp.spread = sa::fwd_spread((int64_t)B * H, fp.nQ, BQ, (int64_t)Sk * D * (f32 ? 8 : 4), cus);
