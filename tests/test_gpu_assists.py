@@ -1,6 +1,7 @@
 """Lists with assistants (up to one Q tile of 128 rows a compute unit): a second workgroup takes the end of a list that is longer than that
 of the tile it shares a compute unit with, and the last of the two to finish adds the parts up."""
 import ctypes
+import gc
 import math
 
 import pytest
@@ -115,13 +116,21 @@ def test_lists_known_to_be_alike_have_no_assistants(gpu, BK):
         assert float((o.float() - want).abs().max()) <= 2e-2
 
 
-def _without_room(fn, spare):
-    """fn() with `spare` more bytes than are held already for it to allocate."""
+def _without_room(fn):
+    """fn() with 16 MiB in one piece for it to allocate, and less than 2 MiB anywhere else."""
+    gc.collect()
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
-    total = torch.cuda.get_device_properties(0).total_memory
-    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + spare) / total)
+    room, filled = torch.empty(16 << 20, dtype=torch.uint8, device="cuda"), []
+    torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved() / torch.cuda.get_device_properties(0).total_memory)
     try:
+        for size in (64 << 20, 8 << 20, 2 << 20):  # (what other tensors left free of their segments)
+            try:
+                while True:
+                    filled.append(torch.empty(size, dtype=torch.uint8, device="cuda"))
+            except torch.OutOfMemoryError:
+                pass
+        del room
         return fn()
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
@@ -136,7 +145,7 @@ def test_no_memory_for_parts(gpu):
     md = compute_mask_kernel(mask, 128, 64)
     assert _native.load().sa_fwd_split_workspace_bytes(B, H, S, S, 128, 128, 64, 0) > 32 << 20
     with_parts = sparse_attention(q, k, v, mask, 128, 64, mask_metadata=md)
-    got = _without_room(lambda: sparse_attention(q, k, v, mask, 128, 64, mask_metadata=md), 24 << 20)
+    got = _without_room(lambda: sparse_attention(q, k, v, mask, 128, 64, mask_metadata=md))
     even = compute_mask_kernel(mask, 128, 64)
     even.list_stats = (16.0, 16)  # (statistics that keep the lists whole)
     assert torch.equal(got, sparse_attention(q, k, v, mask, 128, 64, mask_metadata=even, kernel="default"))
@@ -149,7 +158,7 @@ def test_no_memory_for_parts(gpu):
     assert lib.sa_fwd_split_workspace_bytes(1, 32, 512, 8192, 128, 128, 64, 0) > 24 << 20 and lib.sa_fwd_split_uneven_keys(1, 32, 512, 8192, 128, 128, 64, 0) == 0
     want = sparse_attention(q, k, v, mask, 128, 64, mask_metadata=md)
     with pytest.raises(torch.OutOfMemoryError):
-        _without_room(lambda: sparse_attention(q, k, v, mask, 128, 64, mask_metadata=md), 16 << 20)
+        _without_room(lambda: sparse_attention(q, k, v, mask, 128, 64, mask_metadata=md))
     assert torch.equal(sparse_attention(q, k, v, mask, 128, 64, mask_metadata=md), want)
 
 
