@@ -48,18 +48,18 @@ PEAK_FP32_TFLOPS = 157.3   # MI355X dense fp32 MFMA peak, TFLOP/s
 # `bench.py --traffic-probe` and scaled by what the same counters read for the 1 GiB device copy of the same run
 # (`bench.py --traffic-summary` does the arithmetic).  profiles/hbm_traffic_all_kernels.txt holds the commands.
 TRAFFIC_BYTES = {
-    "forward, causal": (848883396, 268435456),
-    "forward, dense": (808012229, 268435456),
-    "forward, p=0.25": (1326817190, 268435456),
-    "forward, p=0.5": (2860699620, 268435456),
-    "forward, p=0.75": (2932695438, 268435456),
-    "forward, p=0.9": (1417050091, 268435456),
-    "backward, causal": (7253467608, 5242880981),
-    "forward, documents": (1726142490, 536870912),
-    "forward, composed": (1613868558, 268435456),
-    "mask_classify, composed mask 1 GiB": (1073825790, 58880),
-    "decode, 1": (4295549427, 397312),
-    "decode, 16": (1617185477, 5677056),
+    "forward, causal": (852500273, 268435456),
+    "forward, dense": (808013615, 268435456),
+    "forward, p=0.25": (1354688514, 268435456),
+    "forward, p=0.5": (2830369863, 268435456),
+    "forward, p=0.75": (2935829472, 268435456),
+    "forward, p=0.9": (1414969214, 268435456),
+    "backward, causal": (7257962037, 5242880213),
+    "forward, documents": (1722871683, 536870912),
+    "forward, composed": (1619090075, 268435456),
+    "mask_classify, composed mask 1 GiB": (1073825705, 58891),
+    "decode, 1": (4295549299, 397312),
+    "decode, 16": (1617185434, 5677109),
 }
 TRAFFIC_SOURCE = "profiles/hbm_traffic_all_kernels.txt"
 # The sources each kernel is built from.  The counters were read with kernels built from sources of the digests in
@@ -72,7 +72,7 @@ KERNEL_FILES = {
     "decode": ("sparse_decode.hip", "fwd_common.h", "kernels.h"),
     "backward": ("sparse_bwd.hip", "places.h", "fwd_common.h", "kernels.h"),
 }
-TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "03a779714c1c5b97", "mask_classify": "ceddea2e80ec4703", "decode": "bfb067ef9a00552d",
+TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "a1fe56c4d144428b", "mask_classify": "ceddea2e80ec4703", "decode": "bfb067ef9a00552d",
                                 "backward": "8c4c01fcae1ae3a8"}
 
 

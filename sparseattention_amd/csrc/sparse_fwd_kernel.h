@@ -1517,7 +1517,7 @@ __global__ __launch_bounds__(NW * 64 * (TW ? 2 : 1), (NW >= 4 && D <= 128) ? 2 :
 }
 
 // HOW 0: one workgroup per Q tile, 1: persistent workgroups, 2: lists shared by workgroups (SP), 3: ragged sizes (RG; its form by the head dim),
-// 4: lists walked in two halves (TW)
+// 4: lists walked in two halves (TW), 5: lists with assistants (AS)
 template <int DT, int D, int NW, int MODE, bool PK, int HOW, int RGD, bool SD>
 hipError_t launch_form(const FwdParams &p, hipStream_t stream) {
     // Eight waves fill a CU's register file on their own, so that workgroup can have most of the LDS: 4 stages.

@@ -187,10 +187,15 @@ bool fwd_in_halves(int64_t tiles, int Sk, int BQ, int BK, int D, int dtype, int 
 //   causal     256 tiles  D = 128  16 chunks 22.5 | 21.1   20 24.2 | 20.2 (160 tiles)   32 36.8 | 29.0   D = 64  32 26.2 | 20.6
 //              192 tiles  16 20.7 | 18.4   48 50.3 | 35.1
 //   documents of 64 ... 1024  256 tiles 32 chunks 22.2 | 20.1, D = 64 16.5 | 14.7   192 tiles 16 17.5 | 15.9   160 tiles 20 17.4 | 15.8
-//   every key  256 tiles 16 24.9 | 25.4   32 41.5 | 41.3, D = 64 27.0 | 27.4   192 tiles 16 21.6 | 22.2   48 52.3 | 52.6
-//   blocks     256 tiles 16 24.0 | 24.3   32 36.5 | 36.8   window of 200 keys 16 13.6 | 14.2   32 13.0 | 13.7   (nothing to assist: the second tile's counts)
+// Lists with nothing to assist pay for the place and the counts of the tile beside, about 0.4 us, and for second workgroups that end at once, about 0.3.  Where
+// the lists are known to be alike they get none (sa_fwd_split_uneven_keys); where nothing is known:
+//   every key  256 tiles 16 22.3 | 23.0   32 38.2 | 39.8, D = 64 27.4 | 27.3   192 tiles 16 21.1 | 21.6   48 50.8 | 51.8
+//   blocks of 128 keys, a half empty, three masks  16 18.2 | 19.3, 17.4 | 18.5, 19.6 | 20.3   32 28.8 | 29.6, 27.3 | 26.3, 25.4 | 26.4   192 tiles 48 40.8 | 35.6, 34.5 | 34.9, 36.5 | 35.3
+//   window of 200 keys  16 12.4 | 13.2   32 12.5 | 13.1, D = 64 9.5 | 9.8   192 tiles 48 12.2 | 12.4   of 1000 keys  32 23.6 | 25.4   192 tiles 48 23.8 | 24.0
 //   16 chunks at D = 64: causal 16.7 | 15.9, every key 17.7 | 18.4.  12 chunks: causal 17.1 | 17.5.
-// The error against float64 is the same or less: causal S1024 bf16 2.4582e-3 | 2.4574e-3, S2048 fp16 3.1558e-4 | 3.1554e-4.
+// A whole call on a fresh causal mask of S1024 27.0 | 25.6.  Other bits than one workgroup a list gives, since each part's P is rounded against a reference value
+// of its own.  The error against float64 is less in all of 46 cases (nine shapes, causal, documents and blocks, both types), by 0.003 to 0.07 %: causal S1024
+// bf16 2.4710e-3 | 2.4701e-3, S2048 fp16 3.1557e-4 | 3.1547e-4.
 // From 49 chunks on halves stay: causal 64 chunks of S4096 54.1 | 46.6, but every key 68.0 | 77.6, causal Sq 2048 Sk 4096 61.0 | 66.9.
 bool fwd_assists(int64_t planes, int nQ, int Sk, int BQ, int BK, int D, int dtype, int cus) {
     const int64_t tiles = planes * nQ;
@@ -223,11 +228,13 @@ int fwd_halves_least(int BQ, int D) { return BQ == 64 ? 5 : (D == 64 ? 13 : 16);
 // An odd number of planes an XCD cannot be taken two by two (two XCDs shared a pair, one its long lists): then up to 6 MiB, else one by one.
 //   B1 H24 S4096 causal 113.9 | 105.5, blocks 114.7 | 113.9, documents 62.3 | 57.8   B3 H24 311 | 282, 276 | 280, 137 | 124
 //   one by one  B5 H8 S4096 187 | 179, blocks 166.3 | 166.2, documents 87.8 | 82.3   B1 H8 S16384 537 | 460, documents 69 | 75
+//   (documents of one plane an XCD go either way by mask, -26 ... +20 % over 63 of them at S8192 ... 32768, -1.8 % in the mean)
 // Planes that are an odd number of fours (12 heads, 4 heads) took two by two leave one XCD the long lists of a pair and another its short ones; side
 // by side a plane's Q tiles go to two XCDs in turn, by twos:
 //   causal B3 H12 S2048 60.9 | 54.4   B1 H4 S16384 347 | 304   B1 H12 S8192 D = 64 137 | 132   B1 H12 S4096 84.3 | 81.4   B5 H12 S1024 31.3 | 30.9
 //   documents B3 H12 S2048 37.2 | 34.3   B5 H12 S1024 29.8 | 27.9   blocks 87.5 | 86.0, 36.3 | 38.1   every key 98.8 | 99.3
 //   window of 500 keys B3 H12 S2048 37.4 | 38.4   B1 H12 S8192 D = 64 25.3 | 27.4 (one by one, not by twos: 24.1 | 25.8 for 25.0 | 25.8 at S4096)
+//   (on another device 36.3 | 35.0, 24.1 | 25.1, of 1000 keys B3 H12 S2048 46.2 | 41.1: no reason to leave windows out where they are known)
 //   float32 B3 H12 S1152 D = 64 causal 154.5 | 110.8, documents 125.6 | 108.5
 // float32, whose chunks keep the matrix unit busy four to eight times as long: causal B2 H16 S1024 D64 144.2 | 88.9, B4 H12 148.8 | 108.0,
 // B1 H8 S4096 479 | 321, BLOCK_Q 128 B3 H8 S2048 281 | 199; documents B2 H16 S1024 120.7 | 89.2; every key 144.5 | 144.3; D = 128 B1 H16 S2048 313 | 311.
