@@ -72,8 +72,8 @@ KERNEL_FILES = {
     "decode": ("sparse_decode.hip", "fwd_common.h", "kernels.h"),
     "backward": ("sparse_bwd.hip", "places.h", "fwd_common.h", "kernels.h"),
 }
-TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "a1fe56c4d144428b", "mask_classify": "ceddea2e80ec4703", "decode": "bfb067ef9a00552d",
-                                "backward": "8c4c01fcae1ae3a8"}
+TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "fdca7a10bd4b8336", "mask_classify": "ceddea2e80ec4703", "decode": "bfb067ef9a00552d",
+                                "backward": "5813d3b0f7dca388"}
 
 
 def kernel_sources_sha16(which=None):

@@ -65,6 +65,10 @@ SA_PLACES_FN SidePlace side_place(int n, int spread, int planes, int tiles) {
 //     blocks        1683, 1621 | 1670, 1649 (1721, 1674)   1275, 1261 | 1283, 1235 (1307, 1277)
 //     window of 512 326 | 321 (324)   261 | 251 (251)
 //     every key     2917 | 2918 (2916)   2211 | 2189 (2200)
+// The passes apart, keys + queries, two by two | with 4.5, 9 and 18 MiB held (two, four and eight planes of B8 H16 S4096):
+//   B8 H16 S4096  causal 1187 + 488 | 1179 + 487   1203 + 432   1200 + 412   blocks 1243 + 502 | 1269 + 508   1262 + 510   1282 + 524   every key 2209 + 724 | 2213 + 733   2196 + 745   2205 + 757
+//   B8 H16 S2048  causal  346 + 153 |  319 + 151    318 + 146    328 + 140   blocks  378 + 162 |  369 + 167    366 + 159    364 + 178   documents 200 + 88 | 202 + 91   178 + 83   185 + 77
+//   B2 H16 S8192  causal 1098 + 408 | 1112 + 439   1115 + 402   1116 + 378   blocks 1201 + 451 | 1176 + 454   1183 + 452   1200 + 470   documents 191 + 79 | 184 + 75   178 + 73   173 + 70
 // Runs of one side differ by up to 3 %.  Causal lists of few rounds of workgroups would gain by more planes than that, where blocks lose.
 // The three passes in one launch and the two at D = 64 gain nothing by it (D = 64 causal B1 H16 S4096 144 | 138, B8 H16 S1024 92.8 | 94.4).
 inline int bwd_spread(int planes, int64_t plane_bytes) {

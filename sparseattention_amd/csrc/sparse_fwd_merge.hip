@@ -193,7 +193,7 @@ bool fwd_in_halves(int64_t tiles, int Sk, int BQ, int BK, int D, int dtype, int 
 //   blocks of 128 keys, a half empty, three masks  16 18.2 | 19.3, 17.4 | 18.5, 19.6 | 20.3   32 28.8 | 29.6, 27.3 | 26.3, 25.4 | 26.4   192 tiles 48 40.8 | 35.6, 34.5 | 34.9, 36.5 | 35.3
 //   window of 200 keys  16 12.4 | 13.2   32 12.5 | 13.1, D = 64 9.5 | 9.8   192 tiles 48 12.2 | 12.4   of 1000 keys  32 23.6 | 25.4   192 tiles 48 23.8 | 24.0
 //   16 chunks at D = 64: causal 16.7 | 15.9, every key 17.7 | 18.4.  12 chunks: causal 17.1 | 17.5.
-// A whole call on a fresh causal mask of S1024 27.0 | 25.6.  Other bits than one workgroup a list gives, since each part's P is rounded against a reference value
+// A whole call on a fresh causal mask of S1024 26.9 | 24.8, on another device 27.0 | 25.6.  Other bits than one workgroup a list gives, since each part's P is rounded against a reference value
 // of its own.  The error against float64 is less in all of 46 cases (nine shapes, causal, documents and blocks, both types), by 0.003 to 0.07 %: causal S1024
 // bf16 2.4710e-3 | 2.4701e-3, S2048 fp16 3.1557e-4 | 3.1547e-4.
 // From 49 chunks on halves stay: causal 64 chunks of S4096 54.1 | 46.6, but every key 68.0 | 77.6, causal Sq 2048 Sk 4096 61.0 | 66.9.
