@@ -48,18 +48,18 @@ PEAK_FP32_TFLOPS = 157.3   # MI355X dense fp32 MFMA peak, TFLOP/s
 # `bench.py --traffic-probe` and scaled by what the same counters read for the 1 GiB device copy of the same run
 # (`bench.py --traffic-summary` does the arithmetic).  profiles/hbm_traffic_all_kernels.txt holds the commands.
 TRAFFIC_BYTES = {
-    "forward, causal": (852500273, 268435456),
-    "forward, dense": (808013615, 268435456),
-    "forward, p=0.25": (1354688514, 268435456),
-    "forward, p=0.5": (2830369863, 268435456),
-    "forward, p=0.75": (2935829472, 268435456),
-    "forward, p=0.9": (1414969214, 268435456),
-    "backward, causal": (7257962037, 5242880213),
-    "forward, documents": (1722871683, 536870912),
-    "forward, composed": (1619090075, 268435456),
-    "mask_classify, composed mask 1 GiB": (1073825705, 58891),
-    "decode, 1": (4295549299, 397312),
-    "decode, 16": (1617185434, 5677109),
+    "forward, causal": (855432373, 268435456),
+    "forward, dense": (808016666, 268435456),
+    "forward, p=0.25": (1400919032, 268435456),
+    "forward, p=0.5": (2950406111, 268435456),
+    "forward, p=0.75": (3010779272, 268435456),
+    "forward, p=0.9": (1425153721, 268435456),
+    "backward, causal": (7270587958, 5242880853),
+    "forward, documents": (1772745329, 536870912),
+    "forward, composed": (1632765807, 268435456),
+    "mask_classify, composed mask 1 GiB": (1073825790, 58880),
+    "decode, 1": (4295549726, 397312),
+    "decode, 16": (1617185562, 5677056),
 }
 TRAFFIC_SOURCE = "profiles/hbm_traffic_all_kernels.txt"
 # The sources each kernel is built from.  The counters were read with kernels built from sources of the digests in
@@ -73,7 +73,7 @@ KERNEL_FILES = {
     "backward": ("sparse_bwd.hip", "places.h", "fwd_common.h", "kernels.h"),
 }
 TRAFFIC_KERNEL_SOURCES_SHA16 = {"forward": "fdca7a10bd4b8336", "mask_classify": "ceddea2e80ec4703", "decode": "bfb067ef9a00552d",
-                                "backward": "5813d3b0f7dca388"}
+                                "backward": "a23eaf1f5eb0dfa4"}
 
 
 def kernel_sources_sha16(which=None):

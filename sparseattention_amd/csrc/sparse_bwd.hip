@@ -782,7 +782,6 @@ hipError_t launch_bwd_ds(const BwdParams &dq, const BwdParams &dk, const BwdPara
     static unsigned long long attr_done_q = 0;
     if (const hipError_t e0 = allow_dynamic_smem(kern_q, BwdDqLds<128>::bytes, attr_done_q); e0 != hipSuccess) return e0;
     const int planes = dq.B * dq.H;
-    const int64_t plane_bytes = (int64_t)(dq.nR > dk.nR ? dq.nR : dk.nR) * (128 * 2 * 128 * 2);
     for (int p0 = 0; p0 < planes; p0 += group) {
         BwdLaunch l{};
         l.pass[0] = dk;
@@ -794,7 +793,7 @@ hipError_t launch_bwd_ds(const BwdParams &dq, const BwdParams &dk, const BwdPara
             p->planes = planes - p0 < group ? planes - p0 : group;
             p->ds = ds;
             p->far = FAR;
-            p->spread = bwd_spread(p->planes, plane_bytes);
+            p->spread = bwd_spread(p->planes, dq.nR > dk.nR ? dq.nR : dk.nR);
         }
         l.tiles[0] = l.pass[0].planes * dk.nR;
         hipLaunchKernelGGL(kern, dim3((unsigned)l.tiles[0]), dim3(256), smem, stream, l);
